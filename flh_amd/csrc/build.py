@@ -12,12 +12,14 @@ import sys
 
 HERE = pathlib.Path(__file__).resolve().parent
 OUT = HERE.parent / "libflh_hip.so"
-SOURCES = ["capi.hip", "reference_abi.hip", "gemm_i4.hip", "gemm_i4_decode.hip", "gemm_f6.hip", "fwht_quant.hip", "fwht_mfma.hip", "rope_cache.hip", "decode_attention.hip", "prefill_attention.hip"]
+SOURCES = ["capi.hip", "reference_abi.hip", "gemm_i4.hip", "gemm_i4_decode.hip", "gemm_f6.hip", "gemm_f6_large_row.hip", "gemm_f6_large_group.hip", "fwht_quant.hip", "fwht_mfma.hip", "rope_cache.hip", "decode_attention.hip", "prefill_attention.hip"]
+# matrix-core results land in ordinary VGPRs when a kernel fits 256 registers (no copies out of AGPRs)
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+# ... except where the accumulators fill the accumulation registers
+AGPR_FORM = {"gemm_f6_large_row.hip"}
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    # matrix-core results land in ordinary VGPRs when a kernel fits 256 registers (no copies out of AGPRs)
-    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Wno-unused-command-line-argument", "-Wno-unknown-attributes",
 ]
 
@@ -31,7 +33,8 @@ def build(verbose=True, extra=(), out=None, tag=""):
     objs = []
     for s in SOURCES:
         o = HERE / (s + tag + ".o")
-        cmd = [hipcc, *[f for f in FLAGS if f != "-shared"], *extra, "-c", str(HERE / s), "-o", str(o)]
+        form = [] if s in AGPR_FORM else VGPR_FORM
+        cmd = [hipcc, *[f for f in FLAGS if f != "-shared"], *form, *extra, "-c", str(HERE / s), "-o", str(o)]
         if verbose:
             print(" ".join(cmd), flush=True)
         r = subprocess.run(cmd, capture_output=True, text=True)

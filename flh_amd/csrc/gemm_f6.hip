@@ -22,7 +22,7 @@
 // number m that sits in wave half h takes one piece as its operand, and the 48 bytes of a wave half are three
 // 16-byte chunks.
 //
-// Tiling as the int8 kernel: workgroup = 4 waves (2 x 2), wave tile of 32 x 32 MFMA tiles, K advances by 128 codes
+// Tiling (launches that fill the chip with larger tiles take the kernels of gemm_f6_large.h): workgroup = 4 waves (2 x 2), wave tile of 32 x 32 MFMA tiles, K advances by 128 codes
 // (96 bytes per row) per stage, stages form a ring in LDS filled by direct-to-LDS loads.  Chunk c of tile row r
 // sits in slot 6 r + (c ^ ((r >> 3) & 1)): sixteen consecutive rows read at one logical chunk touch sixteen
 // different groups of four banks.  Fragment reads run half a stage ahead of the MFMAs that use them.
@@ -32,6 +32,7 @@
 
 #include "gemm_i4.h"
 #include "f6_codes.h"
+#include "gemm_f6_large.h"
 
 namespace flh {
 
@@ -56,14 +57,14 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), ((BM / WM) * (BN / WN) 
 void gemm_f6_kernel(const GemmArgs p) {
   constexpr int TM = WM / 32, TN = WN / 32;
   constexpr int WAVES_N = BN / WN;
-  constexpr int WAVES = (BM / WM) * (BN / WN);        // 4, or 8 (two per SIMD from one workgroup)
+  constexpr int WAVES = (BM / WM) * (BN / WN);
   constexpr int T = 64 * WAVES;
   constexpr int STAGE = (BM + BN) * kBlockBytes;
   constexpr int TI = (BM + BN) * 6 / 64;              // 1 KiB load instructions per stage
   constexpr int NI_LO = TI / WAVES, NI_X = TI % WAVES; // the first NI_X waves issue one more than the others
   constexpr int NI = NI_LO + (NI_X ? 1 : 0);
   constexpr int EPI_PITCH = WN * 2 + kEpiPadF6;
-  static_assert((WAVES == 4 || WAVES == 8) && BM % 64 == 0 && BN % 64 == 0, "tile shape");
+  static_assert(WAVES == 4 && BM % 64 == 0 && BN % 64 == 0, "tile shape");
   static_assert(!SWIGLU || (EPI != kInt32 && WAVES_N == 2), "gate | up halves are the two wave columns");
   static_assert(!ROPE || (EPI != kInt32 && BN == 128 && WN == 64 && !SWIGLU), "a tile column is one head of 128");
   constexpr int BNC = SWIGLU ? BN / 2 : BN;           // output channels per tile
@@ -668,50 +669,84 @@ int total_n_f6(const GemmArgs& a) {
   return n;
 }
 
+// The large-tile kernels (gemm_f6_large.h) take launches with at least eight steps of K and rows of whole 16-byte stores.
+// Group scales come to LDS in pieces of eight groups from dword-aligned rows, two groups at a time, and a tile's last
+// block of eight must leave the next tile's first one time to arrive.
+bool large_supported(const GemmArgs& a, bool grouped) {
+  const int kt = a.K >> 7;
+  if (kt < 8 || a.N % 8) return false;
+  for (int s = 1; s < a.n_seg; ++s)
+    if (a.seg_N[s] % 8) return false;
+  if (!grouped) return true;
+  auto off4 = [](const void* q) { return ((uintptr_t)q & 3) != 0; };
+  if (kt % 2 || (kt % 8 && kt % 8 < 6) || off4(a.As) || off4(a.Bs) || off4(a.Bs2)) return false;
+  for (int s = 1; s < a.n_seg; ++s)
+    if (off4(a.seg_Bs[s])) return false;
+  return (uint64_t)(a.M > total_n_f6(a) ? a.M : total_n_f6(a)) * kt < (1ull << 31);
+}
+// Which large tile a launch over `columns` weight rows takes: 256 x 256 (kWide), 256 x 128 (kNarrow) or neither.  Measured
+// at M = 64 .. 4096 on the Llama widths with weights that come from HBM (us; K = 4096 unless stated):
+//  * one scale per row: as soon as 128 x 128 tiles would come more than one to a compute unit, a large tile is faster
+//    (1024 x 6144 tokens x channels: 25 against 29; 2048 x 4096: 25 against 27; 1024 x 4096, one tile each: 19 against 17).
+//    Of the two, a 256 x 128 tile takes 0.62 of the time of a 256 x 256 one; a round that is not full costs the mean of its
+//    share and a whole one, as the part clocks up (wide against narrow: 2048 x 28672, 3.5 rounds: 142 against 165; 2048 x
+//    4096, half a round: 30 against 25; 1531 x 6144, 0.56 of a round against 1.13: 34 against 39).
+//  * token scales: a round of 256 x 128 tiles takes 29.5, a round of 128 x 128 ones 16.6 (2048 x 28672: 208 against 223;
+//    1024 x 12288, 1.5 rounds of large tiles: 56 against 51).
+//  * group scales: the large tile from one 128 x 128 tile per compute unit on (1024 x 4096: 30 against 32; 2048 x 28672:
+//    229 against 303).
+enum LargeTile { kNoLarge = 0, kWide = 1, kNarrow = 2 };
+LargeTile large_choice(const GemmArgs& a, int epi, long columns) {
+  const bool grouped = epi != kRowScale;
+  if (!large_supported(a, grouped)) return kNoLarge;
+  const int forced = g_tune_tile.load(std::memory_order_relaxed);
+  if (forced == 256) return grouped || g_tune_ks.load(std::memory_order_relaxed) == 2 ? kNarrow : kWide;
+  if (forced) return kNoLarge;
+  auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((columns + bn - 1) / bn); };
+  auto rounds = [](long t) { return (t + 255) / 256; };
+  const long small = tiles(128, 128), narrow = tiles(256, 128), wide = tiles(256, 256);
+  if (epi == kGroupScale) return small >= 256 ? kNarrow : kNoLarge;
+  if (epi == kTokenGroup) return rounds(narrow) * 29.5 < rounds(small) * 16.6 ? kNarrow : kNoLarge;
+  if (small <= 256) return kNoLarge;
+  auto cost = [&](long t) { return 0.5 * (rounds(t) + t / 256.0); };
+  return cost(wide) <= 0.62 * cost(narrow) ? kWide : kNarrow;
+}
+// 128 x 128 tiles below that, down to 192 of them (with more than 64 rows; group scales on both sides: 224), else 64 x 64
+// (512 x 6144: 19 against 21 with row scales, 22 against 22 with token scales, 33 against 26 with group scales)
+int small_choice(const GemmArgs& a, int epi, long columns) {
+  const int forced = g_tune_tile.load(std::memory_order_relaxed);
+  if (forced) return forced == 64 ? 64 : 128;
+  const long small = (long)((a.M + 127) / 128) * ((columns + 127) / 128);
+  return a.M > 64 && small >= (epi == kGroupScale ? 224 : 192) ? 128 : 64;
+}
+
 template <int EPI>
 int launch_f6_grouped(const GemmArgs& a, hipStream_t stream) {
   const int n_all = total_n_f6(a);
-  auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n_all + bn - 1) / bn); };
-  int tile = tiles(128, 128) >= 200 ? 128 : 64;
-  const int forced = g_tune_tile.load(std::memory_order_relaxed);
-  if (forced == 128 || forced == 64) tile = forced;
-  if (tile == 128) return launch_f6<128, 128, 64, 64, 3, EPI>(a, stream);
+  if (large_choice(a, EPI, n_all)) return f6l::launch_large_group(a, EPI == kTokenGroup, a.R ? f6l::kResidual : f6l::kPlain, stream);
+  if (small_choice(a, EPI, n_all) == 128) return launch_f6<128, 128, 64, 64, 3, EPI>(a, stream);
   return launch_f6<64, 64, 32, 32, 3, EPI>(a, stream);
 }
 
-// SwiGLU launches: tiles by the number of 64-channel output tiles (128 weight rows of [gate | up] each)
+// SwiGLU launches: the weight rows are those of gate and up together
 template <int EPI>
 int launch_f6_swiglu(const GemmArgs& a, hipStream_t stream) {
-  auto tiles = [&](int bm, int bnc) { return (long)((a.M + bm - 1) / bm) * ((a.N + bnc - 1) / bnc); };
-  int tile = tiles(128, 64) >= 200 ? 128 : 64;
-  const int forced = g_tune_tile.load(std::memory_order_relaxed);
-  // (the eight-wave tile of launch_f6_by_shape only when forced: with one workgroup per compute unit nothing overlaps
-  // this epilogue's exchange and stores -- 155.5 against 150.0 us on weights from HBM, 152 against 133 us on cached ones)
-  if constexpr (EPI == kRowScale)
-    if (forced == 256) tile = 256;
-  if (forced == 128 || forced == 64) tile = forced;
-  if constexpr (EPI == kRowScale)
-    if (tile == 256) return launch_f6<256, 128, 64, 64, 4, EPI, true>(a, stream);
-  if (tile == 128) return launch_f6<128, 128, 64, 64, 3, EPI, true>(a, stream);
+  const long columns = 2 * (long)a.N;
+  if (const LargeTile large = large_choice(a, EPI, columns)) {
+    if constexpr (EPI == kRowScale) return f6l::launch_large_row(a, large == kWide, f6l::kSwiglu, stream);
+    else return f6l::launch_large_group(a, EPI == kTokenGroup, f6l::kSwiglu, stream);
+  }
+  if (small_choice(a, EPI, columns) == 128) return launch_f6<128, 128, 64, 64, 3, EPI, true>(a, stream);
   return launch_f6<64, 64, 32, 32, 3, EPI, true>(a, stream);
 }
 
-// flh_gemm_set_tuning overrides the tile choice (256 / 128 / 64; the hook through which the tests cover every variant)
 template <int EPI>
 int launch_f6_by_shape(const GemmArgs& a, hipStream_t stream) {
-  const int env_tile = g_tune_tile.load(std::memory_order_relaxed);
   const int n_all = total_n_f6(a);
-  auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n_all + bn - 1) / bn); };
-  // Measured at M = 2048 / 4096 on the Llama shapes.  With the same weights launched back to back (they then sit in the
-  // last-level cache) two 128 x 128 workgroups per compute unit beat one 256 x 128 workgroup of eight waves by 2-6 %;
-  // with weights that come from HBM -- every launch of a model, whose layers' weights do not fit that cache -- the
-  // eight-wave tile with its four-stage ring is 12-16 % faster at every shape (gate + up 148 against 170 us, q + k + v
-  // 79 against 90, down 61 against 72, o 27.5 against 31.5): it requests three quarters of the operand bytes per unit
-  // of matrix work and a step further ahead.  It is taken as soon as there is one such tile per compute unit.
-  int tile = tiles(256, 128) >= 256 ? 256 : tiles(128, 128) >= 256 ? 128 : 64;
-  if (env_tile == 256 || env_tile == 128 || env_tile == 64) tile = env_tile;
-  if (tile == 256) return launch_f6<256, 128, 64, 64, 4, EPI>(a, stream);
-  if (tile == 128) return launch_f6<128, 128, 64, 64, 3, EPI>(a, stream);
+  if constexpr (EPI == kRowScale)
+    if (const LargeTile large = large_choice(a, EPI, n_all))
+      return f6l::launch_large_row(a, large == kWide, a.R ? f6l::kResidual : f6l::kPlain, stream);
+  if (small_choice(a, EPI, n_all) == 128) return launch_f6<128, 128, 64, 64, 3, EPI>(a, stream);
   return launch_f6<64, 64, 32, 32, 3, EPI>(a, stream);
 }
 
@@ -868,14 +903,12 @@ extern "C" int flh_gemm_f6_qkv_rope_o16(const uint8_t* A6, const flh_half* a_sca
   g.rope_T = (int)T;
   g.rope_max_len = (int)max_len;
   g.rope_hkv = (int)Hkv;
-  // 128 x 128 tiles (a tile column = one head)
-  if (rows_only) {
-    const int forced = g_tune_tile.load(std::memory_order_relaxed);
-    const long tiles256 = (long)((g.M + 255) / 256) * ((total_n_f6(g) + 127) / 128);
-    if (forced == 256 || (forced == 0 && tiles256 >= 256))
-      return launch_f6<256, 128, 64, 64, 4, kRowScale, false, true>(g, (hipStream_t)stream);
-    return launch_f6<128, 128, 64, 64, 3, kRowScale, false, true>(g, (hipStream_t)stream);
+  if (const LargeTile large = large_choice(g, rows_only ? kRowScale : a_cols == 1 ? kTokenGroup : kGroupScale, total_n_f6(g))) {
+    if (rows_only) return f6l::launch_large_row(g, large == kWide, f6l::kRope, (hipStream_t)stream);
+    return f6l::launch_large_group(g, a_cols == 1, f6l::kRope, (hipStream_t)stream);
   }
+  // 128 x 128 tiles (a tile column = one head)
+  if (rows_only) return launch_f6<128, 128, 64, 64, 3, kRowScale, false, true>(g, (hipStream_t)stream);
   if (a_cols == 1) return launch_f6<128, 128, 64, 64, 3, kTokenGroup, false, true>(g, (hipStream_t)stream);
   return launch_f6<128, 128, 64, 64, 3, kGroupScale, false, true>(g, (hipStream_t)stream);
 }
