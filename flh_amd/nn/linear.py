@@ -32,13 +32,14 @@ class LinearFLH(torch.nn.Module):
             self.register_buffer("bias", torch.zeros(out_features, dtype=dtype, device=device))
         else:
             self.bias = None
-        # Opt-in (extension): run prefill-sized calls on the 6-bit matrix instruction (same bits, no unpack in the loop).
-        # The layer then holds its weights a second time, re-encoded at 6 bits per code: 0.75 byte per weight on top of the
-        # 0.5 of `w_packed`, i.e. 2.5 x the weight memory.  False (default): never.  True: every call of at least
-        # `six_bit_min_rows` rows.  "auto" (or None): where it is faster even with the pass that re-encodes the activations
-        # -- weights with a scale per group of 128.  `prepare_six_bit()` builds the second encoding at once (a loader calls
-        # it); otherwise it is built on first use.  It is rebuilt whenever `w_packed` has been written to or replaced
-        # (in-place copies, load_state_dict, .to(device)): keyed on the buffer's storage address and version counter.
+        # Prefill-sized calls run on the 6-bit matrix instruction where that is faster (extension; same bits, no unpack in the
+        # loop).  Its operands are re-encoded at 6 bits per code, 0.75 byte per weight next to the 0.5 of `w_packed`.
+        # False (default): nothing is kept; a call of at least TRANSIENT_ROWS rows encodes its weights into a buffer that
+        # goes back with the call.  True: the layer keeps the encoding (2.5 x the weight memory) and every call of at
+        # least `six_bit_min_rows` rows uses it.  "auto" (or None): kept for weights with a scale per group of 128.
+        # `prepare_six_bit()` builds the kept encoding at once (a loader calls it); otherwise it is built on first use.  It
+        # is rebuilt whenever `w_packed` has been written to or replaced (in-place copies, load_state_dict, .to(device)):
+        # keyed on the buffer's storage address and version counter.
         self.six_bit = False
         self.six_bit_min_rows = 256
         self._w6 = None
@@ -47,13 +48,27 @@ class LinearFLH(torch.nn.Module):
     def drop_six_bit_weights(self):
         self._w6 = self._w6_key = None
 
+    # Rows from which a call is faster on the 6-bit instruction although it encodes the weights first: (one scale per
+    # channel, a scale per group of 128).  At 3000 rows of 4096 x 11008 the pass takes 12 us and the GEMM 94 instead of 126
+    # (2048 rows: 70 instead of 85, even with the pass and its launch); with a scale per group at 700 rows 12 us and 47
+    # (token scales) or 57 (group scales) instead of 68 or 80 (512 rows of 4096 x 4096: 6 and 16 or 19 against 22 or 25).
+    TRANSIENT_ROWS = (2560, 640)
+
+    def _keeps_six_bit(self, grouped):
+        return self.six_bit is True or (self.six_bit is not False and grouped)
+
+    def _six_bit_rows(self, grouped):
+        return self.six_bit_min_rows if self._keeps_six_bit(grouped) else self.TRANSIENT_ROWS[1 if grouped else 0]
+
     def prepare_six_bit(self):
-        """Build the 6-bit encoding of the weights now if this layer's setting can make use of it (at load time, rather
-        than inside the first long call)."""
-        if self.wants_six_bit(self.six_bit_min_rows):
+        """Build the 6-bit encoding of the weights now if this layer's setting keeps one (at load time, rather than inside
+        the first long call)."""
+        if self.wants_six_bit(self.six_bit_min_rows) and self._keeps_six_bit(self.w_scale.view(self.out_features, -1).size(1) > 1):
             self._six_bit_weights()
 
     def _six_bit_weights(self):
+        if not self._keeps_six_bit(self.w_scale.view(self.out_features, -1).size(1) > 1):
+            return _pkg._CUDA.encode_f6(self.w_packed.view(self.out_features, self.in_features // 2))
         key = (self.w_packed.data_ptr(), self.w_packed._version, self.w_packed.device)
         if self._w6 is None or self._w6_key != key:
             self._w6 = _pkg._CUDA.encode_f6(self.w_packed.view(self.out_features, self.in_features // 2))
@@ -63,20 +78,20 @@ class LinearFLH(torch.nn.Module):
     def wants_six_bit(self, n_rows):
         """Whether a call with `n_rows` per-token-quantised rows takes the 6-bit matrix instruction (a producer can then
         write the activations in that format directly, rotate_and_quantize_f6)."""
-        if self.six_bit is False or n_rows < self.six_bit_min_rows or self.in_features % 128 or not self.w_packed.is_cuda:
+        if (n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS[1]) or self.in_features % 128 or not self.w_packed.is_cuda:
             return False
         cols = self.w_scale.view(self.out_features, -1).size(1)
-        if cols == 1:
-            return self.six_bit is True
-        return cols == self.in_features // 128 and self.weight_group_size == 128
+        if cols != 1 and not (cols == self.in_features // 128 and self.weight_group_size == 128):
+            return False
+        return n_rows >= self._six_bit_rows(cols != 1)
 
     def _six_bit_applies(self, rows, a_scale, w_scale, group):
-        if self.six_bit is False or not (rows.is_cuda and rows.size(0) >= self.six_bit_min_rows
-                                         and self.in_features % 128 == 0):
+        n = rows.size(0)
+        if (n < self.six_bit_min_rows and n < self.TRANSIENT_ROWS[1]) or not rows.is_cuda or self.in_features % 128:
             return False
         per_row = a_scale.size(1) == 1 and w_scale.size(1) == 1
         grouped = group == 128 and w_scale.size(1) == self.in_features // 128 and a_scale.size(1) in (1, w_scale.size(1))
-        return grouped or (per_row and self.six_bit is True)
+        return (grouped or per_row) and n >= self._six_bit_rows(not per_row)
 
     # ------------------------------------------------------------------ kernels
     def forward(self, x, a_scale=None, a_zero=None, x_is_packed=False, is_symmetric=None, residual=None):
@@ -190,6 +205,11 @@ class LinearFLH(torch.nn.Module):
                    and (w_scale.size(1) == 1 or (group == 128 and w_scale.size(1) == 32)))
         if fusable:
             y = ops.rotate_quantize_gemm_i4(rows, w, w_scale)
+        elif rows.size(0) >= self.TRANSIENT_ROWS[1] and self.in_features in (4096, 11008, 14336) and self.wants_six_bit(rows.size(0)) and (
+                hadamard in (True, "fast") or (hadamard == "exact" and self.in_features == 4096)):
+            # long calls: the quantiser writes the 6-bit operand format
+            q, s = ops.rotate_and_quantize_f6(rows, hadamard=hadamard)
+            return self.forward(q, s, x_is_packed=True).view(*lead, self.out_features)
         else:
             q, s = ops.rotate_and_quantize_i4(rows, hadamard=hadamard)
             y = ops.gemm_i4_dequant(q, w, s, w_scale, group)
