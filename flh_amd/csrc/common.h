@@ -80,7 +80,12 @@ __device__ __forceinline__ void load_to_lds16(const void* gptr, unsigned lds_bas
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
 
-// the same with a wave-uniform base address in scalar registers plus a 32-bit per-lane offset
+// 4 bytes per lane: lane i writes lds_base + 4 * i
+__device__ __forceinline__ void load_to_lds4(const void* gptr, unsigned lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
+}
+
+// load_to_lds16 with a wave-uniform base address in scalar registers plus a 32-bit per-lane offset
 __device__ __forceinline__ void load_to_lds16(const void* sbase, unsigned voffset, unsigned lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(sbase) : "memory", "m0");
 }

@@ -74,14 +74,6 @@ __device__ __forceinline__ T* wave_uniform(T* q) {
               (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v));
 }
 
-// fp16(fp16(x cos) + fp16(rotate_half(x) sin)) of one channel pair (c, c + 64), as rope_cache.hip rounds it
-__device__ __forceinline__ void rope_pair(_Float16& x1, _Float16& x2, _Float16 c1, _Float16 c2, _Float16 s1, _Float16 s2) {
-  const _Float16 a1 = (_Float16)round_here((float)x1 * (float)c1), r1 = (_Float16)round_here(-1.f * (float)x2 * (float)s1);
-  const _Float16 a2 = (_Float16)round_here((float)x2 * (float)c2), r2 = (_Float16)round_here(1.f * (float)x1 * (float)s2);
-  x1 = (_Float16)round_here((float)a1 + (float)r1);
-  x2 = (_Float16)round_here((float)a2 + (float)r2);
-}
-
 // The last step of the outputs: ROWS rows of 128 fp16 values, staged in LDS by this wave (kPitch bytes apart, the first
 // row being row m_first of the launch), leave as whole row segments.  wcol: which 128 of the tile's weight rows the values belong to.
 template <int ROWS, int OUT>

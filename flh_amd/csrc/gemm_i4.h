@@ -45,9 +45,23 @@ struct GemmArgs {
   const __half* R;
 };
 
+// fp16(fp16(x cos) + fp16(rotate_half(x) sin)) of one channel pair (c, c + 64), as rope_cache.hip rounds it
+__device__ __forceinline__ void rope_pair(_Float16& x1, _Float16& x2, _Float16 c1, _Float16 c2, _Float16 s1, _Float16 s2) {
+  const _Float16 a1 = (_Float16)round_here((float)x1 * (float)c1), r1 = (_Float16)round_here(-1.f * (float)x2 * (float)s1);
+  const _Float16 a2 = (_Float16)round_here((float)x2 * (float)c2), r2 = (_Float16)round_here(1.f * (float)x1 * (float)s2);
+  x1 = (_Float16)round_here((float)a1 + (float)r1);
+  x2 = (_Float16)round_here((float)a2 + (float)r2);
+}
+
 // Small-M (decode) kernels: weight-streaming, split over K inside a workgroup.
 constexpr int kDecodeMaxM = 64;
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group);
 int gemm_decode_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
+
+// Between decoding and prefill: small tiles over the whole of K (gemm_i4_stream.hip).
+bool gemm_stream_supports(const GemmArgs& a, int epi, int group);
+int gemm_stream_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
+bool gemm_stream_rope_supports(const GemmArgs& a, int epi);
+int gemm_stream_rope_dispatch(const GemmArgs& a, hipStream_t stream);
 
 }  // namespace flh

@@ -755,6 +755,7 @@ int launch_grouped(const GemmArgs& a, int group, bool small, hipStream_t stream)
 
 int gemm_dispatch(GemmArgs a, int epi, int group, hipStream_t stream) {
   if (a.M == 0 || a.N == 0) return FLH_OK;
+  if (gemm_stream_supports(a, epi, group)) return gemm_stream_dispatch(a, epi, stream);
   if (gemm_decode_supports(a, epi, group)) return gemm_decode_dispatch(a, epi, stream);
   switch (epi) {
     case kRowScale: return launch_by_shape<kRowScale>(a, stream);
@@ -788,9 +789,10 @@ int launch_swiglu(const GemmArgs& a, int group, hipStream_t stream) {
   }
 }
 
-// q / k / v launches with the rotary embedding and the cache write in the epilogue: 128-column tiles only
+// q / k / v launches with the rotary embedding and the cache write in the epilogue: 128-column tiles, or the small ones
 template <int EPI>
 int launch_qkv_rope(const GemmArgs& a, hipStream_t stream) {
+  if (gemm_stream_rope_supports(a, EPI)) return gemm_stream_rope_dispatch(a, stream);
   const long tiles256 = (long)((a.M + 255) / 256) * (total_n(a) / 128), tiles128 = (long)((a.M + 127) / 128) * (total_n(a) / 128);
   int tile = tiles256 > 256 && !prefers_small_tiles(tiles256, tiles128) ? 256 : 128;
   const int forced = g_tune_tile.load(std::memory_order_relaxed);

@@ -1,0 +1,402 @@
+// int4 x int4 GEMM + dequant for launches between decoding and prefill: up to a few hundred tokens, and a handful of tokens
+// against many output channels.  Same arithmetic as gemm_i4.hip (codes x 16 as int8 on the matrix cores, exact int32 sums per
+// group, one fused multiply-add per group in ascending order, identical epilogue roundings): same bits.
+//
+// Why.  The 64 x 64 tiles of gemm_i4.hip leave most of the chip idle here (4096 channels, 45 tokens: 64 workgroups), each
+// with one latency per 128 codes of K; a K split (gemm_i4_decode.hip) needs every group's sums of a tile in LDS, which ends
+// at 16 tokens.  Here a workgroup owns a small tile (BM x BN below) for the whole of K, so there is one per compute unit from
+// 32 x 4096 outputs on, and each wave folds its own 16 x 16 tiles in order.  Operands come through a ring of LDS stages of
+// four groups (256 bytes of every row) filled by direct-to-LDS loads two stages ahead; fragments, and the scales from a
+// table in LDS, are read into registers one stage ahead of the products.  (Fragments straight from memory reach 16 bytes
+// per clock and compute unit, sixteen half lines per load: 17-25 us where this kernel takes 11-17.)
+//
+// What bounds it: the vector ALU.  A 16 x 16 x 128 product is 32 clocks of MFMA next to 24 instructions of unpacking (12 more
+// per further tile of the wave) and 12 of folding (8 with one scale per token), and the one or two waves of a SIMD overlap
+// little.  Deeper rings (6 stages) changed nothing up to one workgroup per compute unit and cost the second resident beyond.
+//
+// us per launch, weights from HBM, group scales on both sides, before -> after (K x N):
+//   17-64 tokens: 4096 x 4096 21.1 -> 8.2, 11008 x 4096 50 -> 17, 14336 x 4096 68 -> 21, 4096 x 28672 40 -> 20 (32), 31 (64)
+//   128: 4096 x 4096 21.7 -> 10.9, 4096 x 6144 22.2 -> 14.3;  256: 4096 x 4096 21.8 -> 15.7;  512: 4096 x 1024 18.3 -> 10.3
+//   16 tokens: 4096 x 28672 22.5 -> 15.7, 4096 x 14336 13.9 -> 9.8 (5 and 3.7 TB/s of weights)
+// and with one scale per row: 64 tokens 4096 x 14336 28.4 -> 13, 4096 x 4096 8.3 -> 6.5; 128: 11008 x 4096 25 -> 18.
+#include "gemm_i4.h"
+
+namespace flh {
+namespace {
+
+// What a launch does with its results: rows of D, or q / k / v with the rotary embedding (two tiles half a head apart)
+enum StreamOut { kStreamPlain = 0, kStreamRope = 1 };
+
+constexpr int kStageGroups = 4;                    // groups of 128 codes per stage: 256 bytes of every row
+constexpr int kRowBytes = kStageGroups * 64;
+constexpr int kStreamMaxGroups = 128;              // scales of a row that fit beside the ring (K <= 16384)
+
+// product of element H (0 / 1) of two fp16 pairs, exact in float32
+template <int H>
+__device__ __forceinline__ float mul_halves(unsigned a, unsigned b) {
+  float d;
+  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(d) : "v"(a), "v"(b));
+  else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+}
+// fma(v, element H of the fp16 pair s, acc)
+template <int H>
+__device__ __forceinline__ float fma_half(float v, unsigned s, float acc) {
+  float d;
+  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(v), "v"(s), "v"(acc));
+  else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(v), "v"(s), "v"(acc));
+  return d;
+}
+
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) uint8_t lds_byte;
+template <typename T>
+__device__ __forceinline__ T from_lds(const lds_byte* q) { return *(const __attribute__((address_space(3))) T*)q; }
+
+template <int TN>
+struct StageRegs {                                 // a wave's operands of one stage
+  v4i a[kStageGroups], b[TN][kStageGroups];
+  v2u sa, sb[TN][4];                               // scales of the four groups: the lane's token, its four channels
+};
+
+template <int WM, int WN, int TN, int S, int EPI, int OUT>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const GemmArgs p) {
+  constexpr bool GROUPED = EPI != kRowScale;
+  constexpr int WAVES = WM * WN, RA = 16 * WM, RB = 16 * TN * WN, ROWS = RA + RB;
+  constexpr int STAGE = ROWS * kRowBytes;
+  constexpr int NA = RA / 4 / WAVES, NB = RB / 4 / WAVES, NI = NA + NB;   // 1 KiB load instructions per wave and stage
+  constexpr int SROWS = EPI == kGroupScale ? ROWS : RB;   // rows of the scale table: tokens, then channels
+  static_assert(RA / 4 % WAVES == 0 && RB / 4 % WAVES == 0 && (S - 2) * NI < 64, "loads per stage");
+  static_assert(OUT == kStreamPlain || (TN == 2 && WN == 1), "partner tiles");
+  extern __shared__ __align__(16) uint8_t lds[];
+  lds_byte* ring = (lds_byte*)lds;                 // (typed: a generic pointer would make the reads wait for all loads)
+  lds_byte* scales = ring + S * STAGE;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, c = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  const unsigned L = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int bn = L / p.tiles_m, bm = L % p.tiles_m;       // the blocks of one weight stripe sit next to each other on a die
+
+  const uint8_t* B = p.B;
+  const __half* Bs = p.Bs;
+  void* Dp = p.D;
+  int N = p.N, seg = 0, t = bn;
+  for (int s = 1; s < p.n_seg; ++s)
+    if (bn >= p.seg_tile0[s]) B = p.seg_B[s], Bs = p.seg_Bs[s], Dp = p.seg_D[s], N = p.seg_N[s], seg = s, t = bn - p.seg_tile0[s];
+  const int Kb = p.K >> 1, KT = p.K >> 7;
+  const int stages = (KT + kStageGroups - 1) / kStageGroups;
+  const int m0 = bm * RA;
+  // first channel of the block's tile j
+  auto first = [&](int j) {
+    return OUT == kStreamPlain ? (t * (TN * WN) + j) * 16 : (t >> 2) * 128 + (t & 3) * 16 + j * 64;
+  };
+  auto b_row = [&](int row) { return min(first(row >> 4) + (row & 15), N - 1); };      // row of B behind LDS row RA + row
+
+  auto first_group = [&](int s) { return min(s * kStageGroups, KT - kStageGroups); };   // the last stage ends with the row
+
+  // scales first, as their rows are: [row][KT / 2 pairs, an odd number of slots] in LDS, every wave a share of them
+  const int pitch = (KT >> 1) | 1;
+  if constexpr (GROUPED) {
+    const float inv = 1.0f / (float)pitch;
+    const int total = SROWS * pitch;
+    for (int f0 = wave * 64; f0 < total; f0 += WAVES * 64) {
+      const int f = min(f0 + lane, total - 1);
+      int row = (int)((float)f * inv);             // f < 2^14: off by one at most
+      row += (f >= (row + 1) * pitch ? 1 : 0) - (f < row * pitch ? 1 : 0);
+      const int pair = min(f - row * pitch, (KT >> 1) - 1), chan = row - (SROWS - RB);
+      const __half* q = chan < 0 ? p.As + (size_t)min(m0 + row, p.M - 1) * KT
+                                 : Bs + (size_t)b_row(chan) * KT;
+      load_to_lds4(q + 2 * pair, (unsigned)(uintptr_t)scales + f0 * 4);
+    }
+  }
+
+  // operands: a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16)
+  const int lrow = lane >> 4;
+  const uint8_t* src[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (i < NA) {
+      const int row = (wave * NA + i) * 4 + lrow;
+      src[i] = p.A + (size_t)min(m0 + row, p.M - 1) * Kb + ((lane & 15) ^ (row & 15)) * 16;
+    } else {
+      const int row = (wave * NB + i - NA) * 4 + lrow;
+      src[i] = B + (size_t)b_row(row) * Kb + ((lane & 15) ^ (row & 15)) * 16;
+    }
+  }
+  const unsigned base = (unsigned)(uintptr_t)ring;
+  auto request = [&](int s, int slot) {            // slot: byte offset of the ring slot
+    const size_t off = (size_t)first_group(s) * 64;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int row = i < NA ? (wave * NA + i) * 4 : RA + (wave * NB + i - NA) * 4;
+      load_to_lds16(src[i] + off, base + slot + row * kRowBytes);
+    }
+  };
+  int chunk[kStageGroups];                         // of the lane's row
+#pragma unroll
+  for (int g = 0; g < kStageGroups; ++g) chunk[g] = r * kRowBytes + ((g * 4 + c) ^ r) * 16;
+  auto read = [&](int s, int slot, StageRegs<TN>& q) {
+    const lds_byte* st = ring + slot;
+#pragma unroll
+    for (int g = 0; g < kStageGroups; ++g) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) q.b[j][g] = from_lds<v4i>(st + chunk[g] + (RA + (wn * TN + j) * 16) * kRowBytes);
+      q.a[g] = from_lds<v4i>(st + chunk[g] + wm * 16 * kRowBytes);
+    }
+    if constexpr (GROUPED) {
+      const int at = first_group(s) >> 1;
+      auto two = [&](int row) {
+        const __attribute__((address_space(3))) unsigned* e = (const __attribute__((address_space(3))) unsigned*)scales + row * pitch + at;
+        return v2u{e[0], e[1]};
+      };
+      if constexpr (EPI == kGroupScale) q.sa = two(wm * 16 + r);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q.sb[j][e] = two(SROWS - RB + (wn * TN + j) * 16 + 4 * c + e);
+    }
+  };
+  v4i acc[TN];
+  float out[TN][4];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    acc[j] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[j][e] = 0.f;
+  }
+  auto product = [&](const v4i& a, const v4i& b, v4i d) {
+    v4i alo, ahi, blo, bhi;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      alo[e] = (a[e] << 4) & (int)0xF0F0F0F0, ahi[e] = a[e] & (int)0xF0F0F0F0;
+      blo[e] = (b[e] << 4) & (int)0xF0F0F0F0, bhi[e] = b[e] & (int)0xF0F0F0F0;
+    }
+    d = __builtin_amdgcn_mfma_i32_16x16x64_i8(blo, alo, d, 0, 0, 0);
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(bhi, ahi, d, 0, 0, 0);
+  };
+  auto fold = [&](auto G, int j, const v4i& d, const StageRegs<TN>& q) {
+    constexpr int g = decltype(G)::value, w = g / 2, h = g % 2;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float v = (float)d[e];                 // 256 x the exact sum
+      const unsigned sb = q.sb[j][e][w];
+      if constexpr (EPI == kGroupScale) out[j][e] = __builtin_fmaf(v, mul_halves<h>(q.sa[w], sb), out[j][e]);
+      else out[j][e] = fma_half<h>(v, sb, out[j][e]);
+    }
+  };
+  auto multiply = [&](const StageRegs<TN>& q) {    // a whole stage: all products, then their folds in ascending order
+    if constexpr (GROUPED) {
+      v4i d[kStageGroups][TN];
+#pragma unroll
+      for (int g = 0; g < kStageGroups; ++g)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) d[g][j] = product(q.a[g], q.b[j][g], v4i{0, 0, 0, 0});
+      static_for<kStageGroups>([&](auto G) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fold(G, j, d[decltype(G)::value][j], q);
+      });
+    } else {
+#pragma unroll
+      for (int g = 0; g < kStageGroups; ++g)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[j] = product(q.a[g], q.b[j][g], acc[j]);
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < stages) request(s, s * STAGE);
+  const bool live = m0 + wm * 16 < p.M;
+  // every wave's loads of the oldest stage but `newer` are in LDS, every wave has its last stage in registers
+  auto arrive = [&](bool steady) {
+    if (steady) wait_vmcnt<(S - 2) * NI>();
+    else wait_vmcnt<0>();
+    wait_lgkmcnt0();
+    barrier_no_fence();
+  };
+  StageRegs<TN> q0, q1;
+  int slot = 0;                                    // of stage s
+  auto step = [&](int s, StageRegs<TN>& cur, StageRegs<TN>& next) {     // s + 1 < stages
+    arrive(s + S - 1 < stages);
+    if (s + S < stages) request(s + S, slot);
+    slot = slot == (S - 1) * STAGE ? 0 : slot + STAGE;
+    if (live) {
+      read(s + 1, slot, next);
+      __builtin_amdgcn_sched_barrier(0);           // (the reads have the products' time to arrive)
+      multiply(cur);
+    }
+  };
+  auto last = [&](const StageRegs<TN>& q) {
+    if (!live) return;
+    const int skip = (stages - 1) * kStageGroups - first_group(stages - 1);   // groups that the stage before has done
+    static_for<kStageGroups>([&](auto G) {
+      constexpr int g = decltype(G)::value;
+      if (g < skip) return;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if constexpr (GROUPED) fold(G, j, product(q.a[g], q.b[j][g], v4i{0, 0, 0, 0}), q);
+        else acc[j] = product(q.a[g], q.b[j][g], acc[j]);
+      }
+    });
+  };
+  arrive(stages >= S);                             // stage 0; slot S - 1 is free
+  if (S - 1 < stages) request(S - 1, (S - 1) * STAGE);
+  if (live) read(0, 0, q0);
+  int s = 0;
+  for (; s + 2 < stages; s += 2) {
+    step(s, q0, q1);
+    step(s + 1, q1, q0);
+  }
+  if (s + 1 < stages) {
+    step(s, q0, q1);
+    last(q1);
+  } else {
+    last(q0);
+  }
+
+  // lane: token r, channels 4 c + e of each tile
+  const int m = m0 + wm * 16 + r;
+  if (m >= p.M) return;
+  _Float16 y[TN][4];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v;
+      if constexpr (EPI == kGroupScale) v = out[j][e] * 0.00390625f;
+      else if constexpr (EPI == kTokenGroup) v = round_here(out[j][e] * 0.00390625f) * __half2float(p.As[m]);
+      else {
+        const float s_a = __half2float(p.As[m]), s_b = __half2float(Bs[min(first(wn * TN + j) + 4 * c + e, N - 1)]) * 0.00390625f;
+        v = (float)acc[j][e] * (s_a * s_b);
+      }
+      y[j][e] = (_Float16)round_here(v);
+    }
+  if constexpr (OUT == kStreamRope) {
+    const int head = t >> 2, ch = (t & 3) * 16 + 4 * c;
+    if (head * 128 >= N) return;
+    const int b = m / p.rope_T, tok = m - b * p.rope_T;
+    __half* dst = (__half*)Dp + (size_t)m * N + head * 128 + ch;
+    if (seg > 0) {
+      const long long slot = p.rope_pos[tok];
+      if (slot < 0 || slot >= (long long)p.rope_max_len) return;
+      dst = (__half*)Dp + (((size_t)b * p.rope_hkv + head) * p.rope_max_len + (size_t)slot) * 128 + ch;
+    }
+    if (seg < 2) {
+      const __half *ct = p.rope_cos + (size_t)tok * 128 + ch, *st = p.rope_sin + (size_t)tok * 128 + ch;
+      const h4 c1 = *(const h4*)ct, c2 = *(const h4*)(ct + 64), s1 = *(const h4*)st, s2 = *(const h4*)(st + 64);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rope_pair(y[0][e], y[1][e], c1[e], c2[e], s1[e], s2[e]);
+    }
+    *(h4*)dst = h4{y[0][0], y[0][1], y[0][2], y[0][3]};
+    *(h4*)(dst + 64) = h4{y[1][0], y[1][1], y[1][2], y[1][3]};
+  } else {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = first(wn * TN + j) + 4 * c;
+      const size_t at = (size_t)m * N + n;
+      if (N % 4 == 0) {
+        if (n >= N) continue;
+        h4 v = {y[j][0], y[j][1], y[j][2], y[j][3]};
+        if (p.R) v = v + *(const h4*)((const _Float16*)p.R + at);   // (R may be D: read before the store)
+        *(h4*)((_Float16*)Dp + at) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) ((_Float16*)Dp)[at + e] = p.R ? y[j][e] + ((const _Float16*)p.R)[at + e] : y[j][e];
+      }
+    }
+  }
+}
+
+template <int WM, int WN, int TN, int S, int EPI, int OUT>
+int launch_stream(GemmArgs a, hipStream_t stream) {
+  constexpr int RA = 16 * WM, RB = 16 * TN * WN, BN = RB;
+  a.tiles_m = (a.M + RA - 1) / RA;
+  auto tiles = [&](int n) { return OUT == kStreamRope ? (n + 127) / 128 * 4 : (n + BN - 1) / BN; };
+  a.tiles_n = tiles(a.N);
+  for (int s = 1; s < a.n_seg; ++s) {
+    a.seg_tile0[s] = a.tiles_n;
+    a.tiles_n += tiles(a.seg_N[s]);
+  }
+  constexpr size_t ring = (size_t)S * (RA + RB) * kRowBytes;
+    // (rounded up to whole load instructions)
+  auto table = [](int kt) { return EPI == kRowScale ? 0 : ((size_t)((kt / 2) | 1) * (EPI == kGroupScale ? RA + RB : RB) * 4 + 255) / 256 * 256; };
+  auto kern = gemm_i4_stream_kernel<WM, WN, TN, S, EPI, OUT>;
+  static LdsGrant grant;                               // per instantiation; sized for the longest rows it takes
+  if (int rc = reserve_lds((const void*)kern, ring + table(kStreamMaxGroups), grant, "gemm (stream)")) return rc;
+  hipLaunchKernelGGL(kern, dim3(a.tiles_m * a.tiles_n), dim3(64 * WM * WN), ring + table(a.K >> 7), stream, a);
+  return check_launch("gemm_i4_stream");
+}
+
+long stream_columns(const GemmArgs& a) {
+  long n = a.N;
+  for (int s = 1; s < a.n_seg; ++s) n += a.seg_N[s];
+  return n;
+}
+
+// Tiles, tokens x channels: 16 x 64 for up to 16 tokens, else 32 x 32, or 64 x 32 (half the weight traffic, a fifth less
+// vector work) where two of its workgroups per compute unit remain and the tokens fill it as well as the smaller tile (256
+// tokens: 4096 x 4096 15.7 against 18.1 us; 128: 4096 x 6144, 1.5 of its workgroups, 15.7 against 14.3).
+template <int EPI>
+int launch_stream_by_shape(const GemmArgs& a, hipStream_t stream) {
+  if (a.M <= 16) return launch_stream<1, 4, 1, 3, EPI, kStreamPlain>(a, stream);
+  const long large = (long)((a.M + 63) / 64) * ((stream_columns(a) + 31) / 32);
+  if (large >= 512 && (a.M + 31) / 32 % 2 == 0) return launch_stream<4, 1, 2, 3, EPI, kStreamPlain>(a, stream);
+  return launch_stream<2, 2, 1, 3, EPI, kStreamPlain>(a, stream);
+}
+
+// what the kernel can take: whole stages, and group scales that dword loads can fetch two at a time
+bool stream_takes(const GemmArgs& a, int epi, int group) {
+  const int kt = a.K >> 7;
+  if (epi == kInt32 || kt < kStageGroups) return false;
+  if (epi == kRowScale) return true;
+  auto off4 = [](const void* q) { return ((uintptr_t)q & 3) != 0; };
+  if (group != 128 || a.b_cols == 1 || kt % 2 || kt > kStreamMaxGroups || off4(a.Bs) || (a.a_cols > 1 && off4(a.As))) return false;
+  for (int s = 1; s < a.n_seg; ++s)
+    if (off4(a.seg_Bs[s])) return false;
+  return true;
+}
+
+}  // namespace
+
+// Which launches are faster here than on the kernels on either side.  us, this kernel against the other (K = 4096 unless
+// stated; "large" counts 64 x 32 tiles):
+//  * up to 16 tokens, against the K split of the decode kernel: from 224 workgroups of 64 channels on (one token x 28672
+//    channels 15.4 against 17.0, x 14336 9.7 against 10.0), with five or more tokens from 172 (16 x 11008 9.4 against 11.4;
+//    one token x 12288 9.5 against 8.9, 16 x 6144 8.3 against 8.6).
+//  * 17 .. 64 tokens: always, but for one scale per row on at most 128 blocks of 32 channels, where the decode kernel takes 32
+//    (32 x 4096 6.0 against 6.3; 64 x 4096 8.3 against 6.5).
+//  * more, group-scaled weights, against 64 x 64 and 128 x 128 tiles: up to 640 large tiles, 768 if K is short (128 x 12288,
+//    768: 24 against 27; 192 x 12288, 1152: 35 against 33; 384 x 4096, 768: 22.3 against 25.1, but 64 against 60 for K = 11008).
+//  * more, one scale per row, against the K-split tiles: up to 384 (128 x 6144 11.1 against 12.1; 256 x 4096, 512: 12.0
+//    against 11.9; 128 x 12288, 768: 17.7 against 17.0).
+// (A forced tile goes to the tile kernels.)
+bool gemm_stream_supports(const GemmArgs& a, int epi, int group) {
+  if (!stream_takes(a, epi, group) || g_tune_tile.load(std::memory_order_relaxed) || g_tune_ks.load(std::memory_order_relaxed))
+    return false;
+  const long columns = stream_columns(a);
+  if (a.M <= 16) return columns >= (a.M >= 5 ? 172 : 224) * 64;
+  if (a.M <= 64) return epi != kRowScale || a.M > 32 || columns > 128 * 32;
+  const long large = (long)((a.M + 63) / 64) * ((columns + 31) / 32);
+  return large <= (epi == kRowScale ? 384 : a.K <= 8192 ? 768 : 640);
+}
+
+int gemm_stream_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
+  if (epi == kRowScale) return launch_stream_by_shape<kRowScale>(a, stream);
+  return a.a_cols == 1 ? launch_stream_by_shape<kTokenGroup>(a, stream) : launch_stream_by_shape<kGroupScale>(a, stream);
+}
+
+// q / k / v with the rotary embedding and the cache write, group-scaled weights: the alternative is 128 x 128 tiles only
+// (48 or 96 of them for the Llama widths).
+bool gemm_stream_rope_supports(const GemmArgs& a, int epi) {
+  return epi != kRowScale && stream_takes(a, kGroupScale, 128) && !g_tune_tile.load(std::memory_order_relaxed) &&
+         (long)((a.M + 63) / 64) * (stream_columns(a) / 32) <= 768;
+}
+
+int gemm_stream_rope_dispatch(const GemmArgs& a, hipStream_t stream) {
+  return a.a_cols == 1 ? launch_stream<4, 1, 2, 3, kTokenGroup, kStreamRope>(a, stream)
+                       : launch_stream<4, 1, 2, 3, kGroupScale, kStreamRope>(a, stream);
+}
+
+}  // namespace flh
