@@ -29,7 +29,6 @@ are stored in it (by stage name) -- the taps the parity tests compare with the C
 """
 import torch
 
-from ..nn.fused import SiluMulQuant
 from ..nn.linear import LinearFLH
 from ..nn.normalization import RMSNorm
 from ..nn.quantization import ActQuantizer
@@ -161,7 +160,6 @@ class W4A4DecoderLayer(torch.nn.Module):
             return ActQuantizer(bits=4, group_size=act_group_size, sym=True, use_hadamard=False, packed_output=True)
         self.attn_quantizer1, self.attn_quantizer2 = quantiser(), quantiser()
         self.mlp_quantizer1, self.mlp_quantizer2 = quantiser(), quantiser()
-        self._silu_mul_quant = SiluMulQuant(act_group_size)
         self._norm16 = {}     # fp16 copies of the norm weights for the fused kernels: name -> (version, tensor)
 
     @classmethod
@@ -471,11 +469,12 @@ class W4A4DecoderLayer(torch.nn.Module):
         return self._output_projection(x, out, cache, fold_residual)
 
     def _residual_in_gemm(self, rows):
-        """Whether o_proj / down_proj add the residual stream in their own epilogue: the fused prefill path of the group
-        configuration, whose norm + quantiser launch has no addition of its own (measured at 2048 tokens: 728 against
-        736 us per layer).  The token configuration keeps the addition inside its norm + rotation launch, which is cheaper
-        than the extra read in the GEMM's epilogue burst (8 x 512 tokens: 888 against 910 us)."""
-        return self.fused and self.record is None and rows > 64 and self.activation == "group"
+        """Whether o_proj / down_proj add the residual stream in their own epilogue: the fused path of the group
+        configuration, whose norm + quantiser launch has no addition of its own (2048 tokens: 728 against 736 us per
+        layer; at decode sizes it takes two launches of 3-4 us off a layer).  The token configuration keeps the addition
+        inside its norm + rotation launch, which is cheaper than the extra read in the GEMM's epilogue burst (8 x 512
+        tokens: 888 against 910 us)."""
+        return self.fused and self.record is None and rows > 0 and self.activation == "group"
 
     def _online_qkv_applies(self):
         """q / k / v in the layout the decode GEMM with its own norm + quantiser takes: no bias, one scale per channel or
@@ -527,7 +526,8 @@ class W4A4DecoderLayer(torch.nn.Module):
             mid = _ops().silu_mul(gate, up) if self.fused else torch.nn.functional.silu(gate) * up
             s, z, q = self._token_quant("mlp_mid", mid, consumers=(self.down_proj,))
         elif self.fused and self.record is None:
-            s, z, q = self._silu_mul_quant(gate, up)
+            q, s = _ops().silu_mul_and_quantize_i4_gs(gate.contiguous(), up.contiguous(), self.act_group_size, False)
+            z = None                                # (symmetric codes: no zero points to fill)
         else:
             s, z, q = self._group_quant("mlp_mid", self.mlp_quantizer2, torch.nn.functional.silu(gate) * up)
         if fold_residual and self._residual_in_gemm(rows):
