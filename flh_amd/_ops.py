@@ -778,6 +778,26 @@ def add_rmsnorm(x, weight=None, eps=1e-5, add=None, return_sum=False):
     return (total, out) if return_sum else out
 
 
+def embed(ids, table, positions, cos_table, sin_table, hadamard=False):
+    """A model step's look-ups in one launch: ids int64 [...] into table [vocab, hidden] fp16 (hadamard: every 128 channels
+    rotated and divided by sqrt(128)), positions int64 [T] into the rotary tables [max_len, d] fp16 -> (fp16 [..., hidden],
+    cos [T, d], sin [T, d]).  An index outside its table gives a row of NaNs."""
+    for t in (ids, table, positions, cos_table, sin_table):
+        _check(t.is_cuda and t.device == table.device and t.is_contiguous(), "tensors must be contiguous and on one CUDA device")
+    _check(ids.dtype == torch.int64 and positions.dtype == torch.int64 and positions.dim() == 1, "ids and positions must be int64")
+    _check(all(t.dtype == torch.float16 and t.dim() == 2 and t.numel() for t in (table, cos_table, sin_table)),
+           "the tables must be 2D float16")
+    _check(cos_table.shape == sin_table.shape, "cos and sin tables must have one shape")
+    hidden, d = table.size(1), cos_table.size(1)
+    _check(hidden % (128 if hadamard else 8) == 0 and d % 8 == 0, "table widths")
+    out = torch.empty((*ids.shape, hidden), dtype=torch.float16, device=table.device)
+    cos, sin = (torch.empty((positions.numel(), d), dtype=torch.float16, device=table.device) for _ in range(2))
+    _run("flh_embed_f16", table.device, ids.data_ptr(), table.data_ptr(), out.data_ptr(), ids.numel(), table.size(0), hidden,
+         int(bool(hadamard)), positions.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+         positions.numel(), cos_table.size(0), d, _stream(table))
+    return out, cos, sin
+
+
 def silu_mul_rotate_and_quantize_i4(gate, up):
     """Decode-sized batches: rotate_and_quantize_i4(silu(gate) * up, hadamard="fast") in one launch that never stores the
     product: gate, up [M, K] fp16 with K = 11008 or 14336, M <= 256 -> (q [M, K/2] u8, scales [M, 1] fp16)."""

@@ -253,6 +253,54 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const __half* __restrict_
   *(h8*)(out + i * 8) = o;
 }
 
+// A model step's look-ups in one launch: the embedding rows of `ids`, for the group configuration with every 128 channels
+// rotated (fp16 butterflies, then float32 1 / sqrt(128) and one rounding, as flh_fwht_f16_inplace and torch's division round
+// them), and the rows of the rotary tables at `positions`.  One 16-byte chunk per lane: first `rows` x hidden, then T x dim
+// of cos and of sin.  An index outside its table gives a row of NaNs.
+// What bounds it is the launch: three to six kernels of 4-5 us each (one of them 12 us for 16 rows of a large table) -> 5 us.
+template <bool HAD>
+__global__ __launch_bounds__(256) void embed_kernel(const long long* __restrict__ ids, const __half* __restrict__ table,
+                                                    __half* __restrict__ out, uint32_t rows, uint32_t vocab, uint32_t hidden,
+                                                    const long long* __restrict__ positions, const __half* __restrict__ cos_table,
+                                                    const __half* __restrict__ sin_table, __half* __restrict__ cos,
+                                                    __half* __restrict__ sin, uint32_t T, uint32_t max_len, uint32_t dim) {
+  const uint32_t per_row = hidden / 8, per_pos = dim / 8, blocks = (rows * per_row + 255) / 256;   // blocks of the first part
+  const _Float16 bad = (_Float16)__builtin_nanf("");
+  const h8 nans = {bad, bad, bad, bad, bad, bad, bad, bad};
+  if (blockIdx.x < blocks) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= rows * per_row) return;                  // (whole groups of 16 lanes when HAD: hidden is a multiple of 128)
+    const uint32_t row = i / per_row, pos = i % per_row;
+    const int lir = HAD ? group_chunk<16>(pos % 16) : 0;
+    const uint32_t chunk = HAD ? pos / 16 * 16 + lir : pos;
+    const long long id = ids[row];
+    const bool known = id >= 0 && id < (long long)vocab;
+    h8 x = known ? *(const h8*)(table + (size_t)id * hidden + chunk * 8) : nans;
+    if constexpr (HAD) {
+      h2 v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = h2{x[2 * e], x[2 * e + 1]};
+      fwht_group_f16<128>(v, lir);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[2 * e] = (_Float16)round_here((float)v[e].x * 0.08838834764831845f);
+        x[2 * e + 1] = (_Float16)round_here((float)v[e].y * 0.08838834764831845f);
+      }
+    }
+    *(h8*)(out + (size_t)row * hidden + chunk * 8) = x;
+    return;
+  }
+  uint32_t i = (blockIdx.x - blocks) * 256u + threadIdx.x;
+  const bool second = i >= T * per_pos;
+  if (second) i -= T * per_pos;
+  if (i >= T * per_pos) return;
+  const uint32_t t = i / per_pos, chunk = i % per_pos;
+  const long long pos = positions[t];
+  const bool known = pos >= 0 && pos < (long long)max_len;
+  const h8 x = known ? *(const h8*)((second ? sin_table : cos_table) + (size_t)pos * dim + chunk * 8) : nans;
+  *(h8*)((second ? sin : cos) + (size_t)t * dim + chunk * 8) = x;
+}
+
 // RMSNorm in front of the group kernel, one workgroup per token row of K = 8 * chunks values (K <= 16384):
 // y = fp16( float(x) * rsqrt(sum(x^2) / K + eps) [* float(weight)] ) with the statistics in float32
 // (flh/nn/normalization.py:12-20), then transform + quantise per group of G as group_kernel<G, HAD, true>.
@@ -921,6 +969,26 @@ extern "C" int flh_silu_mul_f16(const flh_half* gate, const flh_half* up, flh_ha
   hipLaunchKernelGGL(silu_mul_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                      (const __half*)gate, (const __half*)up, (__half*)out, n / 8);
   return check_launch("silu_mul_kernel");
+}
+
+extern "C" int flh_embed_f16(const int64_t* ids, const flh_half* table, flh_half* out, uint32_t rows, uint32_t vocab,
+                             uint32_t hidden, int hadamard, const int64_t* positions, const flh_half* cos_table,
+                             const flh_half* sin_table, flh_half* cos, flh_half* sin, uint32_t T, uint32_t max_len,
+                             uint32_t head_dim, void* stream) {
+  if (!ids || !table || !out || !positions || !cos_table || !sin_table || !cos || !sin) return fail(FLH_EINVAL, "embed: null pointer");
+  if (misaligned16(table, out) || misaligned16(cos_table, sin_table, cos, sin)) return fail(FLH_EINVAL, "embed: tables and outputs must be 16-byte aligned");
+  if (vocab == 0 || max_len == 0) return fail(FLH_EINVAL, "embed: the tables must not be empty");
+  if (hidden == 0 || hidden % (hadamard ? 128 : 8)) return fail(FLH_EINVAL, "embed: hidden (%u) must be a multiple of %d", hidden, hadamard ? 128 : 8);
+  if (head_dim == 0 || head_dim % 8) return fail(FLH_EINVAL, "embed: head_dim (%u) must be a multiple of 8", head_dim);
+  const uint64_t first = (uint64_t)rows * (hidden / 8), second = 2ull * T * (head_dim / 8);
+  if (first + second > 0x7FFFFFFFull) return fail(FLH_EINVAL, "embed: too many elements for one launch");
+  const unsigned blocks = (unsigned)((first + 255) / 256 + (second + 255) / 256);
+  if (blocks == 0) return FLH_OK;
+  auto kern = hadamard ? embed_kernel<true> : embed_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (const long long*)ids, (const __half*)table,
+                     (__half*)out, rows, vocab, hidden, (const long long*)positions, (const __half*)cos_table,
+                     (const __half*)sin_table, (__half*)cos, (__half*)sin, T, max_len, head_dim);
+  return check_launch("embed_kernel");
 }
 
 extern "C" int flh_add_rmsnorm_f16(const flh_half* x, const flh_half* add, const flh_half* weight, float eps, flh_half* out,

@@ -5,7 +5,7 @@ Data flow of the reference's FLH_LlamaForCausalLM.forward (flh/quantized_model/m
 embedding -> [group configuration only: Hadamard of every 128 channels of the embeddings] -> decoder layers ->
 final RMSNorm -> lm_head), with the layers of decoder_layer.py.  The int4 linears, the rotary embedding, attention and
 the norms (the final one with the last residual addition in its launch) are this library's kernels on the fused path;
-the embedding and the head are stock torch ops, as in the reference.
+the head is a stock torch op, as in the reference; the embedding and the rotary rows are one look-up launch.
 Weights are random (there are no checkpoints here): `random_init` draws fp16 weights layer by layer on the device and
 quantises them through the same kernels a loader would use.
 """
@@ -249,12 +249,33 @@ class W4A4LlamaModel(torch.nn.Module):
         values either way."""
         if cache is None:
             return rotary_tables(positions, self.shape.head_dim, self.shape.rope_theta)
+        table = self._rotary_table(cache, positions.device)
+        return table[0].index_select(0, positions), table[1].index_select(0, positions)
+
+    def _rotary_table(self, cache, device):
         table = getattr(cache, "rotary_table", None)
         if table is None:
-            table = rotary_tables(torch.arange(cache.max_len, device=positions.device), self.shape.head_dim,
-                                  self.shape.rope_theta)
+            table = rotary_tables(torch.arange(cache.max_len, device=device), self.shape.head_dim, self.shape.rope_theta)
             cache.rotary_table = table
-        return table[0].index_select(0, positions), table[1].index_select(0, positions)
+        return table
+
+    def _look_up(self, input_ids, positions, cache):
+        """embed(input_ids) and _rotary(positions, cache): one launch on the fused path with a static cache (the same bits)
+        -- unless the embedding is more than a look-up or takes part in a backward pass."""
+        e = self.embed_tokens
+        w = e.weight
+        plain = (type(self).embed is W4A4LlamaModel.embed and type(e) is torch.nn.Embedding and e.max_norm is None
+                 and not e._forward_hooks and not e._forward_pre_hooks and not (torch.is_grad_enabled() and w.requires_grad))
+        if not (plain and self.fused and cache is not None and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
+                and w.data_ptr() % 16 == 0 and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0
+                and input_ids.is_cuda and input_ids.dtype == torch.int64 and positions.dtype == torch.int64
+                and positions.dim() == 1 and input_ids.numel() > 0):
+            cos, sin = self._rotary(positions, cache)
+            return self.embed(input_ids), cos, sin
+        import flh_amd
+        cos, sin = self._rotary_table(cache, positions.device)
+        return flh_amd._CUDA.embed(input_ids.contiguous(), w.detach(), positions.contiguous(), cos, sin,
+                                   hadamard=self.activation == "group")
 
     def forward(self, input_ids, positions, cache=None, return_hidden=False):
         """input_ids [B, T] int64, positions [T] int64 (the same for every sequence of the batch).  cache: None (a
@@ -269,8 +290,7 @@ class W4A4LlamaModel(torch.nn.Module):
             if not torch.cuda.is_current_stream_capturing() and not torch.equal(
                     positions, torch.arange(cache.kv_len - t, cache.kv_len, dtype=positions.dtype, device=positions.device)):
                 raise ValueError("positions must be arange(kv_len - T, kv_len) of the cache (cache.advance(T) returns them)")
-        x = self.embed(input_ids)
-        cos, sin = self._rotary(positions, cache)
+        x, cos, sin = self._look_up(input_ids, positions, cache)
         pending = None            # the last MLP output, added inside the next layer's first launch
         for i, layer in enumerate(self.layers):
             x, pending, _ = layer.forward_deferred(x, pending, cos, sin, cache.layer(i) if cache is not None else None,

@@ -316,6 +316,15 @@ int flh_silu_mul_rotate_quant_i4(const flh_half* gate, const flh_half* up, uint8
 int flh_add_rmsnorm_f16(const flh_half* x, const flh_half* add, const flh_half* weight, float eps, flh_half* out,
                         flh_half* sum_out, uint32_t M, uint32_t K, void* stream);
 
+/* What a model step looks up, in one launch: out[r] = table[ids[r]] (r < rows, `hidden` fp16 channels; hadamard != 0: every
+ * 128 of them rotated as flh_fwht_f16_inplace rotates them, times 1 / sqrt(128) in float32, rounded once -- the group
+ * configuration's embeddings, flh/quantized_model/modeling_llama.py:672), and cos[t], sin[t] = rows positions[t] of the
+ * rotary tables [max_len, head_dim].  hidden a multiple of 8 (128 with hadamard), head_dim of 8; an index outside its table
+ * gives a row of NaNs. */
+int flh_embed_f16(const int64_t* ids, const flh_half* table, flh_half* out, uint32_t rows, uint32_t vocab, uint32_t hidden,
+                  int hadamard, const int64_t* positions, const flh_half* cos_table, const flh_half* sin_table, flh_half* cos,
+                  flh_half* sin, uint32_t T, uint32_t max_len, uint32_t head_dim, void* stream);
+
 /* The same product on its own: out[i] = fp16(fp16(silu(gate[i])) * up[i]) for n fp16 values (n a multiple of 8; out may
  * be gate or up).  One launch for the two torch kernels of modeling_llama.py:522-526 where no quantiser follows directly. */
 int flh_silu_mul_f16(const flh_half* gate, const flh_half* up, flh_half* out, uint64_t n, void* stream);
