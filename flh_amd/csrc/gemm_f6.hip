@@ -693,8 +693,9 @@ bool large_supported(const GemmArgs& a, bool grouped) {
 //    4096, half a round: 30 against 25; 1531 x 6144, 0.56 of a round against 1.13: 34 against 39).
 //  * token scales: a round of 256 x 128 tiles takes 29.5, a round of 128 x 128 ones 16.6 (2048 x 28672: 208 against 223;
 //    1024 x 12288, 1.5 rounds of large tiles: 56 against 51).
-//  * group scales: the large tile from one 128 x 128 tile per compute unit on (1024 x 4096: 30 against 32; 2048 x 28672:
-//    229 against 303).
+//  * group scales: from one 128 x 128 tile per compute unit on, a round of large tiles takes 31, the small ones 10 and 21.6
+//    more per round (1024 x 4096: 30 against 32; 2048 x 28672: 229 against 303; 640 x 11008, 258 large tiles, two rounds for
+//    one: 64 against 53).
 enum LargeTile { kNoLarge = 0, kWide = 1, kNarrow = 2 };
 LargeTile large_choice(const GemmArgs& a, int epi, long columns) {
   const bool grouped = epi != kRowScale;
@@ -705,7 +706,7 @@ LargeTile large_choice(const GemmArgs& a, int epi, long columns) {
   auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((columns + bn - 1) / bn); };
   auto rounds = [](long t) { return (t + 255) / 256; };
   const long small = tiles(128, 128), narrow = tiles(256, 128), wide = tiles(256, 256);
-  if (epi == kGroupScale) return small >= 256 ? kNarrow : kNoLarge;
+  if (epi == kGroupScale) return small >= 256 && rounds(narrow) * 31.0 <= 10.0 + rounds(small) * 21.6 ? kNarrow : kNoLarge;
   if (epi == kTokenGroup) return rounds(narrow) * 29.5 < rounds(small) * 16.6 ? kNarrow : kNoLarge;
   if (small <= 256) return kNoLarge;
   auto cost = [&](long t) { return 0.5 * (rounds(t) + t / 256.0); };

@@ -367,10 +367,13 @@ bool stream_takes(const GemmArgs& a, int epi, int group) {
 //    one token x 12288 9.5 against 8.9, 16 x 6144 8.3 against 8.6).
 //  * 17 .. 64 tokens: always, but for one scale per row on at most 128 blocks of 32 channels, where the decode kernel takes 32
 //    (32 x 4096 6.0 against 6.3; 64 x 4096 8.3 against 6.5).
-//  * more, group-scaled weights, against 64 x 64 and 128 x 128 tiles: up to 640 large tiles, 768 if K is short (128 x 12288,
-//    768: 24 against 27; 192 x 12288, 1152: 35 against 33; 384 x 4096, 768: 22.3 against 25.1, but 64 against 60 for K = 11008).
-//  * more, one scale per row, against the K-split tiles: up to 384 (128 x 6144 11.1 against 12.1; 256 x 4096, 512: 12.0
-//    against 11.9; 128 x 12288, 768: 17.7 against 17.0).
+//  * more, group-scaled weights, against 64 x 64 and 128 x 128 tiles: up to 768 large tiles, 512 if K is long (128 x 12288,
+//    768: 24 against 27; 192 x 12288, 1152: 35 against 33; 384 x 4096, 768: 22.3 against 25.1, but 64 against 60 for K = 11008,
+//    where 300 x 4096, 640, takes 69 against 59 on weights that are in the last-level cache).
+//  * more, one scale per row, against the K-split tiles: up to 384, 256 if K is long (128 x 6144 11.1 against 12.1; 256 x 4096,
+//    512: 12.0 against 11.9; 128 x 12288, 768: 17.7 against 17.0; 180 x 4096, 384, K = 11008: 28 against 26).
+//  * and no more tokens than 1280, 512 with one scale per row: on 1024 channels the tiles fill the chip by then (1500 tokens, token
+//    scales, with their quantiser: 31.6 against 29.5; 700, one scale per row: 16.6 against 16.1).
 // (A forced tile goes to the tile kernels.)
 bool gemm_stream_supports(const GemmArgs& a, int epi, int group) {
   if (!stream_takes(a, epi, group) || g_tune_tile.load(std::memory_order_relaxed) || g_tune_ks.load(std::memory_order_relaxed))
@@ -378,8 +381,9 @@ bool gemm_stream_supports(const GemmArgs& a, int epi, int group) {
   const long columns = stream_columns(a);
   if (a.M <= 16) return columns >= (a.M >= 5 ? 172 : 224) * 64;
   if (a.M <= 64) return epi != kRowScale || a.M > 32 || columns > 128 * 32;
+  if (a.M > (epi == kRowScale ? 512 : 1280)) return false;
   const long large = (long)((a.M + 63) / 64) * ((columns + 31) / 32);
-  return large <= (epi == kRowScale ? 384 : a.K <= 8192 ? 768 : 640);
+  return large <= (epi == kRowScale ? 128 : 256) * (a.K <= 8192 ? 3 : 2);
 }
 
 int gemm_stream_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
