@@ -402,6 +402,77 @@ std::vector<Tensor> rmsnorm_and_quantize_i4_gs(const Tensor& x, const c10::optio
   return {q, s};
 }
 
+// ---- the modules' calls on a few rows, views and allocations included ------------------------------------------------------
+// What ActQuantizer and LinearFLH do around the ops above -- flatten, check, allocate, restore the leading dimensions -- in one
+// call each (a decode-sized launch takes 4-15 us, the Python around one took 4-6).  A call that is not of the plain form gives
+// nothing, and the module's general path serves or refuses it.
+bool plain(const Tensor& t, torch::ScalarType type, const Tensor& like) {
+  return t.is_cuda() && t.scalar_type() == type && t.is_contiguous() && t.device() == like.device();
+}
+
+// rows of x (K / width of them in each), or -1
+int64_t plain_rows(const Tensor& x, torch::ScalarType type, int64_t width) {
+  if (width <= 0 || x.dim() < 1 || !plain(x, type, x) || x.size(-1) != width || x.numel() == 0) return -1;
+  return x.numel() / width;
+}
+
+bool plain_weights(const Tensor& x, const Tensor& w, const Tensor& w_scale, int64_t K, int64_t N) {
+  return K > 0 && N > 0 && K % 128 == 0 && plain(w, torch::kUInt8, x) && plain(w_scale, torch::kFloat16, x) &&
+         w.numel() == N * (K / 2) && w_scale.numel() > 0 && w_scale.numel() % N == 0;
+}
+
+Tensor empty_rows(const Tensor& x, int64_t width, const torch::TensorOptions& options) {
+  std::vector<int64_t> sizes = x.sizes().vec();
+  sizes.back() = width;
+  return torch::empty(sizes, options);
+}
+
+c10::optional<Tensor> linear_i4(const Tensor& x, const Tensor& a_scale, const Tensor& w, const Tensor& w_scale, int64_t K,
+                                int64_t N, int64_t group, int64_t row_limit) {
+  const int64_t M = plain_rows(x, torch::kUInt8, K / 2);
+  if (M < 0 || M >= row_limit || !plain_weights(x, w, w_scale, K, N) || !plain(a_scale, torch::kFloat16, x) ||
+      a_scale.numel() == 0 || a_scale.numel() % M)
+    return c10::nullopt;
+  Tensor D = empty_rows(x, N, a_scale.options());
+  Launch l(x);
+  ok(flh_gemm_i4_o16(u8(x), u8(w), h(a_scale), h(w_scale), hm(D), M, N, K, (int)(a_scale.numel() / M),
+                     (int)(w_scale.numel() / N), (int)group, stream_of(x)));
+  return D;
+}
+
+// mode: FLH_HAD_F32 / FLH_HAD_MFMA, or -1: the default for this K (rotate_and_quantize_i4's True)
+c10::optional<Tensor> linear_online_i4(const Tensor& x, const Tensor& w, const Tensor& w_scale, int64_t K, int64_t N,
+                                       int64_t group, int64_t mode, int64_t row_limit) {
+  const int64_t M = plain_rows(x, torch::kFloat16, K);
+  if (M < 0 || M >= row_limit || !plain_weights(x, w, w_scale, K, N)) return c10::nullopt;
+  if (mode < 0) mode = K == 11008 || K == 14336 ? FLH_HAD_MFMA : FLH_HAD_F32;
+  const int64_t cols = w_scale.numel() / N;
+  Tensor D = empty_rows(x, N, x.options());
+  Launch l(x);
+  if (M <= 2 && K == 4096 && mode == FLH_HAD_F32 && (cols == 1 || (group == 128 && cols == 32))) {
+    ok(flh_rotate_quant_gemm_i4_o16(h(x), u8(w), h(w_scale), hm(D), M, N, K, (int)cols, stream_of(x)));
+    return D;
+  }
+  Tensor q = torch::empty({M, K / 2}, x.options().dtype(torch::kUInt8));
+  Tensor s = torch::empty({M, 1}, x.options());
+  ok(flh_rotate_quant_i4(h(x), (uint8_t*)q.data_ptr(), hm(s), nullptr, (uint32_t)M, (uint32_t)K, (int)mode, 0, 0, 1.0f,
+                         stream_of(x)));
+  ok(flh_gemm_i4_o16(u8(q), u8(w), h(s), h(w_scale), hm(D), M, N, K, 1, (int)cols, (int)group, stream_of(x)));
+  return D;
+}
+
+// groups of 128 along the last dimension: {scales [..., K / 128], codes [..., K / 2]}, or nothing
+std::vector<Tensor> quantize_groups(const Tensor& x, bool hadamard, double scale_mul) {
+  if (x.dim() < 1 || !plain(x, torch::kFloat16, x) || x.numel() == 0 || x.size(-1) % 128) return {};
+  const int64_t K = x.size(-1);
+  Tensor q = empty_rows(x, K / 2, x.options().dtype(torch::kUInt8));
+  Tensor s = empty_rows(x, K / 128, x.options());
+  Launch l(x);
+  ok(flh_group_quant_i4(h(x), (uint8_t*)q.data_ptr(), hm(s), (uint32_t)(x.numel() / 128), 128, hadamard ? 1 : 0,
+                        (float)scale_mul, stream_of(x)));
+  return {s, q};
+}
+
 // ---- rotary embedding + cache write -----------------------------------------------------------------------------------
 Tensor rope_kv_cache_(Tensor q, const Tensor& k, const Tensor& v, const Tensor& cos, const Tensor& sin,
                       const Tensor& positions, Tensor k_cache, Tensor v_cache) {
@@ -469,6 +540,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rotate_quantize_gemm_i4_multi", &rotate_quantize_gemm_i4_multi, py::arg("x"), py::arg("Bs"), py::arg("B_scales"));
   m.def("rope_kv_cache_", &rope_kv_cache_, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cos"), py::arg("sin"),
         py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"));
+  m.def("linear_i4", &linear_i4);
+  m.def("linear_online_i4", &linear_online_i4);
+  m.def("quantize_groups", &quantize_groups);
   m.def("hadamard_transform_half", &hadamard_transform_half, py::arg("x"));
   m.def("hadamard_transform_128_half", &hadamard_transform_half, py::arg("x"));   // the name flh/cuda/hadamard.py:35 calls
   m.def("hadamard_transform_64_half", &hadamard_transform_64_half, py::arg("x"));

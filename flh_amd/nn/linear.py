@@ -48,17 +48,24 @@ class LinearFLH(torch.nn.Module):
     def drop_six_bit_weights(self):
         self._w6 = self._w6_key = None
 
-    # Rows from which a call is faster on the 6-bit instruction although it encodes the weights first: (one scale per
-    # channel, a scale per group of 128).  At 3000 rows of 4096 x 11008 the pass takes 12 us and the GEMM 94 instead of 126
-    # (2048 rows: 70 instead of 85, even with the pass and its launch); with a scale per group at 700 rows 12 us and 47
-    # (token scales) or 57 (group scales) instead of 68 or 80 (512 rows of 4096 x 4096: 6 and 16 or 19 against 22 or 25).
-    TRANSIENT_ROWS = (2560, 640)
+    # A call that encodes its weights for the 6-bit instruction first is faster from these rows on (one scale per channel, a
+    # scale per group of 128) if it also has more 128 x 128 tiles than that -- less fills the chip with neither kernel, and the
+    # passes over the operands are all that differs.  us, encoding included, against the int8 kernels: group scales 2048 x 1024
+    # (rows x channels, K = 4096; 128 tiles) 30 against 24, 1024 x 4096 (256) 45 against 38, 1280 x 4096 (320) 47 against 52,
+    # 640 x 11008 (430) 65 against 58, 700 x 11008 (516) 76 against 81, 1024 x 14336 83 against 102; one scale per channel 2048 x 4096 (512) 41 against 34,
+    # 2048 x 11008 84 against 88, 3000 x 11008 106 against 126.
+    TRANSIENT_ROWS, TRANSIENT_TILES = (2560, 641), (512, 256)
 
     def _keeps_six_bit(self, grouped):
         return self.six_bit is True or (self.six_bit is not False and grouped)
 
-    def _six_bit_rows(self, grouped):
-        return self.six_bit_min_rows if self._keeps_six_bit(grouped) else self.TRANSIENT_ROWS[1 if grouped else 0]
+    def _six_bit_rows(self, grouped, columns=None):
+        """Rows from which a launch over `columns` channels (this layer's, unless it shares the launch) takes the 6-bit
+        instruction."""
+        if self._keeps_six_bit(grouped):
+            return self.six_bit_min_rows
+        tiles = -(-(columns or self.out_features) // 128)
+        return max(self.TRANSIENT_ROWS[grouped], 128 * (self.TRANSIENT_TILES[grouped] // tiles) + 1)
 
     def prepare_six_bit(self):
         """Build the 6-bit encoding of the weights now if this layer's setting keeps one (at load time, rather than inside
@@ -75,23 +82,31 @@ class LinearFLH(torch.nn.Module):
             self._w6_key = key
         return self._w6
 
-    def wants_six_bit(self, n_rows):
+    def wants_six_bit(self, n_rows, columns=None):
         """Whether a call with `n_rows` per-token-quantised rows takes the 6-bit matrix instruction (a producer can then
-        write the activations in that format directly, rotate_and_quantize_f6)."""
+        write the activations in that format directly, rotate_and_quantize_f6).  `columns`: channels of the whole launch,
+        where several layers share one."""
         if (n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS[1]) or self.in_features % 128 or not self.w_packed.is_cuda:
             return False
         cols = self.w_scale.view(self.out_features, -1).size(1)
         if cols != 1 and not (cols == self.in_features // 128 and self.weight_group_size == 128):
             return False
-        return n_rows >= self._six_bit_rows(cols != 1)
+        return n_rows >= self._six_bit_rows(cols != 1, columns)
 
-    def _six_bit_applies(self, rows, a_scale, w_scale, group):
+    def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)
         if (n < self.six_bit_min_rows and n < self.TRANSIENT_ROWS[1]) or not rows.is_cuda or self.in_features % 128:
             return False
         per_row = a_scale.size(1) == 1 and w_scale.size(1) == 1
         grouped = group == 128 and w_scale.size(1) == self.in_features // 128 and a_scale.size(1) in (1, w_scale.size(1))
-        return (grouped or per_row) and n >= self._six_bit_rows(not per_row)
+        return (grouped or per_row) and n >= self._six_bit_rows(not per_row, columns)
+
+    def _group(self):
+        return self.weight_group_size if self.weight_group_size > 0 else (self.in_group_size or 128)
+
+    def _few_rows(self, w_scale):
+        """Rows below which no call of this layer takes the 6-bit instruction."""
+        return self._six_bit_rows(w_scale.numel() > self.out_features)
 
     # ------------------------------------------------------------------ kernels
     def forward(self, x, a_scale=None, a_zero=None, x_is_packed=False, is_symmetric=None, residual=None):
@@ -99,6 +114,13 @@ class LinearFLH(torch.nn.Module):
         fp16 (as returned by ActQuantizer).  Returns fp16 [..., N].  `residual` (extension; fp16 [..., N]): returns
         residual + forward(x, ...) from the same launch -- the layer output rounded to fp16 as always, then one fp16
         addition in the GEMM's epilogue instead of a separate pass over both tensors."""
+        if residual is None and a_scale is not None:
+            w, w_scale = self._buffers.get("w_packed"), self._buffers.get("w_scale")
+            if w is not None and w_scale is not None:
+                y = _pkg._CUDA.linear_i4(x, a_scale, w, w_scale, self.in_features, self.out_features, self._group(),
+                                         self._few_rows(w_scale))
+                if y is not None:
+                    return y if self.bias is None else y + self.bias
         lead = x.shape[:-1]
         if residual is not None and self.bias is not None:
             return residual + self.forward(x, a_scale, a_zero, x_is_packed, is_symmetric)
@@ -150,7 +172,8 @@ class LinearFLH(torch.nn.Module):
         a_rows = a_scale.reshape(rows.size(0), -1)
         w_scales = [l.w_scale.view(l.out_features, -1) for l in layers]
         encoded = rows.size(1) * 4 == first.in_features * 3      # activations already in the 6-bit format
-        if encoded or all(l._six_bit_applies(rows, a_rows, ws, group) for l, ws in zip(layers, w_scales)):
+        columns = sum(l.out_features for l in layers)
+        if encoded or all(l._six_bit_applies(rows, a_rows, ws, group, columns) for l, ws in zip(layers, w_scales)):
             # every layer opted into the 6-bit matrix instruction: one launch there as well
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
             ys = ops.gemm_f6_dequant_multi(a6, [l._six_bit_weights() for l in layers], a_rows.contiguous(), w_scales)
@@ -177,7 +200,7 @@ class LinearFLH(torch.nn.Module):
         group = gate_layer.weight_group_size if gate_layer.weight_group_size > 0 else (gate_layer.in_group_size or 128)
         a_rows = a_scale.reshape(rows.size(0), -1)
         encoded = rows.size(1) * 4 == k * 3                     # activations already in the 6-bit format
-        six = [l._six_bit_applies(rows, a_rows, l.w_scale.view(n, -1), group) for l in (gate_layer, up_layer)]
+        six = [l._six_bit_applies(rows, a_rows, l.w_scale.view(n, -1), group, 2 * n) for l in (gate_layer, up_layer)]
         if encoded or all(six):
             ops = _pkg._CUDA
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
@@ -189,6 +212,8 @@ class LinearFLH(torch.nn.Module):
                                       up_layer.w_scale.view(n, -1), group)
         return y.view(*lead, n)
 
+    _ONLINE_MODES = {"exact": 1, "fast": 2}        # FLH_HAD_F32, FLH_HAD_MFMA
+
     def forward_online(self, x, hadamard=True):
         """fp16 activations [..., K] -> fp16 [..., N] with the activation side done here: whole-row rotation
         (`hadamard`: as in rotate_and_quantize_i4), one symmetric int4 scale per token, then the GEMM -- the
@@ -196,6 +221,12 @@ class LinearFLH(torch.nn.Module):
         has no module of its own there.  One or two tokens of K = 4096 with the bit-exact rotation take the
         single-launch decode path; the outputs are the same bits either way."""
         ops = _pkg._CUDA
+        buf, mode = self._buffers, -1 if hadamard is True else self._ONLINE_MODES.get(hadamard)
+        if mode is not None and buf.get("w_packed") is not None and buf.get("w_scale") is not None:
+            y = ops.linear_online_i4(x, buf["w_packed"], buf["w_scale"], self.in_features, self.out_features, self._group(),
+                                     mode, self._few_rows(buf["w_scale"]))
+            if y is not None:
+                return y if self.bias is None else y + self.bias
         lead = x.shape[:-1]
         rows = x.reshape(-1, x.size(-1)).contiguous()
         w = self.w_packed.view(self.out_features, self.in_features // 2)

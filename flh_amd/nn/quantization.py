@@ -100,6 +100,11 @@ class ActQuantizer(torch.nn.Module):
         quantisation and the division of the scales by sqrt(128) in one kernel; scale shape
         [..., K/128].  per_token=True: normalised rotation of the whole row in float32 and
         one scale per row, shape [..., 1]."""
+        if not self.per_token:
+            # (the reference's "scales / sqrt(128)" rides on the same launch, see below)
+            r = _pkg._CUDA.quantize_groups(x, self.use_hadamard, _INV_SQRT_128 if self.use_hadamard else 1.0)
+            if r:
+                return r[0], None, r[1]
         lead, k = x.shape[:-1], x.shape[-1]
         if self.per_token:
             q, s = _pkg._CUDA.rotate_and_quantize_i4(x.reshape(-1, k), hadamard=self.use_hadamard,

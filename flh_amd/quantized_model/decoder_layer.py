@@ -229,7 +229,8 @@ class W4A4DecoderLayer(torch.nn.Module):
         """Whether the quantiser in front of `consumers` should write the 6-bit operand format directly: every consumer
         would re-encode the nibbles for the 6-bit matrix instruction anyway."""
         return (bool(consumers) and self.activation == "token" and self.fused and self.record is None
-                and width in self._F6_WIDTHS and all(l.wants_six_bit(n_rows) for l in consumers))
+                and width in self._F6_WIDTHS
+                and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers))
 
     def _rotation_mode(self, rows, k):
         """hadamard argument of the whole-row ops for `rows` rows of k channels."""
@@ -429,8 +430,8 @@ class W4A4DecoderLayer(torch.nn.Module):
             return None
         layers = (self.q_proj, self.k_proj, self.v_proj)
         group = self.q_proj.weight_group_size if self.q_proj.weight_group_size > 0 else (self.q_proj.in_group_size or 128)
-        six = all(l._six_bit_applies(codes.reshape(rows, -1), scales.reshape(rows, -1), l.w_scale.view(l.out_features, -1), group)
-                  for l in layers)
+        six = all(l._six_bit_applies(codes.reshape(rows, -1), scales.reshape(rows, -1), l.w_scale.view(l.out_features, -1), group,
+                                       sum(c.out_features for c in layers)) for l in layers)
         return "f6" if six else "i4"
 
     def _attention_after_fused_qkv(self, x, codes, scales, cos, sin, kv_cache, positions, fold_residual, mode):
