@@ -778,6 +778,24 @@ def add_rmsnorm(x, weight=None, eps=1e-5, add=None, return_sum=False):
     return (total, out) if return_sum else out
 
 
+LINEAR_F16_MAX_ROWS = 16
+
+
+def linear_f16(x, w):
+    """x [..., K] @ w[N, K]^T for up to 16 rows of fp16, float32 accumulation, K a multiple of 128 (a decode step's head)."""
+    _check(x.is_cuda and w.is_cuda and x.device == w.device, "tensors must be on one CUDA device")
+    _check(x.dtype == torch.float16 and w.dtype == torch.float16 and w.dim() == 2 and x.dim() >= 1, "float16 x [..., K] and w [N, K]")
+    _check(x.is_contiguous() and w.is_contiguous(), "tensors must be contiguous")
+    N, K = w.shape
+    _check(x.size(-1) == K and K > 0 and K % 128 == 0, "x.shape[-1] must equal w.shape[1], a multiple of 128")
+    M = x.numel() // K
+    _check(M <= LINEAR_F16_MAX_ROWS, "at most 16 rows")
+    y = torch.empty((*x.shape[:-1], N), dtype=torch.float16, device=x.device)
+    if M and N:
+        _run("flh_linear_f16", x.device, x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, _stream(x))
+    return y
+
+
 def embed(ids, table, positions, cos_table, sin_table, hadamard=False):
     """A model step's look-ups in one launch: ids int64 [...] into table [vocab, hidden] fp16 (hadamard: every 128 channels
     rotated and divided by sqrt(128)), positions int64 [T] into the rotary tables [max_len, d] fp16 -> (fp16 [..., hidden],

@@ -80,6 +80,11 @@ __device__ __forceinline__ void load_to_lds16(const void* gptr, unsigned lds_bas
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
 
+// the same for data that is read once (non-temporal: it does not displace what the caches hold)
+__device__ __forceinline__ void load_to_lds16_nt(const void* gptr, unsigned lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
+}
+
 // 4 bytes per lane: lane i writes lds_base + 4 * i
 __device__ __forceinline__ void load_to_lds4(const void* gptr, unsigned lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");

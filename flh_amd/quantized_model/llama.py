@@ -5,7 +5,8 @@ Data flow of the reference's FLH_LlamaForCausalLM.forward (flh/quantized_model/m
 embedding -> [group configuration only: Hadamard of every 128 channels of the embeddings] -> decoder layers ->
 final RMSNorm -> lm_head), with the layers of decoder_layer.py.  The int4 linears, the rotary embedding, attention and
 the norms (the final one with the last residual addition in its launch) are this library's kernels on the fused path;
-the head is a stock torch op, as in the reference; the embedding and the rotary rows are one look-up launch.
+the embedding and the rotary rows are one look-up launch, and a decode step's fp16 head is a kernel of its own (a stock
+torch op for more rows, as in the reference).
 Weights are random (there are no checkpoints here): `random_init` draws fp16 weights layer by layer on the device and
 quantises them through the same kernels a loader would use.
 """
@@ -296,7 +297,23 @@ class W4A4LlamaModel(torch.nn.Module):
             x, pending, _ = layer.forward_deferred(x, pending, cos, sin, cache.layer(i) if cache is not None else None,
                                                    positions)
         x = self._final_norm(x, pending)
-        return x if return_hidden else self.lm_head(x)
+        return x if return_hidden else self._head(x)
+
+    def _head(self, x):
+        """lm_head(x): for a decode step's rows on the fused path this library's kernel (the same float32 accumulation in
+        another order; the vendor's reads the weights at 5.7 TB/s, this one at 6.8) -- unless the head is more than a plain
+        fp16 product or takes part in a backward pass."""
+        h = self.lm_head
+        w = h.weight
+        if (self.fused and type(h) is torch.nn.Linear and h.bias is None and not h._forward_hooks and not h._forward_pre_hooks
+                and 0 < x.numel() <= 16 * x.size(-1) and x.is_cuda and x.device == w.device and x.dtype == w.dtype == torch.float16
+                and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.size(1) == x.size(-1) and w.size(1) % 128 == 0
+                and not (torch.is_grad_enabled() and (w.requires_grad or x.requires_grad))
+                and not torch.is_autocast_enabled()):
+            import flh_amd
+            x = x.contiguous()
+            return flh_amd._CUDA.linear_f16(x if x.data_ptr() % 16 == 0 else x.clone(), w.detach())
+        return h(x)
 
     def _final_norm(self, x, pending):
         """The last residual addition and the final RMSNorm: one launch on the fused path (the roundings of the two

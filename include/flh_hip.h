@@ -316,6 +316,10 @@ int flh_silu_mul_rotate_quant_i4(const flh_half* gate, const flh_half* up, uint8
 int flh_add_rmsnorm_f16(const flh_half* x, const flh_half* add, const flh_half* weight, float eps, flh_half* out,
                         flh_half* sum_out, uint32_t M, uint32_t K, void* stream);
 
+/* fp16 linear for up to 16 rows: y [M, N] = fp16(x [M, K] . w [N, K]^T), float32 accumulation -- the language-model head of a
+ * decode step (flh/quantized_model/modeling_llama.py:693).  K a multiple of 128. */
+int flh_linear_f16(const flh_half* x, const flh_half* w, flh_half* y, uint32_t M, uint32_t N, uint32_t K, void* stream);
+
 /* What a model step looks up, in one launch: out[r] = table[ids[r]] (r < rows, `hidden` fp16 channels; hadamard != 0: every
  * 128 of them rotated as flh_fwht_f16_inplace rotates them, times 1 / sqrt(128) in float32, rounded once -- the group
  * configuration's embeddings, flh/quantized_model/modeling_llama.py:672), and cos[t], sin[t] = rows positions[t] of the
