@@ -336,13 +336,14 @@ long stream_columns(const GemmArgs& a) {
 }
 
 // Tiles, tokens x channels: 16 x 64 for up to 16 tokens, else 32 x 32, or 64 x 32 (half the weight traffic, a fifth less
-// vector work) where two of its workgroups per compute unit remain and the tokens fill it as well as the smaller tile (256
-// tokens: 4096 x 4096 15.7 against 18.1 us; 128: 4096 x 6144, 1.5 of its workgroups, 15.7 against 14.3).
+// vector work) where nearly two of its workgroups per compute unit remain and the tokens fill it as well as the smaller tile
+// (64 tokens: 4096 x 14336, 448 workgroups, 17.0 against 18.3 us; 256: 4096 x 4096, 512, 15.7 against 18.1; 128: 4096 x 6144,
+// 384, 15.7 against 14.3).
 template <int EPI>
 int launch_stream_by_shape(const GemmArgs& a, hipStream_t stream) {
   if (a.M <= 16) return launch_stream<1, 4, 1, 3, EPI, kStreamPlain>(a, stream);
   const long large = (long)((a.M + 63) / 64) * ((stream_columns(a) + 31) / 32);
-  if (large >= 512 && (a.M + 31) / 32 % 2 == 0) return launch_stream<4, 1, 2, 3, EPI, kStreamPlain>(a, stream);
+  if (large >= 448 && (a.M + 31) / 32 % 2 == 0) return launch_stream<4, 1, 2, 3, EPI, kStreamPlain>(a, stream);
   return launch_stream<2, 2, 1, 3, EPI, kStreamPlain>(a, stream);
 }
 
