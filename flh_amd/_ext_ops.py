@@ -27,6 +27,7 @@ rotate_quantize_gemm_i4_multi = _ext.rotate_quantize_gemm_i4_multi
 linear_i4 = _ext.linear_i4
 linear_online_i4 = _ext.linear_online_i4
 quantize_groups = _ext.quantize_groups
+quantize_rows = _ext.quantize_rows
 hadamard_transform_half = _ext.hadamard_transform_half
 hadamard_transform_128_half = _ext.hadamard_transform_128_half
 hadamard_transform_64_half = _ext.hadamard_transform_64_half

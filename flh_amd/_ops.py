@@ -979,4 +979,4 @@ def linear_i4(*args):
     return None
 
 
-linear_online_i4 = quantize_groups = linear_i4
+linear_online_i4 = quantize_groups = quantize_rows = linear_i4

@@ -473,6 +473,19 @@ std::vector<Tensor> quantize_groups(const Tensor& x, bool hadamard, double scale
   return {s, q};
 }
 
+// whole rows, one scale each: {scales [..., 1], codes [..., K / 2]}, or nothing
+std::vector<Tensor> quantize_rows(const Tensor& x, int64_t mode, double clip_ratio) {
+  if (x.dim() < 1 || !plain(x, torch::kFloat16, x) || x.numel() == 0 || x.size(-1) % 2) return {};
+  const int64_t K = x.size(-1);
+  if (mode < 0) mode = K == 11008 || K == 14336 ? FLH_HAD_MFMA : FLH_HAD_F32;
+  Tensor q = empty_rows(x, K / 2, x.options().dtype(torch::kUInt8));
+  Tensor s = empty_rows(x, 1, x.options());
+  Launch l(x);
+  ok(flh_rotate_quant_i4(h(x), (uint8_t*)q.data_ptr(), hm(s), nullptr, (uint32_t)(x.numel() / K), (uint32_t)K, (int)mode, 0, 0,
+                         (float)clip_ratio, stream_of(x)));
+  return {s, q};
+}
+
 // ---- rotary embedding + cache write -----------------------------------------------------------------------------------
 Tensor rope_kv_cache_(Tensor q, const Tensor& k, const Tensor& v, const Tensor& cos, const Tensor& sin,
                       const Tensor& positions, Tensor k_cache, Tensor v_cache) {
@@ -543,6 +556,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_i4", &linear_i4);
   m.def("linear_online_i4", &linear_online_i4);
   m.def("quantize_groups", &quantize_groups);
+  m.def("quantize_rows", &quantize_rows);
   m.def("hadamard_transform_half", &hadamard_transform_half, py::arg("x"));
   m.def("hadamard_transform_128_half", &hadamard_transform_half, py::arg("x"));   // the name flh/cuda/hadamard.py:35 calls
   m.def("hadamard_transform_64_half", &hadamard_transform_64_half, py::arg("x"));

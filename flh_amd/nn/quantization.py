@@ -100,11 +100,14 @@ class ActQuantizer(torch.nn.Module):
         quantisation and the division of the scales by sqrt(128) in one kernel; scale shape
         [..., K/128].  per_token=True: normalised rotation of the whole row in float32 and
         one scale per row, shape [..., 1]."""
-        if not self.per_token:
+        if self.per_token:
+            mode = -1 if self.use_hadamard is True else 0 if self.use_hadamard is False else None
+            r = _pkg._CUDA.quantize_rows(x, mode, self.input_clip_ratio) if mode is not None else None
+        else:
             # (the reference's "scales / sqrt(128)" rides on the same launch, see below)
-            r = _pkg._CUDA.quantize_groups(x, self.use_hadamard, _INV_SQRT_128 if self.use_hadamard else 1.0)
-            if r:
-                return r[0], None, r[1]
+            r = _pkg._CUDA.quantize_groups(x, bool(self.use_hadamard), _INV_SQRT_128 if self.use_hadamard else 1.0)
+        if r:
+            return r[0], None, r[1]
         lead, k = x.shape[:-1], x.shape[-1]
         if self.per_token:
             q, s = _pkg._CUDA.rotate_and_quantize_i4(x.reshape(-1, k), hadamard=self.use_hadamard,

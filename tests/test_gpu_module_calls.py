@@ -1,4 +1,4 @@
-"""The modules' native calls (linear_i4, linear_online_i4, quantize_groups) against the general path of the same modules, bit for
+"""The modules' native calls (linear_i4, linear_online_i4, quantize_groups, quantize_rows) against the general path of the same modules, bit for
 bit, over the forms a caller may use, and the row counts around which a layer changes its kernel."""
 import pytest
 
@@ -13,7 +13,7 @@ class General:
         self._ops = ops
 
     def __getattr__(self, name):
-        return (lambda *a: None) if name in ("linear_i4", "linear_online_i4", "quantize_groups") else getattr(self._ops, name)
+        return (lambda *a: None) if name in ("linear_i4", "linear_online_i4", "quantize_groups", "quantize_rows") else getattr(self._ops, name)
 
 
 @pytest.fixture
@@ -41,7 +41,8 @@ def test_linear_on_quantised_rows(both, lead, group, bias):
     torch.manual_seed(sum(lead))
     lin, x = layer(512, 264, group, bias), torch.randn(*lead, 512, device="cuda").half()
     for q in (ActQuantizer(bits=4, group_size=128, packed_output=True), ActQuantizer(bits=4, group_size=128, packed_output=True, use_hadamard=False),
-              ActQuantizer(bits=4, packed_output=True, per_token=True)):
+              ActQuantizer(bits=4, packed_output=True, per_token=True),
+              ActQuantizer(bits=4, packed_output=True, per_token=True, use_hadamard=False, input_clip_ratio=0.9)):
         if group == 64 and not q.per_token:
             continue
         (s, z, c), (s2, z2, c2) = both(lambda: q(x))
