@@ -83,6 +83,8 @@ _SIG = {
     "flh_rotate_quant_f6": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_int, _PTR, _c.c_float, _PTR, _PTR, _c.c_uint32, _c.c_uint32,
                                       _c.c_int, _c.c_float, _PTR]),
     "flh_silu_mul_f16": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_uint64, _PTR]),
+    "flh_rmsnorm_group_quant_f6": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _c.c_float, _PTR]),
+    "flh_silu_mul_group_quant_f6": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _PTR]),
     "flh_linear_f16": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _c.c_uint32, _PTR]),
     "flh_embed_f16": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _c.c_uint32, _c.c_int, _PTR, _PTR, _PTR, _PTR, _PTR,
                                 _c.c_uint32, _c.c_uint32, _c.c_uint32, _PTR]),

@@ -367,6 +367,39 @@ def group_quantize_f6(x, hadamard=True, *, scale_mul=1.0):
     return [q6, s]
 
 
+def _f6_rows(x):
+    _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
+           "Input tensor must be a contiguous 2D float16 CUDA tensor")
+    M, K = x.shape
+    _check(K % 128 == 0 and K > 0, "Last dimension must be a multiple of 128")
+    return (M, K, torch.empty((M, K // 128 * 96), dtype=torch.uint8, device=x.device),
+            torch.empty((M, K // 128), dtype=torch.float16, device=x.device))
+
+
+def rmsnorm_group_quantize_f6(x, weight, eps):
+    """rmsnorm_and_quantize_i4_gs(x, weight, eps, 128) of x [M, K] with the codes in the format of encode_f6."""
+    M, K, q6, s = _f6_rows(x)
+    _check(K <= 16384, "Last dimension must be at most 16384")
+    if weight is not None:
+        _check(weight.is_cuda and weight.dtype == torch.float16 and weight.is_contiguous() and weight.numel() == K
+               and weight.device == x.device, "weight must be a contiguous float16 CUDA tensor of K values")
+    if M:
+        _run("flh_rmsnorm_group_quant_f6", x.device, x.data_ptr(), weight.data_ptr() if weight is not None else None,
+             q6.data_ptr(), s.data_ptr(), M, K, float(eps), _stream(x))
+    return [q6, s]
+
+
+def silu_mul_group_quantize_f6(gate, up):
+    """silu_mul_and_quantize_i4_gs(gate, up, 128) of [M, K] tensors with the codes in the format of encode_f6."""
+    M, K, q6, s = _f6_rows(gate)
+    _check(up.is_cuda and up.dtype == torch.float16 and up.shape == gate.shape and up.is_contiguous()
+           and up.device == gate.device, "gate and up must be contiguous float16 CUDA tensors of one shape")
+    if M:
+        _run("flh_silu_mul_group_quant_f6", gate.device, gate.data_ptr(), up.data_ptr(), q6.data_ptr(), s.data_ptr(), M, K,
+             _stream(gate))
+    return [q6, s]
+
+
 def _check_f6(A6, B6):
     _check(A6.is_cuda and B6.is_cuda, "tensors must be CUDA")
     _check(A6.dtype == torch.uint8 and B6.dtype == torch.uint8, "encoded operands must be uint8")

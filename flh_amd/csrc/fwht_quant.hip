@@ -218,10 +218,11 @@ __global__ __launch_bounds__(256) void group_kernel(const __half* __restrict__ x
 // SwiGLU in front of the group kernel: x = fp16( float(fp16(silu(gate))) * float(up) ) -- the two roundings
 // of torch's fp16 silu and fp16 multiply (flh/quantized_model/modeling_llama.py:522-526 feeds exactly this
 // product to the quantiser of down_proj) -- then transform + quantise as group_kernel<G, HAD, true>.
-template <int G, bool HAD>
+template <int G, bool HAD, bool F6 = false>
 __global__ __launch_bounds__(256) void silu_mul_group_kernel(const __half* __restrict__ gate,
                                                              const __half* __restrict__ up, uint8_t* __restrict__ q,
-                                                             __half* __restrict__ scales, uint32_t R, float scale_mul) {
+                                                             __half* __restrict__ scales, uint32_t R, float scale_mul,
+                                                             uint32_t tokens = 0, uint32_t groups_per_token = 1) {
   constexpr int LPR = G / 8;
   const uint32_t gl = blockIdx.x * 256u + threadIdx.x;
   const uint32_t row = gl / LPR;
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(256) void silu_mul_group_kernel(const __half* __res
     else v[i >> 1].x = prod;
   }
   if constexpr (HAD) fwht_group_f16<G>(v, lir);
-  group_finish<G>(v, lir, valid, row, q, scales, scale_mul);
+  group_finish<G, F6>(v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
 }
 
 // the SwiGLU product alone, eight values per thread
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const long long* __restrict_
 // RMSNorm in front of the group kernel, one workgroup per token row of K = 8 * chunks values (K <= 16384):
 // y = fp16( float(x) * rsqrt(sum(x^2) / K + eps) [* float(weight)] ) with the statistics in float32
 // (flh/nn/normalization.py:12-20), then transform + quantise per group of G as group_kernel<G, HAD, true>.
-template <int G, bool HAD>
+template <int G, bool HAD, bool F6 = false>
 __global__ __launch_bounds__(256) void rmsnorm_group_kernel(const __half* __restrict__ x,
                                                             const __half* __restrict__ weight, uint8_t* __restrict__ q,
                                                             __half* __restrict__ scales, uint32_t K, float eps,
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(256) void rmsnorm_group_kernel(const __half* __rest
       }
       if constexpr (HAD) fwht_group_f16<G>(v, lir);
       const uint32_t row = token * (K / G) + c / LPR;
-      group_finish<G>(v, lir, true, row, q, scales, scale_mul);
+      group_finish<G, F6>(v, lir, true, row, q, scales, scale_mul, gridDim.x, K / G);   // (a quad is inside one group)
     }
   }
 }
@@ -969,6 +970,35 @@ extern "C" int flh_silu_mul_f16(const flh_half* gate, const flh_half* up, flh_ha
   hipLaunchKernelGGL(silu_mul_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                      (const __half*)gate, (const __half*)up, (__half*)out, n / 8);
   return check_launch("silu_mul_kernel");
+}
+
+// The two producers of the group configuration writing the 6-bit operand format: groups of 128, no rotation.  A pass that
+// re-encodes the nibbles costs 4-6 us per 1000 tokens in front of every GEMM.
+extern "C" int flh_rmsnorm_group_quant_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales,
+                                          uint32_t M, uint32_t K, float eps, void* stream) {
+  if (!x || !encoded || !scales) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: null pointer");
+  if (misaligned16(x, encoded) || (weight && misaligned16(weight)))
+    return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: x, weight and encoded must be 16-byte aligned");
+  if (!(eps >= 0.f)) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: eps must not be negative");
+  if (K == 0 || K % 128 || K > 16384u) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: K (%u) must be a multiple of 128, at most 16384", K);
+  if ((uint64_t)M * (K / 128) > 0xFFFFFFFFull) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: too many groups");
+  if (M == 0) return FLH_OK;
+  hipLaunchKernelGGL((rmsnorm_group_kernel<128, false, true>), dim3(M), dim3(256), 0, (hipStream_t)stream, (const __half*)x,
+                     (const __half*)weight, encoded, (__half*)scales, K, eps, 1.0f);
+  return check_launch("rmsnorm_group_kernel (6-bit output)");
+}
+
+extern "C" int flh_silu_mul_group_quant_f6(const flh_half* gate, const flh_half* up, uint8_t* encoded, flh_half* scales,
+                                           uint32_t M, uint32_t K, void* stream) {
+  if (!gate || !up || !encoded || !scales) return fail(FLH_EINVAL, "silu_mul_group_quant_f6: null pointer");
+  if (misaligned16(gate, up, encoded)) return fail(FLH_EINVAL, "silu_mul_group_quant_f6: gate, up and encoded must be 16-byte aligned");
+  if (K == 0 || K % 128) return fail(FLH_EINVAL, "silu_mul_group_quant_f6: K (%u) must be a positive multiple of 128", K);
+  if ((uint64_t)M * (K / 128) > 0x0FFFFFFFull) return fail(FLH_EINVAL, "silu_mul_group_quant_f6: too many groups");
+  if (M == 0) return FLH_OK;
+  const uint32_t R = M * (K / 128);
+  hipLaunchKernelGGL((silu_mul_group_kernel<128, false, true>), dim3((unsigned)(((uint64_t)R * 16 + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, (const __half*)gate, (const __half*)up, encoded, (__half*)scales, R, 1.0f, M, K / 128);
+  return check_launch("silu_mul_group_kernel (6-bit output)");
 }
 
 extern "C" int flh_embed_f16(const int64_t* ids, const flh_half* table, flh_half* out, uint32_t rows, uint32_t vocab,

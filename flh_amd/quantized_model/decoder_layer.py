@@ -232,6 +232,13 @@ class W4A4DecoderLayer(torch.nn.Module):
                 and width in self._F6_WIDTHS
                 and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers))
 
+    def _group_six_bit_for(self, consumers, n_rows, width):
+        """_six_bit_for of the group configuration: the consumers' codes and scales in groups of 128."""
+        return (bool(consumers) and self.activation == "group" and self.fused and self.record is None
+                and self.act_group_size == 128 and width % 128 == 0 and width <= 16384
+                and all(l.in_group_size == 128 and l.w_scale.numel() == l.out_features * (width // 128) > l.out_features
+                        and l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers))
+
     def _rotation_mode(self, rows, k):
         """hadamard argument of the whole-row ops for `rows` rows of k channels."""
         fast = self.fast_rotation and self.fused and self.record is None and k == 4096 and rows > 64
@@ -260,6 +267,10 @@ class W4A4DecoderLayer(torch.nn.Module):
     def _norm_quant(self, stage, norm, norm_name, quantizer, x, consumers=()):
         if self.activation == "token":
             return self._token_quant(stage, x, norm, norm_name, consumers)
+        if self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)):
+            q, s = _ops().rmsnorm_group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), self._norm_weight16(norm_name, norm),
+                                                    norm.eps)
+            return s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
         if self.fused:
             q, s = _ops().rmsnorm_and_quantize_i4_gs(x.reshape(-1, x.size(-1)).contiguous(),
                                                      self._norm_weight16(norm_name, norm), norm.eps,
@@ -402,7 +413,7 @@ class W4A4DecoderLayer(torch.nn.Module):
         """quantiser + o_proj on the attention output `out` [B, T, hidden]; (stream, block output or None, cache) as
         _attention returns them."""
         s, z, q = (self._token_quant("attn_out", out, consumers=(self.o_proj,)) if self.activation == "token"
-                   else self._group_quant("attn_out", self.attn_quantizer2, out))
+                   else self._group_quant("attn_out", self.attn_quantizer2, out, (self.o_proj,)))
         if fold_residual and self._residual_in_gemm(out.numel() // out.size(-1)):
             # prefill: the residual addition in o_proj's epilogue; nothing is left pending
             return self.o_proj(q, s, z, x_is_packed=True, residual=x), None, cache
@@ -491,7 +502,10 @@ class W4A4DecoderLayer(torch.nn.Module):
         cols = g.w_scale.view(g.out_features, -1).size(1)
         return g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
 
-    def _group_quant(self, stage, quantizer, x):
+    def _group_quant(self, stage, quantizer, x, consumers=()):
+        if self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)):
+            q, s = _ops().group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), False)
+            return s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
         s, z, q = quantizer(x)
         self._tap(stage + ".input", x.reshape(-1, x.size(-1)))
         self._tap(stage + ".codes", q.reshape(-1, q.size(-1)))
@@ -526,6 +540,9 @@ class W4A4DecoderLayer(torch.nn.Module):
             # (the library's product kernel when fused, so that every fused path sees the same fp16 product)
             mid = _ops().silu_mul(gate, up) if self.fused else torch.nn.functional.silu(gate) * up
             s, z, q = self._token_quant("mlp_mid", mid, consumers=(self.down_proj,))
+        elif self._group_six_bit_for((self.down_proj,), rows, gate.size(-1)):
+            q, s = _ops().silu_mul_group_quantize_f6(gate.reshape(rows, -1).contiguous(), up.reshape(rows, -1).contiguous())
+            s, z, q = s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
         elif self.fused and self.record is None:
             q, s = _ops().silu_mul_and_quantize_i4_gs(gate.contiguous(), up.contiguous(), self.act_group_size, False)
             z = None                                # (symmetric codes: no zero points to fill)

@@ -189,6 +189,14 @@ int flh_gemm_f6_i32(const uint8_t* A6, const uint8_t* B6, int32_t* C, size_t M, 
 int flh_group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard,
                        float scale_mul, void* stream);
 
+/* flh_rmsnorm_group_quant_i4 and flh_silu_mul_group_quant_i4 (groups of 128, no rotation, scale_mul 1) writing the 6-bit operand
+ * format: x, gate, up [M, K] -> encoded [M rows, K / 128 * 96 bytes] as flh_encode_f6 lays it out, scales [M, K / 128].  The
+ * bytes equal flh_encode_f6 of the nibble output, the scales are the same.  No counterpart in the reference. */
+int flh_rmsnorm_group_quant_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales, uint32_t M,
+                               uint32_t K, float eps, void* stream);
+int flh_silu_mul_group_quant_f6(const flh_half* gate, const flh_half* up, uint8_t* encoded, flh_half* scales, uint32_t M,
+                                uint32_t K, void* stream);
+
 /* The whole-row rotation + per-token quantiser writing the 6-bit operand format directly (no flh_encode_f6 pass):
  * encoded [M rows, K / 128 * 96 bytes] as flh_encode_f6 lays it out, scales [M].  hadamard FLH_HAD_NONE / FLH_HAD_F32 with
  * K = 512 .. 8192 a power of two, optionally with the prologues of flh_rmsnorm_rotate_quant_i4 (rmsnorm != 0; weight [K]

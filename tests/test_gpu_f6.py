@@ -170,3 +170,19 @@ def test_several_weight_matrices_in_one_launch(ops, m, ns, k, scales):
     single = ops.gemm_f6_dequant_o16 if scales == "rows" else ops.gemm_f6_dequant_o16_gs
     for D, B6, Bs in zip(got, B6s, Bss):
         assert torch.equal(D, single(A6, B6, As, Bs))
+
+
+@pytest.mark.parametrize("m,k", [(1, 128), (3, 384), (33, 4096), (70, 11008)])
+def test_group_producers_with_6bit_output(m, k):
+    """RMSNorm + quantiser and SwiGLU + quantiser writing the 6-bit format: the bytes of encode_f6 on their nibble output."""
+    from flh_amd import _ops as ops
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    x, up = (torch.randn(m, k, device="cuda", generator=gen).half() for _ in range(2))
+    w = (torch.rand(k, device="cuda", generator=gen) + 0.5).half()
+    for weight in (w, None):
+        q, s = ops.rmsnorm_and_quantize_i4_gs(x, weight, 1e-5, 128)
+        q6, s6 = ops.rmsnorm_group_quantize_f6(x, weight, 1e-5)
+        assert torch.equal(q6, ops.encode_f6(q)) and torch.equal(s6, s)
+    q, s = ops.silu_mul_and_quantize_i4_gs(x, up, 128)
+    q6, s6 = ops.silu_mul_group_quantize_f6(x, up)
+    assert torch.equal(q6, ops.encode_f6(q)) and torch.equal(s6, s)
