@@ -53,6 +53,23 @@ __device__ __forceinline__ void rope_pair(_Float16& x1, _Float16& x2, _Float16 c
   x2 = (_Float16)round_here((float)a2 + (float)r2);
 }
 
+// product of element H (0 / 1) of two fp16 pairs, exact in float32
+template <int H>
+__device__ __forceinline__ float mul_halves(unsigned a, unsigned b) {
+  float d;
+  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(d) : "v"(a), "v"(b));
+  else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+}
+// fma(v, element H of the fp16 pair s, acc)
+template <int H>
+__device__ __forceinline__ float fma_half(float v, unsigned s, float acc) {
+  float d;
+  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(v), "v"(s), "v"(acc));
+  else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(v), "v"(s), "v"(acc));
+  return d;
+}
+
 // Small-M (decode) kernels: weight-streaming, split over K inside a workgroup.
 constexpr int kDecodeMaxM = 64;
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group);

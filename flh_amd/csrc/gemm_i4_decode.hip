@@ -12,8 +12,14 @@
 // 4096 x 4096 weight matrix is requested at once, which is what a latency-bound stream needs.
 // Partial sums meet in LDS:
 //   * one scale per row: the eight waves' int32 tiles are added and dequantised;
-//   * scale groups of 128: every group's int32 tile is kept in LDS and the fp32 result is built
+//   * scale groups of 128: every group's tile is kept in LDS (as float32) and the fp32 result is built
 //     by one fused multiply-add per group in ascending order, exactly as the prefill kernel does.
+// What bounds it, beside the weights (in-kernel timestamps, 4096 x 14336 with group scales, 16 tokens, of 14.5 us): the scale
+// tables took 3.4 us before the first weight was requested and the fold 2.4 at the end.  The scales now come as they are, by
+// direct-to-LDS loads behind the first weights; tiles are stored as float32 by the waves that made them and folded without
+// bank conflicts, two groups of scales per read.  us, weights from HBM, before -> after: 16 tokens 4096 x 14336 (N x K) 16.5 ->
+// 14.2 (token scales 15.0 -> 12.7), 4096 x 11008 13.3 -> 11.4, 6144 x 4096 8.6 -> 7.9, 4096 x 4096 6.5 -> 5.8; one token 4096 x
+// 14336 12.3 -> 11.8 with token scales, 12.5 -> 12.9 with group scales.
 #include <atomic>
 #include "gemm_i4.h"
 #include "rotate_row.h"
@@ -64,26 +70,87 @@ __device__ __forceinline__ void store_f16(const GemmArgs& p, const DecodeWeights
   ((_Float16*)w.D)[at] = v;
 }
 
-// Partial sums in LDS -> outputs.  Lane l of a tile holds token l % 16 and channels 4 (l / 16) + i, i = 0..3.
-// a_scales: one scale per token (row-scale epilogue); sA / sB: the group tables (group epilogue).
+// Group scales wait in LDS as they are: row after row (the tokens if they have group scales, then the 16 channels) of KT
+// halves, an odd number of dwords apart.  They come by direct-to-LDS loads that are requested behind the first weights and waited for last;
+// rows that dword loads cannot fetch (an odd number of groups, an odd element offset, one scale per channel) are filled half by half.
+__host__ __device__ constexpr int scale_pitch(int KT) { return ((KT + 1) >> 1) | 1; }   // dwords per row
+
+__device__ __forceinline__ void request_scales(const GemmArgs& p, const DecodeWeights& w, unsigned* table, int KT, int tid) {
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pitch = scale_pitch(KT), tokens = p.a_cols > 1 ? p.M : 0, rows = tokens + 16;   // (at most 16 tokens)
+  auto row_of = [&](int row) {
+    return row < tokens ? p.As + (size_t)row * KT : w.Bs + (size_t)min(w.n0 + row - tokens, w.N - 1) * p.b_cols;
+  };
+  if (p.b_cols > 1 && ((uintptr_t)w.Bs & 3) == 0 && (tokens == 0 || ((uintptr_t)p.As & 3) == 0) && KT % 2 == 0) {
+    const float inv = 1.0f / (float)pitch;
+    const int total = rows * pitch;
+    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned*)table;
+    for (int f0 = wave * 64; f0 < total; f0 += kWaves * 64) {
+      const int f = min(f0 + lane, total - 1);
+      int row = (int)((float)f * inv);               // f < 2^12: off by one at most
+      row += (f >= (row + 1) * pitch ? 1 : 0) - (f < row * pitch ? 1 : 0);
+      load_to_lds4(row_of(row) + 2 * min(f - row * pitch, (KT >> 1) - 1), base + f0 * 4);
+    }
+  } else {
+    for (int i = tid; i < rows * KT; i += kWaves * 64) {
+      const int row = i / KT, g = i - row * KT;
+      ((__half*)(table + row * pitch))[g] = row_of(row)[row >= tokens && p.b_cols == 1 ? 0 : g];
+    }
+    if (KT % 2)
+      for (int row = tid; row < rows; row += kWaves * 64) ((__half*)(table + row * pitch))[KT] = __half(0.f);
+  }
+}
+// dwords of the table, rounded up to whole load instructions
+__host__ __device__ constexpr size_t scale_table_dwords(int KT) { return ((size_t)32 * scale_pitch(KT) + 63) / 64 * 64; }
+
+// The token's and, with one scale per row, the channel's scale of the value that thread `tid` finishes first: requested with the
+// weights, one latency less at the end.
+struct FirstScales {
+  float a, b;
+};
+template <int EPI>
+__device__ __forceinline__ FirstScales first_scales(const GemmArgs& p, const DecodeWeights& w, const __half* a_scales, int tid) {
+  const int gm = min((tid >> 8) * 16 + ((tid >> 2) & 15), p.M - 1), gn = min(w.n0 + ((tid >> 6) & 3) * 4 + (tid & 3), w.N - 1);
+  FirstScales f{0.f, 0.f};
+  if (a_scales && EPI != kInt32 && (EPI == kRowScale || p.a_cols == 1)) f.a = __half2float(a_scales[gm]);
+  if constexpr (EPI == kRowScale) f.b = __half2float(w.Bs[gn]);
+  return f;
+}
+
+// Partial sums in LDS -> outputs.  Lane l of a tile holds token l % 16 and channels 4 (l / 16) + i, i = 0..3; a thread
+// finishes the value at its own place of the tile (reads without bank conflicts).
+// Groups: float32 tiles of 256 x the sums, one fused multiply-add per group in ascending order, the exact 2^-8 at the end.
 template <int MT, int EPI>
-__device__ __forceinline__ void decode_finish(const GemmArgs& p, const DecodeWeights& w, const int* red, const float* sA,
-                                              const float* sB, const __half* a_scales, int tid) {
+__device__ __forceinline__ void decode_finish(const GemmArgs& p, const DecodeWeights& w, const int* red, const unsigned* table,
+                                              const __half* a_scales, const FirstScales& first, int tid) {
   const int KT = p.K >> 7;
   for (int idx = tid; idx < MT * 256; idx += kWaves * 64) {
-    const int mt = idx >> 8, m = (idx >> 4) & 15, n = idx & 15;
-    const int pos = (((n >> 2) * 16 + m) << 2) + (n & 3);
+    const int mt = idx >> 8, pos = idx & 255, m = (pos >> 2) & 15, n = (pos >> 6) * 4 + (pos & 3);
     const int gm = mt * 16 + m, gn = w.n0 + n;
     if (gm >= p.M || gn >= w.N) continue;
     if constexpr (EPI == kGroupScale) {
+      const int pitch = scale_pitch(KT);
+      const float* v = (const float*)red + mt * 256 + pos;
+      const bool token = p.a_cols == 1;
+      const unsigned *ra = table + m * pitch, *rb = table + ((token ? 0 : p.M) + n) * pitch;
       float out = 0.f;
-      if (p.a_cols == 1 && p.b_cols > 1) {           // one scale per token: applied once, after the groups
-        for (int g = 0; g < KT; ++g)
-          out = __builtin_fmaf((float)(red[(g * MT + mt) * 256 + pos] >> 8), sB[g * 16 + n], out);
-        out = round_here(out) * sA[m];
+      if (token) {                                   // one scale per token: applied once, after the groups
+        const float s_a = idx == tid ? first.a : __half2float(a_scales[gm]);
+#pragma unroll 8
+        for (int g = 0; g < KT / 2; ++g) {
+          out = fma_half<0>(v[2 * g * MT * 256], rb[g], out);
+          out = fma_half<1>(v[(2 * g + 1) * MT * 256], rb[g], out);
+        }
+        if (KT % 2) out = fma_half<0>(v[(KT - 1) * MT * 256], rb[KT / 2], out);
+        out = round_here(out * 0.00390625f) * s_a;
       } else {
-        for (int g = 0; g < KT; ++g)
-          out = __builtin_fmaf((float)(red[(g * MT + mt) * 256 + pos] >> 8), sA[g * 16 + m] * sB[g * 16 + n], out);
+#pragma unroll 8
+        for (int g = 0; g < KT / 2; ++g) {
+          out = __builtin_fmaf(v[2 * g * MT * 256], mul_halves<0>(ra[g], rb[g]), out);
+          out = __builtin_fmaf(v[(2 * g + 1) * MT * 256], mul_halves<1>(ra[g], rb[g]), out);
+        }
+        if (KT % 2) out = __builtin_fmaf(v[(KT - 1) * MT * 256], mul_halves<0>(ra[KT / 2], rb[KT / 2]), out);
+        out *= 0.00390625f;
       }
       store_f16(p, w, gm, gn, (_Float16)round_here(out));
     } else {
@@ -94,16 +161,19 @@ __device__ __forceinline__ void decode_finish(const GemmArgs& p, const DecodeWei
         ((int32_t*)w.D)[(size_t)gm * w.N + gn] = sum >> 8;
       } else {
         // sum = 256 * (exact contraction); the weight scale carries the matching exact 2^-8
-        const float sa = __half2float(a_scales[gm]), sb = __half2float(w.Bs[gn]) * 0.00390625f;
+        const float sa = idx == tid ? first.a : __half2float(a_scales[gm]);
+        const float sb = (idx == tid ? first.b : __half2float(w.Bs[gn])) * 0.00390625f;
         store_f16(p, w, gm, gn, (_Float16)round_here((float)sum * (sa * sb)));
       }
     }
   }
 }
 
+__device__ __forceinline__ v4f tile_as_float(const v4i& t) { return v4f{(float)t[0], (float)t[1], (float)t[2], (float)t[3]}; }
+
 template <int MT, int EPI>
 __global__ __launch_bounds__(kWaves * 64) void gemm_i4_decode_kernel(const GemmArgs p) {
-  extern __shared__ __align__(16) int red[];   // int32 tiles: [wave | group][MT][64 lanes][4]; then the scale tables
+  extern __shared__ __align__(16) int red[];   // tiles: [wave | group][MT][64 lanes][4], int32 | float32; then the scales
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
@@ -116,16 +186,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_decode_kernel(const GemmA
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) aptr[mt] = p.A + (size_t)min(mt * 16 + r, p.M - 1) * Kb + c * 16;
 
-  float* sA = (float*)(red + KT * MT * 256);    // group mode: scales as float, [g][16]
-  float* sB = sA + KT * 16;
-  if constexpr (EPI == kGroupScale) {
-    for (int i = tid; i < 16 * KT; i += kWaves * 64) {
-      const int row = i / KT, g = i - row * KT;
-      sA[g * 16 + row] = row < p.M ? __half2float(p.As[(size_t)row * p.a_cols + (p.a_cols > 1 ? g : 0)]) : 0.f;
-      sB[g * 16 + row] = n0 + row < w.N ? __half2float(w.Bs[(size_t)(n0 + row) * p.b_cols + (p.b_cols > 1 ? g : 0)]) : 0.f;
-    }
-  }
-
+  unsigned* table = (unsigned*)(red + KT * MT * 256);   // group mode
+  const FirstScales first = first_scales<EPI>(p, w, p.As, tid);
   v4i acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = v4i{0, 0, 0, 0};
@@ -154,7 +216,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_decode_kernel(const GemmA
         acc[mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bhi, ahi, acc[mt], 0, 0, 0);
         if constexpr (EPI == kGroupScale) {
           const int g = 2 * ds + half;
-          if (g < KT) *(v4i*)(red + ((g * MT + mt) * 64 + lane) * 4) = acc[mt];
+          if (g < KT) *(v4f*)(red + ((g * MT + mt) * 64 + lane) * 4) = tile_as_float(acc[mt]);
           acc[mt] = v4i{0, 0, 0, 0};
         }
       }
@@ -165,6 +227,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_decode_kernel(const GemmA
   v4i b0[2], b1[2], a0[MT][2], a1[MT][2];
   int ds = wave;
   if (ds < ND) load(ds, b0, a0);
+  if constexpr (EPI == kGroupScale) request_scales(p, w, table, KT, tid);
   for (; ds < ND; ds += 2 * kWaves) {
     const bool more = ds + kWaves < ND;
     if (more) load(ds + kWaves, b1, a1);
@@ -178,19 +241,20 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_decode_kernel(const GemmA
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) *(v4i*)(red + ((wave * MT + mt) * 64 + lane) * 4) = acc[mt];
   }
+  if constexpr (EPI == kGroupScale) wait_vmcnt<0>();     // the scales
   __syncthreads();
 
-  decode_finish<MT, EPI>(p, w, red, sA, sB, p.As, tid);
+  decode_finish<MT, EPI>(p, w, red, table, p.As, first, tid);
 }
 
 template <int MT, int EPI>
 int launch_decode(const GemmArgs& a, hipStream_t stream) {
   const int KT = a.K >> 7;
-  const size_t smem = EPI == kGroupScale ? (size_t)KT * MT * 1024 + (size_t)KT * 128 : (size_t)kWaves * MT * 1024;
+  const size_t smem = EPI == kGroupScale ? (size_t)KT * MT * 1024 + scale_table_dwords(KT) * 4 : (size_t)kWaves * MT * 1024;
   auto kern = gemm_i4_decode_kernel<MT, EPI>;
   if constexpr (EPI == kGroupScale) {
     static LdsGrant grant;                             // per instantiation; sized for the longest rows it takes
-    if (int rc = reserve_lds((const void*)kern, (size_t)kGroupMaxKT * MT * 1024 + (size_t)kGroupMaxKT * 128, grant, "gemm (decode)"))
+    if (int rc = reserve_lds((const void*)kern, (size_t)kGroupMaxKT * MT * 1024 + scale_table_dwords(kGroupMaxKT) * 4, grant, "gemm (decode)"))
       return rc;
   }
   GemmArgs g = a;
@@ -223,9 +287,9 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
   constexpr int K = 4096, Kb = K / 2, KT = K / 128, ND = KT / 2, NDW = ND / kWaves;
   constexpr int ROW = Kb + 16;                 // code rows 16 bytes apart in the banks
   constexpr int TILES = EPI == kGroupScale ? KT : 2 * kWaves;   // at least the 16 KB the rotation stages in
-  extern __shared__ __align__(16) int red[];   // int32 tiles [wave | group][64 lanes][4], sB [KT][16], sA [16], codes, scales
-  float* sB = (float*)(red + TILES * 256);
-  float* sA = sB + KT * 16;
+  extern __shared__ __align__(16) int red[];   // tiles [wave | group][64 lanes][4], channel scales, maxima, codes, token scales
+  unsigned* table = (unsigned*)(red + TILES * 256);
+  float* sA = (float*)(table + (EPI == kGroupScale ? scale_table_dwords(KT) : 0));   // scratch of the rotation
   uint8_t* codes = (uint8_t*)(sA + 16);
   __half* tok = (__half*)(codes + kRotateGemmMaxTokens * ROW);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -243,12 +307,8 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
     b[i][0] = *(const v4i*)(bptr + (size_t)ds * 128);
     b[i][1] = *(const v4i*)(bptr + (size_t)ds * 128 + 64);
   }
-  if constexpr (EPI == kGroupScale) {
-    for (int i = tid; i < 16 * KT; i += kWaves * 64) {
-      const int row = i / KT, g = i - row * KT;
-      sB[g * 16 + row] = n0 + row < w.N ? __half2float(w.Bs[(size_t)(n0 + row) * KT + g]) : 0.f;
-    }
-  }
+  if constexpr (EPI == kGroupScale) request_scales(p, w, table, KT, tid);
+  FirstScales first = first_scales<EPI>(p, w, nullptr, tid);
   for (int row = 0; row < p.M; ++row) {
     if constexpr (NORM || ADD)
       rotate_quant_row_8waves<NORM, ADD>(x + (size_t)row * K, (float*)red, sA, codes + row * ROW, tok + row, norm, wave,
@@ -258,7 +318,6 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
       rotate_quant_row_8waves(x + (size_t)row * K, (float*)red, sA, codes + row * ROW, tok + row, norm, wave);
   }
   __syncthreads();
-  if (tid < 16) sA[tid] = tid < p.M ? __half2float(tok[tid]) : 0.f;
 
   v4i acc = {0, 0, 0, 0};
   const uint8_t* arow = codes + min(r, p.M - 1) * ROW + c * 16;
@@ -273,20 +332,22 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
       acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(blo, alo, acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(bhi, ahi, acc, 0, 0, 0);
       if constexpr (EPI == kGroupScale) {
-        *(v4i*)(red + ((2 * ds + half) * 64 + lane) * 4) = acc;
+        *(v4f*)(red + ((2 * ds + half) * 64 + lane) * 4) = tile_as_float(acc);
         acc = v4i{0, 0, 0, 0};
       }
     }
   }
   if constexpr (EPI != kGroupScale) *(v4i*)(red + (wave * 64 + lane) * 4) = acc;
+  if constexpr (EPI == kGroupScale) wait_vmcnt<0>();     // the scales
   __syncthreads();
-  decode_finish<1, EPI>(p, w, red, sA, sB, tok, tid);
+  first.a = __half2float(tok[min((tid >> 2) & 15, p.M - 1)]);
+  decode_finish<1, EPI>(p, w, red, table, tok, first, tid);
 }
 
 template <int EPI>
 int launch_rotate_decode(const __half* x, const GemmArgs& a, hipStream_t stream, const DecodePrologue* pro = nullptr) {
   constexpr int K = 4096, KT = K / 128;
-  constexpr size_t smem = (size_t)(EPI == kGroupScale ? KT : 2 * kWaves) * 1024 + KT * 64 + 64 +
+  constexpr size_t smem = (size_t)(EPI == kGroupScale ? KT : 2 * kWaves) * 1024 + (EPI == kGroupScale ? scale_table_dwords(KT) * 4 : 0) + 64 +
                           kRotateGemmMaxTokens * (K / 2 + 16) + 32;
   static_assert(smem <= 64 * 1024, "fits the default dynamic LDS limit");
   GemmArgs g = a;

@@ -31,23 +31,6 @@ constexpr int kStageGroups = 4;                    // groups of 128 codes per st
 constexpr int kRowBytes = kStageGroups * 64;
 constexpr int kStreamMaxGroups = 128;              // scales of a row that fit beside the ring (K <= 16384)
 
-// product of element H (0 / 1) of two fp16 pairs, exact in float32
-template <int H>
-__device__ __forceinline__ float mul_halves(unsigned a, unsigned b) {
-  float d;
-  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(d) : "v"(a), "v"(b));
-  else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(d) : "v"(a), "v"(b));
-  return d;
-}
-// fma(v, element H of the fp16 pair s, acc)
-template <int H>
-__device__ __forceinline__ float fma_half(float v, unsigned s, float acc) {
-  float d;
-  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(v), "v"(s), "v"(acc));
-  else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(v), "v"(s), "v"(acc));
-  return d;
-}
-
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) uint8_t lds_byte;
