@@ -50,11 +50,15 @@ class LinearFLH(torch.nn.Module):
 
     # A call that encodes its weights for the 6-bit instruction first is faster from these rows on (one scale per channel, a
     # scale per group of 128) if it also has more 128 x 128 tiles than that -- less fills the chip with neither kernel, and the
-    # passes over the operands are all that differs.  us, encoding included, against the int8 kernels: group scales 2048 x 1024
-    # (rows x channels, K = 4096; 128 tiles) 30 against 24, 1024 x 4096 (256) 45 against 38, 1280 x 4096 (320) 47 against 52,
-    # 640 x 11008 (430) 65 against 58, 700 x 11008 (516) 76 against 81, 1024 x 14336 83 against 102; one scale per channel 2048 x 4096 (512) 41 against 34,
-    # 2048 x 11008 84 against 88, 3000 x 11008 106 against 126.
-    TRANSIENT_ROWS, TRANSIENT_TILES = (2560, 641), (512, 256)
+    # passes over the operands are all that differs; with group scales a long K needs fewer.  us, encoding included, against the
+    # int8 kernels: group scales 2048 x 1024 (rows x channels, K = 4096; 128 tiles) 30 against 24, 1024 x 4096 (256) 45 against
+    # 38, 1280 x 4096 (320) 47 against 52, 640 x 11008 (430) 65 against 58, 700 x 11008 (516) 76 against 81, 1024 x 14336 83
+    # against 102, 700 x 4096 (192) of K = 11008 76 against 78, of K = 14336 95 against 104; one scale per channel 2048 x 4096
+    # (512) 41 against 34, 2048 x 11008 84 against 88, 3000 x 11008 106 against 126.
+    TRANSIENT_ROWS = (2560, 641)
+
+    def _transient_tiles(self, grouped):
+        return 512 if not grouped else 256 if self.in_features <= 8192 else 191
 
     def _keeps_six_bit(self, grouped):
         return self.six_bit is True or (self.six_bit is not False and grouped)
@@ -65,7 +69,7 @@ class LinearFLH(torch.nn.Module):
         if self._keeps_six_bit(grouped):
             return self.six_bit_min_rows
         tiles = -(-(columns or self.out_features) // 128)
-        return max(self.TRANSIENT_ROWS[grouped], 128 * (self.TRANSIENT_TILES[grouped] // tiles) + 1)
+        return max(self.TRANSIENT_ROWS[grouped], 128 * (self._transient_tiles(grouped) // tiles) + 1)
 
     def prepare_six_bit(self):
         """Build the 6-bit encoding of the weights now if this layer's setting keeps one (at load time, rather than inside
