@@ -21,6 +21,18 @@ from ..nn.quantization import fast_hadamard_transform
 from .decoder_layer import StaticKVCache, W4A4DecoderLayer, rotary_tables
 
 
+def _stock_call(module, cls):
+    """Whether calling `module` is `cls.forward` on plain tensors and nothing else, so that a kernel of this library may stand in
+    for it: no hooks (the module's or global ones), no forward of its own, no trace, no forward-mode or functorch transform."""
+    g = torch.nn.modules.module
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                     or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                     or g._global_backward_pre_hooks)
+            and not torch.jit.is_tracing() and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._are_functorch_transforms_active())
+
+
 class LlamaShape:
     """The numbers that define a Llama-style stack."""
 
@@ -265,8 +277,8 @@ class W4A4LlamaModel(torch.nn.Module):
         -- unless the embedding is more than a look-up or takes part in a backward pass."""
         e = self.embed_tokens
         w = e.weight
-        plain = (type(self).embed is W4A4LlamaModel.embed and type(e) is torch.nn.Embedding and e.max_norm is None
-                 and not e._forward_hooks and not e._forward_pre_hooks and not (torch.is_grad_enabled() and w.requires_grad))
+        plain = (type(self).embed is W4A4LlamaModel.embed and _stock_call(e, torch.nn.Embedding) and e.max_norm is None
+                 and not (torch.is_grad_enabled() and w.requires_grad))
         if not (plain and self.fused and cache is not None and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
                 and w.data_ptr() % 16 == 0 and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0
                 and input_ids.is_cuda and input_ids.dtype == torch.int64 and positions.dtype == torch.int64
@@ -305,7 +317,7 @@ class W4A4LlamaModel(torch.nn.Module):
         fp16 product or takes part in a backward pass."""
         h = self.lm_head
         w = h.weight
-        if (self.fused and type(h) is torch.nn.Linear and h.bias is None and not h._forward_hooks and not h._forward_pre_hooks
+        if (self.fused and _stock_call(h, torch.nn.Linear) and h.bias is None
                 and 0 < x.numel() <= 16 * x.size(-1) and x.is_cuda and x.device == w.device and x.dtype == w.dtype == torch.float16
                 and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.size(1) == x.size(-1) and w.size(1) % 128 == 0
                 and not (torch.is_grad_enabled() and (w.requires_grad or x.requires_grad))

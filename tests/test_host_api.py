@@ -402,3 +402,30 @@ def test_model_checkpoint_directory_uses_the_references_key_names(tmp_path):
     del raw["model.layers.0.self_attn.k_proj.w_scale"]
     with pytest.raises(KeyError):
         W4A4LlamaModel(shape, activation="group", device="cpu").load_reference_state_dict(raw)
+
+
+def test_stock_call_refuses_modules_that_do_more():
+    """The model's head and embedding kernels stand in for a plain module call only."""
+    from flh_amd.quantized_model.llama import _stock_call
+    Linear = torch.nn.Linear
+    assert _stock_call(Linear(4, 4), Linear) and _stock_call(torch.nn.Embedding(4, 4), torch.nn.Embedding)
+    assert not _stock_call(type("Wrapped", (Linear,), {})(4, 4), Linear)
+    for register in ("register_forward_hook", "register_forward_pre_hook", "register_full_backward_hook"):
+        m = Linear(4, 4)
+        handle = getattr(m, register)(lambda *a: None)
+        assert not _stock_call(m, Linear), register
+        handle.remove()
+        assert _stock_call(m, Linear), register
+    m = Linear(4, 4)
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    try:
+        assert not _stock_call(m, Linear)
+    finally:
+        handle.remove()
+    with torch.autograd.forward_ad.dual_level():
+        assert not _stock_call(m, Linear)
+    seen = []
+    torch.func.vmap(lambda x: (seen.append(_stock_call(m, Linear)), x)[1])(torch.zeros(2, 4))
+    assert seen == [False] and _stock_call(m, Linear)
+    m.forward = lambda x: x
+    assert not _stock_call(m, Linear)
