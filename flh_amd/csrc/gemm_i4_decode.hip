@@ -14,12 +14,14 @@
 //   * one scale per row: the eight waves' int32 tiles are added and dequantised;
 //   * scale groups of 128: every group's tile is kept in LDS (as float32) and the fp32 result is built
 //     by one fused multiply-add per group in ascending order, exactly as the prefill kernel does.
-// What bounds it, beside the weights (in-kernel timestamps, 4096 x 14336 with group scales, 16 tokens, of 14.5 us): the scale
-// tables took 3.4 us before the first weight was requested and the fold 2.4 at the end.  The scales now come as they are, by
-// direct-to-LDS loads behind the first weights; tiles are stored as float32 by the waves that made them and folded without
-// bank conflicts, two groups of scales per read.  us, weights from HBM, before -> after: 16 tokens 4096 x 14336 (N x K) 16.5 ->
-// 14.2 (token scales 15.0 -> 12.7), 4096 x 11008 13.3 -> 11.4, 6144 x 4096 8.6 -> 7.9, 4096 x 4096 6.5 -> 5.8; one token 4096 x
-// 14336 12.3 -> 11.8 with token scales, 12.5 -> 12.9 with group scales.
+// What bounds it, beside the weights (in-kernel timestamps, 4096 x 14336 with group scales, 16 tokens, when it took 14.5 us):
+// the scale tables took 3.4 us before the first weight was requested and the fold 2.4 at the end.  The scales now come as they
+// are, by direct-to-LDS loads behind the first weights; tiles are stored as float32 by the waves that made them and folded
+// without bank conflicts, two groups of scales per read, eight pairs of groups read ahead of their multiply-adds (a pair at a
+// time the chain waits for LDS at every pair: one token 4096 x 14336 12.7 us with group scales where the eight take 10.9).
+// us, weights from HBM, against scales as float tables and integer tiles (N x K), token scales / group scales:
+//   16 tokens: 4096 x 14336 14.8 / 15.1 -> 11.4 / 11.5, 4096 x 11008 12.4 / 12.7 -> 9.9 / 9.8, 6144 x 4096 8.5 / 8.4 -> 7.4 /
+//   7.4, 4096 x 4096 6.5 / 6.6 -> 5.5 / 5.6;  one token: 4096 x 14336 11.9 / 12.0 -> 10.3 / 10.9, 4096 x 4096 5.7 / 5.7 -> 5.1 / 5.2
 #include <atomic>
 #include "gemm_i4.h"
 #include "rotate_row.h"
@@ -92,6 +94,7 @@ __device__ __forceinline__ void request_scales(const GemmArgs& p, const DecodeWe
       load_to_lds4(row_of(row) + 2 * min(f - row * pitch, (KT >> 1) - 1), base + f0 * 4);
     }
   } else {
+#pragma nounroll
     for (int i = tid; i < rows * KT; i += kWaves * 64) {
       const int row = i / KT, g = i - row * KT;
       ((__half*)(table + row * pitch))[g] = row_of(row)[row >= tokens && p.b_cols == 1 ? 0 : g];
@@ -117,39 +120,70 @@ __device__ __forceinline__ FirstScales first_scales(const GemmArgs& p, const Dec
   return f;
 }
 
+// out = fma(sum, scale, out) over the groups in ascending order: v[g * MT * 256] the sums, ra and rb the token's and the channel's
+// scales, two to a dword (TOKEN: the channel's alone).  Eight pairs of groups are read ahead of their multiply-adds, by hand:
+// a loop with inline assembly is not unrolled, and a pair at a time waits for LDS at every pair.
+template <int MT, bool TOKEN>
+__device__ __forceinline__ float fold_groups(const float* v, const unsigned* ra, const unsigned* rb, int KT) {
+  constexpr int kAhead = 8;
+  const int pairs = KT >> 1;
+  float out = 0.f;
+  auto fold = [&](float lo, float hi, unsigned a, unsigned b) {
+    if constexpr (TOKEN) {
+      out = fma_half<0>(lo, b, out);
+      out = fma_half<1>(hi, b, out);
+    } else {
+      out = __builtin_fmaf(lo, mul_halves<0>(a, b), out);
+      out = __builtin_fmaf(hi, mul_halves<1>(a, b), out);
+    }
+  };
+  auto batch = [&](int g, auto whole) {
+    constexpr bool WHOLE = decltype(whole)::value;
+    float lo[kAhead], hi[kAhead];
+    unsigned a[kAhead], b[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int at = WHOLE ? g + u : min(g + u, pairs - 1);
+      lo[u] = v[2 * at * MT * 256], hi[u] = v[(2 * at + 1) * MT * 256];
+      a[u] = TOKEN ? 0u : ra[at], b[u] = rb[at];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (WHOLE || g + u < pairs) fold(lo[u], hi[u], a[u], b[u]);
+  };
+  int g = 0;
+  for (; g + kAhead <= pairs; g += kAhead) batch(g, std::true_type{});
+  if (g < pairs) batch(g, std::false_type{});
+  if (KT & 1) {
+    const float last = v[(KT - 1) * MT * 256];
+    if constexpr (TOKEN) out = fma_half<0>(last, rb[pairs], out);
+    else out = __builtin_fmaf(last, mul_halves<0>(ra[pairs], rb[pairs]), out);
+  }
+  return out;
+}
+
 // Partial sums in LDS -> outputs.  Lane l of a tile holds token l % 16 and channels 4 (l / 16) + i, i = 0..3; a thread
 // finishes the value at its own place of the tile (reads without bank conflicts).
 // Groups: float32 tiles of 256 x the sums, one fused multiply-add per group in ascending order, the exact 2^-8 at the end.
-template <int MT, int EPI>
+// KTC: the groups of a row where they are known (one scale per token then, and the channels' rows of the table without padding).
+template <int MT, int EPI, int KTC = 0>
 __device__ __forceinline__ void decode_finish(const GemmArgs& p, const DecodeWeights& w, const int* red, const unsigned* table,
                                               const __half* a_scales, const FirstScales& first, int tid) {
-  const int KT = p.K >> 7;
+  const int KT = KTC ? KTC : p.K >> 7;
   for (int idx = tid; idx < MT * 256; idx += kWaves * 64) {
     const int mt = idx >> 8, pos = idx & 255, m = (pos >> 2) & 15, n = (pos >> 6) * 4 + (pos & 3);
     const int gm = mt * 16 + m, gn = w.n0 + n;
     if (gm >= p.M || gn >= w.N) continue;
     if constexpr (EPI == kGroupScale) {
-      const int pitch = scale_pitch(KT);
+      const int pitch = KTC ? KTC / 2 : scale_pitch(KT);
       const float* v = (const float*)red + mt * 256 + pos;
-      const bool token = p.a_cols == 1;
-      const unsigned *ra = table + m * pitch, *rb = table + ((token ? 0 : p.M) + n) * pitch;
-      float out = 0.f;
-      if (token) {                                   // one scale per token: applied once, after the groups
+      float out;
+      if (KTC || p.a_cols == 1) {                    // one scale per token: applied once, after the groups
         const float s_a = idx == tid ? first.a : __half2float(a_scales[gm]);
-#pragma unroll 8
-        for (int g = 0; g < KT / 2; ++g) {
-          out = fma_half<0>(v[2 * g * MT * 256], rb[g], out);
-          out = fma_half<1>(v[(2 * g + 1) * MT * 256], rb[g], out);
-        }
-        if (KT % 2) out = fma_half<0>(v[(KT - 1) * MT * 256], rb[KT / 2], out);
+        out = fold_groups<MT, true>(v, nullptr, table + n * pitch, KT);
         out = round_here(out * 0.00390625f) * s_a;
       } else {
-#pragma unroll 8
-        for (int g = 0; g < KT / 2; ++g) {
-          out = __builtin_fmaf(v[2 * g * MT * 256], mul_halves<0>(ra[g], rb[g]), out);
-          out = __builtin_fmaf(v[(2 * g + 1) * MT * 256], mul_halves<1>(ra[g], rb[g]), out);
-        }
-        if (KT % 2) out = __builtin_fmaf(v[(KT - 1) * MT * 256], mul_halves<0>(ra[KT / 2], rb[KT / 2]), out);
+        out = fold_groups<MT, false>(v, table + m * pitch, table + (p.M + n) * pitch, KT);
         out *= 0.00390625f;
       }
       store_f16(p, w, gm, gn, (_Float16)round_here(out));
@@ -289,7 +323,7 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
   constexpr int TILES = EPI == kGroupScale ? KT : 2 * kWaves;   // at least the 16 KB the rotation stages in
   extern __shared__ __align__(16) int red[];   // tiles [wave | group][64 lanes][4], channel scales, maxima, codes, token scales
   unsigned* table = (unsigned*)(red + TILES * 256);
-  float* sA = (float*)(table + (EPI == kGroupScale ? scale_table_dwords(KT) : 0));   // scratch of the rotation
+  float* sA = (float*)(table + (EPI == kGroupScale ? 16 * KT / 2 : 0));   // scratch of the rotation
   uint8_t* codes = (uint8_t*)(sA + 16);
   __half* tok = (__half*)(codes + kRotateGemmMaxTokens * ROW);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -307,7 +341,18 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
     b[i][0] = *(const v4i*)(bptr + (size_t)ds * 128);
     b[i][1] = *(const v4i*)(bptr + (size_t)ds * 128 + 64);
   }
-  if constexpr (EPI == kGroupScale) request_scales(p, w, table, KT, tid);
+  // The scales, 16 rows of 64 bytes one behind the other: one load instruction of one wave (with the other kernel's request, its
+  // divisions and its branch for rows of any kind, a token took 11.5 us through 6144 channels with the prologues; now 10.9).
+  if constexpr (EPI == kGroupScale) {
+    static_assert(kWaves * 64 == 16 * KT && KT == 32, "a load instruction, or a half per thread");
+    if (((uintptr_t)w.Bs & 15) == 0) {
+      if (wave == kWaves - 1)
+        load_to_lds16(w.Bs + (size_t)min(n0 + (lane >> 2), w.N - 1) * KT + (lane & 3) * 8,
+                      (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned*)table);
+    } else {
+      ((__half*)table)[tid] = w.Bs[(size_t)min(n0 + (tid >> 5), w.N - 1) * KT + (tid & 31)];
+    }
+  }
   FirstScales first = first_scales<EPI>(p, w, nullptr, tid);
   for (int row = 0; row < p.M; ++row) {
     if constexpr (NORM || ADD)
@@ -341,13 +386,13 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
   if constexpr (EPI == kGroupScale) wait_vmcnt<0>();     // the scales
   __syncthreads();
   first.a = __half2float(tok[min((tid >> 2) & 15, p.M - 1)]);
-  decode_finish<1, EPI>(p, w, red, table, tok, first, tid);
+  decode_finish<1, EPI, EPI == kGroupScale ? KT : 0>(p, w, red, table, tok, first, tid);
 }
 
 template <int EPI>
 int launch_rotate_decode(const __half* x, const GemmArgs& a, hipStream_t stream, const DecodePrologue* pro = nullptr) {
   constexpr int K = 4096, KT = K / 128;
-  constexpr size_t smem = (size_t)(EPI == kGroupScale ? KT : 2 * kWaves) * 1024 + (EPI == kGroupScale ? scale_table_dwords(KT) * 4 : 0) + 64 +
+  constexpr size_t smem = (size_t)(EPI == kGroupScale ? KT : 2 * kWaves) * 1024 + (EPI == kGroupScale ? 16 * KT * 2 : 0) + 64 +
                           kRotateGemmMaxTokens * (K / 2 + 16) + 32;
   static_assert(smem <= 64 * 1024, "fits the default dynamic LDS limit");
   GemmArgs g = a;

@@ -132,3 +132,32 @@ def test_norm_prologue_argument_errors(ops):
         ops.rmsnorm_rotate_quantize_gemm_i4_multi(x, x[:1], None, 1e-5, [B], [S])
     with pytest.raises(RuntimeError):
         ops.rmsnorm_rotate_quantize_gemm_i4_multi(x, None, torch.ones(100, dtype=torch.float16, device="cuda"), 1e-5, [B], [S])
+
+
+@pytest.mark.parametrize("m", [1, 3, 16])
+@pytest.mark.parametrize("a_token", [False, True])
+@pytest.mark.parametrize("groups", [1, 2, 3, 14, 16, 17, 18, 31, 34, 86, 127, 128])
+def test_fold_of_any_number_of_groups(ops, gemm_tuning, m, a_token, groups):
+    """The decode kernel reads eight pairs of groups ahead of their multiply-adds: counts around whole batches and odd ones,
+    against the same rows of a longer batch on the tile kernel (the same bits by the arithmetic)."""
+    k, n = 128 * groups, 40
+    w, s = weights(n, k, groups, seed=groups)
+    rng = np.random.default_rng(groups + m)
+    a = dev(rng.integers(0, 256, size=(32, k // 2), dtype=np.uint8))
+    sa = dev(rng.uniform(0.005, 0.02, size=(32, 1 if a_token else groups)).astype(np.float16))
+    wd, sd = dev(w), dev(s)
+    got = ops.gemm_i4_dequant(a[:m], wd, sa[:m], sd, 128)
+    gemm_tuning(64)
+    assert torch.equal(got, ops.gemm_i4_dequant(a, wd, sa, sd, 128)[:m])
+
+
+@pytest.mark.parametrize("offset", [1, 2, 8])
+@pytest.mark.parametrize("n", [40, 4096])
+def test_group_scales_at_any_element_offset(ops, n, offset):
+    """Sixteen-byte aligned scales come by one load instruction per workgroup, others half by half."""
+    w, s = weights(n, 4096, 32, seed=n)
+    x, wd, sd = dev(syn.activations(3, 4096, seed=offset)), dev(w), dev(s)
+    moved = torch.empty(n * 32 + offset, dtype=torch.float16, device="cuda")[offset:].view(n, 32)
+    moved.copy_(sd)
+    assert moved.data_ptr() % 16 == 2 * offset % 16
+    assert torch.equal(ops.rotate_quantize_gemm_i4(x, wd, moved), ops.rotate_quantize_gemm_i4(x, wd, sd))
