@@ -342,13 +342,30 @@ bool stream_takes(const GemmArgs& a, int epi, int group) {
   return true;
 }
 
+// Up to 16 tokens (K = 4096; us, this kernel against the decode kernel; one scale per row / token scales / group scales).
+//  * Up to 16384 channels, one workgroup of 64 per compute unit: beyond 12288, where the decode kernel has more than three of
+//    its workgroups on one (one token: x 13312 8.1 / 8.8 / 9.0 against 9.2 / 9.5 / 9.5, x 12288 7.8 / 8.6 / 8.8 against 7.6 /
+//    8.5 / 8.3), with five or more tokens from 172 workgroups on (16 x 11008 7.8 / 8.6 / 8.8 against 9.7 / 9.9 / 9.9, 5 x 11008
+//    7.6 / 8.4 / 8.7 against 8.0 / 8.6 / 8.3; 16 x 6144 with group scales 8.3 against 7.5).
+//  * Beyond, the compute units that get one workgroup more set the time and the decode kernel's grows with the channels: with
+//    few tokens only if the last round has enough workgroups (one token: x 17408 11.5 / 12.2 / 12.4 against 10.6 / 11.7 /
+//    10.7, x 22016 12.4 / 13.1 / 13.5 against 12.4 / 13.1 / 12.4, x 28672 13.9 / 14.7 / 15.0 against 15.2 / 16.0 / 14.6;
+//    5 x 18432 12.0 / 12.6 / 13.1 against 12.3 / 11.9 / 11.3, 8 x 18432 12.1 / 12.9 / 13.1 against 13.1 / 12.5 / 12.1).
+//    Not where the decode kernel's tiles of every group leave a compute unit one workgroup (one token x 22016, K = 11008,
+//    token scales: 30 against 41).
+bool takes_few_tokens(const GemmArgs& a, int epi, long columns) {
+  const bool row = epi == kRowScale, token = a.a_cols == 1;
+  if (columns <= 16384 || a.M > (row ? 4 : token ? 6 : 8) || (!row && a.K > 8192))
+    return a.M >= 5 ? columns >= 172 * 64 : columns > 12288;
+  const long last = (columns - 1) % 16384 + 1;             // channels of the last round
+  return last * 3 >= 16384 && (row || token || a.M > 6 || last >= 9830);   // a third, or six tenths
+}
+
 }  // namespace
 
 // Which launches are faster here than on the kernels on either side.  us, this kernel against the other (K = 4096 unless
 // stated; "large" counts 64 x 32 tiles):
-//  * up to 16 tokens, against the K split of the decode kernel: from 224 workgroups of 64 channels on (one token x 28672
-//    channels 15.4 against 17.0, x 14336 9.7 against 10.0), with five or more tokens from 172 (16 x 11008 9.4 against 11.4;
-//    one token x 12288 9.5 against 8.9, 16 x 6144 8.3 against 8.6).
+//  * up to 16 tokens, against the K split of the decode kernel: takes_few_tokens below.
 //  * 17 .. 64 tokens: always, but for one scale per row on at most 128 blocks of 32 channels, where the decode kernel takes 32
 //    (32 x 4096 6.0 against 6.3; 64 x 4096 8.3 against 6.5).
 //  * more, group-scaled weights, against 64 x 64 and 128 x 128 tiles: up to 768 large tiles, 512 if K is long (128 x 12288,
@@ -363,7 +380,7 @@ bool gemm_stream_supports(const GemmArgs& a, int epi, int group) {
   if (!stream_takes(a, epi, group) || g_tune_tile.load(std::memory_order_relaxed) || g_tune_ks.load(std::memory_order_relaxed))
     return false;
   const long columns = stream_columns(a);
-  if (a.M <= 16) return columns >= (a.M >= 5 ? 172 : 224) * 64;
+  if (a.M <= 16) return takes_few_tokens(a, epi, columns);
   if (a.M <= 64) return epi != kRowScale || a.M > 32 || columns > 128 * 32;
   if (a.M > (epi == kRowScale ? 512 : 1280)) return false;
   const long large = (long)((a.M + 63) / 64) * ((columns + 31) / 32);

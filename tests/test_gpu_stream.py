@@ -32,7 +32,7 @@ def operands(m, ns, k, kind, seed):
 
 KINDS = ["row", "token", "group"]
 # 16 x 64, 32 x 32 and 64 x 32 tiles; K of one stage, of stages the last of which is short, and the longest with a table
-SHAPES = [(5, 11010, 512), (16, 11013, 768), (1, 14336, 2816), (17, 36, 512), (33, 250, 768), (45, 1023, 11008), (64, 64, 16384),
+SHAPES = [(5, 11010, 512), (4, 12304, 512), (2, 17408, 512), (7, 22016, 512), (16, 11013, 768), (1, 14336, 2816), (17, 36, 512), (33, 250, 768), (45, 1023, 11008), (64, 64, 16384),
           (65, 100, 1280), (100, 1030, 1024), (127, 8200, 512), (250, 2090, 2816), (64, 20000, 768)]
 
 
