@@ -691,11 +691,13 @@ bool large_supported(const GemmArgs& a, bool grouped) {
 //    Of the two, a 256 x 128 tile takes 0.62 of the time of a 256 x 256 one; a round that is not full costs the mean of its
 //    share and a whole one, as the part clocks up (wide against narrow: 2048 x 28672, 3.5 rounds: 142 against 165; 2048 x
 //    4096, half a round: 30 against 25; 1531 x 6144, 0.56 of a round against 1.13: 34 against 39).
-//  * token scales: a round of 256 x 128 tiles takes 29.5, a round of 128 x 128 ones 16.6 (2048 x 28672: 208 against 223;
-//    1024 x 12288, 1.5 rounds of large tiles: 56 against 51).
-//  * group scales: from one 128 x 128 tile per compute unit on, a round of large tiles takes 31, the small ones 10 and 21.6
-//    more per round (1024 x 4096: 30 against 32; 2048 x 28672: 229 against 303; 640 x 11008, 258 large tiles, two rounds for
-//    one: 64 against 53).
+//  * token scales: a round of 256 x 128 tiles takes 23.7 and its tiles 6.2 a full round (3 once), of 128 x 128 ones 7.8 and 7.8
+//    (6 once; two share a compute unit, so a part of a round costs its part).  Large against small: 2048 x 28672 208 against
+//    223; 512 x 11008 32 against 34; 1024 x 12288, 1.5 rounds of large tiles, 56 against 51; 384 x 11008, 258 small tiles, 31.5
+//    against 29.2; 3000 x 11008, 1032 large tiles, 146 against 136; 2400 x 14336 157 against 141.
+//  * group scales: from one 128 x 128 tile per compute unit on, a round of large tiles takes 31, of small ones 21.6, and up to
+//    three rounds of them 10 more (1024 x 4096: 30 against 32; 2048 x 28672: 229 against 303; 640 x 11008, 258 large tiles, two
+//    rounds for one: 64 against 53; 1400 x 11008, 516 large tiles, three rounds against four small ones: 90 against 83).
 enum LargeTile { kNoLarge = 0, kWide = 1, kNarrow = 2 };
 LargeTile large_choice(const GemmArgs& a, int epi, long columns) {
   const bool grouped = epi != kRowScale;
@@ -706,8 +708,9 @@ LargeTile large_choice(const GemmArgs& a, int epi, long columns) {
   auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((columns + bn - 1) / bn); };
   auto rounds = [](long t) { return (t + 255) / 256; };
   const long small = tiles(128, 128), narrow = tiles(256, 128), wide = tiles(256, 256);
-  if (epi == kGroupScale) return small >= 256 && rounds(narrow) * 31.0 <= 10.0 + rounds(small) * 21.6 ? kNarrow : kNoLarge;
-  if (epi == kTokenGroup) return rounds(narrow) * 29.5 < rounds(small) * 16.6 ? kNarrow : kNoLarge;
+  if (epi == kGroupScale) return small >= 256 && rounds(narrow) * 31.0 <= (small <= 768 ? 10.0 : 0.0) + rounds(small) * 21.6 ? kNarrow : kNoLarge;
+  if (epi == kTokenGroup)
+    return 3.0 + 23.7 * rounds(narrow) + 6.2 * narrow / 256 < 6.0 + 7.8 * rounds(small) + 7.8 * small / 256 ? kNarrow : kNoLarge;
   if (small <= 256) return kNoLarge;
   auto cost = [&](long t) { return 0.5 * (rounds(t) + t / 256.0); };
   return cost(wide) <= 0.62 * cost(narrow) ? kWide : kNarrow;
