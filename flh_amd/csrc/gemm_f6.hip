@@ -684,36 +684,47 @@ bool large_supported(const GemmArgs& a, bool grouped) {
     if (off4(a.seg_Bs[s])) return false;
   return (uint64_t)(a.M > total_n_f6(a) ? a.M : total_n_f6(a)) * kt < (1ull << 31);
 }
-// Which large tile a launch over `columns` weight rows takes: 256 x 256 (kWide), 256 x 128 (kNarrow) or neither.  Measured
-// at M = 64 .. 4096 on the Llama widths with weights that come from HBM (us; K = 4096 unless stated):
-//  * one scale per row: as soon as 128 x 128 tiles would come more than one to a compute unit, a large tile is faster
-//    (1024 x 6144 tokens x channels: 25 against 29; 2048 x 4096: 25 against 27; 1024 x 4096, one tile each: 19 against 17).
-//    Of the two, a 256 x 128 tile takes 0.62 of the time of a 256 x 256 one; a round that is not full costs the mean of its
-//    share and a whole one, as the part clocks up (wide against narrow: 2048 x 28672, 3.5 rounds: 142 against 165; 2048 x
-//    4096, half a round: 30 against 25; 1531 x 6144, 0.56 of a round against 1.13: 34 against 39).
-//  * token scales: a round of 256 x 128 tiles takes 23.7 and its tiles 6.2 a full round (3 once), of 128 x 128 ones 7.8 and 7.8
-//    (6 once; two share a compute unit, so a part of a round costs its part).  Large against small: 2048 x 28672 208 against
-//    223; 512 x 11008 32 against 34; 1024 x 12288, 1.5 rounds of large tiles, 56 against 51; 384 x 11008, 258 small tiles, 31.5
-//    against 29.2; 3000 x 11008, 1032 large tiles, 146 against 136; 2400 x 14336 157 against 141.
-//  * group scales: from one 128 x 128 tile per compute unit on, a round of large tiles takes 31, of small ones 21.6, and up to
-//    three rounds of them 10 more (1024 x 4096: 30 against 32; 2048 x 28672: 229 against 303; 640 x 11008, 258 large tiles, two
-//    rounds for one: 64 against 53; 1400 x 11008, 516 large tiles, three rounds against four small ones: 90 against 83).
-enum LargeTile { kNoLarge = 0, kWide = 1, kNarrow = 2 };
-LargeTile large_choice(const GemmArgs& a, int epi, long columns) {
+// Which large tile a launch over `columns` weight rows takes: 256 x 256 (kWide), 256 x 128 (kNarrow) or neither.
+// Beyond 256 tiles of 128 x 128 the shape with the least of  once + per_round * rounds of 256 tiles + per_256 *
+// tiles / 256,  least squares over launches of M = 256 .. 5000 on the Llama widths (K = 4096, weights from HBM, us; longer K
+// scales all three alike).  The pick is within 2 % of the fastest shape on all but 2 of 260 launches (within 4 % there), those
+// of K = 11008 and 14336 included.  With the rotary epilogue, whose loads and index arithmetic the next tile does not cover in a
+// persistent workgroup, a large tile pays less; with token scales never there (700 x 6144 35 against 32, 4096 x 12288 208 against
+// 192); one scale per row and up to 512 tokens as without it (512 x 12288 32 against 34).  Group scales with exactly one small
+// tile per compute unit: the large one (1024 x 11008 x 4096 72 against 78); token scales with at most one large tile on each:
+// the large one unless hardly any compute unit would get a second small one (384 x 12288, 288 small tiles, 32.4 / 30.5).
+// Some of both sides, small / 256 x 128 / 256 x 256:
+//   one scale per row   640 x 11008 29.1 / 40.6 / 31.9, 2048 x 11008 76 / 67 / 68, 2400 x 4096 40 / 41 / 35;  with the rotary
+//                       epilogue 1000 x 6144 28.4 / 30.0 / 42.0, 2560 x 6144 57 / 59 / 53, 3000 x 6144 69 / 78 / 87
+//   token scales        384 x 11008 29.2 / 31.5, 512 x 11008 34 / 32, 3000 x 11008 136 / 146, 2048 x 28672 223 / 208
+//   group scales        1024 x 4096 32 / 30, 640 x 11008 53 / 64, 1400 x 11008 83 / 90, 2048 x 28672 303 / 229
+enum LargeTile { kNoLarge = 0, kNarrow = 1, kWide = 2 };
+struct LaunchCost {
+  double once, per_round, per_256;
+  double of(long tiles) const { return once + per_round * ((tiles + 255) / 256) + per_256 * tiles / 256; }
+};
+// [rotary epilogue][128 x 128, 256 x 128, 256 x 256]
+constexpr LaunchCost kRowCost[2][3] = {{{6.2, 6.3, 6.7}, {5.3, 11.1, 11.8}, {4.1, 21.5, 17.6}},
+                                       {{6.3, 8.6, 4.5}, {6.1, 18.1, 8.4}, {6.0, 30.6, 16.9}}};
+constexpr LaunchCost kTokenCost[2][2] = {{{6.1, 9.5, 6.2}, {5.1, 20.2, 9.9}}, {{6.2, 11.1, 4.5}, {5.7, 26.9, 5.9}}};
+constexpr LaunchCost kGroupCost[2][2] = {{{6.7, 16.6, 4.2}, {5.4, 22.9, 8.3}}, {{6.9, 17.6, 3.4}, {6.0, 29.3, 6.5}}};
+LargeTile large_choice(const GemmArgs& a, int epi, long columns, bool rope = false) {
   const bool grouped = epi != kRowScale;
   if (!large_supported(a, grouped)) return kNoLarge;
   const int forced = g_tune_tile.load(std::memory_order_relaxed);
   if (forced == 256) return grouped || g_tune_ks.load(std::memory_order_relaxed) == 2 ? kNarrow : kWide;
   if (forced) return kNoLarge;
   auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((columns + bn - 1) / bn); };
-  auto rounds = [](long t) { return (t + 255) / 256; };
-  const long small = tiles(128, 128), narrow = tiles(256, 128), wide = tiles(256, 256);
-  if (epi == kGroupScale) return small >= 256 && rounds(narrow) * 31.0 <= (small <= 768 ? 10.0 : 0.0) + rounds(small) * 21.6 ? kNarrow : kNoLarge;
-  if (epi == kTokenGroup)
-    return 3.0 + 23.7 * rounds(narrow) + 6.2 * narrow / 256 < 6.0 + 7.8 * rounds(small) + 7.8 * small / 256 ? kNarrow : kNoLarge;
-  if (small <= 256) return kNoLarge;
-  auto cost = [&](long t) { return 0.5 * (rounds(t) + t / 256.0); };
-  return cost(wide) <= 0.62 * cost(narrow) ? kWide : kNarrow;
+  const long small = tiles(128, 128), narrow = tiles(256, 128);
+  if (small <= 256) return epi == kGroupScale && small == 256 ? kNarrow : kNoLarge;
+  if (grouped) {
+    if (epi == kTokenGroup && !rope && narrow <= 256) return small > 272 ? kNarrow : kNoLarge;
+    const LaunchCost* cost = epi == kTokenGroup ? kTokenCost[rope] : kGroupCost[rope];
+    return cost[1].of(narrow) < cost[0].of(small) ? kNarrow : kNoLarge;
+  }
+  const LaunchCost* cost = kRowCost[rope && a.M > 512];
+  const double s = cost[0].of(small), n = cost[1].of(narrow), w = cost[2].of(tiles(256, 256));
+  return w <= n && w < s ? kWide : n < s ? kNarrow : kNoLarge;
 }
 // 128 x 128 tiles below that, down to 192 of them (with more than 64 rows; group scales on both sides: 224), else 64 x 64
 // (512 x 6144: 19 against 21 with row scales, 22 against 22 with token scales, 33 against 26 with group scales)
@@ -919,7 +930,7 @@ extern "C" int flh_gemm_f6_qkv_rope_o16(const uint8_t* A6, const flh_half* a_sca
   g.rope_T = (int)T;
   g.rope_max_len = (int)max_len;
   g.rope_hkv = (int)Hkv;
-  if (const LargeTile large = large_choice(g, rows_only ? kRowScale : a_cols == 1 ? kTokenGroup : kGroupScale, total_n_f6(g))) {
+  if (const LargeTile large = large_choice(g, rows_only ? kRowScale : a_cols == 1 ? kTokenGroup : kGroupScale, total_n_f6(g), true)) {
     if (rows_only) return f6l::launch_large_row(g, large == kWide, f6l::kRope, (hipStream_t)stream);
     return f6l::launch_large_group(g, a_cols == 1, f6l::kRope, (hipStream_t)stream);
   }
