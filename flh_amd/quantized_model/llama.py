@@ -276,10 +276,9 @@ class W4A4LlamaModel(torch.nn.Module):
         """embed(input_ids) and _rotary(positions, cache): one launch on the fused path with a static cache (the same bits)
         -- unless the embedding is more than a look-up or takes part in a backward pass."""
         e = self.embed_tokens
-        w = e.weight
-        plain = (type(self).embed is W4A4LlamaModel.embed and _stock_call(e, torch.nn.Embedding) and e.max_norm is None
-                 and not (torch.is_grad_enabled() and w.requires_grad))
-        if not (plain and self.fused and cache is not None and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
+        plain = type(self).embed is W4A4LlamaModel.embed and _stock_call(e, torch.nn.Embedding) and e.max_norm is None
+        w = e.weight if plain else None            # (another module need not have a weight)
+        if not (plain and self.fused and cache is not None and not (torch.is_grad_enabled() and w.requires_grad) and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
                 and w.data_ptr() % 16 == 0 and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0
                 and input_ids.is_cuda and input_ids.dtype == torch.int64 and positions.dtype == torch.int64
                 and positions.dim() == 1 and input_ids.numel() > 0):
@@ -316,9 +315,9 @@ class W4A4LlamaModel(torch.nn.Module):
         another order; the vendor's reads the weights at 5.7 TB/s, this one at 6.8) -- unless the head is more than a plain
         fp16 product or takes part in a backward pass."""
         h = self.lm_head
-        w = h.weight
-        if (self.fused and _stock_call(h, torch.nn.Linear) and h.bias is None
-                and 0 < x.numel() <= 16 * x.size(-1) and x.is_cuda and x.device == w.device and x.dtype == w.dtype == torch.float16
+        plain = self.fused and _stock_call(h, torch.nn.Linear) and h.bias is None
+        w = h.weight if plain else None            # (another module need not have a weight)
+        if (plain and 0 < x.numel() <= 16 * x.size(-1) and x.is_cuda and x.device == w.device and x.dtype == w.dtype == torch.float16
                 and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.size(1) == x.size(-1) and w.size(1) % 128 == 0
                 and not (torch.is_grad_enabled() and (w.requires_grad or x.requires_grad))
                 and not torch.is_autocast_enabled()):

@@ -429,3 +429,34 @@ def test_stock_call_refuses_modules_that_do_more():
     assert seen == [False] and _stock_call(m, Linear)
     m.forward = lambda x: x
     assert not _stock_call(m, Linear)
+
+
+class _Wrapped(torch.nn.Module):
+    """A module in the place of an embedding or a head that has no weight of its own."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, x):
+        return self.inner(x) + 1
+
+
+def _small_model():
+    from flh_amd.quantized_model import LlamaShape, W4A4LlamaModel
+    return W4A4LlamaModel(LlamaShape(128, 2, 1, 128, 1, 32), activation="token", device="cpu")
+
+
+@pytest.mark.parametrize("wrap", [_Wrapped, torch.nn.Sequential])
+@pytest.mark.parametrize("cached", [False, True])
+def test_model_with_another_head_or_embedding(wrap, cached):
+    """_head and _look_up call whatever module stands there."""
+    model = _small_model()
+    ids, positions = torch.tensor([[3, 5]]), torch.arange(2)
+    with torch.no_grad():
+        cache = model.new_cache(1, 4) if cached else None
+        x = torch.randn(1, 1, 128).half()
+        model.embed_tokens, model.lm_head = wrap(model.embed_tokens), wrap(model.lm_head)
+        assert torch.equal(model._head(x), model.lm_head(x))
+        got, cos, sin = model._look_up(ids, positions, cache)
+        assert torch.equal(got, model.embed_tokens(ids)) and cos.shape == sin.shape == (2, 64)
