@@ -15,6 +15,7 @@ import math
 import os
 
 import torch
+from torch.utils._device import DeviceContext
 
 from ..nn.normalization import RMSNorm
 from ..nn.quantization import fast_hadamard_transform
@@ -23,14 +24,17 @@ from .decoder_layer import StaticKVCache, W4A4DecoderLayer, rotary_tables
 
 def _stock_call(module, cls):
     """Whether calling `module` is `cls.forward` on plain tensors and nothing else, so that a kernel of this library may stand in
-    for it: no hooks (the module's or global ones), no forward of its own, no trace, no forward-mode or functorch transform."""
+    for it: no hooks (the module's or global ones), no forward of its own, no weight of another tensor class, no trace, no
+    forward-mode or functorch transform, no mode that sees torch's operations (a default device is none)."""
     g = torch.nn.modules.module
-    return (type(module) is cls and "forward" not in module.__dict__
+    return (type(module) is cls and "forward" not in module.__dict__ and module._compiled_call_impl is None
+            and type(getattr(module, "weight", None)) in (torch.nn.Parameter, torch.Tensor, type(None))
             and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
                      or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
                      or g._global_backward_pre_hooks)
             and not torch.jit.is_tracing() and torch.autograd.forward_ad._current_level < 0
-            and not torch._C._are_functorch_transforms_active())
+            and not torch._C._are_functorch_transforms_active() and not torch._C._len_torch_dispatch_stack()
+            and all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack()))
 
 
 class LlamaShape:
@@ -276,7 +280,8 @@ class W4A4LlamaModel(torch.nn.Module):
         """embed(input_ids) and _rotary(positions, cache): one launch on the fused path with a static cache (the same bits)
         -- unless the embedding is more than a look-up or takes part in a backward pass."""
         e = self.embed_tokens
-        plain = type(self).embed is W4A4LlamaModel.embed and _stock_call(e, torch.nn.Embedding) and e.max_norm is None
+        plain = (all(getattr(type(self), f) is getattr(W4A4LlamaModel, f) and f not in self.__dict__ for f in ("embed", "_rotary"))
+                 and _stock_call(e, torch.nn.Embedding) and e.max_norm is None)
         w = e.weight if plain else None            # (another module need not have a weight)
         if not (plain and self.fused and cache is not None and not (torch.is_grad_enabled() and w.requires_grad) and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
                 and w.data_ptr() % 16 == 0 and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0

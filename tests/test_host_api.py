@@ -460,3 +460,53 @@ def test_model_with_another_head_or_embedding(wrap, cached):
         assert torch.equal(model._head(x), model.lm_head(x))
         got, cos, sin = model._look_up(ids, positions, cache)
         assert torch.equal(got, model.embed_tokens(ids)) and cos.shape == sin.shape == (2, 64)
+
+
+def test_stock_call_refuses_other_tensors_and_modes():
+    """A weight of another tensor class, and modes that see torch's operations, get the module call; a default device is no such
+    mode."""
+    from flh_amd.quantized_model.llama import _stock_call
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Other(torch.Tensor):
+        pass
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    m = torch.nn.Linear(4, 4)
+    for mode in (Function(), Dispatch()):
+        with mode:
+            assert not _stock_call(m, torch.nn.Linear)
+    with torch.device("cpu"):
+        assert _stock_call(m, torch.nn.Linear)
+    m.weight = torch.nn.Parameter(m.weight.detach().as_subclass(Other))
+    assert not _stock_call(m, torch.nn.Linear)
+
+
+@pytest.mark.parametrize("name", ["embed", "_rotary"])
+@pytest.mark.parametrize("on_instance", [False, True])
+def test_look_up_calls_a_method_of_its_own(monkeypatch, name, on_instance):
+    """A model that overrides embed or _rotary, in a subclass or on the object, has them called."""
+    import flh_amd.quantized_model.llama as llama
+    model, called = _small_model(), []
+    stock = getattr(llama.W4A4LlamaModel, name)
+
+    def own(*args):
+        called.append(name)
+        return stock(model, *args[-(1 if name == "embed" else 2):])
+    if on_instance:
+        setattr(model, name, own)
+    else:
+        model.__class__ = type("Sub", (llama.W4A4LlamaModel,), {name: own})
+    seen = []
+    monkeypatch.setattr(llama, "_stock_call", lambda *a: (seen.append(a), True)[1])   # would the kernel stand in?
+    with torch.no_grad():
+        model._look_up(torch.tensor([[3]]), torch.arange(1), model.new_cache(1, 4))
+    assert called == [name] and not seen
