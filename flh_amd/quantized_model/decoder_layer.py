@@ -28,6 +28,7 @@ launches and, for one or two tokens, the o_proj quantiser inside its GEMM.
 are stored in it (by stage name) -- the taps the parity tests compare with the CPU oracle stage by stage.
 """
 import torch
+from torch.utils._device import DeviceContext
 
 from ..nn.linear import LinearFLH
 from ..nn.normalization import RMSNorm
@@ -120,6 +121,21 @@ class StaticKVCache:
 
     def layer(self, index):
         return StaticKVCache._Layer(self, index)
+
+
+def _stock_call(module, cls):
+    """Whether calling `module` is `cls.forward` on plain tensors and nothing else, so that a kernel of this library may stand in
+    for it: no hooks (the module's or global ones), no forward of its own, no weight of another tensor class, no trace, no
+    forward-mode or functorch transform, no mode that sees torch's operations (a default device is none)."""
+    g = torch.nn.modules.module
+    return (type(module) is cls and "forward" not in module.__dict__ and module._compiled_call_impl is None
+            and type(getattr(module, "weight", None)) in (torch.nn.Parameter, torch.Tensor, type(None))
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                     or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                     or g._global_backward_pre_hooks)
+            and not torch.jit.is_tracing() and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._are_functorch_transforms_active() and not torch._C._len_torch_dispatch_stack()
+            and all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack()))
 
 
 class W4A4DecoderLayer(torch.nn.Module):
@@ -503,7 +519,9 @@ class W4A4DecoderLayer(torch.nn.Module):
         return g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
 
     def _group_quant(self, stage, quantizer, x, consumers=()):
-        if self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)):
+        if (self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)) and _stock_call(quantizer, ActQuantizer)
+                and not quantizer.use_hadamard and not quantizer.per_token):
+            # (a quantiser that does more, or something else, is called: its consumers re-encode its codes)
             q, s = _ops().group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), False)
             return s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
         s, z, q = quantizer(x)

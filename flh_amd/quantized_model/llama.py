@@ -15,26 +15,10 @@ import math
 import os
 
 import torch
-from torch.utils._device import DeviceContext
 
 from ..nn.normalization import RMSNorm
 from ..nn.quantization import fast_hadamard_transform
-from .decoder_layer import StaticKVCache, W4A4DecoderLayer, rotary_tables
-
-
-def _stock_call(module, cls):
-    """Whether calling `module` is `cls.forward` on plain tensors and nothing else, so that a kernel of this library may stand in
-    for it: no hooks (the module's or global ones), no forward of its own, no weight of another tensor class, no trace, no
-    forward-mode or functorch transform, no mode that sees torch's operations (a default device is none)."""
-    g = torch.nn.modules.module
-    return (type(module) is cls and "forward" not in module.__dict__ and module._compiled_call_impl is None
-            and type(getattr(module, "weight", None)) in (torch.nn.Parameter, torch.Tensor, type(None))
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
-                     or g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
-                     or g._global_backward_pre_hooks)
-            and not torch.jit.is_tracing() and torch.autograd.forward_ad._current_level < 0
-            and not torch._C._are_functorch_transforms_active() and not torch._C._len_torch_dispatch_stack()
-            and all(type(m) is DeviceContext for m in torch.overrides._get_current_function_mode_stack()))
+from .decoder_layer import StaticKVCache, W4A4DecoderLayer, _stock_call, rotary_tables
 
 
 class LlamaShape:

@@ -510,3 +510,26 @@ def test_look_up_calls_a_method_of_its_own(monkeypatch, name, on_instance):
     with torch.no_grad():
         model._look_up(torch.tensor([[3]]), torch.arange(1), model.new_cache(1, 4))
     assert called == [name] and not seen
+
+
+@pytest.mark.parametrize("change", ["hook", "replaced", "rotating", "per_token", "none"])
+def test_long_blocks_call_the_attention_output_quantizer(monkeypatch, change):
+    """The 6-bit quantiser stands in for attn_quantizer2 only if that is the plain one without a rotation."""
+    import flh_amd
+    layer, calls = _small_model().layers[0], []
+    layer.activation = "group"
+    monkeypatch.setattr(type(layer), "_group_six_bit_for", lambda self, *a: True)
+    codes, scales = torch.zeros(4, 64, dtype=torch.uint8), torch.zeros(4, 1).half()
+
+    class Ops:
+        group_quantize_f6 = staticmethod(lambda x, hadamard: (calls.append("six_bit"), (torch.zeros(4, 96, dtype=torch.uint8), scales))[1])
+        quantize_rows = quantize_groups = staticmethod(lambda *a: (calls.append("module"), (scales, codes))[1])
+    monkeypatch.setattr(flh_amd, "_CUDA", Ops)
+    if change == "hook":
+        layer.attn_quantizer2.register_forward_hook(lambda *a: None)
+    elif change == "replaced":
+        layer.attn_quantizer2 = type("Own", (ActQuantizer,), {})(bits=4, group_size=128, use_hadamard=False, packed_output=True)
+    elif change != "none":
+        setattr(layer.attn_quantizer2, {"rotating": "use_hadamard"}.get(change, change), True)
+    layer._group_quant("attn_out", layer.attn_quantizer2, torch.zeros(4, 128).half(), (layer.o_proj,))
+    assert calls == ["six_bit" if change == "none" else "module"]
