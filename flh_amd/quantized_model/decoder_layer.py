@@ -220,13 +220,14 @@ class W4A4DecoderLayer(torch.nn.Module):
             self.record[name] = value.clone()      # a copy: q is rotated in place later on
 
     def _norm_weight16(self, name, norm):
-        """The norm weight as the fused kernels take it (fp16; exact for weights that came from an fp16 checkpoint),
-        converted once per version of the parameter."""
+        """The norm weight as the fused kernels take it (fp16, 16-byte aligned; exact for weights that came from an fp16
+        checkpoint), converted once per version of the parameter."""
         w = norm.weight
         key = (w.data_ptr(), w._version)
         hit = self._norm16.get(name)
         if hit is None or hit[0] != key:
-            hit = (key, w.detach().to(torch.float16).contiguous())
+            w16 = w.detach().to(torch.float16).contiguous()
+            hit = (key, w16 if w16.data_ptr() % 16 == 0 else w16.clone())
             self._norm16[name] = hit
         return hit[1]
 

@@ -533,3 +533,12 @@ def test_long_blocks_call_the_attention_output_quantizer(monkeypatch, change):
         setattr(layer.attn_quantizer2, {"rotating": "use_hadamard"}.get(change, change), True)
     layer._group_quant("attn_out", layer.attn_quantizer2, torch.zeros(4, 128).half(), (layer.o_proj,))
     assert calls == ["six_bit" if change == "none" else "module"]
+
+
+def test_norm_weight_at_any_offset_reaches_the_kernels_aligned():
+    """An fp16 norm weight that is a view at an odd element offset of a larger buffer."""
+    layer = _small_model().layers[0]
+    layer.input_layernorm.weight = torch.nn.Parameter(torch.rand(129).half()[1:])
+    w = layer._norm_weight16("input_layernorm", layer.input_layernorm)
+    assert layer.input_layernorm.weight.data_ptr() % 16 and w.data_ptr() % 16 == 0
+    assert torch.equal(w, layer.input_layernorm.weight)
