@@ -35,8 +35,9 @@ class LinearFLH(torch.nn.Module):
         # Prefill-sized calls run on the 6-bit matrix instruction where that is faster (extension; same bits, no unpack in the
         # loop).  Its operands are re-encoded at 6 bits per code, 0.75 byte per weight next to the 0.5 of `w_packed`.
         # False (default): nothing is kept; a call of at least TRANSIENT_ROWS rows encodes its weights into a buffer that
-        # goes back with the call.  True: the layer keeps the encoding (2.5 x the weight memory) and every call of at
-        # least `six_bit_min_rows` rows uses it.  "auto" (or None): kept for weights with a scale per group of 128.
+        # goes back with the call.  "never": not even that, for callers without that memory to spare.  True: the layer keeps
+        # the encoding (2.5 x the weight memory) and every call of at least `six_bit_min_rows` rows uses it.  "auto" (or
+        # None): kept for weights with a scale per group of 128.
         # `prepare_six_bit()` builds the kept encoding at once (a loader calls it); otherwise it is built on first use.  It
         # is rebuilt whenever `w_packed` has been written to or replaced (in-place copies, load_state_dict, .to(device)):
         # keyed on the buffer's storage address and version counter.
@@ -56,16 +57,19 @@ class LinearFLH(torch.nn.Module):
     # against 102, 700 x 4096 (192) of K = 11008 76 against 78, of K = 14336 95 against 104; one scale per channel 2048 x 4096
     # (512) 41 against 34, 2048 x 11008 84 against 88, 3000 x 11008 106 against 126.
     TRANSIENT_ROWS = (2560, 641)
+    _NO_ROWS = 1 << 62                             # more rows than any call has
 
     def _transient_tiles(self, grouped):
         return 512 if not grouped else 256 if self.in_features <= 8192 else 191
 
     def _keeps_six_bit(self, grouped):
-        return self.six_bit is True or (self.six_bit is not False and grouped)
+        return self.six_bit is True or (self.six_bit not in (False, "never") and grouped)
 
     def _six_bit_rows(self, grouped, columns=None):
         """Rows from which a launch over `columns` channels (this layer's, unless it shares the launch) takes the 6-bit
         instruction."""
+        if self.six_bit == "never":
+            return self._NO_ROWS
         if self._keeps_six_bit(grouped):
             return self.six_bit_min_rows
         tiles = -(-(columns or self.out_features) // 128)

@@ -185,8 +185,9 @@ class W4A4DecoderLayer(torch.nn.Module):
         `input_layernorm` / `post_attention_layernorm` [hidden]; quantised round-to-nearest ("group": as they are,
         "token": after the rotation of their input side).  weight_group_size: None = 128 for "group" and one scale
         per output channel for "token"; 128 with "token" is the Llama-3 arrangement; <= 0 one scale per channel.
-        six_bit: LinearFLH.six_bit of the seven projections -- False (default), True or "auto" (group-scaled weights);
-        anything but False costs a second copy of the weights (2.5 x the weight memory), built here."""
+        six_bit: LinearFLH.six_bit of the seven projections -- False (default), "never", True or "auto" (group-scaled
+        weights); the last two cost a second copy of the weights (2.5 x the weight memory), built here, and False a
+        temporary one of a launch's weights in a long call."""
         hidden, inter = weights["q_proj"].size(1), weights["gate_proj"].size(0)
         device = weights["q_proj"].device
         if weight_group_size is None:
@@ -234,8 +235,8 @@ class W4A4DecoderLayer(torch.nn.Module):
     _F6_WIDTHS = (512, 1024, 2048, 4096, 8192, 11008, 14336)
 
     def set_six_bit(self, six_bit):
-        """LinearFLH.six_bit of the seven projections (False, True, or "auto" / None), with the second encoding of the
-        weights built at once where the setting can use it."""
+        """LinearFLH.six_bit of the seven projections (False, "never", True, or "auto" / None), with the second encoding of
+        the weights built at once where the setting keeps one."""
         for name in self.PROJECTIONS:
             lin = getattr(self, name)
             lin.six_bit = None if six_bit == "auto" else six_bit

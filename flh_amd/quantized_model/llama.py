@@ -226,10 +226,11 @@ class W4A4LlamaModel(torch.nn.Module):
         return model
 
     def set_six_bit(self, six_bit):
-        """Whether prefill-sized calls of the layers' linears run on the 6-bit matrix instruction: False (default), True,
-        or "auto" (only where it pays even with a re-encoding pass: weights with a scale per group of 128).  Anything but
-        False makes every such linear hold a second, 6-bit copy of its weights -- 0.75 byte per weight on top of 0.5,
-        about + 5 GB for a 7B model -- which is built here, not inside the first long call."""
+        """How prefill-sized calls of the layers' linears come by the operands of the 6-bit matrix instruction.  False (default):
+        long calls encode the weights of a launch for themselves, 0.75 byte per weight for as long as the launch takes
+        (gate and up of a 4096 x 14336 MLP: 88 MB).  "never": they do not, and stay on the int8 instruction.  True, or "auto"
+        (only weights with a scale per group of 128): every such linear holds a second, 6-bit copy of its weights -- 0.75
+        byte per weight on top of 0.5, about + 5 GB for a 7B model -- which is built here, not inside the first long call."""
         for layer in self.layers:
             layer.set_six_bit(six_bit)
 

@@ -542,3 +542,16 @@ def test_norm_weight_at_any_offset_reaches_the_kernels_aligned():
     w = layer._norm_weight16("input_layernorm", layer.input_layernorm)
     assert layer.input_layernorm.weight.data_ptr() % 16 and w.data_ptr() % 16 == 0
     assert torch.equal(w, layer.input_layernorm.weight)
+
+
+@pytest.mark.parametrize("group", [128, 4096])
+def test_six_bit_never(group):
+    """six_bit = "never": no number of rows takes the 6-bit instruction, and nothing is kept; False: long calls do."""
+    lin = LinearFLH(4096, 11008, device="meta", in_group_size=128, group_size=group)
+    grouped = group == 128
+    rows = lambda: lin._six_bit_rows(grouped)
+    assert lin.six_bit is False and rows() < 10000 and not lin._keeps_six_bit(grouped)
+    lin.six_bit = "never"
+    assert rows() > 2 ** 40 and lin._few_rows(lin.w_scale) == rows() and not lin._keeps_six_bit(grouped)
+    lin.six_bit = "auto"
+    assert lin._keeps_six_bit(grouped) is grouped
