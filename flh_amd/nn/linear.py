@@ -90,6 +90,8 @@ class LinearFLH(torch.nn.Module):
             self._w6_key = key
         return self._w6
 
+    _SIX_BIT_MAX_ROWS = ((1 << 32) - 1) // 96       # rows of either operand that the 6-bit launches index; more go to int8
+
     def wants_six_bit(self, n_rows, columns=None):
         """Whether a call with `n_rows` per-token-quantised rows takes the 6-bit matrix instruction (a producer can then
         write the activations in that format directly, rotate_and_quantize_f6).  `columns`: channels of the whole launch,
@@ -99,7 +101,7 @@ class LinearFLH(torch.nn.Module):
         cols = self.w_scale.view(self.out_features, -1).size(1)
         if cols != 1 and not (cols == self.in_features // 128 and self.weight_group_size == 128):
             return False
-        return n_rows >= self._six_bit_rows(cols != 1, columns)
+        return self._six_bit_rows(cols != 1, columns) <= n_rows <= self._SIX_BIT_MAX_ROWS
 
     def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)
@@ -107,7 +109,7 @@ class LinearFLH(torch.nn.Module):
             return False
         per_row = a_scale.size(1) == 1 and w_scale.size(1) == 1
         grouped = group == 128 and w_scale.size(1) == self.in_features // 128 and a_scale.size(1) in (1, w_scale.size(1))
-        return (grouped or per_row) and n >= self._six_bit_rows(not per_row, columns)
+        return (grouped or per_row) and self._six_bit_rows(not per_row, columns) <= n <= self._SIX_BIT_MAX_ROWS
 
     def _group(self):
         return self.weight_group_size if self.weight_group_size > 0 else (self.in_group_size or 128)

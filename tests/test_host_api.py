@@ -555,3 +555,13 @@ def test_six_bit_never(group):
     assert rows() > 2 ** 40 and lin._few_rows(lin.w_scale) == rows() and not lin._keeps_six_bit(grouped)
     lin.six_bit = "auto"
     assert lin._keeps_six_bit(grouped) is grouped
+
+
+@pytest.mark.parametrize("n,takes", [(44739242, True), (44739243, False)])
+def test_rows_beyond_the_six_bit_launches_stay_on_int8(n, takes):
+    """The 6-bit launches index 2^32 / 96 rows, the int8 ones 4 GiB of codes: more rows of K = 128."""
+    class Rows:
+        is_cuda, size = True, staticmethod(lambda d: n if d == 0 else 64)
+    lin = LinearFLH(128, 1024, device="meta", in_group_size=128, group_size=128)
+    scales = torch.empty(1, 1, device="meta")
+    assert lin._six_bit_applies(Rows, scales.expand(n, 1), scales.expand(1024, 1), 128) is takes
