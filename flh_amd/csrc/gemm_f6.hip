@@ -690,8 +690,9 @@ bool large_supported(const GemmArgs& a, bool grouped) {
 // scales all three alike).  The pick is within 2 % of the fastest shape on all but 2 of 260 launches (within 4 % there), those
 // of K = 11008 and 14336 included.  With the rotary epilogue, whose loads and index arithmetic the next tile does not cover in a
 // persistent workgroup, a large tile pays less; with token scales never there (700 x 6144 35 against 32, 4096 x 12288 208 against
-// 192); one scale per row and up to 512 tokens as without it (512 x 12288 32 against 34).  Group scales with exactly one small
-// tile per compute unit: the large one (1024 x 11008 x 4096 72 against 78); token scales with at most one large tile on each:
+// 192); one scale per row and up to 512 tokens as without it (512 x 12288 32 against 34).  Group scales with 224 .. 256 small
+// tiles: the large ones, except with the rotary epilogue (1024 x 11008 x 4096 72 against 78, 640 x 4096 x 6144 33 against 34.5,
+// 256 x 4096 x 14336 32 against 34.5;  640 x 6144 with it 39 against 36); token scales with at most one large tile on each:
 // the large one unless hardly any compute unit would get a second small one (384 x 12288, 288 small tiles, 32.4 / 30.5).
 // Some of both sides, small / 256 x 128 / 256 x 256:
 //   one scale per row   640 x 11008 29.1 / 40.6 / 31.9, 2048 x 11008 76 / 67 / 68, 2400 x 4096 40 / 41 / 35;  with the rotary
@@ -716,7 +717,7 @@ LargeTile large_choice(const GemmArgs& a, int epi, long columns, bool rope = fal
   if (forced) return kNoLarge;
   auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((columns + bn - 1) / bn); };
   const long small = tiles(128, 128), narrow = tiles(256, 128);
-  if (small <= 256) return epi == kGroupScale && small == 256 ? kNarrow : kNoLarge;
+  if (small <= 256) return epi == kGroupScale && small >= 224 && !rope ? kNarrow : kNoLarge;
   if (grouped) {
     if (epi == kTokenGroup && !rope && narrow <= 256) return small > 272 ? kNarrow : kNoLarge;
     const LaunchCost* cost = epi == kTokenGroup ? kTokenCost[rope] : kGroupCost[rope];
