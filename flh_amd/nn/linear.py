@@ -50,30 +50,37 @@ class LinearFLH(torch.nn.Module):
         self._w6 = self._w6_key = None
 
     # A call that encodes its weights for the 6-bit instruction first is faster from these rows on (one scale per channel, a
-    # scale per group of 128) if it also has more 128 x 128 tiles than that -- less fills the chip with neither kernel, and the
-    # passes over the operands are all that differs; with group scales a long K needs fewer.  us, encoding included, against the
-    # int8 kernels: group scales 2048 x 1024 (rows x channels, K = 4096; 128 tiles) 30 against 24, 1024 x 4096 (256) 45 against
-    # 38, 1280 x 4096 (320) 47 against 52, 640 x 11008 (430) 65 against 58, 700 x 11008 (516) 76 against 81, 1024 x 14336 83
-    # against 102, 700 x 4096 (192) of K = 11008 76 against 78, of K = 14336 95 against 104; one scale per channel 2048 x 4096
-    # (512) 41 against 34, 2048 x 11008 84 against 88, 3000 x 11008 106 against 126.
+    # scale per group of 128) if it also has more 128 x 128 tiles than _transient_tiles -- less fills the chip with neither
+    # kernel, and the passes over the operands are all that differs; with group scales a long K needs fewer, with one scale per
+    # channel packed codes, which are encoded as well, more.  us, all encodings included, against the int8 kernels (rows x
+    # channels, K = 4096 unless stated, tiles):
+    #   group scales, packed codes: 2048 x 1024 (128) 30 against 24, 1024 x 4096 (256) 45 against 39, 1280 x 4096 (320) 47
+    #   against 53, 641 x 11008 (516) 74 against 79, 1024 x 14336 (896) 80 against 102; 700 x 4096 (192) of K = 11008 73 against
+    #   74, of K = 14336 92 against 99
+    #   one scale per channel, codes from the quantiser in the 6-bit format: 2048 x 4096 (512) 35 against 33, 2560 x 4096 (640) 40
+    #   against 43, 3000 x 11008 (2064) 104 against 125; packed codes: 2560 x 4096 52 against 49, 3000 x 6144 (1152) 78 against
+    #   76, 3600 x 6144 (1392) 81 against 84
+    # (Below 2560 rows one scale per channel stays on int8, although 2048 x 11008 takes 70 against 80 by now.)
     TRANSIENT_ROWS = (2560, 641)
     _NO_ROWS = 1 << 62                             # more rows than any call has
 
-    def _transient_tiles(self, grouped):
-        return 512 if not grouped else 256 if self.in_features <= 8192 else 191
+    def _transient_tiles(self, grouped, nibbles):
+        if grouped:
+            return 256 if self.in_features <= 8192 else 191
+        return 1280 if nibbles and self.in_features <= 8192 else 512
 
     def _keeps_six_bit(self, grouped):
         return self.six_bit is True or (self.six_bit not in (False, "never") and grouped)
 
-    def _six_bit_rows(self, grouped, columns=None):
+    def _six_bit_rows(self, grouped, columns=None, nibbles=False):
         """Rows from which a launch over `columns` channels (this layer's, unless it shares the launch) takes the 6-bit
-        instruction."""
+        instruction.  nibbles: its activations come as packed codes, to be encoded as well."""
         if self.six_bit == "never":
             return self._NO_ROWS
         if self._keeps_six_bit(grouped):
             return self.six_bit_min_rows
         tiles = -(-(columns or self.out_features) // 128)
-        return max(self.TRANSIENT_ROWS[grouped], 128 * (self._transient_tiles(grouped) // tiles) + 1)
+        return max(self.TRANSIENT_ROWS[grouped], 128 * (self._transient_tiles(grouped, nibbles) // tiles) + 1)
 
     def prepare_six_bit(self):
         """Build the 6-bit encoding of the weights now if this layer's setting keeps one (at load time, rather than inside
@@ -109,14 +116,14 @@ class LinearFLH(torch.nn.Module):
             return False
         per_row = a_scale.size(1) == 1 and w_scale.size(1) == 1
         grouped = group == 128 and w_scale.size(1) == self.in_features // 128 and a_scale.size(1) in (1, w_scale.size(1))
-        return (grouped or per_row) and self._six_bit_rows(not per_row, columns) <= n <= self._SIX_BIT_MAX_ROWS
+        return (grouped or per_row) and self._six_bit_rows(not per_row, columns, True) <= n <= self._SIX_BIT_MAX_ROWS
 
     def _group(self):
         return self.weight_group_size if self.weight_group_size > 0 else (self.in_group_size or 128)
 
-    def _few_rows(self, w_scale):
-        """Rows below which no call of this layer takes the 6-bit instruction."""
-        return self._six_bit_rows(w_scale.numel() > self.out_features)
+    def _few_rows(self, w_scale, nibbles=False):
+        """Rows below which no call of this layer (on packed codes, if `nibbles`) takes the 6-bit instruction."""
+        return self._six_bit_rows(w_scale.numel() > self.out_features, None, nibbles)
 
     # ------------------------------------------------------------------ kernels
     def forward(self, x, a_scale=None, a_zero=None, x_is_packed=False, is_symmetric=None, residual=None):
@@ -128,7 +135,7 @@ class LinearFLH(torch.nn.Module):
             w, w_scale = self._buffers.get("w_packed"), self._buffers.get("w_scale")
             if w is not None and w_scale is not None:
                 y = _pkg._CUDA.linear_i4(x, a_scale, w, w_scale, self.in_features, self.out_features, self._group(),
-                                         self._few_rows(w_scale))
+                                         self._few_rows(w_scale, True))
                 if y is not None:
                     return y if self.bias is None else y + self.bias
         lead = x.shape[:-1]

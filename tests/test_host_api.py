@@ -565,3 +565,12 @@ def test_rows_beyond_the_six_bit_launches_stay_on_int8(n, takes):
     lin = LinearFLH(128, 1024, device="meta", in_group_size=128, group_size=128)
     scales = torch.empty(1, 1, device="meta")
     assert lin._six_bit_applies(Rows, scales.expand(n, 1), scales.expand(1024, 1), 128) is takes
+
+
+def test_packed_codes_need_more_tiles_for_the_per_call_encoding():
+    """One scale per channel, K = 4096: codes that the call encodes as well take the 6-bit instruction beyond 1280 tiles of
+    128 x 128, codes in its format from 2560 rows on; the native call's limit is the former."""
+    lin = LinearFLH(4096, 6144, device="meta", in_group_size=128, group_size=4096)
+    assert lin._six_bit_rows(False) == 2560 and lin._six_bit_rows(False, None, True) == lin._few_rows(lin.w_scale, True) == 3329
+    lin = LinearFLH(11008, 4096, device="meta", in_group_size=128, group_size=11008)
+    assert lin._six_bit_rows(False) == lin._six_bit_rows(False, None, True) == 2560
