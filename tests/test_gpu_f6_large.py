@@ -94,3 +94,29 @@ def test_qkv_rope(ops, gemm_tuning, batch, t, hq, hkv, kind, tile):
     gemm_tuning(*tile)
     got = ops.gemm_f6_qkv_rope(ops.encode_f6(a), sa, [ops.encode_f6(w) for w in ws], sw, cos, sin, pos, caches[2], caches[3], batch)
     assert torch.equal(got, want) and torch.equal(caches[2], caches[0]) and torch.equal(caches[3], caches[1])
+
+
+@pytest.mark.parametrize("kind", ["token", "group"])
+@pytest.mark.parametrize("k", [1792, 2048, 2816])
+def test_blocks_of_scales_across_tiles(ops, gemm_tuning, kind, k):
+    """Several tiles per workgroup with two full blocks of eight scale groups, and with two and three the last of which is short:
+    the double buffer's turn carries over into the next tile.  Every form of launch, more than 256 tiles of 256 x 128 each."""
+    m, ns, n, hq, hkv = 2200, [5000, 1032, 3336], 2208, 20, 6
+    a_cols, b_cols = scale_columns(kind, k)
+    a, ws, sa, sw = operands(m, ns, k, a_cols, b_cols, k)
+    _, (g, u), _, (sg, su) = operands(m, [n, n], k, a_cols, b_cols, k + 1)
+    _, wr, _, sr = operands(m, [hq * 128, hkv * 128, hkv * 128], k, a_cols, b_cols, k + 2)
+    rng = np.random.default_rng(k)
+    res = dev(rng.standard_normal((m, ns[0])).astype(np.float16))
+    cos, sin = (dev(rng.uniform(-1, 1, (m, 128)).astype(np.float16)) for _ in range(2))
+    pos = torch.arange(3, 3 + m, device="cuda")
+    caches = [torch.zeros(1, hkv, m + 3, 128, dtype=torch.float16, device="cuda") for _ in range(4)]
+    want = [*ops.gemm_i4_dequant_multi(a, ws, sa, sw, 128), ops.gemm_i4_dequant_add(a, ws[0], sa, sw[0], res, 128),
+            ops.gemm_i4_swiglu(a, g, u, sa, sg, su, 128),
+            ops.gemm_i4_qkv_rope(a, sa, wr, sr, cos, sin, pos, caches[0], caches[1], 1, 128), caches[0], caches[1]]
+    a6, w6, r6 = ops.encode_f6(a), [ops.encode_f6(w) for w in ws], [ops.encode_f6(w) for w in wr]
+    gemm_tuning(256, 2)
+    got = [*ops.gemm_f6_dequant_multi(a6, w6, sa, sw), ops.gemm_f6_dequant_add(a6, w6[0], sa, sw[0], res),
+           ops.gemm_f6_swiglu(a6, ops.encode_f6(g), ops.encode_f6(u), sa, sg, su),
+           ops.gemm_f6_qkv_rope(a6, sa, r6, sr, cos, sin, pos, caches[2], caches[3], 1), caches[2], caches[3]]
+    assert all(torch.equal(x, y) for x, y in zip(got, want))

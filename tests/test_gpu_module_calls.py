@@ -80,3 +80,54 @@ def test_rows_around_the_change_to_the_six_bit_instruction(group, n):
     for m in (rows - 1, rows):
         s, z, c = q(x[:m].contiguous())
         assert torch.equal(lin(c, s, z, x_is_packed=True), y[:m])
+
+
+@pytest.mark.parametrize("k,hadamard", [(4096, True), (4096, "exact"), (4096, "fast"), (11008, True), (11008, "fast")])
+@pytest.mark.parametrize("group,bias", [(128, False), (128, True), (-1, False)])
+def test_online_linear_around_the_change_to_the_six_bit_instruction(monkeypatch, k, hadamard, group, bias):
+    """The last row count that stays on the int8 kernel and the first whose quantiser writes the 6-bit format, also with a leading
+    batch dimension: rotate_and_quantize_i4 + gemm_i4_dequant (+ bias)."""
+    import flh_amd
+    ops, n = flh_amd._CUDA, 4096
+    lin = layer(k, n, group, bias)
+    first = lin._six_bit_rows(group > 0)
+    assert 600 < first <= 2560
+    x = torch.randn(first + 1, k, device="cuda").half()
+    q, s = ops.rotate_and_quantize_i4(x, hadamard=hadamard)
+    want = ops.gemm_i4_dequant(q, lin.w_packed.view(n, k // 2), s, lin.w_scale.view(n, -1), 128)
+    if bias:
+        want = want + lin.bias
+    calls = []
+
+    class Counted(General):
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(self._ops, name)
+    monkeypatch.setattr(flh_amd, "_CUDA", Counted(ops))
+    for rows in (first - 1, first):
+        calls.clear()
+        y = lin.forward_online(x[:rows], hadamard=hadamard)
+        assert ("rotate_and_quantize_f6" in calls) == (rows == first) and torch.equal(y, want[:rows])
+    even = first + first % 2
+    assert torch.equal(lin.forward_online(x[:even].view(2, -1, k), hadamard=hadamard), want[:even].view(2, -1, n))
+    lin.six_bit = "never"
+    calls.clear()
+    assert torch.equal(lin.forward_online(x, hadamard=hadamard), want) and "rotate_and_quantize_f6" not in calls
+
+
+@pytest.mark.parametrize("group", [128, -1])
+def test_never_keeps_packed_codes_off_the_six_bit_instruction(monkeypatch, group):
+    import flh_amd
+    lin = layer(4096, 11008, group, False)
+    x = torch.randn(2600, 4096, device="cuda").half()
+    q, s = flh_amd._CUDA.rotate_and_quantize_i4(x) if group < 0 else flh_amd._CUDA.hadamard_and_quantize_i4(x.view(-1, 128))
+    q, s = q.view(2600, -1), s.view(2600, -1)
+    want = lin(q, s, x_is_packed=True)
+    lin.six_bit = "never"
+
+    class NoEncoding(General):
+        def __getattr__(self, name):
+            assert name != "encode_f6"
+            return getattr(self._ops, name)
+    monkeypatch.setattr(flh_amd, "_CUDA", NoEncoding(flh_amd._CUDA))
+    assert torch.equal(lin(q, s, x_is_packed=True), want)
