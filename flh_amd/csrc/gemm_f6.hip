@@ -60,11 +60,9 @@ void gemm_f6_kernel(const GemmArgs p) {
   constexpr int WAVES = (BM / WM) * (BN / WN);
   constexpr int T = 64 * WAVES;
   constexpr int STAGE = (BM + BN) * kBlockBytes;
-  constexpr int TI = (BM + BN) * 6 / 64;              // 1 KiB load instructions per stage
-  constexpr int NI_LO = TI / WAVES, NI_X = TI % WAVES; // the first NI_X waves issue one more than the others
-  constexpr int NI = NI_LO + (NI_X ? 1 : 0);
+  constexpr int TI = (BM + BN) * 6 / 64, NI = TI / WAVES;   // 1 KiB load instructions per stage: of the workgroup, of a wave
   constexpr int EPI_PITCH = WN * 2 + kEpiPadF6;
-  static_assert(WAVES == 4 && BM % 64 == 0 && BN % 64 == 0, "tile shape");
+  static_assert(WAVES == 4 && BM % 64 == 0 && BN % 64 == 0 && TI % WAVES == 0, "tile shape");
   static_assert(!SWIGLU || (EPI != kInt32 && WAVES_N == 2), "gate | up halves are the two wave columns");
   static_assert(!ROPE || (EPI != kInt32 && BN == 128 && WN == 64 && !SWIGLU), "a tile column is one head of 128");
   constexpr int BNC = SWIGLU ? BN / 2 : BN;           // output channels per tile
@@ -109,14 +107,14 @@ void gemm_f6_kernel(const GemmArgs p) {
   const int m0 = tile_m * BM, n0 = seg_tile * BNC;
 
   // per-lane byte offsets of this wave's NI load instructions inside A resp. B (stage 0)
-  const int my_ni = NI_LO + (wave < NI_X ? 1 : 0);     // wave-uniform
-  const int first_i = wave * NI_LO + (wave < NI_X ? wave : NI_X);
+  const int first_i = wave * NI;
   unsigned voff[NI];
   int src_of[NI];                                      // 0: activations, 1: weights, 2: the up matrix (SWIGLU)
   static_assert(!SWIGLU || (BNC * 6) % 64 == 0, "a load instruction never straddles gate | up");
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int slot = (min(first_i + i, TI - 1)) * 64 + lane;
+    // (the bound never holds; without it the compiler folds the addresses into a form that costs the 64 x 64 tiles 2-3 %)
+    const int slot = min(first_i + i, TI - 1) * 64 + lane;
     const bool isA = __builtin_amdgcn_readfirstlane(slot < BM * 6);
     const int s = isA ? slot : slot - BM * 6;
     const int r = s / 6, c = (s % 6) ^ ((r >> 3) & 1);
@@ -134,18 +132,12 @@ void gemm_f6_kernel(const GemmArgs p) {
     const uint8_t* kb2 = SWIGLU ? p.B2 + (size_t)k * wN * kBlockBytes : kb;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
-      if (i < NI_LO || i < my_ni)
-        load_to_lds16(src_of[i] == 0 ? ka : src_of[i] == 1 ? kb : kb2, voff[i], base + i * 1024);
+      load_to_lds16(src_of[i] == 0 ? ka : src_of[i] == 1 ? kb : kb2, voff[i], base + i * 1024);
   };
   // wait until at most `stages` stages of this wave's loads are still in flight
   auto wait_stages = [&](auto stages_tag) {
     constexpr int S = decltype(stages_tag)::value;
-    if constexpr (NI_X == 0) {
-      wait_vmcnt<S * NI_LO>();
-    } else {
-      if (wave < NI_X) wait_vmcnt<S * (NI_LO + 1)>();
-      else wait_vmcnt<S * NI_LO>();
-    }
+    wait_vmcnt<S * NI>();
   };
 
   v16f acc[TM][TN];                                    // exact integer sums (grouped: the float32 result so far)

@@ -16,7 +16,10 @@ struct Shape {
 };
 
 // A value of an accumulator where it is used and not before: left to itself, the compiler fetches most of the 256
-// accumulation registers of a 128 x 128 wave tile ahead of the branches of the epilogue, and spills.
+// accumulation registers of a 128 x 128 wave tile ahead of the branches of the epilogue, and spills.  The compiler does not see
+// that the instruction reads a matrix result and inserts no wait states for it: at least 18 cycles have to lie between the last
+// MFMA into a register and this read.  They do: the first value read is of acc[0][0], 15 MFMAs (of 8 passes or more) and the scale
+// product's MFMAs after its last one, and the last MFMA, into acc[3][0], is followed by three quarters of the epilogue.
 template <bool IN_AGPR>
 __device__ __forceinline__ float accumulator(float v) {
   if constexpr (IN_AGPR) {

@@ -5,7 +5,7 @@
 // Why.  The 64 x 64 tiles of gemm_i4.hip leave most of the chip idle here (4096 channels, 45 tokens: 64 workgroups), each
 // with one latency per 128 codes of K; a K split (gemm_i4_decode.hip) needs every group's sums of a tile in LDS, which ends
 // at 16 tokens.  Here a workgroup owns a small tile (BM x BN below) for the whole of K, so there is one per compute unit from
-// 32 x 4096 outputs on, and each wave folds its own 16 x 16 tiles in order.  Operands come through a ring of LDS stages of
+// 33 tokens x 4096 channels on, and each wave folds its own 16 x 16 tiles in order.  Operands come through a ring of LDS stages of
 // four groups (256 bytes of every row) filled by direct-to-LDS loads two stages ahead; fragments, and the scales from a
 // table in LDS, are read into registers one stage ahead of the products.  (Fragments straight from memory reach 16 bytes
 // per clock and compute unit, sixteen half lines per load: 17-25 us where this kernel takes 11-17.)

@@ -191,7 +191,7 @@ class LinearFLH(torch.nn.Module):
         encoded = rows.size(1) * 4 == first.in_features * 3      # activations already in the 6-bit format
         columns = sum(l.out_features for l in layers)
         if encoded or all(l._six_bit_applies(rows, a_rows, ws, group, columns) for l, ws in zip(layers, w_scales)):
-            # every layer opted into the 6-bit matrix instruction: one launch there as well
+            # every layer takes the 6-bit matrix instruction here: one launch there as well
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
             ys = ops.gemm_f6_dequant_multi(a6, [l._six_bit_weights() for l in layers], a_rows.contiguous(), w_scales)
         else:
