@@ -878,8 +878,9 @@ def main():
     xs = torch.randn(1, M, 4096, generator=gen).half().to(dev)
     cos, sin = rotary_tables(torch.arange(M, device=dev), 128)
     with torch.no_grad():
+        # (a long call of the "fused" layer encodes its weights for the 6-bit instruction in the call)
         for label, fused_form, six in (("module_by_module", False, False), ("fused", True, False),
-                                       ("fused,6bit_matrix_instruction", True, True)):
+                                       ("fused,6bit_weights_kept", True, True)):
             layer = W4A4DecoderLayer.from_float(lw, 32, 32, fused=fused_form, six_bit=six)
             layer_fig[f"prefill_T={M},{label}_us"] = round(wall_us(lambda: layer(xs, cos, sin), reps=20), 1)
             if six:
@@ -903,9 +904,9 @@ def main():
                 layer.fast_rotation = True
                 layer_fig["token_configuration,prefill_8x512,fused,matrix_core_rotation_us"] = round(
                     wall_us(lambda: layer(xs8, cos8, sin8), reps=20), 1)
-                # ... and with the seven linears on the 6-bit matrix instruction as well (a second encoding of the weights)
+                # ... and with the 6-bit encoding of the weights kept instead of made in each long call
                 layer.set_six_bit(True)
-                layer_fig["token_configuration,prefill_8x512,fused,matrix_core_rotation,6bit_matrix_instruction_us"] = round(
+                layer_fig["token_configuration,prefill_8x512,fused,matrix_core_rotation,6bit_weights_kept_us"] = round(
                     wall_us(lambda: layer(xs8, cos8, sin8), reps=20), 1)
             del layer
     del lw, xs, xs8
@@ -928,8 +929,8 @@ def main():
     # The Llama-3-8B decode step (32 layers, batch x 1 token, attention over 2048 cached positions, grouped queries 32 / 8,
     # intermediate 14336 with the 28 x 512 online rotation, group-of-128 weight scales, fp16 head of 128 256 rows), random
     # weights, captured into one graph and replayed.  The int4 linears and their quantisers (with the norms, residual
-    # additions and SiLU inside), the rotary embedding, the cache write and attention are this library's kernels; the
-    # embedding, the final norm and the fp16 head are torch's.  "everything else" = whole step minus the same step's
+    # additions and SiLU inside), the look-ups of embedding and rotary rows, the rotary embedding, the cache write, attention, the
+    # final norm and the fp16 head are this library's kernels.  "everything else" = whole step minus the same step's
     # linears-and-quantisers graph.  Lower bound of the step:
     # all int4 weights and scales + the fp16 head + the cached keys / values once over HBM.
     from flh_amd.quantized_model import LlamaShape, W4A4LlamaModel
