@@ -10,14 +10,15 @@
 //
 // What bounds it.  A compute unit loads 64 bytes per clock into LDS and reads 256, its SIMD needs 32 clocks per MFMA.  A
 // step of a 128 x 128 tile (four waves of 64 x 64) is 384 clocks of loads for 256 of MFMAs, a step of the 256 x 256 tile
-// 768 for 1024.  Timestamps at 8192 x 14336 x 4096: 1450-1580 clocks per step of the 256 x 256 tile (1150 without its
-// loads, 1050 without its fragment reads as well), 9700 per tile for the outputs, at 1.3-1.4 GHz -- the part is at its
-// power limit, and what is left is the energy of the loads.  Prefetching the slabs into L2 changed nothing.
-// us per launch, weights from HBM, against the tiles this replaces (two workgroups of 128 x 128 per compute unit, or one of
-// 256 x 128 on eight waves of 64 x 64) and the int8 kernel:
-//   one scale per row, 8192 x 14336 x 4096:  264 (3.64 POP/s) against 372 and 378;  4096 x 4096 x 11008: 92 against 118, 136
-//   token scales,      8192 x 14336 x 4096:  392 (2.45)       against 429 and 599;  2048 x 28672 x 4096: 202 against 221, 304
-//   group scales,      8192 x 14336 x 4096:  435 (2.21)       against 575 and 701;  2048 x 28672 x 4096: 220 against 291, 356
+// 768 for 1024.  In-kernel timestamps at 8192 x 14336 x 4096: 1450-1580 clocks per step of the 256 x 256 tile (1150 without
+// its loads, 1050 without its fragment reads as well), 9700 per tile for the outputs.  Counters: the matrix pipe is busy half of
+// the clocks a compute unit has work, at 1.83 GHz in launches that stand alone, where light ones run at 2.4, and launches back
+// to back take 296 us instead of 262 -- the part is at its power limit.  Prefetching the slabs into L2 changed nothing.
+// us per launch, weights from HBM, alone - back to back where they differ, against the tiles this replaces (two workgroups of
+// 128 x 128 per compute unit, or one of 256 x 128 on eight waves of 64 x 64) and the int8 kernel:
+//   one scale per row, 8192 x 14336 x 4096:  262 - 296 (3.67 - 3.25 POP/s) against 372 and 378;  4096 x 4096 x 11008: 88 against 118, 136
+//   token scales,      8192 x 14336 x 4096:  406 - 423 (2.37 - 2.27) against 429 and 599;  2048 x 28672 x 4096: 202 against 221, 304
+//   group scales,      8192 x 14336 x 4096:  438 - 448 (2.20 - 2.15) against 575 and 701;  2048 x 28672 x 4096: 222 against 291, 356
 #pragma once
 #include "gemm_i4.h"
 #include "lane_ops.h"

@@ -8,10 +8,12 @@
 // tile's scale products come from one more MFMA, an outer product of the two scale vectors (exact in float32, in the
 // layout of the sums), instead of a conversion and a multiplication per output on the vector ALU.
 //
-// The loop is bound by instruction issue: per step a wave issues 16 MFMAs (each holds the issue port for 16 clocks), 128
-// multiply-adds of 4 clocks, and its LDS reads and loads.  A wave of 64 x 128 outputs has the fewest of the latter two;
-// four of them, one per SIMD with up to 512 registers, were faster than eight of 32 x 128 (8192 x 14336 x 4096: 414 against
-// 436 us with token scales, 444 against 479 us with group scales).
+// What bounds it: one wave per SIMD, which issues everything in turn.  Counters at 2048 x 28672 x 4096, per step of one group,
+// outputs included: 1800 clocks with token scales, 1970 with group scales, of which vector instructions hold the issue port 712
+// resp. 820 (128 of 178 are the fold's multiply-adds, 4 clocks each, with token scales), the matrix pipe is busy 512 resp. 770
+// and LDS 500 resp. 530, a third of that in bank conflicts; with token scales some 570 clocks are in none of the first two.  A
+// wave of 64 x 128 outputs has the fewest LDS reads and loads per MFMA; four of them, one per SIMD with up to 512 registers,
+// were faster than eight of 32 x 128 (8192 x 14336 x 4096: 414 against 436 us with token scales, 444 against 479 with group scales).
 #include "gemm_f6_large.h"
 
 namespace flh {
