@@ -261,6 +261,10 @@ class W4A4LlamaModel(torch.nn.Module):
             cache.rotary_table = table
         return table
 
+    def _look_up_rows(self, hidden, t):
+        """Tokens that one look-up launch beside `t` rotary rows takes: 2^31 - 1 pieces of eight values."""
+        return (2 ** 31 - 1 - 2 * t * (self.shape.head_dim // 8)) // (hidden // 8)
+
     def _look_up(self, input_ids, positions, cache):
         """embed(input_ids) and _rotary(positions, cache): one launch on the fused path with a static cache (the same bits)
         -- unless the embedding is more than a look-up or takes part in a backward pass."""
@@ -271,7 +275,7 @@ class W4A4LlamaModel(torch.nn.Module):
         if not (plain and self.fused and cache is not None and not (torch.is_grad_enabled() and w.requires_grad) and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
                 and w.data_ptr() % 16 == 0 and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0
                 and input_ids.is_cuda and input_ids.dtype == torch.int64 and positions.dtype == torch.int64
-                and positions.dim() == 1 and input_ids.numel() > 0):
+                and positions.dim() == 1 and 0 < input_ids.numel() <= self._look_up_rows(w.size(1), positions.numel())):
             cos, sin = self._rotary(positions, cache)
             return self.embed(input_ids), cos, sin
         import flh_amd

@@ -574,3 +574,15 @@ def test_packed_codes_need_more_tiles_for_the_per_call_encoding():
     assert lin._six_bit_rows(False) == 2560 and lin._six_bit_rows(False, None, True) == lin._few_rows(lin.w_scale, True) == 3329
     lin = LinearFLH(11008, 4096, device="meta", in_group_size=128, group_size=11008)
     assert lin._six_bit_rows(False) == lin._six_bit_rows(False, None, True) == 2560
+
+
+def test_look_up_launch_stays_within_its_limit():
+    """Tokens beyond what one look-up launch indexes get the module call: the model's line is the last count that the C entry takes
+    (one more is refused there, before any launch)."""
+    model, lib = _small_model(), _lib.load()
+    limit = model._look_up_rows(128, 2)
+    chunks = lambda rows: rows * 16 + 2 * 2 * 8
+    assert chunks(limit) <= 2 ** 31 - 1 < chunks(limit + 1)
+    at = (torch.zeros(64, dtype=torch.int64).data_ptr() + 15) // 16 * 16
+    assert lib.flh_embed_f16(at, at, at, limit + 1, 32, 128, 0, at, at, at, at, at, 2, 4, 64, None) != 0
+    assert "too many elements" in lib.flh_last_error().decode()
