@@ -75,10 +75,11 @@ class LinearFLH(torch.nn.Module):
     def _six_bit_rows(self, grouped, columns=None, nibbles=False):
         """Rows from which a launch over `columns` channels (this layer's, unless it shares the launch) takes the 6-bit
         instruction.  nibbles: its activations come as packed codes, to be encoded as well."""
-        if self.six_bit == "never":
-            return self._NO_ROWS
-        if self._keeps_six_bit(grouped):
-            return self.six_bit_min_rows
+        if self.six_bit is not False:                  # (the default first: every small call asks)
+            if self.six_bit == "never":
+                return self._NO_ROWS
+            if self._keeps_six_bit(grouped):
+                return self.six_bit_min_rows
         tiles = -(-(columns or self.out_features) // 128)
         return max(self.TRANSIENT_ROWS[grouped], 128 * (self._transient_tiles(grouped, nibbles) // tiles) + 1)
 
