@@ -679,8 +679,8 @@ bool large_supported(const GemmArgs& a, bool grouped) {
 // Which large tile a launch over `columns` weight rows takes: 256 x 256 (kWide), 256 x 128 (kNarrow) or neither.
 // Beyond 256 tiles of 128 x 128 the shape with the least of  once + per_round * rounds of 256 tiles + per_256 *
 // tiles / 256,  least squares over launches of M = 256 .. 5000 on the Llama widths (K = 4096, weights from HBM, us; longer K
-// scales all three alike).  The pick is within 2 % of the fastest shape on all but 2 of 260 launches (within 4 % there), those
-// of K = 11008 and 14336 included.  With the rotary epilogue, whose loads and index arithmetic the next tile does not cover in a
+// scales all three alike).  The pick is within 2 % of the fastest shape on all but 1 of 521 launches (4 % there), those of K =
+// 11008 and 14336 included.  With the rotary epilogue, whose loads and index arithmetic the next tile does not cover in a
 // persistent workgroup, a large tile pays less; with token scales never there (700 x 6144 35 against 32, 4096 x 12288 208 against
 // 192); one scale per row and up to 512 tokens as without it (512 x 12288 32 against 34).  Group scales with 224 .. 256 small
 // tiles: the large ones, except with the rotary epilogue (1024 x 11008 x 4096 72 against 78, 640 x 4096 x 6144 33 against 34.5,
