@@ -447,16 +447,18 @@ c10::optional<Tensor> linear_online_i4(const Tensor& x, const Tensor& w, const T
   if (M < 0 || M >= row_limit || !plain_weights(x, w, w_scale, K, N)) return c10::nullopt;
   if (mode < 0) mode = K == 11008 || K == 14336 ? FLH_HAD_MFMA : FLH_HAD_F32;
   const int64_t cols = w_scale.numel() / N;
-  Tensor D = empty_rows(x, N, x.options());
   Launch l(x);
   if (M <= 2 && K == 4096 && mode == FLH_HAD_F32 && (cols == 1 || (group == 128 && cols == 32))) {
+    Tensor D = empty_rows(x, N, x.options());
     ok(flh_rotate_quant_gemm_i4_o16(h(x), u8(w), h(w_scale), hm(D), M, N, K, (int)cols, stream_of(x)));
     return D;
   }
+  // (codes and scales before the output, as on the general path: behind it, 770 x 4096 x 4096 took 37.7 us instead of 36.5)
   Tensor q = torch::empty({M, K / 2}, x.options().dtype(torch::kUInt8));
   Tensor s = torch::empty({M, 1}, x.options());
   ok(flh_rotate_quant_i4(h(x), (uint8_t*)q.data_ptr(), hm(s), nullptr, (uint32_t)M, (uint32_t)K, (int)mode, 0, 0, 1.0f,
                          stream_of(x)));
+  Tensor D = empty_rows(x, N, x.options());
   ok(flh_gemm_i4_o16(u8(q), u8(w), h(s), h(w_scale), hm(D), M, N, K, 1, (int)cols, (int)group, stream_of(x)));
   return D;
 }
