@@ -247,15 +247,22 @@ class W4A4DecoderLayer(torch.nn.Module):
         """Whether the quantiser in front of `consumers` should write the 6-bit operand format directly: every consumer
         would re-encode the nibbles for the 6-bit matrix instruction anyway."""
         return (bool(consumers) and self.activation == "token" and self.fused and self.record is None
-                and width in self._F6_WIDTHS
-                and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers))
+                and width in self._F6_WIDTHS and self._take_six_bit(consumers, n_rows))
+
+    @staticmethod
+    def _take_six_bit(consumers, n_rows):
+        """(Another module in a projection's place, or one with hooks, is given the packed codes that it documents.)"""
+        return (all(isinstance(l, LinearFLH) for l in consumers)
+                and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers)
+                and all(_stock_call(l, LinearFLH) for l in consumers))
 
     def _group_six_bit_for(self, consumers, n_rows, width):
         """_six_bit_for of the group configuration: the consumers' codes and scales in groups of 128."""
         return (bool(consumers) and self.activation == "group" and self.fused and self.record is None
                 and self.act_group_size == 128 and width % 128 == 0 and width <= 16384
-                and all(l.in_group_size == 128 and l.w_scale.numel() == l.out_features * (width // 128) > l.out_features
-                        and l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers))
+                and all(isinstance(l, LinearFLH) and l.in_group_size == 128
+                        and l.w_scale.numel() == l.out_features * (width // 128) > l.out_features for l in consumers)
+                and self._take_six_bit(consumers, n_rows))
 
     def _rotation_mode(self, rows, k):
         """hadamard argument of the whole-row ops for `rows` rows of k channels."""

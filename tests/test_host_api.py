@@ -586,3 +586,46 @@ def test_look_up_launch_stays_within_its_limit():
     at = (torch.zeros(64, dtype=torch.int64).data_ptr() + 15) // 16 * 16
     assert lib.flh_embed_f16(at, at, at, limit + 1, 32, 128, 0, at, at, at, at, at, 2, 4, 64, None) != 0
     assert "too many elements" in lib.flh_last_error().decode()
+
+
+class _OtherProjection(torch.nn.Module):
+    """A module in a projection's place that has nothing of LinearFLH but its call."""
+
+    def forward(self, codes, a_scale, a_zero=None, x_is_packed=False, **kwargs):
+        self.seen = (codes.size(-1), sorted(kwargs))
+        return torch.ones(*codes.shape[:-1], 128).half()
+
+
+def _layer_without_a_gpu(monkeypatch, activation):
+    import flh_amd
+    from flh_amd.quantized_model import W4A4DecoderLayer
+    layer = _small_model().layers[0]
+    layer.activation = activation
+
+    class Ops:
+        quantize_groups = staticmethod(lambda x, *a: (torch.ones(*x.shape[:-1], 1).half(), torch.zeros(*x.shape[:-1], 64, dtype=torch.uint8)))
+    monkeypatch.setattr(flh_amd, "_CUDA", Ops)
+    monkeypatch.setattr(W4A4DecoderLayer, "_F6_WIDTHS", (128,))
+    monkeypatch.setattr(LinearFLH, "wants_six_bit", lambda self, *a: True)
+    return layer
+
+
+@pytest.mark.parametrize("rows", [4, 1000])
+def test_another_output_projection_gets_packed_codes(monkeypatch, rows):
+    """A replaced o_proj is called with the codes of attn_quantizer2, at any length."""
+    layer = _layer_without_a_gpu(monkeypatch, "group")
+    layer.o_proj = _OtherProjection()
+    layer._output_projection(torch.zeros(1, rows, 128).half(), torch.zeros(1, rows, 128).half(), None, True)
+    assert layer.o_proj.seen[0] == 64
+
+
+@pytest.mark.parametrize("activation", ["token", "group"])
+@pytest.mark.parametrize("change", ["none", "hook", "replaced"])
+def test_six_bit_codes_go_to_plain_projections_only(monkeypatch, activation, change):
+    layer = _layer_without_a_gpu(monkeypatch, activation)
+    lin = LinearFLH(256, 128, device="cpu", in_group_size=128, group_size=128)
+    if change == "hook":
+        lin.register_forward_pre_hook(lambda *a: None)
+    consumers = (_OtherProjection() if change == "replaced" else lin,)
+    takes = layer._group_six_bit_for(consumers, 1000, 256) if activation == "group" else layer._six_bit_for(consumers, 1000, 128)
+    assert takes is (change == "none")
