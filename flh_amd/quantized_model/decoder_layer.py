@@ -439,8 +439,8 @@ class W4A4DecoderLayer(torch.nn.Module):
         _attention returns them."""
         s, z, q = (self._token_quant("attn_out", out, consumers=(self.o_proj,)) if self.activation == "token"
                    else self._group_quant("attn_out", self.attn_quantizer2, out, (self.o_proj,)))
-        if fold_residual and self._residual_in_gemm(out.numel() // out.size(-1)):
-            # prefill: the residual addition in o_proj's epilogue; nothing is left pending
+        if fold_residual and self._residual_in_gemm(out.numel() // out.size(-1), self.o_proj):
+            # the residual addition in o_proj's epilogue; nothing is left pending
             return self.o_proj(q, s, z, x_is_packed=True, residual=x), None, cache
         y = self.o_proj(q, s, z, x_is_packed=True)
         self._tap("o_proj", y)
@@ -505,13 +505,15 @@ class W4A4DecoderLayer(torch.nn.Module):
         out = _ops().prefill_attention(qs, keys, values, past)
         return self._output_projection(x, out, cache, fold_residual)
 
-    def _residual_in_gemm(self, rows):
+    def _residual_in_gemm(self, rows, linear):
         """Whether o_proj / down_proj add the residual stream in their own epilogue: the fused path of the group
         configuration, whose norm + quantiser launch has no addition of its own (2048 tokens: 728 against 736 us per
         layer; at decode sizes it takes two launches of 3-4 us off a layer).  The token configuration keeps the addition
         inside its norm + rotation launch, which is cheaper than the extra read in the GEMM's epilogue burst (8 x 512
-        tokens: 888 against 910 us)."""
-        return self.fused and self.record is None and rows > 0 and self.activation == "group"
+        tokens: 888 against 910 us).  Up to 64 rows a plain `linear` only: another module there, or a hook, sees the product
+        by itself."""
+        return (self.fused and self.record is None and self.activation == "group"
+                and (rows > 64 or (rows > 0 and _stock_call(linear, LinearFLH))))
 
     def _online_qkv_applies(self):
         """q / k / v in the layout the decode GEMM with its own norm + quantiser takes: no bias, one scale per channel or
@@ -575,7 +577,7 @@ class W4A4DecoderLayer(torch.nn.Module):
             z = None                                # (symmetric codes: no zero points to fill)
         else:
             s, z, q = self._group_quant("mlp_mid", self.mlp_quantizer2, torch.nn.functional.silu(gate) * up)
-        if fold_residual and self._residual_in_gemm(rows):
+        if fold_residual and self._residual_in_gemm(rows, self.down_proj):
             return self.down_proj(q, s, z, x_is_packed=True, residual=x), None
         y = self.down_proj(q, s, z, x_is_packed=True)
         self._tap("down_proj", y)

@@ -629,3 +629,21 @@ def test_six_bit_codes_go_to_plain_projections_only(monkeypatch, activation, cha
     consumers = (_OtherProjection() if change == "replaced" else lin,)
     takes = layer._group_six_bit_for(consumers, 1000, 256) if activation == "group" else layer._six_bit_for(consumers, 1000, 128)
     assert takes is (change == "none")
+
+
+@pytest.mark.parametrize("change", ["none", "hook", "replaced"])
+def test_few_rows_add_the_residual_in_plain_projections_only(monkeypatch, change):
+    """Group configuration, a decode step: another module in o_proj's place, or a hook on it, sees the product by itself."""
+    layer, seen = _layer_without_a_gpu(monkeypatch, "group"), []
+    x = torch.zeros(1, 4, 128).half()
+    monkeypatch.setattr(LinearFLH, "forward", lambda self, q, s, z, x_is_packed, residual=None: (seen.append(residual), x)[1])
+    if change == "hook":
+        layer.o_proj.register_forward_hook(lambda *a: None)
+    elif change == "replaced":
+        layer.o_proj = _OtherProjection()
+    stream, y, _ = layer._output_projection(x, torch.zeros(1, 4, 128).half(), None, True)
+    if change == "none":
+        assert seen[0] is x and y is None
+    else:
+        assert stream is x and y is not None
+        assert layer.o_proj.seen == (64, []) if change == "replaced" else seen == [None]
