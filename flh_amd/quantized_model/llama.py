@@ -272,10 +272,11 @@ class W4A4LlamaModel(torch.nn.Module):
         plain = (all(getattr(type(self), f) is getattr(W4A4LlamaModel, f) and f not in self.__dict__ for f in ("embed", "_rotary"))
                  and _stock_call(e, torch.nn.Embedding) and e.max_norm is None)
         w = e.weight if plain else None            # (another module need not have a weight)
-        if not (plain and self.fused and cache is not None and not (torch.is_grad_enabled() and w.requires_grad) and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous()
-                and w.data_ptr() % 16 == 0 and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0
-                and input_ids.is_cuda and input_ids.dtype == torch.int64 and positions.dtype == torch.int64
-                and positions.dim() == 1 and 0 < input_ids.numel() <= self._look_up_rows(w.size(1), positions.numel())):
+        if not (plain and self.fused and cache is not None and not (torch.is_grad_enabled() and w.requires_grad)
+                and w.is_cuda and w.dtype == torch.float16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and w.size(1) % 128 == 0 and self.shape.head_dim % 8 == 0 and input_ids.is_cuda and input_ids.dtype == torch.int64
+                and positions.dtype == torch.int64 and positions.dim() == 1
+                and 0 < input_ids.numel() <= self._look_up_rows(w.size(1), positions.numel())):
             cos, sin = self._rotary(positions, cache)
             return self.embed(input_ids), cos, sin
         import flh_amd
