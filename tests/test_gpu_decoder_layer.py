@@ -170,3 +170,22 @@ def test_fast_rotation_option_changes_almost_nothing():
             layer.fast_rotation = False
             d0, _ = layer(x[:, :1].contiguous(), cos[:1], sin[:1])
             assert torch.equal(d0, d1)
+
+
+@pytest.mark.parametrize("activation", ["token", "group"])
+@pytest.mark.parametrize("t", [5, 300])
+def test_hooks_on_projections_see_packed_codes_and_leave_the_bits(activation, t):
+    """Hooks on o_proj and down_proj of a layer that keeps its 6-bit weights: they are given what the quantisers pack, up to 64 rows
+    the product without the residual, and the layer's bits stay."""
+    w, _ = make()
+    layer = W4A4DecoderLayer.from_float(w, 4, 2, activation=activation, weight_group_size=128, six_bit=True)
+    x = torch.randn(1, t, 512, generator=torch.Generator().manual_seed(2)).half().cuda()
+    cos, sin = rotary_tables(torch.arange(t, device="cuda"), 128)
+    want = layer(x, cos, sin)
+    seen = []
+    for name in ("o_proj", "down_proj"):
+        getattr(layer, name).register_forward_hook(lambda m, args, kwargs, out: seen.append((args[0].size(-1), "residual" in kwargs)),
+                                                   with_kwargs=True)
+    got = layer(x, cos, sin)
+    assert torch.equal(got[0], want[0]) and all(torch.equal(a, b) for a, b in zip(got[1], want[1]))
+    assert [s[0] for s in seen] == [256, 512] and (t > 64 or not any(s[1] for s in seen))
