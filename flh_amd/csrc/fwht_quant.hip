@@ -242,6 +242,113 @@ __global__ __launch_bounds__(256) void silu_mul_group_kernel(const __half* __res
   group_finish<G, F6>(v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
 }
 
+// The group kernels for groups of 128 and launches that fill the chip: FOUR lanes own a group, 32 values each (lane p
+// the chunks p, p + 4, p + 8, p + 12), so that of the seven butterfly strides only 8 and 16 cross lanes, and the row's maximum,
+// scale and reciprocal are computed by four lanes instead of sixteen.  A lane's four code words are turned inside its wave
+// through LDS, so that it stores sixteen consecutive bytes (32 codes; 6-bit output: one whole 24-byte piece).  Same
+// operations in the same order as group_kernel, the same bytes.
+// What bounds it: memory (4096-wide rows rotated and quantised, us, sixteen lanes -> four, inputs from HBM: 16384 rows 40.3 -> 29.5
+// = 5.7 TB/s, 8192 20.4 -> 15.9, 4096 10.1 -> 9.4; 6-bit output 49.3 -> 40.4, 25.4 -> 21.8, 14.3 -> 12.0), where the sixteen-lane form
+// is bound by its 165 instructions per eight values, 80 here.  Non-temporal loads and stores: equal or slower (30.6, 31.3).  The
+// SwiGLU product in front of it: 55.6 against 51.4 us, its exponentials want the sixteen lanes' parallelism; not here.
+constexpr uint32_t kQuadRows = 64;                    // groups per workgroup of four waves
+template <int CTRL>
+__device__ __forceinline__ void quad_cross(h2 (&v)[4][4], _Float16 sg) {
+  const h2 sgn = {sg, sg};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const h2 o = __builtin_bit_cast(h2, dpp_i<CTRL>(__builtin_bit_cast(int, v[j][i])));
+      v[j][i] = __builtin_elementwise_fma(v[j][i], sgn, o);
+    }
+}
+__device__ __forceinline__ void butterfly(h2& a, h2& b) {
+  const h2 s = a + b, d = a - b;
+  a = s, b = d;
+}
+template <bool HAD, bool F6>
+__global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
+                                                         __half* __restrict__ scales, uint32_t R, float scale_mul,
+                                                         uint32_t tokens, uint32_t groups_per_token) {
+  __shared__ unsigned turned[256 * 4];
+  const int tid = threadIdx.x, p = tid & 3;
+  const uint32_t row0 = blockIdx.x * kQuadRows, row = row0 + (tid >> 2);
+  const bool valid = row < R;
+  const uint32_t at = ((valid ? row : R - 1) - row0) * 256 + p * 16;   // bytes from the workgroup's first group
+  const char* xb = (const char*)x + (size_t)row0 * 256;
+  h2 v[4][4];                                          // [chunk][pair]
+  h8 raw[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) raw[j] = *(const h8*)(xb + (at + j * 64));
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[j][i] = h2{raw[j][2 * i], raw[j][2 * i + 1]};
+  if constexpr (HAD) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {                    // {a + b, a - b} of a pair, one instruction
+        unsigned d;
+        asm("v_pk_add_f16 %0, %1, %1 op_sel:[0,1] op_sel_hi:[0,1] neg_hi:[0,1]" : "=v"(d) : "v"(__builtin_bit_cast(unsigned, v[j][i])));
+        v[j][i] = __builtin_bit_cast(h2, d);
+      }
+      butterfly(v[j][0], v[j][1]), butterfly(v[j][2], v[j][3]);
+      butterfly(v[j][0], v[j][2]), butterfly(v[j][1], v[j][3]);
+    }
+    quad_cross<kDppQuadXor1>(v, p & 1 ? (_Float16)-1.0f : (_Float16)1.0f);
+    quad_cross<kDppQuadXor2>(v, p & 2 ? (_Float16)-1.0f : (_Float16)1.0f);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      butterfly(v[0][i], v[1][i]), butterfly(v[2][i], v[3][i]);
+      butterfly(v[0][i], v[2][i]), butterfly(v[1][i], v[3][i]);
+    }
+  }
+  float m = lane_abs_max(v[0]);
+#pragma unroll
+  for (int j = 1; j < 4; ++j) {
+    const float mj = lane_abs_max(v[j]);
+    asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m), "v"(mj));
+  }
+  m = max_across<kDppQuadXor1>(m);
+  m = max_across<kDppQuadXor2>(m);
+  _Float16 s = scale_of_max(m);
+  if (s <= (_Float16)1e-6f) s = (_Float16)1.0f;
+  const float r = reciprocal_of_scale(s);
+  const bool careful = __builtin_amdgcn_ballot_w64((float)s < 6.2e-5f) != 0;   // as in group_finish
+  const h2 hb = {(_Float16)65504.0f, (_Float16)65504.0f};
+  unsigned w[4];
+  auto codes = [&](auto careful_tag) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      w[j] = nibbles8<decltype(careful_tag)::value>(__builtin_bit_cast(unsigned, v[j][0]), __builtin_bit_cast(unsigned, v[j][1]),
+                                                    __builtin_bit_cast(unsigned, v[j][2]), __builtin_bit_cast(unsigned, v[j][3]), r, hb);
+  };
+  if (careful) codes(std::true_type{});
+  else codes(std::false_type{});
+  // the group's sixteen words, blocks of four swapped by the group's place in the wave: no bank conflicts
+  const int swap = (tid >> 4) & 3;
+  unsigned* const line = turned + (tid >> 2) * 16;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) line[4 * (j ^ swap) + p] = w[j];
+  __builtin_amdgcn_wave_barrier();                     // (the wave's own words, LDS operations of a wave complete in order)
+  const v4i o = *(const v4i*)(line + 4 * (p ^ swap));
+  if (!valid) return;
+  if constexpr (F6) {
+    const unsigned long long q0 = bf6_of_nibbles((unsigned)o[0]), q1 = bf6_of_nibbles((unsigned)o[1]),
+                             q2 = bf6_of_nibbles((unsigned)o[2]), q3 = bf6_of_nibbles((unsigned)o[3]);
+    const size_t block = (size_t)(row % groups_per_token) * tokens + row / groups_per_token;
+    unsigned long long* dst = (unsigned long long*)(q + block * kF6BlockBytes + 48 * (p & 1) + 24 * (p >> 1));
+    dst[0] = q0 | (q1 << 48);
+    dst[1] = (q1 >> 16) | (q2 << 32);
+    dst[2] = (q2 >> 32) | (q3 << 16);
+  } else {
+    *(v4i*)(q + (size_t)row0 * 64 + tid * 16) = o;
+  }
+  if (p == 0) scales[row] = scale_mul == 1.0f ? __builtin_bit_cast(__half, s) : __float2half(round_here((float)s * scale_mul));
+}
+
 // the SwiGLU product alone, eight values per thread
 __global__ __launch_bounds__(256) void silu_mul_kernel(const __half* __restrict__ gate, const __half* __restrict__ up,
                                                        __half* __restrict__ out, uint64_t chunks) {
@@ -727,10 +834,25 @@ int launch_wave_rms(const __half* x, const __half* w, float eps, uint8_t* q, __h
   return check_launch("rmsnorm_rotate_quant_wave");
 }
 
+// Groups of 128 from which four lanes per group are the faster form: below, a quarter of the wavefronts does not fill the
+// chip (us, sixteen lanes / four, groups of 128; rotated 8192 groups 2.52 / 2.76, 16384 3.30 / 3.21, 65536 6.40 / 6.14; not
+// rotated 32000 3.72 / 3.89, 65536 5.62 / 5.40; 6-bit output 8192 2.73 / 2.95, 16384 3.76 / 3.51).
+constexpr uint32_t quad_min_rows(bool had, bool f6) { return had || f6 ? 16384 : 65536; }
+template <bool HAD, bool F6>
+int launch_group_quad(const __half* x, uint8_t* q, __half* s, uint32_t R, float scale_mul, uint32_t tokens,
+                      uint32_t groups_per_token, hipStream_t stream) {
+  hipLaunchKernelGGL((group_quad_kernel<HAD, F6>), dim3((unsigned)(((uint64_t)R + kQuadRows - 1) / kQuadRows)), dim3(256), 0,
+                     stream, x, q, s, R, scale_mul, tokens, groups_per_token);
+  return check_launch("group_quad_kernel");
+}
+
 template <int G>
 int launch_group(const __half* x, uint8_t* q, __half* s, __half* y, uint32_t R, bool had, bool quant,
                  float scale_mul, hipStream_t stream) {
   constexpr int LPR = G / 8;
+  if (G == 128 && quant && R >= quad_min_rows(had, false))
+    return had ? launch_group_quad<true, false>(x, q, s, R, scale_mul, 0, 1, stream)
+               : launch_group_quad<false, false>(x, q, s, R, scale_mul, 0, 1, stream);
   const dim3 grid((unsigned)(((uint64_t)R * LPR + 255) / 256)), block(256);
   auto go = [&](auto off32_tag) {
     constexpr bool OFF32 = decltype(off32_tag)::value;
@@ -1056,6 +1178,9 @@ extern "C" int flh_group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half*
   const uint32_t R = M * (K / 128);
   const dim3 grid((unsigned)(((uint64_t)R * 16 + 255) / 256)), block(256);
   const __half* xh = (const __half*)x;
+  if (R >= quad_min_rows(hadamard != 0, true))
+    return hadamard ? launch_group_quad<true, true>(xh, encoded, (__half*)scales, R, scale_mul, M, K / 128, (hipStream_t)stream)
+                    : launch_group_quad<false, true>(xh, encoded, (__half*)scales, R, scale_mul, M, K / 128, (hipStream_t)stream);
   if (hadamard)
     hipLaunchKernelGGL((group_kernel<128, true, true, true>), grid, block, 0, (hipStream_t)stream, xh, encoded,
                        (__half*)scales, nullptr, R, scale_mul, M, K / 128);
