@@ -676,51 +676,55 @@ bool large_supported(const GemmArgs& a, bool grouped) {
     if (off4(a.seg_Bs[s])) return false;
   return (uint64_t)(a.M > total_n_f6(a) ? a.M : total_n_f6(a)) * kt < (1ull << 31);
 }
-// Which large tile a launch over `columns` weight rows takes: 256 x 256 (kWide), 256 x 128 (kNarrow) or neither.
-// Beyond 256 tiles of 128 x 128 the shape with the least of  once + per_round * rounds of 256 tiles + per_256 *
-// tiles / 256,  least squares over launches of M = 256 .. 5000 on the Llama widths (K = 4096, weights from HBM, us; longer K
-// scales all three alike).  The pick is within 2 % of the fastest shape on all but 1 of 521 launches (4 % there), those of K =
-// 11008 and 14336 included.  With the rotary epilogue, whose loads and index arithmetic the next tile does not cover in a
-// persistent workgroup, a large tile pays less; with token scales never there (700 x 6144 35 against 32, 4096 x 12288 208 against
-// 192); one scale per row and up to 512 tokens as without it (512 x 12288 32 against 34).  Group scales with 224 .. 256 small
-// tiles: the large ones, except with the rotary epilogue (1024 x 11008 x 4096 72 against 78, 640 x 4096 x 6144 33 against 34.5,
-// 256 x 4096 x 14336 32 against 34.5;  640 x 6144 with it 39 against 36); token scales with at most one large tile on each:
-// the large one unless hardly any compute unit would get a second small one (384 x 12288, 288 small tiles, 32.4 / 30.5).
-// Some of both sides, small / 256 x 128 / 256 x 256:
-//   one scale per row   640 x 11008 29.1 / 40.6 / 31.9, 2048 x 11008 76 / 67 / 68, 2400 x 4096 40 / 41 / 35;  with the rotary
-//                       epilogue 1000 x 6144 28.4 / 30.0 / 42.0, 2560 x 6144 57 / 59 / 53, 3000 x 6144 69 / 78 / 87
-//   token scales        384 x 11008 29.2 / 31.5, 512 x 11008 34 / 32, 3000 x 11008 136 / 146, 2048 x 28672 223 / 208
-//   group scales        1024 x 4096 32 / 30, 640 x 11008 53 / 64, 1400 x 11008 83 / 90, 2048 x 28672 303 / 229
-enum LargeTile { kNoLarge = 0, kNarrow = 1, kWide = 2 };
+// Which kernel of gemm_f6_large.h a launch over `columns` weight rows takes: tiles of 256 x 256 (kWide, one scale per row only),
+// 256 x 128 (kNarrow), 128 x 128 (kSquare, group scales only) or none of them (kNoLarge: the tiles of this file).
+// The shape with the least of  once + per_round * rounds of 256 tiles + per_256 * tiles / 256,  least squares over launches of M =
+// 256 .. 5000 on the Llama widths (K = 4096, weights from HBM, us; longer K scales all alike).
+// One scale per row: beyond 256 tiles of 128 x 128; the pick is within 2 % of the fastest shape on all but 1 of 521 launches (4 %
+// there), those of K = 11008 and 14336 included.  With the rotary epilogue, whose loads and index arithmetic the next tile does
+// not cover in a persistent workgroup, a large tile pays less; up to 512 tokens as without it (512 x 12288 32 against 34).
+//   small / 256 x 128 / 256 x 256: 640 x 11008 29.1 / 40.6 / 31.9, 2048 x 11008 76 / 67 / 68, 2400 x 4096 40 / 41 / 35;  with the
+//   rotary epilogue 1000 x 6144 28.4 / 30.0 / 42.0, 2560 x 6144 57 / 59 / 53, 3000 x 6144 69 / 78 / 87
+// Group and token scales: from the second round of 64 x 64 tiles on (the third with token scales); rotary launches, which have no
+// 64 x 64 tiles, always.  The pick is within 2 % of the fastest on 468 of 476 launches of M = 70 .. 5000 (12 % on 640 x 12288
+// with token scales).  With group scales on both sides the 128 x 128 tiles of this file are the fastest nowhere.
+//   64 x 64 / 128 x 128 here / square / 256 x 128: token scales 384 x 4096 15.6 / 22 / 17.8 / 26, 600 x 4096 20.5 / 24 / 18.6 / 26,
+//   768 x 12288 - / 50 / 54 / 56, 1000 x 28672 - / 115 / 119 / 104, 2048 x 4096 - / 32 / 35 / 30;  group scales 256 x 4096 15.1 / - /
+//   18.6 / 29, 384 x 4096 x 14336 56 / 98 / 53 / 77, 1000 x 4096 x 14336 112 / 101 / 65 / 80, 2048 x 28672 - / 289 / 246 / 207
+enum LargeTile { kNoLarge = 0, kNarrow = 1, kWide = 2, kSquare = 3 };
 struct LaunchCost {
   double once, per_round, per_256;
   double of(long tiles) const { return once + per_round * ((tiles + 255) / 256) + per_256 * tiles / 256; }
 };
-// [rotary epilogue][128 x 128, 256 x 128, 256 x 256]
+// [rotary epilogue]: [128 x 128, 256 x 128, 256 x 256]; token scales [128 x 128, square, 256 x 128]; group scales [square, 256 x 128]
 constexpr LaunchCost kRowCost[2][3] = {{{6.2, 6.3, 6.7}, {5.3, 11.1, 11.8}, {4.1, 21.5, 17.6}},
                                        {{6.3, 8.6, 4.5}, {6.1, 18.1, 8.4}, {6.0, 30.6, 16.9}}};
-constexpr LaunchCost kTokenCost[2][2] = {{{6.1, 9.5, 6.2}, {5.1, 20.2, 9.9}}, {{6.2, 11.1, 4.5}, {5.7, 26.9, 5.9}}};
-constexpr LaunchCost kGroupCost[2][2] = {{{6.7, 16.6, 4.2}, {5.4, 22.9, 8.3}}, {{6.9, 17.6, 3.4}, {6.0, 29.3, 6.5}}};
+constexpr LaunchCost kTokenCost[2][3] = {{{8.3, 6.4, 8.8}, {4.7, 10.7, 6.0}, {2.5, 17.8, 9.6}},
+                                         {{8.5, 6.7, 9.1}, {4.3, 12.5, 6.0}, {2.1, 22.9, 8.0}}};
+constexpr LaunchCost kGroupCost[2][2] = {{{4.6, 11.1, 6.7}, {3.1, 19.5, 10.4}}, {{4.9, 13.3, 5.5}, {3.1, 24.5, 7.9}}};
 LargeTile large_choice(const GemmArgs& a, int epi, long columns, bool rope = false) {
   const bool grouped = epi != kRowScale;
   if (!large_supported(a, grouped)) return kNoLarge;
-  const int forced = g_tune_tile.load(std::memory_order_relaxed);
-  if (forced == 256) return grouped || g_tune_ks.load(std::memory_order_relaxed) == 2 ? kNarrow : kWide;
+  const int forced = g_tune_tile.load(std::memory_order_relaxed), forced_ks = g_tune_ks.load(std::memory_order_relaxed);
+  if (forced == 128 && forced_ks == 2) return grouped ? kSquare : kNoLarge;
+  if (forced == 256) return grouped || forced_ks == 2 ? kNarrow : kWide;
   if (forced) return kNoLarge;
   auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((columns + bn - 1) / bn); };
   const long small = tiles(128, 128), narrow = tiles(256, 128);
-  if (small <= 256) return epi == kGroupScale && small >= 224 && !rope ? kNarrow : kNoLarge;
   if (grouped) {
-    if (epi == kTokenGroup && !rope && narrow <= 256) return small > 272 ? kNarrow : kNoLarge;
-    const LaunchCost* cost = epi == kTokenGroup ? kTokenCost[rope] : kGroupCost[rope];
-    return cost[1].of(narrow) < cost[0].of(small) ? kNarrow : kNoLarge;
+    if (!rope && tiles(64, 64) <= (epi == kTokenGroup ? 512 : 288)) return kNoLarge;
+    if (epi == kGroupScale) return kGroupCost[rope][1].of(narrow) < kGroupCost[rope][0].of(small) ? kNarrow : kSquare;
+    const LaunchCost* cost = kTokenCost[rope];
+    const double s = cost[0].of(small), q = cost[1].of(small), n = cost[2].of(narrow);
+    return n <= s && n < q ? kNarrow : q < s ? kSquare : kNoLarge;
   }
+  if (small <= 256) return kNoLarge;
   const LaunchCost* cost = kRowCost[rope && a.M > 512];
   const double s = cost[0].of(small), n = cost[1].of(narrow), w = cost[2].of(tiles(256, 256));
   return w <= n && w < s ? kWide : n < s ? kNarrow : kNoLarge;
 }
-// 128 x 128 tiles below that, down to 192 of them (with more than 64 rows; group scales on both sides: 224), else 64 x 64
-// (512 x 6144: 19 against 21 with row scales, 22 against 22 with token scales, 33 against 26 with group scales)
+// Launches without one of those: 128 x 128 tiles of this file down to 192 of them (with more than 64 rows; group scales on both
+// sides, for the K and alignments the others do not take: 224), else 64 x 64 (512 x 6144 with one scale per row: 19 against 21)
 int small_choice(const GemmArgs& a, int epi, long columns) {
   const int forced = g_tune_tile.load(std::memory_order_relaxed);
   if (forced) return forced == 64 ? 64 : 128;
@@ -731,7 +735,8 @@ int small_choice(const GemmArgs& a, int epi, long columns) {
 template <int EPI>
 int launch_f6_grouped(const GemmArgs& a, hipStream_t stream) {
   const int n_all = total_n_f6(a);
-  if (large_choice(a, EPI, n_all)) return f6l::launch_large_group(a, EPI == kTokenGroup, a.R ? f6l::kResidual : f6l::kPlain, stream);
+  if (const LargeTile large = large_choice(a, EPI, n_all))
+    return f6l::launch_large_group(a, EPI == kTokenGroup, large == kNarrow, a.R ? f6l::kResidual : f6l::kPlain, stream);
   if (small_choice(a, EPI, n_all) == 128) return launch_f6<128, 128, 64, 64, 3, EPI>(a, stream);
   return launch_f6<64, 64, 32, 32, 3, EPI>(a, stream);
 }
@@ -742,7 +747,7 @@ int launch_f6_swiglu(const GemmArgs& a, hipStream_t stream) {
   const long columns = 2 * (long)a.N;
   if (const LargeTile large = large_choice(a, EPI, columns)) {
     if constexpr (EPI == kRowScale) return f6l::launch_large_row(a, large == kWide, f6l::kSwiglu, stream);
-    else return f6l::launch_large_group(a, EPI == kTokenGroup, f6l::kSwiglu, stream);
+    else return f6l::launch_large_group(a, EPI == kTokenGroup, large == kNarrow, f6l::kSwiglu, stream);
   }
   if (small_choice(a, EPI, columns) == 128) return launch_f6<128, 128, 64, 64, 3, EPI, true>(a, stream);
   return launch_f6<64, 64, 32, 32, 3, EPI, true>(a, stream);
@@ -925,7 +930,7 @@ extern "C" int flh_gemm_f6_qkv_rope_o16(const uint8_t* A6, const flh_half* a_sca
   g.rope_hkv = (int)Hkv;
   if (const LargeTile large = large_choice(g, rows_only ? kRowScale : a_cols == 1 ? kTokenGroup : kGroupScale, total_n_f6(g), true)) {
     if (rows_only) return f6l::launch_large_row(g, large == kWide, f6l::kRope, (hipStream_t)stream);
-    return f6l::launch_large_group(g, a_cols == 1, f6l::kRope, (hipStream_t)stream);
+    return f6l::launch_large_group(g, a_cols == 1, large == kNarrow, f6l::kRope, (hipStream_t)stream);
   }
   // 128 x 128 tiles (a tile column = one head)
   if (rows_only) return launch_f6<128, 128, 64, 64, 3, kRowScale, false, true>(g, (hipStream_t)stream);
