@@ -50,6 +50,7 @@ _SIG = {
     "flh_rotate_quant_gemm_i4_o16": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _c.c_size_t, _c.c_size_t, _c.c_size_t,
                                                 _c.c_int, _PTR]),
     "flh_encode_f6": (_c.c_int, [_PTR, _PTR, _c.c_size_t, _c.c_size_t, _PTR]),
+    "flh_encode_f6_multi": (_c.c_int, [_c.c_int, _PTR, _PTR, _PTR, _c.c_size_t, _PTR]),
     "flh_gemm_f6_o16": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _PTR, _c.c_size_t, _c.c_size_t, _c.c_size_t, _PTR]),
     "flh_group_quant_f6": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _c.c_int, _c.c_float, _PTR]),
     "flh_gemm_f6_o16_gs": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _PTR, _c.c_size_t, _c.c_size_t, _c.c_size_t, _c.c_int,

@@ -352,6 +352,25 @@ def encode_f6(packed):
     return out
 
 
+def encode_f6_many(packed):
+    """[encode_f6(p) for p in packed] of one to four matrices with the same K in one launch."""
+    import ctypes
+    n = len(packed)
+    _check(1 <= n <= 4, "one to four matrices")
+    for p in packed:
+        _check(p.is_cuda and p.dtype == torch.uint8 and p.dim() == 2 and p.is_contiguous() and p.device == packed[0].device,
+               "packed codes must be contiguous 2D uint8 CUDA tensors on one device")
+        _check(p.size(1) == packed[0].size(1), "the matrices must share K")
+    K = packed[0].size(1) * 2
+    _check(K % 128 == 0, "K must be a multiple of 128")
+    outs = [torch.empty((p.size(0), K // 128 * 96), dtype=torch.uint8, device=p.device) for p in packed]
+    ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
+    if K:
+        _run("flh_encode_f6_multi", packed[0].device, n, ptrs(packed), ptrs(outs), (ctypes.c_size_t * n)(*[p.size(0) for p in packed]), K,
+             _stream(packed[0]))
+    return outs
+
+
 def group_quantize_f6(x, hadamard=True, *, scale_mul=1.0):
     """hadamard_and_quantize_i4 / quant_and_pack_i4 over groups of 128 of x [M, K] fp16, with the codes
     written in the format of encode_f6: -> [q6 [M, K/128 * 96] u8, scales [M, K/128] fp16]."""

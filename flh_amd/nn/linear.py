@@ -34,8 +34,7 @@ class LinearFLH(torch.nn.Module):
             self.bias = None
         # Prefill-sized calls run on the 6-bit matrix instruction where that is faster (extension; same bits, no unpack in the
         # loop).  Its operands are re-encoded at 6 bits per code, 0.75 byte per weight next to the 0.5 of `w_packed`.
-        # False (default): nothing is kept; a call of at least TRANSIENT_ROWS rows encodes its weights into a buffer that
-        # goes back with the call.  "never": not even that, for callers without that memory to spare.  True: the layer keeps
+        # False (default): nothing is kept; a long call (_six_bit_rows) encodes its weights into a buffer that goes back with it.  "never": not even that, for callers without that memory to spare.  True: the layer keeps
         # the encoding (2.5 x the weight memory) and every call of at least `six_bit_min_rows` rows uses it.  "auto" (or
         # None): kept for weights with a scale per group of 128.
         # `prepare_six_bit()` builds the kept encoding at once (a loader calls it); otherwise it is built on first use.  It
@@ -49,39 +48,42 @@ class LinearFLH(torch.nn.Module):
     def drop_six_bit_weights(self):
         self._w6 = self._w6_key = None
 
-    # A call that encodes its weights for the 6-bit instruction first is faster from these rows on (one scale per channel, a
-    # scale per group of 128) if it also has more 128 x 128 tiles than _transient_tiles -- less fills the chip with neither
-    # kernel, and the passes over the operands are all that differs; with group scales a long K needs fewer, with one scale per
-    # channel packed codes, which are encoded as well, more.  us, all encodings included, against the int8 kernels (rows x
-    # channels, K = 4096 unless stated, tiles):
-    #   group scales, packed codes: 2048 x 1024 (128) 30 against 24, 1024 x 4096 (256) 45 against 39, 1280 x 4096 (320) 47
-    #   against 53, 641 x 11008 (516) 74 against 79, 1024 x 14336 (896) 80 against 102; 700 x 4096 (192) of K = 11008 73 against
-    #   74, of K = 14336 92 against 99
-    #   one scale per channel, codes from the quantiser in the 6-bit format: 2048 x 4096 (512) 35 against 33, 2560 x 4096 (640) 40
-    #   against 43, 3000 x 11008 (2064) 104 against 125; packed codes: 2560 x 4096 52 against 49, 3000 x 6144 (1152) 78 against
-    #   76, 3600 x 6144 (1392) 81 against 84
-    # (Below 2560 rows one scale per channel stays on int8, although 2048 x 11008 takes 70 against 80 by now.)
+    # A call that encodes its weights for the 6-bit instruction first is faster from these rows on (one scale per channel;
+    # group-scaled weights with a scale per token; group scales on both sides) if it also has more 128 x 128 tiles than
+    # _transient_tiles -- less fills the chip with neither kernel, and the passes over the operands are all that differs.
+    # Packed codes, which the call encodes as well, need more.  us, int8 / 6-bit with the weights encoded (codes from the
+    # quantiser in the 6-bit format, which costs it 1-3 us more) / packed codes encoded as well, rows x channels, K = 4096 unless stated:
+    #   one scale per channel: 2048 x 4096 34.5 / 34.9 / 40.7, 3000 x 4096 49 / 43 / 52, 2400 x 11008 109 / 82 / 90; 2048 x 11008 89 / 79 / 87 in
+    #   a graph, 84 / 84 as separate calls, and a layer of 1400 tokens whose gate and up change over is slower, 380 / 409
+    #   a scale per token: 640 x 4096 25.7 / 28.5 / 28.4, 1280 x 4096 45 / 35 / 42, 1000 x 14336 95 / 70 / 79, 640 x 4096 of K = 11008 63 / 54 / 58
+    #   group scales: 512 x 4096 25.7 / 26.3 / 29.5, 640 x 4096 31.8 / 30.0 / 30.2, 1000 x 4096 38 / 33 / 33, 512 x 4096 of K = 11008 60 / 54 / 57;
+    #   320 x 11008 52 / 43 / 46, but the host's part of the encoding makes a layer of 300 or 450 tokens slower (245 / 262; 500: 271 / 263)
     TRANSIENT_ROWS = (2560, 641)
+    TRANSIENT_ROWS_GROUPS = 513
     _NO_ROWS = 1 << 62                             # more rows than any call has
 
-    def _transient_tiles(self, grouped, nibbles):
+    def _transient_tiles(self, grouped, nibbles, groups=False):
+        long_k = self.in_features > 8192
+        if grouped and groups:
+            return (128 if nibbles else 95) if long_k else 160 if nibbles else 143
         if grouped:
-            return 256 if self.in_features <= 8192 else 191
-        return 1280 if nibbles and self.in_features <= 8192 else 512
+            return 191 if long_k else 256
+        return 1280 if nibbles and not long_k else 512
 
     def _keeps_six_bit(self, grouped):
         return self.six_bit is True or (self.six_bit not in (False, "never") and grouped)
 
-    def _six_bit_rows(self, grouped, columns=None, nibbles=False):
+    def _six_bit_rows(self, grouped, columns=None, nibbles=False, groups=False):
         """Rows from which a launch over `columns` channels (this layer's, unless it shares the launch) takes the 6-bit
-        instruction.  nibbles: its activations come as packed codes, to be encoded as well."""
-        if self.six_bit is not False:                  # (the default first: every small call asks)
+        instruction.  nibbles: its activations come as packed codes, to be encoded as well; groups: with a scale per group of 128."""
+        if self.six_bit is not False:
             if self.six_bit == "never":
                 return self._NO_ROWS
             if self._keeps_six_bit(grouped):
                 return self.six_bit_min_rows
+        first = self.TRANSIENT_ROWS_GROUPS if grouped and groups else self.TRANSIENT_ROWS[grouped]
         tiles = -(-(columns or self.out_features) // 128)
-        return max(self.TRANSIENT_ROWS[grouped], 128 * (self._transient_tiles(grouped, nibbles) // tiles) + 1)
+        return max(first, 128 * (self._transient_tiles(grouped, nibbles, groups) // tiles) + 1)
 
     def prepare_six_bit(self):
         """Build the 6-bit encoding of the weights now if this layer's setting keeps one (at load time, rather than inside
@@ -98,33 +100,42 @@ class LinearFLH(torch.nn.Module):
             self._w6_key = key
         return self._w6
 
+    @staticmethod
+    def _six_bit_weights_of(layers):
+        """[l._six_bit_weights() for l in layers], encodings that are not kept built in one launch."""
+        if 1 < len(layers) <= 4 and all(type(l) is LinearFLH and l.in_features == layers[0].in_features
+                                        and not l._keeps_six_bit(l.w_scale.numel() > l.out_features) for l in layers):
+            return _pkg._CUDA.encode_f6_many([l.w_packed.view(l.out_features, l.in_features // 2) for l in layers])
+        return [l._six_bit_weights() for l in layers]
+
     _SIX_BIT_MAX_ROWS = ((1 << 32) - 1) // 96       # rows of either operand that the 6-bit launches index; more go to int8
 
-    def wants_six_bit(self, n_rows, columns=None):
-        """Whether a call with `n_rows` per-token-quantised rows takes the 6-bit matrix instruction (a producer can then
-        write the activations in that format directly, rotate_and_quantize_f6).  `columns`: channels of the whole launch,
-        where several layers share one."""
-        if (n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS[1]) or self.in_features % 128 or not self.w_packed.is_cuda:
+    def wants_six_bit(self, n_rows, columns=None, groups=False):
+        """Whether a call with `n_rows` rows quantised per token (or, `groups`, per group of 128) takes the 6-bit matrix
+        instruction (a producer can then write the activations in that format directly, rotate_and_quantize_f6).
+        `columns`: channels of the whole launch, where several layers share one."""
+        if (n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS_GROUPS) or self.in_features % 128 or not self.w_packed.is_cuda:
             return False
         cols = self.w_scale.view(self.out_features, -1).size(1)
         if cols != 1 and not (cols == self.in_features // 128 and self.weight_group_size == 128):
             return False
-        return self._six_bit_rows(cols != 1, columns) <= n_rows <= self._SIX_BIT_MAX_ROWS
+        return self._six_bit_rows(cols != 1, columns, False, groups) <= n_rows <= self._SIX_BIT_MAX_ROWS
 
     def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)
-        if (n < self.six_bit_min_rows and n < self.TRANSIENT_ROWS[1]) or not rows.is_cuda or self.in_features % 128:
+        if (n < self.six_bit_min_rows and n < self.TRANSIENT_ROWS_GROUPS) or not rows.is_cuda or self.in_features % 128:
             return False
         per_row = a_scale.size(1) == 1 and w_scale.size(1) == 1
         grouped = group == 128 and w_scale.size(1) == self.in_features // 128 and a_scale.size(1) in (1, w_scale.size(1))
-        return (grouped or per_row) and self._six_bit_rows(not per_row, columns, True) <= n <= self._SIX_BIT_MAX_ROWS
+        return ((grouped or per_row)
+                and self._six_bit_rows(not per_row, columns, True, a_scale.size(1) > 1) <= n <= self._SIX_BIT_MAX_ROWS)
 
     def _group(self):
         return self.weight_group_size if self.weight_group_size > 0 else (self.in_group_size or 128)
 
-    def _few_rows(self, w_scale, nibbles=False):
+    def _few_rows(self, w_scale, nibbles=False, groups=False):
         """Rows below which no call of this layer (on packed codes, if `nibbles`) takes the 6-bit instruction."""
-        return self._six_bit_rows(w_scale.numel() > self.out_features, None, nibbles)
+        return self._six_bit_rows(w_scale.numel() > self.out_features, None, nibbles, groups)
 
     # ------------------------------------------------------------------ kernels
     def forward(self, x, a_scale=None, a_zero=None, x_is_packed=False, is_symmetric=None, residual=None):
@@ -135,8 +146,10 @@ class LinearFLH(torch.nn.Module):
         if residual is None and a_scale is not None:
             w, w_scale = self._buffers.get("w_packed"), self._buffers.get("w_scale")
             if w is not None and w_scale is not None:
-                y = _pkg._CUDA.linear_i4(x, a_scale, w, w_scale, self.in_features, self.out_features, self._group(),
-                                         self._few_rows(w_scale, True))
+                k, least = self.in_features, self.TRANSIENT_ROWS_GROUPS
+                few = (least if self.six_bit is False and 2 * x.numel() < least * k      # below every line: asked for no further
+                       else self._few_rows(w_scale, True, a_scale.size(-1) > 1))
+                y = _pkg._CUDA.linear_i4(x, a_scale, w, w_scale, k, self.out_features, self._group(), few)
                 if y is not None:
                     return y if self.bias is None else y + self.bias
         lead = x.shape[:-1]
@@ -194,7 +207,7 @@ class LinearFLH(torch.nn.Module):
         if encoded or all(l._six_bit_applies(rows, a_rows, ws, group, columns) for l, ws in zip(layers, w_scales)):
             # every layer takes the 6-bit matrix instruction here: one launch there as well
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            ys = ops.gemm_f6_dequant_multi(a6, [l._six_bit_weights() for l in layers], a_rows.contiguous(), w_scales)
+            ys = ops.gemm_f6_dequant_multi(a6, LinearFLH._six_bit_weights_of(layers), a_rows.contiguous(), w_scales)
         else:
             ys = ops.gemm_i4_dequant_multi(rows, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
                                            a_rows, w_scales, group)
@@ -222,7 +235,7 @@ class LinearFLH(torch.nn.Module):
         if encoded or all(six):
             ops = _pkg._CUDA
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            y = ops.gemm_f6_swiglu(a6, gate_layer._six_bit_weights(), up_layer._six_bit_weights(), a_rows.contiguous(),
+            y = ops.gemm_f6_swiglu(a6, *LinearFLH._six_bit_weights_of((gate_layer, up_layer)), a_rows.contiguous(),
                                    gate_layer.w_scale.view(n, -1), up_layer.w_scale.view(n, -1))
             return y.view(*lead, n)
         y = _pkg._CUDA.gemm_i4_swiglu(rows, gate_layer.w_packed.view(n, k // 2), up_layer.w_packed.view(n, k // 2),
@@ -241,8 +254,9 @@ class LinearFLH(torch.nn.Module):
         ops = _pkg._CUDA
         buf, mode = self._buffers, -1 if hadamard is True else self._ONLINE_MODES.get(hadamard)
         if mode is not None and buf.get("w_packed") is not None and buf.get("w_scale") is not None:
-            y = ops.linear_online_i4(x, buf["w_packed"], buf["w_scale"], self.in_features, self.out_features, self._group(),
-                                     mode, self._few_rows(buf["w_scale"]))
+            k, least = self.in_features, self.TRANSIENT_ROWS_GROUPS
+            few = least if self.six_bit is False and x.numel() < least * k else self._few_rows(buf["w_scale"])
+            y = ops.linear_online_i4(x, buf["w_packed"], buf["w_scale"], k, self.out_features, self._group(), mode, few)
             if y is not None:
                 return y if self.bias is None else y + self.bias
         lead = x.shape[:-1]
@@ -254,7 +268,7 @@ class LinearFLH(torch.nn.Module):
                    and (w_scale.size(1) == 1 or (group == 128 and w_scale.size(1) == 32)))
         if fusable:
             y = ops.rotate_quantize_gemm_i4(rows, w, w_scale)
-        elif rows.size(0) >= self.TRANSIENT_ROWS[1] and self.in_features in (4096, 11008, 14336) and self.wants_six_bit(rows.size(0)) and (
+        elif rows.size(0) >= self.TRANSIENT_ROWS_GROUPS and self.in_features in (4096, 11008, 14336) and self.wants_six_bit(rows.size(0)) and (
                 hadamard in (True, "fast") or (hadamard == "exact" and self.in_features == 4096)):
             # long calls: the quantiser writes the 6-bit operand format
             q, s = ops.rotate_and_quantize_f6(rows, hadamard=hadamard)

@@ -247,13 +247,13 @@ class W4A4DecoderLayer(torch.nn.Module):
         """Whether the quantiser in front of `consumers` should write the 6-bit operand format directly: every consumer
         would re-encode the nibbles for the 6-bit matrix instruction anyway."""
         return (bool(consumers) and self.activation == "token" and self.fused and self.record is None
-                and width in self._F6_WIDTHS and self._take_six_bit(consumers, n_rows))
+                and width in self._F6_WIDTHS and self._take_six_bit(consumers, n_rows, False))
 
     @staticmethod
-    def _take_six_bit(consumers, n_rows):
+    def _take_six_bit(consumers, n_rows, groups):
         """(Another module in a projection's place, or one with hooks, is given the packed codes that it documents.)"""
         return (all(isinstance(l, LinearFLH) for l in consumers)
-                and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers)) for l in consumers)
+                and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers), groups) for l in consumers)
                 and all(_stock_call(l, LinearFLH) for l in consumers))
 
     def _group_six_bit_for(self, consumers, n_rows, width):
@@ -262,7 +262,7 @@ class W4A4DecoderLayer(torch.nn.Module):
                 and self.act_group_size == 128 and width % 128 == 0 and width <= 16384
                 and all(isinstance(l, LinearFLH) and l.in_group_size == 128
                         and l.w_scale.numel() == l.out_features * (width // 128) > l.out_features for l in consumers)
-                and self._take_six_bit(consumers, n_rows))
+                and self._take_six_bit(consumers, n_rows, True))
 
     def _rotation_mode(self, rows, k):
         """hadamard argument of the whole-row ops for `rows` rows of k channels."""
@@ -494,7 +494,7 @@ class W4A4DecoderLayer(torch.nn.Module):
         rows, a_rows = codes.reshape(b * t, -1), scales.reshape(b * t, -1)
         if mode == "f6":
             a6 = rows.contiguous() if rows.size(1) * 4 == self.hidden_size * 3 else _ops().encode_f6(rows.contiguous())
-            qs = _ops().gemm_f6_qkv_rope(a6, a_rows.contiguous(), [l._six_bit_weights() for l in layers], w_scales,
+            qs = _ops().gemm_f6_qkv_rope(a6, a_rows.contiguous(), LinearFLH._six_bit_weights_of(layers), w_scales,
                                          cos.contiguous(), sin.contiguous(), slots, keys, values, b)
         else:
             qs = _ops().gemm_i4_qkv_rope(rows, a_rows, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],

@@ -181,6 +181,9 @@ void quant_and_pack_host_gs(int group_size, const flh_half* data, uint8_t* quant
  * the 24 bytes at offset 48 h + 24 m; a code c is stored as sign << 5 | {0, 12, 16, 18, 20, 21, 22, 23, 24}[|c|].
  * --------------------------------------------------------------------------------- */
 int flh_encode_f6(const uint8_t* packed_i4, uint8_t* encoded, size_t rows, size_t K, void* stream);
+/* The same for 1 .. 4 matrices of one K in one launch (the weight matrices of a launch of several). */
+int flh_encode_f6_multi(int count, const uint8_t* const* packed_i4, uint8_t* const* encoded, const size_t* rows, size_t K,
+                        void* stream);
 int flh_gemm_f6_o16(const uint8_t* A6, const uint8_t* B6, const flh_half* a_scale, const flh_half* b_scale,
                     flh_half* D, size_t M, size_t N, size_t K, void* stream);
 int flh_gemm_f6_i32(const uint8_t* A6, const uint8_t* B6, int32_t* C, size_t M, size_t N, size_t K, void* stream);
