@@ -199,7 +199,7 @@ __global__ __launch_bounds__(512, 1) void gemm_f6_large_group_kernel(const GemmA
   issue((STAGES - 1) * STAGE);
   // load instructions of a wave in the stages that may be outstanding when one is needed: all but that and the one in use
   static_assert(!TALL || STAGES == 4, "two stages are nine instructions");
-  constexpr int kBehind = TALL ? 9 : (STAGES - 2) * 3;
+  constexpr int kBehind = TALL ? 9 : (STAGES - 3) * 3;
   wait_vmcnt<kBehind + 3>();
   __syncthreads();
 
@@ -281,8 +281,9 @@ __global__ __launch_bounds__(512, 1) void gemm_f6_large_group_kernel(const GemmA
         if constexpr (s > NT && m == 1) read_fragment(NEXT, std::integral_constant<int, j>{}, nx);   // (B_j: done with)
         if constexpr (s == 2 * NT - 1) read_fragment(NEXT, A1, nx);
       } else {
-        if constexpr (s == NT) read_fragment(NEXT, A0, nx), read_fragment(NEXT, I0, nx);
-        if constexpr (s == NT + 1) read_fragment(NEXT, I1, nx);
+        if constexpr (s == 0) read_fragment(NEXT, A0, nx);
+        if constexpr (s == 1) read_fragment(NEXT, I0, nx);
+        if constexpr (s == 2) read_fragment(NEXT, I1, nx);
       }
       if constexpr (ODD && s == 2 * NT - 3)            // the next pair's scales: of this tile, or the next one's first
         read_scales(LAST ? 0 : kt + 1, (sblk - (LAST || !((kt + 1) & 7) ? 1 : 2)) & 1);

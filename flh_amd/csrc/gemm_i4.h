@@ -81,4 +81,9 @@ int gemm_stream_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
 bool gemm_stream_rope_supports(const GemmArgs& a, int epi);
 int gemm_stream_rope_dispatch(const GemmArgs& a, hipStream_t stream);
 
+// 128 x 128 tiles of eight waves for group-scaled weights (gemm_i4_square.hip).
+enum SquareOut { kSquarePlain = 0, kSquareSwiglu = 1, kSquareRope = 2 };
+bool gemm_square_takes(const GemmArgs& a);
+int gemm_square_dispatch(const GemmArgs& a, SquareOut out, hipStream_t stream);
+
 }  // namespace flh

@@ -753,8 +753,24 @@ int launch_grouped(const GemmArgs& a, int group, bool small, hipStream_t stream)
   return launch<128, 128, 64, 64, 3, EPI>(a, stream);
 }
 
+// Launches over `columns` weight rows that take the eight-wave tiles of gemm_i4_square.hip: from 144 tiles of 128 x 128 on, with token
+// scales up to one per compute unit.  us, present tiles (here or in gemm_i4_stream.hip) / those, K = 4096 unless stated:
+//   token scales  512 x 4096 (128 tiles) 21 / 25, 640 x 4096 (160) 28 / 26, 800 x 4096 (224) 32 / 27, 250 x 11008 (172) 27 / 26, 250 x 14336 (224)
+//                 32 / 27, 400 x 11008 (344) 45 / 47, 1280 x 4096 (320) 45 / 47;  800 x 4096 of K = 11008 75 / 61
+//   group scales  512 x 4096 25 / 27, 640 x 4096 31 / 27, 250 x 14336 38 / 28, 400 x 11008 54 / 48, 1280 x 4096 53 / 50, 1000 x 14336 98 / 93;
+//                 640 x 4096 of K = 11008 74 / 62
+//   with SwiGLU   1 .. 128 x 22016 (172) 34 / 28 and 39 / 28, 320 x 22016 (516) 70 / 71 and 82 / 74
+bool takes_square(const GemmArgs& a, long columns) {
+  const int tile = g_tune_tile.load(std::memory_order_relaxed), ks = g_tune_ks.load(std::memory_order_relaxed);
+  if (tile || ks) return tile == 128 && ks == 2 && gemm_square_takes(a);
+  const long tiles = (long)((a.M + 127) / 128) * ((columns + 127) / 128);
+  return tiles >= 144 && (a.a_cols > 1 || tiles <= 256) && gemm_square_takes(a);
+}
+
 int gemm_dispatch(GemmArgs a, int epi, int group, hipStream_t stream) {
   if (a.M == 0 || a.N == 0) return FLH_OK;
+  if (epi == kGroupScale && group == 128 && (a.M > kDecodeMaxM || g_tune_tile.load(std::memory_order_relaxed)) && takes_square(a, total_n(a)))
+    return gemm_square_dispatch(a, kSquarePlain, stream);
   if (gemm_stream_supports(a, epi, group)) return gemm_stream_dispatch(a, epi, stream);
   if (gemm_decode_supports(a, epi, group)) return gemm_decode_dispatch(a, epi, stream);
   switch (epi) {
@@ -774,6 +790,7 @@ int gemm_dispatch(GemmArgs a, int epi, int group, hipStream_t stream) {
 // two wave columns of a workgroup)
 template <int EPI>
 int launch_swiglu(const GemmArgs& a, int group, hipStream_t stream) {
+  if (EPI != kRowScale && takes_square(a, 2 * (long)a.N)) return gemm_square_dispatch(a, kSquareSwiglu, stream);
   auto tiles = [&](int bm) { return (long)((a.M + bm - 1) / bm) * ((a.N + 63) / 64); };
   int tile = tiles(256) > 256 ? (prefers_small_tiles(tiles(256), tiles(128)) ? 128 : 256) : tiles(128) >= 160 ? 128 : 64;
   const int forced = g_tune_tile.load(std::memory_order_relaxed);
@@ -792,6 +809,7 @@ int launch_swiglu(const GemmArgs& a, int group, hipStream_t stream) {
 // q / k / v launches with the rotary embedding and the cache write in the epilogue: 128-column tiles, or the small ones
 template <int EPI>
 int launch_qkv_rope(const GemmArgs& a, hipStream_t stream) {
+  if (EPI != kRowScale && takes_square(a, total_n(a))) return gemm_square_dispatch(a, kSquareRope, stream);
   if (gemm_stream_rope_supports(a, EPI)) return gemm_stream_rope_dispatch(a, stream);
   const long tiles256 = (long)((a.M + 255) / 256) * (total_n(a) / 128), tiles128 = (long)((a.M + 127) / 128) * (total_n(a) / 128);
   int tile = tiles256 > 256 && !prefers_small_tiles(tiles256, tiles128) ? 256 : 128;

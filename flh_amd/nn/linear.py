@@ -56,7 +56,8 @@ class LinearFLH(torch.nn.Module):
     #   one scale per channel: 2048 x 4096 34.5 / 34.9 / 40.7, 3000 x 4096 49 / 43 / 52, 2400 x 11008 109 / 82 / 90; 2048 x 11008 89 / 79 / 87 in
     #   a graph, 84 / 84 as separate calls, and a layer of 1400 tokens whose gate and up change over is slower, 380 / 409
     #   a scale per token: 640 x 4096 25.7 / 28.5 / 28.4, 1280 x 4096 45 / 35 / 42, 1000 x 14336 95 / 70 / 79, 640 x 4096 of K = 11008 63 / 54 / 58
-    #   group scales: 512 x 4096 25.7 / 26.3 / 29.5, 640 x 4096 31.8 / 30.0 / 30.2, 1000 x 4096 38 / 33 / 33, 512 x 4096 of K = 11008 60 / 54 / 57;
+    #   group scales: 640 x 4096 27 / 30 / 30, 1000 x 4096 28 / 33 / 33, 640 x 11008 52 / 51 / 55, 800 x 11008 74 / 68 / 70, 1000 x 14336 98 / 76 / 84,
+    #   512 x 4096 of K = 11008 60 / 54 / 57;
     #   320 x 11008 52 / 43 / 46, but the host's part of the encoding makes a layer of 300 or 450 tokens slower (245 / 262; 500: 271 / 263)
     TRANSIENT_ROWS = (2560, 641)
     TRANSIENT_ROWS_GROUPS = 513
@@ -65,7 +66,7 @@ class LinearFLH(torch.nn.Module):
     def _transient_tiles(self, grouped, nibbles, groups=False):
         long_k = self.in_features > 8192
         if grouped and groups:
-            return (128 if nibbles else 95) if long_k else 160 if nibbles else 143
+            return (128 if nibbles else 95) if long_k else 256
         if grouped:
             return 191 if long_k else 256
         return 1280 if nibbles and not long_k else 512
