@@ -95,6 +95,24 @@ __device__ __forceinline__ void load_to_lds16(const void* sbase, unsigned voffse
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(sbase) : "memory", "m0");
 }
 
+// a pointer that is the same in every lane, as scalar registers
+template <typename T>
+__device__ __forceinline__ T* wave_uniform(T* q) {
+  const uint64_t v = (uint64_t)q;
+  return (T*)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+              (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v));
+}
+
+// buffer descriptor of `bytes` from `base` on (wave-uniform); loads beyond read zero
+__device__ __forceinline__ v4i buffer_of(const uint8_t* base, unsigned bytes) {
+  const uint64_t b = (uint64_t)wave_uniform(base);
+  return v4i{(int)(unsigned)b, (int)(unsigned)(b >> 32), (int)bytes, 0x00020000};
+}
+__device__ __forceinline__ void buffer_advance(v4i& d, uint64_t step) {
+  const uint64_t b = ((uint64_t)(unsigned)d[1] << 32 | (unsigned)d[0]) + step;
+  d[0] = (int)(unsigned)b, d[1] = (int)(unsigned)(b >> 32);
+}
+
 // Workgroup barrier without the memory fence of __syncthreads(): the fence makes every wave wait for ALL of
 // its outstanding LDS reads and global loads, which drains a software pipeline at every use.  For callers
 // that order their own memory traffic with explicit waits; the "memory" clobber keeps the compiler from

@@ -67,23 +67,7 @@ __device__ __forceinline__ Tile tile_of(const GemmArgs& p, unsigned L) {
   return t;
 }
 
-// a pointer that is the same in every lane, as scalar registers
-template <typename T>
-__device__ __forceinline__ T* wave_uniform(T* q) {
-  const uint64_t v = (uint64_t)q;
-  return (T*)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-              (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v));
-}
-
-// ---- operand loads through buffer descriptors: `bytes` from `base` on, anything beyond reads as zero
-__device__ __forceinline__ v4i buffer_of(const uint8_t* base, unsigned bytes) {
-  const uint64_t b = (uint64_t)wave_uniform(base);
-  return v4i{(int)(unsigned)b, (int)(unsigned)(b >> 32), (int)bytes, 0x00020000};
-}
-__device__ __forceinline__ void buffer_advance(v4i& d, uint64_t step) {
-  const uint64_t b = ((uint64_t)(unsigned)d[1] << 32 | (unsigned)d[0]) + step;
-  d[0] = (int)(unsigned)b, d[1] = (int)(unsigned)(b >> 32);
-}
+// ---- operand loads through buffer descriptors
 // 3 KiB in three instructions: lane i's 16 bytes at voff, + 1024, + 2048 go to lds_base + 16 i, + 1024, + 2048
 __device__ __forceinline__ void load_block_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\t"

@@ -19,6 +19,16 @@
 // receives element i % 4 of the 8-byte rows addressed by lanes i / 4 + 4 j, j = 0..3), i.e. four consecutive keys for
 // the lane's channel straight from the row-major tile.  Online softmax in base 2 per lane; only the running maximum is
 // exchanged between the two lanes of a query per key block.
+//
+// Sixteen fragments of four registers serve both products: while the scores' MFMAs use up the step's K, V is read into the
+// registers they leave, and the next step's K while the second product uses up V; the second half of the exponentials sits
+// between MFMAs too.  A wave waits for LDS only at the step's one barrier.
+// What bounds it: power on long launches (8192 tokens of 32 heads: 1.8 GHz, where the form that read fragments right before
+// use ran at 2.0, and took 15 % more clocks per step; MFMAs alone take 364 us at 1.8 GHz, the fragment reads add 59, the loads 57, the
+// exponentials 36), clocks on short ones.  us before -> now: 1 x 8192 tokens 602 -> 597, 1 x 4096 of 8 key / value heads 181 -> 171,
+// 1 x 2048 54 -> 49.4, 2 x 1500 behind 100 82 -> 76, 1 x 1000 behind 531 36.7 -> 31.8, 1 x 513 15.3 -> 13.5, 8 x 512 37.5 -> 36.5.
+// Not taken: a running maximum that may lag behind by 8 powers of two, 3-6 % faster (fewer rescaled steps) but with the largest
+// probabilities rounded instead of 1 (largest error at 1000 behind 531 9.7e-5 -> 1.6e-4); raised wave priority around the MFMAs: nothing.
 #include <atomic>
 
 #include "lane_ops.h"
@@ -43,6 +53,19 @@ __device__ __forceinline__ int chunk_at(int r, int c) { return r * (kHeadDim * 2
 // four consecutive rows, which must fall into four different quarters of the 256-byte bank line
 __device__ __forceinline__ int v_swizzle(int r) { return (r & 3) << 2; }
 __device__ __forceinline__ int v_chunk_at(int r, int c) { return r * (kHeadDim * 2) + ((c ^ v_swizzle(r)) << 4); }
+
+// 1 KiB: lane i's 16 bytes at voff go to lds_base + 16 i
+__device__ __forceinline__ void load_rows_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
+}
+// the same four times, 1 KiB further in memory and in LDS each
+__device__ __forceinline__ void load_four_rows_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\t"
+               "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
+               "buffer_load_dwordx4 %1, %2, 0 offen offset:1024 lds\n\t"
+               "buffer_load_dwordx4 %1, %2, 0 offen offset:2048 lds\n\t"
+               "buffer_load_dwordx4 %1, %2, 0 offen offset:3072 lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
+}
 
 __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half* __restrict__ q,
                                                                    const __half* __restrict__ k_cache,
@@ -78,40 +101,34 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half*
   const int total_keys = past + T;
   const int block_keys = min(past + (qb + 1) * kQueriesPerBlock, total_keys);   // slots any query of the block sees
   const int n_steps = (block_keys + kKeysPerStep - 1) / kKeysPerStep;
-  const __half* kbase = k_cache + ((size_t)b * Hkv + hkv) * (size_t)max_len * kHeadDim;
-  const __half* vbase = v_cache + ((size_t)b * Hkv + hkv) * (size_t)max_len * kHeadDim;
+  // steps with a key that some query of this wave sees, and whether the last of them has one in its second tile of 32
+  const int wave_limit = past + min(q_first + 31, T - 1);
+  const int live_steps = __builtin_amdgcn_readfirstlane(q_first < T ? wave_limit / kKeysPerStep + 1 : 0);
+  const bool half_step = __builtin_amdgcn_readfirstlane(wave_limit % kKeysPerStep < 32);
+  const size_t cache = ((size_t)b * Hkv + hkv) * (size_t)max_len * kHeadDim;
   const unsigned lds0 = (unsigned)(size_t)lds;
 
-  // one load instruction moves four key rows (1 KiB); a wave issues four for K and four for V per step.  A full step
-  // takes its rows from a wave-uniform base (the step's first key) plus per-lane byte offsets that never change; the
-  // last step of a sequence may run past the end and clamps its rows.
-  unsigned k_off[4], v_off[4];
+  // one load instruction moves four key rows (1 KiB); a wave issues four for K and four for V per step.  The descriptors
+  // cover what is left of a step's 64 rows: rows past the end arrive as zeros
+  unsigned k_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = (wave * 4 + i) * 4 + (lane >> 4);
     k_off[i] = (unsigned)(r * kHeadDim + ((lane & 15) ^ (r & 15)) * 8) * 2;
-    v_off[i] = (unsigned)(r * kHeadDim + ((lane & 15) ^ v_swizzle(r)) * 8) * 2;
   }
-  auto issue = [&](int step, int buf) {
-    const int first = step * kKeysPerStep;
-    if (first + kKeysPerStep <= total_keys) {
-      const __half* kb = kbase + (size_t)first * kHeadDim;
-      const __half* vb = vbase + (size_t)first * kHeadDim;
+  const unsigned v_off = (unsigned)((wave * 16 + (lane >> 4)) * kHeadDim + ((lane & 15) ^ v_swizzle(lane >> 4)) * 8) * 2;
+  const uint8_t *k_next = (const uint8_t*)(k_cache + cache), *v_next = (const uint8_t*)(v_cache + cache);   // the steps requested next
+  int k_left = total_keys, v_left = total_keys;        // keys from there on
+  auto rows_left = [](int keys) { return (unsigned)__builtin_amdgcn_readfirstlane(max(0, min(keys, kKeysPerStep)) * (kHeadDim * 2)); };
+  auto issue_k = [&](int buf) {
+    const v4i d = buffer_of(k_next, rows_left(k_left));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        load_to_lds16(kb, k_off[i], lds0 + buf * kTileBytes + (wave * 4 + i) * 1024);
-        load_to_lds16(vb, v_off[i], lds0 + (2 + buf) * kTileBytes + (wave * 4 + i) * 1024);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int inst = wave * 4 + i;                 // 0 .. 15
-        const int r = inst * 4 + (lane >> 4);
-        const size_t row = (size_t)min(first + r, total_keys - 1) * kHeadDim;
-        load_to_lds16(kbase + row + ((lane & 15) ^ (r & 15)) * 8, lds0 + buf * kTileBytes + inst * 1024);
-        load_to_lds16(vbase + row + ((lane & 15) ^ v_swizzle(r)) * 8, lds0 + (2 + buf) * kTileBytes + inst * 1024);
-      }
-    }
+    for (int i = 0; i < 4; ++i) load_rows_to_lds(d, k_off[i], lds0 + buf * kTileBytes + (wave * 4 + i) * 1024);
+    k_next += kTileBytes, k_left -= kKeysPerStep;
+  };
+  auto issue_v = [&](int buf) {
+    load_four_rows_to_lds(buffer_of(v_next, rows_left(v_left)), v_off, lds0 + (2 + buf) * kTileBytes + wave * 4096);
+    v_next += kTileBytes, v_left -= kKeysPerStep;
   };
 
   v16f o[4];                                           // O^T: [channel tile], lane = query, register r = channel 8 (r/4) + 4 h + r % 4
@@ -122,6 +139,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half*
   float m_run = -INFINITY, l_run = 0.f;                // running maximum (scaled, base 2) and this lane's share of the sum
   const int q_limit = past + my_q;                     // last visible slot of this lane's query
 
+  // K fragment 2 s + kt of a step: rows 32 kt + n, channels 16 s + 8 h .. + 7 (chunk 2 s + h; s enters the swizzled address by XOR)
+  const int k_at = chunk_at(n, h);
   // per-lane offsets of the V^T transpose loads: lane i of a group of 16 addresses the 8-byte piece (i % 4) of the
   // 32-byte run of channels the group's sixteen lanes will own, in key row i / 4 of the four keys of one load
   const int grp = lane >> 4, gi = lane & 15;
@@ -133,45 +152,46 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half*
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) tr_off[dt] = v_chunk_at(4 * (grp >> 1) + tr_key, 4 * dt + tr_chunk0) + tr_half;
 
-  issue(0, 0);
-  for (int step = 0; step < n_steps; ++step) {
-    const int buf = step & 1;
+  h8 f[16];                                            // the fragments of one operand: K's during the scores, V's afterwards
+  auto read_k = [&](auto j_, int buf, int at) {
+    constexpr int j = decltype(j_)::value;
+    f[j] = *(const h8*)(lds + buf * kTileBytes + (at ^ ((j >> 1) << 5)) + (j & 1) * (32 * kHeadDim * 2));
+  };
+  // V fragment 4 (2 kt + ks) + dt: this half-wave's slots 8 h .. 8 h + 7 are keys 32 kt + 16 ks + 4 h + {0..3} and + 8 + {0..3}
+  // (rows 32 kt + 16 ks and + 8 on: multiples of four, which the V swizzle does not see)
+  auto read_v = [&](auto j_, int buf) {
+    constexpr int j = decltype(j_)::value;
+    const uint8_t* at = lds + (2 + buf) * kTileBytes + tr_off[j & 3] + (j >> 2) * (16 * kHeadDim * 2);
+    const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)at);
+    const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(at + 8 * (kHeadDim * 2)));
+    f[j] = __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+  // Step `step` with K and V of it in the buffers of parity P
+  auto run = [&](auto p_, int step) {
+    constexpr int P = decltype(p_)::value;
     wait_vmcnt<0>();
-    __syncthreads();                                   // tile `step` is complete; everybody is done with the other buffer
-    if (step + 1 < n_steps) issue(step + 1, buf ^ 1);
-    const uint8_t* kt_lds = lds + buf * kTileBytes;
-    const uint8_t* vt_lds = lds + (2 + buf) * kTileBytes;
-
-    // keys a wave's queries cannot see cost it nothing: a 32-key tile past the wave's last query is skipped
-    // (the wave still takes part in the loads and barriers of the step)
-    const int wave_limit = past + min(q_first + 31, T - 1);
-    const int live_tiles = __builtin_amdgcn_readfirstlane(
-        step * kKeysPerStep > wave_limit ? 0 : (step * kKeysPerStep + 32 > wave_limit ? 1 : 2));
-    if (live_tiles == 0) continue;
-
-    // ---- S^T = K Q^T for two tiles of 32 keys: all fragments are requested first, then the two accumulator chains
-    // alternate (a tile the wave cannot see is computed and masked like any other: straight-line code schedules better)
-    h8 kf[2][8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) kf[kt][s] = *(const h8*)(kt_lds + chunk_at(kt * 32 + n, 2 * s + h));
-    __builtin_amdgcn_sched_barrier(0);                 // (keeps the compiler from sinking the reads to their uses)
+    __syncthreads();                                   // V of this step and K of the next are complete; everybody has read the buffers refilled here
+    issue_k(P);
+    issue_v(P ^ 1);
+    if (step >= live_steps) return;
+    // ---- S^T = K Q^T for two tiles of 32 keys; every fragment's registers take one of V's
     v16f st[2];
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[kt][r] = 0.f;
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kt][s], qf[s], st[kt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<16>([&](auto j_) {
+      constexpr int j = decltype(j_)::value;
+      st[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[j], qf[j >> 1], st[j & 1], 0, 0, 0);
+      read_v(j_, P);
+      __builtin_amdgcn_sched_barrier(0);
+    });
     // ---- causal mask, online softmax in base 2 on scale_log2 * s (register r of tile kt: key = 64 step + 32 kt +
     // 8 (r/4) + 4 h + r % 4)
     const int key0 = step * kKeysPerStep + 4 * h;
-    const bool diagonal = __builtin_amdgcn_readfirstlane(step * kKeysPerStep + kKeysPerStep - 1 > past + q_first);
-    float mx = -INFINITY;
-    if (diagonal) {                                    // (a branch of its own: most steps carry no mask arithmetic at all;
+    if (step * kKeysPerStep + kKeysPerStep - 1 > past + q_first) {   // (a branch of its own: most steps carry no mask arithmetic at all;
       asm volatile("" ::: "memory");                   //  the empty statement keeps the compiler from predicating it)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -180,24 +200,17 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half*
           if (key0 + 32 * kt + 8 * (r >> 2) + (r & 3) > q_limit) st[kt][r] = -INFINITY;
     }
     __builtin_amdgcn_sched_barrier(0);
+    float mx[4];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int c = 0; c < 4; ++c) {
+      mx[c] = fmaxf(st[c >> 1][8 * (c & 1)], st[c >> 1][8 * (c & 1) + 1]);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[kt][r]);
-    mx = fmaxf(mx, lane_xor_f<32>(mx)) * scale_log2;   // (the scale is positive: the maximum commutes with it)
-    const float m_new = fmaxf(m_run, mx);              // finite from the first step on: slot 0 is visible to every query
-    float sum = 0.f;
-    h8 pb[2][2];                                       // P^T as B operand: [tile][step of 16 slots]
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][8 * ks + i], scale_log2, -m_new));
-          sum += p;
-          pb[kt][ks][i] = (_Float16)p;
-        }
+      for (int r = 2; r < 8; ++r) mx[c] = fmaxf(mx[c], st[c >> 1][8 * (c & 1) + r]);
+    }
+    float top = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_int(top), __float_as_int(top), false, false);
+    top = fmaxf(__int_as_float(halves[0]), __int_as_float(halves[1])) * scale_log2;   // (the scale is positive: the maximum commutes with it)
+    const float m_new = fmaxf(m_run, top);             // finite from the first step on: slot 0 is visible to every query
     // rescale what has been accumulated -- unless no lane's maximum moved (the common case after the first steps)
     if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -208,26 +221,49 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half*
         for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
       m_run = m_new;
     }
+    float sum = 0.f;
+    h8 pb[2][2];                                       // P^T as B operand: [tile][step of 16 slots]
+    auto two = [&](auto kt_, auto i_) {                // probabilities 2 i and 2 i + 1 of a tile
+      constexpr int kt = decltype(kt_)::value, i = decltype(i_)::value;
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][2 * i], scale_log2, -m_run));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][2 * i + 1], scale_log2, -m_run));
+      sum += p0, sum += p1;
+      pb[kt][i >> 2][(2 * i) & 7] = (_Float16)p0, pb[kt][i >> 2][(2 * i + 1) & 7] = (_Float16)p1;
+    };
+    static_for<8>([&](auto i_) { two(std::integral_constant<int, 0>{}, i_); });
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- O^T += V^T P^T, a tile's MFMAs between the next tile's exponentials; every fragment's registers take one of the next step's K
+    int k_now = k_at;
+    asm("" : "+v"(k_now));                             // (eight addresses kept across the steps are registers there are not)
+    const bool half = half_step && step + 1 == live_steps;
+    static_for<8>([&](auto j_) {
+      constexpr int j = decltype(j_)::value;
+      o[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[j], pb[0][j >> 2], o[j & 3], 0, 0, 0);
+      read_k(j_, P ^ 1, k_now);
+      two(std::integral_constant<int, 1>{}, j_);
+      __builtin_amdgcn_sched_barrier(0);
+    });
     l_run += sum;
-    // ---- O^T += V^T P^T
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      if (kt >= live_tiles) break;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        // this half-wave's slots 8 h .. 8 h + 7 are keys 32 kt + 16 ks + 4 h + {0..3} and + 8 + {0..3}
-        // (rows 32 kt + 16 ks and + 8 on: multiples of four, which the V swizzle does not see)
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const uint8_t* at = vt_lds + tr_off[dt] + (32 * kt + 16 * ks) * (kHeadDim * 2);
-          const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)at);
-          const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(at + 8 * (kHeadDim * 2)));
-          const h8 a = __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[kt][ks], o[dt], 0, 0, 0);
-        }
-      }
-    }
+    if (half) return;                                  // (the wave's last step, whose second tile it does not see)
+    static_for<8>([&](auto j_) {
+      constexpr int j = decltype(j_)::value + 8;
+      o[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[j], pb[1][(j >> 2) & 1], o[j & 3], 0, 0, 0);
+      read_k(std::integral_constant<int, j>{}, P ^ 1, k_now);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
+  issue_k(0);
+  issue_v(0);
+  issue_k(1);
+  wait_vmcnt<8>();                                     // K of step 0
+  barrier_no_fence();
+  static_for<16>([&](auto j_) { read_k(j_, 0, k_at); });
+  for (int step = 0; step < n_steps; step += 2) {
+    run(std::integral_constant<int, 0>{}, step);
+    if (step + 1 < n_steps) run(std::integral_constant<int, 1>{}, step + 1);
   }
+  wait_vmcnt<0>();                                     // (zeros requested past the last step must not land in the staging tiles)
 
   // ---- normalise, transpose through LDS, store whole rows
   const float l_all = l_run + lane_xor_f<32>(l_run);

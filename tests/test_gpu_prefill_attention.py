@@ -93,3 +93,12 @@ def test_prefill_attention_argument_checks():
     with pytest.raises(RuntimeError):
         ops.prefill_attention(q, torch.zeros(1, 3, 8, 128, dtype=torch.float16, device="cuda"),
                               torch.zeros(1, 3, 8, 128, dtype=torch.float16, device="cuda"), 0)
+
+
+@pytest.mark.parametrize("spare", [0, 70])
+@pytest.mark.parametrize("t,past", [(1, 62), (1, 63), (1, 64), (33, 31), (63, 0), (65, 0), (96, 33), (97, 160), (128, 64), (161, 95)])
+def test_prefill_attention_at_the_edges_of_key_blocks(t, past, spare):
+    """Key counts around the blocks of 64 and the tiles of 32, blocks whose last waves have no query or see half a key block,
+    a cache that ends with the last key and one with garbage behind it."""
+    print(f"case prefill attention edges t={t} past={past} spare={spare}", flush=True)
+    run(2, t, 4, 2, past, t + past, max_len=past + t + spare)
