@@ -20,6 +20,17 @@ gemm_i4_dequant_o16_gs = _ext.gemm_i4_dequant_o16_gs
 gemm_i4_dequant_multi = _ext.gemm_i4_dequant_multi
 gemm_i4_swiglu = _ext.gemm_i4_swiglu
 gemm_i4_dequant_add = _ext.gemm_i4_dequant_add
+gemm_i4_qkv_rope = _ext.gemm_i4_qkv_rope
+encode_f6_many = _ext.encode_f6_many
+group_quantize_f6 = _ext.group_quantize_f6
+rmsnorm_group_quantize_f6 = _ext.rmsnorm_group_quantize_f6
+silu_mul_group_quantize_f6 = _ext.silu_mul_group_quantize_f6
+gemm_f6_dequant_o16 = _ext.gemm_f6_dequant_o16
+gemm_f6_dequant_o16_gs = _ext.gemm_f6_dequant_o16_gs
+gemm_f6_dequant_add = _ext.gemm_f6_dequant_add
+gemm_f6_qkv_rope = _ext.gemm_f6_qkv_rope
+gemm_f6_swiglu = _ext.gemm_f6_swiglu
+gemm_f6_dequant_multi = _ext.gemm_f6_dequant_multi
 prefill_attention = _ext.prefill_attention
 rope_kv_cache_ = _ext.rope_kv_cache_
 rotate_quantize_gemm_i4 = _ext.rotate_quantize_gemm_i4
@@ -56,5 +67,13 @@ def rmsnorm_rotate_and_quantize_i4(x, weight, eps, hadamard=True, clip_ratio=1.0
                                                           return_rotated))
 
 
-def __getattr__(name):        # ops the extension does not wrap (6-bit path, int32 output, tuning hook, ...)
+def add_rmsnorm_rotate_and_quantize_i4(x, add, weight, eps, hadamard=True, clip_ratio=1.0):
+    return tuple(_ext.add_rmsnorm_rotate_and_quantize_i4_mode(x, add, weight, eps, _ops._whole_row_mode(hadamard), clip_ratio))
+
+
+def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None):
+    return tuple(_ext.rotate_and_quantize_f6_mode(x, _ops._f6_mode(x, hadamard, eps, add) if x.dim() == 2 else 0, clip_ratio, norm_weight, eps, add))
+
+
+def __getattr__(name):        # ops the extension does not wrap (one matrix's encoding, int32 output, tuning hook, ...)
     return getattr(_ops, name)

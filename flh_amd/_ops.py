@@ -961,6 +961,18 @@ def add_rmsnorm_rotate_and_quantize_i4(x, add, weight, eps, hadamard=True, clip_
     return total, q, s
 
 
+def _f6_mode(x, hadamard, eps, add):
+    """hadamard argument of rotate_and_quantize_f6 -> mode of the C ABI."""
+    K = x.size(-1)
+    dense = K in (11008, 14336)
+    _check(dense or K in (512, 1024, 2048, 4096, 8192), "Last dimension must be a power of two in 512 .. 8192, 11008 or 14336")
+    if dense:
+        _check(hadamard in (True, "fast") and eps is None and add is None, "K = 11008 / 14336: matrix-core rotation, no prologue")
+        return FLH_HAD_MFMA
+    _check(hadamard != "fast" or K == 4096, "power-of-two K: the matrix-core rotation ('fast') exists for K = 4096")
+    return _whole_row_mode(hadamard)
+
+
 def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None):
     """rotate_and_quantize_i4 (one scale per token) with the codes written in the 6-bit operand format of gemm_f6_*
     directly: x [M, K] fp16 -> (encoded [M, K / 128 * 96] u8, scales [M, 1] fp16), the bytes of encode_f6(q).
@@ -970,14 +982,7 @@ def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, e
     _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
            "Input tensor must be a contiguous 2D float16 CUDA tensor")
     M, K = x.shape
-    dense = K in (11008, 14336)
-    _check(dense or K in (512, 1024, 2048, 4096, 8192), "Last dimension must be a power of two in 512 .. 8192, 11008 or 14336")
-    if dense:
-        _check(hadamard in (True, "fast") and eps is None and add is None, "K = 11008 / 14336: matrix-core rotation, no prologue")
-        mode = FLH_HAD_MFMA
-    else:
-        _check(hadamard != "fast" or K == 4096, "power-of-two K: the matrix-core rotation ('fast') exists for K = 4096")
-        mode = _whole_row_mode(hadamard)
+    mode = _f6_mode(x, hadamard, eps, add)
     _check(add is None or eps is not None, "the residual addition comes with the RMSNorm prologue (eps)")
     if add is not None:
         _check(add.is_cuda and add.dtype == torch.float16 and add.shape == x.shape and add.is_contiguous()

@@ -111,18 +111,19 @@ Tensor gemm_i4_dequant_o16_gs(const Tensor& A, const Tensor& B, const Tensor& A_
   return gemm_checked(A, B, A_scale, B_scale, group_size);
 }
 
+void check_output_shaped(const Tensor& t, const char* what, int64_t M, int64_t N, const Tensor& A) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat16 && t.is_contiguous() && t.device() == A.device(), what,
+              " must be a contiguous float16 CUDA tensor on the operands' device");
+  TORCH_CHECK(t.numel() == M * N && t.dim() >= 1 && t.size(-1) == N, what, " must have the shape of the output");
+}
+
 // fp16(residual + gemm): a decoder layer's residual addition in the GEMM's epilogue; `out` may be the residual itself
 Tensor gemm_i4_dequant_add(const Tensor& A, const Tensor& B, const Tensor& A_scale, const Tensor& B_scale,
                            const Tensor& residual, int64_t group_size, const c10::optional<Tensor>& out) {
   check_gemm_inputs(A, B, A_scale, B_scale);
   const int64_t M = A.size(0), N = B.size(0), K = A.size(1) * 2;
-  auto shaped = [&](const Tensor& t, const char* what) {
-    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat16 && t.is_contiguous() && t.device() == A.device(), what,
-                " must be a contiguous float16 CUDA tensor on the operands' device");
-    TORCH_CHECK(t.numel() == M * N && t.dim() >= 1 && t.size(-1) == N, what, " must have the shape of the output");
-  };
-  shaped(residual, "the residual");
-  if (out.has_value()) shaped(*out, "out");
+  check_output_shaped(residual, "the residual", M, N, A);
+  if (out.has_value()) check_output_shaped(*out, "out", M, N, A);
   Tensor D = out.has_value() ? *out : torch::empty({M, N}, A_scale.options());
   if (M == 0 || N == 0) return D;
   Launch l(A);
@@ -199,6 +200,286 @@ std::vector<Tensor> gemm_i4_dequant_multi(const Tensor& A, const std::vector<Ten
   Launch l(A);
   ok(flh_gemm_i4_o16_multi(u8(A), h(A_scale), (int)Bs.size(), b, bs, d, n, M, K, (int)A_scale.size(1),
                            (int)B_scales[0].size(1), (int)group_size, stream_of(A)));
+  return Ds;
+}
+
+// ---- q / k / v with the rotary embedding and the cache write in the GEMM's epilogue ------------------------------------------
+struct RopeShape { int64_t T, Hq, Hkv, max_len; };
+
+RopeShape check_rope_cache(int64_t M, int64_t batch, const std::vector<Tensor>& Bs, const Tensor& cos, const Tensor& sin,
+                           const Tensor& positions, const Tensor& k_cache, const Tensor& v_cache, const Tensor& A) {
+  TORCH_CHECK(batch > 0 && M % batch == 0, "the rows of A must be batch * T tokens");
+  const int64_t T = M / batch;
+  TORCH_CHECK(Bs[0].size(0) % 128 == 0 && Bs[1].size(0) % 128 == 0 && Bs[1].size(0) == Bs[2].size(0),
+              "q / k / v must have whole heads of 128 channels, k and v the same number");
+  const int64_t Hq = Bs[0].size(0) / 128, Hkv = Bs[1].size(0) / 128;
+  for (const Tensor* c : {&cos, &sin})
+    TORCH_CHECK(c->is_cuda() && c->scalar_type() == torch::kFloat16 && c->is_contiguous() && c->dim() == 2 && c->size(0) == T &&
+                    c->size(1) == 128 && c->device() == A.device(),
+                "cos / sin must be contiguous float16 CUDA tensors [T, 128]");
+  TORCH_CHECK(positions.is_cuda() && positions.scalar_type() == torch::kInt64 && positions.is_contiguous() &&
+                  positions.numel() == T && positions.device() == A.device(),
+              "positions must be a contiguous int64 CUDA tensor [T]");
+  for (const Tensor* c : {&k_cache, &v_cache})
+    TORCH_CHECK(c->is_cuda() && c->scalar_type() == torch::kFloat16 && c->is_contiguous() && c->dim() == 4 &&
+                    c->device() == A.device() && c->size(0) == batch && c->size(1) == Hkv && c->size(3) == 128 &&
+                    c->sizes() == k_cache.sizes(),
+                "the caches must be contiguous float16 CUDA tensors [batch, kv_heads, max_len, 128]");
+  return {T, Hq, Hkv, k_cache.size(2)};
+}
+
+// the operands of q, k and v for the C ABI
+struct ThreeOf {
+  const uint8_t* b[3];
+  const flh_half* s[3];
+  ThreeOf(const std::vector<Tensor>& Bs, const std::vector<Tensor>& Ss) {
+    for (int i = 0; i < 3; ++i) b[i] = u8(Bs[i]), s[i] = h(Ss[i]);
+  }
+};
+
+Tensor gemm_i4_qkv_rope(const Tensor& A, const Tensor& A_scale, const std::vector<Tensor>& Bs, const std::vector<Tensor>& B_scales,
+                        const Tensor& cos, const Tensor& sin, const Tensor& positions, Tensor k_cache, Tensor v_cache, int64_t batch,
+                        int64_t group_size) {
+  TORCH_CHECK(Bs.size() == 3 && B_scales.size() == 3, "three weight matrices (q, k, v), one scale tensor each");
+  for (int i = 0; i < 3; ++i) {
+    check_gemm_inputs(A, Bs[i], A_scale, B_scales[i]);
+    TORCH_CHECK(B_scales[i].size(1) == B_scales[0].size(1), "B_scale shapes");
+  }
+  const int64_t M = A.size(0), K = A.size(1) * 2;
+  const RopeShape r = check_rope_cache(M, batch, Bs, cos, sin, positions, k_cache, v_cache, A);
+  Tensor q_out = torch::empty({batch, r.T, r.Hq, 128}, A_scale.options());
+  if (M == 0) return q_out;
+  const ThreeOf w(Bs, B_scales);
+  Launch l(A);
+  ok(flh_gemm_i4_qkv_rope_o16(u8(A), h(A_scale), w.b, w.s, h(cos), h(sin), (const int64_t*)positions.data_ptr(), hm(q_out),
+                              hm(k_cache), hm(v_cache), (uint32_t)batch, (uint32_t)r.T, (uint32_t)r.Hq, (uint32_t)r.Hkv,
+                              (uint32_t)r.max_len, K, (int)A_scale.size(1), (int)B_scales[0].size(1), (int)group_size, stream_of(A)));
+  return q_out;
+}
+
+// ---- the 6-bit operand format -------------------------------------------------------------------------------------------
+std::vector<Tensor> encode_f6_many(const std::vector<Tensor>& packed) {
+  TORCH_CHECK(!packed.empty() && packed.size() <= 4, "one to four matrices");
+  for (const Tensor& p : packed) {
+    TORCH_CHECK(p.is_cuda() && p.scalar_type() == torch::kUInt8 && p.dim() == 2 && p.is_contiguous() &&
+                    p.device() == packed[0].device(),
+                "packed codes must be contiguous 2D uint8 CUDA tensors on one device");
+    TORCH_CHECK(p.size(1) == packed[0].size(1), "the matrices must share K");
+  }
+  const int64_t K = packed[0].size(1) * 2;
+  TORCH_CHECK(K % 128 == 0, "K must be a multiple of 128");
+  std::vector<Tensor> outs;
+  const uint8_t* in[4];
+  uint8_t* out[4];
+  size_t rows[4];
+  for (size_t i = 0; i < packed.size(); ++i) {
+    outs.push_back(torch::empty({packed[i].size(0), K / 128 * 96}, packed[i].options()));
+    in[i] = u8(packed[i]);
+    out[i] = (uint8_t*)outs[i].data_ptr();
+    rows[i] = (size_t)packed[i].size(0);
+  }
+  if (K) {
+    Launch l(packed[0]);
+    ok(flh_encode_f6_multi((int)packed.size(), in, out, rows, K, stream_of(packed[0])));
+  }
+  return outs;
+}
+
+struct F6Rows {   // rows of fp16 values and where their codes and group scales go
+  int64_t M, K;
+  Tensor q, s;
+  explicit F6Rows(const Tensor& x) {
+    TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat16 && x.dim() == 2 && x.is_contiguous(),
+                "Input tensor must be a contiguous 2D float16 CUDA tensor");
+    M = x.size(0), K = x.size(1);
+    TORCH_CHECK(K % 128 == 0 && K > 0, "Last dimension must be a multiple of 128");
+  }
+  void allocate(const Tensor& x) {
+    q = torch::empty({M, K / 128 * 96}, x.options().dtype(torch::kUInt8));
+    s = torch::empty({M, K / 128}, x.options());
+  }
+};
+
+std::vector<Tensor> group_quantize_f6(const Tensor& x, bool hadamard, double scale_mul) {
+  F6Rows r(x);
+  r.allocate(x);
+  if (r.M) {
+    Launch l(x);
+    ok(flh_group_quant_f6(h(x), (uint8_t*)r.q.data_ptr(), hm(r.s), (uint32_t)r.M, (uint32_t)r.K, hadamard ? 1 : 0, (float)scale_mul,
+                          stream_of(x)));
+  }
+  return {r.q, r.s};
+}
+
+std::vector<Tensor> rmsnorm_group_quantize_f6(const Tensor& x, const c10::optional<Tensor>& weight, double eps) {
+  F6Rows r(x);
+  TORCH_CHECK(r.K <= 16384, "Last dimension must be at most 16384");
+  if (weight.has_value())
+    TORCH_CHECK(weight->is_cuda() && weight->scalar_type() == torch::kFloat16 && weight->is_contiguous() &&
+                    weight->numel() == r.K && weight->device() == x.device(),
+                "weight must be a contiguous float16 CUDA tensor of K values");
+  r.allocate(x);
+  if (r.M) {
+    Launch l(x);
+    ok(flh_rmsnorm_group_quant_f6(h(x), weight.has_value() ? h(*weight) : nullptr, (uint8_t*)r.q.data_ptr(), hm(r.s), (uint32_t)r.M,
+                                  (uint32_t)r.K, (float)eps, stream_of(x)));
+  }
+  return {r.q, r.s};
+}
+
+std::vector<Tensor> silu_mul_group_quantize_f6(const Tensor& gate, const Tensor& up) {
+  F6Rows r(gate);
+  TORCH_CHECK(up.is_cuda() && up.scalar_type() == torch::kFloat16 && up.sizes() == gate.sizes() && up.is_contiguous() &&
+                  up.device() == gate.device(),
+              "gate and up must be contiguous float16 CUDA tensors of one shape");
+  r.allocate(gate);
+  if (r.M) {
+    Launch l(gate);
+    ok(flh_silu_mul_group_quant_f6(h(gate), h(up), (uint8_t*)r.q.data_ptr(), hm(r.s), (uint32_t)r.M, (uint32_t)r.K, stream_of(gate)));
+  }
+  return {r.q, r.s};
+}
+
+// K of the encoded operands
+int64_t check_f6(const Tensor& A6, const Tensor& B6) {
+  TORCH_CHECK(A6.is_cuda() && B6.is_cuda(), "tensors must be CUDA");
+  TORCH_CHECK(A6.scalar_type() == torch::kUInt8 && B6.scalar_type() == torch::kUInt8, "encoded operands must be uint8");
+  TORCH_CHECK(A6.is_contiguous() && B6.is_contiguous(), "tensors must be contiguous");
+  TORCH_CHECK(A6.dim() == 2 && B6.dim() == 2 && A6.size(1) == B6.size(1) && A6.size(1) % 96 == 0,
+              "encoded operands must be 2D with equal K");
+  TORCH_CHECK(A6.device() == B6.device(), "tensors must be on one device");
+  return A6.size(1) / 96 * 128;
+}
+void check_f6_scale(const Tensor& S, int64_t rows, const Tensor& A6, const char* what) {
+  TORCH_CHECK(S.is_cuda() && S.scalar_type() == torch::kFloat16 && S.is_contiguous() && S.dim() == 2 && S.size(0) == rows &&
+                  S.device() == A6.device(),
+              what, " must be a contiguous float16 CUDA tensor, one row of scales per row of its operand");
+}
+void check_f6_columns(const Tensor& A_scale, const Tensor& B_scale, int64_t ng) {
+  const int64_t a = A_scale.size(1), b = B_scale.size(1);
+  TORCH_CHECK((a == 1 && b == 1) || (b == ng && (a == 1 || a == ng)), "scale columns must be (1, 1), (1, K/128) or (K/128, K/128)");
+}
+
+Tensor gemm_f6_dequant_o16(const Tensor& A6, const Tensor& B6, const Tensor& A_scale, const Tensor& B_scale) {
+  const int64_t K = check_f6(A6, B6), M = A6.size(0), N = B6.size(0);
+  TORCH_CHECK(A_scale.is_cuda() && B_scale.is_cuda() && A_scale.scalar_type() == torch::kFloat16 &&
+                  B_scale.scalar_type() == torch::kFloat16,
+              "scales must be float16 CUDA tensors");
+  TORCH_CHECK(A_scale.is_contiguous() && B_scale.is_contiguous() && A_scale.numel() == M && B_scale.numel() == N,
+              "one scale per row of A and of B expected");
+  TORCH_CHECK(A_scale.device() == A6.device() && B_scale.device() == A6.device(), "tensors must be on one device");
+  Tensor D = torch::empty({M, N}, A_scale.options());
+  if (M == 0 || N == 0) return D;
+  Launch l(A6);
+  ok(flh_gemm_f6_o16(u8(A6), u8(B6), h(A_scale), h(B_scale), hm(D), M, N, K, stream_of(A6)));
+  return D;
+}
+
+Tensor gemm_f6_dequant_o16_gs(const Tensor& A6, const Tensor& B6, const Tensor& A_scale, const Tensor& B_scale) {
+  const int64_t K = check_f6(A6, B6), M = A6.size(0), N = B6.size(0), ng = K / 128;
+  check_f6_scale(A_scale, M, A6, "A_scale");
+  check_f6_scale(B_scale, N, A6, "B_scale");
+  TORCH_CHECK(A_scale.size(1) == 1 || A_scale.size(1) == ng, "A_scale must be [M, K/128] or [M, 1]");
+  TORCH_CHECK(B_scale.size(1) == ng, "B_scale must be [N, K/128]");
+  Tensor D = torch::empty({M, N}, A_scale.options());
+  if (M == 0 || N == 0) return D;
+  Launch l(A6);
+  ok(flh_gemm_f6_o16_gs(u8(A6), u8(B6), h(A_scale), h(B_scale), hm(D), M, N, K, (int)A_scale.size(1), (int)ng, stream_of(A6)));
+  return D;
+}
+
+Tensor gemm_f6_dequant_add(const Tensor& A6, const Tensor& B6, const Tensor& A_scale, const Tensor& B_scale, const Tensor& residual,
+                           const c10::optional<Tensor>& out) {
+  const int64_t K = check_f6(A6, B6), M = A6.size(0), N = B6.size(0);
+  check_f6_scale(A_scale, M, A6, "A_scale");
+  check_f6_scale(B_scale, N, A6, "B_scale");
+  check_f6_columns(A_scale, B_scale, K / 128);
+  check_output_shaped(residual, "the residual", M, N, A6);
+  if (out.has_value()) check_output_shaped(*out, "out", M, N, A6);
+  Tensor D = out.has_value() ? *out : torch::empty({M, N}, A_scale.options());
+  if (M == 0 || N == 0) return D;
+  Launch l(A6);
+  ok(flh_gemm_f6_add_o16(u8(A6), u8(B6), h(A_scale), h(B_scale), h(residual), hm(D), M, N, K, (int)A_scale.size(1),
+                         (int)B_scale.size(1), stream_of(A6)));
+  return D;
+}
+
+Tensor gemm_f6_qkv_rope(const Tensor& A6, const Tensor& A_scale, const std::vector<Tensor>& B6s, const std::vector<Tensor>& B_scales,
+                        const Tensor& cos, const Tensor& sin, const Tensor& positions, Tensor k_cache, Tensor v_cache, int64_t batch) {
+  TORCH_CHECK(B6s.size() == 3 && B_scales.size() == 3, "three weight matrices (q, k, v), one scale tensor each");
+  int64_t K = 0;
+  for (int i = 0; i < 3; ++i) {
+    K = check_f6(A6, B6s[i]);
+    check_f6_scale(B_scales[i], B6s[i].size(0), A6, "B_scale");
+    TORCH_CHECK(B_scales[i].size(1) == B_scales[0].size(1), "B_scale shapes");
+  }
+  const int64_t M = A6.size(0);
+  check_f6_scale(A_scale, M, A6, "A_scale");
+  check_f6_columns(A_scale, B_scales[0], K / 128);
+  const RopeShape r = check_rope_cache(M, batch, B6s, cos, sin, positions, k_cache, v_cache, A6);
+  Tensor q_out = torch::empty({batch, r.T, r.Hq, 128}, A_scale.options());
+  if (M == 0) return q_out;
+  const ThreeOf w(B6s, B_scales);
+  Launch l(A6);
+  ok(flh_gemm_f6_qkv_rope_o16(u8(A6), h(A_scale), w.b, w.s, h(cos), h(sin), (const int64_t*)positions.data_ptr(), hm(q_out),
+                              hm(k_cache), hm(v_cache), (uint32_t)batch, (uint32_t)r.T, (uint32_t)r.Hq, (uint32_t)r.Hkv,
+                              (uint32_t)r.max_len, K, (int)A_scale.size(1), (int)B_scales[0].size(1), stream_of(A6)));
+  return q_out;
+}
+
+Tensor gemm_f6_swiglu(const Tensor& A6, const Tensor& B6_gate, const Tensor& B6_up, const Tensor& A_scale, const Tensor& gate_scale,
+                      const Tensor& up_scale) {
+  const int64_t K = check_f6(A6, B6_gate), M = A6.size(0), N = B6_gate.size(0);
+  TORCH_CHECK(check_f6(A6, B6_up) == K && B6_up.size(0) == N, "gate and up must have the same shapes");
+  check_f6_scale(A_scale, M, A6, "A_scale");
+  check_f6_scale(gate_scale, N, A6, "gate_scale");
+  check_f6_scale(up_scale, N, A6, "up_scale");
+  TORCH_CHECK(up_scale.sizes() == gate_scale.sizes(), "weight scales must be [N, 1] or [N, K/128], the same for gate and up");
+  check_f6_columns(A_scale, gate_scale, K / 128);
+  Tensor D = torch::empty({M, N}, A_scale.options());
+  if (M == 0 || N == 0) return D;
+  Launch l(A6);
+  ok(flh_gemm_f6_swiglu_o16(u8(A6), u8(B6_gate), u8(B6_up), h(A_scale), h(gate_scale), h(up_scale), hm(D), M, N, K,
+                            (int)A_scale.size(1), (int)gate_scale.size(1), stream_of(A6)));
+  return D;
+}
+
+std::vector<Tensor> gemm_f6_dequant_multi(const Tensor& A6, const std::vector<Tensor>& B6s, const Tensor& A_scale,
+                                          const std::vector<Tensor>& B_scales) {
+  TORCH_CHECK(B6s.size() == B_scales.size() && !B6s.empty() && B6s.size() <= 4,
+              "one to four weight matrices, one scale tensor each");
+  int64_t K = 0;
+  bool empty = A6.dim() == 2 && A6.size(0) == 0;
+  for (size_t i = 0; i < B6s.size(); ++i) {
+    K = check_f6(A6, B6s[i]);
+    check_f6_scale(B_scales[i], B6s[i].size(0), A6, "B_scale");
+    TORCH_CHECK(B_scales[i].size(1) == B_scales[0].size(1), "B_scale shapes");
+    empty = empty || B6s[i].size(0) == 0;
+  }
+  const int64_t M = A6.size(0);
+  check_f6_scale(A_scale, M, A6, "A_scale");
+  check_f6_columns(A_scale, B_scales[0], K / 128);
+  std::vector<Tensor> Ds;
+  if (empty) {
+    const bool rows = A_scale.size(1) == 1 && B_scales[0].size(1) == 1;
+    for (size_t i = 0; i < B6s.size(); ++i)
+      Ds.push_back(rows ? gemm_f6_dequant_o16(A6, B6s[i], A_scale, B_scales[i]) : gemm_f6_dequant_o16_gs(A6, B6s[i], A_scale, B_scales[i]));
+    return Ds;
+  }
+  const uint8_t* b[4];
+  const flh_half* bs[4];
+  flh_half* d[4];
+  size_t n[4];
+  for (size_t i = 0; i < B6s.size(); ++i) {
+    Ds.push_back(torch::empty({M, B6s[i].size(0)}, A_scale.options()));
+    b[i] = u8(B6s[i]);
+    bs[i] = h(B_scales[i]);
+    d[i] = hm(Ds[i]);
+    n[i] = (size_t)B6s[i].size(0);
+  }
+  Launch l(A6);
+  ok(flh_gemm_f6_o16_multi(u8(A6), h(A_scale), (int)B6s.size(), b, bs, d, n, M, K, (int)A_scale.size(1), (int)B_scales[0].size(1),
+                           stream_of(A6)));
   return Ds;
 }
 
@@ -348,6 +629,60 @@ std::vector<Tensor> rmsnorm_rotate_and_quantize_i4_mode(const Tensor& x, const c
                                    (float)clip_ratio, stream_of(x)));
   }
   if (return_rotated) return {q, s, y};
+  return {q, s};
+}
+
+// x + add, then RMSNorm, rotation and quantiser: {x + add, codes, scales}
+std::vector<Tensor> add_rmsnorm_rotate_and_quantize_i4_mode(const Tensor& x, const Tensor& add, const c10::optional<Tensor>& weight,
+                                                            double eps, int64_t mode, double clip_ratio) {
+  TORCH_CHECK(x.is_cuda() && add.is_cuda() && x.device() == add.device(), "Input tensors must be on CUDA");
+  TORCH_CHECK(x.scalar_type() == torch::kFloat16 && add.scalar_type() == torch::kFloat16, "Input tensors must be float16 (half)");
+  TORCH_CHECK(x.dim() == 2 && x.sizes() == add.sizes() && x.is_contiguous() && add.is_contiguous(),
+              "x and add must be contiguous 2D tensors of one shape");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(K == 512 || K == 1024 || K == 2048 || K == 4096 || K == 8192,
+              "Last dimension must be 512, 1024, 2048, 4096 or 8192");
+  if (weight.has_value())
+    TORCH_CHECK(weight->is_cuda() && weight->scalar_type() == torch::kFloat16 && weight->is_contiguous() && weight->numel() == K,
+                "weight must be a contiguous float16 CUDA tensor of K values");
+  Tensor total = torch::empty_like(x);
+  Tensor q = torch::empty({M, K / 2}, x.options().dtype(torch::kUInt8));
+  Tensor s = torch::empty({M, 1}, x.options());
+  if (M) {
+    Launch l(x);
+    ok(flh_add_rmsnorm_rotate_quant_i4(h(x), h(add), hm(total), weight.has_value() ? h(*weight) : nullptr, (float)eps,
+                                       (uint8_t*)q.data_ptr(), hm(s), (uint32_t)M, (uint32_t)K, (int)mode, (float)clip_ratio,
+                                       stream_of(x)));
+  }
+  return {total, q, s};
+}
+
+// codes in the 6-bit operand format: {codes, scales}, behind {x + add, ...} if there is one
+std::vector<Tensor> rotate_and_quantize_f6_mode(const Tensor& x, int64_t mode, double clip_ratio, const c10::optional<Tensor>& norm_weight,
+                                                const c10::optional<double>& eps, const c10::optional<Tensor>& add) {
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat16 && x.dim() == 2 && x.is_contiguous(),
+              "Input tensor must be a contiguous 2D float16 CUDA tensor");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(!add.has_value() || eps.has_value(), "the residual addition comes with the RMSNorm prologue (eps)");
+  if (add.has_value())
+    TORCH_CHECK(add->is_cuda() && add->scalar_type() == torch::kFloat16 && add->sizes() == x.sizes() && add->is_contiguous() &&
+                    add->device() == x.device(),
+                "add must be a contiguous float16 CUDA tensor of x's shape");
+  if (norm_weight.has_value())
+    TORCH_CHECK(eps.has_value() && norm_weight->is_cuda() && norm_weight->scalar_type() == torch::kFloat16 &&
+                    norm_weight->is_contiguous() && norm_weight->numel() == K && norm_weight->device() == x.device(),
+                "norm_weight must be a contiguous float16 CUDA tensor of K values (with eps)");
+  Tensor q = torch::empty({M, K / 128 * 96}, x.options().dtype(torch::kUInt8));
+  Tensor s = torch::empty({M, 1}, x.options());
+  Tensor total;
+  if (add.has_value()) total = torch::empty_like(x);
+  if (M) {
+    Launch l(x);
+    ok(flh_rotate_quant_f6(h(x), add.has_value() ? h(*add) : nullptr, add.has_value() ? hm(total) : nullptr, eps.has_value() ? 1 : 0,
+                           norm_weight.has_value() ? h(*norm_weight) : nullptr, (float)eps.value_or(0.0), (uint8_t*)q.data_ptr(), hm(s),
+                           (uint32_t)M, (uint32_t)K, (int)mode, (float)clip_ratio, stream_of(x)));
+  }
+  if (add.has_value()) return {total, q, s};
   return {q, s};
 }
 
@@ -555,6 +890,23 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rotate_quantize_gemm_i4_multi", &rotate_quantize_gemm_i4_multi, py::arg("x"), py::arg("Bs"), py::arg("B_scales"));
   m.def("rope_kv_cache_", &rope_kv_cache_, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cos"), py::arg("sin"),
         py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"));
+  m.def("gemm_i4_qkv_rope", &gemm_i4_qkv_rope, py::arg("A"), py::arg("A_scale"), py::arg("Bs"), py::arg("B_scales"), py::arg("cos"),
+        py::arg("sin"), py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"), py::arg("batch"), py::arg("group_size") = 128);
+  m.def("encode_f6_many", &encode_f6_many, py::arg("packed"));
+  m.def("group_quantize_f6", &group_quantize_f6, py::arg("x"), py::arg("hadamard") = true, py::kw_only(), py::arg("scale_mul") = 1.0);
+  m.def("rmsnorm_group_quantize_f6", &rmsnorm_group_quantize_f6, py::arg("x"), py::arg("weight"), py::arg("eps"));
+  m.def("silu_mul_group_quantize_f6", &silu_mul_group_quantize_f6, py::arg("gate"), py::arg("up"));
+  m.def("gemm_f6_dequant_o16", &gemm_f6_dequant_o16, py::arg("A6"), py::arg("B6"), py::arg("A_scale"), py::arg("B_scale"));
+  m.def("gemm_f6_dequant_o16_gs", &gemm_f6_dequant_o16_gs, py::arg("A6"), py::arg("B6"), py::arg("A_scale"), py::arg("B_scale"));
+  m.def("gemm_f6_dequant_add", &gemm_f6_dequant_add, py::arg("A6"), py::arg("B6"), py::arg("A_scale"), py::arg("B_scale"),
+        py::arg("residual"), py::arg("out") = py::none());
+  m.def("gemm_f6_qkv_rope", &gemm_f6_qkv_rope, py::arg("A6"), py::arg("A_scale"), py::arg("B6s"), py::arg("B_scales"), py::arg("cos"),
+        py::arg("sin"), py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"), py::arg("batch"));
+  m.def("gemm_f6_swiglu", &gemm_f6_swiglu, py::arg("A6"), py::arg("B6_gate"), py::arg("B6_up"), py::arg("A_scale"),
+        py::arg("gate_scale"), py::arg("up_scale"));
+  m.def("gemm_f6_dequant_multi", &gemm_f6_dequant_multi, py::arg("A6"), py::arg("B6s"), py::arg("A_scale"), py::arg("B_scales"));
+  m.def("add_rmsnorm_rotate_and_quantize_i4_mode", &add_rmsnorm_rotate_and_quantize_i4_mode);
+  m.def("rotate_and_quantize_f6_mode", &rotate_and_quantize_f6_mode);
   m.def("linear_i4", &linear_i4);
   m.def("linear_online_i4", &linear_online_i4);
   m.def("quantize_groups", &quantize_groups);

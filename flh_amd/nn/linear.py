@@ -93,8 +93,8 @@ class LinearFLH(torch.nn.Module):
             self._six_bit_weights()
 
     def _six_bit_weights(self):
-        if not self._keeps_six_bit(self.w_scale.view(self.out_features, -1).size(1) > 1):
-            return _pkg._CUDA.encode_f6(self.w_packed.view(self.out_features, self.in_features // 2))
+        if not self._keeps_six_bit(self.w_scale.numel() > self.out_features):
+            return _pkg._CUDA.encode_f6_many([self.w_packed.view(self.out_features, self.in_features // 2)])[0]
         key = (self.w_packed.data_ptr(), self.w_packed._version, self.w_packed.device)
         if self._w6 is None or self._w6_key != key:
             self._w6 = _pkg._CUDA.encode_f6(self.w_packed.view(self.out_features, self.in_features // 2))
@@ -115,16 +115,20 @@ class LinearFLH(torch.nn.Module):
         """Whether a call with `n_rows` rows quantised per token (or, `groups`, per group of 128) takes the 6-bit matrix
         instruction (a producer can then write the activations in that format directly, rotate_and_quantize_f6).
         `columns`: channels of the whole launch, where several layers share one."""
-        if (n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS_GROUPS) or self.in_features % 128 or not self.w_packed.is_cuda:
+        if self._below_six_bit(n_rows) or self.in_features % 128 or not self.w_packed.is_cuda:
             return False
-        cols = self.w_scale.view(self.out_features, -1).size(1)
+        cols = self.w_scale.numel() // self.out_features
         if cols != 1 and not (cols == self.in_features // 128 and self.weight_group_size == 128):
             return False
         return self._six_bit_rows(cols != 1, columns, False, groups) <= n_rows <= self._SIX_BIT_MAX_ROWS
 
+    def _below_six_bit(self, n_rows):
+        """Whether `n_rows` rows are fewer than any setting takes to the 6-bit instruction."""
+        return n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS_GROUPS
+
     def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)
-        if (n < self.six_bit_min_rows and n < self.TRANSIENT_ROWS_GROUPS) or not rows.is_cuda or self.in_features % 128:
+        if self._below_six_bit(n) or not rows.is_cuda or self.in_features % 128:
             return False
         per_row = a_scale.size(1) == 1 and w_scale.size(1) == 1
         grouped = group == 128 and w_scale.size(1) == self.in_features // 128 and a_scale.size(1) in (1, w_scale.size(1))
@@ -232,15 +236,16 @@ class LinearFLH(torch.nn.Module):
         group = gate_layer.weight_group_size if gate_layer.weight_group_size > 0 else (gate_layer.in_group_size or 128)
         a_rows = a_scale.reshape(rows.size(0), -1)
         encoded = rows.size(1) * 4 == k * 3                     # activations already in the 6-bit format
-        six = [l._six_bit_applies(rows, a_rows, l.w_scale.view(n, -1), group, 2 * n) for l in (gate_layer, up_layer)]
-        if encoded or all(six):
+        both = (gate_layer, up_layer)
+        if encoded or not any(l._below_six_bit(rows.size(0)) for l in both) and all(
+                l._six_bit_applies(rows, a_rows, l.w_scale.view(n, -1), group, 2 * n) for l in both):
             ops = _pkg._CUDA
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            y = ops.gemm_f6_swiglu(a6, *LinearFLH._six_bit_weights_of((gate_layer, up_layer)), a_rows.contiguous(),
+            y = ops.gemm_f6_swiglu(a6, *LinearFLH._six_bit_weights_of(both), a_rows.contiguous(),
                                    gate_layer.w_scale.view(n, -1), up_layer.w_scale.view(n, -1))
             return y.view(*lead, n)
         y = _pkg._CUDA.gemm_i4_swiglu(rows, gate_layer.w_packed.view(n, k // 2), up_layer.w_packed.view(n, k // 2),
-                                      a_scale.reshape(rows.size(0), -1), gate_layer.w_scale.view(n, -1),
+                                      a_rows, gate_layer.w_scale.view(n, -1),
                                       up_layer.w_scale.view(n, -1), group)
         return y.view(*lead, n)
 

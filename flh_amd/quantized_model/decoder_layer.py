@@ -466,7 +466,7 @@ class W4A4DecoderLayer(torch.nn.Module):
             return None
         layers = (self.q_proj, self.k_proj, self.v_proj)
         group = self.q_proj.weight_group_size if self.q_proj.weight_group_size > 0 else (self.q_proj.in_group_size or 128)
-        six = all(l._six_bit_applies(codes.reshape(rows, -1), scales.reshape(rows, -1), l.w_scale.view(l.out_features, -1), group,
+        six = not any(l._below_six_bit(rows) for l in layers) and all(l._six_bit_applies(codes.reshape(rows, -1), scales.reshape(rows, -1), l.w_scale.view(l.out_features, -1), group,
                                        sum(c.out_features for c in layers)) for l in layers)
         return "f6" if six else "i4"
 
@@ -518,15 +518,16 @@ class W4A4DecoderLayer(torch.nn.Module):
     def _online_qkv_applies(self):
         """q / k / v in the layout the decode GEMM with its own norm + quantiser takes: no bias, one scale per channel or
         per group of 128, the same for all three."""
-        cols = {l.w_scale.view(l.out_features, -1).size(1) for l in (self.q_proj, self.k_proj, self.v_proj)}
-        if any(l.bias is not None for l in (self.q_proj, self.k_proj, self.v_proj)) or len(cols) != 1:
+        layers = (self.q_proj, self.k_proj, self.v_proj)
+        cols = {l.w_scale.numel() // l.out_features for l in layers}
+        if any(l.bias is not None for l in layers) or len(cols) != 1:
             return False
         c = cols.pop()
         return c == 1 or (c == self.hidden_size // 128 and self.q_proj.weight_group_size == 128)
 
     def _swiglu_gemm_applies(self):
         g = self.gate_proj
-        cols = g.w_scale.view(g.out_features, -1).size(1)
+        cols = g.w_scale.numel() // g.out_features
         return g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
 
     def _group_quant(self, stage, quantizer, x, consumers=()):
