@@ -18,7 +18,7 @@
 //   17-64 tokens: 4096 x 4096 21.1 -> 8.2, 11008 x 4096 50 -> 17, 14336 x 4096 68 -> 21, 4096 x 28672 40 -> 20 (32), 31 (64)
 //   128: 4096 x 4096 21.7 -> 10.9, 4096 x 6144 22.2 -> 14.3;  256: 4096 x 4096 21.8 -> 15.7;  512: 4096 x 1024 18.3 -> 10.3
 //   16 tokens: 4096 x 28672 22.5 -> 15.7, 4096 x 14336 13.9 -> 9.8 (5 and 3.7 TB/s of weights)
-// and with one scale per row: 64 tokens 4096 x 14336 28.4 -> 13, 4096 x 4096 8.3 -> 6.5; 128: 11008 x 4096 25 -> 18.
+// One scale per row has a kernel of its own below (gemm_i4_dealt_kernel).
 #include "gemm_i4.h"
 
 namespace flh {
@@ -37,6 +37,21 @@ typedef __attribute__((address_space(3))) uint8_t lds_byte;
 template <typename T>
 __device__ __forceinline__ T from_lds(const lds_byte* q) { return *(const __attribute__((address_space(3))) T*)q; }
 
+// channels n .. n + 3 of row m
+__device__ __forceinline__ void store_four(const GemmArgs& p, void* Dp, int N, int m, int n, const _Float16 (&y)[4]) {
+  const size_t at = (size_t)m * N + n;
+  if (N % 4 == 0) {
+    if (n >= N) return;
+    h4 v = {y[0], y[1], y[2], y[3]};
+    if (p.R) v = v + *(const h4*)((const _Float16*)p.R + at);   // (R may be D: read before the store)
+    *(h4*)((_Float16*)Dp + at) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) ((_Float16*)Dp)[at + e] = p.R ? y[e] + ((const _Float16*)p.R)[at + e] : y[e];
+  }
+}
+
 template <int TN>
 struct StageRegs {                                 // a wave's operands of one stage
   v4i a[kStageGroups], b[TN][kStageGroups];
@@ -45,7 +60,6 @@ struct StageRegs {                                 // a wave's operands of one s
 
 template <int WM, int WN, int TN, int S, int EPI, int OUT>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const GemmArgs p) {
-  constexpr bool GROUPED = EPI != kRowScale;
   constexpr int WAVES = WM * WN, RA = 16 * WM, RB = 16 * TN * WN, ROWS = RA + RB;
   constexpr int STAGE = ROWS * kRowBytes;
   constexpr int NA = RA / 4 / WAVES, NB = RB / 4 / WAVES, NI = NA + NB;   // 1 KiB load instructions per wave and stage
@@ -80,7 +94,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
 
   // scales first, as their rows are: [row][KT / 2 pairs, an odd number of slots] in LDS, every wave a share of them
   const int pitch = (KT >> 1) | 1;
-  if constexpr (GROUPED) {
+  {
     const float inv = 1.0f / (float)pitch;
     const int total = SROWS * pitch;
     for (int f0 = wave * 64; f0 < total; f0 += WAVES * 64) {
@@ -127,28 +141,24 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
       for (int j = 0; j < TN; ++j) q.b[j][g] = from_lds<v4i>(st + chunk[g] + (RA + (wn * TN + j) * 16) * kRowBytes);
       q.a[g] = from_lds<v4i>(st + chunk[g] + wm * 16 * kRowBytes);
     }
-    if constexpr (GROUPED) {
-      const int at = first_group(s) >> 1;
-      auto two = [&](int row) {
-        const __attribute__((address_space(3))) unsigned* e = (const __attribute__((address_space(3))) unsigned*)scales + row * pitch + at;
-        return v2u{e[0], e[1]};
-      };
-      if constexpr (EPI == kGroupScale) q.sa = two(wm * 16 + r);
+    const int at = first_group(s) >> 1;
+    auto two = [&](int row) {
+      const __attribute__((address_space(3))) unsigned* e = (const __attribute__((address_space(3))) unsigned*)scales + row * pitch + at;
+      return v2u{e[0], e[1]};
+    };
+    if constexpr (EPI == kGroupScale) q.sa = two(wm * 16 + r);
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q.sb[j][e] = two(SROWS - RB + (wn * TN + j) * 16 + 4 * c + e);
-    }
+      for (int e = 0; e < 4; ++e) q.sb[j][e] = two(SROWS - RB + (wn * TN + j) * 16 + 4 * c + e);
   };
-  v4i acc[TN];
   float out[TN][4];
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    acc[j] = v4i{0, 0, 0, 0};
+  for (int j = 0; j < TN; ++j)
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[j][e] = 0.f;
-  }
-  auto product = [&](const v4i& a, const v4i& b, v4i d) {
+  auto product = [&](const v4i& a, const v4i& b) {
+    v4i d = {0, 0, 0, 0};
     v4i alo, ahi, blo, bhi;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -169,22 +179,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
     }
   };
   auto multiply = [&](const StageRegs<TN>& q) {    // a whole stage: all products, then their folds in ascending order
-    if constexpr (GROUPED) {
-      v4i d[kStageGroups][TN];
+    v4i d[kStageGroups][TN];
 #pragma unroll
-      for (int g = 0; g < kStageGroups; ++g)
+    for (int g = 0; g < kStageGroups; ++g)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) d[g][j] = product(q.a[g], q.b[j][g], v4i{0, 0, 0, 0});
-      static_for<kStageGroups>([&](auto G) {
+      for (int j = 0; j < TN; ++j) d[g][j] = product(q.a[g], q.b[j][g]);
+    static_for<kStageGroups>([&](auto G) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) fold(G, j, d[decltype(G)::value][j], q);
-      });
-    } else {
-#pragma unroll
-      for (int g = 0; g < kStageGroups; ++g)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[j] = product(q.a[g], q.b[j][g], acc[j]);
-    }
+      for (int j = 0; j < TN; ++j) fold(G, j, d[decltype(G)::value][j], q);
+    });
   };
 
 #pragma unroll
@@ -217,10 +220,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
       constexpr int g = decltype(G)::value;
       if (g < skip) return;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        if constexpr (GROUPED) fold(G, j, product(q.a[g], q.b[j][g], v4i{0, 0, 0, 0}), q);
-        else acc[j] = product(q.a[g], q.b[j][g], acc[j]);
-      }
+      for (int j = 0; j < TN; ++j) fold(G, j, product(q.a[g], q.b[j][g]), q);
     });
   };
   arrive(stages >= S);                             // stage 0; slot S - 1 is free
@@ -248,11 +248,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
     for (int e = 0; e < 4; ++e) {
       float v;
       if constexpr (EPI == kGroupScale) v = out[j][e] * 0.00390625f;
-      else if constexpr (EPI == kTokenGroup) v = round_here(out[j][e] * 0.00390625f) * __half2float(p.As[m]);
-      else {
-        const float s_a = __half2float(p.As[m]), s_b = __half2float(Bs[min(first(wn * TN + j) + 4 * c + e, N - 1)]) * 0.00390625f;
-        v = (float)acc[j][e] * (s_a * s_b);
-      }
+      else v = round_here(out[j][e] * 0.00390625f) * __half2float(p.As[m]);
       y[j][e] = (_Float16)round_here(v);
     }
   if constexpr (OUT == kStreamRope) {
@@ -277,38 +273,208 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int n = first(wn * TN + j) + 4 * c;
-      const size_t at = (size_t)m * N + n;
-      if (N % 4 == 0) {
-        if (n >= N) continue;
-        h4 v = {y[j][0], y[j][1], y[j][2], y[j][3]};
-        if (p.R) v = v + *(const h4*)((const _Float16*)p.R + at);   // (R may be D: read before the store)
-        *(h4*)((_Float16*)Dp + at) = v;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) ((_Float16*)Dp)[at + e] = p.R ? y[j][e] + ((const _Float16*)p.R)[at + e] : y[j][e];
-      }
+      store_four(p, Dp, N, m, n, y[j]);
     }
   }
 }
 
-template <int WM, int WN, int TN, int S, int EPI, int OUT>
-int launch_stream(GemmArgs a, hipStream_t stream) {
-  constexpr int RA = 16 * WM, RB = 16 * TN * WN, BN = RB;
+template <int RA, int RB, int OUT>
+void set_stream_tiles(GemmArgs& a) {
   a.tiles_m = (a.M + RA - 1) / RA;
-  auto tiles = [&](int n) { return OUT == kStreamRope ? (n + 127) / 128 * 4 : (n + BN - 1) / BN; };
+  auto tiles = [&](int n) { return OUT == kStreamRope ? (n + 127) / 128 * 4 : (n + RB - 1) / RB; };
   a.tiles_n = tiles(a.N);
   for (int s = 1; s < a.n_seg; ++s) {
     a.seg_tile0[s] = a.tiles_n;
     a.tiles_n += tiles(a.seg_N[s]);
   }
+}
+
+template <int WM, int WN, int TN, int S, int EPI, int OUT>
+int launch_stream(GemmArgs a, hipStream_t stream) {
+  constexpr int RA = 16 * WM, RB = 16 * TN * WN;
+  set_stream_tiles<RA, RB, OUT>(a);
   constexpr size_t ring = (size_t)S * (RA + RB) * kRowBytes;
     // (rounded up to whole load instructions)
-  auto table = [](int kt) { return EPI == kRowScale ? 0 : ((size_t)((kt / 2) | 1) * (EPI == kGroupScale ? RA + RB : RB) * 4 + 255) / 256 * 256; };
+  auto table = [](int kt) { return ((size_t)((kt / 2) | 1) * (EPI == kGroupScale ? RA + RB : RB) * 4 + 255) / 256 * 256; };
   auto kern = gemm_i4_stream_kernel<WM, WN, TN, S, EPI, OUT>;
   static LdsGrant grant;                               // per instantiation; sized for the longest rows it takes
   if (int rc = reserve_lds((const void*)kern, ring + table(kStreamMaxGroups), grant, "gemm (stream)")) return rc;
   hipLaunchKernelGGL(kern, dim3(a.tiles_m * a.tiles_n), dim3(64 * WM * WN), ring + table(a.K >> 7), stream, a);
+  return check_launch("gemm_i4_stream");
+}
+
+// One scale per row: a stage's four groups are dealt out to the four waves.  Wave w multiplies group w for the whole tile -- 16
+// tokens x 64 channels as four 16 x 16 products, 32 or 64 tokens x 32 channels as one or two 32 x 32 ones -- so that an operand is
+// unpacked once and not by every wave whose product it enters; the integer sums meet at the end, through the ring's LDS.
+// (Group scales have to be folded in order: handing the sums over stage by stage costs what the unpacking saves, 45 x 4096 x
+// 11008 15.8 -> 16.7.  Two waves per 16 x 16 tile, two groups each, the same: 16.0.)
+template <int TOK, int S>
+__global__ __launch_bounds__(256) void gemm_i4_dealt_kernel(const GemmArgs p) {
+  constexpr bool SMALL = TOK == 16;
+  constexpr int RA = TOK, RB = SMALL ? 64 : 32, STAGE = (RA + RB) * kRowBytes, NI = (RA + RB) / 16;
+  constexpr int TT = SMALL ? 1 : TOK / 32, C = SMALL ? 1 : 2;   // token tiles; 16-byte pieces of a row's group per lane
+  static_assert((RA + RB) % 16 == 0 && (S - 2) * NI < 64 && 12 * TT * 1024 <= S * STAGE, "loads per stage, exchange");
+  extern __shared__ __align__(16) uint8_t lds[];
+  lds_byte* ring = (lds_byte*)lds;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r = lane % (SMALL ? 16 : 32), c = lane / (SMALL ? 16 : 32);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned L = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int bn = L / p.tiles_m, bm = L % p.tiles_m;
+
+  const uint8_t* B = p.B;
+  const __half* Bs = p.Bs;
+  void* Dp = p.D;
+  int N = p.N, t = bn;
+  for (int s = 1; s < p.n_seg; ++s)
+    if (bn >= p.seg_tile0[s]) B = p.seg_B[s], Bs = p.seg_Bs[s], Dp = p.seg_D[s], N = p.seg_N[s], t = bn - p.seg_tile0[s];
+  const int Kb = p.K >> 1, KT = p.K >> 7;
+  const int stages = (KT + kStageGroups - 1) / kStageGroups;
+  const int m0 = bm * RA, n0 = t * RB;
+  auto first_group = [&](int s) { return min(s * kStageGroups, KT - kStageGroups); };   // the last stage ends with the row
+
+  // a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16)
+  const uint8_t* src[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = (i * 4 + wave) * 4 + (lane >> 4);
+    src[i] = (row < RA ? p.A + (size_t)min(m0 + row, p.M - 1) * Kb : B + (size_t)min(n0 + max(row - RA, 0), N - 1) * Kb) +
+             ((lane & 15) ^ (row & 15)) * 16;
+  }
+  const unsigned base = (unsigned)(uintptr_t)ring;
+  auto request = [&](int s, int slot) {
+    const size_t off = (size_t)first_group(s) * 64;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) load_to_lds16(src[i] + off, base + slot + (i * 4 + wave) * (4 * kRowBytes));
+  };
+  int piece[C];                                    // of the wave's group in the lane's row
+#pragma unroll
+  for (int i = 0; i < C; ++i) piece[i] = r * kRowBytes + ((wave * 4 + c + 2 * i) ^ (r & 15)) * 16;
+  struct Operands { v4i a[TT][C], b[SMALL ? 4 : C]; };
+  auto read = [&](int slot, Operands& q) {
+    const lds_byte* st = ring + slot;
+#pragma unroll
+    for (int i = 0; i < (SMALL ? 4 : C); ++i)
+      q.b[i] = from_lds<v4i>(st + (SMALL ? piece[0] + i * (16 * kRowBytes) : piece[SMALL ? 0 : i]) + RA * kRowBytes);
+#pragma unroll
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+      for (int i = 0; i < C; ++i) q.a[j][i] = from_lds<v4i>(st + piece[i] + j * (32 * kRowBytes));
+  };
+  auto lo = [](v4i x) { return (x << 4) & (int)0xF0F0F0F0; };
+  auto hi = [](v4i x) { return x & (int)0xF0F0F0F0; };
+  v16i wide[TT];                                   // 32 x 32: quarter q (registers 4 q ..) is folded by wave q
+  v4i part[4];                                     // 16 x 16: tile q
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[i] = v4i{0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < TT; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) wide[j][i] = 0;
+  auto multiply = [&](const Operands& q) {
+    if constexpr (SMALL) {
+      const v4i al = lo(q.a[0][0]), ah = hi(q.a[0][0]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        part[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo(q.b[i]), al, part[i], 0, 0, 0);
+        part[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi(q.b[i]), ah, part[i], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const v4i bl = lo(q.b[i]), bh = hi(q.b[i]);
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+          wide[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bl, lo(q.a[j][i]), wide[j], 0, 0, 0);
+          wide[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bh, hi(q.a[j][i]), wide[j], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < stages) request(s, s * STAGE);
+  // every wave's loads of the oldest stage but `newer` are in LDS, every wave has its last stage in registers
+  auto arrive = [&](bool steady) {
+    if (steady) wait_vmcnt<(S - 2) * NI>();
+    else wait_vmcnt<0>();
+    wait_lgkmcnt0();
+    barrier_no_fence();
+  };
+  Operands q0, q1;
+  int slot = 0;                                    // of stage s
+  auto step = [&](int s, Operands& cur, Operands& next) {   // s + 1 < stages
+    arrive(s + S - 1 < stages);
+    if (s + S < stages) request(s + S, slot);
+    slot = slot == (S - 1) * STAGE ? 0 : slot + STAGE;
+    read(slot, next);
+    __builtin_amdgcn_sched_barrier(0);             // (the reads have the products' time to arrive)
+    multiply(cur);
+  };
+  auto last = [&](const Operands& q) {             // without the groups that the stage before has done
+    if (wave >= (stages - 1) * kStageGroups - first_group(stages - 1)) multiply(q);
+  };
+  arrive(stages >= S);                             // stage 0; slot S - 1 is free
+  if (S - 1 < stages) request(S - 1, (S - 1) * STAGE);
+  read(0, q0);
+  int s = 0;
+  for (; s + 2 < stages; s += 2) {
+    step(s, q0, q1);
+    step(s + 1, q1, q0);
+  }
+  if (s + 1 < stages) {
+    step(s, q0, q1);
+    last(q1);
+  } else {
+    last(q0);
+  }
+
+  // every wave's quarter of the sums: [token tile][receiver][sender after it][lane]
+  wait_lgkmcnt0();
+  barrier_no_fence();                              // nobody reads the ring any more
+  v4i sum[TT];
+#pragma unroll
+  for (int j = 0; j < TT; ++j)
+    static_for<4>([&](auto V) {
+      constexpr int v = decltype(V)::value;
+      const v4i d = SMALL ? part[v] : v4i{wide[j][4 * v], wide[j][4 * v + 1], wide[j][4 * v + 2], wide[j][4 * v + 3]};
+      if (wave == v) sum[j] = d;
+      else *(__attribute__((address_space(3))) v4i*)(ring + (j * 12 + v * 3 + ((wave - v + 3) & 3)) * 1024 + lane * 16) = d;
+    });
+  wait_lgkmcnt0();
+  barrier_no_fence();
+#pragma unroll
+  for (int j = 0; j < TT; ++j)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) sum[j] += from_lds<v4i>(ring + (j * 12 + wave * 3 + i) * 1024 + lane * 16);
+
+  // lane: token r of each token tile, four channels
+  const int n = n0 + wave * (SMALL ? 16 : 8) + 4 * c;
+#pragma unroll
+  for (int j = 0; j < TT; ++j) {
+    const int m = m0 + j * 32 + r;
+    if (m >= p.M) return;
+    const float s_a = __half2float(p.As[m]);
+    _Float16 y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float s_b = __half2float(Bs[min(n + e, N - 1)]) * 0.00390625f;
+      y[e] = (_Float16)round_here((float)sum[j][e] * (s_a * s_b));
+    }
+    store_four(p, Dp, N, m, n, y);
+  }
+}
+
+template <int TOK, int S>
+int launch_dealt(GemmArgs a, hipStream_t stream) {
+  constexpr int RA = TOK, RB = TOK == 16 ? 64 : 32;
+  set_stream_tiles<RA, RB, kStreamPlain>(a);
+  constexpr size_t ring = (size_t)S * (RA + RB) * kRowBytes;
+  auto kern = gemm_i4_dealt_kernel<TOK, S>;
+  static LdsGrant grant;
+  if (int rc = reserve_lds((const void*)kern, ring, grant, "gemm (stream)")) return rc;
+  hipLaunchKernelGGL(kern, dim3(a.tiles_m * a.tiles_n), dim3(256), ring, stream, a);
   return check_launch("gemm_i4_stream");
 }
 
@@ -318,16 +484,27 @@ long stream_columns(const GemmArgs& a) {
   return n;
 }
 
-// Tiles, tokens x channels: 16 x 64 for up to 16 tokens, else 32 x 32, or 64 x 32 (half the weight traffic, a fifth less
+// Tiles with group scales, tokens x channels: 16 x 64 for up to 16 tokens, else 32 x 32, or 64 x 32 (half the weight traffic, a fifth less
 // vector work) where nearly two of its workgroups per compute unit remain and the tokens fill it as well as the smaller tile
 // (64 tokens: 4096 x 14336, 448 workgroups, 17.0 against 18.3 us; 256: 4096 x 4096, 512, 15.7 against 18.1; 128: 4096 x 6144,
 // 384, 15.7 against 14.3).
 template <int EPI>
-int launch_stream_by_shape(const GemmArgs& a, hipStream_t stream) {
+int launch_grouped_by_shape(const GemmArgs& a, hipStream_t stream) {
   if (a.M <= 16) return launch_stream<1, 4, 1, 3, EPI, kStreamPlain>(a, stream);
   const long large = (long)((a.M + 63) / 64) * ((stream_columns(a) + 31) / 32);
   if (large >= 448 && (a.M + 31) / 32 % 2 == 0) return launch_stream<4, 1, 2, 3, EPI, kStreamPlain>(a, stream);
   return launch_stream<2, 2, 1, 3, EPI, kStreamPlain>(a, stream);
+}
+
+// ... and with one scale per row: 16 x 64 for up to 16 tokens, else 32 x 32 while three workgroups per compute unit hold all of
+// them, with a longer ring where one does, and 64 x 32 beyond or where K is long.  us, 32 x 32 (ring of 3, of 5) / 64 x 32, K = 4096 unless stated:
+//   45 x 4096 of K = 11008 (256 workgroups of 32 x 32) 11.2, 9.2 / 12.7;  45 x 11008 (688) 9.5, 10.8 / 10.3;  128 x 6144 (768) 9.3, 10.8 / 10.0;
+//   64 x 14336 (896) 13.1 / 11.4;  64 x 28672 (1792) 21.4, 24.1 / 20.5;  128 x 4096 of K = 11008 (512) 15.2, 15.5 / 13.5
+int launch_rows_by_shape(const GemmArgs& a, hipStream_t stream) {
+  if (a.M <= 16) return launch_dealt<16, 3>(a, stream);
+  const long columns = (stream_columns(a) + 31) / 32, small = (long)((a.M + 31) / 32) * columns, large = (long)((a.M + 63) / 64) * columns;
+  if (small > 768 || (a.K > 8192 && small > 256 && large <= 256)) return launch_dealt<64, 3>(a, stream);
+  return small <= 256 ? launch_dealt<32, 5>(a, stream) : launch_dealt<32, 3>(a, stream);
 }
 
 // what the kernel can take: whole stages, and group scales that dword loads can fetch two at a time
@@ -366,30 +543,30 @@ bool takes_few_tokens(const GemmArgs& a, int epi, long columns) {
 // Which launches are faster here than on the kernels on either side.  us, this kernel against the other (K = 4096 unless
 // stated; "large" counts 64 x 32 tiles):
 //  * up to 16 tokens, against the K split of the decode kernel: takes_few_tokens below.
-//  * 17 .. 64 tokens: always, but for one scale per row on at most 128 blocks of 32 channels, where the decode kernel takes 32
-//    (32 x 4096 6.0 against 6.3; 64 x 4096 8.3 against 6.5).
+//  * 17 .. 64 tokens: always (one scale per row, 32 x 4096 5.0 against 5.7, 17 x 4096 4.9 against 5.1).
 //  * more, group-scaled weights, against 64 x 64 and 128 x 128 tiles: up to 768 large tiles, 512 if K is long (128 x 12288,
 //    768: 24 against 27; 192 x 12288, 1152: 35 against 33; 384 x 4096, 768: 22.3 against 25.1, but 64 against 60 for K = 11008,
 //    where 300 x 4096, 640, takes 69 against 59 on weights that are in the last-level cache).
-//  * more, one scale per row, against the K-split tiles: up to 384, 256 if K is long (128 x 6144 11.1 against 12.1; 256 x 4096,
-//    512: 12.0 against 11.9; 128 x 12288, 768: 17.7 against 17.0; 180 x 4096, 384, K = 11008: 28 against 26).
-//  * and no more tokens than 1280, 512 with one scale per row: on 1024 channels the tiles fill the chip by then (1500 tokens, token
-//    scales, with their quantiser: 31.6 against 29.5; 700, one scale per row: 16.6 against 16.1).
+//  * more, one scale per row, against the K-split tiles: up to 768 (256 x 6144, 768: 14.4 against 15.4; 320 x 6144, 960: 17.0 against
+//    15.0; 300 x 4096, 640: 12.1 against 12.6; 400 x 4096, 896: 15.0 against 13.5; 128 x 22016, 1376: 26.5 against 24.5; K = 11008: 300 x
+//    4096, 640, 27.5 against 34.5, 400 x 4096, 896, 33.1 against 33.6).
+//  * and no more tokens than 1280: on 1024 channels the tiles fill the chip by then (1500 tokens, token scales, with their
+//    quantiser: 31.6 against 29.5; one scale per row: 1000 8.8 against 10.1).
 // (A forced tile goes to the tile kernels.)
 bool gemm_stream_supports(const GemmArgs& a, int epi, int group) {
   if (!stream_takes(a, epi, group) || g_tune_tile.load(std::memory_order_relaxed) || g_tune_ks.load(std::memory_order_relaxed))
     return false;
   const long columns = stream_columns(a);
   if (a.M <= 16) return takes_few_tokens(a, epi, columns);
-  if (a.M <= 64) return epi != kRowScale || a.M > 32 || columns > 128 * 32;
-  if (a.M > (epi == kRowScale ? 512 : 1280)) return false;
+  if (a.M <= 64) return true;
+  if (a.M > 1280) return false;
   const long large = (long)((a.M + 63) / 64) * ((columns + 31) / 32);
-  return large <= (epi == kRowScale ? 128 : 256) * (a.K <= 8192 ? 3 : 2);
+  return large <= (epi == kRowScale || a.K <= 8192 ? 768 : 512);
 }
 
 int gemm_stream_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
-  if (epi == kRowScale) return launch_stream_by_shape<kRowScale>(a, stream);
-  return a.a_cols == 1 ? launch_stream_by_shape<kTokenGroup>(a, stream) : launch_stream_by_shape<kGroupScale>(a, stream);
+  if (epi == kRowScale) return launch_rows_by_shape(a, stream);
+  return a.a_cols == 1 ? launch_grouped_by_shape<kTokenGroup>(a, stream) : launch_grouped_by_shape<kGroupScale>(a, stream);
 }
 
 // q / k / v with the rotary embedding and the cache write, group-scaled weights: the alternative is 128 x 128 tiles only
