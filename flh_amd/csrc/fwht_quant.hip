@@ -835,9 +835,10 @@ int launch_wave_rms(const __half* x, const __half* w, float eps, uint8_t* q, __h
 }
 
 // Groups of 128 from which four lanes per group are the faster form: below, a quarter of the wavefronts does not fill the
-// chip (us, sixteen lanes / four, groups of 128; rotated 8192 groups 2.52 / 2.76, 16384 3.30 / 3.21, 65536 6.40 / 6.14; not
-// rotated 32000 3.72 / 3.89, 65536 5.62 / 5.40; 6-bit output 8192 2.73 / 2.95, 16384 3.76 / 3.51).
-constexpr uint32_t quad_min_rows(bool had, bool f6) { return had || f6 ? 16384 : 65536; }
+// chip, least of all just beyond a full round of it (us, inputs from HBM, sixteen lanes / four: rotated 18490 groups 3.40 / 3.82, 32768 4.10 /
+// 4.28, 49152 5.70 / 5.73 and 4.35 / 3.96 from the caches, 65536 6.65 / 6.51; not rotated 49152 5.15 / 5.15, 65536 6.21 / 5.66; 6-bit output, rotated
+// and not, 18432 4.26 / 4.45 and 3.80 / 3.93, 24576 4.80 / 4.70 and 4.20 / 4.16, 32768 5.55 / 5.03 and 4.75 / 4.50).
+constexpr uint32_t quad_min_rows(bool had, bool f6) { return f6 ? 24576 : had ? 49152 : 65536; }
 template <bool HAD, bool F6>
 int launch_group_quad(const __half* x, uint8_t* q, __half* s, uint32_t R, float scale_mul, uint32_t tokens,
                       uint32_t groups_per_token, hipStream_t stream) {
