@@ -26,6 +26,33 @@ __device__ __forceinline__ unsigned long long bf6_of_nibbles(unsigned w) {
   return p0 | (p1 << 12) | (p2 << 24) | (p3 << 36);
 }
 
+// 32 whole numbers in -8 .. 7 as fp16 pairs -> their 6-bit codes, code k at bits 6 k of 192 (one instruction, 64 clocks; the table
+// above takes 35 instructions for eight)
+typedef unsigned u6 __attribute__((ext_vector_type(6)));
+__device__ __forceinline__ u6 bf6_of_wholes(const unsigned (&h)[16]) {
+  typedef unsigned u16 __attribute__((ext_vector_type(16)));
+  typedef _Float16 h32 __attribute__((ext_vector_type(32)));
+  u16 v;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = h[i];
+  return __builtin_amdgcn_cvt_scalef32_pk32_bf6_f16(__builtin_bit_cast(h32, v), 1.0f);
+}
+// bytes from a block's start to the six of its chunk of eight codes c16 = 0 .. 15
+__device__ __forceinline__ int f6_chunk_at(int c16) { return 48 * ((c16 >> 2) & 1) + 24 * (c16 >> 3) + 6 * (c16 & 3); }
+// chunk k = 0 .. 3 of what bf6_of_wholes gave
+template <int K>
+__device__ __forceinline__ void f6_store_six(const u6& r, uint8_t* dst) {
+  typedef unsigned u32_at2 __attribute__((aligned(2)));
+  constexpr int w = K / 2 * 3;
+  if constexpr (K % 2 == 0) {
+    *(u32_at2*)dst = r[w];
+    *(unsigned short*)(dst + 4) = (unsigned short)r[w + 1];
+  } else {
+    *(u32_at2*)dst = __builtin_amdgcn_alignbit(r[w + 2], r[w + 1], 16);
+    *(unsigned short*)(dst + 4) = (unsigned short)(r[w + 2] >> 16);
+  }
+}
+
 // Store the eight codes of one lane (nibble dword w, chunk c16 = 0 .. 15 of a 128-code block) into the block's 96 bytes.
 // A lane's codes are 48 bits; the four lanes of a hardware quad must own the chunks 4 p .. 4 p + 3 of one 24-byte piece
 // with chunk index and quad position differing by a constant XOR (the lane labellings of the quantiser kernels do):

@@ -523,21 +523,21 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const __half* __restri
 // ------------------------------------------------------------------------------------
 // 2. wave-per-row kernel, float32 butterflies, K = 512 * J: four rows per workgroup, rotate_quant_row (rotate_row.h)
 // ------------------------------------------------------------------------------------
-template <int J, bool HAD, bool EXACT_NORM, bool RMS = false>
+template <int J, bool HAD, bool EXACT_NORM, bool RMS, bool F6>
 __global__ __launch_bounds__(256) void rotate_quant_wave_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
                                                                 __half* __restrict__ scales,
                                                                 __half* __restrict__ y_out, uint32_t M, float norm,
                                                                 float clip, const __half* __restrict__ rms_weight = nullptr,
                                                                 float rms_eps = 0.f, const __half* add = nullptr,
-                                                                __half* sum_out = nullptr, uint32_t f6 = 0) {
+                                                                __half* sum_out = nullptr) {
   constexpr int K = 512 * J;
   const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
   if (row >= M) return;  // wave-uniform
-  // f6: q is the encoded matrix of M rows in the 6-bit operand format instead of [M, K / 2] nibbles
-  rotate_quant_row<J, HAD, EXACT_NORM, RMS>(x + (size_t)row * K, f6 ? q : q + (size_t)row * (K / 2), scales + row,
+  // F6: q is the encoded matrix of M rows in the 6-bit operand format instead of [M, K / 2] nibbles
+  rotate_quant_row<J, HAD, EXACT_NORM, RMS, F6>(x + (size_t)row * K, F6 ? q : q + (size_t)row * (K / 2), scales + row,
                                             y_out ? y_out + (size_t)row * K : nullptr, norm, clip, rms_weight, rms_eps,
                                             add ? add + (size_t)row * K : nullptr,
-                                            add ? sum_out + (size_t)row * K : nullptr, f6 ? M : 0u, row);
+                                            add ? sum_out + (size_t)row * K : nullptr, M, row);
 }
 
 constexpr int kGenericThreads = 1024;      // one workgroup per compute unit (LDS): two waves per SIMD hide latencies
@@ -753,24 +753,21 @@ bool factor_hadamard(uint32_t K, int* Kd, int* P) {
   return true;
 }
 
-template <int J>
+template <int J, bool F6 = false>
 int launch_wave(const __half* x, uint8_t* q, __half* s, __half* y, uint32_t M, bool had, float clip,
-                hipStream_t stream, uint32_t f6 = 0) {
+                hipStream_t stream) {
   constexpr int K = 512 * J;
   int lg = 0;
   while ((1 << lg) < K) ++lg;
-  const bool even = (lg % 2) == 0;
   const dim3 grid((M + 3) / 4), block(256);
   if (!had)
-    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, false, true>), grid, block, 0, stream, x, q, s, y, M, 1.0f, clip,
-                       (const __half*)nullptr, 0.f, (const __half*)nullptr, (__half*)nullptr, f6);
-  else if (even)
-    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, true>), grid, block, 0, stream, x, q, s, y, M,
-                       1.0f / (float)(1 << (lg / 2)), clip, (const __half*)nullptr, 0.f, (const __half*)nullptr,
-                       (__half*)nullptr, f6);
+    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, false, true, false, F6>), grid, block, 0, stream, x, q, s, y, M, 1.0f, clip);
+  else if (lg % 2 == 0)
+    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, true, false, F6>), grid, block, 0, stream, x, q, s, y, M,
+                       1.0f / (float)(1 << (lg / 2)), clip);
   else
-    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, false>), grid, block, 0, stream, x, q, s, y, M,
-                       sqrtf((float)K), clip, (const __half*)nullptr, 0.f, (const __half*)nullptr, (__half*)nullptr, f6);
+    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, false, false, F6>), grid, block, 0, stream, x, q, s, y, M, sqrtf((float)K),
+                       clip);
   return check_launch("rotate_quant_wave");
 }
 
@@ -814,23 +811,22 @@ __global__ __launch_bounds__(512) void add_rmsnorm_rotate_quant_row8_kernel(cons
 // 3.9 against 5.0 us for 512; from 1024 rows on the wave-per-row kernel is the faster one
 constexpr uint32_t kRow8MaxRows = 512;
 
-template <int J>
+template <int J, bool F6 = false>
 int launch_wave_rms(const __half* x, const __half* w, float eps, uint8_t* q, __half* s, __half* y, uint32_t M, bool had,
-                    float clip, hipStream_t stream, const __half* add = nullptr, __half* sum_out = nullptr,
-                    uint32_t f6 = 0) {
+                    float clip, hipStream_t stream, const __half* add = nullptr, __half* sum_out = nullptr) {
   constexpr int K = 512 * J;
   int lg = 0;
   while ((1 << lg) < K) ++lg;
   const dim3 grid((M + 3) / 4), block(256);
   if (!had)
-    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, false, true, true>), grid, block, 0, stream, x, q, s, y, M, 1.0f,
-                       clip, w, eps, add, sum_out, f6);
+    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, false, true, true, F6>), grid, block, 0, stream, x, q, s, y, M, 1.0f,
+                       clip, w, eps, add, sum_out);
   else if (lg % 2 == 0)
-    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, true, true>), grid, block, 0, stream, x, q, s, y, M,
-                       1.0f / (float)(1 << (lg / 2)), clip, w, eps, add, sum_out, f6);
+    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, true, true, F6>), grid, block, 0, stream, x, q, s, y, M,
+                       1.0f / (float)(1 << (lg / 2)), clip, w, eps, add, sum_out);
   else
-    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, false, true>), grid, block, 0, stream, x, q, s, y, M,
-                       sqrtf((float)K), clip, w, eps, add, sum_out, f6);
+    hipLaunchKernelGGL((rotate_quant_wave_kernel<J, true, false, true, F6>), grid, block, 0, stream, x, q, s, y, M,
+                       sqrtf((float)K), clip, w, eps, add, sum_out);
   return check_launch("rmsnorm_rotate_quant_wave");
 }
 
@@ -1068,19 +1064,19 @@ extern "C" int flh_rotate_quant_f6(const flh_half* x, const flh_half* add, flh_h
   const bool had = hadamard != FLH_HAD_NONE;
   if (rmsnorm) {
     switch (K / 512) {
-      case 1: return launch_wave_rms<1>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh, 1);
-      case 2: return launch_wave_rms<2>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh, 1);
-      case 4: return launch_wave_rms<4>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh, 1);
-      case 8: return launch_wave_rms<8>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh, 1);
-      default: return launch_wave_rms<16>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh, 1);
+      case 1: return launch_wave_rms<1, true>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh);
+      case 2: return launch_wave_rms<2, true>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh);
+      case 4: return launch_wave_rms<4, true>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh);
+      case 8: return launch_wave_rms<8, true>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh);
+      default: return launch_wave_rms<16, true>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh);
     }
   }
   switch (K / 512) {
-    case 1: return launch_wave<1>(xh, encoded, sh, nullptr, M, had, clip_ratio, st, 1);
-    case 2: return launch_wave<2>(xh, encoded, sh, nullptr, M, had, clip_ratio, st, 1);
-    case 4: return launch_wave<4>(xh, encoded, sh, nullptr, M, had, clip_ratio, st, 1);
-    case 8: return launch_wave<8>(xh, encoded, sh, nullptr, M, had, clip_ratio, st, 1);
-    default: return launch_wave<16>(xh, encoded, sh, nullptr, M, had, clip_ratio, st, 1);
+    case 1: return launch_wave<1, true>(xh, encoded, sh, nullptr, M, had, clip_ratio, st);
+    case 2: return launch_wave<2, true>(xh, encoded, sh, nullptr, M, had, clip_ratio, st);
+    case 4: return launch_wave<4, true>(xh, encoded, sh, nullptr, M, had, clip_ratio, st);
+    case 8: return launch_wave<8, true>(xh, encoded, sh, nullptr, M, had, clip_ratio, st);
+    default: return launch_wave<16, true>(xh, encoded, sh, nullptr, M, had, clip_ratio, st);
   }
 }
 

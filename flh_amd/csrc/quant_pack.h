@@ -61,24 +61,28 @@ constexpr unsigned kPairBias = kQuadBias + (kQuadBias << 16);     // for two qua
 // CAREFUL also clamps the values to +-bound and the quotients to [-8, 7]; it is needed only
 // for clipping (clip_ratio < 1) or a subnormal scale, chosen once per row.
 template <bool CAREFUL>
+__device__ __forceinline__ unsigned quotients2(unsigned y, float rinv, h2 hb) {
+  if constexpr (CAREFUL)
+    y = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(h2, y), -hb), hb));
+  unsigned h = mul_halves(y, rinv);
+  if constexpr (CAREFUL) {
+    const h2 lo8 = {(_Float16)-8.0f, (_Float16)-8.0f}, hi7 = {(_Float16)7.0f, (_Float16)7.0f};
+    h = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(h2, h), lo8), hi7));
+  }
+  return h;
+}
+template <bool CAREFUL>
 __device__ __forceinline__ unsigned nibbles8(unsigned y01, unsigned y23, unsigned y45, unsigned y67, float rinv, h2 hb) {
   unsigned t[2];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    unsigned ya = u == 0 ? y01 : y45, yb = u == 0 ? y23 : y67;
-    if constexpr (CAREFUL) {
-      ya = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(h2, ya), -hb), hb));
-      yb = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(h2, yb), -hb), hb));
-    }
-    unsigned ha = mul_halves(ya, rinv), hbq = mul_halves(yb, rinv);
-    if constexpr (CAREFUL) {
-      const h2 lo8 = {(_Float16)-8.0f, (_Float16)-8.0f}, hi7 = {(_Float16)7.0f, (_Float16)7.0f};
-      ha = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(h2, ha), lo8), hi7));
-      hbq = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(h2, hbq), lo8), hi7));
-    }
-    t[u] = quad_nibbles(ha, hbq);
-  }
+  for (int u = 0; u < 2; ++u)
+    t[u] = quad_nibbles(quotients2<CAREFUL>(u == 0 ? y01 : y45, rinv, hb), quotients2<CAREFUL>(u == 0 ? y23 : y67, rinv, hb));
   return ((t[1] << 16) + t[0] - kPairBias) ^ 0x88888888u;
+}
+// rint of two fp16 quotients, as fp16 (zeros are +0): for the hardware's conversion to the 6-bit format
+__device__ __forceinline__ unsigned whole2(unsigned h) {
+  const h2 magic = {(_Float16)1544.0f, (_Float16)1544.0f};
+  return __builtin_bit_cast(unsigned, (__builtin_bit_cast(h2, h) + magic) - magic);
 }
 
 }  // namespace flh

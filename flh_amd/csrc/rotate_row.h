@@ -71,6 +71,22 @@ __device__ __forceinline__ void stage_swap(float (&v)[N]) {
   }
 }
 
+// acc + (half SEL of w)^2;  s * (half SEL of w), with the sign of a zero product (-0 + -0 = -0, +0 + -0 = +0)
+template <int SEL>
+__device__ __forceinline__ float square_half(unsigned w, float acc) {
+  float d;
+  if constexpr (SEL == 0) asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel_hi:[1,1,0]" : "=v"(d) : "v"(w), "v"(acc));
+  else asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(d) : "v"(w), "v"(acc));
+  return d;
+}
+template <int SEL>
+__device__ __forceinline__ float times_half(float s, unsigned w) {
+  float d;
+  if constexpr (SEL == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(s), "v"(w), "v"(-0.f));
+  else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(s), "v"(w), "v"(-0.f));
+  return d;
+}
+
 // RMS: the row is first normalised as flh/nn/normalization.py:12-20 does -- float32 sum of squares / K,
 // x * (1 / sqrt(. + eps)) [* weight] with every product rounded to float32, then fp16 -- and that fp16 row is
 // what the rotation and the quantiser see.
@@ -80,10 +96,16 @@ __device__ __forceinline__ void stage_swap(float (&v)[N]) {
 // hidden = residual + attention output; residual = hidden; hidden = norm(hidden)) without a launch of its own.
 // sum_row overlaps neither input.
 //
-// f6_rows > 0: the codes leave in the operand format of the 6-bit matrix instruction (gemm_f6.hip: K-slab-major blocks
+// F6: the codes leave in the operand format of the 6-bit matrix instruction (gemm_f6.hip: K-slab-major blocks
 // of 96 bytes per 128 codes and row) -- q_row is then the BASE of the encoded matrix, f6_rows its row count and f6_row
 // this row's index.
-template <int J, bool HAD, bool EXACT_NORM, bool RMS = false>
+//
+// What bounds it: instructions, 1500-1900 per row.  The whole-number codes become 6-bit ones in one conversion per 32 (the table
+// took 35 instructions per 8 and an exchange between lanes), the careful form is a branch of its own around all segments, and a
+// value's conversion and multiplication are one instruction.  us, before -> now, 8192 rows of 4096, rows from HBM: 6-bit codes 32.1 ->
+// 26.4, behind the norm 41.2 -> 32.3, behind addition and norm 53.8 -> 45.0;  nibbles 26.8 -> 26.0, 35.5 -> 30.6, 48.6 -> 42.1.
+// Five or six wavefronts per SIMD instead of four (96 and 80 registers): 26.7 and 35.0 us, 38.3 and 42.0 behind the norm.
+template <int J, bool HAD, bool EXACT_NORM, bool RMS = false, bool F6 = false>
 __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_row, uint8_t* q_row, __half* scale_dst,
                                                  __half* y_row, float norm, float clip,
                                                  const __half* __restrict__ rms_weight = nullptr, float rms_eps = 0.f,
@@ -111,27 +133,29 @@ __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_ro
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
         const unsigned w = (unsigned)raw[j][d];
-        const h2 t = __builtin_bit_cast(h2, w);
-        ss = __builtin_fmaf((float)t[0], (float)t[0], ss);
-        ss = __builtin_fmaf((float)t[1], (float)t[1], ss);
+        ss = square_half<0>(w, ss);
+        ss = square_half<1>(w, ss);
       }
     ss = wave_sum(ss);
     const float inv = 1.0f / __builtin_sqrtf(ss / (float)K + rms_eps);
+    if (rms_weight) {
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      v4i wv = {0, 0, 0, 0};
-      if (rms_weight) wv = *(const v4i*)(rms_weight + j * 512 + c * 8);
+      for (int j = 0; j < J; ++j) {
+        const v4i wv = *(const v4i*)(rms_weight + j * 512 + c * 8);
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const unsigned w = (unsigned)raw[j][d], ww = (unsigned)wv[d];
-        const h2 t = __builtin_bit_cast(h2, w), g = __builtin_bit_cast(h2, ww);
-        float a = round_here((float)t[0] * inv), b = round_here((float)t[1] * inv);
-        if (rms_weight) {
-          a = round_here(a * (float)g[0]);
-          b = round_here(b * (float)g[1]);
+        for (int d = 0; d < 4; ++d) {
+          const unsigned w = (unsigned)raw[j][d], ww = (unsigned)wv[d];
+          raw[j][d] = (int)pack_f16(times_half<0>(times_half<0>(inv, w), ww), times_half<1>(times_half<1>(inv, w), ww));
         }
-        raw[j][d] = (int)pack_f16(a, b);
       }
+    } else {
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const unsigned w = (unsigned)raw[j][d];
+          raw[j][d] = (int)pack_f16(times_half<0>(inv, w), times_half<1>(inv, w));
+        }
     }
   }
 
@@ -226,18 +250,30 @@ __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_ro
   // was clipped: only then are the clamps needed
   const bool careful = __builtin_amdgcn_readfirstlane((float)s < 6.2e-5f || clip < 1.0f);
   const h2 hb = {(_Float16)mx, (_Float16)mx};
-  unsigned* qr = (unsigned*)q_row + c;
+  auto store = [&](auto careful_tag) __attribute__((always_inline)) {
+    constexpr bool CAREFUL = decltype(careful_tag)::value;
+    if constexpr (F6) {                                // chunk c of segment j sits in 128-code block 4 j + c / 16
+      uint8_t* dst = q_row + ((size_t)(c >> 4) * f6_rows + f6_row) * kF6BlockBytes + f6_chunk_at(c & 15);
+      const size_t step = (size_t)4 * f6_rows * kF6BlockBytes;
+      static_for<(J + 3) / 4>([&](auto u_tag) {
+        constexpr int u = decltype(u_tag)::value;
+        unsigned h[16];
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const unsigned w = careful ? nibbles8<true>(yp[4 * j], yp[4 * j + 1], yp[4 * j + 2], yp[4 * j + 3], r, hb)
-                               : nibbles8<false>(yp[4 * j], yp[4 * j + 1], yp[4 * j + 2], yp[4 * j + 3], r, hb);
-    if (f6_rows) {                                     // wave-uniform; chunk c of segment j sits in 128-code block 4 j + c / 16
-      const size_t block = (size_t)(4 * j + (c >> 4)) * f6_rows + f6_row;
-      f6_store_chunk(w, c & 15, q_row + block * kF6BlockBytes, true);
+        for (int i = 0; i < 16; ++i) h[i] = 16 * u + i < N / 2 ? whole2(quotients2<CAREFUL>(yp[(16 * u + i) % (N / 2)], r, hb)) : 0u;
+        const u6 codes = bf6_of_wholes(h);
+        static_for<(J < 4 ? J : 4)>([&](auto k_tag) {
+          f6_store_six<decltype(k_tag)::value>(codes, dst);
+          dst += step;
+        });
+      });
     } else {
-      qr[j * 64] = w;
+      unsigned* qr = (unsigned*)q_row + c;
+#pragma unroll
+      for (int j = 0; j < J; ++j) qr[j * 64] = nibbles8<CAREFUL>(yp[4 * j], yp[4 * j + 1], yp[4 * j + 2], yp[4 * j + 3], r, hb);
     }
-  }
+  };
+  if (careful) store(std::true_type{});
+  else store(std::false_type{});
   if (lane == 0) *scale_dst = __builtin_bit_cast(__half, s);
 }
 
