@@ -34,6 +34,18 @@
 namespace flh {
 namespace {
 
+// Whole codes (fp16 pairs) of a quad of values that the lower lanes keep (lo: two packed registers) and of one that the upper
+// lanes keep (up): out = the kept quad's two registers of the lower lanes, then the upper lanes' two.
+template <bool CAREFUL>
+__device__ __forceinline__ void wholes_of_quads(const unsigned* lo, const unsigned* up, float rinv, h2 hb, unsigned* out) {
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    auto sw = __builtin_amdgcn_permlane32_swap(whole2(quotients2<CAREFUL>(lo[d], rinv, hb)), whole2(quotients2<CAREFUL>(up[d], rinv, hb)),
+                                               false, false);
+    out[d] = sw[0], out[2 + d] = sw[1];
+  }
+}
+
 // Quantise one block column (32 j' x 64 t' of a row, this lane: block j', 32 codes) and store
 // its 16 bytes.  y[mt][2 g + u]: packed fp16 pairs, t' = 32 mt + 8 g + 4 h + 2 u (+1).
 // CAREFUL also clamps the values to +-bound and the quotients to [-8, 7]; it is needed only
@@ -243,22 +255,28 @@ __global__ __launch_bounds__(256, 2) void rotate_quant_mfma4096_kernel(const __h
     const bool careful = __builtin_amdgcn_readfirstlane((float)s16 < 6.2e-5f || clip < 1.0f);
     const h2 hb = {(_Float16)mx, (_Float16)mx};
     uint8_t* qr = q + (size_t)row * 2048;
+    if constexpr (F6) {
+      // this lane: codes 32 h .. 32 h + 31 of block j' = 32 nt + col = the piece (h, j' % 2) of 128-code block j' / 2
+      auto emit = [&](auto careful_tag) {
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const v4i out = careful ? quantise_block<true>(y[0][nt], y[1][nt], rinv, hb)
-                              : quantise_block<false>(y[0][nt], y[1][nt], rinv, hb);
-      if constexpr (F6) {
-        // this lane: codes 32 h .. 32 h + 31 of block j' = 32 nt + col = the piece (h, j' % 2) of 128-code block j' / 2
-        const int jp = 32 * nt + col;
-        const unsigned long long c0 = bf6_of_nibbles((unsigned)out[0]), c1 = bf6_of_nibbles((unsigned)out[1]),
-                                 c2 = bf6_of_nibbles((unsigned)out[2]), c3 = bf6_of_nibbles((unsigned)out[3]);
-        v2i* dst = (v2i*)(q + ((size_t)(jp >> 1) * M + row) * kF6BlockBytes + 48 * h + 24 * (jp & 1));
-        dst[0] = v2i{(int)(unsigned)c0, (int)((unsigned)(c0 >> 32) | ((unsigned)c1 << 16))};
-        dst[1] = v2i{(int)(unsigned)(c1 >> 16), (int)(unsigned)c2};
-        dst[2] = v2i{(int)((unsigned)(c2 >> 32) | ((unsigned)c3 << 16)), (int)(unsigned)(c3 >> 16)};
-      } else {
-        *(v4i*)(qr + (32 * nt + col) * 32 + 16 * h) = out;
-      }
+        for (int nt = 0; nt < 2; ++nt) {
+          const int jp = 32 * nt + col;
+          unsigned codes[16];
+#pragma unroll
+          for (int g = 0; g < 4; ++g) wholes_of_quads<decltype(careful_tag)::value>(y[0][nt] + 2 * g, y[1][nt] + 2 * g, rinv, hb, codes + 4 * g);
+          const u6 c = bf6_of_wholes(codes);
+          v2i* dst = (v2i*)(q + ((size_t)(jp >> 1) * M + row) * kF6BlockBytes + 48 * h + 24 * (jp & 1));
+#pragma unroll
+          for (int i = 0; i < 3; ++i) dst[i] = v2i{(int)c[2 * i], (int)c[2 * i + 1]};
+        }
+      };
+      if (careful) emit(std::true_type{});
+      else emit(std::false_type{});
+    } else {
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+        *(v4i*)(qr + (32 * nt + col) * 32 + 16 * h) = careful ? quantise_block<true>(y[0][nt], y[1][nt], rinv, hb)
+                                                               : quantise_block<false>(y[0][nt], y[1][nt], rinv, hb);
     }
     if (lane == 0) scales[row] = __builtin_bit_cast(__half, s16);
   }
@@ -561,7 +579,7 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
 #pragma unroll
         for (int u = 0; u < 8; ++u) y[u] = scale_pack_f16(w[nt][2 * u], w[nt][2 * u + 1], c);
         const v2i out = quantise_half_block<decltype(careful_tag)::value>(y, rinv, hb);
-        if constexpr (F6) {
+        if constexpr (F6) {                            // (the hardware's conversion in the table's place: 8192 x 14336 94 -> 96.6 us)
           // this lane: codes 32 mt + 16 h + 0 .. 15 of block j' = 32 nt + col, i.e. 12 bytes at byte 12 h of the piece
           // (half mt, sub-block j' % 2) of 128-code block j' / 2
           const int jp = 32 * nt + col;

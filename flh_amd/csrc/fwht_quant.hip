@@ -144,10 +144,8 @@ __device__ __forceinline__ float max_across(float m) {
 //
 // F6 (G = 128 only): the codes leave in the operand format of the 6-bit matrix instruction instead -- 6 bits per
 // code, the 96-byte block of this group at ((row % groups_per_token) * tokens + row / groups_per_token) * 96
-// (K-slab-major, see gemm_f6.hip).  A lane's eight codes are 48 bits; the four lanes of a quad own one 24-byte
-// piece of the block (chunks 4 p .. 4 p + 3, in an order that depends on the quad), and three of them store eight
-// bytes each after fetching their successor's bits from the lane whose chunk index is one higher (chunk index
-// and quad position differ by a constant XOR inside a quad, so that lane is the xor-1 resp. xor-3 partner).
+// (K-slab-major, see gemm_f6.hip), a lane's eight as six bytes.  The conversion is the hardware's, a quarter full (18432 groups
+// rotated 4.28 -> 4.03 us against a table and eight-byte stores behind an exchange between lanes).
 template <int G, bool F6 = false, bool OFF32 = false>
 __device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool valid, uint32_t row, uint8_t* __restrict__ q,
                                              __half* __restrict__ scales, float scale_mul, uint32_t tokens = 0,
@@ -168,14 +166,27 @@ __device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool val
   const h2 hb = {(_Float16)65504.0f, (_Float16)65504.0f};   // no clipping in the group kernels
   const unsigned y01 = __builtin_bit_cast(unsigned, v[0]), y23 = __builtin_bit_cast(unsigned, v[1]),
                  y45 = __builtin_bit_cast(unsigned, v[2]), y67 = __builtin_bit_cast(unsigned, v[3]);
-  const unsigned w = careful ? nibbles8<true>(y01, y23, y45, y67, r, hb) : nibbles8<false>(y01, y23, y45, y67, r, hb);
+  unsigned w = 0;
+  u6 six;
   if constexpr (F6) {
-    const size_t block = (size_t)(row % groups_per_token) * tokens + row / groups_per_token;
-    f6_store_chunk(w, lir, q + block * kF6BlockBytes, valid);
+    unsigned h[16] = {};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned y = __builtin_bit_cast(unsigned, v[i]);
+      h[i] = whole2(careful ? quotients2<true>(y, r, hb) : quotients2<false>(y, r, hb));
+    }
+    six = bf6_of_wholes(h);
+  } else {
+    w = careful ? nibbles8<true>(y01, y23, y45, y67, r, hb) : nibbles8<false>(y01, y23, y45, y67, r, hb);
   }
   if (valid) {
     using offset_t = std::conditional_t<OFF32, uint32_t, size_t>;
-    if constexpr (!F6) *(unsigned*)(q + ((offset_t)row * (LPR * 4) + (offset_t)lir * 4)) = w;
+    if constexpr (F6) {
+      const size_t block = (size_t)(row % groups_per_token) * tokens + row / groups_per_token;
+      f6_store_six<0>(six, q + block * kF6BlockBytes + f6_chunk_at(lir));
+    } else {
+      *(unsigned*)(q + ((offset_t)row * (LPR * 4) + (offset_t)lir * 4)) = w;
+    }
     // the stored scale may carry a constant factor (the reference divides its scales by sqrt(G) in a
     // second kernel after the unnormalised transform): float32 product, then fp16; the codes above use s
     if (lir == 0) *(__half*)((char*)scales + (offset_t)row * 2) = scale_mul == 1.0f ? __builtin_bit_cast(__half, s) : __float2half(round_here((float)s * scale_mul));
@@ -245,10 +256,11 @@ __global__ __launch_bounds__(256) void silu_mul_group_kernel(const __half* __res
 // The group kernels for groups of 128 and launches that fill the chip: FOUR lanes own a group, 32 values each (lane p
 // the chunks p, p + 4, p + 8, p + 12), so that of the seven butterfly strides only 8 and 16 cross lanes, and the row's maximum,
 // scale and reciprocal are computed by four lanes instead of sixteen.  A lane's four code words are turned inside its wave
-// through LDS, so that it stores sixteen consecutive bytes (32 codes; 6-bit output: one whole 24-byte piece).  Same
+// through LDS, so that it stores sixteen consecutive bytes (32 codes; 6-bit output: the whole numbers are, and a lane converts and
+// stores one 24-byte piece).  Same
 // operations in the same order as group_kernel, the same bytes.
 // What bounds it: memory (4096-wide rows rotated and quantised, us, sixteen lanes -> four, inputs from HBM: 16384 rows 40.3 -> 29.5
-// = 5.7 TB/s, 8192 20.4 -> 15.9, 4096 10.1 -> 9.4; 6-bit output 49.3 -> 40.4, 25.4 -> 21.8, 14.3 -> 12.0), where the sixteen-lane form
+// = 5.7 TB/s, 8192 20.4 -> 15.9, 4096 10.1 -> 9.4; 6-bit output 524288 groups 51 -> 39, 65536 9.1 -> 6.9; a table in the conversion's place 46 and 7.8, six-byte stores without the turn through LDS 56), where the sixteen-lane form
 // is bound by its 165 instructions per eight values, 80 here.  Non-temporal loads and stores: equal or slower (30.6, 31.3).  The
 // SwiGLU product in front of it: 55.6 against 51.4 us, its exponentials want the sixteen lanes' parallelism; not here.
 constexpr uint32_t kQuadRows = 64;                    // groups per workgroup of four waves
@@ -271,7 +283,7 @@ template <bool HAD, bool F6>
 __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
                                                          __half* __restrict__ scales, uint32_t R, float scale_mul,
                                                          uint32_t tokens, uint32_t groups_per_token) {
-  __shared__ unsigned turned[256 * 4];
+  __shared__ __align__(16) unsigned turned[256 * (F6 ? 16 : 4)];
   const int tid = threadIdx.x, p = tid & 3;
   const uint32_t row0 = blockIdx.x * kQuadRows, row = row0 + (tid >> 2);
   const bool valid = row < R;
@@ -318,6 +330,36 @@ __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restric
   const float r = reciprocal_of_scale(s);
   const bool careful = __builtin_amdgcn_ballot_w64((float)s < 6.2e-5f) != 0;   // as in group_finish
   const h2 hb = {(_Float16)65504.0f, (_Float16)65504.0f};
+  if constexpr (F6) {
+    unsigned h[16];
+    auto wholes = [&](auto careful_tag) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) h[i] = whole2(quotients2<decltype(careful_tag)::value>(__builtin_bit_cast(unsigned, v[i >> 2][i & 3]), r, hb));
+    };
+    if (careful) wholes(std::true_type{});
+    else wholes(std::false_type{});
+    // the group's sixteen chunks, places of row and column XORed by the group: no bank conflicts either way
+    const int g = (tid >> 2) & 3;
+    v4i* const line = (v4i*)turned + (tid >> 2) * 16;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      line[4 * (j ^ g) + (p ^ g)] = v4i{(int)h[4 * j], (int)h[4 * j + 1], (int)h[4 * j + 2], (int)h[4 * j + 3]};
+    __builtin_amdgcn_wave_barrier();                   // (the wave's own, LDS operations of a wave complete in order)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const v4i o = line[4 * (p ^ g) + (k ^ g)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) h[4 * k + i] = (unsigned)o[i];
+    }
+    if (!valid) return;
+    const u6 six = bf6_of_wholes(h);
+    const size_t block = (size_t)(row % groups_per_token) * tokens + row / groups_per_token;
+    v2i* dst = (v2i*)(q + block * kF6BlockBytes + 48 * (p & 1) + 24 * (p >> 1));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) dst[i] = v2i{(int)six[2 * i], (int)six[2 * i + 1]};
+    if (p == 0) scales[row] = scale_mul == 1.0f ? __builtin_bit_cast(__half, s) : __float2half(round_here((float)s * scale_mul));
+    return;
+  }
   unsigned w[4];
   auto codes = [&](auto careful_tag) {
 #pragma unroll
@@ -335,17 +377,7 @@ __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restric
   __builtin_amdgcn_wave_barrier();                     // (the wave's own words, LDS operations of a wave complete in order)
   const v4i o = *(const v4i*)(line + 4 * (p ^ swap));
   if (!valid) return;
-  if constexpr (F6) {
-    const unsigned long long q0 = bf6_of_nibbles((unsigned)o[0]), q1 = bf6_of_nibbles((unsigned)o[1]),
-                             q2 = bf6_of_nibbles((unsigned)o[2]), q3 = bf6_of_nibbles((unsigned)o[3]);
-    const size_t block = (size_t)(row % groups_per_token) * tokens + row / groups_per_token;
-    unsigned long long* dst = (unsigned long long*)(q + block * kF6BlockBytes + 48 * (p & 1) + 24 * (p >> 1));
-    dst[0] = q0 | (q1 << 48);
-    dst[1] = (q1 >> 16) | (q2 << 32);
-    dst[2] = (q2 >> 32) | (q3 << 16);
-  } else {
-    *(v4i*)(q + (size_t)row0 * 64 + tid * 16) = o;
-  }
+  *(v4i*)(q + (size_t)row0 * 64 + tid * 16) = o;
   if (p == 0) scales[row] = scale_mul == 1.0f ? __builtin_bit_cast(__half, s) : __float2half(round_here((float)s * scale_mul));
 }
 
@@ -833,8 +865,8 @@ int launch_wave_rms(const __half* x, const __half* w, float eps, uint8_t* q, __h
 // Groups of 128 from which four lanes per group are the faster form: below, a quarter of the wavefronts does not fill the
 // chip, least of all just beyond a full round of it (us, inputs from HBM, sixteen lanes / four: rotated 18490 groups 3.40 / 3.82, 32768 4.10 /
 // 4.28, 49152 5.70 / 5.73 and 4.35 / 3.96 from the caches, 65536 6.65 / 6.51; not rotated 49152 5.15 / 5.15, 65536 6.21 / 5.66; 6-bit output, rotated
-// and not, 18432 4.26 / 4.45 and 3.80 / 3.93, 24576 4.80 / 4.70 and 4.20 / 4.16, 32768 5.55 / 5.03 and 4.75 / 4.50).
-constexpr uint32_t quad_min_rows(bool had, bool f6) { return f6 ? 24576 : had ? 49152 : 65536; }
+// and not, 16384 3.83 / 3.41 and 3.42 / 3.14, 18432 4.07 / 4.03 and 3.62 / 3.53, 24576 4.55 / 4.27 and 4.00 / 3.75).
+constexpr uint32_t quad_min_rows(bool had, bool f6) { return f6 ? 16384 : had ? 49152 : 65536; }
 template <bool HAD, bool F6>
 int launch_group_quad(const __half* x, uint8_t* q, __half* s, uint32_t R, float scale_mul, uint32_t tokens,
                       uint32_t groups_per_token, hipStream_t stream) {

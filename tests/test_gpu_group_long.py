@@ -22,7 +22,7 @@ def rows_of(r, seed):
 
 @pytest.mark.parametrize("f6", [False, True])
 @pytest.mark.parametrize("had", [False, True])
-@pytest.mark.parametrize("r", [24575, 24576, 49152 + 37, 65536 + 64 * 3 + 1])
+@pytest.mark.parametrize("r", [16383, 16384, 16384 + 37, 49152 + 37, 65536 + 64 * 3 + 1])
 def test_long_batches_bit_exact(r, had, f6):
     from flh_amd import _ops
     from oracle import pack, quant
