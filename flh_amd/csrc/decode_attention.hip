@@ -37,7 +37,10 @@ __device__ __forceinline__ _Float16 rope_value(_Float16 x, _Float16 xp, _Float16
 // bytes in the cache as the stand-alone rotary / cache kernel writes -- also for a slot in kv_len .. max_len - 1, which
 // attention does not read: the first workgroup of every (sequence, key / value head) writes it there, as the
 // stand-alone kernel would.
-template <int D, int REP, int CHUNK, bool ROPE>
+//
+// Values pass the caches by (16 x 32 / 8 heads x 4096 61 -> 59 us).  AHEAD: keys as well, and both are requested before anything else (rule:
+// launch_attention).
+template <int D, int REP, int CHUNK, bool ROPE, bool AHEAD>
 __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
     const __half* __restrict__ q, __half* k_cache, __half* v_cache, float* __restrict__ partials, uint32_t Hkv,
     uint32_t kv_len, uint32_t max_len, uint32_t splits, float scale, const __half* __restrict__ k_new,
@@ -53,8 +56,38 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
   __shared__ float red[kAttnThreads / 64][REP * D];    // the waves' weighted values
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t split = blockIdx.x % splits, bh = blockIdx.x / splits;   // bh = b * Hkv + kvh
+  // One or two queries per key: the chunks of one place in all the caches next to each other, whose strides are often a power of two; more
+  // (more work per chunk, fewer caches): the chunks of a cache.  us, chunks of a cache -> of one place: 8 x 32 / 32 x 2048 52.5 -> 46.1, 16 x 32 / 32 x
+  // 2048 101 -> 91, 8 x 32 / 32 x 1024 29.4 -> 26.2, 12 x 32 / 16 x 1024 25.8 -> 24.6, 5 x 32 / 32 x 777 16.8 -> 16.8;  4 x 32 / 8 x 2048 14.7 -> 17.2
+  const uint32_t caches = gridDim.x / splits;
+  const uint32_t split = REP <= 2 ? blockIdx.x / caches : blockIdx.x % splits, bh = REP <= 2 ? blockIdx.x % caches : blockIdx.x / splits;   // bh = b * Hkv + kvh
   const uint32_t t0 = split * CHUNK;
+  const uint32_t n_live = kv_len > t0 ? min((uint32_t)CHUNK, kv_len - t0) : 0u;
+  const uint32_t last = n_live ? n_live - 1 : 0;       // rows past the live range read the last live one again (any valid address)
+
+  // Scores on the matrix cores: wave w owns the keys 16 w .. 16 w + 15 as the rows of a 16 x 16 tile whose columns are
+  // the query heads; a lane holds eight consecutive channels (block `kb` of the step's 32) of key row `krow`.
+  // Values: wave w takes rows 16 w .. 16 w + 15 of the chunk, a lane one channel pair (one channel for D = 64) of each.
+  const int krow = lane & 15, kb = lane >> 4;
+  typedef std::conditional_t<D == 128, unsigned, unsigned short> raw_t;
+  h8 ka[KS];
+  raw_t vr[RPW];
+  __half* const vbase = v_cache + ((size_t)bh * max_len + t0) * D;
+  auto request = [&]() __attribute__((always_inline)) {
+    const __half* kr = k_cache + ((size_t)bh * max_len + t0 + min((uint32_t)(wave * RPW + krow), last)) * D + kb * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const v4i* src = (const v4i*)(kr + ks * 32);
+      ka[ks] = __builtin_bit_cast(h8, AHEAD ? __builtin_nontemporal_load(src) : *src);
+    }
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const raw_t* src = (const raw_t*)(vbase + (size_t)min((uint32_t)(wave * RPW + i), last) * D) + lane;
+      vr[i] = __builtin_nontemporal_load(src);
+    }
+    if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (AHEAD) request();
   uint32_t slot = 0xFFFFFFFFu;                         // cache slot of the new token (ROPE), if it is inside kv_len
   if constexpr (ROPE) {
     const long long pos = positions[0];
@@ -81,54 +114,30 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
       qs[i] = qf[i];
     }
   }
-
-  // Scores on the matrix cores: wave w owns the keys 16 w .. 16 w + 15 as the rows of a 16 x 16 tile whose columns are
-  // the query heads; a lane holds eight consecutive channels (block `kb` of the step's 32) of key row `krow`.
-  const int krow = lane & 15, kb = lane >> 4;
-  const uint32_t t = t0 + wave * RPW + krow;
-  const bool live = t < kv_len;
-  h8 ka[KS];
-  if (ROPE && t == slot) {                             // the new key: rotate it, keep it, and store it in its slot
-    const __half* src = k_new + (size_t)bh * D;
-    __half* dst = k_cache + ((size_t)bh * max_len + t) * D;
+  if constexpr (!AHEAD) request();
+  if (ROPE && slot - t0 < (uint32_t)CHUNK && (slot - t0) / RPW == (uint32_t)wave) {
+    // the new token's wave: key (rotated) and value take the place of what the cache held, here and there
+    const uint32_t r = (slot - t0) % RPW;
+    if ((uint32_t)krow == r) {
+      const __half* src = k_new + (size_t)bh * D;
+      __half* dst = k_cache + ((size_t)bh * max_len + slot) * D;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c0 = ks * 32 + kb * 8, p0 = c0 ^ (D / 2);
-      const h8 x = *(const h8*)(src + c0), xp = *(const h8*)(src + p0);
-      const h8 cc = *(const h8*)(cos + c0), ss = *(const h8*)(sin + c0);
-      h8 y;
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c0 = ks * 32 + kb * 8, p0 = c0 ^ (D / 2);
+        const h8 x = *(const h8*)(src + c0), xp = *(const h8*)(src + p0);
+        const h8 cc = *(const h8*)(cos + c0), ss = *(const h8*)(sin + c0);
+        h8 y;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = rope_value(x[e], xp[e], cc[e], ss[e], c0 < D / 2);
-      ka[ks] = y;
-      *(h8*)(dst + c0) = y;
+        for (int e = 0; e < 8; ++e) y[e] = rope_value(x[e], xp[e], cc[e], ss[e], c0 < D / 2);
+        ka[ks] = y;
+        *(h8*)(dst + c0) = y;
+      }
     }
-  } else {
-    const __half* kr = k_cache + ((size_t)bh * max_len + (live ? t : 0)) * D + kb * 8;
+    const raw_t fresh = ((const raw_t*)(v_new + (size_t)bh * D))[lane];
+    ((raw_t*)(vbase + (size_t)(slot - t0) * D))[lane] = fresh;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) ka[ks] = *(const h8*)(kr + ks * 32);
-  }
-  // Values: wave w takes rows 16 w .. 16 w + 15 of the chunk, a lane one channel pair (one channel for D = 64) of
-  // each; requested now, the loads travel while the scores and the softmax pieces are computed.  Rows past the live
-  // range read the last live row again (any valid address) and are zeroed: their probability is zero, but 0 x NaN is not.
-  const uint32_t n_live = kv_len > t0 ? min((uint32_t)CHUNK, kv_len - t0) : 0u;
-  __half* vbase = v_cache + ((size_t)bh * max_len + t0) * D;
-  float vv0[RPW], vv1[D == 128 ? RPW : 1];
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    const uint32_t row = wave * RPW + i;               // wave-uniform
-    const bool fresh = ROPE && t0 + row == slot;
-    const bool have = row < n_live;
-    const __half* src = fresh ? v_new + (size_t)bh * D : vbase + (size_t)(have ? row : (n_live ? n_live - 1 : 0)) * D;
-    if constexpr (D == 128) {
-      h2 v = *(const h2*)(src + 2 * lane);
-      if (fresh) *(h2*)(vbase + (size_t)row * D + 2 * lane) = v;
-      vv0[i] = have ? (float)v[0] : 0.f;
-      vv1[i] = have ? (float)v[1] : 0.f;
-    } else {
-      const __half v = src[lane];
-      if (fresh) vbase[(size_t)row * D + lane] = v;
-      vv0[i] = have ? __half2float(v) : 0.f;
-    }
+    for (int i = 0; i < RPW; ++i)
+      if ((uint32_t)i == r) vr[i] = fresh;
   }
   __syncthreads();                                     // the queries are in LDS
   {
@@ -151,7 +160,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
   __syncthreads();
 
   // softmax pieces of this chunk, head h by wave h (REP > 4: two heads per wave)
-  float* out = partials + (size_t)blockIdx.x * partial_floats<D>(REP);
+  float* out = partials + ((size_t)bh * splits + split) * partial_floats<D>(REP);
   for (int h = wave; h < REP; h += kAttnThreads / 64) {
     const float s = sc[h][lane];
     const float m = wave_max(s);
@@ -164,7 +173,20 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
     }
   }
   __syncthreads();
-  // weighted values: every wave its own rows for all heads, then the four waves' sums in a fixed order
+  // weighted values: every wave its own rows for all heads, then the four waves' sums in a fixed order (rows past the live
+  // range as zeros: their probability is zero, but 0 x NaN is not)
+  float vv0[RPW], vv1[D == 128 ? RPW : 1];
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
+    const bool have = (uint32_t)(wave * RPW + i) < n_live;
+    if constexpr (D == 128) {
+      const h2 v = __builtin_bit_cast(h2, vr[i]);
+      vv0[i] = have ? (float)v[0] : 0.f;
+      vv1[i] = have ? (float)v[1] : 0.f;
+    } else {
+      vv0[i] = have ? (float)__builtin_bit_cast(_Float16, vr[i]) : 0.f;
+    }
+  }
 #pragma unroll
   for (int h = 0; h < REP; ++h) {
     float a0 = 0.f, a1 = 0.f;
@@ -250,12 +272,17 @@ int launch_attention(const __half* q, __half* k, __half* v, __half* out, float* 
                      uint32_t kv_len, uint32_t max_len, float scale, const NewToken& nt, hipStream_t stream) {
   const uint32_t splits = (kv_len + kChunk - 1) / kChunk;
   const dim3 grid(B * Hkv * splits), block(kAttnThreads);
-  if (nt.k)
-    hipLaunchKernelGGL((decode_attention_partial_kernel<D, REP, kChunk, true>), grid, block, 0, stream, q, k, v, partials,
-                       Hkv, kv_len, max_len, splits, scale, nt.k, nt.v, nt.cos, nt.sin, nt.positions);
-  else
-    hipLaunchKernelGGL((decode_attention_partial_kernel<D, REP, kChunk, false>), grid, block, 0, stream, q, k, v, partials,
-                       Hkv, kv_len, max_len, splits, scale, nt.k, nt.v, nt.cos, nt.sin, nt.positions);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, block, 0, stream, q, k, v, partials, Hkv, kv_len, max_len, splits, scale, nt.k, nt.v, nt.cos, nt.sin,
+                       nt.positions);
+  };
+  // Requested ahead, and past the caches, everywhere but for grouped queries on more chunks than two rounds of the chip hold, and eight queries per key.  us, with
+  // the combine launch, otherwise -> ahead, sequences x heads / key-value heads x positions: 5 x 32 / 32 x 777 18.6 -> 16.9, 1 x 32 / 8 x 2048
+  // 10.7 -> 10.3, 8 x 32 / 8 x 1024 15.1 -> 13.9, 10 x 32 / 8 x 2048 26.7 -> 25.0, 14 x 32 / 8 x 2048 (3584 chunks) 32.6 -> 31.7, 16 x 32 / 32 x 777
+  // 42.6 -> 39.0;  16 x 32 / 8 x 2048 (4096) 35.2 -> 37.3, 16 x 32 / 8 x 4096 59 -> 65, 8 x 32 / 4 x 3000 21.9 -> 23.3
+  const bool ahead = REP == 1 || (REP <= 4 && (uint64_t)B * Hkv * splits <= 3584);
+  if (nt.k) ahead ? go(decode_attention_partial_kernel<D, REP, kChunk, true, true>) : go(decode_attention_partial_kernel<D, REP, kChunk, true, false>);
+  else ahead ? go(decode_attention_partial_kernel<D, REP, kChunk, false, true>) : go(decode_attention_partial_kernel<D, REP, kChunk, false, false>);
   if (int rc = check_launch("decode_attention (partials)")) return rc;
   hipLaunchKernelGGL((decode_attention_combine_kernel<D>), dim3(B * Hkv * REP), dim3(256), 0, stream, partials, out,
                      (uint32_t)REP, splits);

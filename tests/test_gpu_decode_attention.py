@@ -119,3 +119,24 @@ def test_rotary_decode_attention_argument_errors():
         _ops.decode_attention_rope(q, kn, kn, cs, cs, pos.int(), k, k.clone(), 4)
     with pytest.raises(RuntimeError):
         _ops.decode_attention_rope(q, kn, kn, cs, cs, pos, k, k.clone(), 17)
+
+
+@pytest.mark.parametrize("b,hq,hkv,n", [(7, 8, 8, 65), (2, 8, 2, 200), (57, 32, 8, 449), (3, 16, 2, 130)])
+def test_new_token_in_any_wave_and_chunk(b, hq, hkv, n):
+    """The rotary form, whose keys and values are requested before the slot is known: the new token in every wave of a chunk, and in
+    the first and the last chunk, against the cache write as its own launch, on either side of the rule for early requests."""
+    import flh_amd
+    ops = flh_amd._CUDA
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen).half()
+    q, kn, vn, cos, sin = rnd(b, hq, 128), rnd(b, hkv, 128), rnd(b, hkv, 128), rnd(1, 128), rnd(1, 128)
+    for slot in (0, 17, 33, 63, 64, n - 1):
+        keys, values = rnd(b, hkv, n + 3, 128), rnd(b, hkv, n + 3, 128)
+        keys[:, :, slot], values[:, :, slot] = float("nan"), float("nan")     # what the slot held is not used
+        k2, v2 = keys.clone(), values.clone()
+        pos = torch.tensor([slot], device="cuda")
+        got = ops.decode_attention_rope(q, kn, vn, cos, sin, pos, keys, values, n)
+        q2 = q.clone().view(b, 1, hq, 128)
+        ops.rope_kv_cache_(q2, kn.view(b, 1, hkv, 128), vn.view(b, 1, hkv, 128), cos, sin, pos, k2, v2)
+        assert torch.equal(keys, k2) and torch.equal(values, v2)
+        assert torch.equal(got, ops.decode_attention(q2.view(b, hq, 128), k2, v2, n)) and torch.isfinite(got).all()
