@@ -301,8 +301,15 @@ int launch_decode(const GemmArgs& a, hipStream_t stream) {
 // requests its share of the weights, then rotates, quantises and packs the tokens into LDS itself -- all eight
 // waves on each row, rotate_quant_row_8waves: the additions of the stand-alone kernel in the same order, so the
 // codes and scales are the same bits -- while the weights are still on their way from HBM.  The rotation is
-// repeated by every workgroup (about a microsecond per token); what it saves is a whole launch in front of the
-// GEMM, which is worth more than that for one or two tokens and outputs up to about 12 K channels.
+// repeated by every workgroup (about a microsecond per token, two with the norm); what it saves is a whole launch
+// in front of the GEMM, which is worth more than that for one or two tokens and outputs up to about 8 K channels
+// (the callers' rules say where).
+//
+// T tiles of 16 channels per workgroup.  Two rotations that share a compute unit get in each other's way: with one
+// tile each, what goes beyond 256 workgroups paid for a second rotation.  A workgroup that owns two tiles requests
+// the weights of both, rotates once, and multiplies one tile after the other from the same codes in LDS.  One token,
+// us, one tile / two: norm and residual 4096 x 5120 10.4 / 8.7, 6144 10.4 / 8.8, 8192 10.9 / 9.5 (group scales 11.6 /
+// 10.4); two tokens, rotation only, 6144 9.2 / 8.5.
 //
 // NORM / ADD: the tokens are RMS-normalised first (NORM), after a residual addition x + add (ADD) -- the prologues of
 // flh_rmsnorm_rotate_quant_i4 / flh_add_rmsnorm_rotate_quant_i4 with the same roundings, so again the same bits as the
@@ -314,7 +321,7 @@ struct DecodePrologue {
   __half* sum_out;            // ADD
 };
 
-template <int EPI, bool NORM = false, bool ADD = false>
+template <int EPI, int T, bool NORM, bool ADD>
 __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(const __half* __restrict__ x,
                                                                             const GemmArgs p, float norm,
                                                                             const DecodePrologue pro) {
@@ -323,37 +330,42 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
   constexpr int TILES = EPI == kGroupScale ? KT : 2 * kWaves;   // at least the 16 KB the rotation stages in
   extern __shared__ __align__(16) int red[];   // tiles [wave | group][64 lanes][4], channel scales, maxima, codes, token scales
   unsigned* table = (unsigned*)(red + TILES * 256);
-  float* sA = (float*)(table + (EPI == kGroupScale ? 16 * KT / 2 : 0));   // scratch of the rotation
+  constexpr int TABLE = EPI == kGroupScale ? 16 * KT / 2 : 0;   // dwords of a tile's scales
+  float* sA = (float*)(table + T * TABLE);     // scratch of the rotation
   uint8_t* codes = (uint8_t*)(sA + 16);
   __half* tok = (__half*)(codes + kRotateGemmMaxTokens * ROW);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, c = lane >> 4;
-  const DecodeWeights w = decode_weights(p, blockIdx.x);
-  const int n0 = w.n0;
+  auto tile = [&](int t) { return decode_weights(p, min((int)blockIdx.x * T + t, p.tiles_n - 1)); };
 
-  // this wave's weights first: all of them are in flight while the tokens are rotated
-  const uint8_t* bptr = w.B + (size_t)min(n0 + r, w.N - 1) * Kb + c * 16;
-  v4i b[NDW][2];
+  // this wave's weights first, of all its tiles: they are in flight while the tokens are rotated
+  v4i b[T][NDW][2];
+  FirstScales first[T];
+  static_for<T>([&](auto t_tag) {
+    constexpr int t = decltype(t_tag)::value;
+    const DecodeWeights w = tile(t);
+    const uint8_t* bptr = w.B + (size_t)min(w.n0 + r, w.N - 1) * Kb + c * 16;
 #pragma unroll
-  for (int i = 0; i < NDW; ++i) {
-    const int ds = wave + i * kWaves;
-    b[i][0] = *(const v4i*)(bptr + (size_t)ds * 128);
-    b[i][1] = *(const v4i*)(bptr + (size_t)ds * 128 + 64);
-  }
-  // The scales, 16 rows of 64 bytes one behind the other: one load instruction of one wave (with the other kernel's request, its
-  // divisions and its branch for rows of any kind, a token took 11.5 us through 6144 channels with the prologues; now 10.9).
-  if constexpr (EPI == kGroupScale) {
-    static_assert(kWaves * 64 == 16 * KT && KT == 32, "a load instruction, or a half per thread");
-    if (((uintptr_t)w.Bs & 15) == 0) {
-      if (wave == kWaves - 1)
-        load_to_lds16(w.Bs + (size_t)min(n0 + (lane >> 2), w.N - 1) * KT + (lane & 3) * 8,
-                      (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned*)table);
-    } else {
-      ((__half*)table)[tid] = w.Bs[(size_t)min(n0 + (tid >> 5), w.N - 1) * KT + (tid & 31)];
+    for (int i = 0; i < NDW; ++i) {
+      const int ds = wave + i * kWaves;
+      b[t][i][0] = *(const v4i*)(bptr + (size_t)ds * 128);
+      b[t][i][1] = *(const v4i*)(bptr + (size_t)ds * 128 + 64);
     }
-  }
-  FirstScales first = first_scales<EPI>(p, w, nullptr, tid);
+    // The scales, 16 rows of 64 bytes one behind the other: one load instruction of one wave (with the other kernel's request, its
+    // divisions and its branch for rows of any kind, a token took 11.5 us through 6144 channels with the prologues; 10.9 with this).
+    if constexpr (EPI == kGroupScale) {
+      static_assert(kWaves * 64 == 16 * KT && KT == 32, "a load instruction, or a half per thread");
+      if (((uintptr_t)w.Bs & 15) == 0) {
+        if (wave == kWaves - 1 - t % kWaves)
+          load_to_lds16(w.Bs + (size_t)min(w.n0 + (lane >> 2), w.N - 1) * KT + (lane & 3) * 8,
+                        (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned*)(table + t * TABLE));
+      } else {
+        ((__half*)(table + t * TABLE))[tid] = w.Bs[(size_t)min(w.n0 + (tid >> 5), w.N - 1) * KT + (tid & 31)];
+      }
+    }
+    first[t] = first_scales<EPI>(p, w, nullptr, tid);
+  });
   for (int row = 0; row < p.M; ++row) {
     if constexpr (NORM || ADD)
       rotate_quant_row_8waves<NORM, ADD>(x + (size_t)row * K, (float*)red, sA, codes + row * ROW, tok + row, norm, wave,
@@ -364,48 +376,65 @@ __global__ __launch_bounds__(kWaves * 64) void rotate_gemm_i4_decode_kernel(cons
   }
   __syncthreads();
 
-  v4i acc = {0, 0, 0, 0};
   const uint8_t* arow = codes + min(r, p.M - 1) * ROW + c * 16;
+  static_for<T>([&](auto t_tag) {
+    constexpr int t = decltype(t_tag)::value;
+    if (t > 0) __syncthreads();                          // the tile before is finished
+    v4i acc = {0, 0, 0, 0};
 #pragma unroll
-  for (int i = 0; i < NDW; ++i) {
-    const int ds = wave + i * kWaves;
+    for (int i = 0; i < NDW; ++i) {
+      const int ds = wave + i * kWaves;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      v4i blo, bhi, alo, ahi;
-      unpack_lo_hi(b[i][half], blo, bhi);
-      unpack_lo_hi(*(const v4i*)(arow + ds * 128 + half * 64), alo, ahi);
-      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(blo, alo, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(bhi, ahi, acc, 0, 0, 0);
-      if constexpr (EPI == kGroupScale) {
-        *(v4f*)(red + ((2 * ds + half) * 64 + lane) * 4) = tile_as_float(acc);
-        acc = v4i{0, 0, 0, 0};
+      for (int half = 0; half < 2; ++half) {
+        v4i blo, bhi, alo, ahi;
+        unpack_lo_hi(b[t][i][half], blo, bhi);
+        unpack_lo_hi(*(const v4i*)(arow + ds * 128 + half * 64), alo, ahi);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(blo, alo, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(bhi, ahi, acc, 0, 0, 0);
+        if constexpr (EPI == kGroupScale) {
+          *(v4f*)(red + ((2 * ds + half) * 64 + lane) * 4) = tile_as_float(acc);
+          acc = v4i{0, 0, 0, 0};
+        }
       }
     }
-  }
-  if constexpr (EPI != kGroupScale) *(v4i*)(red + (wave * 64 + lane) * 4) = acc;
-  if constexpr (EPI == kGroupScale) wait_vmcnt<0>();     // the scales
-  __syncthreads();
-  first.a = __half2float(tok[min((tid >> 2) & 15, p.M - 1)]);
-  decode_finish<1, EPI, EPI == kGroupScale ? KT : 0>(p, w, red, table, tok, first, tid);
+    if constexpr (EPI != kGroupScale) *(v4i*)(red + (wave * 64 + lane) * 4) = acc;
+    if constexpr (EPI == kGroupScale && t == 0) wait_vmcnt<0>();   // the scales, of every tile
+    __syncthreads();
+    first[t].a = __half2float(tok[min((tid >> 2) & 15, p.M - 1)]);
+    if ((int)blockIdx.x * T + t < p.tiles_n)
+      decode_finish<1, EPI, EPI == kGroupScale ? KT : 0>(p, tile(t), red, table + t * TABLE, tok, first[t], tid);
+  });
+}
+
+template <int EPI, int T>
+int launch_rotate_decode(const __half* x, const GemmArgs& g, hipStream_t stream, const DecodePrologue* pro) {
+  constexpr int K = 4096, KT = K / 128;
+  constexpr size_t smem = (size_t)(EPI == kGroupScale ? KT : 2 * kWaves) * 1024 + (EPI == kGroupScale ? T * 16 * KT * 2 : 0) + 64 +
+                          kRotateGemmMaxTokens * (K / 2 + 16) + 32;
+  static_assert(smem <= 64 * 1024, "fits the default dynamic LDS limit");
+  const dim3 grid((g.tiles_n + T - 1) / T), block(kWaves * 64);
+  const DecodePrologue none{nullptr, 0.f, nullptr, nullptr};
+  if (!pro)
+    hipLaunchKernelGGL((rotate_gemm_i4_decode_kernel<EPI, T, false, false>), grid, block, smem, stream, x, g, 1.0f / 64.0f, none);
+  else if (pro->add)
+    hipLaunchKernelGGL((rotate_gemm_i4_decode_kernel<EPI, T, true, true>), grid, block, smem, stream, x, g, 1.0f / 64.0f, *pro);
+  else
+    hipLaunchKernelGGL((rotate_gemm_i4_decode_kernel<EPI, T, true, false>), grid, block, smem, stream, x, g, 1.0f / 64.0f, *pro);
+  return check_launch("rotate_gemm_i4_decode");
 }
 
 template <int EPI>
 int launch_rotate_decode(const __half* x, const GemmArgs& a, hipStream_t stream, const DecodePrologue* pro = nullptr) {
-  constexpr int K = 4096, KT = K / 128;
-  constexpr size_t smem = (size_t)(EPI == kGroupScale ? KT : 2 * kWaves) * 1024 + (EPI == kGroupScale ? 16 * KT * 2 : 0) + 64 +
-                          kRotateGemmMaxTokens * (K / 2 + 16) + 32;
-  static_assert(smem <= 64 * 1024, "fits the default dynamic LDS limit");
   GemmArgs g = a;
-  const int blocks = decode_blocks(g);
-  const dim3 grid(blocks), block(kWaves * 64);
-  const DecodePrologue none{nullptr, 0.f, nullptr, nullptr};
-  if (!pro)
-    hipLaunchKernelGGL((rotate_gemm_i4_decode_kernel<EPI>), grid, block, smem, stream, x, g, 1.0f / 64.0f, none);
-  else if (pro->add)
-    hipLaunchKernelGGL((rotate_gemm_i4_decode_kernel<EPI, true, true>), grid, block, smem, stream, x, g, 1.0f / 64.0f, *pro);
-  else
-    hipLaunchKernelGGL((rotate_gemm_i4_decode_kernel<EPI, true, false>), grid, block, smem, stream, x, g, 1.0f / 64.0f, *pro);
-  return check_launch("rotate_gemm_i4_decode");
+  g.tiles_n = decode_blocks(g);
+  // Two tiles per workgroup where one each would put several rotations on a compute unit and that costs more than the
+  // tiles' turns: with the norm always; without it, two and more tokens while two tiles each still are one round (9.2 ->
+  // 8.5 us at 6144 channels; 11.8 -> 12.1 at 12288), and beyond three and a half rounds (one token 22016 channels 13.2 ->
+  // 12.8, group scales 15.2 -> 14.1; 14336 10.2 either way).  One token without the norm rotates fast enough beside
+  // another workgroup's (8192 7.5 / 7.7, 12288 8.8 / 9.9).
+  const int n = g.tiles_n;
+  const bool two = n > 256 && (pro || n > 896 || (g.M > 1 && n <= 512));
+  return two ? launch_rotate_decode<EPI, 2>(x, g, stream, pro) : launch_rotate_decode<EPI, 1>(x, g, stream, pro);
 }
 
 }  // namespace

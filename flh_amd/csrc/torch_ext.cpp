@@ -536,6 +536,65 @@ std::vector<Tensor> rotate_quantize_gemm_i4_multi(const Tensor& x, const std::ve
   return Ds;
 }
 
+// RMSNorm(x [+ add]), rotation, quantiser and up to four GEMMs: {x + add or nothing, [fp16 [M, N_s] ...]}.  Every workgroup
+// of the one launch repeats the norm and the rotation, 2 us a token: one token gains up to two tiles of 16 channels per compute
+// unit (4096 x 6144 8.8 us against 10.0 for two launches, x 8192 9.5 / 10.2, but x 12288 14.1 / 11.4); two tokens don't at any
+// width (4096 x 1024 9.0 / 8.2, x 6144 11.7 / 10.1) and take the quantiser's launch and the GEMM's: the same bits.
+std::tuple<c10::optional<Tensor>, std::vector<Tensor>> rmsnorm_rotate_quantize_gemm_i4_multi(
+    const Tensor& x, const c10::optional<Tensor>& add, const c10::optional<Tensor>& weight, double eps,
+    const std::vector<Tensor>& Bs, const std::vector<Tensor>& B_scales) {
+  TORCH_CHECK(Bs.size() == B_scales.size() && !Bs.empty() && Bs.size() <= 4,
+              "one to four weight matrices, one scale tensor each");
+  for (size_t s = 0; s < Bs.size(); ++s) {
+    check_rotate_gemm(x, Bs[s], B_scales[s]);
+    TORCH_CHECK(B_scales[s].size(1) == B_scales[0].size(1), "the same scale width for every matrix");
+    TORCH_CHECK(Bs[s].size(0) > 0, "empty weight matrix");
+  }
+  const int64_t M = x.size(0), K = x.size(1);
+  if (add.has_value())
+    TORCH_CHECK(add->is_cuda() && add->scalar_type() == torch::kFloat16 && add->sizes() == x.sizes() && add->is_contiguous() &&
+                    add->device() == x.device(), "add must be a contiguous float16 CUDA tensor of x's shape");
+  if (weight.has_value())
+    TORCH_CHECK(weight->is_cuda() && weight->scalar_type() == torch::kFloat16 && weight->is_contiguous() &&
+                    weight->numel() == K && weight->device() == x.device(),
+                "weight must be a contiguous float16 CUDA tensor of K values");
+  c10::optional<Tensor> total;
+  if (add.has_value()) total = torch::empty_like(x);
+  std::vector<Tensor> Ds;
+  const uint8_t* b[4];
+  const flh_half* bs[4];
+  flh_half* d[4];
+  size_t n[4], channels = 0;
+  for (size_t s = 0; s < Bs.size(); ++s) {
+    Ds.push_back(torch::empty({M, Bs[s].size(0)}, x.options()));
+    b[s] = u8(Bs[s]);
+    bs[s] = h(B_scales[s]);
+    d[s] = hm(Ds[s]);
+    n[s] = (size_t)Bs[s].size(0);
+    channels += n[s];
+  }
+  if (M == 0) return {total, Ds};
+  const int count = (int)Bs.size(), cols = (int)B_scales[0].size(1);
+  const flh_half* w = weight.has_value() ? h(*weight) : nullptr;
+  Launch l(x);
+  // (a weight that the one launch refuses for its alignment is refused at every size)
+  if ((M == 1 && channels <= 8192) || ((uintptr_t)w & 15)) {
+    ok(flh_rmsnorm_rotate_quant_gemm_i4_o16_multi(h(x), add.has_value() ? h(*add) : nullptr, total.has_value() ? hm(*total) : nullptr,
+                                                  w, (float)eps, count, b, bs, d, n, M, K, cols, stream_of(x)));
+    return {total, Ds};
+  }
+  Tensor q = torch::empty({M, K / 2}, x.options().dtype(torch::kUInt8));
+  Tensor s = torch::empty({M, 1}, x.options());
+  if (add.has_value())
+    ok(flh_add_rmsnorm_rotate_quant_i4(h(x), h(*add), hm(*total), w, (float)eps, (uint8_t*)q.data_ptr(), hm(s), (uint32_t)M,
+                                       (uint32_t)K, FLH_HAD_F32, 1.0f, stream_of(x)));
+  else
+    ok(flh_rmsnorm_rotate_quant_i4(h(x), w, (float)eps, (uint8_t*)q.data_ptr(), hm(s), nullptr, (uint32_t)M, (uint32_t)K,
+                                   FLH_HAD_F32, 1.0f, stream_of(x)));
+  ok(flh_gemm_i4_o16_multi(u8(q), h(s), count, b, bs, d, n, M, K, 1, cols, 128, stream_of(x)));
+  return {total, Ds};
+}
+
 // ---- group kernels ------------------------------------------------------------------------------------------------
 void check_rows(const Tensor& x, int64_t width) {
   TORCH_CHECK(x.is_cuda(), "Input tensor must be on CUDA");
@@ -783,7 +842,9 @@ c10::optional<Tensor> linear_online_i4(const Tensor& x, const Tensor& w, const T
   if (mode < 0) mode = K == 11008 || K == 14336 ? FLH_HAD_MFMA : FLH_HAD_F32;
   const int64_t cols = w_scale.numel() / N;
   Launch l(x);
-  if (M <= 2 && K == 4096 && mode == FLH_HAD_F32 && (cols == 1 || (group == 128 && cols == 32))) {
+  // one launch while the rotation that every workgroup repeats costs less than a launch: one token 4096 x 12288 8.8 us against
+  // 9.9, two tokens x 8192 9.0 against 9.0, but two x 12288 11.8 against 10.3 and x 14336 12.5 against 10.7
+  if ((M == 1 || (M == 2 && N <= 8192)) && K == 4096 && mode == FLH_HAD_F32 && (cols == 1 || (group == 128 && cols == 32))) {
     Tensor D = empty_rows(x, N, x.options());
     ok(flh_rotate_quant_gemm_i4_o16(h(x), u8(w), h(w_scale), hm(D), M, N, K, (int)cols, stream_of(x)));
     return D;
@@ -907,6 +968,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_f6_dequant_multi", &gemm_f6_dequant_multi, py::arg("A6"), py::arg("B6s"), py::arg("A_scale"), py::arg("B_scales"));
   m.def("add_rmsnorm_rotate_and_quantize_i4_mode", &add_rmsnorm_rotate_and_quantize_i4_mode);
   m.def("rotate_and_quantize_f6_mode", &rotate_and_quantize_f6_mode);
+  m.def("rmsnorm_rotate_quantize_gemm_i4_multi", &rmsnorm_rotate_quantize_gemm_i4_multi, py::arg("x"), py::arg("add"),
+        py::arg("weight"), py::arg("eps"), py::arg("Bs"), py::arg("B_scales"));
   m.def("linear_i4", &linear_i4);
   m.def("linear_online_i4", &linear_online_i4);
   m.def("quantize_groups", &quantize_groups);

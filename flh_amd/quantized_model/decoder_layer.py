@@ -348,7 +348,7 @@ class W4A4DecoderLayer(torch.nn.Module):
         b, t, _ = x.shape
         if (self.activation == "token" and self.fused and self.record is None and b * t <= 2 and self.hidden_size == 4096
                 and self._online_qkv_applies()):
-            # decode: residual addition, norm, rotation, quantiser and the three projections in one launch
+            # decode: residual addition, norm, rotation, quantiser and the three projections in one launch, two where faster
             layers = [self.q_proj, self.k_proj, self.v_proj]
             total, (qs, ks, vs) = _ops().rmsnorm_rotate_quantize_gemm_i4_multi(
                 x.reshape(b * t, -1).contiguous(), None if add is None else add.reshape(b * t, -1).contiguous(),

@@ -161,3 +161,68 @@ def test_group_scales_at_any_element_offset(ops, n, offset):
     moved.copy_(sd)
     assert moved.data_ptr() % 16 == 2 * offset % 16
     assert torch.equal(ops.rotate_quantize_gemm_i4(x, wd, moved), ops.rotate_quantize_gemm_i4(x, wd, sd))
+
+
+@pytest.mark.parametrize("m", [1, 2, 3])
+@pytest.mark.parametrize("grouped", [False, True])
+@pytest.mark.parametrize("ns", [(4096,), (4112,), (4100, 17), (2048, 2048, 24), (8192,), (4096, 4096, 1), (14352,), (14336,)])
+def test_tiles_per_workgroup(ops, m, grouped, ns):
+    """One and two tiles of 16 channels per workgroup, around the lines (256, 512 and 896 tiles), odd tile counts, a pair
+    that spans two matrices: the outputs bit for bit those of the separate launches, the sum included."""
+    import flh_amd
+    k, cols = 4096, 32 if grouped else 1
+    print(f"case tiles m={m} grouped={grouped} ns={ns}", flush=True)
+    x, add = dev(syn.activations(m, k, seed=m)), dev(syn.activations(m, k, seed=m + 9))
+    nw = dev(np.random.default_rng(3).uniform(0.5, 1.5, k).astype(np.float16))
+    ws = [weights(n, k, cols, seed=n + m) for n in ns]
+    Bs, Ss = [dev(w) for w, _ in ws], [dev(s) for _, s in ws]
+    same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+    q, s = ops.rotate_and_quantize_i4(x, hadamard="exact")
+    want = [ops.gemm_i4_dequant(q, B, s, S, 128) for B, S in zip(Bs, Ss)]
+    assert all(same(a, b) for a, b in zip(ops.rotate_quantize_gemm_i4_multi(x, Bs, Ss), want))
+
+    total, q, s = ops.add_rmsnorm_rotate_and_quantize_i4(x, add, nw, 1e-5)
+    want = [ops.gemm_i4_dequant(q, B, s, S, 128) for B, S in zip(Bs, Ss)]
+    for module in (ops, flh_amd._CUDA):                  # the one launch, and the op that picks one or two
+        got, outs = module.rmsnorm_rotate_quantize_gemm_i4_multi(x, add, nw, 1e-5, Bs, Ss)
+        assert same(got, total) and all(same(a, b) for a, b in zip(outs, want))
+    q, s = ops.rmsnorm_rotate_and_quantize_i4(x, None, 1e-5)
+    want = [ops.gemm_i4_dequant(q, B, s, S, 128) for B, S in zip(Bs, Ss)]
+    for module in (ops, flh_amd._CUDA):
+        got, outs = module.rmsnorm_rotate_quantize_gemm_i4_multi(x, None, None, 1e-5, Bs, Ss)
+        assert got is None and all(same(a, b) for a, b in zip(outs, want))
+
+
+@pytest.mark.parametrize("n", [8192, 8208])
+@pytest.mark.parametrize("m", [1, 2, 3])
+def test_online_linear_on_both_sides_of_the_line(ops, m, n):
+    from flh_amd.nn.linear import LinearFLH
+    w, s = weights(n, 4096, 1, seed=n)
+    layer = LinearFLH(4096, n, group_size=-1).cuda()
+    layer.w_packed = dev(w).flatten()
+    layer.w_scale = dev(s)
+    x = dev(syn.activations(m, 4096, seed=n + m))
+    q, a = ops.rotate_and_quantize_i4(x, hadamard="exact")
+    assert torch.equal(layer.forward_online(x, hadamard="exact"), ops.gemm_i4_dequant(q, dev(w), a, dev(s), 128))
+
+
+def test_norm_prologue_refuses_the_same_at_every_size():
+    """The op that picks one or two launches: what the one launch refuses, it refuses beyond its line as well."""
+    import flh_amd
+    op = flh_amd._CUDA.rmsnorm_rotate_quantize_gemm_i4_multi
+    B = torch.zeros(64, 2048, dtype=torch.uint8, device="cuda")
+    S = torch.ones(64, 1, dtype=torch.float16, device="cuda")
+    odd = torch.ones(4104, dtype=torch.float16, device="cuda")[1:4097]
+    for m in (1, 2):
+        x = torch.zeros(m, 4096, dtype=torch.float16, device="cuda")
+        for add, weight, eps in ((None, odd, 1e-5), (x.clone(), odd, 1e-5), (None, None, -1.0), (x[:, :2048], None, 1e-5),
+                                 (None, torch.ones(100, dtype=torch.float16, device="cuda"), 1e-5)):
+            with pytest.raises(RuntimeError):
+                op(x, add, weight, eps, [B], [S])
+        with pytest.raises(RuntimeError):
+            op(x, None, None, 1e-5, [B, B[:0]], [S, S[:0]])
+        with pytest.raises(RuntimeError):
+            op(torch.zeros(5, 4096, dtype=torch.float16, device="cuda"), None, None, 1e-5, [B], [S])
+    total, outs = op(x[:0], x[:0], None, 1e-5, [B], [S])
+    assert total.shape == (0, 4096) and outs[0].shape == (0, 64)
