@@ -525,10 +525,15 @@ class W4A4DecoderLayer(torch.nn.Module):
         c = cols.pop()
         return c == 1 or (c == self.hidden_size // 128 and self.q_proj.weight_group_size == 128)
 
-    def _swiglu_gemm_applies(self):
+    def _swiglu_gemm_applies(self, rows):
+        """Whether gate and up take the launch that stores silu(gate) * up only: prefill sizes.  Group configuration, us per layer,
+        two outputs -> the product: 4096 tokens 1050 -> 1030, 1000 326 -> 322, 100 102 -> 101, 33 79 -> 84; with one scale per weight
+        row 2048 tokens 679 -> 668, 129 .. 1000 equal, 100 143 -> 150."""
         g = self.gate_proj
         cols = g.w_scale.numel() // g.out_features
-        return g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
+        if self.activation == "group" and (self.act_group_size != 128 or (cols == 1 and rows <= 1024)):
+            return False
+        return rows > 64 and g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
 
     def _group_quant(self, stage, quantizer, x, consumers=()):
         if (self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)) and _stock_call(quantizer, ActQuantizer)
@@ -551,11 +556,18 @@ class W4A4DecoderLayer(torch.nn.Module):
         x, s, z, q = self._residual_norm_quant("mlp_in", self.post_attention_layernorm, "post_attention_layernorm",
                                                self.mlp_quantizer1, x, add, (self.gate_proj, self.up_proj))
         rows = q.numel() // q.size(-1)
-        if (self.activation == "token" and self.fused and self.record is None and rows > 64
-                and self._swiglu_gemm_applies()):
+        if self.fused and self.record is None and self._swiglu_gemm_applies(rows):
             # prefill: gate and up in one launch that stores silu(gate) * up only (no fp16 [M, I] round trips)
-            s, z, q = self._token_quant("mlp_mid", LinearFLH.forward_swiglu(self.gate_proj, self.up_proj, q, s),
-                                        consumers=(self.down_proj,))
+            mid = LinearFLH.forward_swiglu(self.gate_proj, self.up_proj, q, s)
+            if self.activation == "token":
+                s, z, q = self._token_quant("mlp_mid", mid, consumers=(self.down_proj,))
+            else:
+                if self._group_six_bit_for((self.down_proj,), rows, mid.size(-1)):
+                    q, s = _ops().group_quantize_f6(mid.view(rows, -1), False)
+                else:
+                    q, s = _ops().quant_and_pack_i4_gs(mid.view(-1, 128), 128)
+                s, z, q = s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
+                fold_residual = fold_residual and self._residual_in_gemm(rows, self.down_proj)
             if fold_residual:
                 return self.down_proj(q, s, z, x_is_packed=True, residual=x), None
             return x, self.down_proj(q, s, z, x_is_packed=True)

@@ -189,3 +189,23 @@ def test_hooks_on_projections_see_packed_codes_and_leave_the_bits(activation, t)
     got = layer(x, cos, sin)
     assert torch.equal(got[0], want[0]) and all(torch.equal(a, b) for a, b in zip(got[1], want[1]))
     assert [s[0] for s in seen] == [256, 512] and (t > 64 or not any(s[1] for s in seen))
+
+
+@pytest.mark.parametrize("weight_group,six_bit,shapes", [(128, False, [(1, 64), (1, 65), (3, 43), (1, 257), (2, 300), (1, 1100)]),
+                                                         (128, True, [(1, 65), (1, 131)]), (0, False, [(1, 65), (2, 512), (1, 1025)])])
+def test_group_layer_with_the_product_in_the_gemm_gives_the_same_bits(monkeypatch, weight_group, six_bit, shapes):
+    """gate / up as one launch that stores silu(gate) * up against two outputs and the product in the quantiser, on both sides
+    of the lines; 1408 channels: an odd number of tiles."""
+    w, _ = make(inter=1408, seed=11)
+    layer = W4A4DecoderLayer.from_float(w, 4, 2, weight_group_size=weight_group, activation="group", six_bit=six_bit)
+    for b, t in shapes:
+        print(f"case swiglu weight_group={weight_group} six_bit={six_bit} {b} x {t}", flush=True)
+        x = torch.randn(b, t, 512, generator=torch.Generator().manual_seed(t)).half().cuda()
+        got, pending = layer._mlp(x, None)
+        alone = layer.mlp(x)
+        with monkeypatch.context() as m:
+            m.setattr(W4A4DecoderLayer, "_swiglu_gemm_applies", lambda self, rows: False)
+            want, want_pending = layer._mlp(x, None)
+            want_alone = layer.mlp(x)
+        assert (pending is None) == (want_pending is None) and torch.equal(got, want) and torch.equal(alone, want_alone)
+        assert pending is None or torch.equal(pending, want_pending)
