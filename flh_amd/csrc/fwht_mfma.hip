@@ -378,6 +378,9 @@ __device__ __forceinline__ v2i quantise_half_block(const unsigned (&y)[8], float
 // loads, 16-byte chunks XOR-swizzled by the row so that the tile reads are free of bank conflicts), instead of
 // every wave waiting for its X tiles from memory three at a time (in-kernel timestamps for one row of 14336: the
 // main loop took 13 k clocks of a 23 k clock kernel, almost all of it waiting for those tiles).
+// A wave reads the factor fragments of its own output tiles only (with all of them read by every wave, 780 KB at the 128
+// bytes a clock of LDS, one row of 14336 took 6.6 us and with SILU 7.9, now 5.4 and 6.8; 11008 5.5 and 7.0, now 4.8 and 6.2), and the
+// product of SILU is formed while the table is still on its way.
 //
 // SILU (short batches only): the row is the SwiGLU product fp16(fp16(silu(gate)) * up) of two input rows, x = gate and
 // x2 = up -- what the reference's MLP hands to the quantiser of down_proj (flh/quantized_model/modeling_llama.py:522-526).
@@ -445,6 +448,8 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
     return x + (size_t)(r < M ? r : M - 1) * K;        // rows past the end repeat the last one and store nothing
   };
   constexpr uint32_t RPW = SPLIT ? 1u : 4u;            // rows per workgroup and iteration
+  constexpr int NW = SPLIT ? (DT + 3) / 4 : DT;        // j' tiles of a wave: all, or slot, slot + 4 (past the last one: that one again)
+  auto tile_of = [&](int i) { return SPLIT ? min(slot + 4 * i, DT - 1) : i; };
   const uint32_t base0 = blockIdx.x * RPW, stride = gridDim.x * RPW;
   // the first row's first tiles are requested before the factor table, so that both travel together
   if constexpr (SPLIT) {
@@ -469,7 +474,8 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
       const int f = (i + first) % NFRAG;
       load_to_lds16(table + f * 64 + lane, lds0 + f * 1024);
     }
-    wait_vmcnt<0>();
+    if constexpr (SILU) wait_vmcnt<NFRAG / 8>();       // the two rows; the table travels on
+    else wait_vmcnt<0>();
     __syncthreads();
   }
   if constexpr (SILU) {
@@ -482,6 +488,7 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
       for (int e = 0; e < 8; ++e) o[e] = silu_mul_f16(g[e], u[e]);
       g8[i] = o;
     }
+    wait_vmcnt<0>();
     __syncthreads();
   }
   if constexpr (SPLIT) {
@@ -501,14 +508,15 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
     const uint32_t row = SPLIT ? base : base + slot;
     const bool valid = row < M;
     const __half* xr = row_ptr(base);
-    v16f w[DT];                                        // level-2 accumulators of this t' tile, [j' tile]
+    v16f w[NW];                                        // level-2 accumulators of this t' tile, [j' tile of the wave]
 #pragma unroll
-    for (int b = 0; b < DT; ++b)
+    for (int b = 0; b < NW; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) w[b][r] = 0.f;
-    constexpr int AHEAD = DT <= 6 ? 7 : 3, RING = AHEAD + 1;   // factor fragments travel a few fragments ahead
+    constexpr int AHEAD = SPLIT || DT <= 6 ? 7 : 3, RING = AHEAD + 1;   // factor fragments travel a few fragments ahead
+    constexpr int OWN = 2 * DT * NW;                   // the wave's own, in order of use
     h8 fr[RING];
-    auto fetch = [&](int f) { fr[f % RING] = mfrag[f * 64 + lane]; };
+    auto fetch = [&](int f) { fr[f % RING] = mfrag[(f / NW * DT + tile_of(f % NW)) * 64 + lane]; };
 #pragma unroll
     for (int f = 0; f < AHEAD; ++f) fetch(f);
 #pragma unroll
@@ -528,11 +536,10 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int nt = 0; nt < DT; ++nt) {
-          const int f = (kb * 2 + s) * DT + nt;
-          if (f + AHEAD < NFRAG) fetch(f + AHEAD);
-          if (!SPLIT || (nt & 3) == slot)
-            w[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[s]), fr[f % RING], w[nt], 0, 0, 0);
+        for (int nt = 0; nt < NW; ++nt) {
+          const int f = (kb * 2 + s) * NW + nt;
+          if (f + AHEAD < OWN) fetch(f + AHEAD);
+          w[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[s]), fr[f % RING], w[nt], 0, 0, 0);
         }
     }
     if constexpr (!SPLIT) {
@@ -542,10 +549,10 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
       }
     }
 
-    // w[nt][4 g + e]: t' = 32 mt + 8 g + 4 h + e,  j' = 32 nt + col
+    // w[nt][4 g + e]: t' = 32 mt + 8 g + 4 h + e,  j' = 32 tile_of(nt) + col
     float mx = 0.f;
 #pragma unroll
-    for (int nt = 0; nt < DT; ++nt)
+    for (int nt = 0; nt < NW; ++nt)
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         mx = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(w[nt][2 * u]), __builtin_fabsf(w[nt][2 * u + 1])), mx);
@@ -573,11 +580,12 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
     uint8_t* qr = q + (size_t)(valid ? row : M - 1) * (K / 2) + mt * 16 + h * 8;
     auto emit = [&](auto careful_tag) {
 #pragma unroll
-      for (int nt = 0; nt < DT; ++nt) {
-        if (SPLIT && (nt & 3) != slot) continue;
+      for (int i = 0; i < NW; ++i) {
+        const int nt = tile_of(i);
+        if (SPLIT && i > 0 && slot + 4 * i >= DT) continue;   // another wave's
         unsigned y[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) y[u] = scale_pack_f16(w[nt][2 * u], w[nt][2 * u + 1], c);
+        for (int u = 0; u < 8; ++u) y[u] = scale_pack_f16(w[i][2 * u], w[i][2 * u + 1], c);
         const v2i out = quantise_half_block<decltype(careful_tag)::value>(y, rinv, hb);
         if constexpr (F6) {                            // (the hardware's conversion in the table's place: 8192 x 14336 94 -> 96.6 us)
           // this lane: codes 32 mt + 16 h + 0 .. 15 of block j' = 32 nt + col, i.e. 12 bytes at byte 12 h of the piece
