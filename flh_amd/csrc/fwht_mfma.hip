@@ -369,18 +369,17 @@ __device__ __forceinline__ v2i quantise_half_block(const unsigned (&y)[8], float
 // (DT accumulator tiles, few enough registers for two waves per SIMD), then half of every block column
 // of the epilogue.  The pair meets once per row to exchange its maxima through LDS.
 //
-// SPLIT (short batches, one row per workgroup): the four wave pairs share one row instead -- every pair runs
-// level 1, but of level 2 and of the epilogue only the output tiles j' = slot, slot + 4, ...; the row maximum is
-// the maximum over all eight waves.  Every output still accumulates its K blocks in the same order, so the
-// codes are the ones the unsplit kernel produces; a batch of M rows then occupies M compute units instead of
-// M / 4, each with a third to a half of the MFMA work per wave.  Here a row's latency is what counts, and all
-// eight waves read the whole row: it is staged in LDS once, requested together with the factor table (direct-to-LDS
-// loads, 16-byte chunks XOR-swizzled by the row so that the tile reads are free of bank conflicts), instead of
-// every wave waiting for its X tiles from memory three at a time (in-kernel timestamps for one row of 14336: the
-// main loop took 13 k clocks of a 23 k clock kernel, almost all of it waiting for those tiles).
-// A wave reads the factor fragments of its own output tiles only (with all of them read by every wave, 780 KB at the 128
-// bytes a clock of LDS, one row of 14336 took 6.6 us and with SILU 7.9, now 5.4 and 6.8; 11008 5.5 and 7.0, now 4.8 and 6.2), and the
-// product of SILU is formed while the table is still on its way.
+// SPLIT (short batches, one row per workgroup): the four wave pairs share one row instead -- of level 1 a pair runs
+// the blocks kb = slot, slot + 4 (Z, rounded as ever, meets in LDS), of level 2 and of the epilogue the output
+// tiles j' = slot, slot + 4; the row maximum is the maximum over all eight waves.  Every output still accumulates its K
+// blocks in the same order, so the codes are the ones the unsplit kernel produces; a batch of M rows then occupies M
+// compute units instead of M / 4, each with a quarter to a third of the MFMA work per wave.  Here a row's latency is
+// what counts: the row is staged in LDS, requested together with the factor table (direct-to-LDS loads, 16-byte chunks
+// XOR-swizzled by the row so that the tile reads are free of bank conflicts).
+// A wave reads the factor fragments of its own output tiles only, and the product of SILU is formed while the table is
+// still on its way.  us, one row of 14336 / with SILU / 11008 / with SILU: every wave all the fragments and all of level 1 6.6 / 7.9 /
+// 5.5 / 7.0, its own fragments 5.4 / 6.8 / 4.8 / 6.2, its own level 1 as well 5.1 / 6.3 / 4.7 / 6.0 (sixteen waves: the same, 256 rows
+// 6.2 against 6.1).  Bound by the arrival of the row and of the table, whose first access is cold.
 //
 // SILU (short batches only): the row is the SwiGLU product fp16(fp16(silu(gate)) * up) of two input rows, x = gate and
 // x2 = up -- what the reference's MLP hands to the quantiser of down_proj (flh/quantized_model/modeling_llama.py:522-526).
@@ -426,15 +425,9 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
   h8 xa[NB][4];
   auto load_tile = [&](const __half* xr, int kb, int buf) {
     const int j = 32 * kb + col;
-    if constexpr (SPLIT) {
-      const uint8_t* src = xs + j * 128;               // (rows past D hold a copy of the last row, zeroed below)
+    const __half* src = xr + (j < D ? j : D - 1) * 64 + 8 * h;   // padded rows: any valid address, zeroed below
 #pragma unroll
-      for (int s = 0; s < 4; ++s) xa[buf][s] = *(const h8*)(src + (((2 * s + h) ^ (j & 7)) << 4));
-    } else {
-      const __half* src = xr + (j < D ? j : D - 1) * 64 + 8 * h;   // padded rows: any valid address, zeroed below
-#pragma unroll
-      for (int s = 0; s < 4; ++s) xa[buf][s] = *(const h8*)(src + 16 * s);
-    }
+    for (int s = 0; s < 4; ++s) xa[buf][s] = *(const h8*)(src + 16 * s);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto finish_tile = [&](int kb, int buf) {
@@ -491,11 +484,6 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
     wait_vmcnt<0>();
     __syncthreads();
   }
-  if constexpr (SPLIT) {
-#pragma unroll
-    for (int t = 0; t < NB - 1; ++t) load_tile(nullptr, t, t);
-  }
-
   // The wave pairs of row slots 2 and 3 run one phase behind those of slots 0 and 1: every iteration has two
   // workgroup barriers (after the MFMA phase, where a pair exchanges its maxima, and after the quantising
   // phase), and the late pairs pass one extra barrier before the loop, the early pairs one after it.  While
@@ -519,20 +507,52 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
     auto fetch = [&](int f) { fr[f % RING] = mfrag[(f / NW * DT + tile_of(f % NW)) * 64 + lane]; };
 #pragma unroll
     for (int f = 0; f < AHEAD; ++f) fetch(f);
-#pragma unroll
-    for (int kb = 0; kb < DT; ++kb) {
-      if (kb + NB - 1 < DT) load_tile(xr, kb + NB - 1, (kb + NB - 1) % NB);
-      finish_tile(kb, kb % NB);
+    auto level1 = [&](const h8 (&t)[4], v4i (&a)[2]) {
       v16f z;
 #pragma unroll
       for (int r = 0; r < 16; ++r) z[r] = 0.f;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[kb % NB][s], b1(s), z, 0, 0, 0);
-      v4i a[2];
+      for (int s = 0; s < 4; ++s) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(t[s], b1(s), z, 0, 0, 0);
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int u = 0; u < 4; ++u) a[s][u] = (int)pack_f16(z[8 * s + 2 * u], z[8 * s + 2 * u + 1]);
+    };
+    v4i za[SPLIT ? DT : 1][2];
+    if constexpr (SPLIT) {
+      v4i* const zs = (v4i*)(xs + DT * 4096);          // [kb][mt][s][lane], in the place of the up row
+      v4i mine[NW][2];
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        const int j = 32 * tile_of(i) + col;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {                  // (rows past D hold a copy of the last row)
+          const h8 v = *(const h8*)(xs + j * 128 + (((2 * s + h) ^ (j & 7)) << 4));
+          xa[i][s] = j < D ? v : h8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NW; ++i) level1(xa[i], mine[i]);
+#pragma unroll
+      for (int i = 0; i < NW; ++i)                     // (past the last block: that one's values again, from several waves)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) zs[((tile_of(i) * 2 + mt) * 2 + s) * 64 + lane] = mine[i][s];
+      __syncthreads();
+#pragma unroll
+      for (int kb = 0; kb < DT; ++kb)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) za[kb][s] = zs[((kb * 2 + mt) * 2 + s) * 64 + lane];
+    }
+#pragma unroll
+    for (int kb = 0; kb < DT; ++kb) {
+      v4i a[2];
+      if constexpr (SPLIT) {
+        a[0] = za[kb][0], a[1] = za[kb][1];
+      } else {
+        if (kb + NB - 1 < DT) load_tile(xr, kb + NB - 1, (kb + NB - 1) % NB);
+        finish_tile(kb, kb % NB);
+        level1(xa[kb % NB], a);
+      }
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -667,7 +687,7 @@ int launch_dense(const __half* x, uint8_t* q, __half* scales, uint32_t M, float 
   // short batches take one row per workgroup (SPLIT: exactly one -- the grid is M -- with the row staged in LDS),
   // long ones four; 6-bit output (a prefill format) always takes the long-batch kernel
   const bool split = M <= 256 && !f6;
-  const size_t smem = (size_t)NFRAG * 1024 + 64 + (split ? (size_t)DT * 4096 : 0);   // factor fragments, the pairs' maxima, the row
+  const size_t smem = (size_t)NFRAG * 1024 + 64 + (split ? 2 * (size_t)DT * 4096 : 0);   // factor fragments, the pairs' maxima, the row and its first level
   auto kern = f6 ? rotate_quant_mfma_dense_kernel<DT, false, false, true>
                  : split ? rotate_quant_mfma_dense_kernel<DT, true> : rotate_quant_mfma_dense_kernel<DT, false>;
   constexpr int kThreadsDense = 512;
