@@ -369,7 +369,7 @@ __device__ __forceinline__ v2i quantise_half_block(const unsigned (&y)[8], float
 // (DT accumulator tiles, few enough registers for two waves per SIMD), then half of every block column
 // of the epilogue.  The pair meets once per row to exchange its maxima through LDS.
 //
-// SPLIT (short batches, one row per workgroup): the four wave pairs share one row instead -- of level 1 a pair runs
+// SPLIT (short batches, one row per workgroup at a time): the four wave pairs share one row instead -- of level 1 a pair runs
 // the blocks kb = slot, slot + 4 (Z, rounded as ever, meets in LDS), of level 2 and of the epilogue the output
 // tiles j' = slot, slot + 4; the row maximum is the maximum over all eight waves.  Every output still accumulates its K
 // blocks in the same order, so the codes are the ones the unsplit kernel produces; a batch of M rows then occupies M
@@ -444,11 +444,10 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
   constexpr int NW = SPLIT ? (DT + 3) / 4 : DT;        // j' tiles of a wave: all, or slot, slot + 4 (past the last one: that one again)
   auto tile_of = [&](int i) { return SPLIT ? min(slot + 4 * i, DT - 1) : i; };
   const uint32_t base0 = blockIdx.x * RPW, stride = gridDim.x * RPW;
-  // the first row's first tiles are requested before the factor table, so that both travel together
-  if constexpr (SPLIT) {
-    // the whole row into LDS: one instruction moves eight rows of X (64 chunks of 16 bytes), lane p of it the chunk
-    // that belongs at slot p
-    const __half* xr = row_ptr(base0);
+  // SPLIT: a whole row into LDS.  One instruction moves eight rows of X (64 chunks of 16 bytes), lane p of it the chunk
+  // that belongs at slot p
+  auto stage_row = [&](uint32_t base) {
+    const __half* xr = row_ptr(base);
     const unsigned xs0 = (unsigned)(size_t)xs;
     for (int i = wave; i < DT * 4; i += 8) {
       const int j = 8 * i + (lane >> 3), c = (lane & 7) ^ (j & 7);
@@ -456,6 +455,10 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
       if constexpr (SILU)                              // the up row behind the gate row, same slot order
         load_to_lds16(x2 + (xr - x) + (j < D ? j : D - 1) * 64 + c * 8, xs0 + DT * 4096 + i * 1024);
     }
+  };
+  // the first row's first tiles are requested before the factor table, so that both travel together
+  if constexpr (SPLIT) {
+    stage_row(base0);
   } else if (base0 < M) {
 #pragma unroll
     for (int t = 0; t < NB - 1; ++t) load_tile(row_ptr(base0), t, t);
@@ -538,6 +541,8 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
 #pragma unroll
         for (int s = 0; s < 2; ++s) zs[((tile_of(i) * 2 + mt) * 2 + s) * 64 + lane] = mine[i][s];
       __syncthreads();
+      if constexpr (!SILU)                             // every wave is done with the row: the next one travels during the rest
+        if (base + stride < M) stage_row(base + stride);
 #pragma unroll
       for (int kb = 0; kb < DT; ++kb)
 #pragma unroll
@@ -627,8 +632,9 @@ __global__ __launch_bounds__(512) void rotate_quant_mfma_dense_kernel(const __ha
     if (careful) emit(std::true_type{});
     else emit(std::false_type{});
     if (valid && lane == 0 && mt == 0 && (!SPLIT || slot == 0)) scales[row] = __builtin_bit_cast(__half, s16);
+    if constexpr (SILU) break;                         // one row per workgroup
+    if constexpr (SPLIT) wait_vmcnt<0>();              // the next row is there
     barrier_no_fence();                                // end of the quantising phase (see above the loop)
-    if constexpr (SPLIT) break;                        // one row per workgroup: only that row was staged
   }
   if (!late) barrier_no_fence();
 }
@@ -684,16 +690,18 @@ int launch_dense(const __half* x, uint8_t* q, __half* scales, uint32_t M, float 
   constexpr int K = DenseFactor<DT>::D * 64;
   const h8* table = nullptr;
   if (int rc = dense_table<DT>(&table)) return rc;
-  // short batches take one row per workgroup (SPLIT: exactly one -- the grid is M -- with the row staged in LDS),
-  // long ones four; 6-bit output (a prefill format) always takes the long-batch kernel
-  const bool split = M <= 256 && !f6;
+  // short batches take one row per workgroup at a time (SPLIT, the row staged in LDS, the next one requested behind its first
+  // level), long ones four: the line is where three rounds of 256 rows end.  us in a graph, four at a time / one: 11008 300 rows
+  // 10.9 / 7.9, 512 11.3 / 8.2, 768 11.8 / 10.7, 800 11.8 / 13.0; 14336 300 12.7 / 8.6, 512 13.1 / 9.0, 768 13.7 / 12.2, 800 13.7 / 14.8.
+  // 6-bit output (a prefill format) always takes the long-batch kernel
+  const bool split = M <= 768 && !f6;
   const size_t smem = (size_t)NFRAG * 1024 + 64 + (split ? 2 * (size_t)DT * 4096 : 0);   // factor fragments, the pairs' maxima, the row and its first level
   auto kern = f6 ? rotate_quant_mfma_dense_kernel<DT, false, false, true>
                  : split ? rotate_quant_mfma_dense_kernel<DT, true> : rotate_quant_mfma_dense_kernel<DT, false>;
   constexpr int kThreadsDense = 512;
   static LdsGrant grants[3];                           // one per kernel variant
   if (int rc = reserve_lds((const void*)kern, smem, grants[f6 ? 2 : split], "rotate_quant")) return rc;
-  const unsigned blocks = split ? M : ((M + 3) / 4 < 256u ? (M + 3) / 4 : 256u);
+  const unsigned groups = split ? M : (M + 3) / 4, blocks = groups < 256u ? groups : 256u;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreadsDense), smem, stream, x, q, scales, table, M,
                      1.0f / sqrtf((float)K), clip, (const __half*)nullptr);
   return check_launch("rotate_quant_mfma_dense");

@@ -48,3 +48,19 @@ def test_norm_in_float32(weighted):
     y = ops.rmsnorm_rotate_and_quantize_i4(x, w, 1e-5, False, return_rotated=True)[2]
     want = ops.add_rmsnorm(x, w, 1e-5)
     assert torch.isfinite(y).all() and ((y.float() - want.float()).abs() <= want.float().abs() * 2.0 ** -10 + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("k", [11008, 14336])
+def test_dense_rotation_of_rows_one_after_the_other_agrees_with_long_batches(k):
+    """One row at a time per workgroup, up to three one after the other (768 rows), against the kernel of long batches: the same bytes on
+    both sides of every round of 256 workgroups."""
+    from flh_amd import _ops as ops
+    x = torch.randn(1300, k, generator=torch.Generator().manual_seed(k)).half()
+    x[::97] = 0
+    x[5, 3], x[300, 7] = 60000.0, 1e-7
+    x = x.cuda()
+    q_long, s_long = ops.rotate_and_quantize_i4(x)
+    for m in (1, 255, 256, 257, 511, 512, 513, 767, 768, 769, 1023, 1024, 1025):
+        print(f"case dense k={k} m={m}", flush=True)
+        q, s = ops.rotate_and_quantize_i4(x[1300 - m:].contiguous())
+        assert torch.equal(q, q_long[1300 - m:]) and torch.equal(s, s_long[1300 - m:]), m
