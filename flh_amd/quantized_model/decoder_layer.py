@@ -466,8 +466,10 @@ class W4A4DecoderLayer(torch.nn.Module):
             return None
         layers = (self.q_proj, self.k_proj, self.v_proj)
         group = self.q_proj.weight_group_size if self.q_proj.weight_group_size > 0 else (self.q_proj.in_group_size or 128)
-        six = not any(l._below_six_bit(rows) for l in layers) and all(l._six_bit_applies(codes.reshape(rows, -1), scales.reshape(rows, -1), l.w_scale.view(l.out_features, -1), group,
-                                       sum(c.out_features for c in layers)) for l in layers)
+        columns = sum(c.out_features for c in layers)
+        six = not any(l._below_six_bit(rows) for l in layers) and all(
+            l._six_bit_applies(codes.reshape(rows, -1), scales.reshape(rows, -1), l.w_scale.view(l.out_features, -1), group, columns)
+            for l in layers)
         return "f6" if six else "i4"
 
     def _attention_after_fused_qkv(self, x, codes, scales, cos, sin, kv_cache, positions, fold_residual, mode):
