@@ -39,10 +39,10 @@ __device__ __forceinline__ u6 bf6_of_wholes(const unsigned (&h)[16]) {
 }
 // bytes from a block's start to the six of its chunk of eight codes c16 = 0 .. 15
 __device__ __forceinline__ int f6_chunk_at(int c16) { return 48 * ((c16 >> 2) & 1) + 24 * (c16 >> 3) + 6 * (c16 & 3); }
+typedef unsigned u32_at2 __attribute__((aligned(2)));
 // chunk k = 0 .. 3 of what bf6_of_wholes gave
 template <int K>
 __device__ __forceinline__ void f6_store_six(const u6& r, uint8_t* dst) {
-  typedef unsigned u32_at2 __attribute__((aligned(2)));
   constexpr int w = K / 2 * 3;
   if constexpr (K % 2 == 0) {
     *(u32_at2*)dst = r[w];
@@ -51,6 +51,14 @@ __device__ __forceinline__ void f6_store_six(const u6& r, uint8_t* dst) {
     *(u32_at2*)dst = __builtin_amdgcn_alignbit(r[w + 2], r[w + 1], 16);
     *(unsigned short*)(dst + 4) = (unsigned short)(r[w + 2] >> 16);
   }
+}
+// The eight codes of a chunk from their nibbles.  For rows that are not finite throughout: the quotient of a NaN, or of an infinity,
+// is a NaN, of which the nibble packer makes some code (and, by carries, something of its neighbours) and the conversion
+// another one.  By way of the nibbles both formats hold the same codes.
+__device__ __forceinline__ void f6_store_nibbles(unsigned w, uint8_t* dst) {
+  const unsigned long long codes = bf6_of_nibbles(w);
+  *(u32_at2*)dst = (unsigned)codes;
+  *(unsigned short*)(dst + 4) = (unsigned short)(codes >> 32);
 }
 
 }  // namespace flh

@@ -243,8 +243,23 @@ __global__ __launch_bounds__(256, 2) void rotate_quant_mfma4096_kernel(const __h
         for (int u = 0; u < 8; ++u) {
           const float a = w[mt][nt][2 * u], b = w[mt][nt][2 * u + 1];
           y[mt][nt][u] = pack_f16(a, b);
-          mx = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(a), __builtin_fabsf(b)), mx);
+          if constexpr (F6)                  // (the one that keeps NaNs; one instruction, as the other)
+            mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)), mx);
+          else mx = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(a), __builtin_fabsf(b)), mx);
         }
+    bool finite = true;                      // (F6) every y is: none is NaN or rounds to an infinity
+    if constexpr (F6) {
+      finite = __builtin_amdgcn_ballot_w64(!(mx < 65520.f)) == 0;
+      if (__builtin_expect(!finite, 0)) {
+        mx = 0.f;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(__builtin_fabsf(w[mt][nt][r]), mx);
+      }
+    }
     mx = (float)(_Float16)wave_max(mx);      // max |fp16(w)| = fp16(max |w|): rounding is monotonic
     if (clip < 1.0f) mx = (float)(_Float16)round_here(mx * clip);   // clip bound; values are clamped in quantise_block
     _Float16 s16 = scale_of_max(mx);
@@ -261,11 +276,17 @@ __global__ __launch_bounds__(256, 2) void rotate_quant_mfma4096_kernel(const __h
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
           const int jp = 32 * nt + col;
+          v2i* dst = (v2i*)(q + ((size_t)(jp >> 1) * M + row) * kF6BlockBytes + 48 * h + 24 * (jp & 1));
+          if (__builtin_expect(!finite, 0)) {
+            const v4i out = quantise_block<decltype(careful_tag)::value>(y[0][nt], y[1][nt], rinv, hb);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) f6_store_nibbles((unsigned)out[i], (uint8_t*)dst + 6 * i);
+            continue;
+          }
           unsigned codes[16];
 #pragma unroll
           for (int g = 0; g < 4; ++g) wholes_of_quads<decltype(careful_tag)::value>(y[0][nt] + 2 * g, y[1][nt] + 2 * g, rinv, hb, codes + 4 * g);
           const u6 c = bf6_of_wholes(codes);
-          v2i* dst = (v2i*)(q + ((size_t)(jp >> 1) * M + row) * kF6BlockBytes + 48 * h + 24 * (jp & 1));
 #pragma unroll
           for (int i = 0; i < 3; ++i) dst[i] = v2i{(int)c[2 * i], (int)c[2 * i + 1]};
         }

@@ -146,13 +146,14 @@ __device__ __forceinline__ float max_across(float m) {
 // code, the 96-byte block of this group at ((row % groups_per_token) * tokens + row / groups_per_token) * 96
 // (K-slab-major, see gemm_f6.hip), a lane's eight as six bytes.  The conversion is the hardware's, a quarter full (18432 groups
 // rotated 4.28 -> 4.03 us against a table and eight-byte stores behind an exchange between lanes).
-template <int G, bool F6 = false, bool OFF32 = false>
-__device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool valid, uint32_t row, uint8_t* __restrict__ q,
-                                             __half* __restrict__ scales, float scale_mul, uint32_t tokens = 0,
-                                             uint32_t groups_per_token = 1) {
+//
+// FINITE (F6): every value in this wave is.  m: the largest one of the lane.
+template <int G, bool F6, bool OFF32, bool FINITE>
+__device__ __forceinline__ void group_finish_from(float m, const h2 (&v)[4], int lir, bool valid, uint32_t row, uint8_t* __restrict__ q,
+                                                  __half* __restrict__ scales, float scale_mul, uint32_t tokens,
+                                                  uint32_t groups_per_token) {
   static_assert(!F6 || G == 128, "one 6-bit block is 128 codes");
   constexpr int LPR = G / 8;
-  float m = lane_abs_max(v);
   m = max_across<kDppQuadXor1>(m);
   m = max_across<kDppQuadXor2>(m);
   if constexpr (LPR >= 8) m = max_across<kDppRowHalfMirror>(m);
@@ -168,7 +169,7 @@ __device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool val
                  y45 = __builtin_bit_cast(unsigned, v[2]), y67 = __builtin_bit_cast(unsigned, v[3]);
   unsigned w = 0;
   u6 six;
-  if constexpr (F6) {
+  if constexpr (F6 && FINITE) {
     unsigned h[16] = {};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -183,7 +184,9 @@ __device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool val
     using offset_t = std::conditional_t<OFF32, uint32_t, size_t>;
     if constexpr (F6) {
       const size_t block = (size_t)(row % groups_per_token) * tokens + row / groups_per_token;
-      f6_store_six<0>(six, q + block * kF6BlockBytes + f6_chunk_at(lir));
+      uint8_t* dst = q + block * kF6BlockBytes + f6_chunk_at(lir);
+      if constexpr (FINITE) f6_store_six<0>(six, dst);
+      else f6_store_nibbles(w, dst);
     } else {
       *(unsigned*)(q + ((offset_t)row * (LPR * 4) + (offset_t)lir * 4)) = w;
     }
@@ -191,6 +194,41 @@ __device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool val
     // second kernel after the unnormalised transform): float32 product, then fp16; the codes above use s
     if (lir == 0) *(__half*)((char*)scales + (offset_t)row * 2) = scale_mul == 1.0f ? __builtin_bit_cast(__half, s) : __float2half(round_here((float)s * scale_mul));
   }
+}
+
+template <int G, bool F6 = false, bool OFF32 = false>
+__device__ __forceinline__ void group_finish(const h2 (&v)[4], int lir, bool valid, uint32_t row, uint8_t* __restrict__ q,
+                                             __half* __restrict__ scales, float scale_mul, uint32_t tokens = 0,
+                                             uint32_t groups_per_token = 1) {
+  if constexpr (F6) {
+    unsigned y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = __builtin_bit_cast(unsigned, v[i]);
+    const float m = abs_max_or_nan(y);
+    if (__builtin_expect(all_finite(m), 1)) {
+      group_finish_from<G, F6, OFF32, true>(m, v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
+      return;
+    }
+  }
+  group_finish_from<G, F6, OFF32, false>(lane_abs_max(v), v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
+}
+
+template <int G, bool OFF32>
+__device__ __forceinline__ void load_chunk(const __half* src, uint32_t row, int lir, h2 (&v)[4]) {
+  using offset_t = std::conditional_t<OFF32, uint32_t, size_t>;
+  const h8 raw = *(const h8*)((const char*)src + ((offset_t)row * (G * 2) + (offset_t)lir * 16));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = h2{raw[2 * i], raw[2 * i + 1]};
+}
+// one group by its G / 8 lanes (every lane of the wave has to call it; rows past the end work on the last one and store nothing)
+template <int G, bool HAD, bool F6, bool OFF32 = false>
+__device__ __forceinline__ void quantise_group(const __half* x, uint8_t* q, __half* scales, uint32_t row, int lir, uint32_t R, float scale_mul,
+                                               uint32_t tokens, uint32_t groups_per_token) {
+  const bool valid = row < R;
+  h2 v[4];
+  load_chunk<G, OFF32>(x, valid ? row : R - 1, lir, v);
+  if constexpr (HAD) fwht_group_f16<G>(v, lir);
+  group_finish<G, F6, OFF32>(v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
 }
 
 // OFF32: every byte offset of the launch fits 32 bits, so that the addresses are a scalar base plus a 32-bit lane
@@ -205,15 +243,11 @@ __global__ __launch_bounds__(256) void group_kernel(const __half* __restrict__ x
   const uint32_t gl = blockIdx.x * 256u + threadIdx.x;
   const uint32_t row = gl / LPR;
   const int lir = group_chunk<LPR>(gl % LPR);         // the chunk of the row this lane owns
-  const bool valid = row < R;
-  const uint32_t rr = valid ? row : R - 1;
-  const __half* src = QUANT ? x : y_inplace;
-  const h8 raw = *(const h8*)((const char*)src + ((offset_t)rr * (G * 2) + (offset_t)lir * 16));
-  h2 v[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = h2{raw[2 * i], raw[2 * i + 1]};
-  if constexpr (HAD) fwht_group_f16<G>(v, lir);
   if constexpr (!QUANT) {
+    const bool valid = row < R;
+    h2 v[4];
+    load_chunk<G, OFF32>(y_inplace, valid ? row : R - 1, lir, v);
+    fwht_group_f16<G>(v, lir);
     h8 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -222,7 +256,7 @@ __global__ __launch_bounds__(256) void group_kernel(const __half* __restrict__ x
     }
     if (valid) *(h8*)((char*)y_inplace + ((offset_t)row * (G * 2) + (offset_t)lir * 16)) = o;
   } else {
-    group_finish<G, F6, OFF32>(v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
+    quantise_group<G, HAD, F6, OFF32>(x, q, scales, row, lir, R, scale_mul, tokens, groups_per_token);
   }
 }
 
@@ -317,11 +351,18 @@ __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restric
       butterfly(v[0][i], v[2][i]), butterfly(v[1][i], v[3][i]);
     }
   }
-  float m = lane_abs_max(v[0]);
+  unsigned y[16];
 #pragma unroll
-  for (int j = 1; j < 4; ++j) {
-    const float mj = lane_abs_max(v[j]);
-    asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m), "v"(mj));
+  for (int i = 0; i < 16; ++i) y[i] = __builtin_bit_cast(unsigned, v[i >> 2][i & 3]);
+  float m = abs_max_or_nan(y);
+  if (__builtin_expect(!all_finite(m), 0)) {
+    // What becomes of NaNs and infinities depends on the operand order of every addition and on which groups share a wave (see
+    // `careful`): the wave's sixteen groups once more, as the sixteen-lane kernel takes them.
+    const int lane = tid & 63;
+    for (int i = 0; i < 16; i += 4)
+      quantise_group<128, HAD, F6>(x, q, scales, row0 + (tid >> 6) * 16 + i + (lane >> 4), group_chunk<16>(lane & 15), R, scale_mul, tokens,
+                                   groups_per_token);
+    return;
   }
   m = max_across<kDppQuadXor1>(m);
   m = max_across<kDppQuadXor2>(m);
@@ -334,7 +375,7 @@ __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restric
     unsigned h[16];
     auto wholes = [&](auto careful_tag) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) h[i] = whole2(quotients2<decltype(careful_tag)::value>(__builtin_bit_cast(unsigned, v[i >> 2][i & 3]), r, hb));
+      for (int i = 0; i < 16; ++i) h[i] = whole2(quotients2<decltype(careful_tag)::value>(y[i], r, hb));
     };
     if (careful) wholes(std::true_type{});
     else wholes(std::false_type{});
@@ -364,8 +405,7 @@ __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restric
   auto codes = [&](auto careful_tag) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      w[j] = nibbles8<decltype(careful_tag)::value>(__builtin_bit_cast(unsigned, v[j][0]), __builtin_bit_cast(unsigned, v[j][1]),
-                                                    __builtin_bit_cast(unsigned, v[j][2]), __builtin_bit_cast(unsigned, v[j][3]), r, hb);
+      w[j] = nibbles8<decltype(careful_tag)::value>(y[4 * j], y[4 * j + 1], y[4 * j + 2], y[4 * j + 3], r, hb);
   };
   if (careful) codes(std::true_type{});
   else codes(std::false_type{});

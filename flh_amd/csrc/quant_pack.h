@@ -79,6 +79,17 @@ __device__ __forceinline__ unsigned nibbles8(unsigned y01, unsigned y23, unsigne
     t[u] = quad_nibbles(quotients2<CAREFUL>(u == 0 ? y01 : y45, rinv, hb), quotients2<CAREFUL>(u == 0 ? y23 : y67, rinv, hb));
   return ((t[1] << 16) + t[0] - kPairBias) ^ 0x88888888u;
 }
+// The largest |half| of N packed registers by the order of the bit patterns, in which a NaN is the largest: below infinity only if
+// every value is finite (fmaxf and v_pk_max_f16 pass NaNs over).
+template <int N>
+__device__ __forceinline__ float abs_max_or_nan(const unsigned (&y)[N]) {
+  us2 m = __builtin_bit_cast(us2, y[0] & 0x7FFF7FFFu);
+#pragma unroll
+  for (int i = 1; i < N; ++i) m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, y[i] & 0x7FFF7FFFu));
+  return (float)__builtin_bit_cast(_Float16, m.x > m.y ? m.x : m.y);
+}
+// whether the lanes of a wave hold nothing but finite values, of which each gives its abs_max_or_nan
+__device__ __forceinline__ bool all_finite(float m) { return __builtin_amdgcn_ballot_w64(!(m < INFINITY)) == 0; }
 // rint of two fp16 quotients, as fp16 (zeros are +0): for the hardware's conversion to the 6-bit format
 __device__ __forceinline__ unsigned whole2(unsigned h) {
   const h2 magic = {(_Float16)1544.0f, (_Float16)1544.0f};

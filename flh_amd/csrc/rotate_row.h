@@ -161,6 +161,7 @@ __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_ro
 
   unsigned yp[N / 2];                                  // the rotated row as packed fp16 pairs
   float mx = 0.f;                                      // row maximum of |y|, exactly representable in fp16
+  bool finite = true;                                  // (F6) every y is; a row of zeros counts as one that is not
   if constexpr (HAD) {
     float v[N];
     // stride 1 straight from the packed halves: lo + hi and lo - hi are exact float32 sums of fp16 values
@@ -222,14 +223,23 @@ __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_ro
 #pragma unroll
     for (int j = 0; j < J; ++j)
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const unsigned w = (unsigned)raw[j][d];        // (a bit_cast of the vector element itself miscompiles)
-        yp[j * 4 + d] = w;
-        const h2 t = __builtin_bit_cast(h2, w);
+      for (int d = 0; d < 4; ++d) yp[j * 4 + d] = (unsigned)raw[j][d];   // (a bit_cast of the vector element itself miscompiles)
+    if constexpr (F6) {
+      mx = abs_max_or_nan(yp);
+      finite = all_finite(mx);
+    }
+    if (!F6 || !finite) {
+      mx = 0.f;
+#pragma unroll
+      for (int i = 0; i < N / 2; ++i) {
+        const h2 t = __builtin_bit_cast(h2, yp[i]);
         mx = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf((float)t[0]), __builtin_fabsf((float)t[1])), mx);
       }
+    }
   }
   mx = wave_max(mx);
+  // an infinity or a NaN reaches every sum of a rotation: then the maximum is infinite, or zero where all values are NaN
+  if constexpr (F6 && HAD) finite = __builtin_amdgcn_readfirstlane(mx > 0.f && mx < INFINITY);
   if (y_row) {
     // zeros leave the sign-carrying lanes as -0; adding +0 turns them into the +0 the plain butterfly
     // gives (x + 0 = x for every other value).  Codes and scales do not depend on the sign of zero.
@@ -255,6 +265,12 @@ __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_ro
     if constexpr (F6) {                                // chunk c of segment j sits in 128-code block 4 j + c / 16
       uint8_t* dst = q_row + ((size_t)(c >> 4) * f6_rows + f6_row) * kF6BlockBytes + f6_chunk_at(c & 15);
       const size_t step = (size_t)4 * f6_rows * kF6BlockBytes;
+      if (!CAREFUL && __builtin_expect(!finite, 0)) {                       // (clamped quotients are never NaN)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          f6_store_nibbles(nibbles8<false>(yp[4 * j], yp[4 * j + 1], yp[4 * j + 2], yp[4 * j + 3], r, hb), dst + j * step);
+        return;
+      }
       static_for<(J + 3) / 4>([&](auto u_tag) {
         constexpr int u = decltype(u_tag)::value;
         unsigned h[16];
