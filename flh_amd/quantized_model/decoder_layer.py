@@ -530,11 +530,17 @@ class W4A4DecoderLayer(torch.nn.Module):
     def _swiglu_gemm_applies(self, rows):
         """Whether gate and up take the launch that stores silu(gate) * up only: prefill sizes.  Group configuration, us per layer,
         two outputs -> the product: 4096 tokens 1050 -> 1030, 1000 326 -> 322, 100 102 -> 101, 33 79 -> 84; with one scale per weight
-        row 2048 tokens 679 -> 668, 129 .. 1000 equal, 100 143 -> 150."""
+        row 2048 tokens 679 -> 668, 129 .. 1000 equal, 100 143 -> 150.  A launch that does not fill the chip has smaller tiles for two
+        outputs (64 x 32) than for the product (64 x 64): the product from 448 of the latter on, 288 where K is short (us per
+        MLP, hidden x intermediate, rows, tiles): 2048 x 5632 65 (352) 28.4 / 30.2, 4096 x 5632 128 (352) 43.1 / 46.2, 2048 x 6144 65 (384)
+        29.6 / 31.3, 4096 x 7168 65 (448) 49.2 / 47.9, 2048 x 8192 65 (512) 34.6 / 33.3;  1024 x 4096 65 (256) 18.8 / 20.0, 1024 x 2816 160
+        (264) 19.8 / 20.0, 768 x 3072 160 (288) 19.7 / 19.3, 1024 x 3584 160 (336) 21.8 / 21.3."""
         g = self.gate_proj
         cols = g.w_scale.numel() // g.out_features
-        if self.activation == "group" and (self.act_group_size != 128 or (cols == 1 and rows <= 1024)):
-            return False
+        if self.activation == "group":
+            tiles = -(-rows // 64) * -(-2 * g.out_features // 64)
+            if self.act_group_size != 128 or (cols == 1 and rows <= 1024) or tiles < (288 if g.in_features <= 1024 else 448):
+                return False
         return rows > 64 and g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
 
     def _group_quant(self, stage, quantizer, x, consumers=()):

@@ -207,5 +207,8 @@ def test_group_layer_with_the_product_in_the_gemm_gives_the_same_bits(monkeypatc
             m.setattr(W4A4DecoderLayer, "_swiglu_gemm_applies", lambda self, rows: False)
             want, want_pending = layer._mlp(x, None)
             want_alone = layer.mlp(x)
+            m.setattr(W4A4DecoderLayer, "_swiglu_gemm_applies", lambda self, rows: True)    # (also where the rule says no)
+            forced = layer._mlp(x, None)
         assert (pending is None) == (want_pending is None) and torch.equal(got, want) and torch.equal(alone, want_alone)
         assert pending is None or torch.equal(pending, want_pending)
+        assert torch.equal(forced[0], want) and (pending is None or torch.equal(forced[1], want_pending))
