@@ -75,24 +75,25 @@ __device__ __forceinline__ _Float16 silu_mul_f16(_Float16 gate, _Float16 up) {
 
 // 16 bytes per lane from global memory straight into LDS: lane i of the wave writes
 // lds_base + 16 * i (lds_base wave-uniform).  Counted by vmcnt; the compiler does not know
-// about it, so every wait for these loads is written out by hand below.
+// about it, so every wait for these loads is written out by hand below -- the wait state between a scalar write of M0 and
+// a load that reads it included (s_nop 0).
 __device__ __forceinline__ void load_to_lds16(const void* gptr, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
 
 // the same for data that is read once (non-temporal: it does not displace what the caches hold)
 __device__ __forceinline__ void load_to_lds16_nt(const void* gptr, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
 
 // 4 bytes per lane: lane i writes lds_base + 4 * i
 __device__ __forceinline__ void load_to_lds4(const void* gptr, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
 
 // load_to_lds16 with a wave-uniform base address in scalar registers plus a 32-bit per-lane offset
 __device__ __forceinline__ void load_to_lds16(const void* sbase, unsigned voffset, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(sbase) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(sbase) : "memory", "m0");
 }
 
 // a pointer that is the same in every lane, as scalar registers

@@ -70,7 +70,7 @@ __device__ __forceinline__ Tile tile_of(const GemmArgs& p, unsigned L) {
 // ---- operand loads through buffer descriptors
 // 3 KiB in three instructions: lane i's 16 bytes at voff, + 1024, + 2048 go to lds_base + 16 i, + 1024, + 2048
 __device__ __forceinline__ void load_block_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\t"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen offset:1024 lds\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen offset:2048 lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
@@ -78,12 +78,12 @@ __device__ __forceinline__ void load_block_to_lds(const v4i& d, unsigned voff, u
 
 // ... the first 2 KiB of it, and the third
 __device__ __forceinline__ void load_two_thirds_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\t"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen offset:1024 lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
 }
 __device__ __forceinline__ void load_last_third_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\t"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen offset:2048 lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
 }
 

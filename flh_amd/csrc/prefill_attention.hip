@@ -56,11 +56,11 @@ __device__ __forceinline__ int v_chunk_at(int r, int c) { return r * (kHeadDim *
 
 // 1 KiB: lane i's 16 bytes at voff go to lds_base + 16 i
 __device__ __forceinline__ void load_rows_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(voff), "s"(d) : "memory", "m0");
 }
 // the same four times, 1 KiB further in memory and in LDS each
 __device__ __forceinline__ void load_four_rows_to_lds(const v4i& d, unsigned voff, unsigned lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\t"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen offset:1024 lds\n\t"
                "buffer_load_dwordx4 %1, %2, 0 offen offset:2048 lds\n\t"
