@@ -16,8 +16,22 @@ def dev(a):
 
 @pytest.mark.parametrize("k", [512, 640, 768, 896, 1408, 2688])
 @pytest.mark.parametrize("m,ns", [(1, (12416,)), (16, (12544, 72)), (17, (8,)), (17, (136, 40)), (32, (1000, 24)), (33, (264,)), (63, (8200,)),
-                                  (64, (4096, 1024, 1024)), (65, (4104,)), (130, (4096,)), (300, (136,)), (1280, (72,))])
+                                  (64, (4096, 1024, 1024)), (65, (4104,)), (130, (4096,)), (300, (136,)), (1280, (72,)), (64, (14336,)),
+                                  (97, (8200, 24))])
 def test_against_the_square_tiles(gemm_tuning, m, ns, k):
+    """(The last two: more than 768 blocks of 32 x 32, which take the tile of 64 tokens.)"""
+    against_the_square_tiles(gemm_tuning, m, ns, k)
+
+
+@pytest.mark.parametrize("m,ns,k", [(64, (8192,), 8320), (33, (8160, 8), 8448), (100, (4064,), 8576)])
+def test_long_rows(gemm_tuning, m, ns, k):
+    """K beyond 8192 with 257 .. 512 blocks of 32 x 32 and at most 256 of 64 x 32: the tile of 64 tokens again."""
+    columns = -(-sum(ns) // 32)
+    assert 256 < -(-m // 32) * columns <= 512 and -(-m // 64) * columns <= 256
+    against_the_square_tiles(gemm_tuning, m, ns, k)
+
+
+def against_the_square_tiles(gemm_tuning, m, ns, k):
     from flh_amd import _ops as ops
     rng = np.random.default_rng(m + k)
     a, sa = dev(rng.integers(0, 256, size=(m, k // 2), dtype=np.uint8)), dev(syn.weight_scales(m, 1, m))

@@ -59,17 +59,35 @@ def test_largest_sums(gemm_tuning, token):
 
 
 @pytest.mark.parametrize("kind", ["token", "group"])
-@pytest.mark.parametrize("m,n", [(65, 9088), (65, 9216), (640, 3456), (640, 3584), (257, 10920), (257, 11008)])
-def test_around_the_lines(m, n, kind):
-    """144 tiles, 256 tiles, 65 rows: the automatic choice on either side."""
+@pytest.mark.parametrize("m,columns,tiles", [(640, 3584, 140), (1152, 2048, 144), (256, 16384, 256), (256, 16512, 258), (64, 18432, 144),
+                                             (65, 18432, 144)])
+def test_around_the_lines(m, columns, tiles, kind):
+    """The automatic choice on either side of every line: from 144 tiles of 128 x 128 on, with token scales up to 256, plain
+    launches from 65 rows on -- the product of gate and up, and q / k / v, whatever the rows."""
     from flh_amd import _ops as ops
     k = 1024
-    rng = np.random.default_rng(m + n)
-    a, w = (dev(rng.integers(0, 256, size=(r, k // 2), dtype=np.uint8)) for r in (m, n))
-    sa, sw = dev(syn.weight_scales(m, 1 if kind == "token" else 8, m)), dev(syn.weight_scales(n, 8, n))
-    got = ops.gemm_i4_dequant(a, w, sa, sw, 128)
+    assert -(-m // 128) * -(-columns // 128) == tiles
+    rng = np.random.default_rng(m + columns)
+
+    def weights(n):
+        return dev(rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)), dev(syn.weight_scales(n, 8, n))
+    a, sa = dev(rng.integers(0, 256, size=(m, k // 2), dtype=np.uint8)), dev(syn.weight_scales(m, 1 if kind == "token" else 8, m))
+    w, sw = weights(columns)
+    (gate, sg), (up, su) = weights(columns // 2), weights(columns // 2)
+    kv = columns // 128 // 4
+    wr, sr = zip(*[weights(n * 128) for n in (columns // 128 - 2 * kv, kv, kv)])
+    cos, sin = (dev(rng.uniform(-1, 1, (m, 128)).astype(np.float16)) for _ in range(2))
+    pos = torch.arange(m, device="cuda")
+
+    def run():
+        caches = [torch.zeros(1, kv, m, 128, dtype=torch.float16, device="cuda") for _ in range(2)]
+        return [ops.gemm_i4_dequant(a, w, sa, sw, 128), ops.gemm_i4_swiglu(a, gate, up, sa, sg, su, 128),
+                ops.gemm_i4_qkv_rope(a, sa, list(wr), list(sr), cos, sin, pos, *caches, 1, 128), *caches]
+    got = run()
     ops.gemm_set_tuning(128, 1)
     try:
-        assert torch.equal(got, ops.gemm_i4_dequant(a, w, sa, sw, 128))
+        want = run()
     finally:
         ops.gemm_set_tuning(0, 0)
+    for i, (x, y) in enumerate(zip(got, want)):
+        assert torch.equal(x, y), i

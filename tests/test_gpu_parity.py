@@ -27,8 +27,9 @@ def host(t):
 # ------------------------------------------------------------------ GEMM
 GEMM_SHAPES = [(1, 128, 128), (16, 256, 512), (33, 100, 384), (256, 128, 128), (300, 520, 1024),
                (257, 129, 256), (16, 4096, 4096), (64, 1024, 11008),
-               # decode kernel: 1 / 2 / 4 token tiles, odd number of 128-code steps, ragged N
-               (5, 17, 640), (17, 4096, 4096), (48, 200, 1152),
+               # decode kernel: 1 / 2 / 4 token tiles, odd number of 128-code steps, ragged N (from K = 512 on, 17 and more rows with
+               # one scale per row are the dealt kernel's: two and four tiles with short K as well)
+               (5, 17, 640), (17, 4096, 4096), (48, 200, 1152), (17, 100, 384), (32, 72, 128),
                # prefill kernel, every tile shape: 64 x 64, 128 x 128, 256 x 128
                (65, 64, 256), (700, 4200, 512), (1024, 4096, 256), (2048, 4096, 256),
                # ... and the in-workgroup K split: two quads on 256 x 128 and 128 x 128, four on 64 x 64

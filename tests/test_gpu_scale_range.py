@@ -27,6 +27,7 @@ def dev(a):
 KERNELS = {"decode": (5, 40, 1280, (0, 0), False), "stream_16": (16, 11016, 512, (0, 0), False), "stream": (40, 100, 1280, (0, 0), False),
            "stream_64": (64, 14336, 512, (0, 0), False), "tile_64": (100, 72, 1280, (64, 0), False), "tile_128": (130, 136, 1280, (128, 0), False),
            "tile_256": (260, 136, 1280, (256, 0), False), "f6_64": (70, 72, 1280, (64, 0), True), "f6_128": (130, 136, 1280, (128, 0), True),
+           "square": (130, 136, 1792, (128, 2), False), "f6_square": (130, 136, 1792, (128, 2), True),
            "f6_narrow": (260, 136, 1792, (256, 2), True), "f6_wide": (260, 264, 1792, (256, 1), True)}
 
 
