@@ -925,12 +925,12 @@ int launch_group(const __half* x, uint8_t* q, __half* s, __half* y, uint32_t R, 
   const dim3 grid((unsigned)(((uint64_t)R * LPR + 255) / 256)), block(256);
   auto go = [&](auto off32_tag) {
     constexpr bool OFF32 = decltype(off32_tag)::value;
-    if (!quant)
+    if (!quant) {
       hipLaunchKernelGGL((group_kernel<G, true, false, false, OFF32>), grid, block, 0, stream, x, q, s, y, R, scale_mul, 0u, 1u);
-    else if (had)
-      hipLaunchKernelGGL((group_kernel<G, true, true, false, OFF32>), grid, block, 0, stream, x, q, s, y, R, scale_mul, 0u, 1u);
-    else
-      hipLaunchKernelGGL((group_kernel<G, false, true, false, OFF32>), grid, block, 0, stream, x, q, s, y, R, scale_mul, 0u, 1u);
+    } else if constexpr (G != 128 || OFF32) {           // (longer batches of 128 are the four-lane kernel's)
+      if (had) hipLaunchKernelGGL((group_kernel<G, true, true, false, OFF32>), grid, block, 0, stream, x, q, s, y, R, scale_mul, 0u, 1u);
+      else hipLaunchKernelGGL((group_kernel<G, false, true, false, OFF32>), grid, block, 0, stream, x, q, s, y, R, scale_mul, 0u, 1u);
+    }
   };
   if ((uint64_t)R * G * 2 <= 0xFFFFFFFFull) go(std::true_type{});   // the largest array of the launch: the fp16 rows
   else go(std::false_type{});
