@@ -38,8 +38,8 @@ __device__ __forceinline__ _Float16 rope_value(_Float16 x, _Float16 xp, _Float16
 // attention does not read: the first workgroup of every (sequence, key / value head) writes it there, as the
 // stand-alone kernel would.
 //
-// Values pass the caches by (16 x 32 / 8 heads x 4096 61 -> 59 us).  AHEAD: keys as well, and both are requested before anything else (rule:
-// launch_attention).
+// Values pass the caches by (16 x 32 / 8 heads x 4096 64.2 -> 62.6 us, 12 x 32 / 8 x 2048 31.3 -> 30.5).  AHEAD: keys as well, and both
+// are requested before anything else (rule: launch_attention).
 template <int D, int REP, int CHUNK, bool ROPE, bool AHEAD>
 __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
     const __half* __restrict__ q, __half* k_cache, __half* v_cache, float* __restrict__ partials, uint32_t Hkv,
@@ -56,11 +56,14 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
   __shared__ float red[kAttnThreads / 64][REP * D];    // the waves' weighted values
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // One or two queries per key: the chunks of one place in all the caches next to each other, whose strides are often a power of two; more
-  // (more work per chunk, fewer caches): the chunks of a cache.  us, chunks of a cache -> of one place: 8 x 32 / 32 x 2048 52.5 -> 46.1, 16 x 32 / 32 x
-  // 2048 101 -> 91, 8 x 32 / 32 x 1024 29.4 -> 26.2, 12 x 32 / 16 x 1024 25.8 -> 24.6, 5 x 32 / 32 x 777 16.8 -> 16.8;  4 x 32 / 8 x 2048 14.7 -> 17.2
+  // One or two queries per key: the chunks of one place in all the caches next to each other, whose strides are often a power
+  // of two; more (more work per chunk, fewer caches): the chunks of a cache.  us, chunks of a cache -> of one place: 8 x 32 /
+  // 32 x 2048 52.5 -> 46.1, 16 x 32 / 32 x 2048 101 -> 91, 8 x 32 / 32 x 1024 29.4 -> 26.2, 5 x 32 / 32 x 777 16.8 -> 16.8;
+  // two queries per key go either way: 12 x 32 / 16 x 1024 27.6 -> 26.7, 8 x 32 / 16 x 2048 33.9 -> 32.9, 4 x 32 / 16 x 2048
+  // 21.7 -> 22.3, 2 x 32 / 16 x 2048 14.4 -> 16.1;  four: 4 x 32 / 8 x 2048 14.7 -> 17.2
   const uint32_t caches = gridDim.x / splits;
-  const uint32_t split = REP <= 2 ? blockIdx.x / caches : blockIdx.x % splits, bh = REP <= 2 ? blockIdx.x % caches : blockIdx.x / splits;   // bh = b * Hkv + kvh
+  const uint32_t split = REP <= 2 ? blockIdx.x / caches : blockIdx.x % splits;
+  const uint32_t bh = REP <= 2 ? blockIdx.x % caches : blockIdx.x / splits;   // b * Hkv + kvh
   const uint32_t t0 = split * CHUNK;
   const uint32_t n_live = kv_len > t0 ? min((uint32_t)CHUNK, kv_len - t0) : 0u;
   const uint32_t last = n_live ? n_live - 1 : 0;       // rows past the live range read the last live one again (any valid address)
@@ -276,11 +279,13 @@ int launch_attention(const __half* q, __half* k, __half* v, __half* out, float* 
     hipLaunchKernelGGL(kern, grid, block, 0, stream, q, k, v, partials, Hkv, kv_len, max_len, splits, scale, nt.k, nt.v, nt.cos, nt.sin,
                        nt.positions);
   };
-  // Requested ahead, and past the caches, everywhere but for grouped queries on more chunks than two rounds of the chip hold, and eight queries per key.  us, with
-  // the combine launch, otherwise -> ahead, sequences x heads / key-value heads x positions: 5 x 32 / 32 x 777 18.6 -> 16.9, 1 x 32 / 8 x 2048
-  // 10.7 -> 10.3, 8 x 32 / 8 x 1024 15.1 -> 13.9, 10 x 32 / 8 x 2048 26.7 -> 25.0, 14 x 32 / 8 x 2048 (3584 chunks) 32.6 -> 31.7, 16 x 32 / 32 x 777
-  // 42.6 -> 39.0;  16 x 32 / 8 x 2048 (4096) 35.2 -> 37.3, 16 x 32 / 8 x 4096 59 -> 65, 8 x 32 / 4 x 3000 21.9 -> 23.3
-  const bool ahead = REP == 1 || (REP <= 4 && (uint64_t)B * Hkv * splits <= 3584);
+  // Keys and values requested ahead: always with one query per key, and with up to four on at most two chunks per compute unit.
+  // us with the combine launch, replayed over caches that together don't fit the last-level one, otherwise -> ahead, sequences x
+  // heads / key-value heads x positions (chunks): 5 x 32 / 32 x 777 18.8 -> 17.5, 16 x 32 / 32 x 777 45.1 -> 42.3, 8 x 32 / 32 x 2048
+  // 55.0 -> 49.9;  1 x 32 / 8 x 2048 (256) 10.7 -> 10.3, 4 x 32 / 8 x 1024 (512) 11.4 -> 11.1, 14 x 32 / 8 x 300 (560) 11.5 -> 11.9,
+  // 8 x 32 / 8 x 777 (832) 13.0 -> 13.5, 16 x 32 / 8 x 777 (1664) 17.8 -> 19.2, 14 x 32 / 8 x 2048 (3584) 33.3 -> 33.8, 8 x 32 / 4 x 3000
+  // 21.6 -> 24.0.  In a decode step there is less in it: one query per key, 5 x 777, 14.7 -> 14.4 for the kernel.
+  const bool ahead = REP == 1 || (REP <= 4 && (uint64_t)B * Hkv * splits <= 512);
   if (nt.k) ahead ? go(decode_attention_partial_kernel<D, REP, kChunk, true, true>) : go(decode_attention_partial_kernel<D, REP, kChunk, true, false>);
   else ahead ? go(decode_attention_partial_kernel<D, REP, kChunk, false, true>) : go(decode_attention_partial_kernel<D, REP, kChunk, false, false>);
   if (int rc = check_launch("decode_attention (partials)")) return rc;

@@ -121,7 +121,7 @@ def test_rotary_decode_attention_argument_errors():
         _ops.decode_attention_rope(q, kn, kn, cs, cs, pos, k, k.clone(), 17)
 
 
-@pytest.mark.parametrize("b,hq,hkv,n", [(7, 8, 8, 65), (2, 8, 2, 200), (57, 32, 8, 449), (3, 16, 2, 130)])
+@pytest.mark.parametrize("b,hq,hkv,n", [(7, 8, 8, 65), (2, 8, 2, 200), (8, 32, 8, 512), (8, 32, 8, 513), (57, 32, 8, 449), (3, 16, 2, 130)])
 def test_new_token_in_any_wave_and_chunk(b, hq, hkv, n):
     """The rotary form, whose keys and values are requested before the slot is known: the new token in every wave of a chunk, and in
     the first and the last chunk, against the cache write as its own launch, on either side of the rule for early requests."""
