@@ -73,7 +73,8 @@ def add_rmsnorm_rotate_and_quantize_i4(x, add, weight, eps, hadamard=True, clip_
 
 
 def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None):
-    return tuple(_ext.rotate_and_quantize_f6_mode(x, _ops._f6_mode(x, hadamard, eps, add) if x.dim() == 2 else 0, clip_ratio, norm_weight, eps, add))
+    mode = _ops._f6_mode(x, hadamard, eps, add) if x.dim() == 2 else 0
+    return tuple(_ext.rotate_and_quantize_f6_mode(x, mode, clip_ratio, norm_weight, eps, add))
 
 
 def __getattr__(name):        # ops the extension does not wrap (one matrix's encoding, int32 output, tuning hook, ...)

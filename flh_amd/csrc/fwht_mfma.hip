@@ -285,7 +285,8 @@ __global__ __launch_bounds__(256, 2) void rotate_quant_mfma4096_kernel(const __h
           }
           unsigned codes[16];
 #pragma unroll
-          for (int g = 0; g < 4; ++g) wholes_of_quads<decltype(careful_tag)::value>(y[0][nt] + 2 * g, y[1][nt] + 2 * g, rinv, hb, codes + 4 * g);
+          for (int g = 0; g < 4; ++g)
+            wholes_of_quads<decltype(careful_tag)::value>(y[0][nt] + 2 * g, y[1][nt] + 2 * g, rinv, hb, codes + 4 * g);
           const u6 c = bf6_of_wholes(codes);
 #pragma unroll
           for (int i = 0; i < 3; ++i) dst[i] = v2i{(int)c[2 * i], (int)c[2 * i + 1]};
@@ -716,7 +717,8 @@ int launch_dense(const __half* x, uint8_t* q, __half* scales, uint32_t M, float 
   // 10.9 / 7.9, 512 11.3 / 8.2, 768 11.8 / 10.7, 800 11.8 / 13.0; 14336 300 12.7 / 8.6, 512 13.1 / 9.0, 768 13.7 / 12.2, 800 13.7 / 14.8.
   // 6-bit output (a prefill format) always takes the long-batch kernel
   const bool split = M <= 768 && !f6;
-  const size_t smem = (size_t)NFRAG * 1024 + 64 + (split ? 2 * (size_t)DT * 4096 : 0);   // factor fragments, the pairs' maxima, the row and its first level
+  // factor fragments, the pairs' maxima, the row and its first level
+  const size_t smem = (size_t)NFRAG * 1024 + 64 + (split ? 2 * (size_t)DT * 4096 : 0);
   auto kern = f6 ? rotate_quant_mfma_dense_kernel<DT, false, false, true>
                  : split ? rotate_quant_mfma_dense_kernel<DT, true> : rotate_quant_mfma_dense_kernel<DT, false>;
   constexpr int kThreadsDense = 512;

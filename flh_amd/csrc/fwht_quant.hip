@@ -222,8 +222,8 @@ __device__ __forceinline__ void load_chunk(const __half* src, uint32_t row, int 
 }
 // one group by its G / 8 lanes (every lane of the wave has to call it; rows past the end work on the last one and store nothing)
 template <int G, bool HAD, bool F6, bool OFF32 = false>
-__device__ __forceinline__ void quantise_group(const __half* x, uint8_t* q, __half* scales, uint32_t row, int lir, uint32_t R, float scale_mul,
-                                               uint32_t tokens, uint32_t groups_per_token) {
+__device__ __forceinline__ void quantise_group(const __half* x, uint8_t* q, __half* scales, uint32_t row, int lir, uint32_t R,
+                                               float scale_mul, uint32_t tokens, uint32_t groups_per_token) {
   const bool valid = row < R;
   h2 v[4];
   load_chunk<G, OFF32>(x, valid ? row : R - 1, lir, v);
@@ -287,16 +287,17 @@ __global__ __launch_bounds__(256) void silu_mul_group_kernel(const __half* __res
   group_finish<G, F6>(v, lir, valid, row, q, scales, scale_mul, tokens, groups_per_token);
 }
 
-// The group kernels for groups of 128 and launches that fill the chip: FOUR lanes own a group, 32 values each (lane p
-// the chunks p, p + 4, p + 8, p + 12), so that of the seven butterfly strides only 8 and 16 cross lanes, and the row's maximum,
+// The group kernels for groups of 128 and launches that fill the chip: FOUR lanes own a group, 32 values each (lane p the
+// chunks p, p + 4, p + 8, p + 12), so that of the seven butterfly strides only 8 and 16 cross lanes, and the row's maximum,
 // scale and reciprocal are computed by four lanes instead of sixteen.  A lane's four code words are turned inside its wave
-// through LDS, so that it stores sixteen consecutive bytes (32 codes; 6-bit output: the whole numbers are, and a lane converts and
-// stores one 24-byte piece).  Same
-// operations in the same order as group_kernel, the same bytes.
-// What bounds it: memory (4096-wide rows rotated and quantised, us, sixteen lanes -> four, inputs from HBM: 16384 rows 40.3 -> 29.5
-// = 5.7 TB/s, 8192 20.4 -> 15.9, 4096 10.1 -> 9.4; 6-bit output 524288 groups 51 -> 39, 65536 9.1 -> 6.9; a table in the conversion's place 46 and 7.8, six-byte stores without the turn through LDS 56), where the sixteen-lane form
-// is bound by its 165 instructions per eight values, 80 here.  Non-temporal loads and stores: equal or slower (30.6, 31.3).  The
-// SwiGLU product in front of it: 55.6 against 51.4 us, its exponentials want the sixteen lanes' parallelism; not here.
+// through LDS, so that it stores sixteen consecutive bytes (32 codes; 6-bit output: the whole numbers are, and a lane converts
+// and stores one 24-byte piece).  Same operations in the same order as group_kernel, the same bytes.
+// What bounds it: memory.  4096-wide rows rotated and quantised, us, sixteen lanes -> four, replayed over inputs that together
+// don't fit the last-level cache: 16384 rows 34.9 -> 31.8 (5.3 TB/s read + write), 8192 19.2 -> 17.1, 4096 11.2 -> 10.0; 6-bit output
+// 524288 groups 52 -> 41, 65536 9.2 -> 7.2 (of which a table in the conversion's place takes 7 and 0.9, six-byte stores without the
+// turn through LDS 17).  The sixteen-lane form is bound by its 165 instructions per eight values, 80 here.  Non-temporal loads and
+// stores: equal or slower.  The SwiGLU product in front of it: 55.6 against 51.4 us, its exponentials want the sixteen lanes'
+// parallelism; not here.
 constexpr uint32_t kQuadRows = 64;                    // groups per workgroup of four waves
 template <int CTRL>
 __device__ __forceinline__ void quad_cross(h2 (&v)[4][4], _Float16 sg) {
@@ -902,10 +903,11 @@ int launch_wave_rms(const __half* x, const __half* w, float eps, uint8_t* q, __h
   return check_launch("rmsnorm_rotate_quant_wave");
 }
 
-// Groups of 128 from which four lanes per group are the faster form: below, a quarter of the wavefronts does not fill the
-// chip, least of all just beyond a full round of it (us, inputs from HBM, sixteen lanes / four: rotated 18490 groups 3.40 / 3.82, 32768 4.10 /
-// 4.28, 49152 5.70 / 5.73 and 4.35 / 3.96 from the caches, 65536 6.65 / 6.51; not rotated 49152 5.15 / 5.15, 65536 6.21 / 5.66; 6-bit output, rotated
-// and not, 16384 3.83 / 3.41 and 3.42 / 3.14, 18432 4.07 / 4.03 and 3.62 / 3.53, 24576 4.55 / 4.27 and 4.00 / 3.75).
+// Groups of 128 from which four lanes per group are the faster form: below, a quarter of the wavefronts does not fill the chip,
+// least of all just beyond a full round of it (us, inputs from HBM, sixteen lanes / four: rotated 18490 groups 3.40 / 3.82,
+// 32768 4.10 / 4.28, 49152 5.70 / 5.73 and 4.35 / 3.96 from the caches, 65536 6.65 / 6.51; not rotated 49152 5.15 / 5.15, 65536
+// 6.21 / 5.66; 6-bit output, rotated and not, 16384 3.83 / 3.41 and 3.42 / 3.14, 18432 4.07 / 4.03 and 3.62 / 3.53, 24576 4.55
+// / 4.27 and 4.00 / 3.75).
 constexpr uint32_t quad_min_rows(bool had, bool f6) { return f6 ? 16384 : had ? 49152 : 65536; }
 template <bool HAD, bool F6>
 int launch_group_quad(const __half* x, uint8_t* q, __half* s, uint32_t R, float scale_mul, uint32_t tokens,

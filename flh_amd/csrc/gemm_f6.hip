@@ -22,10 +22,11 @@
 // number m that sits in wave half h takes one piece as its operand, and the 48 bytes of a wave half are three
 // 16-byte chunks.
 //
-// Tiling (launches that fill the chip with larger tiles take the kernels of gemm_f6_large.h): workgroup = 4 waves (2 x 2), wave tile of 32 x 32 MFMA tiles, K advances by 128 codes
-// (96 bytes per row) per stage, stages form a ring in LDS filled by direct-to-LDS loads.  Chunk c of tile row r
-// sits in slot 6 r + (c ^ ((r >> 3) & 1)): sixteen consecutive rows read at one logical chunk touch sixteen
-// different groups of four banks.  Fragment reads run half a stage ahead of the MFMAs that use them.
+// Tiling (launches that fill the chip with larger tiles take the kernels of gemm_f6_large.h): workgroup = 4 waves (2 x 2), wave
+// tile of 32 x 32 MFMA tiles, K advances by 128 codes (96 bytes per row) per stage, stages form a ring in LDS filled by
+// direct-to-LDS loads.  Chunk c of tile row r sits in slot 6 r + (c ^ ((r >> 3) & 1)): sixteen consecutive rows read at one
+// logical chunk touch sixteen different groups of four banks.  Fragment reads run half a stage ahead of the MFMAs that use
+// them.
 #include <atomic>
 
 #include <type_traits>
@@ -769,7 +770,7 @@ int launch_f6_by_shape(const GemmArgs& a, hipStream_t stream) {
 // 28672 x 4096 codes: 26.5 us (5.5 TB/s), 36.5 with 48-byte stores straight from the lanes; 4096 x 4096: 6.4 against 7.1.
 // The matrices of one GEMM launch share one launch here as well.
 constexpr int kEncodeRows = 32, kEncodeBlocks = 4;
-struct EncodeArgs {                                    // up to four matrices of one K: 32-row blocks [block0[i], block0[i + 1]) of the launch
+struct EncodeArgs {   // up to four matrices of one K: 32-row blocks [block0[i], block0[i + 1]) of the launch
   const uint8_t* src[kMaxGemmSegments];
   uint8_t* dst[kMaxGemmSegments];
   size_t rows[kMaxGemmSegments];

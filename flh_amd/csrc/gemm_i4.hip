@@ -755,9 +755,11 @@ int launch_grouped(const GemmArgs& a, int group, bool small, hipStream_t stream)
 
 // Launches over `columns` weight rows that take the eight-wave tiles of gemm_i4_square.hip: from 144 tiles of 128 x 128 on, with token
 // scales up to one per compute unit.  us, present tiles (here or in gemm_i4_stream.hip) / those, K = 4096 unless stated:
-//   token scales  512 x 4096 (128 tiles) 21 / 25, 640 x 4096 (160) 28 / 26, 800 x 4096 (224) 32 / 27, 250 x 11008 (172) 27 / 26, 250 x 14336 (224)
+//   token scales  512 x 4096 (128 tiles) 21 / 25, 640 x 4096 (160) 28 / 26, 800 x 4096 (224) 32 / 27, 250 x 11008 (172) 27 / 26,
+//                 250 x 14336 (224)
 //                 32 / 27, 400 x 11008 (344) 45 / 47, 1280 x 4096 (320) 45 / 47;  800 x 4096 of K = 11008 75 / 61
-//   group scales  512 x 4096 25 / 27, 640 x 4096 31 / 27, 250 x 14336 38 / 28, 400 x 11008 54 / 48, 1280 x 4096 53 / 50, 1000 x 14336 98 / 93;
+//   group scales  512 x 4096 25 / 27, 640 x 4096 31 / 27, 250 x 14336 38 / 28, 400 x 11008 54 / 48, 1280 x 4096 53 / 50, 1000 x
+//                 14336 98 / 93;
 //                 640 x 4096 of K = 11008 74 / 62
 //   with SwiGLU   1 .. 128 x 22016 (172) 34 / 28 and 39 / 28, 320 x 22016 (516) 70 / 71 and 82 / 74
 bool takes_square(const GemmArgs& a, long columns) {

@@ -8,11 +8,12 @@
 // the integer sums, exact, and so are the float32 results (a power of two commutes with every rounding of the fold), until the
 // epilogue takes the factor out: the bits of the other kernels.
 //
-// What bounds it: vector instructions.  Per group a wave unpacks three operands (72 shifts and masks, 3.8 clocks each with two waves on
-// a SIMD), converts 32 sums and folds them, around 1400 clocks for the SIMD's two waves, of which the matrix pipe is busy 530.
-// Sums whose first operand is the bits of 1.5 x 2^23, so that a subtraction takes the conversion's place: no faster.
-// us, token / group scales, the tiles this replaces -> this: 1000 x 4096 x 4096 33 -> 26 / 38 -> 27, 250 x 14336 x 4096 32 -> 27 / 38 -> 27,
-// 250 x 28672 x 4096 with SwiGLU 57 -> 52 (group), 128 x 22016 34 -> 28 / 39 -> 29, q / k / v + rotary 512 x 6144 33 -> 28 / 39 -> 30.
+// What bounds it: vector instructions.  Per group a wave unpacks three operands (72 shifts and masks, 3.8 clocks each with two
+// waves on a SIMD), converts 32 sums and folds them, around 1400 clocks for the SIMD's two waves, of which the matrix pipe is
+// busy 530.  Sums whose first operand is the bits of 1.5 x 2^23, so that a subtraction takes the conversion's place: no faster.
+// us, token / group scales, the tiles this replaces -> this: 1000 x 4096 x 4096 33 -> 26 / 38 -> 27, 250 x 14336 x 4096 32 ->
+// 27 / 38 -> 27, 250 x 28672 x 4096 with SwiGLU 57 -> 52 (group), 128 x 22016 34 -> 28 / 39 -> 29, q / k / v + rotary 512 x
+// 6144 33 -> 28 / 39 -> 30.
 #include "gemm_f6_large.h"
 
 namespace flh {
@@ -32,7 +33,8 @@ __device__ __forceinline__ void load_lines_to_lds(const v4i& d, unsigned v0, uns
                "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
                "buffer_load_dwordx4 %3, %5, 0 offen lds\n\t"
                "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
-               "buffer_load_dwordx4 %4, %5, 0 offen lds" ::"s"(lds_base), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(d) : "memory", "m0", "scc");
+               "buffer_load_dwordx4 %4, %5, 0 offen lds" ::"s"(lds_base), "v"(v0), "v"(v1), "v"(v2), "v"(v3),
+               "s"(d) : "memory", "m0", "scc");
 }
 
 template <int EPI, int OUT>
@@ -162,7 +164,11 @@ __global__ __launch_bounds__(512, 1) void gemm_i4_square_kernel(const GemmArgs p
   // Where in a stage's second group the next stage's first fragments are read: at once, and the stage has to have arrived a
   // whole one ahead (group scales 94.4 -> 92.5 us at 1000 x 14336 x 4096), or behind the barrier (token scales: 91.1 -> 89.4)
   constexpr int kReadAt = TOKEN ? 4 : 0;
-  constexpr int kBehind = (kSqStages - (kReadAt ? 2 : 3)) * 4, kStores = OUT == kSwiglu ? 2 : 4;   // as in gemm_f6_large_group.hip
+  // What a wave's waits count, as in gemm_f6_large_group.hip: loads come back in order, four instructions per stage (`issue`), so
+  // that with kBehind outstanding everything older than the stages behind the needed one has arrived -- the scales' requests,
+  // which are older still or come on top, only make a wait longer.  In a tile's first stage the kStores stores of the tile before
+  // are certain to be younger as well, if every wave made them all (`stored`).
+  constexpr int kBehind = (kSqStages - (kReadAt ? 2 : 3)) * 4, kStores = OUT == kSwiglu ? 2 : 4;
   wait_vmcnt<kBehind + 4>();
   __syncthreads();
 
@@ -227,7 +233,8 @@ __global__ __launch_bounds__(512, 1) void gemm_i4_square_kernel(const GemmArgs p
       }
       sums[G][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_op, b_op[t], s < 2 ? zero_i : sums[G][t], 0, 0, 0);
       if constexpr (!(FIRST && G == 0))
-        fold(std::integral_constant<int, u>{}, std::integral_constant<int, 1 - G>{}, std::integral_constant<int, 4 * (s & 3)>{}, chan_last[u]);
+        fold(std::integral_constant<int, u>{}, std::integral_constant<int, 1 - G>{}, std::integral_constant<int, 4 * (s & 3)>{},
+             chan_last[u]);
       if constexpr (!TOKEN && s == 4) prod[0] = __builtin_amdgcn_mfma_f32_32x32x8f16(sav, sbv[0], zero, 0, 0, 0);
       if constexpr (G == 0) {
         if constexpr (s == 0) read_raw(I1, I2, stage);

@@ -497,8 +497,10 @@ int launch_grouped_by_shape(const GemmArgs& a, hipStream_t stream) {
 }
 
 // ... and with one scale per row: 16 x 64 for up to 16 tokens, else 32 x 32 while three workgroups per compute unit hold all of
-// them, with a longer ring where one does, and 64 x 32 beyond or where K is long.  us, 32 x 32 (ring of 3, of 5) / 64 x 32, K = 4096 unless stated:
-//   45 x 4096 of K = 11008 (256 workgroups of 32 x 32) 11.2, 9.2 / 12.7;  45 x 11008 (688) 9.5, 10.8 / 10.3;  128 x 6144 (768) 9.3, 10.8 / 10.0;
+// them, with a longer ring where one does, and 64 x 32 beyond or where K is long.  us, 32 x 32 (ring of 3, of 5) / 64 x 32, K =
+// 4096 unless stated:
+//   45 x 4096 of K = 11008 (256 workgroups of 32 x 32) 11.2, 9.2 / 12.7;  45 x 11008 (688) 9.5, 10.8 / 10.3;  128 x 6144 (768)
+//   9.3, 10.8 / 10.0;
 //   64 x 14336 (896) 13.1 / 11.4;  64 x 28672 (1792) 21.4, 24.1 / 20.5;  128 x 4096 of K = 11008 (512) 15.2, 15.5 / 13.5
 int launch_rows_by_shape(const GemmArgs& a, hipStream_t stream) {
   if (a.M <= 16) return launch_dealt<16, 3>(a, stream);

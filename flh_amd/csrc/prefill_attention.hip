@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const __half*
   auto run = [&](auto p_, int step) {
     constexpr int P = decltype(p_)::value;
     wait_vmcnt<0>();
-    __syncthreads();                                   // V of this step and K of the next are complete; everybody has read the buffers refilled here
+    __syncthreads();   // V of this step and K of the next are complete; everybody has read the buffers refilled here
     issue_k(P);
     issue_v(P ^ 1);
     if (step >= live_steps) return;

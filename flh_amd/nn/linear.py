@@ -34,12 +34,13 @@ class LinearFLH(torch.nn.Module):
             self.bias = None
         # Prefill-sized calls run on the 6-bit matrix instruction where that is faster (extension; same bits, no unpack in the
         # loop).  Its operands are re-encoded at 6 bits per code, 0.75 byte per weight next to the 0.5 of `w_packed`.
-        # False (default): nothing is kept; a long call (_six_bit_rows) encodes its weights into a buffer that goes back with it.  "never": not even that, for callers without that memory to spare.  True: the layer keeps
-        # the encoding (2.5 x the weight memory) and every call of at least `six_bit_min_rows` rows uses it.  "auto" (or
-        # None): kept for weights with a scale per group of 128.
-        # `prepare_six_bit()` builds the kept encoding at once (a loader calls it); otherwise it is built on first use.  It
-        # is rebuilt whenever `w_packed` has been written to or replaced (in-place copies, load_state_dict, .to(device)):
-        # keyed on the buffer's storage address and version counter.
+        # False (default): nothing is kept; a long call (_six_bit_rows) encodes its weights into a buffer that goes back with
+        # it.  "never": not even that, for callers without that memory to spare.  True: the layer keeps the encoding (2.5 x
+        # the weight memory) and every call of at least `six_bit_min_rows` rows uses it.  "auto" (or None): kept for weights
+        # with a scale per group of 128.
+        # `prepare_six_bit()` builds the kept encoding at once (a loader calls it); otherwise it is built on first use.  It is
+        # rebuilt whenever `w_packed` has been written to or replaced (in-place copies, load_state_dict, .to(device)): keyed
+        # on the buffer's storage address and version counter.
         self.six_bit = False
         self.six_bit_min_rows = 256
         self._w6 = None
@@ -53,10 +54,13 @@ class LinearFLH(torch.nn.Module):
     # _transient_tiles -- less fills the chip with neither kernel, and the passes over the operands are all that differs.
     # Packed codes, which the call encodes as well, need more.  us, int8 / 6-bit with the weights encoded (codes from the
     # quantiser in the 6-bit format, which costs it 1-3 us more) / packed codes encoded as well, rows x channels, K = 4096 unless stated:
-    #   one scale per channel: 2048 x 4096 34.5 / 34.9 / 40.7, 3000 x 4096 49 / 43 / 52, 2400 x 11008 109 / 82 / 90; 2048 x 11008 89 / 79 / 87 in
+    #   one scale per channel: 2048 x 4096 34.5 / 34.9 / 40.7, 3000 x 4096 49 / 43 / 52, 2400 x 11008 109 / 82 / 90; 2048 x 11008
+    #   89 / 79 / 87 in
     #   a graph, 84 / 84 as separate calls, and a layer of 1400 tokens whose gate and up change over is slower, 380 / 409
-    #   a scale per token: 640 x 4096 25.7 / 28.5 / 28.4, 1280 x 4096 45 / 35 / 42, 1000 x 14336 95 / 70 / 79, 640 x 4096 of K = 11008 63 / 54 / 58
-    #   group scales: 640 x 4096 27 / 30 / 30, 1000 x 4096 28 / 33 / 33, 640 x 11008 52 / 51 / 55, 800 x 11008 74 / 68 / 70, 1000 x 14336 98 / 76 / 84,
+    #   a scale per token: 640 x 4096 25.7 / 28.5 / 28.4, 1280 x 4096 45 / 35 / 42, 1000 x 14336 95 / 70 / 79, 640 x 4096 of K =
+    #   11008 63 / 54 / 58
+    #   group scales: 640 x 4096 27 / 30 / 30, 1000 x 4096 28 / 33 / 33, 640 x 11008 52 / 51 / 55, 800 x 11008 74 / 68 / 70, 1000 x
+    #   14336 98 / 76 / 84,
     #   512 x 4096 of K = 11008 60 / 54 / 57;
     #   320 x 11008 52 / 43 / 46, but the host's part of the encoding makes a layer of 300 or 450 tokens slower (245 / 262; 500: 271 / 263)
     TRANSIENT_ROWS = (2560, 641)
@@ -275,7 +279,8 @@ class LinearFLH(torch.nn.Module):
                    and (w_scale.size(1) == 1 or (group == 128 and w_scale.size(1) == 32)))
         if fusable:
             y = ops.rotate_quantize_gemm_i4(rows, w, w_scale)
-        elif rows.size(0) >= self.TRANSIENT_ROWS_GROUPS and self.in_features in (4096, 11008, 14336) and self.wants_six_bit(rows.size(0)) and (
+        elif (rows.size(0) >= self.TRANSIENT_ROWS_GROUPS and self.in_features in (4096, 11008, 14336)
+              and self.wants_six_bit(rows.size(0))) and (
                 hadamard in (True, "fast") or (hadamard == "exact" and self.in_features == 4096)):
             # long calls: the quantiser writes the 6-bit operand format
             q, s = ops.rotate_and_quantize_f6(rows, hadamard=hadamard)

@@ -541,7 +541,8 @@ class W4A4DecoderLayer(torch.nn.Module):
             tiles = -(-rows // 64) * -(-2 * g.out_features // 64)
             if self.act_group_size != 128 or (cols == 1 and rows <= 1024) or tiles < (288 if g.in_features <= 1024 else 448):
                 return False
-        return rows > 64 and g.bias is None and self.up_proj.bias is None and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128))
+        return (rows > 64 and g.bias is None and self.up_proj.bias is None
+                and (cols == 1 or (g.weight_group_size == 128 and cols == g.in_features // 128)))
 
     def _group_quant(self, stage, quantizer, x, consumers=()):
         if (self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)) and _stock_call(quantizer, ActQuantizer)
