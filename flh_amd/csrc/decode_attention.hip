@@ -38,9 +38,13 @@ __device__ __forceinline__ _Float16 rope_value(_Float16 x, _Float16 xp, _Float16
 // attention does not read: the first workgroup of every (sequence, key / value head) writes it there, as the
 // stand-alone kernel would.
 //
-// Values pass the caches by (16 x 32 / 8 heads x 4096 64.2 -> 62.6 us, 12 x 32 / 8 x 2048 31.3 -> 30.5).  AHEAD: keys as well, and both
-// are requested before anything else (rule: launch_attention).
-template <int D, int REP, int CHUNK, bool ROPE, bool AHEAD>
+// Values pass the caches by (16 x 32 / 8 heads x 4096 64.2 -> 62.6 us, 12 x 32 / 8 x 2048 31.3 -> 30.5).  With one query per
+// key the keys do as well, and both are requested before anything else.  us with the combine launch, replayed over caches that
+// together don't fit the last-level one, otherwise -> so, sequences x heads / key-value heads x positions: 5 x 32 / 32 x 777
+// 18.7 -> 17.3, 8 x 32 / 32 x 2048 54.6 -> 49.6, 16 x 32 / 32 x 777 44.8 -> 42.1;  grouped queries the same up to two chunks
+// per compute unit (4 x 32 / 8 x 1024 10.3 -> 10.5) and slower beyond (16 x 32 / 8 x 777 17.3 -> 18.7, 8 x 32 / 4 x 3000 21.2
+// -> 24.2).  Inside a decode step there is less in it: 5 x 32 / 32 x 777 14.7 -> 14.4 for the kernel.
+template <int D, int REP, int CHUNK, bool ROPE>
 __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
     const __half* __restrict__ q, __half* k_cache, __half* v_cache, float* __restrict__ partials, uint32_t Hkv,
     uint32_t kv_len, uint32_t max_len, uint32_t splits, float scale, const __half* __restrict__ k_new,
@@ -48,12 +52,14 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
     const long long* __restrict__ positions) {
   static_assert(D == 128 || D == 64, "head dimension");
   static_assert(CHUNK == 64, "one key per lane in the softmax step");
+  constexpr bool AHEAD = REP == 1;
   static_assert(REP <= 16, "the heads of a key / value head are the columns of one matrix tile");
   constexpr int KS = D / 32;                           // matrix steps over the channels
   constexpr int RPW = CHUNK / (kAttnThreads / 64);     // keys / value rows per wave: 16
   __shared__ __align__(16) _Float16 qs[REP * D];       // the query heads
   __shared__ float sc[REP][CHUNK];                     // scores, then probabilities
-  __shared__ float red[kAttnThreads / 64][REP * D];    // the waves' weighted values
+  // the new token's rotated key, later the waves' weighted values
+  __shared__ __align__(16) float red[kAttnThreads / 64][REP * D];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // One or two queries per key: the chunks of one place in all the caches next to each other, whose strides are often a power
@@ -117,23 +123,25 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
       qs[i] = qf[i];
     }
   }
+  // The new token's chunk: its key is rotated like the queries, by all threads through LDS (in its lanes' registers, next to the
+  // requested keys and values, it took 70 registers and with them the eighth wave of a SIMD, most of all where a launch just fits
+  // one round of eight: 16 x 32 / 4 heads x 2048 28.1 -> 24.4 us, 8 x 32 / 8 x 2048 23.3 -> 20.8, 16 x 32 / 8 x 2048 37.5 -> 33.9).
+  _Float16* const new_key = (_Float16*)red[0];
+  const bool fresh_chunk = ROPE && slot - t0 < (uint32_t)CHUNK;
+  if (fresh_chunk) {
+    const _Float16 *kn = (const _Float16*)k_new + (size_t)bh * D, *cf = (const _Float16*)cos, *sf = (const _Float16*)sin;
+    for (int c = tid; c < D; c += kAttnThreads) new_key[c] = rope_value(kn[c], kn[c ^ (D / 2)], cf[c], sf[c], c < D / 2);
+  }
   if constexpr (!AHEAD) request();
-  if (ROPE && slot - t0 < (uint32_t)CHUNK && (slot - t0) / RPW == (uint32_t)wave) {
-    // the new token's wave: key (rotated) and value take the place of what the cache held, here and there
+  __syncthreads();                                     // the queries, and the new key, are in LDS
+  if (fresh_chunk && (slot - t0) / RPW == (uint32_t)wave) {
+    // the new token's wave: key and value take the place of what the cache held, here and there
     const uint32_t r = (slot - t0) % RPW;
     if ((uint32_t)krow == r) {
-      const __half* src = k_new + (size_t)bh * D;
-      __half* dst = k_cache + ((size_t)bh * max_len + slot) * D;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const int c0 = ks * 32 + kb * 8, p0 = c0 ^ (D / 2);
-        const h8 x = *(const h8*)(src + c0), xp = *(const h8*)(src + p0);
-        const h8 cc = *(const h8*)(cos + c0), ss = *(const h8*)(sin + c0);
-        h8 y;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] = rope_value(x[e], xp[e], cc[e], ss[e], c0 < D / 2);
-        ka[ks] = y;
-        *(h8*)(dst + c0) = y;
+        ka[ks] = *(const h8*)(new_key + ks * 32 + kb * 8);
+        *(h8*)(k_cache + ((size_t)bh * max_len + slot) * D + ks * 32 + kb * 8) = ka[ks];
       }
     }
     const raw_t fresh = ((const raw_t*)(v_new + (size_t)bh * D))[lane];
@@ -142,7 +150,6 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
     for (int i = 0; i < RPW; ++i)
       if ((uint32_t)i == r) vr[i] = fresh;
   }
-  __syncthreads();                                     // the queries are in LDS
   {
     v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -279,15 +286,8 @@ int launch_attention(const __half* q, __half* k, __half* v, __half* out, float* 
     hipLaunchKernelGGL(kern, grid, block, 0, stream, q, k, v, partials, Hkv, kv_len, max_len, splits, scale, nt.k, nt.v, nt.cos, nt.sin,
                        nt.positions);
   };
-  // Keys and values requested ahead: always with one query per key, and with up to four on at most two chunks per compute unit.
-  // us with the combine launch, replayed over caches that together don't fit the last-level one, otherwise -> ahead, sequences x
-  // heads / key-value heads x positions (chunks): 5 x 32 / 32 x 777 18.8 -> 17.5, 16 x 32 / 32 x 777 45.1 -> 42.3, 8 x 32 / 32 x 2048
-  // 55.0 -> 49.9;  1 x 32 / 8 x 2048 (256) 10.7 -> 10.3, 4 x 32 / 8 x 1024 (512) 11.4 -> 11.1, 14 x 32 / 8 x 300 (560) 11.5 -> 11.9,
-  // 8 x 32 / 8 x 777 (832) 13.0 -> 13.5, 16 x 32 / 8 x 777 (1664) 17.8 -> 19.2, 14 x 32 / 8 x 2048 (3584) 33.3 -> 33.8, 8 x 32 / 4 x 3000
-  // 21.6 -> 24.0.  In a decode step there is less in it: one query per key, 5 x 777, 14.7 -> 14.4 for the kernel.
-  const bool ahead = REP == 1 || (REP <= 4 && (uint64_t)B * Hkv * splits <= 512);
-  if (nt.k) ahead ? go(decode_attention_partial_kernel<D, REP, kChunk, true, true>) : go(decode_attention_partial_kernel<D, REP, kChunk, true, false>);
-  else ahead ? go(decode_attention_partial_kernel<D, REP, kChunk, false, true>) : go(decode_attention_partial_kernel<D, REP, kChunk, false, false>);
+  if (nt.k) go(decode_attention_partial_kernel<D, REP, kChunk, true>);
+  else go(decode_attention_partial_kernel<D, REP, kChunk, false>);
   if (int rc = check_launch("decode_attention (partials)")) return rc;
   hipLaunchKernelGGL((decode_attention_combine_kernel<D>), dim3(B * Hkv * REP), dim3(256), 0, stream, partials, out,
                      (uint32_t)REP, splits);
