@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
   constexpr int STAGE = ROWS * kRowBytes;
   constexpr int NA = RA / 4 / WAVES, NB = RB / 4 / WAVES, NI = NA + NB;   // 1 KiB load instructions per wave and stage
   constexpr int SROWS = EPI == kGroupScale ? ROWS : RB;   // rows of the scale table: tokens, then channels
-  static_assert(RA / 4 % WAVES == 0 && RB / 4 % WAVES == 0 && (S - 2) * NI < 64, "loads per stage");
+  static_assert(RA / 4 % WAVES == 0 && RB / 4 % WAVES == 0 && (S - 2) * NI < 64 && kRowBytes * 4 == 1024, "loads per stage");
   static_assert(OUT == kStreamPlain || (TN == 2 && WN == 1), "partner tiles");
   extern __shared__ __align__(16) uint8_t lds[];
   lds_byte* ring = (lds_byte*)lds;                 // (typed: a generic pointer would make the reads wait for all loads)
@@ -108,27 +108,30 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
     }
   }
 
-  // operands: a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16)
+  // operands: a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16); a wave's share of either
+  // operand is consecutive KiB of LDS (load_kib_to_lds16: addresses less 1024 i)
   const int lrow = lane >> 4;
-  const uint8_t* src[NI];
+  const uint8_t *src_a[NA], *src_b[NB];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    if (i < NA) {
-      const int row = (wave * NA + i) * 4 + lrow;
-      src[i] = p.A + (size_t)min(m0 + row, p.M - 1) * Kb + ((lane & 15) ^ (row & 15)) * 16;
-    } else {
-      const int row = (wave * NB + i - NA) * 4 + lrow;
-      src[i] = B + (size_t)b_row(row) * Kb + ((lane & 15) ^ (row & 15)) * 16;
-    }
+  for (int i = 0; i < NA; ++i) {
+    const int row = (wave * NA + i) * 4 + lrow;
+    src_a[i] = p.A + (size_t)min(m0 + row, p.M - 1) * Kb + ((lane & 15) ^ (row & 15)) * 16 - 1024 * i;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int row = (wave * NB + i) * 4 + lrow;
+    src_b[i] = B + (size_t)b_row(row) * Kb + ((lane & 15) ^ (row & 15)) * 16 - 1024 * i;
   }
   const unsigned base = (unsigned)(uintptr_t)ring;
   auto request = [&](int s, int slot) {            // slot: byte offset of the ring slot
     const size_t off = (size_t)first_group(s) * 64;
+    const uint8_t *a[NA], *b[NB];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int row = i < NA ? (wave * NA + i) * 4 : RA + (wave * NB + i - NA) * 4;
-      load_to_lds16(src[i] + off, base + slot + row * kRowBytes);
-    }
+    for (int i = 0; i < NA; ++i) a[i] = src_a[i] + off;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) b[i] = src_b[i] + off;
+    load_kib_to_lds16(a, base + slot + wave * NA * 1024);
+    load_kib_to_lds16(b, base + slot + (RA * kRowBytes + wave * NB * 1024));
   };
   int chunk[kStageGroups];                         // of the lane's row
 #pragma unroll
@@ -313,7 +316,7 @@ __global__ __launch_bounds__(256) void gemm_i4_dealt_kernel(const GemmArgs p) {
   constexpr bool SMALL = TOK == 16;
   constexpr int RA = TOK, RB = SMALL ? 64 : 32, STAGE = (RA + RB) * kRowBytes, NI = (RA + RB) / 16;
   constexpr int TT = SMALL ? 1 : TOK / 32, C = SMALL ? 1 : 2;   // token tiles; 16-byte pieces of a row's group per lane
-  static_assert((RA + RB) % 16 == 0 && (S - 2) * NI < 64 && 12 * TT * 1024 <= S * STAGE, "loads per stage, exchange");
+  static_assert((RA + RB) % 16 == 0 && NI <= 8 && (S - 2) * NI < 64 && 12 * TT * 1024 <= S * STAGE, "loads per stage, exchange");
   extern __shared__ __align__(16) uint8_t lds[];
   lds_byte* ring = (lds_byte*)lds;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -333,19 +336,29 @@ __global__ __launch_bounds__(256) void gemm_i4_dealt_kernel(const GemmArgs p) {
   const int m0 = bm * RA, n0 = t * RB;
   auto first_group = [&](int s) { return min(s * kStageGroups, KT - kStageGroups); };   // the last stage ends with the row
 
-  // a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16)
+  // a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16); a wave's rows are consecutive KiB of
+  // LDS (load_kib_to_lds16: addresses less 1024 i, four at a time)
+  constexpr int N0 = NI < 4 ? NI : 4, N1 = NI - N0;
   const uint8_t* src[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int row = (i * 4 + wave) * 4 + (lane >> 4);
+    const int row = (wave * NI + i) * 4 + (lane >> 4);
     src[i] = (row < RA ? p.A + (size_t)min(m0 + row, p.M - 1) * Kb : B + (size_t)min(n0 + max(row - RA, 0), N - 1) * Kb) +
-             ((lane & 15) ^ (row & 15)) * 16;
+             ((lane & 15) ^ (row & 15)) * 16 - 1024 * (i % 4);
   }
   const unsigned base = (unsigned)(uintptr_t)ring;
   auto request = [&](int s, int slot) {
     const size_t off = (size_t)first_group(s) * 64;
+    const unsigned dst = base + slot + wave * NI * 1024;
+    const uint8_t *g[N0], *rest[N1 ? N1 : 1];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) load_to_lds16(src[i] + off, base + slot + (i * 4 + wave) * (4 * kRowBytes));
+    for (int i = 0; i < N0; ++i) g[i] = src[i] + off;
+    load_kib_to_lds16(g, dst);
+    if constexpr (N1 > 0) {
+#pragma unroll
+      for (int i = 0; i < N1; ++i) rest[i] = src[N0 + i] + off;
+      load_kib_to_lds16(rest, dst + 4096);
+    }
   };
   int piece[C];                                    // of the wave's group in the lane's row
 #pragma unroll
