@@ -81,27 +81,23 @@ __device__ __forceinline__ void load_to_lds16(const void* gptr, unsigned lds_bas
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
 
-// N of them (up to four) to consecutive KiB behind one write of M0: an instruction's offset is added to either address, so g[i] is
-// the address less 1024 i
+// N of load_to_lds16 (one, two or four) to consecutive KiB behind one write of M0: an instruction's offset is added to either
+// address, so g[i] is the address less 1024 i
 template <int N>
 __device__ __forceinline__ void load_kib_to_lds16(const uint8_t* const (&g)[N], unsigned lds_base) {
-  static_assert(N >= 1 && N <= 4, "offsets below 4096");
+  static_assert(N == 1 || N == 2 || N == 4, "offsets below 4096");
   if constexpr (N == 1)
     load_to_lds16(g[0], lds_base);
   else if constexpr (N == 2)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\tglobal_load_lds_dwordx4 %2, off offset:1024"
                  ::"s"(lds_base), "v"(g[0]), "v"(g[1]) : "memory", "m0");
-  else if constexpr (N == 3)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\tglobal_load_lds_dwordx4 %2, off offset:1024\n\t"
-                 "global_load_lds_dwordx4 %3, off offset:2048"
-                 ::"s"(lds_base), "v"(g[0]), "v"(g[1]), "v"(g[2]) : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\tglobal_load_lds_dwordx4 %2, off offset:1024\n\t"
                  "global_load_lds_dwordx4 %3, off offset:2048\n\tglobal_load_lds_dwordx4 %4, off offset:3072"
                  ::"s"(lds_base), "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]) : "memory", "m0");
 }
 
-// the same for data that is read once (non-temporal: it does not displace what the caches hold)
+// load_to_lds16 for data that is read once (non-temporal: it does not displace what the caches hold)
 __device__ __forceinline__ void load_to_lds16_nt(const void* gptr, unsigned lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }

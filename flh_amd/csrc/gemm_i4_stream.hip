@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void gemm_i4_dealt_kernel(const GemmArgs p) {
   constexpr bool SMALL = TOK == 16;
   constexpr int RA = TOK, RB = SMALL ? 64 : 32, STAGE = (RA + RB) * kRowBytes, NI = (RA + RB) / 16;
   constexpr int TT = SMALL ? 1 : TOK / 32, C = SMALL ? 1 : 2;   // token tiles; 16-byte pieces of a row's group per lane
-  static_assert((RA + RB) % 16 == 0 && NI <= 8 && (S - 2) * NI < 64 && 12 * TT * 1024 <= S * STAGE, "loads per stage, exchange");
+  static_assert((RA + RB) % 16 == 0 && NI >= 4 && NI <= 6 && (S - 2) * NI < 64 && 12 * TT * 1024 <= S * STAGE, "loads per stage, exchange");
   extern __shared__ __align__(16) uint8_t lds[];
   lds_byte* ring = (lds_byte*)lds;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(256) void gemm_i4_dealt_kernel(const GemmArgs p) {
 
   // a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16); a wave's rows are consecutive KiB of
   // LDS (load_kib_to_lds16: addresses less 1024 i, four at a time)
-  constexpr int N0 = NI < 4 ? NI : 4, N1 = NI - N0;
+  constexpr int N0 = 4, N1 = NI - N0;
   const uint8_t* src[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
