@@ -41,6 +41,8 @@ _SIG = {
                                          _c.c_int, _c.c_int, _c.c_int, _PTR]),
     "flh_rotate_quant_gemm_i4_o16_multi": (_c.c_int, [_PTR, _c.c_int, _PTR, _PTR, _PTR, _PTR, _c.c_size_t, _c.c_size_t,
                                                       _c.c_int, _PTR]),
+    "flh_rmsnorm_group_quant_gemm_i4_o16_multi": (_c.c_int, [_PTR, _PTR, _c.c_float, _c.c_int, _PTR, _PTR, _PTR, _PTR,
+                                                             _c.c_size_t, _c.c_size_t, _PTR]),
     "flh_rmsnorm_rotate_quant_gemm_i4_o16_multi": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _c.c_float, _c.c_int, _PTR, _PTR, _PTR,
                                                               _PTR, _c.c_size_t, _c.c_size_t, _c.c_int, _PTR]),
     "flh_gemm_i4_i32": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_size_t, _c.c_size_t, _c.c_size_t, _PTR]),

@@ -12,7 +12,7 @@ import sys
 
 HERE = pathlib.Path(__file__).resolve().parent
 OUT = HERE.parent / "libflh_hip.so"
-SOURCES = ["capi.hip", "reference_abi.hip", "gemm_i4.hip", "gemm_i4_decode.hip", "gemm_i4_stream.hip", "gemm_i4_square.hip", "gemm_f6.hip", "gemm_f6_large_row.hip", "gemm_f6_large_group.hip", "fwht_quant.hip", "fwht_mfma.hip", "rope_cache.hip", "decode_attention.hip", "prefill_attention.hip", "linear_f16.hip"]
+SOURCES = ["capi.hip", "reference_abi.hip", "gemm_i4.hip", "gemm_i4_decode.hip", "gemm_i4_online.hip", "gemm_i4_stream.hip", "gemm_i4_square.hip", "gemm_f6.hip", "gemm_f6_large_row.hip", "gemm_f6_large_group.hip", "fwht_quant.hip", "fwht_mfma.hip", "rope_cache.hip", "decode_attention.hip", "prefill_attention.hip", "linear_f16.hip"]
 # matrix-core results land in ordinary VGPRs when a kernel fits 256 registers (no copies out of AGPRs)
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 # ... except where the accumulators fill the accumulation registers

@@ -136,6 +136,9 @@ __device__ __forceinline__ void buffer_advance(v4i& d, uint64_t step) {
 // moving memory operations across it.
 __device__ __forceinline__ void barrier_no_fence() { asm volatile("s_barrier" ::: "memory"); }
 
+// ... behind this wave's LDS operations (one piece of assembly: nothing can come between the wait and the barrier)
+__device__ __forceinline__ void barrier_after_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // every LDS (and scalar memory) operation of this wave has completed
 __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 

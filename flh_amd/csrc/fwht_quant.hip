@@ -24,6 +24,7 @@
 #include <type_traits>
 #include "lane_ops.h"
 #include "quant_pack.h"
+#include "group_codes.h"
 #include "f6_codes.h"
 #include "rotate_row.h"
 
@@ -64,15 +65,6 @@ __device__ __forceinline__ unsigned quant_nibble(_Float16 y, float r) {
 //    flip with quad xor 1 / 2, b3 with the mirror inside 8 lanes, b4 with the mirror inside 16:
 //    position = b1*0001 ^ b2*0010 ^ b3*0111 ^ b4*1111.
 // ------------------------------------------------------------------------------------
-template <int LPR>
-__device__ __forceinline__ int group_chunk(int pos) {
-  if constexpr (LPR <= 4) return pos;
-  const int b1 = (pos ^ (pos >> 2)) & 1, b2 = ((pos >> 1) ^ (pos >> 2)) & 1;
-  if constexpr (LPR == 8) return b1 | (b2 << 1) | (pos & 4);
-  const int b3 = ((pos >> 2) ^ (pos >> 3)) & 1;
-  return b1 | (b2 << 1) | (b3 << 2) | (pos & 8);
-}
-
 // butterfly with the partner lane of pattern CTRL: lower lane v + o, upper lane o - v, both as one
 // packed fused multiply-add v * (+-1) + o (the product is exact, so the rounding is that of the sum)
 template <int CTRL>
@@ -108,38 +100,6 @@ __device__ __forceinline__ void fwht_group_f16(h2 (&v)[4], int chunk) {
   if constexpr (G >= 128) group_cross<kDppRowMirror>(v, chunk & 8);
 }
 
-// max |v| over a lane's eight halves, as float: sign bits masked, three packed maxima, one across the pair
-// (written out so that no canonicalising copies are added; NaNs are ignored as fmaxf ignores them)
-__device__ __forceinline__ float lane_abs_max(const h2 (&v)[4]) {
-  unsigned a[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) a[i] = __builtin_bit_cast(unsigned, v[i]) & 0x7FFF7FFFu;
-  unsigned m01, m23, m;
-  asm("v_pk_max_f16 %0, %1, %2" : "=v"(m01) : "v"(a[0]), "v"(a[1]));
-  asm("v_pk_max_f16 %0, %1, %2" : "=v"(m23) : "v"(a[2]), "v"(a[3]));
-  asm("v_pk_max_f16 %0, %1, %2" : "=v"(m) : "v"(m01), "v"(m23));
-  const h2 p = __builtin_bit_cast(h2, m);
-  float lo = (float)p.x, hi = (float)p.y, r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
-  return r;
-}
-
-// max(m, m of the partner lane) in one instruction (the DPP operand feeds the maximum directly; the two wait
-// states a DPP read needs after the write of its source are spelled out, the assembler does not add them here)
-template <int CTRL>
-__device__ __forceinline__ float max_across(float m) {
-  float r;
-  if constexpr (CTRL == kDppQuadXor1)
-    asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(m));
-  else if constexpr (CTRL == kDppQuadXor2)
-    asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(m));
-  else if constexpr (CTRL == kDppRowHalfMirror)
-    asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(m));
-  else
-    asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %1, %1 row_mirror row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(m));
-  return r;
-}
-
 // scale, codes and stores of one row of G values held by LPR = G / 8 adjacent lanes (this lane: chunk `lir`)
 //
 // F6 (G = 128 only): the codes leave in the operand format of the 6-bit matrix instruction instead -- 6 bits per
@@ -154,16 +114,10 @@ __device__ __forceinline__ void group_finish_from(float m, const h2 (&v)[4], int
                                                   uint32_t groups_per_token) {
   static_assert(!F6 || G == 128, "one 6-bit block is 128 codes");
   constexpr int LPR = G / 8;
-  m = max_across<kDppQuadXor1>(m);
-  m = max_across<kDppQuadXor2>(m);
-  if constexpr (LPR >= 8) m = max_across<kDppRowHalfMirror>(m);
-  if constexpr (LPR >= 16) m = max_across<kDppRowMirror>(m);
-  // no division sequences (see scale_of_max): a lane has only eight values to spread them over
-  _Float16 s = scale_of_max(m);
-  if (s <= (_Float16)1e-6f) s = (_Float16)1.0f;
-  const float r = reciprocal_of_scale(s);
-  // |y / s| <= 7.004 unless the scale is subnormal: only then (any row of this wave) clamp the quotients
-  const bool careful = __builtin_amdgcn_ballot_w64((float)s < 6.2e-5f) != 0;
+  const GroupScale scale = group_scale<LPR>(m);
+  const _Float16 s = scale.s;
+  const float r = scale.r;
+  const bool careful = scale.careful;
   const h2 hb = {(_Float16)65504.0f, (_Float16)65504.0f};   // no clipping in the group kernels
   const unsigned y01 = __builtin_bit_cast(unsigned, v[0]), y23 = __builtin_bit_cast(unsigned, v[1]),
                  y45 = __builtin_bit_cast(unsigned, v[2]), y67 = __builtin_bit_cast(unsigned, v[3]);
@@ -844,27 +798,29 @@ int launch_wave(const __half* x, uint8_t* q, __half* s, __half* y, uint32_t M, b
   return check_launch("rotate_quant_wave");
 }
 
-// A few rows of 4096: one workgroup of eight waves per row (rotate_quant_row_8waves: the same additions in the same
+// A few rows of 4096: one workgroup of eight waves per row (rotate_quant_rows_8waves: the same additions in the same
 // order as the wave-per-row kernel, hence the same bytes), so that a decode-sized batch waits for an eighth of a
 // row's arithmetic instead of a whole row's on a single wave.
 __global__ __launch_bounds__(512) void rotate_quant_row8_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
                                                                 __half* __restrict__ scales, float norm) {
-  __shared__ float stage[8 * 8 * 64];
-  __shared__ float wave_max8[8];
+  __shared__ RowScratch<> lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t row = blockIdx.x;
-  rotate_quant_row_8waves(x + row * 4096, stage, wave_max8, q + row * 2048, scales + row, norm, wave);
+  const v4i none = {0, 0, 0, 0};
+  const RowPiece piece[1] = {{row_piece(x + row * 4096, wave), none, none}};
+  rotate_quant_rows_8waves(piece, lds, q + row * 2048, 0, scales + row, norm, wave);
 }
 // ... and with RMSNorm in front (flh_rmsnorm_rotate_quant_i4), the same bytes as rotate_quant_wave_kernel<8, ..., RMS>
 __global__ __launch_bounds__(512) void rmsnorm_rotate_quant_row8_kernel(const __half* __restrict__ x,
                                                                         const __half* __restrict__ weight, float eps,
                                                                         uint8_t* __restrict__ q,
                                                                         __half* __restrict__ scales, float norm) {
-  __shared__ float stage[8 * 8 * 64];
-  __shared__ float wave_max8[8];
+  __shared__ RowScratch<> lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t row = blockIdx.x;
-  rotate_quant_row_8waves<true>(x + row * 4096, stage, wave_max8, q + row * 2048, scales + row, norm, wave, weight, eps);
+  const v4i none = {0, 0, 0, 0};
+  const RowPiece piece[1] = {{row_piece(x + row * 4096, wave), none, weight ? row_piece(weight, wave) : none}};
+  rotate_quant_rows_8waves<true>(piece, lds, q + row * 2048, 0, scales + row, norm, wave, weight != nullptr, eps);
 }
 // ... and with the residual addition in front of that (flh_add_rmsnorm_rotate_quant_i4)
 __global__ __launch_bounds__(512) void add_rmsnorm_rotate_quant_row8_kernel(const __half* __restrict__ x,
@@ -873,12 +829,13 @@ __global__ __launch_bounds__(512) void add_rmsnorm_rotate_quant_row8_kernel(cons
                                                                             const __half* __restrict__ weight, float eps,
                                                                             uint8_t* __restrict__ q,
                                                                             __half* __restrict__ scales, float norm) {
-  __shared__ float stage[8 * 8 * 64];
-  __shared__ float wave_max8[8];
+  __shared__ RowScratch<> lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t row = blockIdx.x;
-  rotate_quant_row_8waves<true, true>(x + row * 4096, stage, wave_max8, q + row * 2048, scales + row, norm, wave, weight,
-                                      eps, add + row * 4096, sum_out + row * 4096);
+  const v4i none = {0, 0, 0, 0};
+  const RowPiece piece[1] = {{row_piece(x + row * 4096, wave), row_piece(add + row * 4096, wave), weight ? row_piece(weight, wave) : none}};
+  rotate_quant_rows_8waves<true, true>(piece, lds, q + row * 2048, 0, scales + row, norm, wave, weight != nullptr, eps,
+                                      sum_out + row * 4096);
 }
 // measured per launch inside a replayed graph: 2.7 against 4.4 us for one row, 3.2 against 4.9 us for 256 rows,
 // 3.9 against 5.0 us for 512; from 1024 rows on the wave-per-row kernel is the faster one

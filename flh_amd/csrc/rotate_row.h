@@ -295,129 +295,162 @@ __device__ __forceinline__ void rotate_quant_row(const __half* __restrict__ x_ro
 
 // One row of 4096 values by the eight waves of a workgroup, for callers where a single row's latency matters:
 // wave w takes the 512 values from 512 w -- strides 1 .. 256 in registers and across lanes as above -- and the
-// strides 512, 1024, 2048 run across the waves through LDS (stage: 8 x 8 x 64 floats, wave_max: 8 floats).
-// The same additions in the same order as rotate_quant_row<8>, hence the same codes and scale.  Every wave of the
-// workgroup must call it (four barriers).
-// RMS: the row is normalised first, as rotate_quant_row<8, ..., RMS> does it.  Every wave reads the whole row once
-// more (it is in the compute unit's cache by then) and sums the squares in exactly that routine's order -- per lane
-// over the eight 512-value segments, then the fixed tree over the lanes -- so that the statistics, the normalised
-// fp16 row and therefore the codes are bit-identical to the wave-per-row kernel's, without a pass over the waves.
-// ADD: the row is x + add_row (fp16), stored to sum_row as well, as in rotate_quant_row.  Every wave forms the whole sum
-// for the statistics and stores only its own segment (the other waves still read x_row and add_row meanwhile).
-template <bool RMS = false, bool ADD = false>
-__device__ __forceinline__ void rotate_quant_row_8waves(const __half* __restrict__ x_row, float* stage, float* wave_max8,
-                                                        uint8_t* q_row, __half* scale_dst, float norm, int wave,
-                                                        const __half* __restrict__ rms_weight = nullptr,
-                                                        float rms_eps = 0.f, const __half* __restrict__ add_row = nullptr,
-                                                        __half* __restrict__ sum_row = nullptr) {
+// strides 512, 1024, 2048 run across the waves through LDS.  The same additions in the same order as
+// rotate_quant_row<8>, hence the same codes and scale.  Every wave of the workgroup must call it (three barriers, one
+// more with RMS).  The caller has requested the row before (RowPiece: a wave's 512 values, and what is added to and
+// multiplied with them), so that loads of its own can be under way behind: the barriers here wait for LDS only.
+// RMS: the row is normalised first, as rotate_quant_row<8, ..., RMS> does it.  Every wave reads the whole row back
+// from LDS and sums the squares in exactly that routine's order -- per lane over the eight 512-value segments, then
+// the fixed tree over the lanes -- so that the statistics, the normalised fp16 row and therefore the codes are
+// bit-identical to the wave-per-row kernel's, without a pass over the waves.
+// ADD: the row is x + add (fp16), stored to sum_row as well, as in rotate_quant_row (every wave its own segment).
+// R rows at a time share the barriers.
+struct RowPiece {
+  v4i x, add, weight;
+};
+template <int R = 1>
+struct RowScratch {
+  float stage[2][R][8 * 8 * 64];
+  v4i row[R][8 * 64];          // RMS
+  float wave_max[R][8];
+};
+__device__ __forceinline__ v4i row_piece(const __half* row, int wave) {
+  return *(const v4i*)(row + wave * 512 + lane_chunk(threadIdx.x & 63) * 8);
+}
+// q_row and sum_row: of the first row, the others q_pitch bytes / 4096 values behind; live: how many of the rows are stored
+template <bool RMS = false, bool ADD = false, int R = 1>
+__device__ __forceinline__ void rotate_quant_rows_8waves(const RowPiece (&in)[R], RowScratch<R>& lds, uint8_t* q_row, int q_pitch,
+                                                         __half* scale_dst, float norm, int wave, bool weighted = false,
+                                                         float rms_eps = 0.f, __half* __restrict__ sum_row = nullptr, int live = R) {
   const int lane = threadIdx.x & 63;
   const int c = lane_chunk(lane);
-  v4i raw = *(const v4i*)(x_row + wave * 512 + c * 8);
-  if constexpr (ADD) {
-    raw = add_h8(raw, *(const v4i*)(add_row + wave * 512 + c * 8));
-    if (sum_row) *(v4i*)(sum_row + wave * 512 + c * 8) = raw;    // (null: another workgroup stores the same sum)
-  }
+  v4i raw[R];
+  static_for<R>([&](auto i_tag) {
+    constexpr int i = decltype(i_tag)::value;
+    raw[i] = in[i].x;
+    if constexpr (ADD) {
+      raw[i] = add_h8(raw[i], in[i].add);
+      if (sum_row && i < live) *(v4i*)(sum_row + i * 4096 + wave * 512 + c * 8) = raw[i];    // (null: another workgroup stores the same sum)
+    }
+    if constexpr (RMS) lds.row[i][wave * 64 + lane] = raw[i];
+  });
   if constexpr (RMS) {
-    float ss = 0.f;
+    barrier_after_lds();
+    static_for<R>([&](auto i_tag) {
+      constexpr int i = decltype(i_tag)::value;
+      float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      v4i seg = *(const v4i*)(x_row + j * 512 + c * 8);
-      if constexpr (ADD) seg = add_h8(seg, *(const v4i*)(add_row + j * 512 + c * 8));
+      for (int j = 0; j < 8; ++j) {
+        const v4i seg = lds.row[i][j * 64 + lane];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const unsigned w = (unsigned)seg[d];
+          const h2 t = __builtin_bit_cast(h2, w);
+          ss = __builtin_fmaf((float)t[0], (float)t[0], ss);
+          ss = __builtin_fmaf((float)t[1], (float)t[1], ss);
+        }
+      }
+      ss = wave_sum(ss);
+      const float inv = 1.0f / __builtin_sqrtf(ss / 4096.0f + rms_eps);
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        const unsigned w = (unsigned)seg[d];
-        const h2 t = __builtin_bit_cast(h2, w);
-        ss = __builtin_fmaf((float)t[0], (float)t[0], ss);
-        ss = __builtin_fmaf((float)t[1], (float)t[1], ss);
+        const unsigned w = (unsigned)raw[i][d], ww = (unsigned)in[i].weight[d];
+        const h2 t = __builtin_bit_cast(h2, w), g = __builtin_bit_cast(h2, ww);
+        float a = round_here((float)t[0] * inv), b = round_here((float)t[1] * inv);
+        if (weighted) {
+          a = round_here(a * (float)g[0]);
+          b = round_here(b * (float)g[1]);
+        }
+        raw[i][d] = (int)pack_f16(a, b);
       }
-    }
-    ss = wave_sum(ss);
-    const float inv = 1.0f / __builtin_sqrtf(ss / 4096.0f + rms_eps);
-    v4i wv = {0, 0, 0, 0};
-    if (rms_weight) wv = *(const v4i*)(rms_weight + wave * 512 + c * 8);
+    });
+  }
+  static_for<R>([&](auto i_tag) {
+    constexpr int row = decltype(i_tag)::value;
+    float v[8];
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const unsigned w = (unsigned)raw[d], ww = (unsigned)wv[d];
-      const h2 t = __builtin_bit_cast(h2, w), g = __builtin_bit_cast(h2, ww);
-      float a = round_here((float)t[0] * inv), b = round_here((float)t[1] * inv);
-      if (rms_weight) {
-        a = round_here(a * (float)g[0]);
-        b = round_here(b * (float)g[1]);
-      }
-      raw[d] = (int)pack_f16(a, b);
+      const int w = raw[row][d];
+      asm("v_fma_mix_f32 %0, %1, 1.0, %1 op_sel:[0,0,1] op_sel_hi:[1,0,1]" : "=v"(v[2 * d]) : "v"(w));
+      asm("v_fma_mix_f32 %0, %1, -1.0, %1 op_sel:[1,0,0] op_sel_hi:[1,0,1]" : "=v"(v[2 * d + 1]) : "v"(w));
     }
-  }
-  float v[8];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const int w = raw[d];
-    asm("v_fma_mix_f32 %0, %1, 1.0, %1 op_sel:[0,0,1] op_sel_hi:[1,0,1]" : "=v"(v[2 * d]) : "v"(w));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %1 op_sel:[1,0,0] op_sel_hi:[1,0,1]" : "=v"(v[2 * d + 1]) : "v"(w));
-  }
+    for (int s = 2; s < 8; s <<= 1)
 #pragma unroll
-  for (int s = 2; s < 8; s <<= 1)
+      for (int i = 0; i < 8; ++i)
+        if ((i & s) == 0) {
+          const float a = v[i], b = v[i + s];
+          v[i] = a + b;
+          v[i + s] = a - b;
+        }
+    const float sg1 = (c & 1) ? -1.f : 1.f, sg2 = (c & 2) ? -1.f : 1.f, sg3 = (c & 4) ? -1.f : 1.f,
+                sg4 = (c & 8) ? -1.f : 1.f;
+    asm volatile("s_nop 1" : "+v"(v[0]), "+v"(v[1]));
+    stage_fmac<kDppQuadXor1>(v, sg1);
+    stage_fmac<kDppQuadXor2>(v, sg2);
+    stage_fmac<kDppRowHalfMirror>(v, sg3);
+    stage_fmac<kDppRowMirror>(v, sg4);
+    asm volatile("s_nop 1" : "+v"(v[7]), "+v"(v[6]));
+    stage_swap<false>(v);
+    stage_swap<true>(v);
+    // across the waves: value e of every lane goes to wave e, which combines the eight waves' copies
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if ((i & s) == 0) {
-        const float a = v[i], b = v[i + s];
-        v[i] = a + b;
-        v[i + s] = a - b;
-      }
-  const float sg1 = (c & 1) ? -1.f : 1.f, sg2 = (c & 2) ? -1.f : 1.f, sg3 = (c & 4) ? -1.f : 1.f,
-              sg4 = (c & 8) ? -1.f : 1.f;
-  asm volatile("s_nop 1" : "+v"(v[0]), "+v"(v[1]));
-  stage_fmac<kDppQuadXor1>(v, sg1);
-  stage_fmac<kDppQuadXor2>(v, sg2);
-  stage_fmac<kDppRowHalfMirror>(v, sg3);
-  stage_fmac<kDppRowMirror>(v, sg4);
-  asm volatile("s_nop 1" : "+v"(v[7]), "+v"(v[6]));
-  stage_swap<false>(v);
-  stage_swap<true>(v);
-  // across the waves: value e of every lane goes to wave e, which combines the eight waves' copies
+    for (int e = 0; e < 8; ++e) lds.stage[0][row][(e * 8 + wave) * 64 + lane] = v[e];
+  });
+  barrier_after_lds();
+  static_for<R>([&](auto i_tag) {
+    constexpr int row = decltype(i_tag)::value;
+    float u[8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) stage[(e * 8 + wave) * 64 + lane] = v[e];
-  __syncthreads();
-  float u[8];
+    for (int w2 = 0; w2 < 8; ++w2) u[w2] = lds.stage[0][row][(wave * 8 + w2) * 64 + lane];
 #pragma unroll
-  for (int w2 = 0; w2 < 8; ++w2) u[w2] = stage[(wave * 8 + w2) * 64 + lane];
+    for (int s = 1; s < 8; s <<= 1)
 #pragma unroll
-  for (int s = 1; s < 8; s <<= 1)
+      for (int i = 0; i < 8; ++i)
+        if ((i & s) == 0) {
+          const float a = u[i], b = u[i + s];
+          u[i] = a + b;
+          u[i + s] = a - b;
+        }
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if ((i & s) == 0) {
-        const float a = u[i], b = u[i + s];
-        u[i] = a + b;
-        u[i + s] = a - b;
-      }
-  __syncthreads();
-#pragma unroll
-  for (int w2 = 0; w2 < 8; ++w2) stage[(wave * 8 + w2) * 64 + lane] = u[w2];
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = stage[(e * 8 + wave) * 64 + lane];
+    for (int w2 = 0; w2 < 8; ++w2) lds.stage[1][row][(wave * 8 + w2) * 64 + lane] = u[w2];
+  });
+  barrier_after_lds();
   // from here on as rotate_quant_row: sign of the lane folded into the power-of-two normalisation
   const bool flipped = __builtin_popcount(c & 15) & 1;
-  float m32 = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; i += 2) m32 = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v[i]), __builtin_fabsf(v[i + 1])), m32);
   const float nf = flipped ? -norm : norm;
-  unsigned yp[4];
+  unsigned yp[R][4];
+  static_for<R>([&](auto i_tag) {
+    constexpr int row = decltype(i_tag)::value;
+    float v[8];
 #pragma unroll
-  for (int i = 0; i < 8; i += 2) yp[i / 2] = scale_pack_f16(v[i], v[i + 1], nf);
-  float mx = (float)__builtin_bit_cast(h2, scale_pack_f16(m32, 0.f, norm))[0];
-  mx = wave_max(mx);
-  if (lane == 0) wave_max8[wave] = mx;
-  __syncthreads();
+    for (int e = 0; e < 8; ++e) v[e] = lds.stage[1][row][(e * 8 + wave) * 64 + lane];
+    float m32 = 0.f;
 #pragma unroll
-  for (int w2 = 0; w2 < 8; ++w2) mx = __builtin_fmaxf(mx, wave_max8[w2]);
-  _Float16 s = scale_of_max(mx);
-  if (s == (_Float16)0.0f) s = (_Float16)1.0f;
-  const float r = reciprocal_of_scale(s);
-  const bool careful = __builtin_amdgcn_readfirstlane((float)s < 6.2e-5f);
-  const h2 hb = {(_Float16)mx, (_Float16)mx};
-  ((unsigned*)q_row)[wave * 64 + c] = careful ? nibbles8<true>(yp[0], yp[1], yp[2], yp[3], r, hb)
-                                              : nibbles8<false>(yp[0], yp[1], yp[2], yp[3], r, hb);
-  if (wave == 0 && lane == 0) *scale_dst = __builtin_bit_cast(__half, s);
+    for (int i = 0; i < 8; i += 2) m32 = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v[i]), __builtin_fabsf(v[i + 1])), m32);
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) yp[row][i / 2] = scale_pack_f16(v[i], v[i + 1], nf);
+    float mx = (float)__builtin_bit_cast(h2, scale_pack_f16(m32, 0.f, norm))[0];
+    mx = wave_max(mx);
+    if (lane == 0) lds.wave_max[row][wave] = mx;
+  });
+  barrier_after_lds();
+  static_for<R>([&](auto i_tag) {
+    constexpr int row = decltype(i_tag)::value;
+    float mx = lds.wave_max[row][0];
+#pragma unroll
+    for (int w2 = 1; w2 < 8; ++w2) mx = __builtin_fmaxf(mx, lds.wave_max[row][w2]);
+    _Float16 s = scale_of_max(mx);
+    if (s == (_Float16)0.0f) s = (_Float16)1.0f;
+    const float r = reciprocal_of_scale(s);
+    const bool careful = __builtin_amdgcn_readfirstlane((float)s < 6.2e-5f);
+    const h2 hb = {(_Float16)mx, (_Float16)mx};
+    const unsigned(&y)[4] = yp[row];
+    if (row >= live) return;
+    ((unsigned*)(q_row + row * q_pitch))[wave * 64 + c] = careful ? nibbles8<true>(y[0], y[1], y[2], y[3], r, hb)
+                                                                  : nibbles8<false>(y[0], y[1], y[2], y[3], r, hb);
+    if (wave == 0 && lane == 0) scale_dst[row] = __builtin_bit_cast(__half, s);
+  });
 }
 
 }  // namespace

@@ -347,16 +347,10 @@ class W4A4DecoderLayer(torch.nn.Module):
         block, None, cache)."""
         b, t, _ = x.shape
         if (self.activation == "token" and self.fused and self.record is None and b * t <= 2 and self.hidden_size == 4096
-                and self._online_qkv_applies()):
+                and self._online_applies((self.q_proj, self.k_proj, self.v_proj))):
             # decode: residual addition, norm, rotation, quantiser and the three projections in one launch, two where faster
-            layers = [self.q_proj, self.k_proj, self.v_proj]
-            total, (qs, ks, vs) = _ops().rmsnorm_rotate_quantize_gemm_i4_multi(
-                x.reshape(b * t, -1).contiguous(), None if add is None else add.reshape(b * t, -1).contiguous(),
-                self._norm_weight16("input_layernorm", self.input_layernorm), self.input_layernorm.eps,
-                [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
-                [l.w_scale.view(l.out_features, -1) for l in layers])
-            if total is not None:
-                x = total.view(x.shape)
+            x, (qs, ks, vs) = self._norm_quant_project([self.q_proj, self.k_proj, self.v_proj], self.input_layernorm,
+                                                       "input_layernorm", x, add)
         else:
             x, s, z, q = self._residual_norm_quant("attn_in", self.input_layernorm, "input_layernorm",
                                                    self.attn_quantizer1, x, add, (self.q_proj, self.k_proj, self.v_proj))
@@ -457,7 +451,7 @@ class W4A4DecoderLayer(torch.nn.Module):
         the int8 kernel), "f6" (codes in the 6-bit format, or layers that would re-encode them) or None."""
         static = isinstance(kv_cache, StaticKVCache._Layer)
         if not (self.fused and self.record is None and rows > 64 and rows > codes.size(0) and self.head_dim == 128
-                and codes.is_cuda and self._online_qkv_applies() and cos.dtype == torch.float16
+                and codes.is_cuda and self._online_applies((self.q_proj, self.k_proj, self.v_proj)) and cos.dtype == torch.float16
                 and tuple(cos.shape) == (rows // codes.size(0), 128) and (positions is not None if static else True)):
             return None
         if codes.size(-1) * 4 == self.hidden_size * 3:
@@ -517,15 +511,24 @@ class W4A4DecoderLayer(torch.nn.Module):
         return (self.fused and self.record is None and self.activation == "group"
                 and (rows > 64 or (rows > 0 and _stock_call(linear, LinearFLH))))
 
-    def _online_qkv_applies(self):
-        """q / k / v in the layout the decode GEMM with its own norm + quantiser takes: no bias, one scale per channel or
-        per group of 128, the same for all three."""
-        layers = (self.q_proj, self.k_proj, self.v_proj)
+    def _online_applies(self, layers):
+        """`layers` on the hidden state in the layout the GEMMs with their own norm + quantiser take: no bias, one scale per
+        channel or per group of 128, the same for all of them."""
         cols = {l.w_scale.numel() // l.out_features for l in layers}
         if any(l.bias is not None for l in layers) or len(cols) != 1:
             return False
         c = cols.pop()
-        return c == 1 or (c == self.hidden_size // 128 and self.q_proj.weight_group_size == 128)
+        return c == 1 or (c == self.hidden_size // 128 and layers[0].weight_group_size == 128)
+
+    def _norm_quant_project(self, layers, norm, norm_name, x, add):
+        """(x + add, outputs) of the residual addition, the norm, the whole-row quantiser and `layers`: one launch for one or two
+        tokens, the bits of the separate ones."""
+        rows = x.numel() // x.size(-1)
+        total, ys = _ops().rmsnorm_rotate_quantize_gemm_i4_multi(
+            x.reshape(rows, -1).contiguous(), None if add is None else add.reshape(rows, -1).contiguous(),
+            self._norm_weight16(norm_name, norm), norm.eps, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
+            [l.w_scale.view(l.out_features, -1) for l in layers])
+        return (x if total is None else total.view(x.shape)), ys
 
     def _swiglu_gemm_applies(self, rows):
         """Whether gate and up take the launch that stores silu(gate) * up only: prefill sizes.  Group configuration, us per layer,
@@ -562,26 +565,32 @@ class W4A4DecoderLayer(torch.nn.Module):
     def _mlp(self, x, add, fold_residual=True):
         """mlp() on the residual stream x + add (add may be None); returns (that sum, the MLP's output) -- or (the stream
         after the block, None) when down_proj adds the residual in its epilogue (`fold_residual`, prefill sizes)."""
-        x, s, z, q = self._residual_norm_quant("mlp_in", self.post_attention_layernorm, "post_attention_layernorm",
-                                               self.mlp_quantizer1, x, add, (self.gate_proj, self.up_proj))
-        rows = q.numel() // q.size(-1)
-        if self.fused and self.record is None and self._swiglu_gemm_applies(rows):
-            # prefill: gate and up in one launch that stores silu(gate) * up only (no fp16 [M, I] round trips)
-            mid = LinearFLH.forward_swiglu(self.gate_proj, self.up_proj, q, s)
-            if self.activation == "token":
-                s, z, q = self._token_quant("mlp_mid", mid, consumers=(self.down_proj,))
-            else:
-                if self._group_six_bit_for((self.down_proj,), rows, mid.size(-1)):
-                    q, s = _ops().group_quantize_f6(mid.view(rows, -1), False)
+        rows = x.numel() // x.size(-1)
+        pair = (self.gate_proj, self.up_proj)
+        if (self.activation == "token" and self.fused and self.record is None and 0 < rows <= 2 and self.hidden_size == 4096
+                and self._online_applies(pair)):
+            x, (gate, up) = self._norm_quant_project(pair, self.post_attention_layernorm, "post_attention_layernorm", x, add)
+            gate, up = gate.view(*x.shape[:-1], -1), up.view(*x.shape[:-1], -1)
+        else:
+            x, s, z, q = self._residual_norm_quant("mlp_in", self.post_attention_layernorm, "post_attention_layernorm",
+                                                   self.mlp_quantizer1, x, add, pair)
+            if self.fused and self.record is None and self._swiglu_gemm_applies(rows):
+                # prefill: gate and up in one launch that stores silu(gate) * up only (no fp16 [M, I] round trips)
+                mid = LinearFLH.forward_swiglu(self.gate_proj, self.up_proj, q, s)
+                if self.activation == "token":
+                    s, z, q = self._token_quant("mlp_mid", mid, consumers=(self.down_proj,))
                 else:
-                    q, s = _ops().quant_and_pack_i4_gs(mid.view(-1, 128), 128)
-                s, z, q = s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
-                fold_residual = fold_residual and self._residual_in_gemm(rows, self.down_proj)
-            if fold_residual:
-                return self.down_proj(q, s, z, x_is_packed=True, residual=x), None
-            return x, self.down_proj(q, s, z, x_is_packed=True)
-        gate, up = self._project([self.gate_proj, self.up_proj], q, s, z)
-        self._tap("gate_proj", gate), self._tap("up_proj", up)
+                    if self._group_six_bit_for((self.down_proj,), rows, mid.size(-1)):
+                        q, s = _ops().group_quantize_f6(mid.view(rows, -1), False)
+                    else:
+                        q, s = _ops().quant_and_pack_i4_gs(mid.view(-1, 128), 128)
+                    s, z, q = s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
+                    fold_residual = fold_residual and self._residual_in_gemm(rows, self.down_proj)
+                if fold_residual:
+                    return self.down_proj(q, s, z, x_is_packed=True, residual=x), None
+                return x, self.down_proj(q, s, z, x_is_packed=True)
+            gate, up = self._project([self.gate_proj, self.up_proj], q, s, z)
+            self._tap("gate_proj", gate), self._tap("up_proj", up)
         if (self.activation == "token" and self.fused and self.record is None and rows <= 256
                 and self.intermediate_size in (11008, 14336)):
             # decode: silu(gate) * up formed inside the rotation's launch, never stored
