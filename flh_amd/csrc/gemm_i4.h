@@ -72,6 +72,8 @@ __device__ __forceinline__ float fma_half(float v, unsigned s, float acc) {
 
 // Small-M (decode) kernels: weight-streaming, split over K inside a workgroup.
 constexpr int kDecodeMaxM = 64;
+bool gemm_dot_supports(const GemmArgs& a, int epi, int group);        // up to four tokens
+int gemm_dot_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group);
 int gemm_decode_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
 

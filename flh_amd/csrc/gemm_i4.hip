@@ -773,6 +773,7 @@ int gemm_dispatch(GemmArgs a, int epi, int group, hipStream_t stream) {
   if (a.M == 0 || a.N == 0) return FLH_OK;
   if (epi == kGroupScale && group == 128 && (a.M > kDecodeMaxM || g_tune_tile.load(std::memory_order_relaxed)) && takes_square(a, total_n(a)))
     return gemm_square_dispatch(a, kSquarePlain, stream);
+  if (gemm_dot_supports(a, epi, group)) return gemm_dot_dispatch(a, epi, stream);
   if (gemm_stream_supports(a, epi, group)) return gemm_stream_dispatch(a, epi, stream);
   if (gemm_decode_supports(a, epi, group)) return gemm_decode_dispatch(a, epi, stream);
   switch (epi) {

@@ -1,4 +1,4 @@
-// int4 x int4 GEMM + dequant for a handful of tokens (decode, M <= 64): the weights are
+// int4 x int4 GEMM + dequant for a handful of tokens (decode, M <= 64; up to four have a kernel of their own at the end): the weights are
 // streamed from HBM exactly once and the contraction is split over K inside a workgroup.
 //
 // Same arithmetic as gemm_i4.hip (codes x 16 as int8 on the matrix cores, exact int32 sums,
@@ -24,6 +24,7 @@
 //   7.4, 4096 x 4096 6.5 / 6.6 -> 5.5 / 5.6;  one token: 4096 x 14336 11.9 / 12.0 -> 10.3 / 10.9, 4096 x 4096 5.7 / 5.7 -> 5.1 / 5.2
 #include <atomic>
 #include "gemm_i4.h"
+#include "lane_ops.h"
 
 namespace flh {
 namespace {
@@ -64,7 +65,8 @@ int decode_blocks(GemmArgs& a) {
 }
 
 // one fp16 output; with a residual (single weight matrix) the stored value is fp16(R + value)
-__device__ __forceinline__ void store_f16(const GemmArgs& p, const DecodeWeights& w, int gm, int gn, _Float16 v) {
+template <typename Args>
+__device__ __forceinline__ void store_f16(const Args& p, const DecodeWeights& w, int gm, int gn, _Float16 v) {
   const size_t at = (size_t)gm * w.N + gn;
   if (p.R) v = v + ((const _Float16*)p.R)[at];
   ((_Float16*)w.D)[at] = v;
@@ -75,7 +77,8 @@ __device__ __forceinline__ void store_f16(const GemmArgs& p, const DecodeWeights
 // rows that dword loads cannot fetch (an odd number of groups, an odd element offset, one scale per channel) are filled half by half.
 __host__ __device__ constexpr int scale_pitch(int KT) { return ((KT + 1) >> 1) | 1; }   // dwords per row
 
-__device__ __forceinline__ void request_scales(const GemmArgs& p, const DecodeWeights& w, unsigned* table, int KT, int tid) {
+template <typename Args>
+__device__ __forceinline__ void request_scales(const Args& p, const DecodeWeights& w, unsigned* table, int KT, int tid) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pitch = scale_pitch(KT), tokens = p.a_cols > 1 ? p.M : 0, rows = tokens + 16;   // (at most 16 tokens)
   auto row_of = [&](int row) {
@@ -118,10 +121,10 @@ __device__ __forceinline__ FirstScales first_scales(const GemmArgs& p, const Dec
   return f;
 }
 
-// out = fma(sum, scale, out) over the groups in ascending order: v[g * MT * 256] the sums, ra and rb the token's and the channel's
+// out = fma(sum, scale, out) over the groups in ascending order: v[g * STRIDE] the sums, ra and rb the token's and the channel's
 // scales, two to a dword (TOKEN: the channel's alone).  Eight pairs of groups are read ahead of their multiply-adds, by hand:
 // a loop with inline assembly is not unrolled, and a pair at a time waits for LDS at every pair.
-template <int MT, bool TOKEN>
+template <int STRIDE, bool TOKEN>
 __device__ __forceinline__ float fold_groups(const float* v, const unsigned* ra, const unsigned* rb, int KT) {
   constexpr int kAhead = 8;
   const int pairs = KT >> 1;
@@ -142,7 +145,7 @@ __device__ __forceinline__ float fold_groups(const float* v, const unsigned* ra,
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int at = WHOLE ? g + u : min(g + u, pairs - 1);
-      lo[u] = v[2 * at * MT * 256], hi[u] = v[(2 * at + 1) * MT * 256];
+      lo[u] = v[2 * at * STRIDE], hi[u] = v[(2 * at + 1) * STRIDE];
       a[u] = TOKEN ? 0u : ra[at], b[u] = rb[at];
     }
 #pragma unroll
@@ -153,7 +156,7 @@ __device__ __forceinline__ float fold_groups(const float* v, const unsigned* ra,
   for (; g + kAhead <= pairs; g += kAhead) batch(g, std::true_type{});
   if (g < pairs) batch(g, std::false_type{});
   if (KT & 1) {
-    const float last = v[(KT - 1) * MT * 256];
+    const float last = v[(KT - 1) * STRIDE];
     if constexpr (TOKEN) out = fma_half<0>(last, rb[pairs], out);
     else out = __builtin_fmaf(last, mul_halves<0>(ra[pairs], rb[pairs]), out);
   }
@@ -177,10 +180,10 @@ __device__ __forceinline__ void decode_finish(const GemmArgs& p, const DecodeWei
       float out;
       if (p.a_cols == 1) {                    // one scale per token: applied once, after the groups
         const float s_a = idx == tid ? first.a : __half2float(a_scales[gm]);
-        out = fold_groups<MT, true>(v, nullptr, table + n * pitch, KT);
+        out = fold_groups<MT * 256, true>(v, nullptr, table + n * pitch, KT);
         out = round_here(out * 0.00390625f) * s_a;
       } else {
-        out = fold_groups<MT, false>(v, table + m * pitch, table + (p.M + n) * pitch, KT);
+        out = fold_groups<MT * 256, false>(v, table + m * pitch, table + (p.M + n) * pitch, KT);
         out *= 0.00390625f;
       }
       store_f16(p, w, gm, gn, (_Float16)round_here(out));
@@ -294,7 +297,168 @@ int launch_decode(const GemmArgs& a, hipStream_t stream) {
   return check_launch("gemm_i4_decode");
 }
 
+// One to four tokens: products by v_dot8_i32_i4 on the packed codes as they are, which need no fragment layout, so that a load takes
+// whole lines of eight weight rows, past the caches (gemm_i4_online.hip has the same, and what it is worth there).  A workgroup of
+// eight waves owns 16 channels; a wave requests all its double steps at once, DOUBLES of them, through buffer descriptors:
+// what lies beyond the matrix or the row reads as zero, without a branch.  Lane l holds piece l % 8 (32 codes) of the lines of rows l / 8
+// and 8 + l / 8; four adjacent lanes make a group.  Up to K = 4096 64 registers, four workgroups per compute unit.
+// What bounds it: first access (3 us), then HBM (6 TB/s between 12288 and 28672 channels).  us, weights from HBM, the kernels above and
+// gemm_i4_stream.hip -> this one, one scale per row / token scales / group scales:
+//   one token   4096 x 1024 3.9 / 4.6 / 4.7 -> 2.8 / 3.2 / 3.3, x 4096 4.6 / 5.1 / 5.2 -> 3.4 / 3.8 / 3.8, x 12288 7.8 / 8.4 / 8.2 -> 6.2 /
+//               6.7 / 6.5, x 28672 14.0 / 15.4 / 15.0 -> 11.4 / 11.9 / 11.9;  14336 x 4096 8.8 / 10.5 / 11.0 -> 7.6 / 8.7 / 8.8
+//   four        4096 x 4096 4.7 / 5.2 / 5.1 -> 3.9 / 4.6 / 4.4, x 28672 13.3 / 14.1 / 14.4 -> 13.1 / 13.3 / 13.1
+struct DotSegment {
+  const uint8_t* B;
+  const __half* Bs;
+  __half* D;
+  int N, tile0;                                // its first block of 16 channels (unused ones: beyond every block)
+};
+struct DotArgs {                               // (small and read without a loop: the arguments come by one round of loads)
+  const uint8_t* A;
+  const __half *As, *R;
+  int M, K, a_cols, b_cols;
+  DotSegment seg[kMaxGemmSegments];
+};
+
+template <int MAXM, int DOUBLES, int EPI>
+__global__ __launch_bounds__(kWaves * 64, DOUBLES == 2 ? 8 : 2) void gemm_i4_dot_kernel(const DotArgs p) {
+  extern __shared__ __align__(16) int red[];   // [group | wave][token][16 channels], float32 | int32; then the scales
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int line_row = lane >> 3, piece = lane & 7;
+  const int block = blockIdx.x;
+  // all of the arguments by one round of scalar loads, not segment after segment
+  asm volatile("" ::"s"(p.A), "s"(p.As), "s"(p.M), "s"(p.K), "s"(p.a_cols), "s"(p.b_cols), "s"(p.seg[1].tile0), "s"(p.seg[2].tile0), "s"(p.seg[3].tile0), "s"(p.seg[0].N), "s"(p.seg[1].N),
+               "s"(p.seg[2].N), "s"(p.seg[3].N), "s"(p.seg[0].B), "s"(p.seg[1].B), "s"(p.seg[2].B), "s"(p.seg[3].B), "s"(p.seg[0].Bs),
+               "s"(p.seg[1].Bs), "s"(p.seg[2].Bs), "s"(p.seg[3].Bs));
+  DecodeWeights w{p.seg[0].B, p.seg[0].Bs, p.seg[0].D, p.seg[0].N, block * 16};
+#pragma unroll
+  for (int s = 1; s < kMaxGemmSegments; ++s)
+    if (block >= p.seg[s].tile0) w = DecodeWeights{p.seg[s].B, p.seg[s].Bs, p.seg[s].D, p.seg[s].N, (block - p.seg[s].tile0) * 16};
+  const int Kb = p.K >> 1, KT = p.K >> 7;
+  const auto rows_b = __builtin_amdgcn_make_buffer_rsrc((void*)(w.B + (size_t)w.n0 * Kb), 0, min(16, w.N - w.n0) * Kb, 0x00020000);
+  const auto rows_a = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, p.M * Kb, 0x00020000);
+  constexpr unsigned kBeyond = 0x80000000u;
+
+  unsigned* table = (unsigned*)(red + KT * MAXM * 16);
+  if constexpr (EPI == kGroupScale) request_scales(p, w, table, KT, tid);   // (first: behind the operands it takes too many registers)
+  v4i a[MAXM][DOUBLES], b[DOUBLES][2];
+  unsigned at[DOUBLES];                        // byte of the row
+#pragma unroll
+  for (int i = 0; i < DOUBLES; ++i) {
+    at[i] = (wave + i * kWaves) * 128 + piece * 16;
+    if ((int)at[i] >= Kb) at[i] = kBeyond;
+  }
+#pragma unroll
+  for (int i = 0; i < DOUBLES; ++i)
+#pragma unroll
+    for (int m = 0; m < MAXM; ++m) a[m][i] = __builtin_amdgcn_raw_buffer_load_b128(rows_a, at[i] + m * Kb, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < DOUBLES; ++i)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) b[i][q] = __builtin_amdgcn_raw_buffer_load_b128(rows_b, at[i] + (q * 8 + line_row) * Kb, 0, 2 /* nt */);
+  __builtin_amdgcn_sched_barrier(0);
+  const int fm = lane >> 4, fn = lane & 15;    // what the lane of wave 0 finishes
+  float s_a = 0.f, s_b = 0.f;
+  if (EPI == kRowScale || p.a_cols == 1) s_a = __half2float(p.As[min(fm, p.M - 1)]);
+  if constexpr (EPI == kRowScale) s_b = __half2float(w.Bs[min(w.n0 + fn, w.N - 1)]);
+
+  auto dot = [](const v4i& x, const v4i& y, int sum) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(x[e], y[e], sum, false);
+    return sum;
+  };
+  const bool odd = lane & 1, high = lane & 2;
+  const int n = (lane & 1) * 8 + line_row;     // the lane's channel of a reduced pair of rows
+  if constexpr (EPI == kRowScale) {
+#pragma unroll
+    for (int m = 0; m < MAXM; ++m) {
+      int p0 = 0, p1 = 0;
+#pragma unroll
+      for (int i = 0; i < DOUBLES; ++i) p0 = dot(b[i][0], a[m][i], p0), p1 = dot(b[i][1], a[m][i], p1);
+      int sum = (odd ? p1 : p0) + dpp_i<kDppQuadXor1>(odd ? p0 : p1);
+      sum += dpp_i<kDppQuadXor2>(sum);
+      sum += dpp_i<kDppRowHalfMirror>(dpp_i<kDppQuadXor1>(sum));   // (lane ^ 6: the other four of the row)
+      if ((lane & 6) == 0) red[(wave * MAXM + m) * 16 + n] = sum;
+    }
+  } else {
+    static_assert(DOUBLES % 2 == 0, "two double steps at a time");
+#pragma unroll
+    for (int i = 0; i < DOUBLES; i += 2)
+#pragma unroll
+      for (int m = 0; m < MAXM; ++m) {
+        // four parts of four lanes: lane k of them gets part k, rows line_row and 8 + line_row of either double step
+        const int p0 = dot(b[i][0], a[m][i], 0), p1 = dot(b[i][1], a[m][i], 0), p2 = dot(b[i + 1][0], a[m][i + 1], 0),
+                  p3 = dot(b[i + 1][1], a[m][i + 1], 0);
+        const int x = (odd ? p1 : p0) + dpp_i<kDppQuadXor1>(odd ? p0 : p1), y = (odd ? p3 : p2) + dpp_i<kDppQuadXor1>(odd ? p2 : p3);
+        const int sum = (high ? y : x) + dpp_i<kDppQuadXor2>(high ? x : y);
+        const int g = 2 * (wave + (i + (high ? 1 : 0)) * kWaves) + (piece >> 2);
+        if (g < KT) ((float*)red)[(g * MAXM + m) * 16 + n] = (float)sum;
+      }
+    wait_vmcnt<0>();                           // the scales
+  }
+  __syncthreads();
+
+  const int gn = w.n0 + fn;
+  if (wave > 0 || fm >= p.M || gn >= w.N) return;
+  if constexpr (EPI == kRowScale) {
+    int sum = 0;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) sum += red[(v * MAXM + fm) * 16 + fn];
+    store_f16(p, w, fm, gn, (_Float16)round_here((float)sum * (s_a * s_b)));
+  } else {
+    const float* v = (const float*)red + fm * 16 + fn;
+    const int pitch = scale_pitch(KT);
+    float out;
+    if (p.a_cols == 1) out = round_here(fold_groups<MAXM * 16, true>(v, nullptr, table + fn * pitch, KT)) * s_a;
+    else out = fold_groups<MAXM * 16, false>(v, table + fm * pitch, table + (p.M + fn) * pitch, KT);
+    store_f16(p, w, fm, gn, (_Float16)round_here(out));
+  }
+}
+
+template <int MAXM, int DOUBLES, int EPI>
+int launch_dot(const GemmArgs& a, hipStream_t stream) {
+  const int KT = a.K >> 7;
+  const size_t smem = EPI == kGroupScale ? (size_t)KT * MAXM * 64 + scale_table_dwords(KT) * 4 : (size_t)kWaves * MAXM * 64;
+  static_assert(EPI != kGroupScale || (2 * DOUBLES * kWaves) * MAXM * 64 + scale_table_dwords(2 * DOUBLES * kWaves) * 4 <= 64 * 1024,
+                "fits the default dynamic LDS limit");
+  DotArgs d{a.A, a.As, a.R, a.M, a.K, a.a_cols, a.b_cols, {}};
+  int blocks = 0;
+  for (int s = 0; s < kMaxGemmSegments; ++s) {
+    d.seg[s].tile0 = 0x7FFFFFFF;
+    if (s > 0 && s >= a.n_seg) continue;
+    d.seg[s] = s == 0 ? DotSegment{a.B, a.Bs, (__half*)a.D, a.N, 0}
+                      : DotSegment{a.seg_B[s], a.seg_Bs[s], (__half*)a.seg_D[s], a.seg_N[s], blocks};
+    blocks += (d.seg[s].N + 15) / 16;
+  }
+  hipLaunchKernelGGL((gemm_i4_dot_kernel<MAXM, DOUBLES, EPI>), dim3(blocks), dim3(kWaves * 64), smem, stream, d);
+  return check_launch("gemm_i4_dot");
+}
+template <int MAXM, int EPI>
+int launch_dot(const GemmArgs& a, hipStream_t stream) {
+  const int steps = (a.K + 256 * kWaves - 1) / (256 * kWaves);   // double steps of a wave
+  if (steps <= 2) return launch_dot<MAXM, 2, EPI>(a, stream);
+  if (steps <= 4) return launch_dot<MAXM, 4, EPI>(a, stream);
+  if (steps <= 6) return launch_dot<MAXM, 6, EPI>(a, stream);
+  return launch_dot<MAXM, 8, EPI>(a, stream);
+}
+template <int EPI>
+int launch_dot(const GemmArgs& a, hipStream_t stream) {
+  return a.M == 1 ? launch_dot<1, EPI>(a, stream) : a.M == 2 ? launch_dot<2, EPI>(a, stream) : launch_dot<4, EPI>(a, stream);
+}
+
 }  // namespace
+
+// Up to four tokens; more than two up to K = 8192, beyond which their codes take the registers of the weights in flight (four tokens 11008
+// x 4096 7.2 / 8.8 / 8.8 -> 7.8 / 9.3 / 9.1; two 7.1 / 8.9 / 9.4 -> 6.8 / 8.2 / 8.3).
+bool gemm_dot_supports(const GemmArgs& a, int epi, int group) {
+  return a.M > 0 && a.M <= 4 && a.K <= 16384 && (epi == kRowScale || (epi == kGroupScale && group == 128)) && (a.M <= 2 || a.K <= 8192);
+}
+
+int gemm_dot_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
+  return epi == kRowScale ? launch_dot<kRowScale>(a, stream) : launch_dot<kGroupScale>(a, stream);
+}
 
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group) {
   if (a.M <= 0 || a.M > kDecodeMaxM) return false;

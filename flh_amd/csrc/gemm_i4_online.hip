@@ -18,7 +18,7 @@
 // HBM: with the requests in the old order, 16 x 16 x 64 products and half lines -> these requests -> dot products -> whole lines
 // past the caches (quantiser and GEMM in two launches):
 //   rotation, 4096 x 4096 6.2 -> 5.3 -> 4.6 -> 3.7 (8.1);  norm and residual, 6144 x 4096 9.9 -> 7.6 -> 6.8 -> 6.2 (10.7);
-//   the same, 28672 x 4096 26.3 -> 19.7 -> 17.6 -> 15.6 (18.7)
+//   the same, 28672 x 4096 26.3 -> 19.7 -> 17.6 -> 15.6 (18.7), 15.0 with tiles a round of workgroups apart instead of side by side
 // Norm and groups, two launches -> one: 6144 x 4096 one token 9.7 -> 5.0, four 9.9 -> 7.2; 22016 x 4096 16.0 -> 11.5, 16.6 -> 14.6.
 #include "gemm_i4.h"
 #include "group_codes.h"
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const Onlin
 
   // tile t of the workgroup: its weights
   auto tile = [&](int t) {
-    const int block = min((int)blockIdx.x * T + t, p.tiles - 1);
+    const int block = min((int)(blockIdx.x + t * gridDim.x), p.tiles - 1);
     OnlineTile w{p.seg[0].B, p.seg[0].Bs, p.seg[0].D, p.seg[0].N, block * 16};
 #pragma unroll
     for (int s = 1; s < kMaxGemmSegments; ++s)
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const Onlin
         return PRO == kNormGroup ? out : round_here(out) * __half2float(tok[m]);
       }
     };
-    if (m < M && (int)blockIdx.x * T + t < p.tiles) {
+    if (m < M && (int)(blockIdx.x + t * gridDim.x) < p.tiles) {
       const OnlineTile w = tile(t);
       const int n = w.n0 + r;
       if (n < w.N) ((_Float16*)w.D)[(size_t)m * w.N + n] = (_Float16)round_here(value());
@@ -363,26 +363,29 @@ int launch_kernel(const OnlineArgs& a, hipStream_t stream) {
   return check_launch("gemm_i4_online");
 }
 
-template <int EPI, int PRO, int T>
-int launch(const OnlineArgs& a, hipStream_t stream) {
-  if (a.M == 1) return launch_kernel<EPI, PRO, T, 1>(a, stream);
-  if (a.M == 2) return launch_kernel<EPI, PRO, T, 2>(a, stream);
-  if constexpr (PRO == kNormGroup)
-    if (a.M > 4) return launch_kernel<EPI, PRO, T, kGroupMaxTokens>(a, stream);
-  return launch_kernel<EPI, PRO, T, 4>(a, stream);
-}
-
 // as many tiles per workgroup as leave one workgroup to a compute unit, at most eight
-template <int EPI, int PRO>
+template <int EPI, int PRO, int MAXM>
 int launch_by_tiles(const OnlineArgs& a, hipStream_t stream) {
   const int per = (a.tiles + 255) / 256;
-  if (per <= 1) return launch<EPI, PRO, 1>(a, stream);
-  if (per == 2) return launch<EPI, PRO, 2>(a, stream);
-  if (per == 3) return launch<EPI, PRO, 3>(a, stream);
-  if (per == 4) return launch<EPI, PRO, 4>(a, stream);
-  if (per <= 6) return launch<EPI, PRO, 6>(a, stream);
-  return launch<EPI, PRO, 8>(a, stream);
+  if (per <= 1) return launch_kernel<EPI, PRO, 1, MAXM>(a, stream);
+  if (per == 2) return launch_kernel<EPI, PRO, 2, MAXM>(a, stream);
+  if constexpr (MAXM <= 2 || PRO == kNormGroup) {      // (more tokens to rotate than two: the callers' rules stop earlier)
+    if (per == 3) return launch_kernel<EPI, PRO, 3, MAXM>(a, stream);
+    if (per == 5) return launch_kernel<EPI, PRO, 5, MAXM>(a, stream);
+    if (per == 6) return launch_kernel<EPI, PRO, 6, MAXM>(a, stream);
+    if (per == 7) return launch_kernel<EPI, PRO, 7, MAXM>(a, stream);
+  }
+  return per <= 4 ? launch_kernel<EPI, PRO, 4, MAXM>(a, stream) : launch_kernel<EPI, PRO, 8, MAXM>(a, stream);
 }
+template <int EPI, int PRO>
+int launch(const OnlineArgs& a, hipStream_t stream) {
+  if (a.M == 1) return launch_by_tiles<EPI, PRO, 1>(a, stream);
+  if (a.M == 2) return launch_by_tiles<EPI, PRO, 2>(a, stream);
+  if constexpr (PRO == kNormGroup)
+    if (a.M > 4) return launch_by_tiles<EPI, PRO, kGroupMaxTokens>(a, stream);
+  return launch_by_tiles<EPI, PRO, 4>(a, stream);
+}
+
 struct OnlineCall {
   const flh_half *x, *add, *weight;
   flh_half* sum_out;
@@ -420,13 +423,13 @@ int online_checked(const char* who, const OnlineCall& call, int count, const uin
     a.tiles += ((int)N[s] + 15) / 16;
   }
   hipStream_t st = (hipStream_t)stream;
-  if (call.groups) return launch_by_tiles<kGroupScale, kNormGroup>(a, st);
+  if (call.groups) return launch<kGroupScale, kNormGroup>(a, st);
   if (b_cols == 1) {
-    if (!call.norm) return launch_by_tiles<kRowScale, kRotate>(a, st);
-    return call.add ? launch_by_tiles<kRowScale, kAddNormRotate>(a, st) : launch_by_tiles<kRowScale, kNormRotate>(a, st);
+    if (!call.norm) return launch<kRowScale, kRotate>(a, st);
+    return call.add ? launch<kRowScale, kAddNormRotate>(a, st) : launch<kRowScale, kNormRotate>(a, st);
   }
-  if (!call.norm) return launch_by_tiles<kTokenGroup, kRotate>(a, st);
-  return call.add ? launch_by_tiles<kTokenGroup, kAddNormRotate>(a, st) : launch_by_tiles<kTokenGroup, kNormRotate>(a, st);
+  if (!call.norm) return launch<kTokenGroup, kRotate>(a, st);
+  return call.add ? launch<kTokenGroup, kAddNormRotate>(a, st) : launch<kTokenGroup, kNormRotate>(a, st);
 }
 
 }  // namespace

@@ -534,17 +534,15 @@ bool stream_takes(const GemmArgs& a, int epi, int group) {
   return true;
 }
 
-// Up to 16 tokens (K = 4096; us, this kernel against the decode kernel; one scale per row / token scales / group scales).
-//  * Up to 16384 channels, one workgroup of 64 per compute unit: beyond 12288, where the decode kernel has more than three of
-//    its workgroups on one (one token: x 13312 8.1 / 8.8 / 9.0 against 9.2 / 9.5 / 9.5, x 12288 7.8 / 8.6 / 8.8 against 7.6 /
-//    8.5 / 8.3), with five or more tokens from 172 workgroups on (16 x 11008 7.8 / 8.6 / 8.8 against 9.7 / 9.9 / 9.9, 5 x 11008
-//    7.6 / 8.4 / 8.7 against 8.0 / 8.6 / 8.3; 16 x 6144 with group scales 8.3 against 7.5).
+// Up to 16 tokens (K = 4096; us, this kernel against the decode kernel; one scale per row / token scales / group scales; one to four
+// tokens come here only where the dot-product kernel does not take them: three and four beyond K = 8192, one and two beyond 16384).
+//  * Up to 16384 channels, one workgroup of 64 per compute unit, with five or more tokens from 172 workgroups on (16 x 11008
+//    7.8 / 8.6 / 8.8 against 9.7 / 9.9 / 9.9, 5 x 11008 7.6 / 8.4 / 8.7 against 8.0 / 8.6 / 8.3; 16 x 6144 with group scales 8.3
+//    against 7.5), with fewer beyond 12288, where the decode kernel has more than three of its workgroups on a compute unit.
 //  * Beyond, the compute units that get one workgroup more set the time and the decode kernel's grows with the channels: with
-//    few tokens only if the last round has enough workgroups (one token: x 17408 11.5 / 12.2 / 12.4 against 10.6 / 11.7 /
-//    10.7, x 22016 12.4 / 13.1 / 13.5 against 12.4 / 13.1 / 12.4, x 28672 13.9 / 14.7 / 15.0 against 15.2 / 16.0 / 14.6;
-//    5 x 18432 12.0 / 12.6 / 13.1 against 12.3 / 11.9 / 11.3, 8 x 18432 12.1 / 12.9 / 13.1 against 13.1 / 12.5 / 12.1).
-//    Not where the decode kernel's tiles of every group leave a compute unit one workgroup (one token x 22016, K = 11008,
-//    token scales: 30 against 41).
+//    few tokens only if the last round has enough workgroups (5 x 18432 12.0 / 12.6 / 13.1 against 12.3 / 11.9 / 11.3, 8 x 18432
+//    12.1 / 12.9 / 13.1 against 13.1 / 12.5 / 12.1).  Not where the decode kernel's tiles of every group leave a compute unit one
+//    workgroup.
 bool takes_few_tokens(const GemmArgs& a, int epi, long columns) {
   const bool row = epi == kRowScale, token = a.a_cols == 1;
   if (columns <= 16384 || a.M > (row ? 4 : token ? 6 : 8) || (!row && a.K > 8192))

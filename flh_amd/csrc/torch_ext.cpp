@@ -537,10 +537,10 @@ std::vector<Tensor> rotate_quantize_gemm_i4_multi(const Tensor& x, const std::ve
 }
 
 // RMSNorm(x [+ add]), rotation, quantiser and up to four GEMMs: {x + add or nothing, [fp16 [M, N_s] ...]}.  Every workgroup
-// of the one launch repeats the norm and the rotation: for one and two tokens that is hidden behind the weights, up to the eight
-// tiles of 16 channels that a workgroup has room for (us, token scales, one launch / two: one token 4096 x 4096 5.0 / 9.0, x 6144 6.2 /
-// 10.1, x 12288 8.4 / 11.8, x 28672 15.6 / 18.7; two x 4096 6.8 / 9.1, x 12288 10.1 / 11.9, x 28672 17.5 / 18.3).  Three tokens
-// are rotated in two turns and don't gain at any width (x 4096 11.1 / 9.1): the quantiser's launch and the GEMM's, the same bits.
+// of the one launch repeats the norm and the rotation.  One token's are hidden behind the weights, up to the eight tiles of 16
+// channels that a workgroup has room for (us, token scales, one launch / two: x 6144 6.0 / 8.1, x 12288 8.1 / 9.9, x 22016 12.7 / 13.2,
+// x 28672 15.0 / 15.2); two tokens' up to two tiles (x 6144 7.8 / 8.7, x 12288 10.1 / 10.0, x 22016 14.8 / 13.3).  Three are rotated in
+// two turns and don't gain at any width: the quantiser's launch and the GEMM's, the same bits.
 constexpr int64_t kOnlineChannels = 8 * 16 * 256;
 
 std::tuple<c10::optional<Tensor>, std::vector<Tensor>> rmsnorm_rotate_quantize_gemm_i4_multi(
@@ -581,7 +581,7 @@ std::tuple<c10::optional<Tensor>, std::vector<Tensor>> rmsnorm_rotate_quantize_g
   const flh_half* w = weight.has_value() ? h(*weight) : nullptr;
   Launch l(x);
   // (a weight that the one launch refuses for its alignment is refused at every size)
-  if ((M <= 2 && channels <= (size_t)kOnlineChannels) || ((uintptr_t)w & 15)) {
+  if ((M == 1 && channels <= (size_t)kOnlineChannels) || (M == 2 && channels <= 8192) || ((uintptr_t)w & 15)) {
     ok(flh_rmsnorm_rotate_quant_gemm_i4_o16_multi(h(x), add.has_value() ? h(*add) : nullptr, total.has_value() ? hm(*total) : nullptr,
                                                   w, (float)eps, count, b, bs, d, n, M, K, cols, stream_of(x)));
     return {total, Ds};
@@ -846,8 +846,9 @@ c10::optional<Tensor> linear_online_i4(const Tensor& x, const Tensor& w, const T
   const int64_t cols = w_scale.numel() / N;
   Launch l(x);
   // one launch while the rotation that every workgroup repeats costs less than a launch (us, one launch / two: one token x 4096 3.7 /
-  // 8.1, x 14336 8.6 / 12.0; two 4.9 / 8.2, 9.5 / 12.0; four x 4096 7.4 / 8.4, but x 14336 12.7 / 12.1)
-  if (M <= (N <= 4096 ? 4 : 2) && N <= kOnlineChannels && K == 4096 && mode == FLH_HAD_F32 && (cols == 1 || (group == 128 && cols == 32))) {
+  // 6.4, x 14336 8.5 / 9.9; two 4.9 / 7.0, 9.5 / 10.2; three 7.3 / 7.2)
+  if ((M == 1 ? N <= kOnlineChannels : M == 2 && N <= 16384) && K == 4096 && mode == FLH_HAD_F32 &&
+      (cols == 1 || (group == 128 && cols == 32))) {
     Tensor D = empty_rows(x, N, x.options());
     ok(flh_rotate_quant_gemm_i4_o16(h(x), u8(w), h(w_scale), hm(D), M, N, K, (int)cols, stream_of(x)));
     return D;

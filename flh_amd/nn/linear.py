@@ -259,8 +259,8 @@ class LinearFLH(torch.nn.Module):
         """fp16 activations [..., K] -> fp16 [..., N] with the activation side done here: whole-row rotation
         (`hadamard`: as in rotate_and_quantize_i4), one symmetric int4 scale per token, then the GEMM -- the
         online-Hadamard linear of the reference's benchmarks (benchmark/nn/benchmark_linear_flh.py:139-222), which
-        has no module of its own there.  One or two tokens of K = 4096 (four up to 4096 channels) with the
-        bit-exact rotation take the single-launch decode path; the outputs are the same bits either way."""
+        has no module of its own there.  One token of K = 4096 (up to 32768 channels; two up to 16384) with
+        the bit-exact rotation takes the single-launch decode path; the outputs are the same bits either way."""
         ops = _pkg._CUDA
         buf, mode = self._buffers, -1 if hadamard is True else self._ONLINE_MODES.get(hadamard)
         if mode is not None and buf.get("w_packed") is not None and buf.get("w_scale") is not None:
@@ -274,7 +274,7 @@ class LinearFLH(torch.nn.Module):
         w = self.w_packed.view(self.out_features, self.in_features // 2)
         w_scale = self.w_scale.view(self.out_features, -1)
         group = self.weight_group_size if self.weight_group_size > 0 else (self.in_group_size or 128)
-        fusable = (0 < rows.size(0) <= (4 if self.out_features <= 4096 else 2) and self.out_features <= 32768
+        fusable = ((rows.size(0) == 1 and self.out_features <= 32768 or rows.size(0) == 2 and self.out_features <= 16384)
                    and self.in_features == 4096 and hadamard in (True, "exact")
                    and (w_scale.size(1) == 1 or (group == 128 and w_scale.size(1) == 32)))
         if fusable:
