@@ -36,6 +36,7 @@ rope_kv_cache_ = _ext.rope_kv_cache_
 rotate_quantize_gemm_i4 = _ext.rotate_quantize_gemm_i4
 rotate_quantize_gemm_i4_multi = _ext.rotate_quantize_gemm_i4_multi
 rmsnorm_rotate_quantize_gemm_i4_multi = _ext.rmsnorm_rotate_quantize_gemm_i4_multi
+rmsnorm_group_quantize_gemm_i4_multi = _ext.rmsnorm_group_quantize_gemm_i4_multi
 linear_i4 = _ext.linear_i4
 linear_online_i4 = _ext.linear_online_i4
 quantize_groups = _ext.quantize_groups

@@ -696,11 +696,13 @@ def decode_attention(q, k_cache, v_cache, kv_len, scale=None, workspace=None):
     return out
 
 
-def decode_attention_rope(q, k_new, v_new, cos, sin, positions, k_cache, v_cache, kv_len, scale=None, workspace=None):
+def decode_attention_rope(q, k_new, v_new, cos, sin, positions, k_cache, v_cache, kv_len, scale=None, workspace=None,
+                          quantize=False):
     """decode_attention with the rotary embedding and the cache write of the new token inside: q [B, Hq, d], k_new /
     v_new [B, Hkv, d] fp16 as projected (not rotated), cos / sin [1, d] or [d] fp16 of the new position, positions (int64
     CUDA tensor, first element = the cache slot of the new token, < kv_len) -> [B, Hq, d] fp16.  k_cache / v_cache receive
-    the rotated key and the value at that slot (the bytes rope_kv_cache_ would write); q is not modified."""
+    the rotated key and the value at that slot (the bytes rope_kv_cache_ would write); q is not modified.
+    quantize (d = 128): (codes [B, Hq * 64] u8, scales [B, Hq] fp16) of quant_and_pack_i4_gs on that output, in the same launches."""
     for t_ in (q, k_new, v_new, cos, sin, k_cache, v_cache):
         _check(t_.is_cuda and t_.dtype == torch.float16 and t_.is_contiguous() and t_.device == q.device,
                "tensors must be contiguous float16 CUDA tensors on one device")
@@ -715,20 +717,27 @@ def decode_attention_rope(q, k_new, v_new, cos, sin, positions, k_cache, v_cache
     _check(d in (64, 128), "head_dim must be 64 or 128")
     _check(Hkv > 0 and Hq % Hkv == 0 and Hq // Hkv in (1, 2, 4, 8), "Hq / Hkv must be 1, 2, 4 or 8")
     _check(0 < kv_len <= max_len, "kv_len must be in 1 .. max_len")
-    out = torch.empty_like(q)
+    if quantize:
+        _check(d == 128, "quantize: head_dim must be 128")
+        codes = torch.empty((B, Hq * 64), dtype=torch.uint8, device=q.device)
+        scales = torch.empty((B, Hq), dtype=torch.float16, device=q.device)
+        out, result = (codes, scales), (codes, scales)
+    else:
+        result = torch.empty_like(q)
+        out = (result,)
     if B == 0:
-        return out
+        return result
     need = int(_lib.load().flh_decode_attention_workspace_bytes(B, Hq, d, int(kv_len)))
     if workspace is None:
         workspace = _default_attention_workspace(q, need)
     else:
         _check(workspace.is_cuda and workspace.dtype == torch.uint8 and workspace.is_contiguous()
                and workspace.device == q.device and workspace.numel() >= need, f"workspace: {need} bytes of uint8 needed")
-    _run("flh_decode_attention_rope_f16", q.device, q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), cos.data_ptr(),
-         sin.data_ptr(), positions.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), B, Hq, Hkv, d,
-         int(kv_len), max_len, float(scale if scale is not None else d ** -0.5), workspace.data_ptr(), workspace.numel(),
-         _stream(q))
-    return out
+    _run("flh_decode_attention_rope_group_quant_i4" if quantize else "flh_decode_attention_rope_f16", q.device, q.data_ptr(),
+         k_new.data_ptr(), v_new.data_ptr(), cos.data_ptr(), sin.data_ptr(), positions.data_ptr(), k_cache.data_ptr(),
+         v_cache.data_ptr(), *(t.data_ptr() for t in out), B, Hq, Hkv, d, int(kv_len), max_len,
+         float(scale if scale is not None else d ** -0.5), workspace.data_ptr(), workspace.numel(), _stream(q))
+    return result
 
 
 def _check_rows(x, width):

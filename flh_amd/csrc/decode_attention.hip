@@ -10,6 +10,7 @@
 // key / value head served by the same read.
 #include <atomic>
 
+#include "group_codes.h"
 #include "lane_ops.h"
 
 namespace flh {
@@ -217,10 +218,14 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_partial_kernel(
 // one workgroup of four waves per (sequence, query head): the chunks' partials -> fp16 output.  Every wave reads all
 // maxima and sums (lane s: chunk s, 64 chunks per pass; two wave reductions) and accumulates the weighted values of
 // every fourth chunk with the chunk's weight read from its lane; the four waves' sums meet in LDS.
-template <int D>
+// QUANT (heads of 128 channels): the head is a group of the quantiser that follows, so its codes and scale leave instead, the
+// bytes of the group quantiser on the fp16 output: a launch of 4.6 us less in a decode step's layer.
+template <int D, bool QUANT = false>
 __global__ __launch_bounds__(256) void decode_attention_combine_kernel(const float* __restrict__ partials,
                                                                        __half* __restrict__ out, uint32_t rep,
-                                                                       uint32_t splits) {
+                                                                       uint32_t splits, uint8_t* __restrict__ codes,
+                                                                       __half* __restrict__ scales) {
+  static_assert(!QUANT || D == 128, "a head is a group");
   __shared__ float acc[4][2][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -263,13 +268,35 @@ __global__ __launch_bounds__(256) void decode_attention_combine_kernel(const flo
   const float inv = l > 0.f ? 1.0f / l : 0.f;
   if constexpr (D == 128) {
     const h2 r = {(_Float16)(a0 * inv), (_Float16)(a1 * inv)};
-    *(h2*)(out + (size_t)bhq * D + 2 * lane) = r;
+    if constexpr (QUANT) {
+      const unsigned y = __builtin_bit_cast(unsigned, r);
+      const h2 mag = __builtin_bit_cast(h2, y & 0x7FFF7FFFu);
+      float m = __builtin_fmaxf((float)mag[0], (float)mag[1]);
+      m = __builtin_fmaxf(m, lane_xor_f<16>(m));
+      m = __builtin_fmaxf(m, lane_xor_f<32>(m));
+      const GroupScale s = group_scale<16>(m);             // (and over the sixteen lanes of a row)
+      // four adjacent lanes hold the eight values of a dword of codes
+      const unsigned y0 = dpp_i<0x00>(y), y1 = dpp_i<0x55>(y), y2 = dpp_i<0xAA>(y), y3 = dpp_i<0xFF>(y);
+      const h2 hb = {(_Float16)65504.0f, (_Float16)65504.0f};
+      const unsigned w = s.careful ? nibbles8<true>(y0, y1, y2, y3, s.r, hb) : nibbles8<false>(y0, y1, y2, y3, s.r, hb);
+      if ((lane & 3) == 0) *(unsigned*)(codes + (size_t)bhq * (D / 2) + lane) = w;
+      if (lane == 0) scales[bhq] = __builtin_bit_cast(__half, s.s);
+    } else {
+      *(h2*)(out + (size_t)bhq * D + 2 * lane) = r;
+    }
   } else {
     out[(size_t)bhq * D + lane] = __float2half(a0 * inv);
   }
 }
 
 constexpr int kChunk = 64;
+
+// where the result goes: fp16, or (heads of 128) int4 codes and a scale per head
+struct AttentionOut {
+  __half* out;
+  uint8_t* codes;
+  __half* scales;
+};
 
 // the new token's inputs of the variant with the rotary embedding and the cache write inside (all null without it)
 struct NewToken {
@@ -278,7 +305,7 @@ struct NewToken {
 };
 
 template <int D, int REP>
-int launch_attention(const __half* q, __half* k, __half* v, __half* out, float* partials, uint32_t B, uint32_t Hkv,
+int launch_attention(const __half* q, __half* k, __half* v, const AttentionOut& out, float* partials, uint32_t B, uint32_t Hkv,
                      uint32_t kv_len, uint32_t max_len, float scale, const NewToken& nt, hipStream_t stream) {
   const uint32_t splits = (kv_len + kChunk - 1) / kChunk;
   const dim3 grid(B * Hkv * splits), block(kAttnThreads);
@@ -289,8 +316,15 @@ int launch_attention(const __half* q, __half* k, __half* v, __half* out, float* 
   if (nt.k) go(decode_attention_partial_kernel<D, REP, kChunk, true>);
   else go(decode_attention_partial_kernel<D, REP, kChunk, false>);
   if (int rc = check_launch("decode_attention (partials)")) return rc;
-  hipLaunchKernelGGL((decode_attention_combine_kernel<D>), dim3(B * Hkv * REP), dim3(256), 0, stream, partials, out,
-                     (uint32_t)REP, splits);
+  auto combine = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(B * Hkv * REP), dim3(256), 0, stream, partials, out.out, (uint32_t)REP, splits, out.codes, out.scales);
+  };
+  if constexpr (D == 128)
+    if (out.codes) {
+      combine(decode_attention_combine_kernel<D, true>);
+      return check_launch("decode_attention (combine)");
+    }
+  combine(decode_attention_combine_kernel<D>);
   return check_launch("decode_attention (combine)");
 }
 
@@ -305,11 +339,11 @@ extern "C" size_t flh_decode_attention_workspace_bytes(uint32_t B, uint32_t Hq, 
 }
 
 namespace {
-int decode_attention_checked(const flh_half* q, flh_half* k_cache, flh_half* v_cache, flh_half* out, uint32_t B, uint32_t Hq,
+int decode_attention_checked(const flh_half* q, flh_half* k_cache, flh_half* v_cache, const AttentionOut& out, uint32_t B, uint32_t Hq,
                              uint32_t Hkv, uint32_t head_dim, uint32_t kv_len, uint32_t max_len, float scale,
                              void* workspace, size_t workspace_bytes, const NewToken& nt, void* stream) {
-  if (!q || !k_cache || !v_cache || !out) return fail(FLH_EINVAL, "decode_attention: null pointer");
-  if (misaligned16(q, k_cache, v_cache, out)) return fail(FLH_EINVAL, "decode_attention: tensors must be 16-byte aligned");
+  if (!q || !k_cache || !v_cache || !(out.out || (out.codes && out.scales))) return fail(FLH_EINVAL, "decode_attention: null pointer");
+  if (misaligned16(q, k_cache, v_cache, out.out, out.codes)) return fail(FLH_EINVAL, "decode_attention: tensors must be 16-byte aligned");
   if (head_dim != 128 && head_dim != 64) return fail(FLH_EINVAL, "decode_attention: head_dim (%u) must be 64 or 128", head_dim);
   if (Hkv == 0 || Hq % Hkv) return fail(FLH_EINVAL, "decode_attention: %u query heads do not divide over %u key / value heads", Hq, Hkv);
   const uint32_t rep = Hq / Hkv;
@@ -323,10 +357,10 @@ int decode_attention_checked(const flh_half* q, flh_half* k_cache, flh_half* v_c
     return fail(FLH_EINVAL, "decode_attention: the workspace has %zu bytes, this call needs %zu", workspace_bytes, need);
   if ((uint64_t)B * Hkv * ((kv_len + kChunk - 1) / kChunk) > 0x7FFFFFFFull) return fail(FLH_EINVAL, "decode_attention: too many chunks");
   const __half* qh = (const __half*)q;
-  __half *kh = (__half*)k_cache, *vh = (__half*)v_cache, *oh = (__half*)out;
+  __half *kh = (__half*)k_cache, *vh = (__half*)v_cache;
   float* ws = (float*)workspace;
   hipStream_t st = (hipStream_t)stream;
-#define FLH_ATTN(D, R) return launch_attention<D, R>(qh, kh, vh, oh, ws, B, Hkv, kv_len, max_len, scale, nt, st)
+#define FLH_ATTN(D, R) return launch_attention<D, R>(qh, kh, vh, out, ws, B, Hkv, kv_len, max_len, scale, nt, st)
   if (head_dim == 128) {
     switch (rep) {
       case 1: FLH_ATTN(128, 1);
@@ -350,21 +384,42 @@ extern "C" int flh_decode_attention_f16(const flh_half* q, const flh_half* k_cac
                                         uint32_t max_len, float scale, void* workspace, size_t workspace_bytes,
                                         void* stream) {
   // (without a new token the kernel only reads the caches)
-  return decode_attention_checked(q, (flh_half*)k_cache, (flh_half*)v_cache, out, B, Hq, Hkv, head_dim, kv_len, max_len, scale,
+  return decode_attention_checked(q, (flh_half*)k_cache, (flh_half*)v_cache, AttentionOut{(__half*)out, nullptr, nullptr}, B, Hq, Hkv, head_dim, kv_len, max_len, scale,
                                   workspace, workspace_bytes, NewToken{nullptr, nullptr, nullptr, nullptr, nullptr}, stream);
 }
+
+namespace {
+int decode_attention_rope_checked(const flh_half* q, const flh_half* k_new, const flh_half* v_new, const flh_half* cos, const flh_half* sin,
+                                  const int64_t* positions, flh_half* k_cache, flh_half* v_cache, const AttentionOut& out, uint32_t B,
+                                  uint32_t Hq, uint32_t Hkv, uint32_t head_dim, uint32_t kv_len, uint32_t max_len, float scale,
+                                  void* workspace, size_t workspace_bytes, void* stream) {
+  if (!k_new || !v_new || !cos || !sin || !positions) return fail(FLH_EINVAL, "decode_attention (rotary): null pointer");
+  if (misaligned16(k_new, v_new, cos, sin)) return fail(FLH_EINVAL, "decode_attention (rotary): tensors must be 16-byte aligned");
+  return decode_attention_checked(q, k_cache, v_cache, out, B, Hq, Hkv, head_dim, kv_len, max_len, scale, workspace, workspace_bytes,
+                                  NewToken{(const __half*)k_new, (const __half*)v_new, (const __half*)cos, (const __half*)sin,
+                                           (const long long*)positions}, stream);
+}
+}  // namespace
 
 extern "C" int flh_decode_attention_rope_f16(const flh_half* q, const flh_half* k_new, const flh_half* v_new,
                                              const flh_half* cos, const flh_half* sin, const int64_t* positions,
                                              flh_half* k_cache, flh_half* v_cache, flh_half* out, uint32_t B, uint32_t Hq,
                                              uint32_t Hkv, uint32_t head_dim, uint32_t kv_len, uint32_t max_len, float scale,
                                              void* workspace, size_t workspace_bytes, void* stream) {
-  if (!k_new || !v_new || !cos || !sin || !positions) return fail(FLH_EINVAL, "decode_attention (rotary): null pointer");
-  if (misaligned16(k_new, v_new, cos, sin)) return fail(FLH_EINVAL, "decode_attention (rotary): tensors must be 16-byte aligned");
-  return decode_attention_checked(q, k_cache, v_cache, out, B, Hq, Hkv, head_dim, kv_len, max_len, scale, workspace,
-                                  workspace_bytes,
-                                  NewToken{(const __half*)k_new, (const __half*)v_new, (const __half*)cos, (const __half*)sin,
-                                           (const long long*)positions}, stream);
+  return decode_attention_rope_checked(q, k_new, v_new, cos, sin, positions, k_cache, v_cache, AttentionOut{(__half*)out, nullptr, nullptr},
+                                       B, Hq, Hkv, head_dim, kv_len, max_len, scale, workspace, workspace_bytes, stream);
+}
+
+extern "C" int flh_decode_attention_rope_group_quant_i4(const flh_half* q, const flh_half* k_new, const flh_half* v_new,
+                                                        const flh_half* cos, const flh_half* sin, const int64_t* positions,
+                                                        flh_half* k_cache, flh_half* v_cache, uint8_t* q_packed, flh_half* scales,
+                                                        uint32_t B, uint32_t Hq, uint32_t Hkv, uint32_t head_dim, uint32_t kv_len,
+                                                        uint32_t max_len, float scale, void* workspace, size_t workspace_bytes,
+                                                        void* stream) {
+  if (head_dim != 128) return fail(FLH_EINVAL, "decode_attention (quantised): head_dim (%u) must be 128, the group of the quantiser", head_dim);
+  return decode_attention_rope_checked(q, k_new, v_new, cos, sin, positions, k_cache, v_cache,
+                                       AttentionOut{nullptr, q_packed, (__half*)scales}, B, Hq, Hkv, head_dim, kv_len, max_len, scale,
+                                       workspace, workspace_bytes, stream);
 }
 
 // ---- the same for callers that cannot allocate ---------------------------------------------------------------------

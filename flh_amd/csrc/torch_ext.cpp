@@ -598,6 +598,58 @@ std::tuple<c10::optional<Tensor>, std::vector<Tensor>> rmsnorm_rotate_quantize_g
   return {total, Ds};
 }
 
+// RMSNorm(x), groups of 128 without rotation and up to four GEMMs with group scales: [fp16 [M, N_s] ...].  The quantiser is repeated by
+// every workgroup of the one launch and the tokens' products grow with it, so fewer channels for more tokens (us, one launch / two:
+// one token x 6144 5.0 / 7.8, x 28672 13.5 / 14.9; two x 28672 14.8 / 15.2; four x 16384 11.2 / 12.1, x 22016 14.7 / 14.4; five x 12288 10.9 /
+// 12.1; six 11.7 / 12.1, x 16384 13.7 / 13.4; eight x 6144 10.3 / 10.2).
+std::vector<Tensor> rmsnorm_group_quantize_gemm_i4_multi(const Tensor& x, const c10::optional<Tensor>& weight, double eps,
+                                                         const std::vector<Tensor>& Bs, const std::vector<Tensor>& B_scales) {
+  TORCH_CHECK(Bs.size() == B_scales.size() && !Bs.empty() && Bs.size() <= 4,
+              "one to four weight matrices, one scale tensor each");
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat16 && x.dim() == 2 && x.is_contiguous(),
+              "x must be a contiguous 2D float16 CUDA tensor");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M <= 8, "at most 8 tokens");
+  TORCH_CHECK(K == 4096, "K must be 4096");
+  if (weight.has_value())
+    TORCH_CHECK(weight->is_cuda() && weight->scalar_type() == torch::kFloat16 && weight->is_contiguous() &&
+                    weight->numel() == K && weight->device() == x.device(),
+                "weight must be a contiguous float16 CUDA tensor of K values");
+  std::vector<Tensor> Ds;
+  const uint8_t* b[4];
+  const flh_half* bs[4];
+  flh_half* d[4];
+  size_t n[4];
+  int64_t channels = 0;
+  for (size_t s = 0; s < Bs.size(); ++s) {
+    const Tensor &B = Bs[s], &S = B_scales[s];
+    TORCH_CHECK(B.is_cuda() && S.is_cuda() && B.device() == x.device() && S.device() == x.device(), "tensors must be on one device");
+    TORCH_CHECK(B.scalar_type() == torch::kUInt8 && B.dim() == 2 && B.is_contiguous() && B.size(1) * 2 == K && B.size(0) > 0,
+                "B must be a contiguous uint8 [N, K/2] tensor");
+    TORCH_CHECK(S.scalar_type() == torch::kFloat16 && S.is_contiguous() && S.dim() == 2 && S.size(0) == B.size(0) && S.size(1) == K / 128,
+                "B_scale must be a contiguous float16 [N, K/128] tensor");
+    Ds.push_back(torch::empty({M, B.size(0)}, x.options()));
+    b[s] = u8(B);
+    bs[s] = h(S);
+    d[s] = hm(Ds[s]);
+    n[s] = (size_t)B.size(0);
+    channels += B.size(0);
+  }
+  if (M == 0) return Ds;
+  const flh_half* w = weight.has_value() ? h(*weight) : nullptr;
+  Launch l(x);
+  const int64_t most = M <= 2 ? kOnlineChannels : M <= 4 ? 16384 : M <= 6 ? 12288 : 0;
+  if (channels <= most && ((uintptr_t)w & 15) == 0) {
+    ok(flh_rmsnorm_group_quant_gemm_i4_o16_multi(h(x), w, (float)eps, (int)Bs.size(), b, bs, d, n, M, K, stream_of(x)));
+    return Ds;
+  }
+  Tensor q = torch::empty({M, K / 2}, x.options().dtype(torch::kUInt8));
+  Tensor s = torch::empty({M, K / 128}, x.options());
+  ok(flh_rmsnorm_group_quant_i4(h(x), w, (uint8_t*)q.data_ptr(), hm(s), (uint32_t)M, (uint32_t)K, (float)eps, 128, 0, 1.0f, stream_of(x)));
+  ok(flh_gemm_i4_o16_multi(u8(q), h(s), (int)Bs.size(), b, bs, d, n, M, K, (int)(K / 128), (int)(K / 128), 128, stream_of(x)));
+  return Ds;
+}
+
 // ---- group kernels ------------------------------------------------------------------------------------------------
 void check_rows(const Tensor& x, int64_t width) {
   TORCH_CHECK(x.is_cuda(), "Input tensor must be on CUDA");
@@ -975,6 +1027,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_rotate_quantize_gemm_i4_multi", &rmsnorm_rotate_quantize_gemm_i4_multi, py::arg("x"), py::arg("add"),
         py::arg("weight"), py::arg("eps"), py::arg("Bs"), py::arg("B_scales"));
   m.def("linear_i4", &linear_i4);
+  m.def("rmsnorm_group_quantize_gemm_i4_multi", &rmsnorm_group_quantize_gemm_i4_multi, py::arg("x"), py::arg("weight"), py::arg("eps"),
+        py::arg("Bs"), py::arg("B_scales"));
   m.def("linear_online_i4", &linear_online_i4);
   m.def("quantize_groups", &quantize_groups);
   m.def("quantize_rows", &quantize_rows);

@@ -346,9 +346,8 @@ class W4A4DecoderLayer(torch.nn.Module):
         cache) -- or, when o_proj adds the residual in its epilogue (`fold_residual`, prefill sizes), (the stream after the
         block, None, cache)."""
         b, t, _ = x.shape
-        if (self.activation == "token" and self.fused and self.record is None and b * t <= 2 and self.hidden_size == 4096
-                and self._online_applies((self.q_proj, self.k_proj, self.v_proj))):
-            # decode: residual addition, norm, rotation, quantiser and the three projections in one launch, two where faster
+        if self._online_rows_apply((self.q_proj, self.k_proj, self.v_proj), b * t):
+            # decode: residual addition, norm, quantiser and the three projections in one launch, two where faster
             x, (qs, ks, vs) = self._norm_quant_project([self.q_proj, self.k_proj, self.v_proj], self.input_layernorm,
                                                        "input_layernorm", x, add)
         else:
@@ -365,11 +364,15 @@ class W4A4DecoderLayer(torch.nn.Module):
                 and positions is not None):
             # one new token against the cache: rotary embedding, cache write and chunked attention in two launches
             keys, values = kv_cache.tensors()
+            codes = self._attention_quantises(b)
             out = _ops().decode_attention_rope(qs.view(b, self.num_heads, self.head_dim),
                                                ks.view(b, self.num_kv_heads, self.head_dim),
                                                vs.view(b, self.num_kv_heads, self.head_dim), cos, sin, positions, keys,
                                                values, kv_cache.owner.kv_len,
-                                               workspace=kv_cache.owner.attention_workspace)
+                                               workspace=kv_cache.owner.attention_workspace, quantize=codes)
+            if codes:
+                q, s = out
+                return self._project_output(x, s.view(b, 1, -1), None, q.view(b, 1, -1), kv_cache, fold_residual)
             out = out.view(b, 1, self.hidden_size)
             cache = kv_cache
             past = kv_cache.owner.kv_len - 1
@@ -433,7 +436,19 @@ class W4A4DecoderLayer(torch.nn.Module):
         _attention returns them."""
         s, z, q = (self._token_quant("attn_out", out, consumers=(self.o_proj,)) if self.activation == "token"
                    else self._group_quant("attn_out", self.attn_quantizer2, out, (self.o_proj,)))
-        if fold_residual and self._residual_in_gemm(out.numel() // out.size(-1), self.o_proj):
+        return self._project_output(x, s, z, q, cache, fold_residual)
+
+    def _attention_quantises(self, rows):
+        """Whether the attention of one new token per sequence stores what attn_quantizer2 would make of its output: heads of one
+        group, and a quantiser that does no more."""
+        quantizer = self.attn_quantizer2
+        return (self.activation == "group" and self.fused and self.record is None and self.head_dim == 128 == self.act_group_size
+                and _stock_call(quantizer, ActQuantizer) and not quantizer.use_hadamard and not quantizer.per_token
+                and not self._group_six_bit_for((self.o_proj,), rows, self.hidden_size))
+
+    def _project_output(self, x, s, z, q, cache, fold_residual):
+        """o_proj on the quantised attention output; returns as _output_projection."""
+        if fold_residual and self._residual_in_gemm(q.numel() // q.size(-1), self.o_proj):
             # the residual addition in o_proj's epilogue; nothing is left pending
             return self.o_proj(q, s, z, x_is_packed=True, residual=x), None, cache
         y = self.o_proj(q, s, z, x_is_packed=True)
@@ -520,14 +535,29 @@ class W4A4DecoderLayer(torch.nn.Module):
         c = cols.pop()
         return c == 1 or (c == self.hidden_size // 128 and layers[0].weight_group_size == 128)
 
+    def _online_rows_apply(self, layers, rows):
+        """Whether `layers` take the launch with norm and quantiser inside: one or two tokens rotated as whole rows, up to eight in
+        groups (which of them by one launch and which by two, the operations know)."""
+        if not (self.fused and self.record is None and 0 < rows <= (2 if self.activation == "token" else 8)
+                and self.hidden_size == 4096 and self._online_applies(layers)):
+            return False
+        if self.activation == "token":
+            return True
+        return (self.act_group_size == 128 and all(l.w_scale.numel() > l.out_features for l in layers)
+                and not self._group_six_bit_for(layers, rows, self.hidden_size))
+
     def _norm_quant_project(self, layers, norm, norm_name, x, add):
-        """(x + add, outputs) of the residual addition, the norm, the whole-row quantiser and `layers`: one launch for one or two
-        tokens, the bits of the separate ones."""
+        """(x + add, outputs) of the residual addition, the norm, the quantiser and `layers`: one launch for few tokens, the bits of
+        the separate ones."""
         rows = x.numel() // x.size(-1)
+        weight = self._norm_weight16(norm_name, norm)
+        w = [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers]
+        scales = [l.w_scale.view(l.out_features, -1) for l in layers]
+        if self.activation == "group":
+            x = x if add is None else x + add
+            return x, _ops().rmsnorm_group_quantize_gemm_i4_multi(x.reshape(rows, -1).contiguous(), weight, norm.eps, w, scales)
         total, ys = _ops().rmsnorm_rotate_quantize_gemm_i4_multi(
-            x.reshape(rows, -1).contiguous(), None if add is None else add.reshape(rows, -1).contiguous(),
-            self._norm_weight16(norm_name, norm), norm.eps, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
-            [l.w_scale.view(l.out_features, -1) for l in layers])
+            x.reshape(rows, -1).contiguous(), None if add is None else add.reshape(rows, -1).contiguous(), weight, norm.eps, w, scales)
         return (x if total is None else total.view(x.shape)), ys
 
     def _swiglu_gemm_applies(self, rows):
@@ -567,8 +597,7 @@ class W4A4DecoderLayer(torch.nn.Module):
         after the block, None) when down_proj adds the residual in its epilogue (`fold_residual`, prefill sizes)."""
         rows = x.numel() // x.size(-1)
         pair = (self.gate_proj, self.up_proj)
-        if (self.activation == "token" and self.fused and self.record is None and 0 < rows <= 2 and self.hidden_size == 4096
-                and self._online_applies(pair)):
+        if self._online_rows_apply(pair, rows):
             x, (gate, up) = self._norm_quant_project(pair, self.post_attention_layernorm, "post_attention_layernorm", x, add)
             gate, up = gate.view(*x.shape[:-1], -1), up.view(*x.shape[:-1], -1)
         else:

@@ -404,6 +404,15 @@ int flh_decode_attention_rope_f16(const flh_half* q, const flh_half* k_new, cons
                                   flh_half* out, uint32_t B, uint32_t Hq, uint32_t Hkv, uint32_t head_dim, uint32_t kv_len,
                                   uint32_t max_len, float scale, void* workspace, size_t workspace_bytes, void* stream);
 
+/* ... with the int4 group quantiser that follows in the decoder layer (flh_group_quant_i4, groups of 128, no rotation, scale_mul 1)
+ * inside as well: heads of 128 channels are its groups.  q_packed [B, Hq * 64] codes and scales [B, Hq] instead of the fp16 output,
+ * the same bytes as the two calls. */
+int flh_decode_attention_rope_group_quant_i4(const flh_half* q, const flh_half* k_new, const flh_half* v_new, const flh_half* cos,
+                                             const flh_half* sin, const int64_t* positions, flh_half* k_cache, flh_half* v_cache,
+                                             uint8_t* q_packed, flh_half* scales, uint32_t B, uint32_t Hq, uint32_t Hkv,
+                                             uint32_t head_dim, uint32_t kv_len, uint32_t max_len, float scale, void* workspace,
+                                             size_t workspace_bytes, void* stream);
+
 /* flh_decode_attention_f16 for callers that cannot allocate device memory and have no workspace to hand over -- code
  * under stream capture, tight serving loops, harnesses that forbid allocation.  No counterpart in the reference.  It
  * allocates nothing: the partial results go to a static device array of flh_decode_attention_static_scratch_bytes()
