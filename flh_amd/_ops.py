@@ -334,11 +334,8 @@ def rmsnorm_rotate_quantize_gemm_i4_multi(x, add, weight, eps, Bs, B_scales):
     return total, Ds
 
 
-GROUP_GEMM_MAX_TOKENS = 8
-
-
 def rmsnorm_group_quantize_gemm_i4_multi(x, weight, eps, Bs, B_scales):
-    """RMSNorm(x) quantised in groups of 128 (no rotation) and up to four GEMMs in one launch: x [M, 4096] fp16 with M <= 8,
+    """RMSNorm(x) quantised in groups of 128 (no rotation) and up to four GEMMs in one launch: x [M, 4096] fp16 with M <= 4,
     weight [4096] fp16 or None, group scales [N, 32] -> [fp16 [M, N_s] ...]; the outputs are those of rmsnorm_and_quantize_i4_gs
     followed by gemm_i4_dequant_multi, bit for bit."""
     import ctypes
@@ -346,7 +343,7 @@ def rmsnorm_group_quantize_gemm_i4_multi(x, weight, eps, Bs, B_scales):
     _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
            "x must be a contiguous 2D float16 CUDA tensor")
     M, K = x.shape
-    _check(M <= GROUP_GEMM_MAX_TOKENS, "at most 8 tokens")
+    _check(M <= ROTATE_GEMM_MAX_TOKENS, "at most 4 tokens")
     _check(K in ROTATE_GEMM_WIDTHS, "K must be 4096")
     if weight is not None:
         _check(weight.is_cuda and weight.dtype == torch.float16 and weight.is_contiguous() and weight.numel() == K

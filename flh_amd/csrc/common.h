@@ -97,6 +97,12 @@ __device__ __forceinline__ void load_kib_to_lds16(const uint8_t* const (&g)[N], 
                  ::"s"(lds_base), "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]) : "memory", "m0");
 }
 
+// ... two, of data that is read once (non-temporal: it does not displace what the caches hold)
+__device__ __forceinline__ void load_kib_to_lds16_nt(const uint8_t* const (&g)[2], unsigned lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt\n\tglobal_load_lds_dwordx4 %2, off offset:1024 nt"
+               ::"s"(lds_base), "v"(g[0]), "v"(g[1]) : "memory", "m0");
+}
+
 // load_to_lds16 for data that is read once (non-temporal: it does not displace what the caches hold)
 __device__ __forceinline__ void load_to_lds16_nt(const void* gptr, unsigned lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(gptr) : "memory", "m0");

@@ -297,6 +297,154 @@ int launch_decode(const GemmArgs& a, hipStream_t stream) {
   return check_launch("gemm_i4_decode");
 }
 
+// Five to sixteen tokens (three and four where the kernel below ends): the kernel above with its weights by direct-to-LDS loads of whole lines, past the caches, that
+// every wave stages for itself: 2 KiB per double step, all of them requested at once; a wave waits for its own loads only.  A
+// step's sums (two groups of 1 KiB) take the place of its operands, so that the LDS of the tiles is that of the stages.
+// 16-byte piece c of row r sits at slot c ^ (r % 8): written lane after lane, and read without bank conflicts.
+// us, weights from HBM, half lines to registers -> this, one scale per row / token scales / group scales: five tokens 4096 x 4096 4.7 /
+// 5.1 / 5.1 -> 3.8 / 4.6 / 4.6, x 6144 6.1 / 6.6 / 6.4 -> 4.8 / 5.9 / 5.7; sixteen x 4096 5.1 / 5.4 / 5.4 -> 3.9 / 4.7 / 4.9, x 6144 7.1 /
+// 7.4 / 7.4 -> 5.5 / 6.2 / 6.3, 14336 x 4096 10.0 -> 9.5 with one scale per row.  Beyond 8192 channels the tokens' half lines, as many as
+// the weights' from sixteen tokens on, are what bounds it.
+template <int STEPS, int EPI>
+__global__ __launch_bounds__(kWaves * 64) void gemm_i4_lines_kernel(const GemmArgs p) {
+  extern __shared__ __align__(16) int red[];   // [wave][step][2 KiB]: operands, then the sums of two groups; then the scales
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, c = lane >> 4;
+  const DecodeWeights w = decode_weights(p, blockIdx.x);
+  const int Kb = p.K >> 1, KT = p.K >> 7, ND = (KT + 1) >> 1;
+  const int mine = (ND - wave + kWaves - 1) / kWaves;      // double steps of this wave, at most STEPS
+
+  unsigned* table = (unsigned*)red + kWaves * STEPS * 512;
+  if constexpr (EPI == kGroupScale) request_scales(p, w, table, KT, tid);
+  const FirstScales first = first_scales<EPI>(p, w, p.As, tid);
+  // (steps that the row does not have: the last one again, neither half of which is used)
+  v4i a[STEPS][2];
+  const uint8_t* arow = p.A + (size_t)min(r, p.M - 1) * Kb + c * 16;
+  auto step_at = [&](int i) { return min(wave + i * kWaves, ND - 1) * 128; };
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    const int at = step_at(i);
+    a[i][0] = *(const v4i*)(arow + at);
+    a[i][1] = *(const v4i*)(arow + (at + 64 < Kb ? at + 64 : at));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const unsigned stage = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int*)red + wave * STEPS * 2048;
+  const int line_row = lane >> 3, piece = ((lane & 7) ^ line_row) * 16;
+  const uint8_t* rows[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) rows[q] = w.B + (size_t)min(w.n0 + q * 8 + line_row, w.N - 1) * Kb;
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    const int at = step_at(i), byte = at + (at + piece < Kb ? piece : piece - 64);   // K = 128 * odd: the last line is half a line
+    const uint8_t* g[2] = {rows[0] + byte, rows[1] + byte - 1024};
+    load_kib_to_lds16_nt(g, stage + i * 2048);
+  }
+
+  v4i acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  static_for<STEPS>([&](auto index) {
+    constexpr int i = decltype(index)::value;
+    wait_vmcnt<2 * (STEPS - 1 - i)>();
+    asm volatile("" ::: "memory");
+    if (i < mine) {
+      int* area = red + (wave * STEPS + i) * 512;
+      const bool second = 2 * (wave + i * kWaves) + 1 < KT;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const v4i b = *(const v4i*)((const uint8_t*)area + r * 128 + ((h * 4 + c) ^ (r & 7)) * 16);
+        v4i blo, bhi, alo, ahi;
+        unpack_lo_hi(b, blo, bhi);
+        if (h == 1 && !second) a[i][1] = v4i{0, 0, 0, 0};
+        unpack_lo_hi(a[i][h], alo, ahi);
+        const v4i zero = {0, 0, 0, 0};
+        acc[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(blo, alo, EPI == kGroupScale ? zero : acc[h], 0, 0, 0);
+        acc[h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bhi, ahi, acc[h], 0, 0, 0);
+      }
+      if constexpr (EPI == kGroupScale) {
+        *(v4f*)(area + lane * 4) = tile_as_float(acc[0]);
+        *(v4f*)(area + 256 + lane * 4) = tile_as_float(acc[1]);
+      }
+    }
+  });
+  if constexpr (EPI != kGroupScale) *(v4i*)(red + wave * STEPS * 512 + lane * 4) = acc[0] + acc[1];
+  __syncthreads();
+
+  const int m = (tid >> 2) & 15, n = (tid >> 6) * 4 + (tid & 3), gn = w.n0 + n;
+  if (tid >= 256 || m >= p.M || gn >= w.N) return;
+  if constexpr (EPI == kGroupScale) {
+    const float* v = (const float*)red + tid;
+    const int pitch = scale_pitch(KT);
+    const unsigned *ra = table + m * pitch, *rb = table + ((p.a_cols > 1 ? p.M : 0) + n) * pitch;
+    float out = 0.f;
+    // eight pairs of groups, a step of every wave, read ahead of their multiply-adds
+    auto fold = [&](auto token) {
+      constexpr bool TOKEN = decltype(token)::value;
+      for (int i = 0; i * 2 * kWaves < KT; ++i) {
+        float lo[kWaves], hi[kWaves];
+        unsigned sa[kWaves], sb[kWaves];
+#pragma unroll
+        for (int u = 0; u < kWaves; ++u) {
+          const int pair = min(i * kWaves + u, ND - 1);
+          lo[u] = v[(u * STEPS + i) * 512], hi[u] = v[(u * STEPS + i) * 512 + 256];
+          sa[u] = TOKEN ? 0u : ra[pair], sb[u] = rb[pair];
+        }
+        auto pair = [&](int u, bool both) {
+          if constexpr (TOKEN) {
+            out = fma_half<0>(lo[u], sb[u], out);
+            if (both) out = fma_half<1>(hi[u], sb[u], out);
+          } else {
+            out = __builtin_fmaf(lo[u], mul_halves<0>(sa[u], sb[u]), out);
+            if (both) out = __builtin_fmaf(hi[u], mul_halves<1>(sa[u], sb[u]), out);
+          }
+        };
+        if ((i + 1) * 2 * kWaves <= KT) {
+#pragma unroll
+          for (int u = 0; u < kWaves; ++u) pair(u, true);
+        } else {
+#pragma unroll
+          for (int u = 0; u < kWaves; ++u)
+            if (2 * (i * kWaves + u) < KT) pair(u, 2 * (i * kWaves + u) + 1 < KT);
+        }
+      }
+    };
+    if (p.a_cols == 1) {
+      fold(std::true_type{});
+      out = round_here(out * 0.00390625f) * first.a;
+    } else {
+      fold(std::false_type{});
+      out *= 0.00390625f;
+    }
+    store_f16(p, w, m, gn, (_Float16)round_here(out));
+  } else {
+    int sum = 0;
+#pragma unroll
+    for (int u = 0; u < kWaves; ++u) sum += red[u * STEPS * 512 + tid];
+    store_f16(p, w, m, gn, (_Float16)round_here((float)sum * (first.a * (first.b * 0.00390625f))));
+  }
+}
+
+template <int STEPS, int EPI>
+int launch_lines(const GemmArgs& a, hipStream_t stream) {
+  const auto lds = [](int kt) { return (size_t)kWaves * STEPS * 2048 + (EPI == kGroupScale ? scale_table_dwords(kt) * 4 : 0); };
+  auto kern = gemm_i4_lines_kernel<STEPS, EPI>;
+  static_assert((size_t)kWaves * STEPS * 2048 + scale_table_dwords(2 * STEPS * kWaves) * 4 <= 160 * 1024, "LDS of a compute unit");
+  static LdsGrant grant;
+  if (int rc = reserve_lds((const void*)kern, lds(2 * STEPS * kWaves), grant, "gemm (lines)")) return rc;
+  GemmArgs g = a;
+  const int blocks = decode_blocks(g);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kWaves * 64), lds(a.K >> 7), stream, g);
+  return check_launch("gemm_i4_lines");
+}
+template <int EPI>
+int launch_lines(const GemmArgs& a, hipStream_t stream) {
+  const int steps = (a.K + 256 * kWaves - 1) / (256 * kWaves);
+  if (steps <= 2) return launch_lines<2, EPI>(a, stream);
+  if constexpr (EPI == kRowScale) {
+    if (steps > 4) return steps <= 6 ? launch_lines<6, EPI>(a, stream) : launch_lines<8, EPI>(a, stream);
+  }
+  return launch_lines<4, EPI>(a, stream);
+}
+
 // One to four tokens: products by v_dot8_i32_i4 on the packed codes as they are, which need no fragment layout, so that a load takes
 // whole lines of eight weight rows, past the caches (gemm_i4_online.hip has the same, and what it is worth there).  A workgroup of
 // eight waves owns 16 channels; a wave requests all its double steps at once, DOUBLES of them, through buffer descriptors:
@@ -451,13 +599,24 @@ int launch_dot(const GemmArgs& a, hipStream_t stream) {
 }  // namespace
 
 // Up to four tokens; more than two up to K = 8192, beyond which their codes take the registers of the weights in flight (four tokens 11008
-// x 4096 7.2 / 8.8 / 8.8 -> 7.8 / 9.3 / 9.1; two 7.1 / 8.9 / 9.4 -> 6.8 / 8.2 / 8.3).
+// x 4096 7.2 / 8.8 / 8.8 -> 7.8 / 9.3 / 9.1; two 7.1 / 8.9 / 9.4 -> 6.8 / 8.2 / 8.3), and with one scale per row up to 12288 channels, where the
+// kernel above takes over (four tokens x 28672 12.5 there, 13.1 here).
 bool gemm_dot_supports(const GemmArgs& a, int epi, int group) {
-  return a.M > 0 && a.M <= 4 && a.K <= 16384 && (epi == kRowScale || (epi == kGroupScale && group == 128)) && (a.M <= 2 || a.K <= 8192);
+  if (a.M <= 0 || a.M > 4 || a.K > 16384 || !(epi == kRowScale || (epi == kGroupScale && group == 128))) return false;
+  if (a.M <= 2) return true;
+  long columns = a.N;
+  for (int s = 1; s < a.n_seg; ++s) columns += a.seg_N[s];
+  return a.K <= 8192 && (epi != kRowScale || columns <= 12288);
 }
 
 int gemm_dot_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
   return epi == kRowScale ? launch_dot<kRowScale>(a, stream) : launch_dot<kGroupScale>(a, stream);
+}
+
+// Sixteen tokens; group scales up to K = 8192: with long rows the scales that have to be there before the first operand and the tiles in
+// the operands' place cost more than whole lines give (five tokens 11008 x 4096 8.7 with half lines, 9.2 so).
+bool gemm_lines_supports(const GemmArgs& a, int epi) {
+  return a.M <= 16 && (epi == kRowScale ? a.K <= 16384 : epi == kGroupScale && a.K <= 8192);
 }
 
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group) {
@@ -468,6 +627,8 @@ bool gemm_decode_supports(const GemmArgs& a, int epi, int group) {
 
 int gemm_decode_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
   const int mt = (a.M + 15) / 16;
+  if (gemm_lines_supports(a, epi))
+    return epi == kGroupScale ? launch_lines<kGroupScale>(a, stream) : launch_lines<kRowScale>(a, stream);
   if (epi == kGroupScale) return launch_decode<1, kGroupScale>(a, stream);
   if (epi == kInt32) {
     if (mt == 1) return launch_decode<1, kInt32>(a, stream);

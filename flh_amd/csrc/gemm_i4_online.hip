@@ -1,4 +1,4 @@
-// int4 x int4 GEMM that quantises its own activations: one to four tokens (eight with group scales) of K = 4096, so few that
+// int4 x int4 GEMM that quantises its own activations: one to four tokens of K = 4096, so few that
 // repeating the quantiser in every workgroup costs less than a launch of its own in front of the GEMM.
 //
 // A workgroup of eight waves owns T tiles of 16 channels, as many as put one workgroup on a compute unit, and every token.  A
@@ -7,13 +7,13 @@
 //   rotate            the whole row rotated, one scale per token (rotate_quant_row_8waves)
 //   norm + rotate     RMSNorm in front, with or without a residual addition in front of that (workgroup 0 stores the sum)
 //   norm + groups     RMSNorm, then one scale per 128 channels, no rotation (rmsnorm_group_kernel)
-// The products, their folds and the epilogue are those of the other kernels: the same bits as quantiser and GEMM in two launches.
+// The sums, their folds and the epilogue are those of the other kernels: the same bits as quantiser and GEMM in two launches.
 //
 // What bounds it: first access, then the weight stream (one token 28672 x 4096 15.6 us, 58.7 MB).  The order of the requests is what
 // hides the quantiser: loads come back in the order they were made, so the token's are made first, then those of all the workgroup's
 // weights, and no barrier in between waits for more than LDS.  All sums of a workgroup's tokens (not of the sixteen that a tile
 // of the matrix instruction has room for) fit LDS, so that one barrier separates the products of all tiles from their folds.
-// Up to four tokens the products are v_dot8_i32_i4 on the packed codes as they are: nothing to unpack, no idle columns, and no
+// The products are v_dot8_i32_i4 on the packed codes as they are: nothing to unpack, no idle columns, and no
 // fragment layout, so that a load takes whole lines of eight weight rows, past the caches.  One token, token scales, us, weights from
 // HBM: with the requests in the old order, 16 x 16 x 64 products and half lines -> these requests -> dot products -> whole lines
 // past the caches (quantiser and GEMM in two launches):
@@ -31,8 +31,7 @@ constexpr int kWaves = 8;
 constexpr int kK = 4096, kRowB = kK / 2, kGroups = kK / 128;
 constexpr int kDoubles = kGroups / 2 / kWaves;     // double steps per wave
 constexpr int kCodePitch = kRowB + 16;             // code rows 16 bytes apart in the banks
-constexpr int kRotateMaxTokens = 4, kGroupMaxTokens = 8;
-constexpr int kDotMaxTokens = 4;
+constexpr int kMaxTokens = 4;
 
 enum Prologue { kRotate = 0, kNormRotate = 1, kAddNormRotate = 2, kNormGroup = 3 };
 
@@ -70,19 +69,17 @@ __host__ __device__ constexpr int lds_bytes(int M) {
   return lds_codes<EPI, PRO, T>(M) + lds_tables<EPI, PRO, T>(M) + (sums > scratch ? sums : scratch);
 }
 
-// MAXM: tokens that the kernel takes, 1, 2, 4 or as many as are allowed.  DOT (up to four): a tile of a wave takes 16 dot products and
-// nine instructions across lanes per token, and one four-byte LDS write without idle lanes, where the matrix instruction takes 96
-// instructions of unpacking and, per group, a 16-byte write of which a token fills a sixteenth.
+// MAXM: tokens that the kernel takes, 1, 2 or 4.  A tile of a wave takes 16 dot products and nine instructions across lanes per
+// token, and one four-byte LDS write without idle lanes, where the matrix instruction takes 96 instructions of unpacking and, per
+// group, a 16-byte write of which a token fills a sixteenth.
 template <int EPI, int PRO, int T, int MAXM>
 __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const OnlineArgs p) {
-  constexpr bool DOT = MAXM <= kDotMaxTokens;
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, c = lane >> 4;          // MFMA: row and piece of a half line
-  const int line_row = lane >> 3, line_piece = lane & 7;   // DOT: eight rows' whole lines
+  const int r = lane & 15, c = lane >> 4;          // what the lane finishes: channel r, token c
+  const int line_row = lane >> 3, line_piece = lane & 7;   // what it loads: whole lines of eight weight rows
   const int M = MAXM <= 2 ? MAXM : p.M;
-  const int MS = DOT ? MAXM : M;                   // tokens' rows per tile and group in the sums
   uint8_t* codes = lds;
   __half* tok = (__half*)(lds + lds_codes<EPI, PRO, T>(M));
   uint8_t* table = (uint8_t*)tok + (PRO == kNormGroup ? M * kGroups * 2 : 16);
@@ -149,18 +146,12 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const Onlin
   // 3. this wave's weights of all tiles, in the order of their use
   v4i b[T][kDoubles][2];
   static_for<T * kDoubles>([&](auto index) {
-    constexpr int at = decltype(index)::value, t = DOT ? at / kDoubles : at % T, i = DOT ? at % kDoubles : at / T;
+    constexpr int t = decltype(index)::value / kDoubles, i = decltype(index)::value % kDoubles;
     const OnlineTile w = tile(t);
     const uint8_t* base = w.B + (size_t)w.n0 * kRowB + i * (kWaves * 128);
-    if constexpr (DOT) {
-      const int last = w.N - 1 - w.n0;
-      b[t][i][0] = __builtin_nontemporal_load((const v4i*)(base + (unsigned)(min(line_row, last) * kRowB + wave * 128 + line_piece * 16)));
-      b[t][i][1] = __builtin_nontemporal_load((const v4i*)(base + (unsigned)(min(8 + line_row, last) * kRowB + wave * 128 + line_piece * 16)));
-    } else {
-      const unsigned offset = min(r, w.N - 1 - w.n0) * kRowB + c * 16 + wave * 128;
-      b[t][i][0] = *(const v4i*)(base + offset);
-      b[t][i][1] = *(const v4i*)(base + offset + 64);
-    }
+    const int last = w.N - 1 - w.n0;
+    b[t][i][0] = __builtin_nontemporal_load((const v4i*)(base + (unsigned)(min(line_row, last) * kRowB + wave * 128 + line_piece * 16)));
+    b[t][i][1] = __builtin_nontemporal_load((const v4i*)(base + (unsigned)(min(8 + line_row, last) * kRowB + wave * 128 + line_piece * 16)));
   });
   __builtin_amdgcn_sched_barrier(0);
 
@@ -230,97 +221,57 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const Onlin
   barrier_after_lds();
 
   // 5. products.  Sums: [tile][group | wave][token][16 channels]
-  if constexpr (DOT) {
-    v4i a[MAXM][kDoubles];
+  v4i a[MAXM][kDoubles];
 #pragma unroll
-    for (int m = 0; m < MAXM; ++m)
+  for (int m = 0; m < MAXM; ++m)
 #pragma unroll
-      for (int i = 0; i < kDoubles; ++i) a[m][i] = *(const v4i*)(codes + min(m, M - 1) * kCodePitch + (wave + i * kWaves) * 128 + line_piece * 16);
-    auto dot = [](v4i x, v4i y, int sum) {
+    for (int i = 0; i < kDoubles; ++i) a[m][i] = *(const v4i*)(codes + min(m, M - 1) * kCodePitch + (wave + i * kWaves) * 128 + line_piece * 16);
+  auto dot = [](v4i x, v4i y, int sum) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(x[e], y[e], sum, false);
-      return sum;
-    };
-    // lane k of four adjacent ones: part k, summed over the four
-    auto gather = [&](int p0, int p1, int p2, int p3) {
-      const bool odd = lane & 1, high = lane & 2;
-      const int x = (odd ? p1 : p0) + dpp_i<kDppQuadXor1>(odd ? p0 : p1), y = (odd ? p3 : p2) + dpp_i<kDppQuadXor1>(odd ? p2 : p3);
-      return (high ? y : x) + dpp_i<kDppQuadXor2>(high ? x : y);
-    };
-    const int n = (lane & 1) * 8 + line_row, half_line = line_piece >> 2;
-    static_for<T>([&](auto t_tag) {
-      constexpr int t = decltype(t_tag)::value;
+    for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(x[e], y[e], sum, false);
+    return sum;
+  };
+  // lane k of four adjacent ones: part k, summed over the four
+  auto gather = [&](int p0, int p1, int p2, int p3) {
+    const bool odd = lane & 1, high = lane & 2;
+    const int x = (odd ? p1 : p0) + dpp_i<kDppQuadXor1>(odd ? p0 : p1), y = (odd ? p3 : p2) + dpp_i<kDppQuadXor1>(odd ? p2 : p3);
+    return (high ? y : x) + dpp_i<kDppQuadXor2>(high ? x : y);
+  };
+  const int n = (lane & 1) * 8 + line_row, half_line = line_piece >> 2;
+  static_for<T>([&](auto t_tag) {
+    constexpr int t = decltype(t_tag)::value;
 #pragma unroll
-      for (int m = 0; m < MAXM; ++m) {
-        // parts: rows line_row and 8 + line_row of either double step
-        if constexpr (EPI == kRowScale) {
-          const int p0 = dot(b[t][1][0], a[m][1], dot(b[t][0][0], a[m][0], 0)), p1 = dot(b[t][1][1], a[m][1], dot(b[t][0][1], a[m][0], 0));
-          const bool odd = lane & 1;
-          int sum = (odd ? p1 : p0) + dpp_i<kDppQuadXor1>(odd ? p0 : p1);
-          sum += dpp_i<kDppQuadXor2>(sum);
-          sum += dpp_i<kDppRowHalfMirror>(dpp_i<kDppQuadXor1>(sum));   // (lane ^ 6: the other four)
-          if ((lane & 6) == 0) ((int*)sums)[((t * kWaves + wave) * MAXM + m) * 16 + n] = sum;
-        } else {
-          const int sum = gather(dot(b[t][0][0], a[m][0], 0), dot(b[t][0][1], a[m][0], 0), dot(b[t][1][0], a[m][1], 0),
-                                 dot(b[t][1][1], a[m][1], 0));
-          const int g = 2 * (wave + ((lane >> 1) & 1) * kWaves) + half_line;
-          ((float*)sums)[((t * kGroups + g) * MAXM + m) * 16 + n] = (float)sum;
-        }
+    for (int m = 0; m < MAXM; ++m) {
+      // parts: rows line_row and 8 + line_row of either double step
+      if constexpr (EPI == kRowScale) {
+        const int p0 = dot(b[t][1][0], a[m][1], dot(b[t][0][0], a[m][0], 0)), p1 = dot(b[t][1][1], a[m][1], dot(b[t][0][1], a[m][0], 0));
+        const bool odd = lane & 1;
+        int sum = (odd ? p1 : p0) + dpp_i<kDppQuadXor1>(odd ? p0 : p1);
+        sum += dpp_i<kDppQuadXor2>(sum);
+        sum += dpp_i<kDppRowHalfMirror>(dpp_i<kDppQuadXor1>(sum));   // (lane ^ 6: the other four)
+        if ((lane & 6) == 0) ((int*)sums)[((t * kWaves + wave) * MAXM + m) * 16 + n] = sum;
+      } else {
+        const int sum = gather(dot(b[t][0][0], a[m][0], 0), dot(b[t][0][1], a[m][0], 0), dot(b[t][1][0], a[m][1], 0),
+                               dot(b[t][1][1], a[m][1], 0));
+        const int g = 2 * (wave + ((lane >> 1) & 1) * kWaves) + half_line;
+        ((float*)sums)[((t * kGroups + g) * MAXM + m) * 16 + n] = (float)sum;
       }
-    });
-  } else {
-    // (an operand piece of the tokens is unpacked once for all tiles)
-    const uint8_t* arow = codes + min(r, M - 1) * kCodePitch + c * 16;
-    v4i acc[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) acc[t] = v4i{0, 0, 0, 0};
-    auto lo = [](v4i v) { return (v << 4) & (int)0xF0F0F0F0; };
-    auto hi = [](v4i v) { return v & (int)0xF0F0F0F0; };
-    const bool live = r < M;
-#pragma unroll
-    for (int i = 0; i < kDoubles; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int step = wave + i * kWaves;
-        const v4i a = *(const v4i*)(arow + step * 128 + h * 64);
-        const v4i alo = lo(a), ahi = hi(a);
-        v4f f[T];
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-          v4i d = EPI == kRowScale ? acc[t] : v4i{0, 0, 0, 0};
-          d = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo(b[t][i][h]), alo, d, 0, 0, 0);
-          d = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi(b[t][i][h]), ahi, d, 0, 0, 0);
-          if constexpr (EPI == kRowScale) acc[t] = d;
-          else f[t] = v4f{(float)d[0], (float)d[1], (float)d[2], (float)d[3]};
-        }
-        if constexpr (EPI != kRowScale)
-          if (live) {
-#pragma unroll
-            for (int t = 0; t < T; ++t) *(v4f*)((float*)sums + ((t * kGroups + 2 * step + h) * M + r) * 16 + c * 4) = f[t];
-          }
-      }
-    if constexpr (EPI == kRowScale)
-      if (live) {
-#pragma unroll
-        for (int t = 0; t < T; ++t) *(v4i*)((int*)sums + ((t * kWaves + wave) * M + r) * 16 + c * 4) = acc[t];
-      }
-  }
+    }
+  });
   if constexpr (EPI != kRowScale) wait_vmcnt<0>();   // the channels' scales
   barrier_after_lds();
 
-  constexpr float kExact = DOT ? 1.f : 0.00390625f;  // the sums of the matrix instruction are 256 times the exact ones
-  // 6. folds: a wave finishes four tokens of a tile, a lane token lane / 16, channel lane % 16
-  const int quads = (M + 3) >> 2;                  // 1, with group scales also 2
-  for (int u = wave; u < T * quads; u += kWaves) {
-    const int t = quads == 1 ? u : u >> 1, m = (quads == 1 ? 0 : (u & 1) * 4) + c;
+  // 6. folds: a wave finishes a tile, a lane token lane / 16, channel lane % 16
+  if (wave < T) {
+    const int t = wave, m = c;
     auto value = [&] {                             // before the rounding to fp16
       if constexpr (EPI == kRowScale) {
         int sum = 0;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) sum += ((const int*)sums)[((t * kWaves + w) * MS + m) * 16 + r];
-        return (float)sum * (__half2float(tok[m]) * (s_row * kExact));
+        for (int w = 0; w < kWaves; ++w) sum += ((const int*)sums)[((t * kWaves + w) * MAXM + m) * 16 + r];
+        return (float)sum * (__half2float(tok[m]) * s_row);
       } else {
-        const float* v = (const float*)sums + (t * kGroups * MS + m) * 16 + r;
+        const float* v = (const float*)sums + (t * kGroups * MAXM + m) * 16 + r;
         const uint8_t* sb = table + t * 1024 + r * 64;
         float out = 0.f;
 #pragma unroll
@@ -329,7 +280,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const Onlin
           const v4i aq = PRO == kNormGroup ? *(const v4i*)(tok + m * kGroups + q * 8) : v4i{0, 0, 0, 0};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float v0 = v[(q * 8 + 2 * e) * MS * 16], v1 = v[(q * 8 + 2 * e + 1) * MS * 16];
+            const float v0 = v[(q * 8 + 2 * e) * MAXM * 16], v1 = v[(q * 8 + 2 * e + 1) * MAXM * 16];
             if constexpr (PRO == kNormGroup) {
               out = __builtin_fmaf(v0, mul_halves<0>((unsigned)aq[e], (unsigned)bq[e]), out);
               out = __builtin_fmaf(v1, mul_halves<1>((unsigned)aq[e], (unsigned)bq[e]), out);
@@ -339,7 +290,6 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_online_kernel(const Onlin
             }
           }
         }
-        out *= kExact;
         return PRO == kNormGroup ? out : round_here(out) * __half2float(tok[m]);
       }
     };
@@ -355,7 +305,7 @@ template <int EPI, int PRO, int T, int MAXM>
 int launch_kernel(const OnlineArgs& a, hipStream_t stream) {
   auto kern = gemm_i4_online_kernel<EPI, PRO, T, MAXM>;
   constexpr size_t most = lds_bytes<EPI, PRO, T>(MAXM);
-  static_assert(most <= 160 * 1024, "LDS of a compute unit");
+  static_assert(T <= kWaves && most <= 160 * 1024, "LDS of a compute unit");
   static LdsGrant grant;
   if (int rc = reserve_lds((const void*)kern, most, grant, "gemm (online)")) return rc;
   const size_t bytes = lds_bytes<EPI, PRO, T>(a.M);
@@ -380,10 +330,7 @@ int launch_by_tiles(const OnlineArgs& a, hipStream_t stream) {
 template <int EPI, int PRO>
 int launch(const OnlineArgs& a, hipStream_t stream) {
   if (a.M == 1) return launch_by_tiles<EPI, PRO, 1>(a, stream);
-  if (a.M == 2) return launch_by_tiles<EPI, PRO, 2>(a, stream);
-  if constexpr (PRO == kNormGroup)
-    if (a.M > 4) return launch_by_tiles<EPI, PRO, kGroupMaxTokens>(a, stream);
-  return launch_by_tiles<EPI, PRO, 4>(a, stream);
+  return a.M == 2 ? launch_by_tiles<EPI, PRO, 2>(a, stream) : launch_by_tiles<EPI, PRO, kMaxTokens>(a, stream);
 }
 
 struct OnlineCall {
@@ -401,9 +348,8 @@ int online_checked(const char* who, const OnlineCall& call, int count, const uin
   if (M == 0) return FLH_OK;
   if (!call.x) return fail(FLH_EINVAL, "%s: null pointer", who);
   if (misaligned16(call.x)) return fail(FLH_EINVAL, "%s: x must be 16-byte aligned", who);
-  const int most = call.groups ? kGroupMaxTokens : kRotateMaxTokens;
-  if (M > (size_t)most)
-    return fail(FLH_EINVAL, "%s: M = %zu, at most %d tokens (more tokens quantise once, in their own launch)", who, M, most);
+  if (M > (size_t)kMaxTokens)
+    return fail(FLH_EINVAL, "%s: M = %zu, at most %d tokens (more tokens quantise once, in their own launch)", who, M, kMaxTokens);
   if (K != kK) return fail(FLH_EINVAL, "%s: K = %zu is not supported (4096)", who, K);
   if (b_cols != 1 && (size_t)b_cols != K / 128)
     return fail(FLH_EINVAL, "%s: weight scale columns (%d) must be 1 or K / 128 = %zu", who, b_cols, K / 128);

@@ -600,8 +600,8 @@ std::tuple<c10::optional<Tensor>, std::vector<Tensor>> rmsnorm_rotate_quantize_g
 
 // RMSNorm(x), groups of 128 without rotation and up to four GEMMs with group scales: [fp16 [M, N_s] ...].  The quantiser is repeated by
 // every workgroup of the one launch and the tokens' products grow with it, so fewer channels for more tokens (us, one launch / two:
-// one token x 6144 5.0 / 7.8, x 28672 13.5 / 14.9; two x 28672 14.8 / 15.2; four x 16384 11.2 / 12.1, x 22016 14.7 / 14.4; five x 12288 10.9 /
-// 12.1; six 11.7 / 12.1, x 16384 13.7 / 13.4; eight x 6144 10.3 / 10.2).
+// one token x 6144 5.0 / 7.8, x 28672 13.5 / 14.9; two x 28672 14.8 / 15.2; four x 16384 11.2 / 12.1, x 22016 14.7 / 14.4; five gain at
+// few channels only: x 6144 8.5 / 8.9, x 12288 11.2 / 10.7).
 std::vector<Tensor> rmsnorm_group_quantize_gemm_i4_multi(const Tensor& x, const c10::optional<Tensor>& weight, double eps,
                                                          const std::vector<Tensor>& Bs, const std::vector<Tensor>& B_scales) {
   TORCH_CHECK(Bs.size() == B_scales.size() && !Bs.empty() && Bs.size() <= 4,
@@ -609,7 +609,7 @@ std::vector<Tensor> rmsnorm_group_quantize_gemm_i4_multi(const Tensor& x, const 
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat16 && x.dim() == 2 && x.is_contiguous(),
               "x must be a contiguous 2D float16 CUDA tensor");
   const int64_t M = x.size(0), K = x.size(1);
-  TORCH_CHECK(M <= 8, "at most 8 tokens");
+  TORCH_CHECK(M <= 4, "at most 4 tokens");
   TORCH_CHECK(K == 4096, "K must be 4096");
   if (weight.has_value())
     TORCH_CHECK(weight->is_cuda() && weight->scalar_type() == torch::kFloat16 && weight->is_contiguous() &&
@@ -638,7 +638,7 @@ std::vector<Tensor> rmsnorm_group_quantize_gemm_i4_multi(const Tensor& x, const 
   if (M == 0) return Ds;
   const flh_half* w = weight.has_value() ? h(*weight) : nullptr;
   Launch l(x);
-  const int64_t most = M <= 2 ? kOnlineChannels : M <= 4 ? 16384 : M <= 6 ? 12288 : 0;
+  const int64_t most = M <= 2 ? kOnlineChannels : 16384;
   if (channels <= most && ((uintptr_t)w & 15) == 0) {
     ok(flh_rmsnorm_group_quant_gemm_i4_o16_multi(h(x), w, (float)eps, (int)Bs.size(), b, bs, d, n, M, K, stream_of(x)));
     return Ds;

@@ -536,9 +536,9 @@ class W4A4DecoderLayer(torch.nn.Module):
         return c == 1 or (c == self.hidden_size // 128 and layers[0].weight_group_size == 128)
 
     def _online_rows_apply(self, layers, rows):
-        """Whether `layers` take the launch with norm and quantiser inside: one or two tokens rotated as whole rows, up to eight in
+        """Whether `layers` take the launch with norm and quantiser inside: one or two tokens rotated as whole rows, up to four in
         groups (which of them by one launch and which by two, the operations know)."""
-        if not (self.fused and self.record is None and 0 < rows <= (2 if self.activation == "token" else 8)
+        if not (self.fused and self.record is None and 0 < rows <= (2 if self.activation == "token" else 4)
                 and self.hidden_size == 4096 and self._online_applies(layers)):
             return False
         if self.activation == "token":

@@ -134,7 +134,7 @@ int flh_rmsnorm_rotate_quant_gemm_i4_o16_multi(const flh_half* x, const flh_half
 
 /* ... and with the prologue of flh_rmsnorm_group_quant_i4 (groups of 128, no rotation, scale_mul 1): x [M, K] fp16 -> RMSNorm ->
  * one int4 scale per 128 channels -> the GEMMs, whose weights have group scales [N, K / 128]; one launch, the bits of the
- * separate ones.  M <= 8, K = 4096. */
+ * separate ones.  M <= 4, K = 4096. */
 int flh_rmsnorm_group_quant_gemm_i4_o16_multi(const flh_half* x, const flh_half* weight, float eps, int count,
                                               const uint8_t* const* B, const flh_half* const* b_scale, flh_half* const* D,
                                               const size_t* N, size_t M, size_t K, void* stream);

@@ -56,7 +56,7 @@ def test_whole_rows(ops, ns, cols):
 @pytest.mark.parametrize("offset", [0, 1])
 def test_groups(ops, ns, offset):
     x, _, w, Bs, Ss = make(ns, 32, sum(ns) + 7, offset)
-    for m in (1, 2, 3, 4, 5, 8):
+    for m in (1, 2, 3, 4):
         for weight in (w, None):
             outs = ops.rmsnorm_group_quantize_gemm_i4_multi(x[:m], weight, 1e-5, Bs, Ss)
             q, a = ops.rmsnorm_and_quantize_i4_gs(x[:m].contiguous(), weight, 1e-5, 128, False)
