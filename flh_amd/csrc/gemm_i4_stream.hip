@@ -92,22 +92,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
 
   auto first_group = [&](int s) { return min(s * kStageGroups, KT - kStageGroups); };   // the last stage ends with the row
 
-  // scales first, as their rows are: [row][KT / 2 pairs, an odd number of slots] in LDS, every wave a share of them
-  const int pitch = (KT >> 1) | 1;
-  {
-    const float inv = 1.0f / (float)pitch;
-    const int total = SROWS * pitch;
-    for (int f0 = wave * 64; f0 < total; f0 += WAVES * 64) {
-      const int f = min(f0 + lane, total - 1);
-      int row = (int)((float)f * inv);             // f < 2^14: off by one at most
-      row += (f >= (row + 1) * pitch ? 1 : 0) - (f < row * pitch ? 1 : 0);
-      const int pair = min(f - row * pitch, (KT >> 1) - 1), chan = row - (SROWS - RB);
-      const __half* q = chan < 0 ? p.As + (size_t)min(m0 + row, p.M - 1) * KT
-                                 : Bs + (size_t)b_row(chan) * KT;
-      load_to_lds4(q + 2 * pair, (unsigned)(uintptr_t)scales + f0 * 4);
-    }
-  }
-
+  const int pitch = (KT >> 1) | 1;                 // of the scale table
   // operands: a load instruction brings 256 bytes of four rows, chunk c of row r to slot c ^ (r % 16); a wave's share of either
   // operand is consecutive KiB of LDS (load_kib_to_lds16: addresses less 1024 i)
   const int lrow = lane >> 4;
@@ -193,8 +178,24 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i4_stream_kernel(const Gemm
     });
   };
 
+  request(0, 0);
+  // scales behind the first stage (in front of it, their addresses took 0.6 us before the first operand was requested), as their rows
+  // are: [row][KT / 2 pairs, an odd number of slots] in LDS, every wave a share of them
+  {
+    const float inv = 1.0f / (float)pitch;
+    const int total = SROWS * pitch;
+    for (int f0 = wave * 64; f0 < total; f0 += WAVES * 64) {
+      const int f = min(f0 + lane, total - 1);
+      int row = (int)((float)f * inv);             // f < 2^14: off by one at most
+      row += (f >= (row + 1) * pitch ? 1 : 0) - (f < row * pitch ? 1 : 0);
+      const int pair = min(f - row * pitch, (KT >> 1) - 1), chan = row - (SROWS - RB);
+      const __half* q = chan < 0 ? p.As + (size_t)min(m0 + row, p.M - 1) * KT
+                                 : Bs + (size_t)b_row(chan) * KT;
+      load_to_lds4(q + 2 * pair, (unsigned)(uintptr_t)scales + f0 * 4);
+    }
+  }
 #pragma unroll
-  for (int s = 0; s < S - 1; ++s)
+  for (int s = 1; s < S - 1; ++s)
     if (s < stages) request(s, s * STAGE);
   const bool live = m0 + wm * 16 < p.M;
   // every wave's loads of the oldest stage but `newer` are in LDS, every wave has its last stage in registers
