@@ -73,9 +73,9 @@ def add_rmsnorm_rotate_and_quantize_i4(x, add, weight, eps, hadamard=True, clip_
     return tuple(_ext.add_rmsnorm_rotate_and_quantize_i4_mode(x, add, weight, eps, _ops._whole_row_mode(hadamard), clip_ratio))
 
 
-def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None):
+def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None, weights=None):
     mode = _ops._f6_mode(x, hadamard, eps, add) if x.dim() == 2 else 0
-    return tuple(_ext.rotate_and_quantize_f6_mode(x, mode, clip_ratio, norm_weight, eps, add))
+    return tuple(_ext.rotate_and_quantize_f6_mode(x, mode, clip_ratio, norm_weight, eps, add, weights))
 
 
 def __getattr__(name):        # ops the extension does not wrap (one matrix's encoding, int32 output, tuning hook, ...)

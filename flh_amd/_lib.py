@@ -84,6 +84,10 @@ _SIG = {
                                                    _c.c_uint32, _c.c_uint32, _c.c_uint32, _c.c_float, _PTR]),
     "flh_add_rmsnorm_rotate_quant_i4": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _c.c_float, _PTR, _PTR, _c.c_uint32, _c.c_uint32,
                                                   _c.c_int, _c.c_float, _PTR]),
+    "flh_group_quant_encode_f6": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _c.c_int, _c.c_float, _PTR, _PTR]),
+    "flh_rmsnorm_group_quant_encode_f6": (_c.c_int, [_PTR, _PTR, _PTR, _PTR, _c.c_uint32, _c.c_uint32, _c.c_float, _PTR, _PTR]),
+    "flh_rotate_quant_encode_f6": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_int, _PTR, _c.c_float, _PTR, _PTR, _c.c_uint32, _c.c_uint32,
+                                             _c.c_int, _c.c_float, _PTR, _PTR]),
     "flh_rotate_quant_f6": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_int, _PTR, _c.c_float, _PTR, _PTR, _c.c_uint32, _c.c_uint32,
                                       _c.c_int, _c.c_float, _PTR]),
     "flh_silu_mul_f16": (_c.c_int, [_PTR, _PTR, _PTR, _c.c_uint64, _PTR]),

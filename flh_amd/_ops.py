@@ -5,6 +5,8 @@ the C ABI in include/flh_hip.h.  torch is used only for device memory and the cu
 stream.  Beyond the nine reference ops it exports the whole-row rotate+quantise op and
 the generalised GEMM (per-token x per-channel scales, int32 output).
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -382,9 +384,14 @@ def encode_f6(packed):
     return out
 
 
-def encode_f6_many(packed):
-    """[encode_f6(p) for p in packed] of one to four matrices with the same K in one launch."""
-    import ctypes
+class _EncodeList(ctypes.Structure):
+    """flh_encode_list"""
+    _fields_ = [("count", ctypes.c_int), ("packed", ctypes.c_void_p * 4), ("encoded", ctypes.c_void_p * 4),
+                ("rows", ctypes.c_size_t * 4), ("K", ctypes.c_size_t)]
+
+
+def _encode_list(packed):
+    """(_EncodeList, encodings to be written) of one to four matrices with the same K."""
     n = len(packed)
     _check(1 <= n <= 4, "one to four matrices")
     for p in packed:
@@ -394,26 +401,42 @@ def encode_f6_many(packed):
     K = packed[0].size(1) * 2
     _check(K % 128 == 0, "K must be a multiple of 128")
     outs = [torch.empty((p.size(0), K // 128 * 96), dtype=torch.uint8, device=p.device) for p in packed]
-    ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
-    if K:
-        _run("flh_encode_f6_multi", packed[0].device, n, ptrs(packed), ptrs(outs), (ctypes.c_size_t * n)(*[p.size(0) for p in packed]), K,
-             _stream(packed[0]))
+    ptrs = lambda ts: (ctypes.c_void_p * 4)(*[t.data_ptr() for t in ts])
+    return _EncodeList(n, ptrs(packed), ptrs(outs), (ctypes.c_size_t * 4)(*[p.size(0) for p in packed]), K), outs
+
+
+def encode_f6_many(packed):
+    """[encode_f6(p) for p in packed] of one to four matrices with the same K in one launch."""
+    e, outs = _encode_list(packed)
+    if e.K:
+        _run("flh_encode_f6_multi", packed[0].device, e.count, e.packed, e.encoded, e.rows, e.K, _stream(packed[0]))
     return outs
 
 
-def group_quantize_f6(x, hadamard=True, *, scale_mul=1.0):
+def _beside(x, weights):
+    """(pointer argument, encodings) of the weights that a quantiser's codes are to meet; (None, []) without any."""
+    if weights is None:
+        return None, []
+    e, outs = _encode_list(weights)
+    _check(weights[0].device == x.device and e.K == x.size(1), "weights must be on x's device and of its K")
+    return ctypes.byref(e), outs
+
+
+def group_quantize_f6(x, hadamard=True, *, scale_mul=1.0, weights=None):
     """hadamard_and_quantize_i4 / quant_and_pack_i4 over groups of 128 of x [M, K] fp16, with the codes
-    written in the format of encode_f6: -> [q6 [M, K/128 * 96] u8, scales [M, K/128] fp16]."""
+    written in the format of encode_f6: -> [q6 [M, K/128 * 96] u8, scales [M, K/128] fp16].  `weights` (this and the next
+    two; one to four packed matrices [rows, K/2]): followed by encode_f6_many(weights), one launch where that is possible."""
     _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
            "Input tensor must be a contiguous 2D float16 CUDA tensor")
     M, K = x.shape
     _check(K % 128 == 0 and K > 0, "Last dimension must be a multiple of 128")
     q6 = torch.empty((M, K // 128 * 96), dtype=torch.uint8, device=x.device)
     s = torch.empty((M, K // 128), dtype=torch.float16, device=x.device)
-    if M:
-        _run("flh_group_quant_f6", x.device, x.data_ptr(), q6.data_ptr(), s.data_ptr(), M, K, int(bool(hadamard)),
-             float(scale_mul), _stream(x))
-    return [q6, s]
+    e, w6 = _beside(x, weights)
+    if M or w6:
+        _run("flh_group_quant_encode_f6", x.device, x.data_ptr(), q6.data_ptr(), s.data_ptr(), M, K, int(bool(hadamard)),
+             float(scale_mul), e, _stream(x))
+    return [q6, s, *w6]
 
 
 def _f6_rows(x):
@@ -425,17 +448,18 @@ def _f6_rows(x):
             torch.empty((M, K // 128), dtype=torch.float16, device=x.device))
 
 
-def rmsnorm_group_quantize_f6(x, weight, eps):
+def rmsnorm_group_quantize_f6(x, weight, eps, weights=None):
     """rmsnorm_and_quantize_i4_gs(x, weight, eps, 128) of x [M, K] with the codes in the format of encode_f6."""
     M, K, q6, s = _f6_rows(x)
     _check(K <= 16384, "Last dimension must be at most 16384")
     if weight is not None:
         _check(weight.is_cuda and weight.dtype == torch.float16 and weight.is_contiguous() and weight.numel() == K
                and weight.device == x.device, "weight must be a contiguous float16 CUDA tensor of K values")
-    if M:
-        _run("flh_rmsnorm_group_quant_f6", x.device, x.data_ptr(), weight.data_ptr() if weight is not None else None,
-             q6.data_ptr(), s.data_ptr(), M, K, float(eps), _stream(x))
-    return [q6, s]
+    e, w6 = _beside(x, weights)
+    if M or w6:
+        _run("flh_rmsnorm_group_quant_encode_f6", x.device, x.data_ptr(), weight.data_ptr() if weight is not None else None,
+             q6.data_ptr(), s.data_ptr(), M, K, float(eps), e, _stream(x))
+    return [q6, s, *w6]
 
 
 def silu_mul_group_quantize_f6(gate, up):
@@ -1012,7 +1036,7 @@ def _f6_mode(x, hadamard, eps, add):
     return _whole_row_mode(hadamard)
 
 
-def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None):
+def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, eps=None, add=None, weights=None):
     """rotate_and_quantize_i4 (one scale per token) with the codes written in the 6-bit operand format of gemm_f6_*
     directly: x [M, K] fp16 -> (encoded [M, K / 128 * 96] u8, scales [M, 1] fp16), the bytes of encode_f6(q).
     K = 512 .. 8192 a power of two (float32 butterflies, `hadamard` True / "exact" / False) -- optionally behind RMSNorm
@@ -1033,12 +1057,13 @@ def rotate_and_quantize_f6(x, hadamard=True, clip_ratio=1.0, norm_weight=None, e
     enc = torch.empty((M, K // 128 * 96), dtype=torch.uint8, device=x.device)
     s = torch.empty((M, 1), dtype=torch.float16, device=x.device)
     total = torch.empty_like(x) if add is not None else None
-    if M:
-        _run("flh_rotate_quant_f6", x.device, x.data_ptr(), add.data_ptr() if add is not None else None,
+    e, w6 = _beside(x, weights)
+    if M or w6:
+        _run("flh_rotate_quant_encode_f6", x.device, x.data_ptr(), add.data_ptr() if add is not None else None,
              total.data_ptr() if total is not None else None, 1 if eps is not None else 0,
              norm_weight.data_ptr() if norm_weight is not None else None, float(eps or 0.0), enc.data_ptr(), s.data_ptr(), M, K,
-             mode, float(clip_ratio), _stream(x))
-    return (total, enc, s) if add is not None else (enc, s)
+             mode, float(clip_ratio), e, _stream(x))
+    return (total, enc, s, *w6) if add is not None else (enc, s, *w6)
 
 
 def rotate_and_quantize_i4(x, hadamard=True, had_group=0, scale_group=0, clip_ratio=1.0, return_rotated=False):

@@ -25,6 +25,7 @@
 #include "lane_ops.h"
 #include "quant_pack.h"
 #include "group_codes.h"
+#include "encode_f6.h"
 #include "f6_codes.h"
 #include "rotate_row.h"
 
@@ -268,13 +269,14 @@ __device__ __forceinline__ void butterfly(h2& a, h2& b) {
   const h2 s = a + b, d = a - b;
   a = s, b = d;
 }
+template <bool F6>
+constexpr int kQuadWords = 256 * (F6 ? 16 : 4);          // LDS of a workgroup
 template <bool HAD, bool F6>
-__global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
-                                                         __half* __restrict__ scales, uint32_t R, float scale_mul,
-                                                         uint32_t tokens, uint32_t groups_per_token) {
-  __shared__ __align__(16) unsigned turned[256 * (F6 ? 16 : 4)];
+__device__ __forceinline__ void group_quad_block(uint32_t block, const __half* __restrict__ x, uint8_t* __restrict__ q,
+                                                 __half* __restrict__ scales, uint32_t R, float scale_mul, uint32_t tokens,
+                                                 uint32_t groups_per_token, unsigned* turned) {
   const int tid = threadIdx.x, p = tid & 3;
-  const uint32_t row0 = blockIdx.x * kQuadRows, row = row0 + (tid >> 2);
+  const uint32_t row0 = block * kQuadRows, row = row0 + (tid >> 2);
   const bool valid = row < R;
   const uint32_t at = ((valid ? row : R - 1) - row0) * 256 + p * 16;   // bytes from the workgroup's first group
   const char* xb = (const char*)x + (size_t)row0 * 256;
@@ -375,6 +377,13 @@ __global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restric
   *(v4i*)(q + (size_t)row0 * 64 + tid * 16) = o;
   if (p == 0) scales[row] = scale_mul == 1.0f ? __builtin_bit_cast(__half, s) : __float2half(round_here((float)s * scale_mul));
 }
+template <bool HAD, bool F6>
+__global__ __launch_bounds__(256) void group_quad_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
+                                                         __half* __restrict__ scales, uint32_t R, float scale_mul,
+                                                         uint32_t tokens, uint32_t groups_per_token) {
+  __shared__ __align__(16) unsigned turned[kQuadWords<F6>];
+  group_quad_block<HAD, F6>(blockIdx.x, x, q, scales, R, scale_mul, tokens, groups_per_token, turned);
+}
 
 // the SwiGLU product alone, eight values per thread
 __global__ __launch_bounds__(256) void silu_mul_kernel(const __half* __restrict__ gate, const __half* __restrict__ up,
@@ -439,15 +448,14 @@ __global__ __launch_bounds__(256) void embed_kernel(const long long* __restrict_
 // RMSNorm in front of the group kernel, one workgroup per token row of K = 8 * chunks values (K <= 16384):
 // y = fp16( float(x) * rsqrt(sum(x^2) / K + eps) [* float(weight)] ) with the statistics in float32
 // (flh/nn/normalization.py:12-20), then transform + quantise per group of G as group_kernel<G, HAD, true>.
-template <int G, bool HAD, bool F6 = false>
-__global__ __launch_bounds__(256) void rmsnorm_group_kernel(const __half* __restrict__ x,
-                                                            const __half* __restrict__ weight, uint8_t* __restrict__ q,
-                                                            __half* __restrict__ scales, uint32_t K, float eps,
-                                                            float scale_mul) {
+template <int G, bool HAD, bool F6>
+__device__ __forceinline__ void rmsnorm_group_block(uint32_t token, uint32_t tokens, const __half* __restrict__ x,
+                                                    const __half* __restrict__ weight, uint8_t* __restrict__ q,
+                                                    __half* __restrict__ scales, uint32_t K, float eps, float scale_mul) {
   constexpr int LPR = G / 8, MAXC = 8;
   __shared__ float part[4];
   const int tid = threadIdx.x;
-  const uint32_t token = blockIdx.x, chunks = K / 8;
+  const uint32_t chunks = K / 8;
   const int lir = group_chunk<LPR>(tid % LPR);
   const uint32_t c0 = (tid / LPR) * LPR + lir;        // chunk of pass 0; pass i adds 256 i
   const __half* xr = x + (size_t)token * K;
@@ -489,9 +497,16 @@ __global__ __launch_bounds__(256) void rmsnorm_group_kernel(const __half* __rest
       }
       if constexpr (HAD) fwht_group_f16<G>(v, lir);
       const uint32_t row = token * (K / G) + c / LPR;
-      group_finish<G, F6>(v, lir, true, row, q, scales, scale_mul, gridDim.x, K / G);   // (a quad is inside one group)
+      group_finish<G, F6>(v, lir, true, row, q, scales, scale_mul, tokens, K / G);   // (a quad is inside one group)
     }
   }
+}
+template <int G, bool HAD, bool F6 = false>
+__global__ __launch_bounds__(256) void rmsnorm_group_kernel(const __half* __restrict__ x,
+                                                            const __half* __restrict__ weight, uint8_t* __restrict__ q,
+                                                            __half* __restrict__ scales, uint32_t K, float eps,
+                                                            float scale_mul) {
+  rmsnorm_group_block<G, HAD, F6>(blockIdx.x, gridDim.x, x, weight, q, scales, K, eps, scale_mul);
 }
 
 // RMSNorm on its own (a model's final norm, in front of an fp16 head), optionally behind the residual addition: one
@@ -551,20 +566,107 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const __half* __restri
 // 2. wave-per-row kernel, float32 butterflies, K = 512 * J: four rows per workgroup, rotate_quant_row (rotate_row.h)
 // ------------------------------------------------------------------------------------
 template <int J, bool HAD, bool EXACT_NORM, bool RMS, bool F6>
-__global__ __launch_bounds__(256) void rotate_quant_wave_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
+__device__ __forceinline__ void rotate_quant_wave_block(uint32_t block, const __half* __restrict__ x, uint8_t* __restrict__ q,
                                                                 __half* __restrict__ scales,
                                                                 __half* __restrict__ y_out, uint32_t M, float norm,
                                                                 float clip, const __half* __restrict__ rms_weight = nullptr,
                                                                 float rms_eps = 0.f, const __half* add = nullptr,
                                                                 __half* sum_out = nullptr) {
   constexpr int K = 512 * J;
-  const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
+  const uint32_t row = block * 4u + (threadIdx.x >> 6);
   if (row >= M) return;  // wave-uniform
   // F6: q is the encoded matrix of M rows in the 6-bit operand format instead of [M, K / 2] nibbles
   rotate_quant_row<J, HAD, EXACT_NORM, RMS, F6>(x + (size_t)row * K, F6 ? q : q + (size_t)row * (K / 2), scales + row,
                                             y_out ? y_out + (size_t)row * K : nullptr, norm, clip, rms_weight, rms_eps,
                                             add ? add + (size_t)row * K : nullptr,
                                             add ? sum_out + (size_t)row * K : nullptr, M, row);
+}
+template <int J, bool HAD, bool EXACT_NORM, bool RMS, bool F6>
+__global__ __launch_bounds__(256) void rotate_quant_wave_kernel(const __half* __restrict__ x, uint8_t* __restrict__ q,
+                                                                __half* __restrict__ scales,
+                                                                __half* __restrict__ y_out, uint32_t M, float norm,
+                                                                float clip, const __half* __restrict__ rms_weight = nullptr,
+                                                                float rms_eps = 0.f, const __half* add = nullptr,
+                                                                __half* sum_out = nullptr) {
+  rotate_quant_wave_block<J, HAD, EXACT_NORM, RMS, F6>(blockIdx.x, x, q, scales, y_out, M, norm, clip, rms_weight, rms_eps, add, sum_out);
+}
+
+// A quantiser and the encoding of the weights that its codes meet, which does not depend on it, in one launch: the quantiser's workgroups
+// first, the encoding's as compute units have room.  Saves the drain between the two and most of the shorter one's time where that one
+// does not fill the memory.  us, two launches -> one (replayed in a graph, weights from memory):
+//   norm and groups, 531 x 4096 beside 28672 / 6144 rows of weights  34.3 -> 29.9 / 14.5 -> 11.4; 2048: 39.4 -> 33.8 / 20.0 -> 17.0;
+//     8192: 58.6 -> 56.6 / 40.0 -> 37.1
+//   groups, beside 4096 rows: 531 x 4096 10.0 -> 7.9, 531 x 14336 23.2 -> 19.1, 2048 35.6 -> 29.8, 4096 51.2 -> 44.2, 6144 66.8 -> 63.0
+//   rotation, 531 x 4096 beside 4096 rows 12.1 -> 9.1, 8192 33.4 -> 30.4; with the norm beside 28672, 2048 41.8 -> 40.6, 8192 63.6 -> 60.2
+// (The two kinds of workgroup share their LDS: 28 KB instead of 16 costs the group quantiser waves, 2048 x 14336 30.5 instead of 29.8.)
+template <typename Quantise>
+__global__ __launch_bounds__(256) void quantise_encode_kernel(const Quantise quantise, uint32_t quant_blocks, const EncodeArgs encode,
+                                                              uint32_t encode_x) {
+  __shared__ __align__(16) uint8_t lds[Quantise::kLds > kEncodeLds ? Quantise::kLds : kEncodeLds];
+  if (blockIdx.x < quant_blocks) {
+    quantise(blockIdx.x, lds);
+  } else {
+    const uint32_t i = blockIdx.x - quant_blocks;
+    encode_f6_block(encode, i % encode_x, i / encode_x, lds);
+  }
+}
+template <bool QUAD>
+struct GroupQuantise {                               // groups of 128, 6-bit output
+  const __half* x;
+  uint8_t* q;
+  __half* scales;
+  uint32_t R;
+  float scale_mul;
+  uint32_t tokens, groups_per_token;
+  static constexpr int kLds = QUAD ? 4 * kQuadWords<true> : 0;
+  __device__ void operator()(uint32_t block, uint8_t* lds) const {
+    if constexpr (QUAD) {
+      group_quad_block<false, true>(block, x, q, scales, R, scale_mul, tokens, groups_per_token, (unsigned*)lds);
+    } else {
+      const uint32_t gl = block * 256u + threadIdx.x;
+      quantise_group<128, false, true>(x, q, scales, gl / 16, group_chunk<16>(gl % 16), R, scale_mul, tokens, groups_per_token);
+    }
+  }
+};
+struct NormGroupQuantise {
+  const __half *x, *weight;
+  uint8_t* q;
+  __half* scales;
+  uint32_t K;
+  float eps;
+  uint32_t tokens;
+  static constexpr int kLds = 0;
+  __device__ void operator()(uint32_t block, uint8_t*) const {
+    rmsnorm_group_block<128, false, true>(block, tokens, x, weight, q, scales, K, eps, 1.0f);
+  }
+};
+template <bool RMS>
+struct RotateQuantise {                              // rows of 4096 rotated, one scale each
+  const __half* x;
+  uint8_t* q;
+  __half* scales;
+  uint32_t M;
+  float clip;
+  const __half* weight;
+  float eps;
+  const __half* add;
+  __half* sum_out;
+  static constexpr int kLds = 0;
+  __device__ void operator()(uint32_t block, uint8_t*) const {
+    rotate_quant_wave_block<8, true, true, RMS, true>(block, x, q, scales, nullptr, M, 1.0f / 64.0f, clip, weight, eps, add, sum_out);
+  }
+};
+// Whether the two take one launch.  A quantiser that fills the memory by itself gains nothing and, where its values no longer fit the
+// caches, loses: 8192 x 11008 (90 M values) 63.4 -> 58.6, 8192 x 14336 (117 M) 83.8 -> 92.9, 32768 x 4096 (134 M) 134.7 -> 138.4 with the
+// norm and 28672 rows, 117.3 -> 115.1 with 6144.
+constexpr uint64_t kBesideValues = 100ull << 20;
+inline bool beside(uint64_t quant_blocks, uint64_t values, const EncodeLaunch& e) {
+  return e.x > 0 && values <= kBesideValues && quant_blocks + (uint64_t)e.x * e.y <= 0x7FFFFFFFull;
+}
+template <typename Quantise>
+int launch_beside(const Quantise& q, uint32_t quant_blocks, const EncodeLaunch& e, hipStream_t stream) {
+  hipLaunchKernelGGL(quantise_encode_kernel<Quantise>, dim3(quant_blocks + e.x * e.y), dim3(256), 0, stream, q, quant_blocks, e.args, e.x);
+  return check_launch("quantise_encode");
 }
 
 constexpr int kGenericThreads = 1024;      // one workgroup per compute unit (LDS): two waves per SIMD hide latencies
@@ -1064,9 +1166,13 @@ extern "C" int flh_add_rmsnorm_rotate_quant_i4(const flh_half* x, const flh_half
   }
 }
 
-extern "C" int flh_rotate_quant_f6(const flh_half* x, const flh_half* add, flh_half* sum_out, int rmsnorm,
-                                   const flh_half* weight, float eps, uint8_t* encoded, flh_half* scales, uint32_t M,
-                                   uint32_t K, int hadamard, float clip_ratio, void* stream) {
+namespace {
+// what a call without weights to encode has, and what one that has launched them separately is left with
+const EncodeLaunch kNoWeights{};
+
+int rotate_quant_f6(const flh_half* x, const flh_half* add, flh_half* sum_out, int rmsnorm, const flh_half* weight, float eps,
+                    uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard, float clip_ratio, const EncodeLaunch& e,
+                    bool* taken, void* stream) {
   const char* who = "rotate_quant_f6";
   if (!x || !encoded || !scales) return fail(FLH_EINVAL, "%s: null pointer", who);
   if (misaligned16(x, encoded)) return fail(FLH_EINVAL, "%s: x and encoded must be 16-byte aligned", who);
@@ -1093,6 +1199,12 @@ extern "C" int flh_rotate_quant_f6(const flh_half* x, const flh_half* add, flh_h
   if (K % 512 || !is_pow2(K / 512) || K > 8192)
     return fail(FLH_EINVAL, "%s: K (%u) must be 512, 1024, 2048, 4096 or 8192 (or 11008 / 14336 on the matrix cores)", who, K);
   const bool had = hadamard != FLH_HAD_NONE;
+  if (K == 4096 && had && beside((M + 3ull) / 4, (uint64_t)M * K, e)) {
+    *taken = true;
+    const uint32_t blocks = (uint32_t)((M + 3ull) / 4);
+    if (rmsnorm) return launch_beside(RotateQuantise<true>{xh, encoded, sh, M, clip_ratio, wh, eps, ah, oh}, blocks, e, st);
+    return launch_beside(RotateQuantise<false>{xh, encoded, sh, M, clip_ratio, nullptr, 0.f, nullptr, nullptr}, blocks, e, st);
+  }
   if (rmsnorm) {
     switch (K / 512) {
       case 1: return launch_wave_rms<1, true>(xh, wh, eps, encoded, sh, nullptr, M, had, clip_ratio, st, ah, oh);
@@ -1111,6 +1223,34 @@ extern "C" int flh_rotate_quant_f6(const flh_half* x, const flh_half* add, flh_h
   }
 }
 
+// a quantiser's call, then the weights if it has not taken them into its launch
+template <typename F>
+int with_weights(const flh_encode_list* weights, uint32_t M, void* stream, F&& quantise) {
+  EncodeLaunch e{};
+  if (weights)
+    if (int rc = encode_launch(weights->count, weights->packed, weights->encoded, weights->rows, weights->K, e)) return rc;
+  bool taken = false;
+  if (M > 0 || !weights)                             // (no rows: there may be no pointers either)
+    if (int rc = quantise(e, &taken)) return rc;
+  if (taken || e.x == 0) return FLH_OK;
+  return flh_encode_f6_multi(weights->count, weights->packed, weights->encoded, weights->rows, weights->K, stream);
+}
+}  // namespace
+
+extern "C" int flh_rotate_quant_f6(const flh_half* x, const flh_half* add, flh_half* sum_out, int rmsnorm,
+                                   const flh_half* weight, float eps, uint8_t* encoded, flh_half* scales, uint32_t M,
+                                   uint32_t K, int hadamard, float clip_ratio, void* stream) {
+  return rotate_quant_f6(x, add, sum_out, rmsnorm, weight, eps, encoded, scales, M, K, hadamard, clip_ratio, kNoWeights, nullptr, stream);
+}
+
+extern "C" int flh_rotate_quant_encode_f6(const flh_half* x, const flh_half* add, flh_half* sum_out, int rmsnorm,
+                                          const flh_half* weight, float eps, uint8_t* encoded, flh_half* scales, uint32_t M,
+                                          uint32_t K, int hadamard, float clip_ratio, const flh_encode_list* weights, void* stream) {
+  return with_weights(weights, M, stream, [&](const EncodeLaunch& e, bool* taken) {
+    return rotate_quant_f6(x, add, sum_out, rmsnorm, weight, eps, encoded, scales, M, K, hadamard, clip_ratio, e, taken, stream);
+  });
+}
+
 extern "C" int flh_silu_mul_f16(const flh_half* gate, const flh_half* up, flh_half* out, uint64_t n, void* stream) {
   if (!gate || !up || !out) return fail(FLH_EINVAL, "silu_mul: null pointer");
   if (misaligned16(gate, up, out)) return fail(FLH_EINVAL, "silu_mul: gate, up and out must be 16-byte aligned");
@@ -1124,8 +1264,9 @@ extern "C" int flh_silu_mul_f16(const flh_half* gate, const flh_half* up, flh_ha
 
 // The two producers of the group configuration writing the 6-bit operand format: groups of 128, no rotation.  A pass that
 // re-encodes the nibbles costs 4-6 us per 1000 tokens in front of every GEMM.
-extern "C" int flh_rmsnorm_group_quant_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales,
-                                          uint32_t M, uint32_t K, float eps, void* stream) {
+namespace {
+int rmsnorm_group_quant_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, float eps,
+                           const EncodeLaunch& e, bool* taken, void* stream) {
   if (!x || !encoded || !scales) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: null pointer");
   if (misaligned16(x, encoded) || (weight && misaligned16(weight)))
     return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: x, weight and encoded must be 16-byte aligned");
@@ -1133,9 +1274,27 @@ extern "C" int flh_rmsnorm_group_quant_f6(const flh_half* x, const flh_half* wei
   if (K == 0 || K % 128 || K > 16384u) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: K (%u) must be a multiple of 128, at most 16384", K);
   if ((uint64_t)M * (K / 128) > 0xFFFFFFFFull) return fail(FLH_EINVAL, "rmsnorm_group_quant_f6: too many groups");
   if (M == 0) return FLH_OK;
-  hipLaunchKernelGGL((rmsnorm_group_kernel<128, false, true>), dim3(M), dim3(256), 0, (hipStream_t)stream, (const __half*)x,
-                     (const __half*)weight, encoded, (__half*)scales, K, eps, 1.0f);
+  const __half *xh = (const __half*)x, *wh = (const __half*)weight;
+  if (beside(M, (uint64_t)M * K, e)) {
+    *taken = true;
+    return launch_beside(NormGroupQuantise{xh, wh, encoded, (__half*)scales, K, eps, M}, M, e, (hipStream_t)stream);
+  }
+  hipLaunchKernelGGL((rmsnorm_group_kernel<128, false, true>), dim3(M), dim3(256), 0, (hipStream_t)stream, xh, wh, encoded,
+                     (__half*)scales, K, eps, 1.0f);
   return check_launch("rmsnorm_group_kernel (6-bit output)");
+}
+}  // namespace
+
+extern "C" int flh_rmsnorm_group_quant_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales,
+                                          uint32_t M, uint32_t K, float eps, void* stream) {
+  return rmsnorm_group_quant_f6(x, weight, encoded, scales, M, K, eps, kNoWeights, nullptr, stream);
+}
+
+extern "C" int flh_rmsnorm_group_quant_encode_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales, uint32_t M,
+                                                 uint32_t K, float eps, const flh_encode_list* weights, void* stream) {
+  return with_weights(weights, M, stream, [&](const EncodeLaunch& e, bool* taken) {
+    return rmsnorm_group_quant_f6(x, weight, encoded, scales, M, K, eps, e, taken, stream);
+  });
 }
 
 extern "C" int flh_silu_mul_group_quant_f6(const flh_half* gate, const flh_half* up, uint8_t* encoded, flh_half* scales,
@@ -1195,8 +1354,9 @@ extern "C" int flh_silu_mul_rotate_quant_i4(const flh_half* gate, const flh_half
                                            (hipStream_t)stream);
 }
 
-extern "C" int flh_group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K,
-                                  int hadamard, float scale_mul, void* stream) {
+namespace {
+int group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard, float scale_mul,
+                   const EncodeLaunch& e, bool* taken, void* stream) {
   if (!x || !encoded || !scales) return fail(FLH_EINVAL, "group_quant_f6: null pointer");
   if (misaligned16(x, encoded)) return fail(FLH_EINVAL, "group_quant_f6: x and encoded must be 16-byte aligned");
   if (!(scale_mul > 0.f)) return fail(FLH_EINVAL, "group_quant_f6: scale_mul must be positive");
@@ -1206,7 +1366,16 @@ extern "C" int flh_group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half*
   const uint32_t R = M * (K / 128);
   const dim3 grid((unsigned)(((uint64_t)R * 16 + 255) / 256)), block(256);
   const __half* xh = (const __half*)x;
-  if (R >= quad_min_rows(hadamard != 0, true))
+  const bool quad = R >= quad_min_rows(hadamard != 0, true);
+  const uint64_t quad_blocks = ((uint64_t)R + kQuadRows - 1) / kQuadRows;
+  if (!hadamard && beside(quad ? quad_blocks : grid.x, (uint64_t)M * K, e)) {
+    *taken = true;
+    __half* sh = (__half*)scales;
+    const hipStream_t st = (hipStream_t)stream;
+    if (quad) return launch_beside(GroupQuantise<true>{xh, encoded, sh, R, scale_mul, M, K / 128}, (uint32_t)quad_blocks, e, st);
+    return launch_beside(GroupQuantise<false>{xh, encoded, sh, R, scale_mul, M, K / 128}, grid.x, e, st);
+  }
+  if (quad)
     return hadamard ? launch_group_quad<true, true>(xh, encoded, (__half*)scales, R, scale_mul, M, K / 128, (hipStream_t)stream)
                     : launch_group_quad<false, true>(xh, encoded, (__half*)scales, R, scale_mul, M, K / 128, (hipStream_t)stream);
   if (hadamard)
@@ -1216,6 +1385,19 @@ extern "C" int flh_group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half*
     hipLaunchKernelGGL((group_kernel<128, false, true, true>), grid, block, 0, (hipStream_t)stream, xh, encoded,
                        (__half*)scales, nullptr, R, scale_mul, M, K / 128);
   return check_launch("group_kernel (6-bit output)");
+}
+}  // namespace
+
+extern "C" int flh_group_quant_f6(const flh_half* x, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K,
+                                  int hadamard, float scale_mul, void* stream) {
+  return group_quant_f6(x, encoded, scales, M, K, hadamard, scale_mul, kNoWeights, nullptr, stream);
+}
+
+extern "C" int flh_group_quant_encode_f6(const flh_half* x, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard,
+                                         float scale_mul, const flh_encode_list* weights, void* stream) {
+  return with_weights(weights, M, stream, [&](const EncodeLaunch& e, bool* taken) {
+    return group_quant_f6(x, encoded, scales, M, K, hadamard, scale_mul, e, taken, stream);
+  });
 }
 
 extern "C" int flh_fwht_f16_inplace(flh_half* x, uint32_t R, int group, void* stream) {

@@ -258,32 +258,53 @@ Tensor gemm_i4_qkv_rope(const Tensor& A, const Tensor& A_scale, const std::vecto
 }
 
 // ---- the 6-bit operand format -------------------------------------------------------------------------------------------
-std::vector<Tensor> encode_f6_many(const std::vector<Tensor>& packed) {
-  TORCH_CHECK(!packed.empty() && packed.size() <= 4, "one to four matrices");
-  for (const Tensor& p : packed) {
-    TORCH_CHECK(p.is_cuda() && p.scalar_type() == torch::kUInt8 && p.dim() == 2 && p.is_contiguous() &&
-                    p.device() == packed[0].device(),
-                "packed codes must be contiguous 2D uint8 CUDA tensors on one device");
-    TORCH_CHECK(p.size(1) == packed[0].size(1), "the matrices must share K");
-  }
-  const int64_t K = packed[0].size(1) * 2;
-  TORCH_CHECK(K % 128 == 0, "K must be a multiple of 128");
+struct EncodeF6 {   // up to four packed matrices of one K and the tensors that their encodings go to
+  flh_encode_list list{};
   std::vector<Tensor> outs;
-  const uint8_t* in[4];
-  uint8_t* out[4];
-  size_t rows[4];
-  for (size_t i = 0; i < packed.size(); ++i) {
-    outs.push_back(torch::empty({packed[i].size(0), K / 128 * 96}, packed[i].options()));
-    in[i] = u8(packed[i]);
-    out[i] = (uint8_t*)outs[i].data_ptr();
-    rows[i] = (size_t)packed[i].size(0);
+  explicit EncodeF6(const std::vector<Tensor>& packed) {
+    TORCH_CHECK(!packed.empty() && packed.size() <= 4, "one to four matrices");
+    for (const Tensor& p : packed) {
+      TORCH_CHECK(p.is_cuda() && p.scalar_type() == torch::kUInt8 && p.dim() == 2 && p.is_contiguous() &&
+                      p.device() == packed[0].device(),
+                  "packed codes must be contiguous 2D uint8 CUDA tensors on one device");
+      TORCH_CHECK(p.size(1) == packed[0].size(1), "the matrices must share K");
+    }
+    const int64_t K = packed[0].size(1) * 2;
+    TORCH_CHECK(K % 128 == 0, "K must be a multiple of 128");
+    list.count = (int)packed.size(), list.K = (size_t)K;
+    for (size_t i = 0; i < packed.size(); ++i) {
+      outs.push_back(torch::empty({packed[i].size(0), K / 128 * 96}, packed[i].options()));
+      list.packed[i] = u8(packed[i]);
+      list.encoded[i] = (uint8_t*)outs[i].data_ptr();
+      list.rows[i] = (size_t)packed[i].size(0);
+    }
   }
-  if (K) {
+};
+
+std::vector<Tensor> encode_f6_many(const std::vector<Tensor>& packed) {
+  EncodeF6 e(packed);
+  if (e.list.K) {
     Launch l(packed[0]);
-    ok(flh_encode_f6_multi((int)packed.size(), in, out, rows, K, stream_of(packed[0])));
+    ok(flh_encode_f6_multi(e.list.count, e.list.packed, e.list.encoded, e.list.rows, e.list.K, stream_of(packed[0])));
   }
-  return outs;
+  return e.outs;
 }
+
+// the weights that the codes of a quantiser on x are to meet, encoded beside it; none: the quantiser alone
+using Weights = c10::optional<std::vector<Tensor>>;
+struct BesideQuantiser {
+  c10::optional<EncodeF6> e;
+  BesideQuantiser(const Weights& weights, const Tensor& x) {
+    if (!weights.has_value()) return;
+    e.emplace(*weights);
+    TORCH_CHECK((*weights)[0].device() == x.device() && e->list.K == (size_t)x.size(1), "weights must be on x's device and of its K");
+  }
+  const flh_encode_list* list() const { return e.has_value() ? &e->list : nullptr; }
+  std::vector<Tensor> with(std::vector<Tensor> out) const {
+    if (e.has_value()) out.insert(out.end(), e->outs.begin(), e->outs.end());
+    return out;
+  }
+};
 
 struct F6Rows {   // rows of fp16 values and where their codes and group scales go
   int64_t M, K;
@@ -300,31 +321,33 @@ struct F6Rows {   // rows of fp16 values and where their codes and group scales 
   }
 };
 
-std::vector<Tensor> group_quantize_f6(const Tensor& x, bool hadamard, double scale_mul) {
+std::vector<Tensor> group_quantize_f6(const Tensor& x, bool hadamard, double scale_mul, const Weights& weights) {
   F6Rows r(x);
+  const BesideQuantiser w(weights, x);
   r.allocate(x);
-  if (r.M) {
+  if (r.M || w.list()) {
     Launch l(x);
-    ok(flh_group_quant_f6(h(x), (uint8_t*)r.q.data_ptr(), hm(r.s), (uint32_t)r.M, (uint32_t)r.K, hadamard ? 1 : 0, (float)scale_mul,
-                          stream_of(x)));
+    ok(flh_group_quant_encode_f6(h(x), (uint8_t*)r.q.data_ptr(), hm(r.s), (uint32_t)r.M, (uint32_t)r.K, hadamard ? 1 : 0,
+                                 (float)scale_mul, w.list(), stream_of(x)));
   }
-  return {r.q, r.s};
+  return w.with({r.q, r.s});
 }
 
-std::vector<Tensor> rmsnorm_group_quantize_f6(const Tensor& x, const c10::optional<Tensor>& weight, double eps) {
+std::vector<Tensor> rmsnorm_group_quantize_f6(const Tensor& x, const c10::optional<Tensor>& weight, double eps, const Weights& weights) {
   F6Rows r(x);
+  const BesideQuantiser w(weights, x);
   TORCH_CHECK(r.K <= 16384, "Last dimension must be at most 16384");
   if (weight.has_value())
     TORCH_CHECK(weight->is_cuda() && weight->scalar_type() == torch::kFloat16 && weight->is_contiguous() &&
                     weight->numel() == r.K && weight->device() == x.device(),
                 "weight must be a contiguous float16 CUDA tensor of K values");
   r.allocate(x);
-  if (r.M) {
+  if (r.M || w.list()) {
     Launch l(x);
-    ok(flh_rmsnorm_group_quant_f6(h(x), weight.has_value() ? h(*weight) : nullptr, (uint8_t*)r.q.data_ptr(), hm(r.s), (uint32_t)r.M,
-                                  (uint32_t)r.K, (float)eps, stream_of(x)));
+    ok(flh_rmsnorm_group_quant_encode_f6(h(x), weight.has_value() ? h(*weight) : nullptr, (uint8_t*)r.q.data_ptr(), hm(r.s),
+                                         (uint32_t)r.M, (uint32_t)r.K, (float)eps, w.list(), stream_of(x)));
   }
-  return {r.q, r.s};
+  return w.with({r.q, r.s});
 }
 
 std::vector<Tensor> silu_mul_group_quantize_f6(const Tensor& gate, const Tensor& up) {
@@ -773,10 +796,12 @@ std::vector<Tensor> add_rmsnorm_rotate_and_quantize_i4_mode(const Tensor& x, con
 
 // codes in the 6-bit operand format: {codes, scales}, behind {x + add, ...} if there is one
 std::vector<Tensor> rotate_and_quantize_f6_mode(const Tensor& x, int64_t mode, double clip_ratio, const c10::optional<Tensor>& norm_weight,
-                                                const c10::optional<double>& eps, const c10::optional<Tensor>& add) {
+                                                const c10::optional<double>& eps, const c10::optional<Tensor>& add,
+                                                const Weights& weights) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kFloat16 && x.dim() == 2 && x.is_contiguous(),
               "Input tensor must be a contiguous 2D float16 CUDA tensor");
   const int64_t M = x.size(0), K = x.size(1);
+  const BesideQuantiser w(weights, x);
   TORCH_CHECK(!add.has_value() || eps.has_value(), "the residual addition comes with the RMSNorm prologue (eps)");
   if (add.has_value())
     TORCH_CHECK(add->is_cuda() && add->scalar_type() == torch::kFloat16 && add->sizes() == x.sizes() && add->is_contiguous() &&
@@ -790,14 +815,15 @@ std::vector<Tensor> rotate_and_quantize_f6_mode(const Tensor& x, int64_t mode, d
   Tensor s = torch::empty({M, 1}, x.options());
   Tensor total;
   if (add.has_value()) total = torch::empty_like(x);
-  if (M) {
+  if (M || w.list()) {
     Launch l(x);
-    ok(flh_rotate_quant_f6(h(x), add.has_value() ? h(*add) : nullptr, add.has_value() ? hm(total) : nullptr, eps.has_value() ? 1 : 0,
-                           norm_weight.has_value() ? h(*norm_weight) : nullptr, (float)eps.value_or(0.0), (uint8_t*)q.data_ptr(), hm(s),
-                           (uint32_t)M, (uint32_t)K, (int)mode, (float)clip_ratio, stream_of(x)));
+    ok(flh_rotate_quant_encode_f6(h(x), add.has_value() ? h(*add) : nullptr, add.has_value() ? hm(total) : nullptr,
+                                  eps.has_value() ? 1 : 0, norm_weight.has_value() ? h(*norm_weight) : nullptr, (float)eps.value_or(0.0),
+                                  (uint8_t*)q.data_ptr(), hm(s), (uint32_t)M, (uint32_t)K, (int)mode, (float)clip_ratio, w.list(),
+                                  stream_of(x)));
   }
-  if (add.has_value()) return {total, q, s};
-  return {q, s};
+  if (add.has_value()) return w.with({total, q, s});
+  return w.with({q, s});
 }
 
 // ---- fused producers -------------------------------------------------------------------------------------------------
@@ -1010,8 +1036,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_i4_qkv_rope", &gemm_i4_qkv_rope, py::arg("A"), py::arg("A_scale"), py::arg("Bs"), py::arg("B_scales"), py::arg("cos"),
         py::arg("sin"), py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"), py::arg("batch"), py::arg("group_size") = 128);
   m.def("encode_f6_many", &encode_f6_many, py::arg("packed"));
-  m.def("group_quantize_f6", &group_quantize_f6, py::arg("x"), py::arg("hadamard") = true, py::kw_only(), py::arg("scale_mul") = 1.0);
-  m.def("rmsnorm_group_quantize_f6", &rmsnorm_group_quantize_f6, py::arg("x"), py::arg("weight"), py::arg("eps"));
+  m.def("group_quantize_f6", &group_quantize_f6, py::arg("x"), py::arg("hadamard") = true, py::kw_only(), py::arg("scale_mul") = 1.0,
+        py::arg("weights") = py::none());
+  m.def("rmsnorm_group_quantize_f6", &rmsnorm_group_quantize_f6, py::arg("x"), py::arg("weight"), py::arg("eps"),
+        py::arg("weights") = py::none());
   m.def("silu_mul_group_quantize_f6", &silu_mul_group_quantize_f6, py::arg("gate"), py::arg("up"));
   m.def("gemm_f6_dequant_o16", &gemm_f6_dequant_o16, py::arg("A6"), py::arg("B6"), py::arg("A_scale"), py::arg("B_scale"));
   m.def("gemm_f6_dequant_o16_gs", &gemm_f6_dequant_o16_gs, py::arg("A6"), py::arg("B6"), py::arg("A_scale"), py::arg("B_scale"));

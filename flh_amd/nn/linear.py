@@ -106,12 +106,25 @@ class LinearFLH(torch.nn.Module):
         return self._w6
 
     @staticmethod
+    def _weights_to_encode(layers):
+        """The packed weights of layers that share their activations and keep no 6-bit encoding, for one launch to encode; None
+        where one of them keeps its own."""
+        if len(layers) <= 4 and all(type(l) is LinearFLH and l.in_features == layers[0].in_features
+                                    and not l._keeps_six_bit(l.w_scale.numel() > l.out_features) for l in layers):
+            return [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers]
+        return None
+
+    @staticmethod
+    def _beside_quantiser(layers):
+        """Arguments of the quantiser in front of `layers` that has it encode their weights as well, if they are to be encoded."""
+        packed = LinearFLH._weights_to_encode(layers)
+        return {} if packed is None or not packed[0].is_cuda else {"weights": packed}
+
+    @staticmethod
     def _six_bit_weights_of(layers):
         """[l._six_bit_weights() for l in layers], encodings that are not kept built in one launch."""
-        if 1 < len(layers) <= 4 and all(type(l) is LinearFLH and l.in_features == layers[0].in_features
-                                        and not l._keeps_six_bit(l.w_scale.numel() > l.out_features) for l in layers):
-            return _pkg._CUDA.encode_f6_many([l.w_packed.view(l.out_features, l.in_features // 2) for l in layers])
-        return [l._six_bit_weights() for l in layers]
+        packed = LinearFLH._weights_to_encode(layers) if len(layers) > 1 else None
+        return [l._six_bit_weights() for l in layers] if packed is None else _pkg._CUDA.encode_f6_many(packed)
 
     _SIX_BIT_MAX_ROWS = ((1 << 32) - 1) // 96       # rows of either operand that the 6-bit launches index; more go to int8
 
@@ -147,12 +160,14 @@ class LinearFLH(torch.nn.Module):
         return self._six_bit_rows(w_scale.numel() > self.out_features, None, nibbles, groups)
 
     # ------------------------------------------------------------------ kernels
-    def forward(self, x, a_scale=None, a_zero=None, x_is_packed=False, is_symmetric=None, residual=None):
+    def forward(self, x, a_scale=None, a_zero=None, x_is_packed=False, is_symmetric=None, residual=None, w6=None):
         """x: packed int4 activations [..., K/2] uint8; a_scale [..., K/in_group] or [..., 1]
         fp16 (as returned by ActQuantizer).  Returns fp16 [..., N].  `residual` (extension; fp16 [..., N]): returns
         residual + forward(x, ...) from the same launch -- the layer output rounded to fp16 as always, then one fp16
-        addition in the GEMM's epilogue instead of a separate pass over both tensors."""
-        if residual is None and a_scale is not None:
+        addition in the GEMM's epilogue instead of a separate pass over both tensors.  `w6` (extension, here and in
+        forward_many and forward_swiglu): with activations in the 6-bit format, the encodings of the weights, a list in the order of
+        the layers, where the quantiser's launch has made them (`weights` of rotate_and_quantize_f6 and its like)."""
+        if residual is None and a_scale is not None and w6 is None:
             w, w_scale = self._buffers.get("w_packed"), self._buffers.get("w_scale")
             if w is not None and w_scale is not None:
                 k, least = self.in_features, self.TRANSIENT_ROWS_GROUPS
@@ -163,7 +178,7 @@ class LinearFLH(torch.nn.Module):
                     return y if self.bias is None else y + self.bias
         lead = x.shape[:-1]
         if residual is not None and self.bias is not None:
-            return residual + self.forward(x, a_scale, a_zero, x_is_packed, is_symmetric)
+            return residual + self.forward(x, a_scale, a_zero, x_is_packed, is_symmetric, w6=w6)
         res = None if residual is None else residual.reshape(-1, self.out_features)
         rows = x.view(-1, x.size(-1))
         w_scale = self.w_scale.view(self.out_features, -1)
@@ -172,7 +187,7 @@ class LinearFLH(torch.nn.Module):
         encoded = rows.size(1) * 4 == self.in_features * 3      # activations already in the 6-bit format
         if encoded or self._six_bit_applies(rows, a_rows, w_scale, group):
             ops = _pkg._CUDA
-            w6 = self._six_bit_weights()
+            w6 = self._six_bit_weights() if w6 is None else w6[0]
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
             if encoded and not ((w_scale.size(1) == 1 and a_rows.size(1) == 1) or
                                 (group == 128 and w_scale.size(1) == self.in_features // 128)):
@@ -197,7 +212,7 @@ class LinearFLH(torch.nn.Module):
         return y.view(*lead, self.out_features)
 
     @staticmethod
-    def forward_many(layers, x, a_scale):
+    def forward_many(layers, x, a_scale, w6=None):
         """[layer(x, a_scale, x_is_packed=True) for layer in layers] in one GEMM launch: for projections that share
         their quantised input (q / k / v, gate / up; at most four), each with its own weights where they are.
         Same bits as the separate calls."""
@@ -216,14 +231,14 @@ class LinearFLH(torch.nn.Module):
         if encoded or all(l._six_bit_applies(rows, a_rows, ws, group, columns) for l, ws in zip(layers, w_scales)):
             # every layer takes the 6-bit matrix instruction here: one launch there as well
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            ys = ops.gemm_f6_dequant_multi(a6, LinearFLH._six_bit_weights_of(layers), a_rows.contiguous(), w_scales)
+            ys = ops.gemm_f6_dequant_multi(a6, w6 or LinearFLH._six_bit_weights_of(layers), a_rows.contiguous(), w_scales)
         else:
             ys = ops.gemm_i4_dequant_multi(rows, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
                                            a_rows, w_scales, group)
         return [(y if l.bias is None else y + l.bias).view(*lead, l.out_features) for y, l in zip(ys, layers)]
 
     @staticmethod
-    def forward_swiglu(gate_layer, up_layer, x, a_scale):
+    def forward_swiglu(gate_layer, up_layer, x, a_scale, w6=None):
         """act_fn(gate_layer(x)) * up_layer(x) of a SwiGLU MLP (flh/quantized_model/modeling_llama.py:522-526) in one
         GEMM launch that stores only the product: x packed codes [..., K/2], a_scale as for forward.  The two
         projections are rounded to fp16 as their own calls would store them, then combined as torch's fp16 silu and
@@ -245,7 +260,7 @@ class LinearFLH(torch.nn.Module):
                 l._six_bit_applies(rows, a_rows, l.w_scale.view(n, -1), group, 2 * n) for l in both):
             ops = _pkg._CUDA
             a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            y = ops.gemm_f6_swiglu(a6, *LinearFLH._six_bit_weights_of(both), a_rows.contiguous(),
+            y = ops.gemm_f6_swiglu(a6, *(w6 or LinearFLH._six_bit_weights_of(both)), a_rows.contiguous(),
                                    gate_layer.w_scale.view(n, -1), up_layer.w_scale.view(n, -1))
             return y.view(*lead, n)
         y = _pkg._CUDA.gemm_i4_swiglu(rows, gate_layer.w_packed.view(n, k // 2), up_layer.w_packed.view(n, k // 2),
@@ -283,8 +298,8 @@ class LinearFLH(torch.nn.Module):
               and self.wants_six_bit(rows.size(0))) and (
                 hadamard in (True, "fast") or (hadamard == "exact" and self.in_features == 4096)):
             # long calls: the quantiser writes the 6-bit operand format
-            q, s = ops.rotate_and_quantize_f6(rows, hadamard=hadamard)
-            return self.forward(q, s, x_is_packed=True).view(*lead, self.out_features)
+            q, s, *w6 = ops.rotate_and_quantize_f6(rows, hadamard=hadamard, **self._beside_quantiser((self,)))
+            return self.forward(q, s, x_is_packed=True, **({"w6": w6} if w6 else {})).view(*lead, self.out_features)
         else:
             q, s = ops.rotate_and_quantize_i4(rows, hadamard=hadamard)
             y = ops.gemm_i4_dequant(q, w, s, w_scale, group)

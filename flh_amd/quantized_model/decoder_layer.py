@@ -270,16 +270,18 @@ class W4A4DecoderLayer(torch.nn.Module):
         return "fast" if fast else True
 
     def _token_quant(self, stage, x, norm=None, norm_name=None, consumers=()):
-        """Whole-row rotation + one scale per token (after RMSNorm when `norm` is given)."""
+        """Whole-row rotation + one scale per token (after RMSNorm when `norm` is given): (scales, zeros, codes).  Codes in the 6-bit
+        format have no zeros: there, as from the other quantisers below, the second value is the list of the consumers' weights
+        that the same call has encoded, or None."""
         rows = x.reshape(-1, x.size(-1)).contiguous()
         mode = self._rotation_mode(rows.size(0), rows.size(1))
         if self._six_bit_for(consumers, rows.size(0), rows.size(1)):
             if norm is not None:
-                q, s = _ops().rotate_and_quantize_f6(rows, hadamard=mode, norm_weight=self._norm_weight16(norm_name, norm),
-                                                     eps=norm.eps)
+                q, s, *w6 = _ops().rotate_and_quantize_f6(rows, hadamard=mode, norm_weight=self._norm_weight16(norm_name, norm),
+                                                          eps=norm.eps, **LinearFLH._beside_quantiser(consumers))
             else:
-                q, s = _ops().rotate_and_quantize_f6(rows, hadamard=mode)
-            return s.view(*x.shape[:-1], 1), None, q.view(*x.shape[:-1], -1)
+                q, s, *w6 = _ops().rotate_and_quantize_f6(rows, hadamard=mode, **LinearFLH._beside_quantiser(consumers))
+            return s.view(*x.shape[:-1], 1), w6 or None, q.view(*x.shape[:-1], -1)
         if norm is not None and self.fused:
             q, s = _ops().rmsnorm_rotate_and_quantize_i4(rows, self._norm_weight16(norm_name, norm), norm.eps, hadamard=mode)
         else:
@@ -293,9 +295,9 @@ class W4A4DecoderLayer(torch.nn.Module):
         if self.activation == "token":
             return self._token_quant(stage, x, norm, norm_name, consumers)
         if self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)):
-            q, s = _ops().rmsnorm_group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), self._norm_weight16(norm_name, norm),
-                                                    norm.eps)
-            return s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
+            q, s, *w6 = _ops().rmsnorm_group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), self._norm_weight16(norm_name, norm),
+                                                         norm.eps, **LinearFLH._beside_quantiser(consumers))
+            return s.view(*x.shape[:-1], -1), w6 or None, q.view(*x.shape[:-1], -1)
         if self.fused:
             q, s = _ops().rmsnorm_and_quantize_i4_gs(x.reshape(-1, x.size(-1)).contiguous(),
                                                      self._norm_weight16(norm_name, norm), norm.eps,
@@ -315,10 +317,11 @@ class W4A4DecoderLayer(torch.nn.Module):
             return (x,) + tuple(self._norm_quant(stage, norm, norm_name, quantizer, x, consumers))
         k = x.size(-1)
         if k in (512, 1024, 2048, 4096, 8192) and self._six_bit_for(consumers, x.numel() // k, k):
-            total, q, s = _ops().rotate_and_quantize_f6(
+            total, q, s, *w6 = _ops().rotate_and_quantize_f6(
                 x.reshape(-1, k).contiguous(), hadamard=self._rotation_mode(x.numel() // k, k),
-                norm_weight=self._norm_weight16(norm_name, norm), eps=norm.eps, add=add.reshape(-1, k).contiguous())
-            return total.view(x.shape), s.view(*x.shape[:-1], 1), None, q.view(*x.shape[:-1], -1)
+                norm_weight=self._norm_weight16(norm_name, norm), eps=norm.eps, add=add.reshape(-1, k).contiguous(),
+                **LinearFLH._beside_quantiser(consumers))
+            return total.view(x.shape), s.view(*x.shape[:-1], 1), w6 or None, q.view(*x.shape[:-1], -1)
         if self.activation == "token" and self.fused and self.record is None and k in (512, 1024, 2048, 4096, 8192):
             total, q, s = _ops().add_rmsnorm_rotate_and_quantize_i4(
                 x.reshape(-1, k).contiguous(), add.reshape(-1, k).contiguous(), self._norm_weight16(norm_name, norm),
@@ -327,9 +330,18 @@ class W4A4DecoderLayer(torch.nn.Module):
         x = x + add
         return (x,) + tuple(self._norm_quant(stage, norm, norm_name, quantizer, x, consumers))
 
+    @staticmethod
+    def _encoded(q, z, layer):
+        """The encoded weights that came with codes `q` of `layer` in the 6-bit format, as arguments of its call: taken out of the
+        list, so that their memory goes back when that call has ended."""
+        if z is None or q.size(-1) * 4 != layer.in_features * 3:
+            return {}
+        w6, z[:] = list(z), []
+        return {"w6": w6}
+
     def _project(self, layers, q, s, z):
         if self.fused:
-            return LinearFLH.forward_many(layers, q, s)
+            return LinearFLH.forward_many(layers, q, s, **self._encoded(q, z, layers[0]))
         return [layer(q, s, z, x_is_packed=True) for layer in layers]
 
     def attention(self, x, cos, sin, kv_cache=None, positions=None):
@@ -355,7 +367,7 @@ class W4A4DecoderLayer(torch.nn.Module):
                                                    self.attn_quantizer1, x, add, (self.q_proj, self.k_proj, self.v_proj))
             mode = self._qkv_rope_applies(b * t, q, s, cos, kv_cache, positions)
             if mode:
-                return self._attention_after_fused_qkv(x, q, s, cos, sin, kv_cache, positions, fold_residual, mode)
+                return self._attention_after_fused_qkv(x, q, s, z, cos, sin, kv_cache, positions, fold_residual, mode)
             qs, ks, vs = self._project([self.q_proj, self.k_proj, self.v_proj], q, s, z)
         self._tap("q_proj", qs), self._tap("k_proj", ks), self._tap("v_proj", vs)
         static = isinstance(kv_cache, StaticKVCache._Layer)
@@ -450,10 +462,14 @@ class W4A4DecoderLayer(torch.nn.Module):
         """o_proj on the quantised attention output; returns as _output_projection."""
         if fold_residual and self._residual_in_gemm(q.numel() // q.size(-1), self.o_proj):
             # the residual addition in o_proj's epilogue; nothing is left pending
-            return self.o_proj(q, s, z, x_is_packed=True, residual=x), None, cache
-        y = self.o_proj(q, s, z, x_is_packed=True)
+            return self._linear(self.o_proj, q, s, z, residual=x), None, cache
+        y = self._linear(self.o_proj, q, s, z)
         self._tap("o_proj", y)
         return x, y, cache
+
+    def _linear(self, layer, q, s, z, **residual):
+        w6 = self._encoded(q, z, layer)
+        return layer(q, s, None if w6 else z, x_is_packed=True, **residual, **w6)
 
     def _own_prefill_attention(self, t):
         """Whether a block of t > 1 new tokens takes this library's causal-attention kernel (heads of 128 channels) instead
@@ -481,7 +497,7 @@ class W4A4DecoderLayer(torch.nn.Module):
             for l in layers)
         return "f6" if six else "i4"
 
-    def _attention_after_fused_qkv(self, x, codes, scales, cos, sin, kv_cache, positions, fold_residual, mode):
+    def _attention_after_fused_qkv(self, x, codes, scales, zeros, cos, sin, kv_cache, positions, fold_residual, mode):
         """The prefill attention block from the quantised input on: q / k / v, rotary embedding and cache write in one
         launch (the bits of the separate launches), torch's fused attention, then the output projection."""
         b, t, _ = x.shape
@@ -505,8 +521,10 @@ class W4A4DecoderLayer(torch.nn.Module):
         rows, a_rows = codes.reshape(b * t, -1), scales.reshape(b * t, -1)
         if mode == "f6":
             a6 = rows.contiguous() if rows.size(1) * 4 == self.hidden_size * 3 else _ops().encode_f6(rows.contiguous())
-            qs = _ops().gemm_f6_qkv_rope(a6, a_rows.contiguous(), LinearFLH._six_bit_weights_of(layers), w_scales,
+            w6 = self._encoded(codes, zeros, self.q_proj).get("w6") or LinearFLH._six_bit_weights_of(layers)
+            qs = _ops().gemm_f6_qkv_rope(a6, a_rows.contiguous(), w6, w_scales,
                                          cos.contiguous(), sin.contiguous(), slots, keys, values, b)
+            del w6
         else:
             qs = _ops().gemm_i4_qkv_rope(rows, a_rows, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
                                          w_scales, cos.contiguous(), sin.contiguous(), slots, keys, values, b, group)
@@ -581,8 +599,9 @@ class W4A4DecoderLayer(torch.nn.Module):
         if (self._group_six_bit_for(consumers, x.numel() // x.size(-1), x.size(-1)) and _stock_call(quantizer, ActQuantizer)
                 and not quantizer.use_hadamard and not quantizer.per_token):
             # (a quantiser that does more, or something else, is called: its consumers re-encode its codes)
-            q, s = _ops().group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), False)
-            return s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
+            q, s, *w6 = _ops().group_quantize_f6(x.reshape(-1, x.size(-1)).contiguous(), False,
+                                                 **LinearFLH._beside_quantiser(consumers))
+            return s.view(*x.shape[:-1], -1), w6 or None, q.view(*x.shape[:-1], -1)
         s, z, q = quantizer(x)
         self._tap(stage + ".input", x.reshape(-1, x.size(-1)))
         self._tap(stage + ".codes", q.reshape(-1, q.size(-1)))
@@ -605,19 +624,20 @@ class W4A4DecoderLayer(torch.nn.Module):
                                                    self.mlp_quantizer1, x, add, pair)
             if self.fused and self.record is None and self._swiglu_gemm_applies(rows):
                 # prefill: gate and up in one launch that stores silu(gate) * up only (no fp16 [M, I] round trips)
-                mid = LinearFLH.forward_swiglu(self.gate_proj, self.up_proj, q, s)
+                mid = LinearFLH.forward_swiglu(self.gate_proj, self.up_proj, q, s, **self._encoded(q, z, self.gate_proj))
                 if self.activation == "token":
                     s, z, q = self._token_quant("mlp_mid", mid, consumers=(self.down_proj,))
                 else:
                     if self._group_six_bit_for((self.down_proj,), rows, mid.size(-1)):
-                        q, s = _ops().group_quantize_f6(mid.view(rows, -1), False)
+                        q, s, *w6 = _ops().group_quantize_f6(mid.view(rows, -1), False,
+                                                             **LinearFLH._beside_quantiser((self.down_proj,)))
                     else:
-                        q, s = _ops().quant_and_pack_i4_gs(mid.view(-1, 128), 128)
-                    s, z, q = s.view(*x.shape[:-1], -1), None, q.view(*x.shape[:-1], -1)
+                        (q, s), w6 = _ops().quant_and_pack_i4_gs(mid.view(-1, 128), 128), []
+                    s, z, q = s.view(*x.shape[:-1], -1), w6 or None, q.view(*x.shape[:-1], -1)
                     fold_residual = fold_residual and self._residual_in_gemm(rows, self.down_proj)
                 if fold_residual:
-                    return self.down_proj(q, s, z, x_is_packed=True, residual=x), None
-                return x, self.down_proj(q, s, z, x_is_packed=True)
+                    return self._linear(self.down_proj, q, s, z, residual=x), None
+                return x, self._linear(self.down_proj, q, s, z)
             gate, up = self._project([self.gate_proj, self.up_proj], q, s, z)
             self._tap("gate_proj", gate), self._tap("up_proj", up)
         if (self.activation == "token" and self.fused and self.record is None and rows <= 256
@@ -638,8 +658,8 @@ class W4A4DecoderLayer(torch.nn.Module):
         else:
             s, z, q = self._group_quant("mlp_mid", self.mlp_quantizer2, torch.nn.functional.silu(gate) * up)
         if fold_residual and self._residual_in_gemm(rows, self.down_proj):
-            return self.down_proj(q, s, z, x_is_packed=True, residual=x), None
-        y = self.down_proj(q, s, z, x_is_packed=True)
+            return self._linear(self.down_proj, q, s, z, residual=x), None
+        y = self._linear(self.down_proj, q, s, z)
         self._tap("down_proj", y)
         return x, y
 

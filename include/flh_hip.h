@@ -216,6 +216,24 @@ int flh_silu_mul_group_quant_f6(const flh_half* gate, const flh_half* up, uint8_
 int flh_rotate_quant_f6(const flh_half* x, const flh_half* add, flh_half* sum_out, int rmsnorm, const flh_half* weight,
                         float eps, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard, float clip_ratio,
                         void* stream);
+/* The three quantisers above together with flh_encode_f6_multi of the weights that their codes are to meet (packed [rows, K / 2] ->
+ * encoded [rows, K / 128 * 96], count 1 .. 4; K of its own; weights null: the quantiser alone), which neither waits for the other:
+ * one launch where the quantiser is a kernel of groups without rotation or of rows of 4096 with float32 butterflies and its input is
+ * no longer than 100 Mi values, else two. */
+typedef struct flh_encode_list {
+  int count;
+  const uint8_t* packed[4];
+  uint8_t* encoded[4];
+  size_t rows[4];
+  size_t K;
+} flh_encode_list;
+int flh_group_quant_encode_f6(const flh_half* x, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard,
+                              float scale_mul, const flh_encode_list* weights, void* stream);
+int flh_rmsnorm_group_quant_encode_f6(const flh_half* x, const flh_half* weight, uint8_t* encoded, flh_half* scales, uint32_t M,
+                                      uint32_t K, float eps, const flh_encode_list* weights, void* stream);
+int flh_rotate_quant_encode_f6(const flh_half* x, const flh_half* add, flh_half* sum_out, int rmsnorm, const flh_half* weight,
+                               float eps, uint8_t* encoded, flh_half* scales, uint32_t M, uint32_t K, int hadamard, float clip_ratio,
+                               const flh_encode_list* weights, void* stream);
 /* Group scales of 128 codes on the same instruction: b_scale [N, K/128], a_scale [M, K/128] (a_cols = K/128) or
  * [M] (a_cols = 1: one scale per token, applied after the groups).  The float32 accumulator makes the fold per
  * group one FMA per output; same bits as flh_gemm_i4_o16 with group = 128 on the same codes and scales. */
