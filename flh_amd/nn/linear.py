@@ -65,6 +65,21 @@ class LinearFLH(torch.nn.Module):
     #   320 x 11008 52 / 43 / 46, but the host's part of the encoding makes a layer of 300 or 450 tokens slower (245 / 262; 500: 271 / 263)
     TRANSIENT_ROWS = (2560, 641)
     TRANSIENT_ROWS_GROUPS = 513
+    # The same lines where a decoder layer's quantiser writes the codes in the 6-bit format and encodes the weights in its own launch:
+    # (rows from which, 128 x 128 tiles that a K up to 8192 needs more of, a longer one).  Effect of the change on a layer of 200 to
+    # 570 us (8B / 7B shapes; qkv 6144 / 12288 channels, gate + up 28672 / 22016, o and down 4096), us by rows:
+    #   group scales: qkv 257 .. 384 -1 .. +2 (144 tiles) / -10 (288), 700 -16 / -7; gate + up 257 .. 384 -2 .. +1 / -6, 385 .. 512 -16 ..
+    #     -20 / -6; down 257 .. 512 -9 .. -11 / -4 .. -5 (96 and 128 tiles); o 257 .. 384 +2 .. +5, 800 -4 / +3, 900 .. 1024 (256) -3 .. -5
+    #   a scale per token: qkv 257 .. 384 -1 / -8, 513 -4 / -7; gate + up 257 .. 384 -1 .. -4 / -6, 385 .. 640 -9 .. -15 / -5 .. -14;
+    #     down (a rotation that shares no launch) 257 .. 512 0 .. +4, 513 .. 640 (160) -6 .. -10
+    #   one scale per channel: gate + up 1024 +4 / +4, 1200 +8, 1400 -13 / +5, 1500 .. 1700 -6 .. -30, 2048 -21 / -33; down 2048 (512) 0,
+    #     2100 .. 2400 -14 .. -24; qkv 1400 .. 2400 0 / -3; o 2100 .. 2400 -4 .. -7
+    # 256 rows and fewer have smaller int8 tiles: a layer of 256 tokens 164 us, of 257 214.  Up to 384 rows the encoding of more than
+    # 24576 channels takes what the faster instruction gives (hidden 8192, gate + up 57344, 257 rows: 547 -> 559 with them).  Hidden sizes
+    # below 4096 keep the lines above: their layers wait for the host, which has more to do here (hidden 2048, 400 tokens 154 / 164).
+    # The whole layer, us: 257 tokens 220 -> 200 and 214 -> 204 (7B, 8B), 400 231 -> 215 and 247 -> 218; a scale per token 640 tokens
+    # 274 -> 250 and 293 -> 280; one scale per channel 2100 tokens 555 -> 516 and 574 -> 520; hidden 5120, 400 tokens 329 -> 294.
+    BESIDE_QUANTISER = ((1409, 512, 512), (257, 255, 128), (257, 255, 95))
     _NO_ROWS = 1 << 62                             # more rows than any call has
 
     def _transient_tiles(self, grouped, nibbles, groups=False):
@@ -80,14 +95,19 @@ class LinearFLH(torch.nn.Module):
 
     def _six_bit_rows(self, grouped, columns=None, nibbles=False, groups=False):
         """Rows from which a launch over `columns` channels (this layer's, unless it shares the launch) takes the 6-bit
-        instruction.  nibbles: its activations come as packed codes, to be encoded as well; groups: with a scale per group of 128."""
+        instruction.  nibbles: its activations come as packed codes, to be encoded as well; groups: with a scale per group of 128.
+        Given `columns` and no nibbles, the quantiser encodes the weights (as wants_six_bit says)."""
         if self.six_bit is not False:
             if self.six_bit == "never":
                 return self._NO_ROWS
             if self._keeps_six_bit(grouped):
                 return self.six_bit_min_rows
-        first = self.TRANSIENT_ROWS_GROUPS if grouped and groups else self.TRANSIENT_ROWS[grouped]
+        groups = grouped and groups
         tiles = -(-(columns or self.out_features) // 128)
+        if columns and not nibbles and (self.in_features >= 4096 if groups else self.in_features in (4096, 11008, 14336)):
+            first, *needs = self.BESIDE_QUANTISER[2 if groups else grouped]
+            return max(first, 385 if tiles > 192 else 0, 128 * (needs[self.in_features > 8192] // tiles) + 1)
+        first = self.TRANSIENT_ROWS_GROUPS if groups else self.TRANSIENT_ROWS[grouped]
         return max(first, 128 * (self._transient_tiles(grouped, nibbles, groups) // tiles) + 1)
 
     def prepare_six_bit(self):
@@ -131,7 +151,7 @@ class LinearFLH(torch.nn.Module):
     def wants_six_bit(self, n_rows, columns=None, groups=False):
         """Whether a call with `n_rows` rows quantised per token (or, `groups`, per group of 128) takes the 6-bit matrix
         instruction (a producer can then write the activations in that format directly, rotate_and_quantize_f6).
-        `columns`: channels of the whole launch, where several layers share one."""
+        `columns`: channels of the whole launch, from a caller whose quantiser is given the weights to encode (_beside_quantiser)."""
         if self._below_six_bit(n_rows) or self.in_features % 128 or not self.w_packed.is_cuda:
             return False
         cols = self.w_scale.numel() // self.out_features
@@ -141,7 +161,7 @@ class LinearFLH(torch.nn.Module):
 
     def _below_six_bit(self, n_rows):
         """Whether `n_rows` rows are fewer than any setting takes to the 6-bit instruction."""
-        return n_rows < self.six_bit_min_rows and n_rows < self.TRANSIENT_ROWS_GROUPS
+        return n_rows < self.six_bit_min_rows and n_rows < self.BESIDE_QUANTISER[-1][0]
 
     def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)

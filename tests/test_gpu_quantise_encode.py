@@ -61,3 +61,31 @@ def test_refusals():
     for bad in ([], _weights(128, (4,)), _weights(256, (1,) * 5)):
         with pytest.raises(RuntimeError):
             P._CUDA.group_quantize_f6(x, False, weights=bad)
+
+
+@pytest.mark.parametrize("activation,weight_group,inter,rows", [("group", 128, 11008, (256, 257, 513)), ("group", 128, 14336, (384, 385, 896, 897)),
+                                                                ("token", 128, 11008, (257, 512, 513)), ("token", 0, 11008, (1408, 1409, 2048, 2049))])
+def test_layer_around_the_lines(activation, weight_group, inter, rows):
+    """The row counts from which the parts of a layer (7B and 8B shapes) take the 6-bit instruction with weights encoded beside the
+    quantiser: the bits of the int8 kernels, and no encoding kept."""
+    from flh_amd.quantized_model import W4A4DecoderLayer, rotary_tables
+    h, kv = 4096, 4096 if inter == 11008 else 1024
+    g = torch.Generator(device="cuda").manual_seed(inter)
+    rand = lambda n, k: (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).half()
+    w = {"q_proj": rand(h, h), "k_proj": rand(kv, h), "v_proj": rand(kv, h), "o_proj": rand(h, h), "gate_proj": rand(inter, h),
+         "up_proj": rand(inter, h), "down_proj": rand(h, inter)}
+    layer = W4A4DecoderLayer.from_float(w, 32, kv // 128, fused=True, activation=activation, weight_group_size=weight_group)
+    x = torch.randn(1, rows[-1], h, device="cuda", generator=g).half()
+    taken = set()
+    for m in rows:
+        cos, sin = rotary_tables(torch.arange(m, device="cuda"), 128)
+        layer.set_six_bit(False)
+        got = layer(x[:, :m].contiguous(), cos, sin)
+        layers = [getattr(layer, n) for n in layer.PROJECTIONS]
+        assert all(l._w6 is None for l in layers)
+        taken.add(tuple(l.wants_six_bit(m, c, activation == "group") for l, c in ((layer.q_proj, h + 2 * kv), (layer.gate_proj, 2 * inter),
+                                                                                  (layer.o_proj, h), (layer.down_proj, h))))
+        layer.set_six_bit("never")
+        want = layer(x[:, :m].contiguous(), cos, sin)
+        assert torch.equal(got[0], want[0]) and all(torch.equal(a, b) for a, b in zip(got[1], want[1]))
+    assert len(taken) > 1
