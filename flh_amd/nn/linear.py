@@ -146,6 +146,20 @@ class LinearFLH(torch.nn.Module):
         packed = LinearFLH._weights_to_encode(layers) if len(layers) > 1 else None
         return [l._six_bit_weights() for l in layers] if packed is None else _pkg._CUDA.encode_f6_many(packed)
 
+    @staticmethod
+    def _six_bit_operands(layers, rows, encoded, w6):
+        """(codes, [weights]) of `layers` in the 6-bit format, from codes that are `encoded` already or packed ones; w6: the weights'
+        encodings, if there are any.  Packed codes and weights that have to be encoded share a launch (us a call, two launches
+        -> one: 600 x 4096 codes, 11008 channels 52.8 -> 51.0, 513 x 11008, 4096 channels 58.4 -> 55.4, 4096 x 4096, 11008 channels with one
+        scale each 122.3 -> 118.7)."""
+        rows = rows.contiguous()
+        if not encoded and w6 is None and len(layers) < 4:
+            packed = LinearFLH._weights_to_encode(layers)
+            if packed is not None:
+                rows, *w6 = _pkg._CUDA.encode_f6_many([rows, *packed])
+                return rows, w6
+        return rows if encoded else _pkg._CUDA.encode_f6(rows), w6 or LinearFLH._six_bit_weights_of(layers)
+
     _SIX_BIT_MAX_ROWS = ((1 << 32) - 1) // 96       # rows of either operand that the 6-bit launches index; more go to int8
 
     def wants_six_bit(self, n_rows, columns=None, groups=False):
@@ -207,8 +221,7 @@ class LinearFLH(torch.nn.Module):
         encoded = rows.size(1) * 4 == self.in_features * 3      # activations already in the 6-bit format
         if encoded or self._six_bit_applies(rows, a_rows, w_scale, group):
             ops = _pkg._CUDA
-            w6 = self._six_bit_weights() if w6 is None else w6[0]
-            a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
+            a6, (w6,) = self._six_bit_operands((self,), rows, encoded, w6)
             if encoded and not ((w_scale.size(1) == 1 and a_rows.size(1) == 1) or
                                 (group == 128 and w_scale.size(1) == self.in_features // 128)):
                 raise ValueError("6-bit activations need per-token x per-channel scales or group-of-128 weight scales")
@@ -250,8 +263,7 @@ class LinearFLH(torch.nn.Module):
         columns = sum(l.out_features for l in layers)
         if encoded or all(l._six_bit_applies(rows, a_rows, ws, group, columns) for l, ws in zip(layers, w_scales)):
             # every layer takes the 6-bit matrix instruction here: one launch there as well
-            a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            ys = ops.gemm_f6_dequant_multi(a6, w6 or LinearFLH._six_bit_weights_of(layers), a_rows.contiguous(), w_scales)
+            ys = ops.gemm_f6_dequant_multi(*LinearFLH._six_bit_operands(layers, rows, encoded, w6), a_rows.contiguous(), w_scales)
         else:
             ys = ops.gemm_i4_dequant_multi(rows, [l.w_packed.view(l.out_features, l.in_features // 2) for l in layers],
                                            a_rows, w_scales, group)
@@ -279,8 +291,8 @@ class LinearFLH(torch.nn.Module):
         if encoded or not any(l._below_six_bit(rows.size(0)) for l in both) and all(
                 l._six_bit_applies(rows, a_rows, l.w_scale.view(n, -1), group, 2 * n) for l in both):
             ops = _pkg._CUDA
-            a6 = rows.contiguous() if encoded else ops.encode_f6(rows.contiguous())
-            y = ops.gemm_f6_swiglu(a6, *(w6 or LinearFLH._six_bit_weights_of(both)), a_rows.contiguous(),
+            a6, weights = LinearFLH._six_bit_operands(both, rows, encoded, w6)
+            y = ops.gemm_f6_swiglu(a6, *weights, a_rows.contiguous(),
                                    gate_layer.w_scale.view(n, -1), up_layer.w_scale.view(n, -1))
             return y.view(*lead, n)
         y = _pkg._CUDA.gemm_i4_swiglu(rows, gate_layer.w_packed.view(n, k // 2), up_layer.w_packed.view(n, k // 2),

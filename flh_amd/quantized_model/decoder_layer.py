@@ -520,8 +520,8 @@ class W4A4DecoderLayer(torch.nn.Module):
         w_scales = [l.w_scale.view(l.out_features, -1) for l in layers]
         rows, a_rows = codes.reshape(b * t, -1), scales.reshape(b * t, -1)
         if mode == "f6":
-            a6 = rows.contiguous() if rows.size(1) * 4 == self.hidden_size * 3 else _ops().encode_f6(rows.contiguous())
-            w6 = self._encoded(codes, zeros, self.q_proj).get("w6") or LinearFLH._six_bit_weights_of(layers)
+            a6, w6 = LinearFLH._six_bit_operands(layers, rows, rows.size(1) * 4 == self.hidden_size * 3,
+                                                 self._encoded(codes, zeros, self.q_proj).get("w6"))
             qs = _ops().gemm_f6_qkv_rope(a6, a_rows.contiguous(), w6, w_scales,
                                          cos.contiguous(), sin.contiguous(), slots, keys, values, b)
             del w6
