@@ -1,4 +1,4 @@
-// int4 x int4 GEMM + dequant for a handful of tokens (decode, M <= 64; up to four have a kernel of their own at the end): the weights are
+// int4 x int4 GEMM + dequant for a handful of tokens (decode, M <= 64; up to sixteen mostly take the kernels at the end): the weights are
 // streamed from HBM exactly once and the contraction is split over K inside a workgroup.
 //
 // Same arithmetic as gemm_i4.hip (codes x 16 as int8 on the matrix cores, exact int32 sums,

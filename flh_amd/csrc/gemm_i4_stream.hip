@@ -558,7 +558,7 @@ bool takes_few_tokens(const GemmArgs& a, int epi, long columns) {
 
 // Which launches are faster here than on the kernels on either side.  us, this kernel against the other (K = 4096 unless
 // stated; "large" counts 64 x 32 tiles):
-//  * up to 16 tokens, against the K split of the decode kernel: takes_few_tokens below.
+//  * up to 16 tokens, against the K split of the decode kernels: takes_few_tokens above.
 //  * 17 .. 64 tokens: always (one scale per row, 32 x 4096 5.0 against 5.7, 17 x 4096 4.9 against 5.1).
 //  * more, group-scaled weights, against 64 x 64 and 128 x 128 tiles: up to 768 large tiles, 512 if K is long (128 x 12288,
 //    768: 24 against 27; 192 x 12288, 1152: 35 against 33; 384 x 4096, 768: 22.3 against 25.1, but 64 against 60 for K = 11008,

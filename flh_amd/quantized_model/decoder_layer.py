@@ -22,7 +22,8 @@ which `fused=False` keeps for comparison.
 token; the weights are rotated the same way offline and carry one scale per output channel
 (`weight_group_size <= 0`, the arrangement of benchmark/nn/benchmark_linear_flh.py:139-222) or per group of 128
 input channels (the Llama-3 configuration).  There `fused=True` means RMSNorm inside the rotation kernel, shared-input
-launches and, for one or two tokens, the o_proj quantiser inside its GEMM.
+launches and, for one or two tokens, norm and quantiser inside the launches of q / k / v, gate / up and o_proj.  In either
+configuration long blocks encode a projection's weights for the 6-bit instruction beside the quantiser in front of it.
 
 `record`: when set to a dict, every quantiser's input / codes / scales and every linear's output of the next call
 are stored in it (by stage name) -- the taps the parity tests compare with the CPU oracle stage by stage.
