@@ -72,14 +72,16 @@ class LinearFLH(torch.nn.Module):
     #     -20 / -6; down 257 .. 512 -9 .. -11 / -4 .. -5 (96 and 128 tiles); o 257 .. 384 +2 .. +5, 800 -4 / +3, 900 .. 1024 (256) -3 .. -5
     #   a scale per token: qkv 257 .. 384 -1 / -8, 513 -4 / -7; gate + up 257 .. 384 -1 .. -4 / -6, 385 .. 640 -9 .. -15 / -5 .. -14;
     #     down (a rotation that shares no launch) 257 .. 512 0 .. +4, 513 .. 640 (160) -6 .. -10
-    #   one scale per channel: gate + up 1024 +4 / +4, 1200 +8, 1400 -13 / +5, 1500 .. 1700 -6 .. -30, 2048 -21 / -33; down 2048 (512) 0,
-    #     2100 .. 2400 -14 .. -24; qkv 1400 .. 2400 0 / -3; o 2100 .. 2400 -4 .. -7
+    #   one scale per channel: gate + up 1024 +4 / +4, 1200 +8, 2048 -21 / -33; down 2048 (512) 0, 2100 .. 2400 -14 .. -24; qkv 1400 .. 2400
+    #     0 / -3; o 2100 .. 2400 -4 .. -7.  1400 .. 1792 gate + up go by the clock: 0 .. -18 / -2 .. -16 where calls have followed each other
+    #     long enough for the power limit, which the int8 instruction meets first, +12 .. +23 / +15 .. +23 in short runs, +8 at 1513 / 7B
+    #     with the inputs of successive calls different; the eighth 256 rows, from 1793 on, cost int8 another round of tiles
     # 256 rows and fewer have smaller int8 tiles: a layer of 256 tokens 164 us, of 257 214.  Up to 384 rows the encoding of more than
     # 24576 channels takes what the faster instruction gives (hidden 8192, gate + up 57344, 257 rows: 547 -> 559 with them).  Hidden sizes
     # below 4096 keep the lines above: their layers wait for the host, which has more to do here (hidden 2048, 400 tokens 154 / 164).
     # The whole layer, us: 257 tokens 220 -> 200 and 214 -> 204 (7B, 8B), 400 231 -> 215 and 247 -> 218; a scale per token 640 tokens
     # 274 -> 250 and 293 -> 280; one scale per channel 2100 tokens 555 -> 516 and 574 -> 520; hidden 5120, 400 tokens 329 -> 294.
-    BESIDE_QUANTISER = ((1409, 512, 512), (257, 255, 128), (257, 255, 95))
+    BESIDE_QUANTISER = ((1793, 512, 512), (257, 255, 128), (257, 255, 95))
     _NO_ROWS = 1 << 62                             # more rows than any call has
 
     def _transient_tiles(self, grouped, nibbles, groups=False):

@@ -64,7 +64,7 @@ def test_refusals():
 
 
 @pytest.mark.parametrize("activation,weight_group,inter,rows", [("group", 128, 11008, (256, 257, 513)), ("group", 128, 14336, (384, 385, 896, 897)),
-                                                                ("token", 128, 11008, (257, 512, 513)), ("token", 0, 11008, (1408, 1409, 2048, 2049))])
+                                                                ("token", 128, 11008, (257, 512, 513)), ("token", 0, 11008, (1792, 1793, 2048, 2049))])
 def test_layer_around_the_lines(activation, weight_group, inter, rows):
     """The row counts from which the parts of a layer (7B and 8B shapes) take the 6-bit instruction with weights encoded beside the
     quantiser: the bits of the int8 kernels, and no encoding kept."""
