@@ -359,7 +359,7 @@ class W4A4DecoderLayer(torch.nn.Module):
         cache) -- or, when o_proj adds the residual in its epilogue (`fold_residual`, prefill sizes), (the stream after the
         block, None, cache)."""
         b, t, _ = x.shape
-        if self._online_rows_apply((self.q_proj, self.k_proj, self.v_proj), b * t):
+        if b * t <= 4 and self._online_rows_apply((self.q_proj, self.k_proj, self.v_proj), b * t):   # (look-ups of modules take time)
             # decode: residual addition, norm, quantiser and the three projections in one launch, two where faster
             x, (qs, ks, vs) = self._norm_quant_project([self.q_proj, self.k_proj, self.v_proj], self.input_layernorm,
                                                        "input_layernorm", x, add)
