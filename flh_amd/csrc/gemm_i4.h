@@ -75,6 +75,7 @@ constexpr int kDecodeMaxM = 64;
 bool gemm_dot_supports(const GemmArgs& a, int epi, int group);        // up to four tokens
 int gemm_dot_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
 bool gemm_lines_supports(const GemmArgs& a, int epi);      // (within gemm_decode_dispatch)
+bool gemm_lines_over_stream(const GemmArgs& a, int epi);
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group);
 int gemm_decode_dispatch(const GemmArgs& a, int epi, hipStream_t stream);
 

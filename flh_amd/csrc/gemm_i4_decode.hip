@@ -297,7 +297,7 @@ int launch_decode(const GemmArgs& a, hipStream_t stream) {
   return check_launch("gemm_i4_decode");
 }
 
-// Five to sixteen tokens (three and four where the kernel below ends): the kernel above with its weights by direct-to-LDS loads of whole lines, past the caches, that
+// Up to sixteen tokens (gemm_lines_supports): the kernel above with its weights by direct-to-LDS loads of whole lines, past the caches, that
 // every wave stages for itself: 2 KiB per double step, all of them requested at once; a wave waits for its own loads only.  A
 // step's sums (two groups of 1 KiB) take the place of its operands, so that the LDS of the tiles is that of the stages.
 // 16-byte piece c of row r sits at slot c ^ (r % 8): written lane after lane, and read without bank conflicts.
@@ -388,22 +388,22 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_i4_lines_kernel(const GemmAr
           lo[u] = v[(u * STEPS + i) * 512], hi[u] = v[(u * STEPS + i) * 512 + 256];
           sa[u] = TOKEN ? 0u : ra[pair], sb[u] = rb[pair];
         }
-        auto pair = [&](int u, bool both) {
+        auto pair = [&](int u) {                 // (an even number of groups: gemm_lines_supports)
           if constexpr (TOKEN) {
             out = fma_half<0>(lo[u], sb[u], out);
-            if (both) out = fma_half<1>(hi[u], sb[u], out);
+            out = fma_half<1>(hi[u], sb[u], out);
           } else {
             out = __builtin_fmaf(lo[u], mul_halves<0>(sa[u], sb[u]), out);
-            if (both) out = __builtin_fmaf(hi[u], mul_halves<1>(sa[u], sb[u]), out);
+            out = __builtin_fmaf(hi[u], mul_halves<1>(sa[u], sb[u]), out);
           }
         };
         if ((i + 1) * 2 * kWaves <= KT) {
 #pragma unroll
-          for (int u = 0; u < kWaves; ++u) pair(u, true);
+          for (int u = 0; u < kWaves; ++u) pair(u);
         } else {
 #pragma unroll
           for (int u = 0; u < kWaves; ++u)
-            if (2 * (i * kWaves + u) < KT) pair(u, 2 * (i * kWaves + u) + 1 < KT);
+            if (2 * (i * kWaves + u) < KT) pair(u);
         }
       }
     };
@@ -598,25 +598,89 @@ int launch_dot(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Up to four tokens; more than two up to K = 8192, beyond which their codes take the registers of the weights in flight (four tokens 11008
-// x 4096 7.2 / 8.8 / 8.8 -> 7.8 / 9.3 / 9.1; two 7.1 / 8.9 / 9.4 -> 6.8 / 8.2 / 8.3), and with one scale per row up to 12288 channels, where the
-// kernel above takes over (four tokens x 28672 12.5 there, 13.1 here).
-bool gemm_dot_supports(const GemmArgs& a, int epi, int group) {
-  if (a.M <= 0 || a.M > 4 || a.K > 16384 || !(epi == kRowScale || (epi == kGroupScale && group == 128))) return false;
-  if (a.M <= 2) return true;
+namespace {
+// Double steps of K that the waves of the two kernels above have room for and the row does not have: a wave's share is two, four, six or
+// eight.  They are multiplied, or another step is loaded again in their place, all the same.  What that costs sets the lines below.
+int idle_steps(const GemmArgs& a) {
+  const int filled = (a.K + 255) / 256, share = (filled + kWaves - 1) / kWaves;
+  return (share + (share & 1)) * kWaves - filled;
+}
+long all_columns(const GemmArgs& a) {
   long columns = a.N;
   for (int s = 1; s < a.n_seg; ++s) columns += a.seg_N[s];
-  return a.K <= 8192 && (epi != kRowScale || columns <= 12288);
+  return columns;
+}
+}  // namespace
+
+// Up to four tokens (us, weights from HBM, one scale per row / token scales / group scales; this kernel against what takes the launch
+// else: the kernels above, beyond 12288 channels gemm_i4_stream.hip).
+//  * One token from K = 1280 on: 1280 x 18432 5.3 / 5.7 / 5.6 against 6.3 / 7.0 / 6.1, 768 x 13824 4.5 / 4.8 / 4.8 against 4.3 / 4.3 / 4.4.
+//  * Two from 1792 on.  On many channels not where the codes of eight double steps take the registers of the weights in flight
+//    (15360 x 13824 25.0 / 29.2 / 27.0 against 22.9 / 24.8 / 24.0), nor with eleven idle steps or more on less than a workgroup of the other
+//    kernel per compute unit (4608 x 13824 9.7 / 9.9 / 9.8 against 9.3 / 9.5 / 9.6, 5376 x 18432 11.7 / 12.3 / 12.3 against 14.3 / 14.7 /
+//    15.3).  It does not take an odd number of groups (group scales, 12416 x 16384 29.4 against 36.2 on half lines).
+//  * Three and four up to K = 8192, for the codes' registers again (four tokens 11008 x 4096 7.8 / 9.3 / 9.1 against 7.2 / 8.8 / 8.8), with few
+//    idle steps (four tokens 2048 x 8192 4.9 / 5.2 / 5.2 against 4.4 / 4.7 / 4.6, 5120 x 5120 6.9 / 8.0 / 7.9 against 6.9 / 7.5 / 7.5, 6656 x
+//    5120 7.4 / 8.6 / 8.5 against 8.0 / 9.0 / 9.1).  Many channels with one scale per row go to the other kernels (4096 x 28672 13.1, whole
+//    lines 12.5); group scales with as few idle steps, from a full round of the other kernel on (token / group scales 3456 x
+//    28672 13.6 / 14.1 against 15.2 / 15.5, 7168 x 13824 15.1 / 14.7 against 13.0 / 13.1), token scales of long rows without (7936 x
+//    16384 17.3 against 15.4).
+bool gemm_dot_supports(const GemmArgs& a, int epi, int group) {
+  if (a.M <= 0 || a.M > 4 || a.K > 16384 || !(epi == kRowScale || (epi == kGroupScale && group == 128))) return false;
+  const int idle = idle_steps(a);
+  const long columns = all_columns(a);
+  const bool row = epi == kRowScale, two = a.K <= 4096;   // two: the share of a wave
+  if (a.M == 1) return a.K >= 1280;
+  if (a.M == 2)
+    return a.K >= 1792 && (columns <= 12288 || (a.K <= 12288 && (idle <= 10 || columns >= 16384)) || (!row && a.K % 256));
+  if (a.K > 8192 || idle > (two ? 4 : 6)) return false;
+  if (columns <= 12288) return true;
+  if (row) return false;
+  return (idle == 0 && two) || (columns >= 16384 && idle <= 4 && (two || idle == 0 || a.a_cols > 1));
 }
 
 int gemm_dot_dispatch(const GemmArgs& a, int epi, hipStream_t stream) {
   return epi == kRowScale ? launch_dot<kRowScale>(a, stream) : launch_dot<kGroupScale>(a, stream);
 }
 
-// Sixteen tokens; group scales up to K = 8192: with long rows the scales that have to be there before the first operand and the tiles in
-// the operands' place cost more than whole lines give (five tokens 11008 x 4096 8.7 with half lines, 9.2 so).
+// Whole lines through LDS instead of half lines to registers (us, five tokens unless stated, this against that).
+//  * One scale per row: from K = 2048 on (2048 x 5120 4.2 against 4.3, 1536 x 5120 4.3 against 3.9).  Every other row of an odd number of
+//    half lines starts inside a line: on many channels only (16 tokens 3200 x 4096 4.3 against 4.1; 3200 x 11008 6.5 against 7.2), and
+//    not beyond K = 4096.  There up to eleven idle steps (5376 x 8192 7.2 against 7.6, 4608 x 5120 6.4 against 6.2).  Shares of six and
+//    eight steps leave a compute unit one workgroup: few channels (9728 x 3072 6.2 against 6.6, x 10240 16.0 against 15.3; 12800 x
+//    3072 7.3 against 7.6, x 8192 15.0 against 13.9; three tokens 14336 x 12288 22.0 against 21.0).
+//  * Group scales wait for their table: an even number of groups, which dword loads fetch (16 tokens 3456 x 3072 5.7 against
+//    5.0), few idle steps (3584 x 5120 5.7 against 6.0; token scales 3072 x 5120 5.9 against 5.5), with a share of four on enough channels
+//    (8192 x 3072 6.8 against 7.1, x 2048 6.5 against 6.3; 6656 x 5120 8.7 against 9.0, 6400 x 3072 6.6 against 5.7), and no longer rows
+//    (11008 x 4096 9.2 against 8.7).
 bool gemm_lines_supports(const GemmArgs& a, int epi) {
-  return a.M <= 16 && (epi == kRowScale ? a.K <= 16384 : epi == kGroupScale && a.K <= 8192);
+  if (a.M > 16 || a.K > 16384) return false;
+  const int idle = idle_steps(a);
+  const long columns = all_columns(a);
+  const bool even = a.K % 256 == 0;
+  if (epi == kRowScale) {
+    if (a.K <= 4096) return a.K >= 2048 && (even || columns >= 8192);
+    if (!even || a.K <= 8192) return even && idle <= 11;
+    return columns <= 4096 ? idle <= 14 : columns <= 10240 && idle <= (a.K > 12288 ? 12 : 8);
+  }
+  if (epi != kGroupScale || !even || a.K > 8192) return false;
+  if (a.K <= 4096) return idle <= 3;
+  return idle <= 1 ? a.a_cols == 1 || columns >= 3072 : idle <= 7 && columns >= 5120;
+}
+
+// Where whole lines have lines of their own against gemm_i4_stream.hip (takes_few_tokens there; elsewhere those of half lines hold): full
+// shares, group scales of two steps only and token scales of four from a full round of that kernel on (token scales 8192 x 13824 16.0
+// against 14.6, 8 tokens x 18432 20.5 against 23.4).  One scale per row also up to three idle steps of two (3840 x 13824 7.5 against
+// 8.0, 3712 x 22016 11.2 against 12.7), some more where that kernel's only round is far from full or its last one short (7424 x 11008 10.9
+// against 12.5, 7936 x 18432 17.0 against 19.8; 7168 x 13824 12.9 against 12.5, 8 tokens 6400 x 28672 23.4 against 20.6, 2048 x 11008
+// 5.9 against 5.3).
+bool gemm_lines_over_stream(const GemmArgs& a, int epi) {
+  const int idle = idle_steps(a);
+  const long columns = all_columns(a);
+  if (!gemm_lines_supports(a, epi) || columns > 32768 || a.K > 8192) return false;
+  const bool two = a.K <= 4096;
+  if (epi != kRowScale) return idle == 0 && (two || (a.a_cols == 1 && columns >= 16384));
+  return idle <= (two ? 3 : 0) || (idle <= (two ? 5 : 7) && (columns <= 12288 || (columns >= 16384 && columns <= 24576)));
 }
 
 bool gemm_decode_supports(const GemmArgs& a, int epi, int group) {

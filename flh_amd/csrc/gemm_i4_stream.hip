@@ -537,17 +537,19 @@ bool stream_takes(const GemmArgs& a, int epi, int group) {
 
 // Up to 16 tokens against gemm_i4_decode.hip (us, K = 4096, this kernel / that one, one scale per row / token scales / group scales; one to
 // four tokens come here only where the dot-product kernel does not take them).
-//  * Where that one takes whole lines, up to 32768 channels: from nine tokens on from 172 workgroups of 64 channels on (16 x 11008 7.7 / 8.2 /
-//    8.4 against 7.6 / 8.2 / 8.1, x 12288 7.9 / 8.4 / 8.5 against 7.9 / 8.4 / 8.4, x 14336 8.3 / 8.7 / 8.8 against 9.3 / 9.9 / 9.8; weights that
-//    the last-level cache holds x 12288 6.6 / 7.7 / 8.0 against 7.1 / 8.0 / 8.0), with fewer only token scales beyond 24576 (5 x
-//    22016 12.6 / 12.7 / 12.8 against 10.6 / 12.0 / 11.3, x 28672 13.9 / 13.9 / 14.0 against 12.5 / 14.1 / 12.9).
-//  * Elsewhere, up to 16384 channels, one workgroup of 64 per compute unit: with five or more tokens from 172 workgroups on, with
-//    fewer beyond 12288 channels, where that kernel has more than three of its workgroups on a compute unit.  Beyond, the compute
-//    units that get one workgroup more set the time and the other kernel's grows with the channels: with few tokens only if the
-//    last round has enough workgroups, and not where that kernel's tiles of every group leave a compute unit one workgroup.
+//  * Against whole lines (gemm_lines_over_stream), up to 32768 channels: from nine tokens on from 172 workgroups of 64 channels on (16 x
+//    11008 7.7 / 8.2 / 8.4 against 7.6 / 8.2 / 8.1, x 12288 7.9 / 8.4 / 8.5 against 7.9 / 8.4 / 8.4, x 14336 8.3 / 8.7 / 8.8 against 9.3 / 9.9 /
+//    9.8; weights that the last-level cache holds x 12288 6.6 / 7.7 / 8.0 against 7.1 / 8.0 / 8.0), with fewer only token scales beyond
+//    24576 (5 x 22016 12.6 / 12.7 / 12.8 against 10.6 / 12.0 / 11.3, x 28672 13.9 / 13.9 / 14.0 against 12.5 / 14.1 / 12.9).
+//  * Else, up to 16384 channels, one workgroup of 64 per compute unit: with five or more tokens from 172 workgroups on, with fewer
+//    beyond 12288 channels, where half lines have more than three workgroups on a compute unit.  Beyond, the compute units that get
+//    one workgroup more set the time and the other kernel's grows with the channels: with few tokens only if the last round has
+//    enough workgroups, and not where that kernel's tiles of every group leave a compute unit one workgroup.  (Drawn against half lines;
+//    beyond 32768 channels, where whole lines may stand in for them, the launches that they get are as fast as on half lines: one
+//    scale per row, 3 to 8 tokens, x 49152 0.99, x 65536 1.00, x 128256 1.01 of the time.)
 bool takes_few_tokens(const GemmArgs& a, int epi, long columns) {
   const bool row = epi == kRowScale, token = a.a_cols == 1;
-  if (gemm_lines_supports(a, epi) && columns <= 32768) return a.M > 8 ? columns >= 172 * 64 : !row && token && columns > 24576;
+  if (gemm_lines_over_stream(a, epi)) return a.M > 8 ? columns >= 172 * 64 : !row && token && columns > 24576;
   if (columns <= 16384 || a.M > (row ? 4 : token ? 6 : 8) || (!row && a.K > 8192))
     return a.M >= 5 ? columns >= 172 * 64 : columns > 12288;
   const long last = (columns - 1) % 16384 + 1;             // channels of the last round
