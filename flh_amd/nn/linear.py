@@ -82,6 +82,7 @@ class LinearFLH(torch.nn.Module):
     # The whole layer, us: 257 tokens 220 -> 200 and 214 -> 204 (7B, 8B), 400 231 -> 215 and 247 -> 218; a scale per token 640 tokens
     # 274 -> 250 and 293 -> 280; one scale per channel 2100 tokens 555 -> 516 and 574 -> 520; hidden 5120, 400 tokens 329 -> 294.
     BESIDE_QUANTISER = ((1793, 512, 512), (257, 255, 128), (257, 255, 95))
+    _LEAST_ROWS = BESIDE_QUANTISER[-1][0]          # the first of all these lines
     _NO_ROWS = 1 << 62                             # more rows than any call has
 
     def _transient_tiles(self, grouped, nibbles, groups=False):
@@ -177,7 +178,7 @@ class LinearFLH(torch.nn.Module):
 
     def _below_six_bit(self, n_rows):
         """Whether `n_rows` rows are fewer than any setting takes to the 6-bit instruction."""
-        return n_rows < self.six_bit_min_rows and n_rows < self.BESIDE_QUANTISER[-1][0]
+        return n_rows < self.six_bit_min_rows and n_rows < self._LEAST_ROWS
 
     def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)

@@ -342,7 +342,7 @@ class W4A4DecoderLayer(torch.nn.Module):
 
     def _project(self, layers, q, s, z):
         if self.fused:
-            return LinearFLH.forward_many(layers, q, s, **self._encoded(q, z, layers[0]))
+            return LinearFLH.forward_many(layers, q, s, **({} if z is None else self._encoded(q, z, layers[0])))
         return [layer(q, s, z, x_is_packed=True) for layer in layers]
 
     def attention(self, x, cos, sin, kv_cache=None, positions=None):
@@ -359,17 +359,17 @@ class W4A4DecoderLayer(torch.nn.Module):
         cache) -- or, when o_proj adds the residual in its epilogue (`fold_residual`, prefill sizes), (the stream after the
         block, None, cache)."""
         b, t, _ = x.shape
-        if b * t <= 4 and self._online_rows_apply((self.q_proj, self.k_proj, self.v_proj), b * t):   # (look-ups of modules take time)
+        qkv = (self.q_proj, self.k_proj, self.v_proj)     # (looking a module up takes the host half a microsecond)
+        if self._online_rows_apply(qkv, b * t):
             # decode: residual addition, norm, quantiser and the three projections in one launch, two where faster
-            x, (qs, ks, vs) = self._norm_quant_project([self.q_proj, self.k_proj, self.v_proj], self.input_layernorm,
-                                                       "input_layernorm", x, add)
+            x, (qs, ks, vs) = self._norm_quant_project(qkv, self.input_layernorm, "input_layernorm", x, add)
         else:
             x, s, z, q = self._residual_norm_quant("attn_in", self.input_layernorm, "input_layernorm",
-                                                   self.attn_quantizer1, x, add, (self.q_proj, self.k_proj, self.v_proj))
+                                                   self.attn_quantizer1, x, add, qkv)
             mode = self._qkv_rope_applies(b * t, q, s, cos, kv_cache, positions)
             if mode:
                 return self._attention_after_fused_qkv(x, q, s, z, cos, sin, kv_cache, positions, fold_residual, mode)
-            qs, ks, vs = self._project([self.q_proj, self.k_proj, self.v_proj], q, s, z)
+            qs, ks, vs = self._project(qkv, q, s, z)
         self._tap("q_proj", qs), self._tap("k_proj", ks), self._tap("v_proj", vs)
         static = isinstance(kv_cache, StaticKVCache._Layer)
         out = None
@@ -469,6 +469,8 @@ class W4A4DecoderLayer(torch.nn.Module):
         return x, y, cache
 
     def _linear(self, layer, q, s, z, **residual):
+        if z is None:
+            return layer(q, s, None, x_is_packed=True, **residual)
         w6 = self._encoded(q, z, layer)
         return layer(q, s, None if w6 else z, x_is_packed=True, **residual, **w6)
 
@@ -557,12 +559,12 @@ class W4A4DecoderLayer(torch.nn.Module):
     def _online_rows_apply(self, layers, rows):
         """Whether `layers` take the launch with norm and quantiser inside: one or two tokens rotated as whole rows, up to four in
         groups (which of them by one launch and which by two, the operations know)."""
-        if not (self.fused and self.record is None and 0 < rows <= (2 if self.activation == "token" else 4)
-                and self.hidden_size == 4096 and self._online_applies(layers)):
+        token = self.activation == "token"
+        if not (0 < rows <= (2 if token else 4) and self.hidden_size == 4096 and self.fused and self.record is None):
             return False
-        if self.activation == "token":
-            return True
-        return (self.act_group_size == 128 and all(l.w_scale.numel() > l.out_features for l in layers)
+        if token:
+            return self._online_applies(layers)
+        return (self.act_group_size == 128 and layers[0].w_scale.numel() > layers[0].out_features and self._online_applies(layers)
                 and not self._group_six_bit_for(layers, rows, self.hidden_size))
 
     def _norm_quant_project(self, layers, norm, norm_name, x, add):
@@ -639,7 +641,7 @@ class W4A4DecoderLayer(torch.nn.Module):
                 if fold_residual:
                     return self._linear(self.down_proj, q, s, z, residual=x), None
                 return x, self._linear(self.down_proj, q, s, z)
-            gate, up = self._project([self.gate_proj, self.up_proj], q, s, z)
+            gate, up = self._project(pair, q, s, z)
             self._tap("gate_proj", gate), self._tap("up_proj", up)
         if (self.activation == "token" and self.fused and self.record is None and rows <= 256
                 and self.intermediate_size in (11008, 14336)):

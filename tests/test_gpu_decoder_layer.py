@@ -191,6 +191,19 @@ def test_hooks_on_projections_see_packed_codes_and_leave_the_bits(activation, t)
     assert [s[0] for s in seen] == [256, 512] and (t > 64 or not any(s[1] for s in seen))
 
 
+@pytest.mark.parametrize("activation", ["token", "group"])
+@pytest.mark.parametrize("tokens", [2, 5])
+def test_a_step_looks_a_projection_up_once(monkeypatch, activation, tokens):
+    """A step of a few tokens waits for the host, which pays for every look-up of a module."""
+    _, layer = make(activation=activation)
+    x = torch.randn(tokens, 1, 512, generator=torch.Generator().manual_seed(7)).half().cuda()
+    cos, sin = rotary_tables(torch.arange(1, device="cuda"), 128)
+    seen, look_up = [], torch.nn.Module.__getattr__
+    monkeypatch.setattr(W4A4DecoderLayer, "__getattr__", lambda self, name: seen.append(name) or look_up(self, name), raising=False)
+    layer(x, cos, sin)
+    assert [seen.count(name) for name in ("k_proj", "v_proj", "up_proj")] == [1, 1, 1]
+
+
 @pytest.mark.parametrize("weight_group,six_bit,shapes", [(128, False, [(1, 64), (1, 65), (3, 43), (1, 257), (2, 300), (1, 1100)]),
                                                          (128, True, [(1, 65), (1, 131)]), (0, False, [(1, 65), (2, 512), (1, 1025)])])
 def test_group_layer_with_the_product_in_the_gemm_gives_the_same_bits(monkeypatch, weight_group, six_bit, shapes):
