@@ -587,9 +587,10 @@ template <int MAXM, int EPI>
 int launch_dot(const GemmArgs& a, hipStream_t stream) {
   const int steps = (a.K + 256 * kWaves - 1) / (256 * kWaves);   // double steps of a wave
   if (steps <= 2) return launch_dot<MAXM, 2, EPI>(a, stream);
-  if (steps <= 4) return launch_dot<MAXM, 4, EPI>(a, stream);
-  if (steps <= 6) return launch_dot<MAXM, 6, EPI>(a, stream);
-  return launch_dot<MAXM, 8, EPI>(a, stream);
+  if constexpr (MAXM <= 2) {                                     // (gemm_dot_supports: more tokens up to K = 8192)
+    if (steps > 4) return steps <= 6 ? launch_dot<MAXM, 6, EPI>(a, stream) : launch_dot<MAXM, 8, EPI>(a, stream);
+  }
+  return launch_dot<MAXM, 4, EPI>(a, stream);
 }
 template <int EPI>
 int launch_dot(const GemmArgs& a, hipStream_t stream) {
