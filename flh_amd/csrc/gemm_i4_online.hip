@@ -313,10 +313,13 @@ int launch_kernel(const OnlineArgs& a, hipStream_t stream) {
   return check_launch("gemm_i4_online");
 }
 
-// as many tiles per workgroup as leave one workgroup to a compute unit, at most eight
+// As many tiles per workgroup as leave one workgroup to a compute unit; beyond eight, as many as leave every compute unit the same number
+// (us, rotation, one scale per row, eight tiles always / so: one token x 33000 19.2 / 14.1, x 40960 21.0 / 15.8, two 24.6 / 20.1; norm and
+// groups, one token x 36864 22.1 / 15.9).  The package's own rules stop at eight tiles and earlier with more tokens (torch_ext.cpp has
+// them); the entry points take every width.
 template <int EPI, int PRO, int MAXM>
 int launch_by_tiles(const OnlineArgs& a, hipStream_t stream) {
-  const int per = (a.tiles + 255) / 256;
+  const int all = (a.tiles + 255) / 256, rounds = (all + 7) / 8, per = (all + rounds - 1) / rounds;
   if (per <= 1) return launch_kernel<EPI, PRO, 1, MAXM>(a, stream);
   if (per == 2) return launch_kernel<EPI, PRO, 2, MAXM>(a, stream);
   if constexpr (MAXM <= 2 || PRO == kNormGroup) {      // (more tokens to rotate than two: the callers' rules stop earlier)

@@ -30,8 +30,9 @@ def make(ns, cols, seed, offset=0):
     return x, add, w, Bs, Ss
 
 
-# one tile per workgroup, a ragged last tile, every tile count, more tiles than one round of workgroups, several matrices
-CHANNELS = [(16,), (40, 8), (4096, 24, 1000), (8200,), (12300,), (16000, 40), (24000,), (28672,), (33000,)]
+# one tile per workgroup, a ragged last tile, every tile count, more tiles than one round of workgroups (two of five and of six), several
+# matrices
+CHANNELS = [(16,), (40, 8), (4096, 24, 1000), (8200,), (12300,), (16000, 40), (24000,), (28672,), (33000,), (44000, 1100)]
 
 
 @pytest.mark.parametrize("ns", CHANNELS)
