@@ -41,8 +41,10 @@ def test_heads_of_64_are_refused(ops):
 
 
 @pytest.mark.parametrize("batch", [1, 2, 3, 5, 7, 9])
-def test_layer_steps(batch):
-    """A decode step of the group configuration, fused and module by module: the same bits."""
+def test_layer_steps(monkeypatch, batch):
+    """A decode step of the group configuration: with norm, quantiser and projections in one launch and the codes out of attention's
+    combine, with all of these in launches of their own (the same bits), and module by module (the same attention block; the MLP's
+    product of silu and up is torch's there, an exponential's last bit apart)."""
     from flh_amd.quantized_model import StaticKVCache, W4A4DecoderLayer
     from flh_amd.quantized_model.decoder_layer import rotary_tables
     gen = torch.Generator(device="cuda").manual_seed(batch)
@@ -53,9 +55,8 @@ def test_layer_steps(batch):
     weights["input_layernorm"] = (torch.rand(h, device="cuda", generator=gen) + 0.5).half()
     layer = W4A4DecoderLayer.from_float(weights, 32, 8, activation="group")
     x = torch.randn(batch, 1, h, device="cuda", generator=gen).half()
-    outs = []
-    for fused in (True, False):
-        layer.fused = fused
+
+    def step(call):
         cache = StaticKVCache(1, batch, 8, 100, 128, "cuda", q_heads=32)
         cache.keys[0].normal_(generator=torch.Generator(device="cuda").manual_seed(1))
         cache.values[0].normal_(generator=torch.Generator(device="cuda").manual_seed(2))
@@ -63,9 +64,22 @@ def test_layer_steps(batch):
         positions = cache.advance(1)
         cos, sin = rotary_tables(positions, 128)
         with torch.no_grad():
-            y, _ = layer(x, cos, sin, cache.layer(0), positions)
-        outs.append((y, cache.keys[0], cache.values[0]))
-    assert torch.equal(outs[0][1], outs[1][1]) and torch.equal(outs[0][2], outs[1][2])
-    # (the product of silu and up is the library's in one and torch's in the other: an exponential's last bit)
-    err = (outs[0][0].float() - outs[1][0].float()).norm() / outs[1][0].float().norm()
+            y, _ = call(x, cos, sin, cache.layer(0), positions)
+        return y, cache.keys[0], cache.values[0]
+
+    # the paths that this is about are the ones that are taken
+    assert layer._attention_quantises(batch)
+    for pair in ((layer.q_proj, layer.k_proj, layer.v_proj), (layer.gate_proj, layer.up_proj)):
+        assert layer._online_rows_apply(pair, batch) == (batch <= 4)
+    whole, attention = step(layer), step(layer.attention)
+    with monkeypatch.context() as apart:
+        apart.setattr(layer, "_attention_quantises", lambda rows: False)
+        apart.setattr(layer, "_online_rows_apply", lambda layers, rows: False)
+        for got, want in ((whole, step(layer)), (attention, step(layer.attention))):
+            assert all(torch.equal(g, w) for g, w in zip(got, want))
+    layer.fused = False
+    assert all(torch.equal(g, w) for g, w in zip(attention, step(layer.attention)))
+    modules = step(layer)
+    assert torch.equal(whole[1], modules[1]) and torch.equal(whole[2], modules[2])
+    err = (whole[0].float() - modules[0].float()).norm() / modules[0].float().norm()
     assert err < 0.02, err

@@ -55,14 +55,29 @@ def test_whole_rows(ops, ns, cols):
 
 @pytest.mark.parametrize("ns", CHANNELS)
 @pytest.mark.parametrize("offset", [0, 1])
-def test_groups(ops, ns, offset):
+@pytest.mark.parametrize("through", ["ctypes", "extension"])
+def test_groups(ops, ns, offset, through):
+    """The one launch (ctypes) and what the decoder layer calls: one launch or two, by tokens and channels (extension)."""
+    import flh_amd._ext_ops as extension
+    op = (ops if through == "ctypes" else extension).rmsnorm_group_quantize_gemm_i4_multi
     x, _, w, Bs, Ss = make(ns, 32, sum(ns) + 7, offset)
     for m in (1, 2, 3, 4):
         for weight in (w, None):
-            outs = ops.rmsnorm_group_quantize_gemm_i4_multi(x[:m], weight, 1e-5, Bs, Ss)
+            outs = op(x[:m], weight, 1e-5, Bs, Ss)
             q, a = ops.rmsnorm_and_quantize_i4_gs(x[:m].contiguous(), weight, 1e-5, 128, False)
             for B, S, got in zip(Bs, Ss, outs):
                 assert torch.equal(got, ops.gemm_i4_dequant(q.view(m, -1), B, a.view(m, -1), S, 128)), (m, weight is None, B.size(0))
+
+
+def test_a_norm_weight_off_the_alignment(ops):
+    """The one launch needs it aligned; the extension takes two."""
+    import flh_amd._ext_ops as extension
+    x, _, w, Bs, Ss = make((600, 40), 32, 9)
+    moved = torch.cat((w[:1], w))[1:]
+    assert moved.data_ptr() % 16 and moved.is_contiguous()
+    for m in (1, 3):
+        want = extension.rmsnorm_group_quantize_gemm_i4_multi(x[:m], w, 1e-5, Bs, Ss)
+        assert all(torch.equal(a, b) for a, b in zip(extension.rmsnorm_group_quantize_gemm_i4_multi(x[:m], moved, 1e-5, Bs, Ss), want))
 
 
 def test_scales_off_the_alignment(ops):
