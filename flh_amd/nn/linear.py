@@ -177,8 +177,9 @@ class LinearFLH(torch.nn.Module):
         return self._six_bit_rows(cols != 1, columns, False, groups) <= n_rows <= self._SIX_BIT_MAX_ROWS
 
     def _below_six_bit(self, n_rows):
-        """Whether `n_rows` rows are fewer than any setting takes to the 6-bit instruction."""
-        return n_rows < self.six_bit_min_rows and n_rows < self._LEAST_ROWS
+        """Whether `n_rows` rows are fewer than this layer takes to the 6-bit instruction in any launch."""
+        return (n_rows < (self._LEAST_ROWS if self.in_features >= 4096 else self.TRANSIENT_ROWS_GROUPS)
+                and (self.six_bit is False or n_rows < self.six_bit_min_rows))
 
     def _six_bit_applies(self, rows, a_scale, w_scale, group, columns=None):
         n = rows.size(0)

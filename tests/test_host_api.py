@@ -647,3 +647,18 @@ def test_few_rows_add_the_residual_in_plain_projections_only(monkeypatch, change
     else:
         assert stream is x and y is not None
         assert layer.o_proj.seen == (64, []) if change == "replaced" else seen == [None]
+
+
+@pytest.mark.parametrize("k", [1024, 2048, 4096, 5120, 8192, 11008, 14336])
+@pytest.mark.parametrize("setting", [False, "never", True, None])
+def test_rows_below_every_six_bit_line(k, setting):
+    """The question that is asked first answers "below" only where no launch of the layer takes the 6-bit instruction, and does so up
+    to the layer's own first line."""
+    from flh_amd.nn import LinearFLH
+    layer = LinearFLH(k, 128, in_group_size=128, group_size=128, no_hadamard=True)
+    layer.six_bit = setting
+    lines = [layer._six_bit_rows(grouped, columns, nibbles, groups) for grouped in (False, True) for groups in (False, True)
+             for nibbles in (False, True) for columns in (None, 128, 6144, 22016, 28672, 1 << 20)]
+    below = [n for n in range(1, 600) if layer._below_six_bit(n)]
+    assert all(n < min(lines) for n in below)
+    assert len(below) == (255 if setting is not False else 256 if k >= 4096 else 512)
