@@ -119,7 +119,6 @@ def gemm_i4_dequant_multi(A, Bs, A_scale, B_scales, group_size=128):
     """gemm_i4_dequant of the same activations against several weight matrices (q / k / v, gate / up) in one
     launch: Bs, B_scales are lists of up to four [N_s, K/2] / [N_s, 1 | K/g] tensors -> list of fp16 [M, N_s],
     each bit-identical to its own gemm_i4_dequant call."""
-    import ctypes
     _check(len(Bs) == len(B_scales) and 1 <= len(Bs) <= 4, "one to four weight matrices, one scale tensor each")
     for B, B_scale in zip(Bs, B_scales):
         _check_gemm_inputs(A, B, A_scale, B_scale)
@@ -164,7 +163,6 @@ def gemm_i4_qkv_rope(A, A_scale, Bs, B_scales, cos, sin, positions, k_cache, v_c
     gemm_i4_dequant_multi(A, Bs, ...) followed by rope_kv_cache_ computes, same bits, in one launch.  A [batch * T, K/2]
     packed codes, Bs = [q, k, v] weights with heads of 128 channels, cos / sin [T, 128], positions [T] int64 (cache slots),
     k_cache / v_cache [batch, kv_heads, max_len, 128] (written in place) -> rotated queries [batch, T, heads, 128]."""
-    import ctypes
     _check(len(Bs) == 3 and len(B_scales) == 3, "three weight matrices (q, k, v), one scale tensor each")
     for B, B_scale in zip(Bs, B_scales):
         _check_gemm_inputs(A, B, A_scale, B_scale)
@@ -273,7 +271,6 @@ def rotate_quantize_gemm_i4(x, B, B_scale):
 def rotate_quantize_gemm_i4_multi(x, Bs, B_scales):
     """rotate_quantize_gemm_i4 for up to four weight matrices that share the tokens, in one launch:
     -> list of fp16 [M, N_s], each bit-identical to its own call."""
-    import ctypes
     _check(len(Bs) == len(B_scales) and 1 <= len(Bs) <= 4, "one to four weight matrices, one scale tensor each")
     _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
            "x must be a contiguous 2D float16 CUDA tensor")
@@ -302,7 +299,6 @@ def rmsnorm_rotate_quantize_gemm_i4_multi(x, add, weight, eps, Bs, B_scales):
     """rotate_quantize_gemm_i4_multi on RMSNorm(x [+ add]) in one launch: x (and add, or None) [M, 4096] fp16 with M <= 4,
     weight [4096] fp16 or None -> (x + add [M, 4096] fp16 or None, [fp16 [M, N_s] ...]); the outputs are those of
     [add_]rmsnorm_rotate_and_quantize_i4 followed by gemm_i4_dequant_multi, bit for bit."""
-    import ctypes
     _check(len(Bs) == len(B_scales) and 1 <= len(Bs) <= 4, "one to four weight matrices, one scale tensor each")
     _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
            "x must be a contiguous 2D float16 CUDA tensor")
@@ -340,7 +336,6 @@ def rmsnorm_group_quantize_gemm_i4_multi(x, weight, eps, Bs, B_scales):
     """RMSNorm(x) quantised in groups of 128 (no rotation) and up to four GEMMs in one launch: x [M, 4096] fp16 with M <= 4,
     weight [4096] fp16 or None, group scales [N, 32] -> [fp16 [M, N_s] ...]; the outputs are those of rmsnorm_and_quantize_i4_gs
     followed by gemm_i4_dequant_multi, bit for bit."""
-    import ctypes
     _check(len(Bs) == len(B_scales) and 1 <= len(Bs) <= 4, "one to four weight matrices, one scale tensor each")
     _check(x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.is_contiguous(),
            "x must be a contiguous 2D float16 CUDA tensor")
@@ -541,7 +536,6 @@ def gemm_f6_dequant_add(A6, B6, A_scale, B_scale, residual, out=None):
 def gemm_f6_qkv_rope(A6, A_scale, B6s, B_scales, cos, sin, positions, k_cache, v_cache, batch):
     """gemm_i4_qkv_rope on operands encoded by encode_f6 (or written by rotate_and_quantize_f6): scales all one column, or
     weight scales [N, K/128] with A_scale [M, 1] or [M, K/128].  Same bits."""
-    import ctypes
     _check(len(B6s) == 3 and len(B_scales) == 3, "three weight matrices (q, k, v), one scale tensor each")
     M = K = None
     for B6, S in zip(B6s, B_scales):
@@ -589,7 +583,6 @@ def gemm_f6_swiglu(A6, B6_gate, B6_up, A_scale, gate_scale, up_scale):
 def gemm_f6_dequant_multi(A6, B6s, A_scale, B_scales):
     """gemm_f6_dequant_o16 (all scales one column) resp. gemm_f6_dequant_o16_gs for up to four encoded weight
     matrices that share the encoded activations, in one launch -> list of fp16 [M, N_s], same bits as the single calls."""
-    import ctypes
     _check(len(B6s) == len(B_scales) and 1 <= len(B6s) <= 4, "one to four weight matrices, one scale tensor each")
     M = K = None
     for B6, S in zip(B6s, B_scales):

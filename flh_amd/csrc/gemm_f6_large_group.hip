@@ -16,10 +16,13 @@
 // 2048 x 4096 x 14336 93 -> 89 / 105 -> 100, 1000 x 4096 x 14336 (128 tiles) - / 91 -> 79; with tiles of 128 x 128 65, 1000 x 4096 x
 // 4096 31 -> 21.  The same four waves with fewer instructions (buffer loads, no clamped offsets) gave 1-3 %.
 //
-// What bounds it now: power (1.95 GHz with token scales), to which everything adds: without the operand loads 294 us instead of
-// 361 (token scales, 8192 x 14336 x 4096), from a cached slab 331, without the fragment reads 323, without the folds 278, the
-// MFMAs alone 173; the outputs of a tile 40.  The 128 x 128 tile: its LDS traffic (24 fragments and 24 KB of loads per step of
-// 256 matrix clocks).
+// What bounds it now: no unit is full.  Of the 1575 clocks of a step with token scales (2048 x 28672, outputs included) the matrix pipe is
+// busy for 512 and vector instructions are issued for 728, LDS beside them for 630, a third of it bank conflicts; with group scales 768,
+// 812 and 692 of 1705 (counters; four waves 1800 and 1970).  A fifth resp. a fourteenth of the clocks is neither matrix nor vector work.
+// On top of that power: 1.82 GHz over 8192 x 14336 x 4096, 2.0 over half of that, 2.2 in launches of 65 us.  Everything adds to
+// both: without the operand loads 294 us instead of 361 (token scales, 8192 x 14336 x 4096), from a cached slab 331, without the fragment
+// reads 323, without the folds 278, the MFMAs alone 173; the outputs of a tile 40.  The 128 x 128 tile: its LDS traffic (24 fragments
+// and 24 KB of loads per step of 256 matrix clocks; 490 of 1076 clocks busy).
 #include "gemm_f6_large.h"
 
 namespace flh {

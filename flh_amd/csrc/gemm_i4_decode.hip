@@ -18,10 +18,10 @@
 // the scale tables took 3.4 us before the first weight was requested and the fold 2.4 at the end.  The scales now come as they
 // are, by direct-to-LDS loads behind the first weights; tiles are stored as float32 by the waves that made them and folded
 // without bank conflicts, two groups of scales per read, eight pairs of groups read ahead of their multiply-adds (a pair at a
-// time the chain waits for LDS at every pair: one token 4096 x 14336 12.7 us with group scales where the eight take 10.9).
-// us, weights from HBM, against scales as float tables and integer tiles (N x K), token scales / group scales:
-//   16 tokens: 4096 x 14336 14.8 / 15.1 -> 11.4 / 11.5, 4096 x 11008 12.4 / 12.7 -> 9.9 / 9.8, 6144 x 4096 8.5 / 8.4 -> 7.4 /
-//   7.4, 4096 x 4096 6.5 / 6.6 -> 5.5 / 5.6;  one token: 4096 x 14336 11.9 / 12.0 -> 10.3 / 10.9, 4096 x 4096 5.7 / 5.7 -> 5.1 / 5.2
+// time the chain waits for LDS at every pair).  What still comes here is long rows with group scales, widths that the kernels at the
+// end are not filled by, and integer output.  us, weights from HBM, against scales as float tables and integer tiles (N x K), token scales /
+// group scales: 16 tokens 4096 x 14336 14.8 / 15.1 -> 11.4 / 11.5, 4096 x 11008 12.4 / 12.7 -> 9.9 / 9.8; now also 5 tokens 5120 x 5120
+// 7.6 / 7.6, 16 tokens 8.7 / 8.6.
 #include <atomic>
 #include "gemm_i4.h"
 #include "lane_ops.h"

@@ -28,6 +28,7 @@ namespace flh {
 namespace {
 
 constexpr int kWaves = 8;
+// The rotations are written for rows of 4096; norm and groups would do at any multiple of 2048 and is measured at this one only.
 constexpr int kK = 4096, kRowB = kK / 2, kGroups = kK / 128;
 constexpr int kDoubles = kGroups / 2 / kWaves;     // double steps per wave
 constexpr int kCodePitch = kRowB + 16;             // code rows 16 bytes apart in the banks

@@ -75,10 +75,16 @@ class LinearFLH(torch.nn.Module):
     #   one scale per channel: gate + up 1024 +4 / +4, 1200 +8, 2048 -21 / -33; down 2048 (512) 0, 2100 .. 2400 -14 .. -24; qkv 1400 .. 2400
     #     0 / -3; o 2100 .. 2400 -4 .. -7.  1400 .. 1792 gate + up go by the clock: 0 .. -18 / -2 .. -16 where calls have followed each other
     #     long enough for the power limit, which the int8 instruction meets first, +12 .. +23 / +15 .. +23 in short runs, +8 at 1513 / 7B
-    #     with the inputs of successive calls different; the eighth 256 rows, from 1793 on, cost int8 another round of tiles
+    #     with the inputs of successive calls different.  The line is 22016 channels': their eighth 256 rows, from 1793 on, cost int8 another
+    #     round of tiles (the launch with its quantiser, 1792 / 1793 rows: int8 141 / 162, 6-bit 134 / 138); 28672 have it at 2049 (int8 190 /
+    #     197, at 2049 224; 6-bit 173 / 177, 187), q / k / v beyond 2048 rows (6144 59 / 59 up to there, 70 / 65 beyond; 12288 98 / 100, 121 /
+    #     113).  What it does to the whole layer of 1793 .. 2048 tokens, long runs / short ones / one input again and again: 22016 -3 .. -8 /
+    #     -17 .. -20 / 0 .. -3 of 440, 28672 +5 .. -2 / -2 .. -10 / +9 .. +13 of 460; of 2100, 28672 -46 / -50 / -42 of 570
     # 256 rows and fewer have smaller int8 tiles: a layer of 256 tokens 164 us, of 257 214.  Up to 384 rows the encoding of more than
     # 24576 channels takes what the faster instruction gives (hidden 8192, gate + up 57344, 257 rows: 547 -> 559 with them).  Hidden sizes
-    # below 4096 keep the lines above: their layers wait for the host, which has more to do here (hidden 2048, 400 tokens 154 / 164).
+    # below 4096 keep the lines above: their layers wait for the host, which has more to do here (hidden 2048, 400 tokens 154 / 164).  So
+    # does whole-row rotation at K = 8192, whose layers were not timed, and a linear that quantises for itself (forward_online), which asks
+    # without columns: its lines are those of an encoding in a launch of its own.
     # The whole layer, us: 257 tokens 220 -> 200 and 214 -> 204 (7B, 8B), 400 231 -> 215 and 247 -> 218; a scale per token 640 tokens
     # 274 -> 250 and 293 -> 280; one scale per channel 2100 tokens 555 -> 516 and 574 -> 520; hidden 5120, 400 tokens 329 -> 294.
     BESIDE_QUANTISER = ((1793, 512, 512), (257, 255, 128), (257, 255, 95))
@@ -168,7 +174,8 @@ class LinearFLH(torch.nn.Module):
     def wants_six_bit(self, n_rows, columns=None, groups=False):
         """Whether a call with `n_rows` rows quantised per token (or, `groups`, per group of 128) takes the 6-bit matrix
         instruction (a producer can then write the activations in that format directly, rotate_and_quantize_f6).
-        `columns`: channels of the whole launch, from a caller whose quantiser is given the weights to encode (_beside_quantiser)."""
+        `columns`: channels of the whole launch, from a caller whose quantiser is given the weights to encode (_beside_quantiser); the
+        lines of BESIDE_QUANTISER are a decoder layer's."""
         if self._below_six_bit(n_rows) or self.in_features % 128 or not self.w_packed.is_cuda:
             return False
         cols = self.w_scale.numel() // self.out_features

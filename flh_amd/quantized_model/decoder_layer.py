@@ -558,7 +558,7 @@ class W4A4DecoderLayer(torch.nn.Module):
 
     def _online_rows_apply(self, layers, rows):
         """Whether `layers` take the launch with norm and quantiser inside: one or two tokens rotated as whole rows, up to four in
-        groups (which of them by one launch and which by two, the operations know)."""
+        groups (the extension's operations take two launches where those are faster, the ctypes ones always one)."""
         token = self.activation == "token"
         if not (0 < rows <= (2 if token else 4) and self.hidden_size == 4096 and self.fused and self.record is None):
             return False
