@@ -253,8 +253,10 @@ class W4A4DecoderLayer(torch.nn.Module):
     @staticmethod
     def _take_six_bit(consumers, n_rows, groups):
         """(Another module in a projection's place, or one with hooks, is given the packed codes that it documents.)"""
-        return (all(isinstance(l, LinearFLH) for l in consumers)
-                and all(l.wants_six_bit(n_rows, sum(c.out_features for c in consumers), groups) for l in consumers)
+        if not all(isinstance(l, LinearFLH) for l in consumers):
+            return False
+        columns = sum(l.out_features for l in consumers)
+        return (all(l.wants_six_bit(n_rows, columns, groups) for l in consumers)
                 and all(_stock_call(l, LinearFLH) for l in consumers))
 
     def _group_six_bit_for(self, consumers, n_rows, width):
